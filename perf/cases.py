@@ -31,30 +31,30 @@ def _dense(name, kind, hidden, heads, kv_heads, head_dim, ff, vocab, layers, pro
 def listed():
     return [
         # a short request to a small model: nothing but latency and launches
-        _dense("small model, first words", "generate", 512, 8, 4, 64, 1376, 8003, 4, 12, 16, dtype=F16, theta=1e4),
+        _dense("small model first words", "generate", 512, 8, 4, 64, 1376, 8003, 4, 12, 16, dtype=F16, theta=1e4),
         # the benchmark's model and prompt: a long document read, an answer begun
-        _dense("qwen3 8b, long prompt", "generate", 4096, 32, 8, 128, 12288, 151936, 36, 8192, 64, qk_norm=True),
+        _dense("qwen3 8b long prompt", "generate", 4096, 32, 8, 128, 12288, 151936, 36, 8192, 64, qk_norm=True),
         # a turn of a conversation
-        _dense("4096 wide, chat turn", "generate", 4096, 32, 8, 128, 14336, 128256, 8, 600, 48, theta=5e5),
+        _dense("4096 wide chat turn", "generate", 4096, 32, 8, 128, 14336, 128256, 8, 600, 48, theta=5e5),
         # a page of text for a model whose width is no power of two, with projection biases
-        _dense("3584 wide, a page", "generate", 3584, 28, 4, 128, 18944, 152064, 4, 900, 16, bias=True),
+        _dense("3584 wide a page", "generate", 3584, 28, 4, 128, 18944, 152064, 4, 900, 16, bias=True),
         # an answer drawn from the distribution
-        _dense("2560 wide, sampled", "generate", 2560, 32, 8, 128, 9728, 151936, 6, 701, 32, qk_norm=True, temperature=0.7, top_p=0.9),
+        _dense("2560 wide sampled", "generate", 2560, 32, 8, 128, 9728, 151936, 6, 701, 32, qk_norm=True, temperature=0.7, top_p=0.9),
         # narrow heads, half precision
-        _dense("2048 wide, heads of 64", "generate", 2048, 32, 8, 64, 8192, 128256, 6, 1024, 32, dtype=F16, theta=5e5),
+        _dense("2048 wide heads of 64", "generate", 2048, 32, 8, 64, 8192, 128256, 6, 1024, 32, dtype=F16, theta=5e5),
         # a server's batch: 32 short conversations on one set of weights
-        _dense("32 sequences, 4096 wide", "batch", 4096, 32, 8, 128, 12288, 151936, 6, 130, 24, qk_norm=True, sequences=32),
+        _dense("32 sequences 4096 wide", "batch", 4096, 32, 8, 128, 12288, 151936, 6, 130, 24, qk_norm=True, sequences=32),
         # a few sequences on a small model
-        _dense("6 sequences, 1024 wide", "batch", 1024, 16, 8, 128, 3072, 151936, 12, 75, 24, qk_norm=True, sequences=6),
+        _dense("6 sequences 1024 wide", "batch", 1024, 16, 8, 128, 3072, 151936, 12, 75, 24, qk_norm=True, sequences=6),
         # drafts of another model checked: a few given tokens at a time, the logits of every one wanted
-        _dense("5120 wide, drafts scored", "verify", 5120, 40, 8, 128, 13824, 152064, 2, 240, 5, bias=True),
+        _dense("5120 wide drafts scored", "verify", 5120, 40, 8, 128, 13824, 152064, 2, 240, 5, bias=True),
         # mixed stacks at widths of their benchmark
         dict(name="retorax 4096 wide", kind="retorax", hidden=4096, heads=32, kv_heads=8, ff=12288, channels=4096, chunk=1536,
              vocab=65536, layers=6, prompt=3000, steps=24),
         dict(name="kavuvik 2048 wide", kind="kavuvik", hidden=2048, heads=16, q_rank=768, kv_rank=512, window=1024, experts=64,
              top=6, expert_ff=768, shared_ff=1536, vocab=65536, layers=5, prompt=1800, steps=24),
         # one token through a layer of FP8 experts and the projections around it
-        dict(name="fp8 experts, one token", kind="fp8", hidden=7168, expert_ff=2048, experts=48, top=8, q_rank=1536, heads=128,
+        dict(name="fp8 experts one token", kind="fp8", hidden=7168, expert_ff=2048, experts=48, top=8, q_rank=1536, heads=128,
              head_dim=192, dtype=BF16),
     ]
 
