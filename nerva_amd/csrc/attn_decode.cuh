@@ -11,7 +11,7 @@ constexpr uint32_t kAttnMaxSplits = 64;   // split-KV partials per kv head
 // KV cache layout (library-owned): [layer][physical block][kv_head][tile of 16 tokens x head_dim]
 // 16-bit, K and V in separate arrays. One (block, kv_head) tile is contiguous
 // (4 KiB at head_dim 128), so a wave streams it with four 1 KiB load instructions.
-// Inside a tile, head_dim 128 is stored in matrix-core operand order (kv_k_elem, kv_v_elem);
+// Inside a tile, head_dim 64 and 128 are stored in matrix-core operand order (kv_k_elem, kv_v_elem);
 // every other head_dim is row-major [token][dim].
 __host__ __device__ __forceinline__ uint64_t kv_tile_offset(uint32_t block_count, uint32_t kv_heads,
                                                             uint32_t head_dim, uint32_t layer,
@@ -20,18 +20,19 @@ __host__ __device__ __forceinline__ uint64_t kv_tile_offset(uint32_t block_count
          kKvBlockTokens * head_dim;
 }
 
-// Element offset of (token row, dim d) inside a K tile. head_dim 128: load j of lane
+__host__ __device__ __forceinline__ bool kv_operand_order(uint32_t head_dim) { return head_dim == 128 || head_dim == 64; }
+// Element offset of (token row, dim d) inside a K tile. In operand order load j of lane
 // l = (d%32/8)*16 + row holds dims 32j + 8*(l/16) .. +7 of token l%16, the A operand of a
 // 16x16x32 matrix-core product over dims.
 __host__ __device__ __forceinline__ uint32_t kv_k_elem(uint32_t head_dim, uint32_t row, uint32_t d) {
-  if (head_dim != 128) return row * head_dim + d;
+  if (!kv_operand_order(head_dim)) return row * head_dim + d;
   return (d / 32) * 512 + (((d % 32) / 8) * 16 + row) * 8 + d % 8;
 }
-// Same for a V tile. head_dim 128: load j of lane l = (row/4)*16 + d%16 holds tokens
+// Same for a V tile: load j of lane l = (row/4)*16 + d%16 holds tokens
 // 4*(l/16) .. +3 of dim 32j + l%16, then of dim 32j + 16 + l%16: the A operands of two
 // 16x16x16 products over tokens (V transposed).
 __host__ __device__ __forceinline__ uint32_t kv_v_elem(uint32_t head_dim, uint32_t row, uint32_t d) {
-  if (head_dim != 128) return row * head_dim + d;
+  if (!kv_operand_order(head_dim)) return row * head_dim + d;
   const uint32_t slab = d / 16, n = d % 16;
   return (slab / 2) * 512 + ((row / 4) * 16 + n) * 8 + (slab % 2) * 4 + row % 4;
 }
@@ -121,6 +122,11 @@ constexpr uint32_t kAttnPlanHeader = 8, kAttnPlanEntry = 8, kAttnPlanWaves = 8;
 __host__ __device__ __forceinline__ uint64_t attn_plan_bytes(uint32_t splits) {
   return (kAttnPlanHeader + static_cast<uint64_t>(splits) * kAttnPlanWaves * kAttnPlanEntry) * sizeof(uint32_t);
 }
+// The shapes of the matrix-core kernels: up to eight query heads a kv head (a wave's sixteen columns hold the hi and the
+// lo half of each), heads of 64 or 128. Everything else takes the general kernel, one token a launch.
+__host__ __device__ __forceinline__ bool attn_matrix_cores(uint32_t heads, uint32_t kv_heads, uint32_t head_dim) {
+  return kv_operand_order(head_dim) && kv_heads != 0 && heads % kv_heads == 0 && heads / kv_heads >= 1 && heads / kv_heads <= 8;
+}
 // Split geometry shared by the kernel and the plan: a split takes ceil(blocks / splits) blocks - or all of
 // them while the context is short (single_blocks, 0 = never): the exchange between splits costs about 3 us
 // whatever the context, and up to some 300 keys one workgroup per kv head has read its keys before that
@@ -173,7 +179,7 @@ inline uint32_t attn_default_splits(uint32_t kv_heads, uint32_t block_count) {
   return splits == 0 ? 1 : splits;
 }
 uint64_t attn_workspace_bytes(uint32_t heads, uint32_t head_dim);
-// Bytes of AttnParams::part_tagged (head_dim 128), zero-initialised once.
+// Bytes of AttnParams::part_tagged (head_dim up to 128), zero-initialised once.
 uint64_t attn_step_workspace_bytes(uint32_t heads);
 // Carves part_acc/part_m/part_l/counters out of a workspace of attn_workspace_bytes().
 void attn_bind_workspace(AttnParams &p, void *workspace);
@@ -182,14 +188,14 @@ hipError_t launch_attn_decode(uint32_t dtype, const AttnParams &p, hipStream_t s
 // Prompt block: rounds and writes the K and V rows of `tokens` consecutive positions
 // (position .. position + tokens - 1) into the cache - bias, per-head RMSNorm (k_norm) and RoPE
 // as in the decode kernel - so that a following launch_attn_decode with append = 0 and the same
-// token block finds every row of the block in place. head_dim 128 only. Uses qkv, k_norm, k_bias,
+// token block finds every row of the block in place. attn_matrix_cores shapes only. Uses qkv, k_norm, k_bias,
 // v_bias, the caches and table, rope_freq / rope_cs and the token strides of `p`.
 hipError_t launch_kv_publish_rows(uint32_t dtype, const AttnParams &p, hipStream_t stream);
 
 // Attention of a prompt block with the K/V tiles of the prefix shared by the block's tokens
 // (attn_prompt.hip): same inputs and outputs as launch_attn_decode for a block (tokens consecutive
 // positions from `position`, rows already in the cache, append = 0, per-token strides, per-token split
-// workspaces, rotation tables per token row), head_dim 128 and GQA factor 1/2/4/8 only.
+// workspaces, rotation tables per token row), attn_matrix_cores shapes only.
 // p.splits = 0 lets the launcher choose.
 hipError_t launch_attn_prompt(uint32_t dtype, const AttnParams &p, hipStream_t stream);
 

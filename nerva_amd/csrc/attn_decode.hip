@@ -7,11 +7,11 @@
 // (precision/block/ops.rs:52-73), apply_rotary_to_heads (common/rope.rs:54-79),
 // exact_blockwise_attention_into (attention/exact/run.rs:13-127).
 //
-// gfx950 mapping of the fast path (head_dim 128, G = heads/kv_heads in {1,2,4,8}):
+// gfx950 mapping of the fast path (head_dim HD = 64 or 128, G = heads/kv_heads up to 8):
 //   grid (kv_heads, splits), 8 waves per workgroup; a wave owns whole 16-token KV
 //   tiles of its workgroup's token range and runs q.K^T and P.V on the matrix cores
 //   (details at attn_fast_body). The cache keeps each tile in matrix-operand order,
-//   so a tile is eight coalesced 1 KiB loads straight into operand registers; two tiles
+//   so a tile is eight (HD = 64: four) coalesced 1 KiB loads straight into operand registers; two tiles
 //   are in flight per wave. LDS only carries q, the new K/V row and the cross-wave
 //   merge. The last workgroup to finish a kv head merges its split partials (arrival
 //   counter; nobody waits), so a layer needs no separate reduce launch.
@@ -50,9 +50,9 @@ __device__ __forceinline__ void token_view(AttnParams &p, uint32_t z) {
 }
 
 // K and V rows of a prompt block into the cache: grid (kv head, token), two waves (key, value).
-template <uint32_t DT>
+template <uint32_t DT, int HD>
 __global__ __launch_bounds__(2 * kWave) void kv_publish_rows_kernel(AttnParams p) {
-  __shared__ __align__(16) uint16_t row16[2][kHD];
+  __shared__ __align__(16) uint16_t row16[2][HD];
   const uint32_t kvh = blockIdx.x, z = blockIdx.y;
   const int lane = threadIdx.x & (kWave - 1);
   const int wave = threadIdx.x / kWave;
@@ -65,37 +65,37 @@ __global__ __launch_bounds__(2 * kWave) void kv_publish_rows_kernel(AttnParams p
     p.block_count = seq.block_count;
     pos = seq.position;
   }
-  const uint32_t A = p.heads * kHD, KV = p.kv_heads * kHD;
+  const uint32_t A = p.heads * HD, KV = p.kv_heads * HD;
   const float *qkv = p.qkv + static_cast<uint64_t>(z) * p.qkv_token_stride;
   const float *rope_cs = p.rope_cs != nullptr ? p.rope_cs + static_cast<uint64_t>(z) * p.rope_token_stride : nullptr;
-  const uint32_t off = (wave == 0 ? A : A + KV) + kvh * kHD;
+  const uint32_t off = (wave == 0 ? A : A + KV) + kvh * HD;
   const uint16_t *bias = wave == 0 ? p.k_bias : p.v_bias;
-  prep_head128<DT>(qkv[off + lane], qkv[off + lane + 64], bias ? bias + kvh * kHD : nullptr, wave == 0 ? p.k_norm : nullptr,
+  prep_head<DT, HD>(qkv[off + pair_of<HD>(lane)], qkv[off + pair_of<HD>(lane) + HD / 2], bias ? bias + kvh * HD : nullptr, wave == 0 ? p.k_norm : nullptr,
                    wave == 0 ? p.rope_freq : nullptr, rope_cs, pos, p.eps, lane, nullptr, row16[wave]);
   __syncthreads();
-  const uint64_t tile = kv_tile_offset(p.block_count, p.kv_heads, kHD, p.layer, p.table[pos / kKvBlockTokens], kvh);
+  const uint64_t tile = kv_tile_offset(p.block_count, p.kv_heads, HD, p.layer, p.table[pos / kKvBlockTokens], kvh);
   const uint32_t row = pos % kKvBlockTokens;
   if (wave == 0) {
-    if (lane < 16)  // K: 16 pieces of 8 consecutive dims
-      *reinterpret_cast<uint4 *>(p.k_cache + tile + kv_k_elem(kHD, row, lane * 8)) =
+    if (lane < HD / 8)  // K: pieces of 8 consecutive dims
+      *reinterpret_cast<uint4 *>(p.k_cache + tile + kv_k_elem(HD, row, lane * 8)) =
           *reinterpret_cast<const uint4 *>(row16[0] + lane * 8);
   } else {
 #pragma unroll
-    for (int i = 0; i < 2; ++i) {  // V: one 16-bit element per dim
+    for (int i = 0; i < HD / kWave; ++i) {  // V: one 16-bit element per dim
       const uint32_t d = lane + i * kWave;
-      p.v_cache[tile + kv_v_elem(kHD, row, d)] = row16[1][d];
+      p.v_cache[tile + kv_v_elem(HD, row, d)] = row16[1][d];
     }
   }
 }
 
 // Launch of the matrix-core attention body (attn_fast_body) for token blocks and batch steps: grid (kv_heads,
 // splits, tokens); the lean variant, two workgroups per CU.
-template <uint32_t DT, int G, int W>
+template <uint32_t DT, int HD, int G, int W>
 __global__ __launch_bounds__(W *kWave, W / 2) void attn_block_kernel(AttnParams p) {
-  __shared__ AttnShared<G, W> sh;
+  __shared__ AttnShared<HD, G, W> sh;
   if (blockIdx.z != 0 || p.seqs != nullptr) token_view(p, blockIdx.z);
-  const RawHeads<G, W> raw = attn_request_raw<G, W>(p, blockIdx.x);
-  attn_fast_body<DT, G, W, 1>(p, p.position, blockIdx.x, blockIdx.y, gridDim.y, sh, raw);
+  const RawHeads<G, W> raw = attn_request_raw<HD, G, W>(p, blockIdx.x);
+  attn_fast_body<DT, HD, G, W, 1>(p, p.position, blockIdx.x, blockIdx.y, gridDim.y, sh, raw);
 }
 
 // ---------------------------------------------------------------------------------------------
@@ -142,10 +142,10 @@ __device__ __forceinline__ void sload4(const uint32_t *p0, const uint32_t *p1, c
 }
 
 // The splits' partials of the step kernel, as (f32 value, tag) words. One (head, split) record is cut
-// into kStepParts parts of 32 dims, each followed by its own copy of the split's m and l, so that a part
+// into HD / 32 parts of 32 dims, each followed by its own copy of the split's m and l, so that a part
 // is read - and its tags cleared - by exactly one merging workgroup.
-constexpr uint32_t kStepParts = 4, kStepPartDims = kHD / kStepParts, kStepPartWords = kStepPartDims + 2;
-constexpr uint32_t kStepRecord = kStepParts * kStepPartWords;
+constexpr uint32_t kStepPartDims = 32, kStepPartWords = kStepPartDims + 2;
+constexpr uint32_t step_record(uint32_t head_dim) { return head_dim / kStepPartDims * kStepPartWords; }
 // One part (32 dims of one head) merged by one workgroup of 512 threads. Thread (dl = t % 32,
 // q = t / 32) takes the splits q, q + 16, q + 32, q + 48: it polls their accumulator word and their m
 // and l words until every tag is up and folds them in split order; the two groups of a wave meet by a lane
@@ -157,14 +157,14 @@ constexpr uint32_t kStepRecord = kStepParts * kStepPartWords;
 // fault word is set - the session hands it out with the token, the operator entry point through its status call -
 // and the outputs it feeds become NaN. A word counts only with this launch's tag, so a partial that lands after
 // its merge gave up is never taken for a later launch's.
-template <uint32_t DT, int G>
+template <uint32_t DT, int HD, int G>
 __device__ __forceinline__ void merge_part_tagged(const AttnParams &p, uint32_t kvh, uint32_t g, uint32_t part, uint32_t S,
                                                   uint32_t active, float *lds_o, float *lds_m, float *lds_l, bool first_part,
                                                   uint32_t tag) {
   const uint32_t spin_limit = p.merge_spin_limit != 0 ? p.merge_spin_limit : kAttnMergeSpinLimit;
   constexpr uint32_t kGroups = 16, kPer = kAttnMaxSplits / kGroups;  // 4 splits per thread at most
   const uint32_t h = kvh * G + g;
-  uint64_t *rec = p.part_tagged + static_cast<uint64_t>(h) * S * kStepRecord + part * kStepPartWords;
+  uint64_t *rec = p.part_tagged + static_cast<uint64_t>(h) * S * step_record(HD) + part * kStepPartWords;
   const uint32_t dl = threadIdx.x % kStepPartDims, q = threadIdx.x / kStepPartDims;
   uint64_t av[kPer], mv[kPer], lv[kPer];
   uint32_t spins = 0;
@@ -173,7 +173,7 @@ __device__ __forceinline__ void merge_part_tagged(const AttnParams &p, uint32_t 
 #pragma unroll
     for (uint32_t i = 0; i < kPer; ++i) {
       // unconditional loads (index clamped): a load under a branch would serialise the round
-      const uint64_t *r = rec + static_cast<uint64_t>(min(q + i * kGroups, active - 1)) * kStepRecord;
+      const uint64_t *r = rec + static_cast<uint64_t>(min(q + i * kGroups, active - 1)) * step_record(HD);
       av[i] = load_tagged(r + dl);
       mv[i] = load_tagged(r + kStepPartDims);
       lv[i] = load_tagged(r + kStepPartDims + 1);
@@ -235,7 +235,7 @@ __device__ __forceinline__ void merge_part_tagged(const AttnParams &p, uint32_t 
       ot = fmaf(lds_o[k * kStepPartDims + dl], f, ot);
     }
     if (Lt > 0.0f && isfinite(Lt)) ot /= Lt;
-    const uint32_t e = h * kHD + part * kStepPartDims + dl;
+    const uint32_t e = h * HD + part * kStepPartDims + dl;
     if (p.out_f32 != nullptr) p.out_f32[e] = ot;
     p.out16[attn_out_elem(p, e)] = enc16<DT>(ot);
   }
@@ -251,43 +251,47 @@ __device__ __forceinline__ void sload8x2(const uint32_t *a, const uint32_t *b, u
                : "memory");
 }
 
-template <int G>
+template <int HD, int G>
 struct StepShared {
-  static constexpr int kRow = kHD + 8;     // 272-byte rows: the operand reads of a lane group spread over the banks
+  static constexpr int kRow = HD + 8;      // 272-byte rows (HD = 64: 144): the operand reads of a lane group spread over the banks
   alignas(16) uint16_t qhl[2 * G][kRow];   // Qx columns: rows 0..G-1 the hi halves of the scaled query heads, G..2G-1 the lo halves
-  alignas(16) uint16_t knew[kHD];
-  alignas(16) uint16_t vnew[kHD];
+  alignas(16) uint16_t knew[HD];
+  alignas(16) uint16_t vnew[HD];
   float wm[8][G], wl[8][G];
-  alignas(16) float wacc[8][G][kHD];
+  alignas(16) float wacc[8][G][HD];
   float merge_o[8][32], merge_m[8], merge_l[8];   // the splits' merge: one entry per wave
   uint32_t is_last;
 };
 
-#define NV_AT_LD32(DST, PTR, OFF) asm volatile("global_load_dword %0, %1, off offset:" #OFF : "=v"(DST) : "v"(PTR) : "memory")
-#define NV_AT_LD16(DST, PTR, OFF) asm volatile("global_load_ushort %0, %1, off offset:" #OFF : "=v"(DST) : "v"(PTR) : "memory")
+#define NV_AT_LD32(DST, PTR, OFF) asm volatile("global_load_dword %0, %1, off offset:%2" : "=v"(DST) : "v"(PTR), "n"(OFF) : "memory")
+#define NV_AT_LD16(DST, PTR, OFF) asm volatile("global_load_ushort %0, %1, off offset:%2" : "=v"(DST) : "v"(PTR), "n"(OFF) : "memory")
 #define NV_AT_TILE_LOAD(F, PHYS)                                                                                 \
   do {                                                                                                           \
-    const uint64_t t_ = kv_tile_offset(p.block_count, p.kv_heads, kHD, p.layer, (PHYS), kvh) + lane * 8;          \
+    const uint64_t t_ = kv_tile_offset(p.block_count, p.kv_heads, HD, p.layer, (PHYS), kvh) + lane * 8;          \
     const uint16_t *kp_ = p.k_cache + t_, *vp_ = p.v_cache + t_;                                                  \
     asm volatile("global_load_dwordx4 %0, %1, off nt" : "=v"(kr[F][0]) : "v"(kp_) : "memory");                    \
     asm volatile("global_load_dwordx4 %0, %1, off offset:1024 nt" : "=v"(kr[F][1]) : "v"(kp_) : "memory");        \
-    asm volatile("global_load_dwordx4 %0, %1, off offset:2048 nt" : "=v"(kr[F][2]) : "v"(kp_) : "memory");        \
-    asm volatile("global_load_dwordx4 %0, %1, off offset:3072 nt" : "=v"(kr[F][3]) : "v"(kp_) : "memory");        \
+    if constexpr (HD == 128) {                                                                                    \
+      asm volatile("global_load_dwordx4 %0, %1, off offset:2048 nt" : "=v"(kr[F][HD / 32 - 2]) : "v"(kp_) : "memory"); \
+      asm volatile("global_load_dwordx4 %0, %1, off offset:3072 nt" : "=v"(kr[F][HD / 32 - 1]) : "v"(kp_) : "memory"); \
+    }                                                                                                             \
     asm volatile("global_load_dwordx4 %0, %1, off nt" : "=v"(vr[F][0]) : "v"(vp_) : "memory");                    \
     asm volatile("global_load_dwordx4 %0, %1, off offset:1024 nt" : "=v"(vr[F][1]) : "v"(vp_) : "memory");        \
-    asm volatile("global_load_dwordx4 %0, %1, off offset:2048 nt" : "=v"(vr[F][2]) : "v"(vp_) : "memory");        \
-    asm volatile("global_load_dwordx4 %0, %1, off offset:3072 nt" : "=v"(vr[F][3]) : "v"(vp_) : "memory");        \
+    if constexpr (HD == 128) {                                                                                    \
+      asm volatile("global_load_dwordx4 %0, %1, off offset:2048 nt" : "=v"(vr[F][HD / 32 - 2]) : "v"(vp_) : "memory"); \
+      asm volatile("global_load_dwordx4 %0, %1, off offset:3072 nt" : "=v"(vr[F][HD / 32 - 1]) : "v"(vp_) : "memory"); \
+    }                                                                                                             \
   } while (0)
-// Waits until at most 8 * TILES of this wave's requests are outstanding (TILES uniform, 0..4).
-#define NV_AT_WAIT_BEHIND(TILES)                                                \
-  do {                                                                          \
-    switch (TILES) {                                                            \
-      case 0u: asm volatile("s_waitcnt vmcnt(0)" ::: "memory"); break;          \
-      case 1u: asm volatile("s_waitcnt vmcnt(8)" ::: "memory"); break;          \
-      case 2u: asm volatile("s_waitcnt vmcnt(16)" ::: "memory"); break;         \
-      case 3u: asm volatile("s_waitcnt vmcnt(24)" ::: "memory"); break;         \
-      default: asm volatile("s_waitcnt vmcnt(32)" ::: "memory"); break;         \
-    }                                                                           \
+// Waits until at most the requests of TILES tiles (HD / 16 each) of this wave are outstanding (TILES uniform, 0..4).
+#define NV_AT_WAIT_BEHIND(TILES)                                                                    \
+  do {                                                                                              \
+    switch (TILES) {                                                                                \
+      case 0u: asm volatile("s_waitcnt vmcnt(0)" ::: "memory"); break;                              \
+      case 1u: asm volatile("s_waitcnt vmcnt(%0)" ::"n"(HD / 16) : "memory"); break;                \
+      case 2u: asm volatile("s_waitcnt vmcnt(%0)" ::"n"(HD / 8) : "memory"); break;                 \
+      case 3u: asm volatile("s_waitcnt vmcnt(%0)" ::"n"(3 * HD / 16) : "memory"); break;            \
+      default: asm volatile("s_waitcnt vmcnt(%0)" ::"n"(HD / 4) : "memory"); break;                 \
+    }                                                                                               \
   } while (0)
 // Hands registers that a wait has just covered to the compiler: every later use depends on this statement.
 #define NV_AT_TAKE_INPUTS()                                                                                        \
@@ -295,20 +299,22 @@ struct StepShared {
                : "+v"(qx0), "+v"(qx1), "+v"(ex0), "+v"(ex1), "+v"(qb0), "+v"(qb1), "+v"(eb0), "+v"(eb1), "+v"(qg0), \
                  "+v"(qg1), "+v"(kg0), "+v"(kg1), "+v"(ra), "+v"(rb))
 #define NV_AT_TAKE_TILE(F)                                                                                         \
-  asm volatile(""                                                                                                  \
-               : "+v"(kr[F][0]), "+v"(kr[F][1]), "+v"(kr[F][2]), "+v"(kr[F][3]), "+v"(vr[F][0]), "+v"(vr[F][1]),   \
-                 "+v"(vr[F][2]), "+v"(vr[F][3]))
+  do {                                                                                                             \
+    asm volatile("" : "+v"(kr[F][0]), "+v"(kr[F][1]), "+v"(vr[F][0]), "+v"(vr[F][1]));                              \
+    if constexpr (HD == 128)                                                                                       \
+      asm volatile("" : "+v"(kr[F][HD / 32 - 2]), "+v"(kr[F][HD / 32 - 1]), "+v"(vr[F][HD / 32 - 2]), "+v"(vr[F][HD / 32 - 1])); \
+  } while (0)
 #define NV_AT_U4(V) make_uint4((V).x, (V).y, (V).z, (V).w)
 
-template <uint32_t DT, int G>
+template <uint32_t DT, int HD, int G>
 __global__ __launch_bounds__(8 * kWave) void attn_step_kernel(AttnParams p) {
   constexpr int W = 8;
   constexpr int kThreads = W * kWave;
-  __shared__ StepShared<G> sh;
+  __shared__ StepShared<HD, G> sh;
   const int lane = threadIdx.x & (kWave - 1);
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
   const uint32_t kvh = blockIdx.x, split = blockIdx.y, S = gridDim.y;
-  const uint32_t A = p.heads * kHD, KV = p.kv_heads * kHD;
+  const uint32_t A = p.heads * HD, KV = p.kv_heads * HD;
   uint64_t *const tr = kvh == 0 && split == 0 ? p.trace : nullptr;
   uint64_t *const trm = kvh == 0 ? p.trace : nullptr;
   link_mark(tr, 7);
@@ -316,31 +322,32 @@ __global__ __launch_bounds__(8 * kWave) void attn_step_kernel(AttnParams p) {
   // ---- 1. head inputs, every one of them requested unconditionally (a missing bias / weight / table
   // reads a stand-in address inside the projection vector and is ignored below)
   const bool q_wave = wave < G, key_wave = wave == (G % W), value_wave = wave == ((G + 1) % W);
-  const uint32_t qoff = (kvh * G + (q_wave ? wave : 0)) * kHD;
-  const uint32_t eoff = (value_wave ? A + KV : A) + kvh * kHD;
+  const uint32_t qoff = (kvh * G + (q_wave ? wave : 0)) * HD;
+  const uint32_t eoff = (value_wave ? A + KV : A) + kvh * HD;
   const uint16_t *stand_in = reinterpret_cast<const uint16_t *>(p.qkv);
   const uint16_t *ebias = value_wave ? p.v_bias : p.k_bias;
-  const float *qp = p.qkv + qoff + lane, *ep = p.qkv + eoff + lane;
-  const uint16_t *qbp = (p.q_bias != nullptr ? p.q_bias + qoff : stand_in) + lane;
-  const uint16_t *ebp = (ebias != nullptr ? ebias + kvh * kHD : stand_in) + lane;
-  const uint16_t *qgp = (p.q_norm != nullptr ? p.q_norm : stand_in) + lane;
-  const uint16_t *kgp = (p.k_norm != nullptr ? p.k_norm : stand_in) + lane;
-  const float *rap = (p.rope_cs != nullptr ? p.rope_cs : (p.rope_freq != nullptr ? p.rope_freq : p.qkv)) + lane;
-  const float *rbp = p.rope_cs != nullptr ? p.rope_cs + 64 + lane : rap;
+  const int pl = pair_of<HD>(lane);
+  const float *qp = p.qkv + qoff + pl, *ep = p.qkv + eoff + pl;
+  const uint16_t *qbp = (p.q_bias != nullptr ? p.q_bias + qoff : stand_in) + pl;
+  const uint16_t *ebp = (ebias != nullptr ? ebias + kvh * HD : stand_in) + pl;
+  const uint16_t *qgp = (p.q_norm != nullptr ? p.q_norm : stand_in) + pl;
+  const uint16_t *kgp = (p.k_norm != nullptr ? p.k_norm : stand_in) + pl;
+  const float *rap = (p.rope_cs != nullptr ? p.rope_cs : (p.rope_freq != nullptr ? p.rope_freq : p.qkv)) + pl;
+  const float *rbp = p.rope_cs != nullptr ? p.rope_cs + HD / 2 + pl : rap;
   float qx0, qx1, ex0, ex1, ra, rb;
   uint32_t qb0, qb1, eb0, eb1, qg0, qg1, kg0, kg1;
   NV_AT_LD32(qx0, qp, 0);
-  NV_AT_LD32(qx1, qp, 256);
+  NV_AT_LD32(qx1, qp, HD * 2);
   NV_AT_LD32(ex0, ep, 0);
-  NV_AT_LD32(ex1, ep, 256);
+  NV_AT_LD32(ex1, ep, HD * 2);
   NV_AT_LD16(qb0, qbp, 0);
-  NV_AT_LD16(qb1, qbp, 128);
+  NV_AT_LD16(qb1, qbp, HD);
   NV_AT_LD16(eb0, ebp, 0);
-  NV_AT_LD16(eb1, ebp, 128);
+  NV_AT_LD16(eb1, ebp, HD);
   NV_AT_LD16(qg0, qgp, 0);
-  NV_AT_LD16(qg1, qgp, 128);
+  NV_AT_LD16(qg1, qgp, HD);
   NV_AT_LD16(kg0, kgp, 0);
-  NV_AT_LD16(kg1, kgp, 128);
+  NV_AT_LD16(kg1, kgp, HD);
   NV_AT_LD32(ra, rap, 0);
   NV_AT_LD32(rb, rbp, 0);
 
@@ -379,7 +386,7 @@ __global__ __launch_bounds__(8 * kWave) void attn_step_kernel(AttnParams p) {
   // started. So: one tile out, the head preparation under its flight, then the rest (the burst takes its
   // 4-5 us either way; what is requested a microsecond later is not served later).
   link_mark(tr, 6);
-  u32x4_t kr[4][4], vr[4][4];
+  u32x4_t kr[4][HD / 32], vr[4][HD / 32];
   if (nt > 0) NV_AT_TILE_LOAD(0, phys[0]);
   link_mark(tr, 8);
 
@@ -394,28 +401,28 @@ __global__ __launch_bounds__(8 * kWave) void attn_step_kernel(AttnParams p) {
   if (has_rope && p.rope_cs == nullptr) sincosf(static_cast<float>(pos) / ra, &rs, &rc);
   if (q_wave) {
     float x0 = qx0, x1 = qx1;
-    head_values<DT>(x0, x1, p.q_bias != nullptr, dec16<DT>(static_cast<uint16_t>(qb0)), dec16<DT>(static_cast<uint16_t>(qb1)),
+    head_values<DT, HD>(x0, x1, p.q_bias != nullptr, dec16<DT>(static_cast<uint16_t>(qb0)), dec16<DT>(static_cast<uint16_t>(qb1)),
                     p.q_norm != nullptr, dec16<DT>(static_cast<uint16_t>(qg0)), dec16<DT>(static_cast<uint16_t>(qg1)),
                     has_rope, rc, rs, p.eps);
     // softmax runs in base 2 on scores scaled by 1/sqrt(d): both folded into the query
-    const float scale = kLog2e / sqrtf(static_cast<float>(kHD));
+    const float scale = kLog2e / sqrtf(static_cast<float>(HD));
     uint16_t h0, l0, h1, l1;
     split16<DT>(x0 * scale, h0, l0);
     split16<DT>(x1 * scale, h1, l1);
-    sh.qhl[wave][lane] = h0;
-    sh.qhl[wave][lane + 64] = h1;
-    sh.qhl[G + wave][lane] = l0;
-    sh.qhl[G + wave][lane + 64] = l1;
+    sh.qhl[wave][pl] = h0;
+    sh.qhl[wave][pl + HD / 2] = h1;
+    sh.qhl[G + wave][pl] = l0;
+    sh.qhl[G + wave][pl + HD / 2] = l1;
   }
   if (owns_new && (key_wave || value_wave)) {
     float x0 = ex0, x1 = ex1;
     const bool norm = key_wave && p.k_norm != nullptr;
-    head_values<DT>(x0, x1, ebias != nullptr, dec16<DT>(static_cast<uint16_t>(eb0)), dec16<DT>(static_cast<uint16_t>(eb1)), norm,
+    head_values<DT, HD>(x0, x1, ebias != nullptr, dec16<DT>(static_cast<uint16_t>(eb0)), dec16<DT>(static_cast<uint16_t>(eb1)), norm,
                     dec16<DT>(static_cast<uint16_t>(kg0)), dec16<DT>(static_cast<uint16_t>(kg1)), key_wave && has_rope, rc, rs,
                     p.eps);
     uint16_t *row = key_wave ? sh.knew : sh.vnew;
-    row[lane] = enc16<DT>(x0);
-    row[lane + 64] = enc16<DT>(x1);
+    row[pl] = enc16<DT>(x0);
+    row[pl + HD / 2] = enc16<DT>(x1);
   }
   // the wave's other tiles of the first four, behind its own head work and before it waits for the others'
   if (nt > 1) NV_AT_TILE_LOAD(1, phys[1]);
@@ -426,22 +433,22 @@ __global__ __launch_bounds__(8 * kWave) void attn_step_kernel(AttnParams p) {
   link_mark(tr, 9);
   if (owns_new && wave == W - 1) {
     // publish the rounded row to the cache in operand order
-    const uint64_t tile = kv_tile_offset(p.block_count, p.kv_heads, kHD, p.layer, sload(p.table + new_block), kvh);
-    if (lane < 16)  // K: 16 pieces of 8 consecutive dims
-      *reinterpret_cast<uint4 *>(p.k_cache + tile + kv_k_elem(kHD, new_row, lane * 8)) =
+    const uint64_t tile = kv_tile_offset(p.block_count, p.kv_heads, HD, p.layer, sload(p.table + new_block), kvh);
+    if (lane < HD / 8)  // K: pieces of 8 consecutive dims
+      *reinterpret_cast<uint4 *>(p.k_cache + tile + kv_k_elem(HD, new_row, lane * 8)) =
           *reinterpret_cast<const uint4 *>(sh.knew + lane * 8);
 #pragma unroll
-    for (int i = 0; i < 2; ++i) {  // V: one 16-bit element per dim
+    for (int i = 0; i < HD / kWave; ++i) {  // V: one 16-bit element per dim
       const uint32_t d = lane + i * kWave;
-      p.v_cache[tile + kv_v_elem(kHD, new_row, d)] = sh.vnew[d];
+      p.v_cache[tile + kv_v_elem(HD, new_row, d)] = sh.vnew[d];
     }
   }
 
   // ---- B operand of the first product: column `col` of Qx for dims j*32 + grp*8 .. +7
   const int col = lane & 15, grp = lane >> 4;
-  uint4 qx[4];
+  uint4 qx[HD / 32];
 #pragma unroll
-  for (int j = 0; j < 4; ++j) {
+  for (int j = 0; j < HD / 32; ++j) {
     const uint4 v = *reinterpret_cast<const uint4 *>(&sh.qhl[col < 2 * G ? col : 0][j * 32 + grp * 8]);
     qx[j] = col < 2 * G ? v : make_uint4(0u, 0u, 0u, 0u);
   }
@@ -449,9 +456,9 @@ __global__ __launch_bounds__(8 * kWave) void attn_step_kernel(AttnParams p) {
 
   // ---- 6. tiles in request order
   float m = -INFINITY, l = 0.0f;  // of column `col` (both copies of a head track the same values)
-  f32x4_t acc[8];                  // O^T[dims s*16 + grp*4 .. +3][col]
+  f32x4_t acc[HD / 16];                  // O^T[dims s*16 + grp*4 .. +3][col]
 #pragma unroll
-  for (int s2 = 0; s2 < 8; ++s2) acc[s2] = f32x4_t{0.0f, 0.0f, 0.0f, 0.0f};
+  for (int s2 = 0; s2 < HD / 16; ++s2) acc[s2] = f32x4_t{0.0f, 0.0f, 0.0f, 0.0f};
 #define NV_AT_STEP(F)                                                                                              \
   do {                                                                                                             \
     const uint32_t t_idx = done + F;                                                                               \
@@ -459,13 +466,13 @@ __global__ __launch_bounds__(8 * kWave) void attn_step_kernel(AttnParams p) {
       /* tiles requested behind this one and not yet consumed: at most three */                                   \
       NV_AT_WAIT_BEHIND(min(nt - t_idx - 1u, 3u));                                                                 \
       NV_AT_TAKE_TILE(F);                                                                                          \
-      uint4 kk[4], vv[4];                                                                                          \
-      _Pragma("unroll") for (int j = 0; j < 4; ++j) {                                                              \
+      uint4 kk[HD / 32], vv[HD / 32];                                                                                          \
+      _Pragma("unroll") for (int j = 0; j < HD / 32; ++j) {                                                              \
         kk[j] = NV_AT_U4(kr[F][j]);                                                                                \
         vv[j] = NV_AT_U4(vr[F][j]);                                                                                \
       }                                                                                                            \
       const uint32_t bb = first + t_idx * W;                                                                       \
-      attn_tile<DT, G, false>(kk, vv, qx, nullptr, bb, n_keys, col, grp, owns_new && bb == new_block, new_row,     \
+      attn_tile<DT, HD, G, false>(kk, vv, qx, nullptr, bb, n_keys, col, grp, owns_new && bb == new_block, new_row,     \
                               sh.knew, sh.vnew, m, l, acc);                                                        \
       if (t_idx + 4u < nt) NV_AT_TILE_LOAD(F, sload(p.table + first + (t_idx + 4u) * W));                          \
     }                                                                                                              \
@@ -483,7 +490,7 @@ __global__ __launch_bounds__(8 * kWave) void attn_step_kernel(AttnParams p) {
   l += __shfl_xor(l, 16, kWave);
   l += __shfl_xor(l, 32, kWave);
 #pragma unroll
-  for (int s2 = 0; s2 < 8; ++s2) {
+  for (int s2 = 0; s2 < HD / 16; ++s2) {
     float4 o;
     o.x = acc[s2][0] + row_shl<G>(acc[s2][0]);
     o.y = acc[s2][1] + row_shl<G>(acc[s2][1]);
@@ -498,8 +505,8 @@ __global__ __launch_bounds__(8 * kWave) void attn_step_kernel(AttnParams p) {
   __syncthreads();
   // every thread owns output elements (g, d): the W waves' scale factors are recomputed per thread
   // (eight exponentials) instead of being shared through another barrier
-  for (int e = threadIdx.x; e < G * kHD; e += kThreads) {
-    const int g = e / kHD, d = e % kHD;
+  for (int e = threadIdx.x; e < G * HD; e += kThreads) {
+    const int g = e / HD, d = e % HD;
     float M = -INFINITY;
 #pragma unroll
     for (int w = 0; w < W; ++w) M = fmaxf(M, sh.wm[w][g]);
@@ -515,13 +522,13 @@ __global__ __launch_bounds__(8 * kWave) void attn_step_kernel(AttnParams p) {
     if (active == 1) {
       // a single split holds every key: this is the final result, nothing to exchange
       if (L > 0.0f && isfinite(L)) o /= L;
-      if (p.out_f32 != nullptr) p.out_f32[h * kHD + d] = o;
-      p.out16[attn_out_elem(p, h * kHD + d)] = enc16<DT>(o);
+      if (p.out_f32 != nullptr) p.out_f32[h * HD + d] = o;
+      p.out16[attn_out_elem(p, h * HD + d)] = enc16<DT>(o);
     } else {
       // The partial leaves as tagged words through device-coherent stores (written through, no cache
       // flush, nobody waits for them to be performed).
       const uint32_t part = d / kStepPartDims, dl = d % kStepPartDims;
-      uint64_t *rec = p.part_tagged + (static_cast<uint64_t>(h) * S + split) * kStepRecord + part * kStepPartWords;
+      uint64_t *rec = p.part_tagged + (static_cast<uint64_t>(h) * S + split) * step_record(HD) + part * kStepPartWords;
       if (p.withhold_split != split + 1u) {
         store_tagged(rec + dl, o, tag);
         if (dl == 0) {
@@ -537,9 +544,9 @@ __global__ __launch_bounds__(8 * kWave) void attn_step_kernel(AttnParams p) {
   // active splits), which polls the other splits' words until every tag is up - two memory round
   // trips after the slowest split's tiles (store, then the poll that finds it), where a ticket taken
   // after the stores have been performed and a merge by the last arriver needed four.
-  for (uint32_t j = split; j < G * kStepParts; j += active) {
+  for (uint32_t j = split; j < G * (HD / kStepPartDims); j += active) {
     link_mark(trm, 16);
-    merge_part_tagged<DT, G>(p, kvh, j % G, j / G, S, active, sh.merge_o[0], sh.merge_m, sh.merge_l, j == split, tag);
+    merge_part_tagged<DT, HD, G>(p, kvh, j % G, j / G, S, active, sh.merge_o[0], sh.merge_m, sh.merge_l, j == split, tag);
     link_mark(trm, 17);
   }
 }
@@ -693,37 +700,50 @@ __global__ __launch_bounds__(kBlock) void attn_generic_kernel(AttnParams p) {
   }
 }
 
+template <uint32_t DT, int HD, int G>
+hipError_t launch_fast(const AttnParams &p, hipStream_t stream) {
+  const dim3 grid(p.kv_heads, p.splits, p.tokens > 1 ? p.tokens : 1);
+  if (p.tokens > 1 || p.seqs != nullptr) {
+    constexpr int W = G == 8 ? kAttnWaves / 2 : kAttnWaves;
+    hipLaunchKernelGGL((attn_block_kernel<DT, HD, G, W>), grid, dim3(W * kWave), 0, stream, p);
+  } else {
+    hipLaunchKernelGGL((attn_step_kernel<DT, HD, G>), grid, dim3(8 * kWave), 0, stream, p);
+  }
+  return hipGetLastError();
+}
+
+template <uint32_t DT, int HD>
+hipError_t launch_fast_hd(const AttnParams &p, hipStream_t stream) {
+  switch (p.heads / p.kv_heads) {
+    case 1: return launch_fast<DT, HD, 1>(p, stream);
+    case 2: return launch_fast<DT, HD, 2>(p, stream);
+    case 3: return launch_fast<DT, HD, 3>(p, stream);
+    case 4: return launch_fast<DT, HD, 4>(p, stream);
+    case 5: return launch_fast<DT, HD, 5>(p, stream);
+    case 6: return launch_fast<DT, HD, 6>(p, stream);
+    case 7: return launch_fast<DT, HD, 7>(p, stream);
+    default: return launch_fast<DT, HD, 8>(p, stream);
+  }
+}
+
 template <uint32_t DT>
 hipError_t launch_dt(const AttnParams &p, hipStream_t stream) {
   const uint32_t group = p.heads / p.kv_heads;
-  const bool fast = p.head_dim == kHD && (group == 1 || group == 2 || group == 4 || group == 8) &&
-                    p.part_acc != nullptr && p.splits >= 1;
-  if (fast) {
-    const dim3 grid(p.kv_heads, p.splits, p.tokens > 1 ? p.tokens : 1);
-    if (p.tokens > 1 || p.seqs != nullptr) {
-      switch (group) {
-        case 1: hipLaunchKernelGGL((attn_block_kernel<DT, 1, kAttnWaves>), grid, dim3(kAttnWaves * kWave), 0, stream, p); break;
-        case 2: hipLaunchKernelGGL((attn_block_kernel<DT, 2, kAttnWaves>), grid, dim3(kAttnWaves * kWave), 0, stream, p); break;
-        case 4: hipLaunchKernelGGL((attn_block_kernel<DT, 4, kAttnWaves>), grid, dim3(kAttnWaves * kWave), 0, stream, p); break;
-        default: hipLaunchKernelGGL((attn_block_kernel<DT, 8, kAttnWaves / 2>), grid, dim3(kAttnWaves / 2 * kWave), 0, stream, p); break;
-      }
-      return hipGetLastError();
-    }
-    if (p.part_tagged == nullptr) return hipErrorInvalidValue;
-    // every active split of a kv head has to be resident while the merges poll: a larger split factor is refused
-    // here, never launched (callers size theirs with attn_default_splits)
-    if (p.splits > 1 && p.splits > attn_resident_splits(p.kv_heads)) return hipErrorInvalidValue;
-    switch (group) {
-      case 1: hipLaunchKernelGGL((attn_step_kernel<DT, 1>), grid, dim3(8 * kWave), 0, stream, p); break;
-      case 2: hipLaunchKernelGGL((attn_step_kernel<DT, 2>), grid, dim3(8 * kWave), 0, stream, p); break;
-      case 4: hipLaunchKernelGGL((attn_step_kernel<DT, 4>), grid, dim3(8 * kWave), 0, stream, p); break;
-      default: hipLaunchKernelGGL((attn_step_kernel<DT, 8>), grid, dim3(8 * kWave), 0, stream, p); break;
-    }
-  } else {
-    if (p.head_dim > 512) return hipErrorInvalidValue;
-    const size_t lds = static_cast<size_t>(3 + kWavesPerBlock) * p.head_dim * sizeof(float);
-    hipLaunchKernelGGL((attn_generic_kernel<DT>), dim3(p.heads), dim3(kBlock), lds, stream, p);
+  const bool block = p.tokens > 1 || p.seqs != nullptr;
+  bool fast = attn_matrix_cores(p.heads, p.kv_heads, p.head_dim) && p.part_acc != nullptr && p.splits >= 1;
+  // every active split of a kv head has to be resident while the merges poll: a larger split factor is refused at the
+  // shapes the split factor is declared for, and left to the general kernel, which has no splits, at the others
+  if (fast && !block && p.splits > 1 && p.splits > attn_resident_splits(p.kv_heads)) {
+    if (p.head_dim == 128 && (group & (group - 1)) == 0) return hipErrorInvalidValue;
+    fast = false;
   }
+  if (fast) {
+    if (!block && p.part_tagged == nullptr) return hipErrorInvalidValue;
+    return p.head_dim == 64 ? launch_fast_hd<DT, 64>(p, stream) : launch_fast_hd<DT, 128>(p, stream);
+  }
+  if (p.head_dim > 512) return hipErrorInvalidValue;
+  const size_t lds = static_cast<size_t>(3 + kWavesPerBlock) * p.head_dim * sizeof(float);
+  hipLaunchKernelGGL((attn_generic_kernel<DT>), dim3(p.heads), dim3(kBlock), lds, stream, p);
   return hipGetLastError();
 }
 
@@ -744,7 +764,7 @@ uint32_t attn_resident_splits(uint32_t kv_heads) {
 }
 
 uint64_t attn_step_workspace_bytes(uint32_t heads) {
-  return static_cast<uint64_t>(heads) * kAttnMaxSplits * kStepRecord * sizeof(uint64_t);
+  return static_cast<uint64_t>(heads) * kAttnMaxSplits * step_record(128) * sizeof(uint64_t);
 }
 
 uint64_t attn_workspace_bytes(uint32_t heads, uint32_t head_dim) {
@@ -765,15 +785,20 @@ void attn_bind_workspace(AttnParams &p, void *workspace) {
 
 hipError_t launch_kv_publish_rows(uint32_t dtype, const AttnParams &p, hipStream_t stream) {
   const bool caches = p.seqs != nullptr || (p.k_cache != nullptr && p.v_cache != nullptr && p.table != nullptr);
-  if (p.qkv == nullptr || !caches || p.tokens == 0 || p.head_dim != static_cast<uint32_t>(kHD) || p.kv_heads == 0)
+  if (p.qkv == nullptr || !caches || p.tokens == 0 || !kv_operand_order(p.head_dim) || p.kv_heads == 0)
     return hipErrorInvalidValue;
   if (p.seqs == nullptr &&
       static_cast<uint64_t>(p.position) + p.tokens > static_cast<uint64_t>(p.block_count) * kKvBlockTokens)
     return hipErrorInvalidValue;
   const dim3 grid(p.kv_heads, p.tokens);
-  if (dtype == kBF16) hipLaunchKernelGGL(kv_publish_rows_kernel<kBF16>, grid, dim3(2 * kWave), 0, stream, p);
-  else if (dtype == kF16) hipLaunchKernelGGL(kv_publish_rows_kernel<kF16>, grid, dim3(2 * kWave), 0, stream, p);
-  else return hipErrorInvalidValue;
+  if (dtype != kBF16 && dtype != kF16) return hipErrorInvalidValue;
+  if (p.head_dim == 64) {
+    if (dtype == kBF16) hipLaunchKernelGGL((kv_publish_rows_kernel<kBF16, 64>), grid, dim3(2 * kWave), 0, stream, p);
+    else hipLaunchKernelGGL((kv_publish_rows_kernel<kF16, 64>), grid, dim3(2 * kWave), 0, stream, p);
+  } else {
+    if (dtype == kBF16) hipLaunchKernelGGL((kv_publish_rows_kernel<kBF16, 128>), grid, dim3(2 * kWave), 0, stream, p);
+    else hipLaunchKernelGGL((kv_publish_rows_kernel<kF16, 128>), grid, dim3(2 * kWave), 0, stream, p);
+  }
   return hipGetLastError();
 }
 
@@ -794,8 +819,7 @@ hipError_t launch_attn_decode(uint32_t dtype, const AttnParams &p, hipStream_t s
     return hipErrorInvalidValue;
   if (p.tokens > 1 || p.seqs != nullptr) {
     // a block of positions or of sequences: host-given positions, matrix-core kernel only
-    const uint32_t group = p.heads / p.kv_heads;
-    const bool fast = p.head_dim == 128 && (group == 1 || group == 2 || group == 4 || group == 8) && p.part_acc != nullptr;
+    const bool fast = attn_matrix_cores(p.heads, p.kv_heads, p.head_dim) && p.part_acc != nullptr;
     // (rows of consecutive positions have to be in the cache before the launch; rows of different
     // sequences can be appended by the launch itself, as the single-token kernel does)
     if (p.cursor != nullptr || (p.append != 0 && p.seqs == nullptr) || !fast || p.tokens == 0 || p.tokens > 65535 ||

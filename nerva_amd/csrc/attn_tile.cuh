@@ -1,4 +1,4 @@
-// Device-side building blocks of the matrix-core decode attention (head_dim 128): head
+// Device-side building blocks of the matrix-core decode attention (head_dim HD = 64 or 128): head
 // preparation (bias, per-head RMSNorm, RoPE), operand helpers, coherent accesses for data
 // exchanged between workgroups of one launch, and the 16-token tile step. Shared by the
 // decode attention kernel (attn_decode.hip) and the prompt-block kernel (attn_prompt.hip).
@@ -9,18 +9,27 @@
 namespace nv {
 namespace attn {
 
-constexpr int kHD = 128;
+constexpr int kHD = 128;        // head_dim of the mixed stacks' kernels
 constexpr int kAttnWaves = 8;   // waves per workgroup of the fast path (group 8 uses half)
 
-// One wave prepares one 128-wide head: lane l owns the RoPE pair (l, l+64).
+// One wave prepares one head: lane l owns the RoPE pair (i, i + HD / 2), i = l % (HD / 2) - at 64 dims both halves of
+// the wave hold the same pairs.
+template <int HD>
+__device__ __forceinline__ int pair_of(int lane) { return lane & (HD / 2 - 1); }
+// Mean square of a head whose pairs the wave holds.
+template <int HD>
+__device__ __forceinline__ float head_mean_square(float x0, float x1) {
+  static_assert(HD == 64 || HD == 128, "pairs of a wave");
+  return wave_sum(x0 * x0 + x1 * x1) / 128.0f;   // (at 64 dims every pair is counted twice)
+}
 // out[] receives f32; when out16 != null the value is rounded first and the 16-bit
 // copy is stored too (K/V that go to the cache).
-// rope_cs (optional): cos at [i], sin at [64 + i] of this step's angles, computed once
+// rope_cs (optional): cos at [i], sin at [HD / 2 + i] of this step's angles, computed once
 // per step; without it the angle pos / rope_freq[i] is evaluated here.
-// (x0, x1) = raw projection values of dims (lane, lane + 64); bias / gamma / rotation of the
+// (x0, x1) = raw projection values of the lane's pair; bias / gamma / rotation of the
 // same two dims, already in registers.
-template <uint32_t DT>
-__device__ __forceinline__ void prep_head128_core(float x0, float x1, bool has_bias, float b0, float b1,
+template <uint32_t DT, int HD>
+__device__ __forceinline__ void prep_head_core(float x0, float x1, bool has_bias, float b0, float b1,
                                                   bool has_gamma, float g0, float g1, bool has_rope, float c,
                                                   float s, float eps, int lane, float *out, uint16_t *out16) {
   if (has_bias) {
@@ -28,8 +37,7 @@ __device__ __forceinline__ void prep_head128_core(float x0, float x1, bool has_b
     x1 += b1;
   }
   if (has_gamma) {
-    const float ss = wave_sum(x0 * x0 + x1 * x1);
-    const float scale = 1.0f / sqrtf(ss / 128.0f + eps);
+    const float scale = 1.0f / sqrtf(head_mean_square<HD>(x0, x1) + eps);
     x0 *= scale * g0;
     x1 *= scale * g1;
   }
@@ -39,19 +47,20 @@ __device__ __forceinline__ void prep_head128_core(float x0, float x1, bool has_b
     x0 = r0;
     x1 = r1;
   }
+  const int at = pair_of<HD>(lane);
   if (out16 != nullptr) {
-    out16[lane] = enc16<DT>(x0);
-    out16[lane + 64] = enc16<DT>(x1);
+    out16[at] = enc16<DT>(x0);
+    out16[at + HD / 2] = enc16<DT>(x1);
     x0 = round16<DT>(x0);
     x1 = round16<DT>(x1);
   }
   if (out != nullptr) {
-    out[lane] = x0;
-    out[lane + 64] = x1;
+    out[at] = x0;
+    out[at + HD / 2] = x1;
   }
 }
-// The same arithmetic on values that stay in registers: (x0, x1) = dims (lane, lane + 64) of one head.
-template <uint32_t DT>
+// The same arithmetic on values that stay in registers: (x0, x1) = the lane's pair of one head.
+template <uint32_t DT, int HD>
 __device__ __forceinline__ void head_values(float &x0, float &x1, bool has_bias, float b0, float b1, bool has_gamma,
                                             float g0, float g1, bool has_rope, float c, float s, float eps) {
   if (has_bias) {
@@ -59,8 +68,7 @@ __device__ __forceinline__ void head_values(float &x0, float &x1, bool has_bias,
     x1 += b1;
   }
   if (has_gamma) {
-    const float ss = wave_sum(x0 * x0 + x1 * x1);
-    const float scale = 1.0f / sqrtf(ss / 128.0f + eps);
+    const float scale = 1.0f / sqrtf(head_mean_square<HD>(x0, x1) + eps);
     x0 *= scale * g0;
     x1 *= scale * g1;
   }
@@ -72,29 +80,30 @@ __device__ __forceinline__ void head_values(float &x0, float &x1, bool has_bias,
   }
 }
 // Same with bias / gamma / rotation fetched here.
-template <uint32_t DT>
-__device__ __forceinline__ void prep_head128(float x0, float x1, const uint16_t *bias,
+template <uint32_t DT, int HD>
+__device__ __forceinline__ void prep_head(float x0, float x1, const uint16_t *bias,
                                              const uint16_t *gamma, const float *rope_freq,
                                              const float *rope_cs, uint32_t pos, float eps, int lane,
                                              float *out, uint16_t *out16) {
+  const int at = pair_of<HD>(lane);
   float b0 = 0.0f, b1 = 0.0f, g0 = 0.0f, g1 = 0.0f, c = 1.0f, s = 0.0f;
   if (bias != nullptr) {
-    b0 = dec16<DT>(bias[lane]);
-    b1 = dec16<DT>(bias[lane + 64]);
+    b0 = dec16<DT>(bias[at]);
+    b1 = dec16<DT>(bias[at + HD / 2]);
   }
   if (gamma != nullptr) {
-    g0 = dec16<DT>(gamma[lane]);
-    g1 = dec16<DT>(gamma[lane + 64]);
+    g0 = dec16<DT>(gamma[at]);
+    g1 = dec16<DT>(gamma[at + HD / 2]);
   }
   if (rope_freq != nullptr) {
     if (rope_cs != nullptr) {
-      c = rope_cs[lane];
-      s = rope_cs[64 + lane];
+      c = rope_cs[at];
+      s = rope_cs[HD / 2 + at];
     } else {
-      sincosf(static_cast<float>(pos) / rope_freq[lane], &s, &c);
+      sincosf(static_cast<float>(pos) / rope_freq[at], &s, &c);
     }
   }
-  prep_head128_core<DT>(x0, x1, bias != nullptr, b0, b1, gamma != nullptr, g0, g1, rope_freq != nullptr, c, s, eps,
+  prep_head_core<DT, HD>(x0, x1, bias != nullptr, b0, b1, gamma != nullptr, g0, g1, rope_freq != nullptr, c, s, eps,
                         lane, out, out16);
 }
 
@@ -173,12 +182,13 @@ __device__ __forceinline__ uint32_t load_coherent(const uint32_t *ptr) {
 // Returns when every store this wave has issued has been performed.
 __device__ __forceinline__ void wait_stores_performed() { asm volatile("s_waitcnt vmcnt(0)" ::: "memory"); }
 
-// Requests one (physical block, kv head) tile: four 1 KiB loads each for K and V.
+// Requests one (physical block, kv head) tile: a 1 KiB load each of K and V for every 32 dims.
+template <int HD>
 __device__ __forceinline__ void attn_load_tile(const AttnParams &p, uint32_t physical_block, uint32_t kvh, int lane,
-                                               uint4 (&k)[4], uint4 (&v)[4]) {
-  const uint64_t tile = kv_tile_offset(p.block_count, p.kv_heads, kHD, p.layer, physical_block, kvh);
+                                               uint4 (&k)[HD / 32], uint4 (&v)[HD / 32]) {
+  const uint64_t tile = kv_tile_offset(p.block_count, p.kv_heads, HD, p.layer, physical_block, kvh);
 #pragma unroll
-  for (int i = 0; i < 4; ++i) {
+  for (int i = 0; i < HD / 32; ++i) {
     k[i] = load_stream(p.k_cache + tile + i * 512 + lane * 8);
     v[i] = load_stream(p.v_cache + tile + i * 512 + lane * 8);
   }
@@ -192,23 +202,23 @@ __device__ __forceinline__ void attn_load_tile(const AttnParams &p, uint32_t phy
 // LAZY_RESCALE = the accumulators are multiplied by alpha only in tiles where some lane's alpha is not 1 (a
 // running maximum that did not move gives exp2(0) = 1 exactly, so the result is the same bits): worth a branch
 // where a wave walks many tiles and the vector ALU is what it waits for (prompt blocks).
-template <uint32_t DT, int G, bool QX_LDS, bool COLUMN_MASKS = false, bool LAZY_RESCALE = false>
-__device__ __forceinline__ void attn_tile(uint4 (&kreg)[4], uint4 (&vreg)[4], const uint4 (&qx)[4],
+template <uint32_t DT, int HD, int G, bool QX_LDS, bool COLUMN_MASKS = false, bool LAZY_RESCALE = false>
+__device__ __forceinline__ void attn_tile(uint4 (&kreg)[HD / 32], uint4 (&vreg)[HD / 32], const uint4 (&qx)[HD / 32],
                                           const uint4 *qx_lds, uint32_t b,
                                           uint32_t n_keys, int col, int grp, bool splice, uint32_t new_row,
                                           const uint16_t *knew, const uint16_t *vnew, float &m, float &l,
-                                          f32x4_t (&acc)[8]) {
+                                          f32x4_t (&acc)[HD / 16]) {
   if (splice) {
     // the row published by this workgroup may not be visible to its own loads yet: take it from LDS
     if (static_cast<uint32_t>(col) == new_row) {  // K operand: lane = (token col, dims grp*8..)
 #pragma unroll
-      for (int j = 0; j < 4; ++j) kreg[j] = *reinterpret_cast<const uint4 *>(knew + j * 32 + grp * 8);
+      for (int j = 0; j < HD / 32; ++j) kreg[j] = *reinterpret_cast<const uint4 *>(knew + j * 32 + grp * 8);
     }
     if (static_cast<uint32_t>(grp) == new_row / 4) {  // V operand: lane = (dim col of a slab, tokens grp*4..)
       const uint32_t e = new_row % 4;
       const uint32_t sh = (e & 1u) * 16u, keep = ~(0xffffu << sh);
 #pragma unroll
-      for (int j = 0; j < 4; ++j) {
+      for (int j = 0; j < HD / 32; ++j) {
         const uint32_t v0 = vnew[(2 * j) * 16 + col], v1 = vnew[(2 * j + 1) * 16 + col];
         if (e < 2) {
           vreg[j].x = (vreg[j].x & keep) | (v0 << sh);
@@ -223,7 +233,7 @@ __device__ __forceinline__ void attn_tile(uint4 (&kreg)[4], uint4 (&vreg)[4], co
   // scores of tokens b*16 + grp*4 + r for column col
   f32x4_t c{0.0f, 0.0f, 0.0f, 0.0f};
 #pragma unroll
-  for (int j = 0; j < 4; ++j) {
+  for (int j = 0; j < HD / 32; ++j) {
     if constexpr (QX_LDS) c = mfma_k32<DT>(kreg[j], qx_lds[j * kWave], c);  // qx_lds: this lane's first operand
     else c = mfma_k32<DT>(kreg[j], qx[j], c);
   }
@@ -260,11 +270,11 @@ __device__ __forceinline__ void attn_tile(uint4 (&kreg)[4], uint4 (&vreg)[4], co
   if constexpr (LAZY_RESCALE) {
     if (__any(alpha != 1.0f)) {
 #pragma unroll
-      for (int s2 = 0; s2 < 8; ++s2) acc[s2] *= alpha;
+      for (int s2 = 0; s2 < HD / 16; ++s2) acc[s2] *= alpha;
     }
   }
 #pragma unroll
-  for (int s2 = 0; s2 < 8; ++s2) {
+  for (int s2 = 0; s2 < HD / 16; ++s2) {
     if constexpr (!LAZY_RESCALE) acc[s2] *= alpha;
     const uint4 &vr = vreg[s2 / 2];
     const uint2 va = (s2 & 1) ? make_uint2(vr.z, vr.w) : make_uint2(vr.x, vr.y);
@@ -279,16 +289,16 @@ __device__ __forceinline__ void attn_tile(uint4 (&kreg)[4], uint4 (&vreg)[4], co
 // its own instead of being done twice, and a K/V tile read from LDS meets twice as many pairs. Columns are masked
 // individually (n_keys by column; a column may find a whole tile masked) and the accumulators are rescaled only
 // in tiles where some running maximum moved.
-template <uint32_t DT>
-__device__ __forceinline__ void attn_tile_wide(const uint4 (&kreg)[4], const uint4 (&vreg)[4], const uint4 (&qhi)[4],
-                                               const uint4 (&qlo)[4], uint32_t b, uint32_t n_keys, int grp, float &m,
-                                               float &l, f32x4_t (&acc)[8]) {
+template <uint32_t DT, int HD>
+__device__ __forceinline__ void attn_tile_wide(const uint4 (&kreg)[HD / 32], const uint4 (&vreg)[HD / 32], const uint4 (&qhi)[HD / 32],
+                                               const uint4 (&qlo)[HD / 32], uint32_t b, uint32_t n_keys, int grp, float &m,
+                                               float &l, f32x4_t (&acc)[HD / 16]) {
   // scores of tokens b*16 + grp*4 + r for this lane's column
   f32x4_t c{0.0f, 0.0f, 0.0f, 0.0f};
 #pragma unroll
-  for (int j = 0; j < 4; ++j) c = mfma_k32<DT>(kreg[j], qhi[j], c);
+  for (int j = 0; j < HD / 32; ++j) c = mfma_k32<DT>(kreg[j], qhi[j], c);
 #pragma unroll
-  for (int j = 0; j < 4; ++j) c = mfma_k32<DT>(kreg[j], qlo[j], c);
+  for (int j = 0; j < HD / 32; ++j) c = mfma_k32<DT>(kreg[j], qlo[j], c);
   float sc[4];
 #pragma unroll
   for (int r = 0; r < 4; ++r) sc[r] = b * kKvBlockTokens + grp * 4 + r < n_keys ? c[r] : -INFINITY;
@@ -315,10 +325,10 @@ __device__ __forceinline__ void attn_tile_wide(const uint4 (&kreg)[4], const uin
   const uint2 pbh = make_uint2(ph[0], ph[1]), pbl = make_uint2(pl[0], pl[1]);
   if (__any(alpha != 1.0f)) {
 #pragma unroll
-    for (int s2 = 0; s2 < 8; ++s2) acc[s2] *= alpha;
+    for (int s2 = 0; s2 < HD / 16; ++s2) acc[s2] *= alpha;
   }
 #pragma unroll
-  for (int s2 = 0; s2 < 8; ++s2) {
+  for (int s2 = 0; s2 < HD / 16; ++s2) {
     const uint4 &vr = vreg[s2 / 2];
     const uint2 va = (s2 & 1) ? make_uint2(vr.z, vr.w) : make_uint2(vr.x, vr.y);
     acc[s2] = mfma_k16<DT>(va, pbh, acc[s2]);
@@ -326,18 +336,18 @@ __device__ __forceinline__ void attn_tile_wide(const uint4 (&kreg)[4], const uin
   }
 }
 
-template <int G, int W>
+template <int HD, int G, int W>
 struct AttnShared {
-  alignas(16) float q_s[G][kHD];
-  alignas(16) uint16_t knew[kHD];
-  alignas(16) uint16_t vnew[kHD];
+  alignas(16) float q_s[G][HD];
+  alignas(16) uint16_t knew[HD];
+  alignas(16) uint16_t vnew[HD];
   float wm[W][G];
   float wl[W][G];
-  alignas(16) float wacc[W][G][kHD];
+  alignas(16) float wacc[W][G][HD];
   float wf[W][G];   // exp(m_w - M_g), 0 for idle waves
   float bM[G];
   uint32_t is_last;
-  alignas(16) uint4 qx_s[4][kWave];  // lean variant: the query operand of the first product
+  alignas(16) uint4 qx_s[HD / 32][kWave];  // lean variant: the query operand of the first product
 };
 
 // ---- hand-over between workgroups of one launch ------------------------------------------
@@ -378,20 +388,20 @@ struct RawHeads {
   uint16_t qg0, qg1, kg0, kg1;   // q_norm / k_norm weight bits
   float rope_a, rope_b;          // cos, sin of this step; without a table: the frequency of the pair
 };
-template <int G, int W>
+template <int HD, int G, int W>
 __device__ __forceinline__ RawHeads<G, W> attn_request_raw(const AttnParams &p, uint32_t kvh) {
-  const int lane = threadIdx.x & (kWave - 1);
+  const int at = pair_of<HD>(threadIdx.x & (kWave - 1));
   const int wave = threadIdx.x / kWave;
-  const uint32_t A = p.heads * kHD, KV = p.kv_heads * kHD;
+  const uint32_t A = p.heads * HD, KV = p.kv_heads * HD;
   RawHeads<G, W> r{};
   // one value, or the sum of its K-slice partials in slice order (all requested at once; a slice that does not
   // exist reads slice 0 again and is left out of the sum)
   const uint32_t slices = p.qkv_slices;
-  auto raw_value = [&](uint32_t at) {
-    if (slices <= 1) return p.qkv[at];
+  auto raw_value = [&](uint32_t i) {
+    if (slices <= 1) return p.qkv[i];
     float part[4];
 #pragma unroll
-    for (uint32_t s = 0; s < 4; ++s) part[s] = p.qkv[at + (s < slices ? s : 0u) * static_cast<uint64_t>(p.qkv_slice_stride)];
+    for (uint32_t s = 0; s < 4; ++s) part[s] = p.qkv[i + (s < slices ? s : 0u) * static_cast<uint64_t>(p.qkv_slice_stride)];
     float sum = 0.0f;
 #pragma unroll
     for (uint32_t s = 0; s < 4; ++s) sum = s < slices ? sum + part[s] : sum;
@@ -399,100 +409,43 @@ __device__ __forceinline__ RawHeads<G, W> attn_request_raw(const AttnParams &p, 
   };
 #pragma unroll
   for (int i = 0; i < (G + W - 1) / W; ++i) {
-    const uint32_t off = (kvh * G + min(wave + i * W, G - 1)) * kHD;  // clamped: the loads are unconditional
-    r.q[i].x0 = raw_value(off + lane);
-    r.q[i].x1 = raw_value(off + lane + 64);
+    const uint32_t off = (kvh * G + min(wave + i * W, G - 1)) * HD;  // clamped: the loads are unconditional
+    r.q[i].x0 = raw_value(off + at);
+    r.q[i].x1 = raw_value(off + at + HD / 2);
     if (p.q_bias != nullptr) {
-      r.q[i].b0 = p.q_bias[off + lane];
-      r.q[i].b1 = p.q_bias[off + lane + 64];
+      r.q[i].b0 = p.q_bias[off + at];
+      r.q[i].b1 = p.q_bias[off + at + HD / 2];
     }
   }
   const bool value_wave = wave == ((G + 1) % W);
-  const uint32_t off = (value_wave ? A + KV : A) + kvh * kHD;
-  r.e.x0 = raw_value(off + lane);
-  r.e.x1 = raw_value(off + lane + 64);
+  const uint32_t off = (value_wave ? A + KV : A) + kvh * HD;
+  r.e.x0 = raw_value(off + at);
+  r.e.x1 = raw_value(off + at + HD / 2);
   const uint16_t *eb = value_wave ? p.v_bias : p.k_bias;
   if (eb != nullptr) {
-    r.e.b0 = eb[kvh * kHD + lane];
-    r.e.b1 = eb[kvh * kHD + lane + 64];
+    r.e.b0 = eb[kvh * HD + at];
+    r.e.b1 = eb[kvh * HD + at + HD / 2];
   }
   if (p.q_norm != nullptr) {
-    r.qg0 = p.q_norm[lane];
-    r.qg1 = p.q_norm[lane + 64];
+    r.qg0 = p.q_norm[at];
+    r.qg1 = p.q_norm[at + HD / 2];
   }
   if (p.k_norm != nullptr) {
-    r.kg0 = p.k_norm[lane];
-    r.kg1 = p.k_norm[lane + 64];
+    r.kg0 = p.k_norm[at];
+    r.kg1 = p.k_norm[at + HD / 2];
   }
   if (p.rope_freq != nullptr) {
     if (p.rope_cs != nullptr) {
-      r.rope_a = p.rope_cs[lane];
-      r.rope_b = p.rope_cs[64 + lane];
+      r.rope_a = p.rope_cs[at];
+      r.rope_b = p.rope_cs[HD / 2 + at];
     } else {
-      r.rope_a = p.rope_freq[lane];
+      r.rope_a = p.rope_freq[at];
     }
   }
   return r;
 }
 
 constexpr int kTicketRound = 32;           // splits read per round by the last workgroup of the ticket protocol
-// The last workgroup of a kv head merges the splits' partials. Each thread owns output elements (g, d)
-// and reads the partials with device-coherent loads, kTicketRound splits per round trip, in split
-// order, so the result does not depend on which workgroup arrived last.
-template <uint32_t DT, int G, int THREADS>
-__device__ __forceinline__ void merge_splits(const AttnParams &p, uint32_t kvh, uint32_t S, uint32_t active, int lane) {
-  for (int e = threadIdx.x; e < G * kHD; e += THREADS) {
-    const int g = e / kHD, d = e % kHD;
-    const uint32_t h = kvh * G + g;
-    const float *pm = p.part_m + h * S, *pl = p.part_l + h * S;
-    const float *src = p.part_acc + static_cast<uint64_t>(h) * S * kHD + d;
-    float M = -INFINITY, L = 0.0f, o = 0.0f;
-    for (uint32_t s0 = 0; s0 < active; s0 += kTicketRound) {
-      float mm[kTicketRound], ll[kTicketRound], aa[kTicketRound];
-      // m and l of this head's splits: the head is the same for all lanes of a wave, so lane i fetches
-      // m of split s0 + i and lane kTicketRound + i its l (one load a lane instead of two per split),
-      // and the values are handed round with lane reads below.
-      static_assert(2 * kTicketRound == kWave && kHD % kWave == 0, "one (m, l) pair per lane pair, one head per wave");
-      const uint32_t si_ml = min(s0 + static_cast<uint32_t>(lane & (kTicketRound - 1)), active - 1);
-      const float ml = load_coherent((lane < kTicketRound ? pm : pl) + si_ml);
-#pragma unroll
-      for (int i = 0; i < kTicketRound; ++i) {
-        // unconditional loads (index clamped): a load under a branch would serialise the round
-        const uint32_t si = min(s0 + i, active - 1);
-        aa[i] = load_coherent(src + static_cast<uint64_t>(si) * kHD);
-      }
-#pragma unroll
-      for (int i = 0; i < kTicketRound; ++i) {
-        mm[i] = __uint_as_float(__builtin_amdgcn_readlane(__float_as_uint(ml), i));
-        ll[i] = __uint_as_float(__builtin_amdgcn_readlane(__float_as_uint(ml), kTicketRound + i));
-      }
-#pragma unroll
-      for (int i = 0; i < kTicketRound; ++i) {
-        const bool on = s0 + i < active;
-        mm[i] = on ? mm[i] : -INFINITY;
-        ll[i] = on ? ll[i] : 0.0f;
-        aa[i] = on ? aa[i] : 0.0f;
-      }
-      float Mc = M;
-#pragma unroll
-      for (int i = 0; i < kTicketRound; ++i) Mc = fmaxf(Mc, mm[i]);
-      const float keep = M > -INFINITY ? attn_exp2(M - Mc) : 0.0f;
-      L *= keep;
-      o *= keep;
-#pragma unroll
-      for (int i = 0; i < kTicketRound; ++i) {
-        const float f = mm[i] > -INFINITY ? attn_exp2(mm[i] - Mc) : 0.0f;
-        L = fmaf(ll[i], f, L);
-        o = fmaf(aa[i], f, o);
-      }
-      M = Mc;
-    }
-    if (L > 0.0f && isfinite(L)) o /= L;
-    if (p.out_f32 != nullptr) p.out_f32[h * kHD + d] = o;
-    p.out16[attn_out_elem(p, h * kHD + d)] = enc16<DT>(o);
-  }
-}
-
 // W waves per workgroup. A workgroup owns one kv head and one contiguous range of
 // 16-token tiles; wave w takes tiles b0+w, b0+w+W, ...  Both products of a tile run on
 // the matrix cores:
@@ -505,9 +458,9 @@ __device__ __forceinline__ void merge_splits(const AttnParams &p, uint32_t kvh, 
 // accumulators are indexed by the same column, so m, l and the rescale never cross lanes.
 // The cache stores tiles in operand order (kv_k_elem / kv_v_elem): every load is one coalesced
 // 1 KiB instruction and lands in the registers the matrix core reads.
-template <uint32_t DT, int G, int W, int IN_FLIGHT = 4>
+template <uint32_t DT, int HD, int G, int W, int IN_FLIGHT = 4>
 __device__ __forceinline__ void attn_fast_body(const AttnParams &p, const uint32_t pos, const uint32_t kvh,
-                                               const uint32_t split, const uint32_t S, AttnShared<G, W> &sh,
+                                               const uint32_t split, const uint32_t S, AttnShared<HD, G, W> &sh,
                                                const RawHeads<G, W> &raw) {
   constexpr int kThreads = W * kWave;
   auto &q_s = sh.q_s;
@@ -533,7 +486,6 @@ __device__ __forceinline__ void attn_fast_body(const AttnParams &p, const uint32
   if (split >= active) return;  // idle splits neither store a partial nor take a ticket
   const uint32_t b0 = split * bps;
   const uint32_t b1 = min(nblk, b0 + bps);
-  const uint32_t A = p.heads * kHD, KV = p.kv_heads * kHD;
   const uint32_t new_block = pos / kKvBlockTokens, new_row = pos % kKvBlockTokens;
   const bool owns_new = p.append != 0 && new_block >= b0 && new_block < b1;
 
@@ -545,7 +497,7 @@ __device__ __forceinline__ void attn_fast_body(const AttnParams &p, const uint32
   // CU can run at a time.
   constexpr int kInFlight = IN_FLIGHT;
   constexpr bool kLean = IN_FLIGHT == 1;  // 128-register budget: the query operand is parked in LDS
-  uint4 kreg[kInFlight][4], vreg[kInFlight][4];
+  uint4 kreg[kInFlight][HD / 32], vreg[kInFlight][HD / 32];
   uint32_t b = b0 + wave;
   // the block-table entries first, all of them, so that no tile request waits behind another tile's data
   uint32_t phys[kInFlight];
@@ -555,7 +507,7 @@ __device__ __forceinline__ void attn_fast_body(const AttnParams &p, const uint32
   asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
 #pragma unroll
   for (int f = 0; f < kInFlight; ++f)
-    if (b + f * W < b1) attn_load_tile(p, phys[f], kvh, lane, kreg[f], vreg[f]);
+    if (b + f * W < b1) attn_load_tile<HD>(p, phys[f], kvh, lane, kreg[f], vreg[f]);
 
   link_mark(tr, 8);
   // ---- q (all workgroups) and the new K/V row (the workgroup whose range holds pos)
@@ -568,17 +520,17 @@ __device__ __forceinline__ void attn_fast_body(const AttnParams &p, const uint32
     for (int i = 0; i < (G + W - 1) / W; ++i) {
       const int g = wave + i * W;
       if (g < G)
-        prep_head128_core<DT>(raw.q[i].x0, raw.q[i].x1, p.q_bias != nullptr, dec16<DT>(raw.q[i].b0),
+        prep_head_core<DT, HD>(raw.q[i].x0, raw.q[i].x1, p.q_bias != nullptr, dec16<DT>(raw.q[i].b0),
                               dec16<DT>(raw.q[i].b1), p.q_norm != nullptr, dec16<DT>(raw.qg0), dec16<DT>(raw.qg1),
                               has_rope, rc, rs, p.eps, lane, q_s[g], nullptr);
     }
     if (owns_new) {
       if (wave == (G % W)) {
-        prep_head128_core<DT>(raw.e.x0, raw.e.x1, p.k_bias != nullptr, dec16<DT>(raw.e.b0), dec16<DT>(raw.e.b1),
+        prep_head_core<DT, HD>(raw.e.x0, raw.e.x1, p.k_bias != nullptr, dec16<DT>(raw.e.b0), dec16<DT>(raw.e.b1),
                               p.k_norm != nullptr, dec16<DT>(raw.kg0), dec16<DT>(raw.kg1), has_rope, rc, rs, p.eps,
                               lane, nullptr, knew);
       } else if (wave == ((G + 1) % W)) {
-        prep_head128_core<DT>(raw.e.x0, raw.e.x1, p.v_bias != nullptr, dec16<DT>(raw.e.b0), dec16<DT>(raw.e.b1), false,
+        prep_head_core<DT, HD>(raw.e.x0, raw.e.x1, p.v_bias != nullptr, dec16<DT>(raw.e.b0), dec16<DT>(raw.e.b1), false,
                               0.0f, 0.0f, false, 1.0f, 0.0f, p.eps, lane, nullptr, vnew);
       }
     }
@@ -587,25 +539,25 @@ __device__ __forceinline__ void attn_fast_body(const AttnParams &p, const uint32
   link_mark(tr, 9);
   if (owns_new && wave == 0) {
     // publish the rounded row to the cache in operand order
-    const uint64_t tile = kv_tile_offset(p.block_count, p.kv_heads, kHD, p.layer, p.table[new_block], kvh);
-    if (lane < 16) {  // K: 16 pieces of 8 consecutive dims
-      *reinterpret_cast<uint4 *>(p.k_cache + tile + kv_k_elem(kHD, new_row, lane * 8)) =
+    const uint64_t tile = kv_tile_offset(p.block_count, p.kv_heads, HD, p.layer, p.table[new_block], kvh);
+    if (lane < HD / 8) {  // K: pieces of 8 consecutive dims
+      *reinterpret_cast<uint4 *>(p.k_cache + tile + kv_k_elem(HD, new_row, lane * 8)) =
           *reinterpret_cast<const uint4 *>(knew + lane * 8);
     }
 #pragma unroll
-    for (int i = 0; i < 2; ++i) {  // V: one 16-bit element per dim
+    for (int i = 0; i < HD / kWave; ++i) {  // V: one 16-bit element per dim
       const uint32_t d = lane + i * kWave;
-      p.v_cache[tile + kv_v_elem(kHD, new_row, d)] = vnew[d];
+      p.v_cache[tile + kv_v_elem(HD, new_row, d)] = vnew[d];
     }
   }
 
   const int col = lane & 15, grp = lane >> 4;
-  const float scale = kLog2e / sqrtf(static_cast<float>(kHD));
+  const float scale = kLog2e / sqrtf(static_cast<float>(HD));
 
   // B operand of the first product: column `col` of Qx for dims j*32 + grp*8 .. +7
-  uint4 qx[4];
+  uint4 qx[HD / 32];
 #pragma unroll
-  for (int j = 0; j < 4; ++j) {
+  for (int j = 0; j < HD / 32; ++j) {
     uint32_t w[4] = {0u, 0u, 0u, 0u};
     if (col < 2 * G) {
       const float *src = &q_s[col < G ? col : col - G][j * 32 + grp * 8];
@@ -624,24 +576,24 @@ __device__ __forceinline__ void attn_fast_body(const AttnParams &p, const uint32
   const uint4 *qx_lds = nullptr;
   if constexpr (kLean) {
 #pragma unroll
-    for (int j = 0; j < 4; ++j) sh.qx_s[j][lane] = qx[j];
+    for (int j = 0; j < HD / 32; ++j) sh.qx_s[j][lane] = qx[j];
     qx_lds = &sh.qx_s[0][lane];
   }
 
   link_mark(tr, 10);
   float m = -INFINITY, l = 0.0f;  // of column `col` (both copies of a head track the same values)
-  f32x4_t acc[8];                  // O^T[dims s*16 + grp*4 .. +3][col]
+  f32x4_t acc[HD / 16];                  // O^T[dims s*16 + grp*4 .. +3][col]
 #pragma unroll
-  for (int s2 = 0; s2 < 8; ++s2) acc[s2] = f32x4_t{0.0f, 0.0f, 0.0f, 0.0f};
+  for (int s2 = 0; s2 < HD / 16; ++s2) acc[s2] = f32x4_t{0.0f, 0.0f, 0.0f, 0.0f};
 
   for (; b < b1; b += kInFlight * W) {
 #pragma unroll
     for (int f = 0; f < kInFlight; ++f) {
       const uint32_t bb = b + f * W;
       if (bb < b1) {
-        attn_tile<DT, G, kLean>(kreg[f], vreg[f], qx, qx_lds, bb, n_keys, col, grp, owns_new && bb == new_block, new_row,
+        attn_tile<DT, HD, G, kLean>(kreg[f], vreg[f], qx, qx_lds, bb, n_keys, col, grp, owns_new && bb == new_block, new_row,
                                  knew, vnew, m, l, acc);
-        if (bb + kInFlight * W < b1) attn_load_tile(p, p.table[bb + kInFlight * W], kvh, lane, kreg[f], vreg[f]);
+        if (bb + kInFlight * W < b1) attn_load_tile<HD>(p, p.table[bb + kInFlight * W], kvh, lane, kreg[f], vreg[f]);
       }
     }
   }
@@ -651,7 +603,7 @@ __device__ __forceinline__ void attn_fast_body(const AttnParams &p, const uint32
   l += __shfl_xor(l, 16, kWave);
   l += __shfl_xor(l, 32, kWave);
 #pragma unroll
-  for (int s2 = 0; s2 < 8; ++s2) {
+  for (int s2 = 0; s2 < HD / 16; ++s2) {
     float4 o;
     o.x = acc[s2][0] + row_shl<G>(acc[s2][0]);
     o.y = acc[s2][1] + row_shl<G>(acc[s2][1]);
@@ -674,8 +626,8 @@ __device__ __forceinline__ void attn_fast_body(const AttnParams &p, const uint32
     if (w == 0) bM[g] = M;
   }
   __syncthreads();
-  for (int e = threadIdx.x; e < G * kHD; e += kThreads) {
-    const int g = e / kHD, d = e % kHD;
+  for (int e = threadIdx.x; e < G * HD; e += kThreads) {
+    const int g = e / HD, d = e % HD;
     float L = 0.0f, o = 0.0f;
 #pragma unroll
     for (int w = 0; w < W; ++w) {
@@ -686,12 +638,12 @@ __device__ __forceinline__ void attn_fast_body(const AttnParams &p, const uint32
     if (active == 1) {
       // a single split holds every key: this is the final result, nothing to exchange
       if (L > 0.0f && isfinite(L)) o /= L;
-      if (p.out_f32 != nullptr) p.out_f32[h * kHD + d] = o;
+      if (p.out_f32 != nullptr) p.out_f32[h * HD + d] = o;
       const uint16_t o16 = enc16<DT>(o);
-      p.out16[attn_out_elem(p, h * kHD + d)] = o16;
+      p.out16[attn_out_elem(p, h * HD + d)] = o16;
     } else {
       // The partial leaves through device-coherent stores (written through, no cache flush).
-      store_coherent(p.part_acc + (static_cast<uint64_t>(h) * S + split) * kHD + d, o);
+      store_coherent(p.part_acc + (static_cast<uint64_t>(h) * S + split) * HD + d, o);
       if (d == 0) {
         store_coherent(p.part_m + h * S + split, bM[g]);
         store_coherent(p.part_l + h * S + split, L);
@@ -715,25 +667,25 @@ __device__ __forceinline__ void attn_fast_body(const AttnParams &p, const uint32
   link_mark(trm, 16);
   // ---- the last workgroup of this kv head merges the splits. Each thread owns (g, d) and reads
   // the partials with device-coherent loads, kTicketRound splits per round trip, in split order.
-  for (int e = threadIdx.x; e < G * kHD; e += kThreads) {
-    const int g = e / kHD, d = e % kHD;
+  for (int e = threadIdx.x; e < G * HD; e += kThreads) {
+    const int g = e / HD, d = e % HD;
     const uint32_t h = kvh * G + g;
     const float *pm = p.part_m + h * S, *pl = p.part_l + h * S;
-    const float *src = p.part_acc + static_cast<uint64_t>(h) * S * kHD + d;
+    const float *src = p.part_acc + static_cast<uint64_t>(h) * S * HD + d;
     float M = -INFINITY, L = 0.0f, o = 0.0f;
     for (uint32_t s0 = 0; s0 < active; s0 += kTicketRound) {
       float mm[kTicketRound], ll[kTicketRound], aa[kTicketRound];
       // m and l of this head's splits: the head is the same for all lanes of a wave, so lane i fetches
       // m of split s0 + i and lane kTicketRound + i its l (one load a lane instead of two per split),
       // and the values are handed round with lane reads below.
-      static_assert(2 * kTicketRound == kWave && kHD % kWave == 0, "one (m, l) pair per lane pair, one head per wave");
+      static_assert(2 * kTicketRound == kWave && HD % kWave == 0, "one (m, l) pair per lane pair, one head per wave");
       const uint32_t si_ml = min(s0 + static_cast<uint32_t>(lane & (kTicketRound - 1)), active - 1);
       const float ml = load_coherent((lane < kTicketRound ? pm : pl) + si_ml);
 #pragma unroll
       for (int i = 0; i < kTicketRound; ++i) {
         // unconditional loads (index clamped): a load under a branch would serialise the round
         const uint32_t si = min(s0 + i, active - 1);
-        aa[i] = load_coherent(src + static_cast<uint64_t>(si) * kHD);
+        aa[i] = load_coherent(src + static_cast<uint64_t>(si) * HD);
       }
 #pragma unroll
       for (int i = 0; i < kTicketRound; ++i) {
@@ -762,8 +714,8 @@ __device__ __forceinline__ void attn_fast_body(const AttnParams &p, const uint32
       M = Mc;
     }
     if (L > 0.0f && isfinite(L)) o /= L;
-    if (p.out_f32 != nullptr) p.out_f32[h * kHD + d] = o;
-    p.out16[attn_out_elem(p, h * kHD + d)] = enc16<DT>(o);
+    if (p.out_f32 != nullptr) p.out_f32[h * HD + d] = o;
+    p.out16[attn_out_elem(p, h * HD + d)] = enc16<DT>(o);
   }
   if (threadIdx.x == 0) __hip_atomic_store(p.counters + kvh, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
   link_mark(trm, 17);

@@ -617,11 +617,12 @@ hipError_t reset_sequence(Session *s, const uint32_t *prompt_tokens, uint32_t pr
 // block through LDS. Batch steps of Qwen3-8B shape, [token][column] rows with every wave fetching its own
 // X pieces against operand order: 2 sequences 3.68 vs 3.50 ms, 8: 4.03 vs 3.62, 16: 4.70 vs 3.88 (operand
 // order through the kernel without the shared block: 4.28, 4.43, 4.78).
+// A single row comes as a row where the projections have a kernel for that (rows_plain).
 // The "block_layout" override forces one layout (1 = rows, 2 = operand order; comparisons).
-uint32_t block_operand_tiles(uint32_t tokens) {
+uint32_t block_operand_tiles(const Session *s, uint32_t tokens) {
   const int forced = tuning(kTuneBlockLayout);
   const bool operand = forced == 1 || forced == 2 ? forced == 2 : tokens > 1;
-  return operand ? gemm_packed_tiles(tokens) : 0u;
+  return operand || !s->rows_plain ? gemm_packed_tiles(tokens) : 0u;
 }
 
 // Prompt tokens begin .. count-1 through every layer in blocks of up to prefill_block_tokens tokens, with the
@@ -644,7 +645,7 @@ hipError_t prefill_blocks(Session *s, uint32_t begin, uint32_t count, uint32_t p
                                      : 0u;
   for (uint32_t first = begin; err == hipSuccess && first < count; first += s->prefill_block_tokens) {
     const uint32_t T = std::min<uint32_t>(s->prefill_block_tokens, count - first);
-    const uint32_t tiles = block_operand_tiles(T);
+    const uint32_t tiles = block_operand_tiles(s, T);
     if (s->dtype == kBF16)
       hipLaunchKernelGGL(embed_rows_kernel<kBF16>, dim3(T), dim3(kBlock), 0, st, s->emb, s->prompt, first, H, s->vocab,
                          s->px, rope_freq, s->prope, s->head_dim / 2);
@@ -894,16 +895,20 @@ hipError_t setup_state(Session *s, int32_t *failure_stage, bool with_weights) {
   const uint64_t off_sampler_keys = c.take(sampler_workspace_bytes(s->vocab));
   const uint64_t off_attn_trace = c.take(L * 32 * 8);
   {
-    // Prompt blocks and batch steps need the matrix-core attention (head_dim 128, GQA factor
-    // 1/2/4/8) and shapes the multi-row kernels take.
-    const uint32_t group = s->heads / s->kv_heads;
-    s->rows_ready = s->head_dim == 128 && (group == 1 || group == 2 || group == 4 || group == 8) && s->hidden <= 16384 &&
-                    gemm_rows_supported(static_cast<uint32_t>(A + 2 * KV), s->hidden, 1) &&
-                    gemm_rows_supported(s->hidden, static_cast<uint32_t>(A), 1) &&
-                    gemm_rows_supported(s->intermediate, s->hidden, 1) &&
-                    gemm_rows_supported(s->hidden, s->intermediate, 1);
+    // Prompt blocks and batch steps need the matrix-core attention and widths that matrix-operand order can hold; with
+    // those every projection has a multi-row kernel, some of them for rows as they come as well (rows_plain).
+    const uint32_t qkv = static_cast<uint32_t>(A + 2 * KV), attn = static_cast<uint32_t>(A);
+    s->rows_plain = gemm_rows_supported(qkv, s->hidden, 1) && gemm_rows_supported(s->hidden, attn, 1) &&
+                    gemm_rows_supported(s->intermediate, s->hidden, 1) && gemm_rows_supported(s->hidden, s->intermediate, 1);
+    s->rows_ready = attn_matrix_cores(s->heads, s->kv_heads, s->head_dim) && s->hidden <= 16384 && s->hidden % 32 == 0 &&
+                    s->intermediate % 32 == 0 && gemm_rows_takes(kGemmF32, qkv, s->hidden, kGemmMaxTokens, 0) &&
+                    gemm_rows_takes(kGemmResidual, s->hidden, attn, kGemmMaxTokens, 0) &&
+                    gemm_rows_takes(kGemmSwiglu, s->intermediate, s->hidden, kGemmMaxTokens, 0) &&
+                    gemm_rows_takes(kGemmResidual, s->hidden, s->intermediate, kGemmMaxTokens, 0);
   }
-  const bool batch_head = s->rows_ready && gemm_rows_supported(s->vocab, s->hidden, 1);
+  // (a batch of sequences of a model with less than 6 MiB of weights a layer runs the sequences' own steps)
+  const bool batch_head = s->rows_ready && (A + KV) * H * 2 + 3 * H * I >= (3u << 20) &&
+                          gemm_rows_takes(kGemmF32, s->vocab, s->hidden, NERVA_HIP_BATCH_MAX_BLOCK_TOKENS, 0);
   const uint64_t off_blogits = batch_head ? c.take(static_cast<uint64_t>(NERVA_HIP_BATCH_MAX_BLOCK_TOKENS) * V * 4) : 0;
   const uint64_t off_btable = c.take(sizeof(BatchTable));
   const uint64_t off_bslots = c.take(static_cast<uint64_t>(NERVA_HIP_BATCH_MAX_BLOCK_TOKENS) * sizeof(Slot));
@@ -929,12 +934,8 @@ hipError_t setup_state(Session *s, int32_t *failure_stage, bool with_weights) {
   s->rope_cs = reinterpret_cast<float *>(s->arena + off_rope_cs);
   s->attn_ws = s->arena + off_attn_ws;
   s->attn_tagged = reinterpret_cast<uint64_t *>(s->arena + off_attn_tagged);
-  {
-    // the plan serves the step kernel (head_dim 128, 1, 2, 4 or 8 query heads per kv head, 8 waves)
-    const uint32_t group = s->kv_heads != 0 ? s->heads / s->kv_heads : 0;
-    if (s->head_dim == 128 && (group == 1 || group == 2 || group == 4 || group == 8))
-      s->attn_plan = reinterpret_cast<uint32_t *>(s->arena + off_attn_plan);
-  }
+  if (attn_matrix_cores(s->heads, s->kv_heads, s->head_dim))   // the plan serves the step kernel
+    s->attn_plan = reinterpret_cast<uint32_t *>(s->arena + off_attn_plan);
   s->sample_ws = s->arena + off_sample_ws;
   s->px = reinterpret_cast<float *>(s->arena + off_px);
   s->pr = reinterpret_cast<float *>(s->arena + off_pr);
@@ -949,19 +950,18 @@ hipError_t setup_state(Session *s, int32_t *failure_stage, bool with_weights) {
   s->pgemm_ws_bytes = pgemm_ws_bytes;
   // Prompt blocks of 512 tokens where all four projections of a layer have the kernel for them (256 weight rows x
   // 256 tokens a workgroup: half the X bytes per product of the 256-token kernel), else of 256 tokens where they
-  // have that kernel (twice the tokens per weight byte of the 128-token one): Qwen3-8B widths qualify for both;
-  // other widths keep 128-token blocks. The "prefill_block_tokens" override caps the choice at 128 or 256.
-  const auto all_four = [&](uint32_t (*slices)(int, uint32_t, uint32_t, uint32_t, uint64_t), uint32_t tokens) {
-    return slices(kGemmF32, static_cast<uint32_t>(A + 2 * KV), s->hidden, tokens, pgemm_ws_bytes) != 0 &&
-           slices(kGemmResidual, s->hidden, static_cast<uint32_t>(A), tokens, pgemm_ws_bytes) != 0 &&
-           slices(kGemmSwiglu, s->intermediate, s->hidden, tokens, pgemm_ws_bytes) != 0 &&
-           slices(kGemmResidual, s->hidden, s->intermediate, tokens, pgemm_ws_bytes) != 0;
+  // have that kernel (twice the tokens per weight byte of the 128-token one): every width that is a multiple of 64
+  // qualifies for both; other widths keep 128-token blocks. The "prefill_block_tokens" override caps the choice.
+  const auto all_four = [&](uint32_t tokens) {
+    return gemm_rows_takes(kGemmF32, static_cast<uint32_t>(A + 2 * KV), s->hidden, tokens, pgemm_ws_bytes) &&
+           gemm_rows_takes(kGemmResidual, s->hidden, static_cast<uint32_t>(A), tokens, pgemm_ws_bytes) &&
+           gemm_rows_takes(kGemmSwiglu, s->intermediate, s->hidden, tokens, pgemm_ws_bytes) &&
+           gemm_rows_takes(kGemmResidual, s->hidden, s->intermediate, tokens, pgemm_ws_bytes);
   };
   const int block_cap = tuning(kTunePrefillBlockTokens);
-  const bool wide = block_cap != 128 && block_operand_tiles(kGemmWideMaxTokens) != 0 && all_four(gemm_wide_slices, kGemmWideMaxTokens);
-  // (a prompt's last block can have any size: 512-token blocks only where the 256-token kernel takes the rest)
-  const bool deep = wide && block_cap != 256 && block_operand_tiles(kGemmDeepMaxTokens) != 0 &&
-                    all_four(gemm_deep_slices, kGemmDeepMaxTokens) && all_four(gemm_deep_slices, kGemmWideMaxTokens + 1);
+  // (a prompt's last block can have any size: larger blocks only where every smaller one has its kernel too)
+  const bool wide = block_cap != 128 && tuning(kTuneBlockLayout) != 1 && all_four(kGemmMaxTokens + 1) && all_four(kGemmWideMaxTokens);
+  const bool deep = wide && block_cap != 256 && all_four(kGemmWideMaxTokens + 1) && all_four(kGemmDeepMaxTokens);
   s->prefill_block_tokens = deep ? kGemmDeepMaxTokens : wide ? kGemmWideMaxTokens : kGemmMaxTokens;
   s->blogits = batch_head ? reinterpret_cast<float *>(s->arena + off_blogits) : nullptr;
   s->btable = reinterpret_cast<BatchTable *>(s->arena + off_btable);
@@ -1317,7 +1317,7 @@ hipError_t enqueue_batch_step(Session *lead, Session *const *seqs, uint32_t T,
   const uint32_t H = lead->hidden, A = lead->heads * lead->head_dim, KV = lead->kv_heads * lead->head_dim,
                  I = lead->intermediate;
   const float *rope_freq = lead->theta > 0.0f ? lead->rope_freq : nullptr;
-  const uint32_t tiles = block_operand_tiles(T);
+  const uint32_t tiles = block_operand_tiles(lead, T);
   BatchTable *host = lead->host_btable;
   uint32_t min_blocks = ~0u;
   for (uint32_t t = 0; t < T; ++t) {

@@ -12,9 +12,7 @@
 // Projections with few rows get their parallelism from K: grid (row groups, K slices); with more than
 // one slice the workgroups write f32 partial sums and gemm_block_finish_kernel adds them in slice order
 // (deterministic) and applies the epilogue.
-#include "gemm_rows.cuh"
-
-#include "activations.cuh"
+#include "gemm_epilogue.cuh"
 
 #include <stdlib.h>
 
@@ -36,64 +34,6 @@ constexpr int kBRowStride = kBK + 16;        // LDS row stride of a W tile in el
                                              // lanes of every such group met in the same banks (4 extra cycles per operand read,
                                              // a third of the kernel's LDS time by the bank-conflict counter); with 32 B they do not
 constexpr int kBWTile = 16 * kBRowStride;    // one 16-row block of W in LDS
-
-typedef __bf16 bf16x8_t __attribute__((ext_vector_type(8)));
-typedef _Float16 f16x8_t __attribute__((ext_vector_type(8)));
-typedef float f32x4_t __attribute__((ext_vector_type(4)));
-typedef uint32_t u32x4_t __attribute__((ext_vector_type(4)));   // a 16-byte piece as a first-class value
-
-template <uint32_t DT>
-__device__ __forceinline__ f32x4_t mfma_k32(u32x4_t a, u32x4_t b, f32x4_t c) {
-  if constexpr (DT == kBF16)
-    return __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8_t, a), __builtin_bit_cast(bf16x8_t, b), c,
-                                                   0, 0, 0);
-  else
-    return __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(f16x8_t, a), __builtin_bit_cast(f16x8_t, b), c, 0,
-                                                  0, 0);
-}
-
-// Epilogue of four consecutive output rows (row .. row + 3) of token t. For SwiGLU `up` holds the up
-// rows' sums, otherwise it is unused.
-template <uint32_t DT, int EPI>
-__device__ __forceinline__ void block_epilogue(const GemmRowsParams &p, uint32_t t, uint32_t row, f32x4_t y, f32x4_t up) {
-  if (p.bias != nullptr) {
-#pragma unroll
-    for (int r = 0; r < 4; ++r) {
-      y[r] += dec16<DT>(p.bias[row + r]);
-      if constexpr (EPI == kGemmSwiglu) up[r] += dec16<DT>(p.bias[p.rows + row + r]);
-    }
-  }
-  const uint64_t at = static_cast<uint64_t>(t) * p.rows + row;
-  if constexpr (EPI == kGemmSwiglu) {
-    uint16_t h[4];
-#pragma unroll
-    for (int r = 0; r < 4; ++r) h[r] = enc16<DT>(silu(y[r]) * up[r]);
-    const uint64_t at16 = p.out_packed_tiles != 0 ? gemm_x_packed_index(p.out_packed_tiles, t, row) : at;
-    *reinterpret_cast<uint2 *>(p.out16 + at16) =
-        make_uint2(h[0] | (static_cast<uint32_t>(h[1]) << 16), h[2] | (static_cast<uint32_t>(h[3]) << 16));
-  } else if constexpr (EPI == kGemmXielu) {
-    const XieluParams act = xielu_params<DT>(p.act);
-    uint16_t h[4];
-#pragma unroll
-    for (int r = 0; r < 4; ++r) h[r] = enc16<DT>(xielu(y[r], act));
-    const uint64_t at16 = p.out_packed_tiles != 0 ? gemm_x_packed_index(p.out_packed_tiles, t, row) : at;
-    *reinterpret_cast<uint2 *>(p.out16 + at16) =
-        make_uint2(h[0] | (static_cast<uint32_t>(h[1]) << 16), h[2] | (static_cast<uint32_t>(h[3]) << 16));
-  } else {
-    if constexpr (EPI == kGemmResidual) {
-      const float4 res = *reinterpret_cast<const float4 *>(p.residual + at);
-      y[0] += res.x;
-      y[1] += res.y;
-      y[2] += res.z;
-      y[3] += res.w;
-      if (p.round_out) {
-#pragma unroll
-        for (int r = 0; r < 4; ++r) y[r] = round16<DT>(y[r]);
-      }
-    }
-    *reinterpret_cast<float4 *>(p.out_f32 + at) = make_float4(y[0], y[1], y[2], y[3]);
-  }
-}
 
 // Grid (row groups, K slices). NR: row tiles per wave (SwiGLU: 2 = the gate tile and its up tile).
 // cols / gridDim.y must be a multiple of kBRing * kBK (the block loop is unrolled by the ring depth, so
@@ -416,6 +356,18 @@ __global__ __launch_bounds__(kFinNormThreads) void gemm_finish_norm_kernel(GemmR
   }
 }
 
+template <uint32_t DT, int EPI>
+hipError_t launch_finish(const GemmRowsParams &p, const float *partials, uint32_t kslices, uint32_t tokcap, hipStream_t stream) {
+  if (EPI == kGemmResidual && p.norm_gamma != nullptr) {   // (the caller asked gemm_rows_fuses_norm first)
+    hipLaunchKernelGGL((gemm_finish_norm_kernel<DT>), dim3(p.tokens), dim3(kFinNormThreads), 0, stream, p, partials, kslices, tokcap);
+  } else {
+    const uint32_t threads = p.rows / 4u * p.tokens;
+    hipLaunchKernelGGL((gemm_block_finish_kernel<DT, EPI>), dim3((threads + 255u) / 256u), dim3(256), 0, stream, p, partials, kslices,
+                       tokcap);
+  }
+  return hipGetLastError();
+}
+
 // K-blocks by which consecutive row groups start their walk apart (the "gemm_block_rotate" override: value - 1)
 inline uint32_t block_rotation() {
   const int want = tuning(kTuneGemmBlockRotate);
@@ -445,15 +397,7 @@ hipError_t launch_block_tt(const GemmRowsParams &p, float *partials, uint32_t ks
                      p, partials, block_rotation());
   hipError_t err = hipGetLastError();
   if (err == hipSuccess && kslices > 1 && !(EPI == kGemmF32 && p.keep_partials != 0)) {
-    if (EPI == kGemmResidual && p.norm_gamma != nullptr) {   // (the caller asked gemm_rows_fuses_norm first)
-      hipLaunchKernelGGL((gemm_finish_norm_kernel<DT>), dim3(p.tokens), dim3(kFinNormThreads), 0, stream, p,
-                         static_cast<const float *>(partials), kslices, kBTokCap);
-    } else {
-      const uint32_t threads = p.rows / 4u * p.tokens;
-      hipLaunchKernelGGL((gemm_block_finish_kernel<DT, EPI>), dim3((threads + 255u) / 256u), dim3(256), 0, stream, p,
-                         static_cast<const float *>(partials), kslices, kBTokCap);
-    }
-    err = hipGetLastError();
+    err = launch_finish<DT, EPI>(p, partials, kslices, kBTokCap, stream);
   }
   return err;
 }
@@ -675,7 +619,8 @@ __global__ __launch_bounds__(PAIRS * 2 * kWave, 2) void gemm_wide_kernel(GemmRow
 }
 
 // ---------------------------------------------------------------------------------------------
-// Token blocks of 257..512 rows (X in operand order with 32 token tiles). What bounds the kernel above is what a
+// Token blocks of 257..512 rows (X in operand order with 32 token tiles; blocks of 129..256 where the kernel above does
+// not take the shape). What bounds the kernel above is what a
 // CU has to pull in, not its matrix cores: every workgroup of 128 weight rows fetches the whole X block from L2
 // (twice the weight bytes per launch), ten operand pieces cross the LDS port for every sixteen products, and every
 // X block is written to LDS through registers. A block of 512 tokens lets a workgroup take 256 weight rows (a
@@ -708,7 +653,10 @@ constexpr size_t deep_lds_bytes(int tpw) { return 2 * static_cast<size_t>(kDXBuf
 // the launch fill the chip - a gate/up pair of 12288 + 12288 rows is 96 workgroups of 128 + 128 rows per token half,
 // 192 in all on 256 CUs, but 128 of 96 + 96). With three tiles a wave the gate tiles and the up tiles of a pair end
 // in different waves (row parts 0, 1: gate, 2, 3: their up tiles), and the up sums cross through LDS at the end.
-template <uint32_t DT, int EPI, int TPW>
+// RAGGED: the rows do not divide into workgroups or the K-blocks into slices of an even number. Rows past the last are
+// the last eight fetched again, their sums dropped; K-blocks past a slice's last are that one fetched again, not
+// multiplied. (A variant of its own: the clamps and the odd end cost the others 2 % of a whole prompt.)
+template <uint32_t DT, int EPI, int TPW, bool RAGGED>
 __global__ __launch_bounds__(8 * kWave, 2) void gemm_deep_kernel(GemmRowsParams p, float *partials, uint32_t units,
                                                                   uint32_t kslices) {
   static_assert(TPW == 3 || TPW == 4, "three or four row tiles a wave");
@@ -726,20 +674,25 @@ __global__ __launch_bounds__(8 * kWave, 2) void gemm_deep_kernel(GemmRowsParams 
   const uint32_t half = in_xcd % halves, unit = (in_xcd / halves) * 8u + (blockIdx.x & 7u);
   if (unit >= units) return;
   const uint32_t group = unit / kslices, slice = unit % kslices;
-  const uint32_t kper = cols / kslices, k0 = slice * kper, nblk = kper / kDK;
+  // K slices: runs of whole K-blocks, as even as they come
+  const uint32_t kblocks = cols / kDK, kfirst = slice * kblocks / kslices;
+  const uint32_t nblk = RAGGED ? (slice + 1) * kblocks / kslices - kfirst : kblocks / kslices, k0 = kfirst * kDK;
 
   // LDS tile slot s = TPW * (row part) + j. Plain: rows 16 s .. of the workgroup's rows. SwiGLU, four tiles a
   // wave: j = 0, 1 the gate tiles 2 rq + j of the workgroup's 128 gate rows, j = 2, 3 their up tiles - a wave's
   // tiles end in the wave that runs the epilogue. SwiGLU, three tiles a wave: parts 0, 1 the six gate tiles of
   // the workgroup's 96 gate rows, parts 2, 3 their up tiles.
-  auto slot_row = [&](int s) -> uint32_t {
+  auto slot_row = [&](int s) -> uint32_t {   // output row
     if constexpr (EPI == kGemmSwiglu && TPW == 4)
-      return ((s >> 1) & 1) * p.rows + group * 128u + (2u * (s >> 2) + (s & 1)) * 16u;
+      return group * 128u + (2u * (s >> 2) + (s & 1)) * 16u;
     else if constexpr (EPI == kGemmSwiglu)
-      return (s / 6) * p.rows + group * 96u + (s % 6) * 16u;
+      return group * 96u + (s % 6) * 16u;
     else
       return group * (16u * kTiles) + s * 16u;
   };
+  auto in_rows = [&](uint32_t row) -> uint32_t { return RAGGED ? min(row, p.rows - 8u) : row; };
+  auto in_slice = [&](uint32_t blk) -> uint32_t { return RAGGED ? min(blk, nblk - 1u) : blk; };
+  auto kept = [&](uint32_t row) -> bool { return !RAGGED || row < p.rows; };
   auto slot_is_up = [&](int s) -> bool { return EPI == kGemmSwiglu && (TPW == 4 ? ((s >> 1) & 1) != 0 : s >= 6); };
   const uint32_t lds0 = static_cast<uint32_t>(reinterpret_cast<uintptr_t>(NV_LDS_PTR(smem)));   // X buffers, then W buffers
   // W requests of this wave: requests kWReq wave .. + kWReq - 1 of the block's 2 kTiles (tile m / 2, rows 8 (m % 2)
@@ -750,7 +703,8 @@ __global__ __launch_bounds__(8 * kWave, 2) void gemm_deep_kernel(GemmRowsParams 
   for (int i = 0; i < kWReq; ++i) {
     const int m = kWReq * wave + i, s_ = m >> 1;
     wsrc[i] = reinterpret_cast<const char *>(p.w) +
-              (static_cast<uint64_t>(slot_row(s_) + (m & 1) * 8u) * cols + k0 + (slot_is_up(s_) ? p.pair_gap : 0u)) * sizeof(uint16_t);
+              (static_cast<uint64_t>(in_rows(slot_row(s_) + (m & 1) * 8u) + (slot_is_up(s_) ? p.rows : 0u)) * cols + k0 +
+               (slot_is_up(s_) ? p.pair_gap : 0u)) * sizeof(uint16_t);
   }
   const uint32_t wlane = ((lane >> 3) * cols) * static_cast<uint32_t>(sizeof(uint16_t)) + (((lane & 7) ^ (lane >> 3)) << 4);
   // X requests of this wave: four consecutive token tiles of one K-step of the half's block
@@ -813,9 +767,9 @@ __global__ __launch_bounds__(8 * kWave, 2) void gemm_deep_kernel(GemmRowsParams 
   // request slots between the products: first the next X block's four pieces, then the W block two ahead
 #define NV_DP_SLOT(IDX, XB, XEN, WEN)                                                               \
   if constexpr ((IDX) < 4) {                                                                        \
-    if constexpr (XEN) { NV_DP_X1((XB) ^ 1, blk_ + 1u, IDX); }                                      \
+    if constexpr (XEN) { NV_DP_X1((XB) ^ 1, in_slice(blk_ + 1u), IDX); }                                      \
   } else if constexpr ((IDX) < 4 + kWReq) {                                                         \
-    if constexpr (WEN) { NV_DP_W1(w_ahead, blk_ + 2u, (IDX) - 4); }                                 \
+    if constexpr (WEN) { NV_DP_W1(w_ahead, in_slice(blk_ + 2u), (IDX) - 4); }                                 \
   }
 #define NV_DP_ITEM(IDX, XB, XEN, WEN)                                                               \
   if constexpr ((IDX) + 2 < 16) { NV_DP_READ_B(XB, (IDX) + 2); }                                    \
@@ -861,7 +815,7 @@ __global__ __launch_bounds__(8 * kWave, 2) void gemm_deep_kernel(GemmRowsParams 
     w_cur = w_cur == static_cast<uint32_t>(2 * kWBuf) ? 0u : w_cur + kWBuf;                          \
   } while (0)
 
-  // start: X block 0, W blocks 0 and 1, in the order they are awaited in (nblk is even and at least 2)
+  // start: X block 0, W blocks 0 and 1, in the order they are awaited in (a W block past the last: the last again)
   uint32_t w_cur = 0;   // byte offset of the W buffer of the block being multiplied (wave-uniform)
   {
     const uint32_t blk_ = 0;
@@ -873,15 +827,21 @@ __global__ __launch_bounds__(8 * kWave, 2) void gemm_deep_kernel(GemmRowsParams 
   for (int i = 0; i < kWReq; ++i) NV_DP_W1(0u, 0u, i);
   __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-  for (int i = 0; i < kWReq; ++i) NV_DP_W1(static_cast<uint32_t>(kWBuf), 1u, i);
+  for (int i = 0; i < kWReq; ++i) NV_DP_W1(static_cast<uint32_t>(kWBuf), in_slice(1u), i);
   __builtin_amdgcn_sched_barrier(0);
   uint32_t blk = 0;
   for (; blk + 2 < nblk; blk += 2) {
     NV_DP_BLOCK(blk, 0, false, true, true);
     NV_DP_BLOCK(blk + 1, 1, false, true, true);
   }
+  // (an odd count ends with the first of these two: what was requested behind its block is the last block again)
   NV_DP_BLOCK(blk, 0, false, true, false);
-  NV_DP_BLOCK(blk + 1, 1, true, false, false);
+  if constexpr (RAGGED) {
+    if (blk + 1 < nblk) NV_DP_BLOCK(blk + 1, 1, true, false, false);
+    else asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+  } else {
+    NV_DP_BLOCK(blk + 1, 1, true, false, false);
+  }
 #undef NV_DP_W1
 #undef NV_DP_X1
 #undef NV_DP_LDS_READ
@@ -913,7 +873,9 @@ __global__ __launch_bounds__(8 * kWave, 2) void gemm_deep_kernel(GemmRowsParams 
       const uint32_t t = half * 256u + (th * 8 + c) * 16u + n;
       if (t < T) {
 #pragma unroll
-        for (int j = 0; j < TPW; ++j) block_epilogue<DT, EPI>(p, t, slot_row(TPW * rq + j) + q * 4u, acc[j][c], meet[(j * 8 + c) * kWave]);
+        for (int j = 0; j < TPW; ++j)
+          if (const uint32_t row = slot_row(TPW * rq + j) + q * 4u; kept(row))
+            block_epilogue<DT, EPI>(p, t, row, acc[j][c], meet[(j * 8 + c) * kWave]);
       }
     }
   } else if (kslices == 1) {
@@ -923,10 +885,12 @@ __global__ __launch_bounds__(8 * kWave, 2) void gemm_deep_kernel(GemmRowsParams 
       if (t < T) {
         if constexpr (EPI == kGemmSwiglu) {
 #pragma unroll
-          for (int j = 0; j < 2; ++j) block_epilogue<DT, EPI>(p, t, slot_row(4 * rq + j) + q * 4u, acc[j][c], acc[j + 2][c]);
+          for (int j = 0; j < 2; ++j)
+            if (const uint32_t row = slot_row(4 * rq + j) + q * 4u; kept(row)) block_epilogue<DT, EPI>(p, t, row, acc[j][c], acc[j + 2][c]);
         } else {
 #pragma unroll
-          for (int j = 0; j < TPW; ++j) block_epilogue<DT, EPI>(p, t, slot_row(TPW * rq + j) + q * 4u, acc[j][c], acc[j][c]);
+          for (int j = 0; j < TPW; ++j)
+            if (const uint32_t row = slot_row(TPW * rq + j) + q * 4u; kept(row)) block_epilogue<DT, EPI>(p, t, row, acc[j][c], acc[j][c]);
         }
       }
     }
@@ -939,7 +903,8 @@ __global__ __launch_bounds__(8 * kWave, 2) void gemm_deep_kernel(GemmRowsParams 
       if (t < T) {
 #pragma unroll
         for (int j = 0; j < TPW; ++j)
-          *reinterpret_cast<float4 *>(part + static_cast<uint64_t>(t) * wrows + slot_row(TPW * rq + j) + q * 4u) =
+          if (const uint32_t row = slot_row(TPW * rq + j) + q * 4u; kept(row))
+            *reinterpret_cast<float4 *>(part + static_cast<uint64_t>(t) * wrows + (slot_is_up(TPW * rq + j) ? p.rows : 0u) + row) =
               make_float4(acc[j][c][0], acc[j][c][1], acc[j][c][2], acc[j][c][3]);
       }
     }
@@ -986,35 +951,57 @@ inline uint32_t deep_slices_for(int epilogue, uint32_t rows, uint32_t cols, int 
   while (slices > 1 && static_cast<uint64_t>(slices) * kDTokCap * wrows * sizeof(float) > workspace_bytes) slices /= 2u;
   return slices;
 }
-// The tile height whose busiest CU has the least to do: rounds of 256 workgroups x rows a workgroup x columns a slice
+// Shapes that divide (rows into workgroups, K into pairs of blocks) of more than 256 token rows: the tile height whose
+// busiest CU has the least to do - rounds of 256 workgroups x rows a workgroup x columns a slice. Other shapes, and blocks
+// of 129..256 rows that the kernel with wave pairs does not take: the tile height and the K slices (any number: a slice
+// is a run of whole K-blocks) of the shortest estimate - 1.5 us a CU for 256 rows x 256 tokens x 64 columns, and for
+// partial sums 4 us and their way to memory and back at 4 TB/s.
 inline DeepPlan deep_plan(int epilogue, uint32_t rows, uint32_t cols, uint32_t tokens, uint64_t workspace_bytes) {
   DeepPlan best{0, 0};
-  if (tokens <= kWTokCap || tokens > kDTokCap || cols % (2u * kDK) != 0) return best;
-  uint64_t best_cost = ~uint64_t{0};
+  if (tokens <= kBTokCap || tokens > kDTokCap || cols % kDK != 0 || rows % 8u != 0) return best;
+  if (tokens > kWTokCap && cols % (2u * kDK) == 0) {
+    uint64_t best_cost = ~uint64_t{0};
+    for (int tpw = 4; tpw >= 3; --tpw) {
+      const uint32_t slices = deep_slices_for(epilogue, rows, cols, tpw, workspace_bytes);
+      if (slices == 0) continue;
+      const uint64_t wgs = static_cast<uint64_t>(rows / deep_wg_rows(epilogue, tpw)) * 2u * slices;
+      const uint64_t cost = (wgs + 255u) / 256u * deep_wg_rows(epilogue, tpw) * (cols / slices);
+      if (cost < best_cost) {
+        best_cost = cost;
+        best = DeepPlan{tpw, slices};
+      }
+    }
+    if (best.tpw != 0) return best;
+  }
+  const uint32_t halves = (tokens + 255u) / 256u, blocks = cols / kDK;
+  double least = 0.0;
   for (int tpw = 4; tpw >= 3; --tpw) {
-    const uint32_t slices = deep_slices_for(epilogue, rows, cols, tpw, workspace_bytes);
-    if (slices == 0) continue;
-    const uint64_t wgs = static_cast<uint64_t>(rows / deep_wg_rows(epilogue, tpw)) * 2u * slices;
-    const uint64_t cost = (wgs + 255u) / 256u * deep_wg_rows(epilogue, tpw) * (cols / slices);
-    if (cost < best_cost) {
-      best_cost = cost;
-      best = DeepPlan{tpw, slices};
+    const uint32_t groups = (rows + deep_wg_rows(epilogue, tpw) - 1) / deep_wg_rows(epilogue, tpw);
+    for (uint32_t slices = 1; slices <= 8u && slices * 2u <= blocks; ++slices) {
+      if (slices > 1 && (epilogue == kGemmSwiglu || static_cast<uint64_t>(slices) * kDTokCap * rows * sizeof(float) > workspace_bytes)) break;
+      const double us = 0.375 * tpw * ((groups * halves * slices + 255u) / 256u) * ((blocks + slices - 1) / slices) +
+                        (slices > 1 ? 4.0 + 8.0 * slices * tokens * rows / 4e6 : 0.0);
+      if (best.tpw == 0 || us < least) {
+        least = us;
+        best = DeepPlan{tpw, slices};
+      }
     }
   }
+  if (best.tpw == 0) best = DeepPlan{4, 1};   // a single K-block
   return best;
 }
 
-template <uint32_t DT, int EPI, int TPW>
+template <uint32_t DT, int EPI, int TPW, bool RAGGED>
 hipError_t launch_deep_tpw(const GemmRowsParams &p, float *partials, uint32_t kslices, hipStream_t stream) {
   static std::once_flag once;
   static hipError_t raised = hipSuccess;
   std::call_once(once, [] {
-    raised = hipFuncSetAttribute(reinterpret_cast<const void *>(&gemm_deep_kernel<DT, EPI, TPW>),
+    raised = hipFuncSetAttribute(reinterpret_cast<const void *>(&gemm_deep_kernel<DT, EPI, TPW, RAGGED>),
                                  hipFuncAttributeMaxDynamicSharedMemorySize, static_cast<int>(deep_lds_bytes(TPW)));
   });
   if (raised != hipSuccess) return raised;
-  const uint32_t units = p.rows / deep_wg_rows(EPI, TPW) * kslices, halves = (p.tokens + 255u) / 256u;
-  hipLaunchKernelGGL((gemm_deep_kernel<DT, EPI, TPW>), dim3((units + 7u) / 8u * 8u * halves), dim3(8 * kWave), deep_lds_bytes(TPW),
+  const uint32_t units = (p.rows + deep_wg_rows(EPI, TPW) - 1) / deep_wg_rows(EPI, TPW) * kslices, halves = (p.tokens + 255u) / 256u;
+  hipLaunchKernelGGL((gemm_deep_kernel<DT, EPI, TPW, RAGGED>), dim3((units + 7u) / 8u * 8u * halves), dim3(8 * kWave), deep_lds_bytes(TPW),
                      stream, p, partials, units, kslices);
   return hipGetLastError();
 }
@@ -1022,18 +1009,13 @@ hipError_t launch_deep_tpw(const GemmRowsParams &p, float *partials, uint32_t ks
 template <uint32_t DT, int EPI>
 hipError_t launch_deep(const GemmRowsParams &p, float *partials, const DeepPlan &plan, hipStream_t stream) {
   const uint32_t kslices = plan.kslices;
-  hipError_t err = plan.tpw == 3 ? launch_deep_tpw<DT, EPI, 3>(p, partials, kslices, stream)
-                                 : launch_deep_tpw<DT, EPI, 4>(p, partials, kslices, stream);
+  const bool ragged = p.rows % deep_wg_rows(EPI, plan.tpw) != 0 || p.cols % (2u * kDK * kslices) != 0;
+  hipError_t err = plan.tpw == 3 ? (ragged ? launch_deep_tpw<DT, EPI, 3, true>(p, partials, kslices, stream)
+                                           : launch_deep_tpw<DT, EPI, 3, false>(p, partials, kslices, stream))
+                                 : (ragged ? launch_deep_tpw<DT, EPI, 4, true>(p, partials, kslices, stream)
+                                           : launch_deep_tpw<DT, EPI, 4, false>(p, partials, kslices, stream));
   if (err == hipSuccess && kslices > 1) {
-    if (EPI == kGemmResidual && p.norm_gamma != nullptr) {   // (the caller asked gemm_rows_fuses_norm first)
-      hipLaunchKernelGGL((gemm_finish_norm_kernel<DT>), dim3(p.tokens), dim3(kFinNormThreads), 0, stream, p,
-                         static_cast<const float *>(partials), kslices, kDTokCap);
-    } else {
-      const uint32_t threads = p.rows / 4u * p.tokens;
-      hipLaunchKernelGGL((gemm_block_finish_kernel<DT, EPI>), dim3((threads + 255u) / 256u), dim3(256), 0, stream, p,
-                         static_cast<const float *>(partials), kslices, kDTokCap);
-    }
-    err = hipGetLastError();
+    err = launch_finish<DT, EPI>(p, partials, kslices, kDTokCap, stream);
   }
   return err;
 }
@@ -1057,15 +1039,7 @@ hipError_t launch_wide(const GemmRowsParams &p, float *partials, uint32_t kslice
                    : pairs == 4 ? launch_wide_pairs<DT, EPI, 4>(p, partials, kslices, stream)
                                 : hipErrorInvalidValue;
   if (err == hipSuccess && kslices > 1) {
-    if (EPI == kGemmResidual && p.norm_gamma != nullptr) {   // (the caller asked gemm_rows_fuses_norm first)
-      hipLaunchKernelGGL((gemm_finish_norm_kernel<DT>), dim3(p.tokens), dim3(kFinNormThreads), 0, stream, p,
-                         static_cast<const float *>(partials), kslices, kWTokCap);
-    } else {
-      const uint32_t threads = p.rows / 4u * p.tokens;
-      hipLaunchKernelGGL((gemm_block_finish_kernel<DT, EPI>), dim3((threads + 255u) / 256u), dim3(256), 0, stream, p,
-                         static_cast<const float *>(partials), kslices, kWTokCap);
-    }
-    err = hipGetLastError();
+    err = launch_finish<DT, EPI>(p, partials, kslices, kWTokCap, stream);
   }
   return err;
 }
@@ -1164,9 +1138,7 @@ uint32_t gemm_wide_slices(int epilogue, uint32_t rows, uint32_t cols, uint32_t t
   return slices;
 }
 
-// Blocks of 257..512 rows: K slices of gemm_deep_kernel, or 0 where it does not take the shape (rows a multiple of 256
-// or 192; a gate/up pair: of 128 or 96). Enough workgroups (row groups x 2 token halves x slices) for three quarters
-// of the CUs, each slice an even number of K-blocks, the partial sums within the workspace.
+// Blocks of 129..512 rows: K slices of gemm_deep_kernel, or 0 where it does not take the shape (rows % 8, cols % 64).
 uint32_t gemm_deep_slices(int epilogue, uint32_t rows, uint32_t cols, uint32_t tokens, uint64_t workspace_bytes) {
   return deep_plan(epilogue, rows, cols, tokens, workspace_bytes).kslices;
 }
@@ -1185,14 +1157,40 @@ bool gemm_rows_fuses_norm(int epilogue, uint32_t rows, uint32_t cols, uint32_t t
     return false;
   // wherever a launch of its own adds the K slices: the deep or the wide kernel's, or the shared-X kernel's for smaller blocks
   if (tokens > kWTokCap) return gemm_deep_slices(epilogue, rows, cols, tokens, workspace_bytes) > 1;
-  if (tokens > kBTokCap) return gemm_wide_slices(epilogue, rows, cols, tokens, workspace_bytes) > 1;
-  return gemm_block_plan(epilogue, rows, cols, tokens, workspace_bytes).kslices > 1;
+  if (tokens > kBTokCap) {
+    const uint32_t wide = gemm_wide_slices(epilogue, rows, cols, tokens, workspace_bytes);
+    return (wide != 0 ? wide : gemm_deep_slices(epilogue, rows, cols, tokens, workspace_bytes)) > 1;
+  }
+  const uint32_t block = gemm_block_plan(epilogue, rows, cols, tokens, workspace_bytes).kslices;
+  if (block != 0 || gemm_rows_supported(rows, cols, tokens)) return block > 1;
+  return gemm_flow_plan(epilogue, rows, cols, tokens, workspace_bytes).kslices > 1;
 }
 
 uint64_t gemm_block_workspace_bytes(uint32_t rows_max) {
   // room for 8 slices of the widest plain projection (or 2 of a gate/up pair of that width) at the deep kernel's
   // token stride
   return static_cast<uint64_t>(8) * kDTokCap * rows_max * sizeof(float);
+}
+
+namespace {
+template <uint32_t DT>
+hipError_t launch_finish_dt(int epilogue, const GemmRowsParams &p, const float *partials, uint32_t kslices, uint32_t tokcap, hipStream_t stream) {
+  switch (epilogue) {
+    case kGemmF32: return launch_finish<DT, kGemmF32>(p, partials, kslices, tokcap, stream);
+    case kGemmResidual: return launch_finish<DT, kGemmResidual>(p, partials, kslices, tokcap, stream);
+    case kGemmXielu: return launch_finish<DT, kGemmXielu>(p, partials, kslices, tokcap, stream);
+    case kGemmSwiglu: return launch_finish<DT, kGemmSwiglu>(p, partials, kslices, tokcap, stream);
+    default: return hipErrorInvalidValue;
+  }
+}
+}  // namespace
+
+hipError_t launch_gemm_finish(uint32_t dtype, int epilogue, const GemmRowsParams &p, const float *partials, uint32_t kslices,
+                              uint32_t tokcap, hipStream_t stream) {
+  if (p.rows % 4 != 0 || partials == nullptr) return hipErrorInvalidValue;
+  if (dtype == kBF16) return launch_finish_dt<kBF16>(epilogue, p, partials, kslices, tokcap, stream);
+  if (dtype == kF16) return launch_finish_dt<kF16>(epilogue, p, partials, kslices, tokcap, stream);
+  return hipErrorInvalidValue;
 }
 
 hipError_t launch_gemm_wide(uint32_t dtype, int epilogue, const GemmRowsParams &p, uint32_t kslices, hipStream_t stream) {

@@ -310,16 +310,26 @@ bool gemm_rows_supported(uint32_t rows, uint32_t cols, uint32_t tokens) {
   return rows >= 16 && cols != 0 && cols % (kGW * kKB) == 0 && tokens >= 1 && tokens <= kGemmMaxTokens;
 }
 
+bool gemm_rows_takes(int epilogue, uint32_t rows, uint32_t cols, uint32_t tokens, uint64_t workspace_bytes) {
+  if (tokens > kGemmMaxTokens)
+    return (tokens <= kGemmWideMaxTokens && gemm_wide_slices(epilogue, rows, cols, tokens, workspace_bytes) != 0) ||
+           gemm_deep_slices(epilogue, rows, cols, tokens, workspace_bytes) != 0;
+  return gemm_rows_supported(rows, cols, tokens) || gemm_flow_plan(epilogue, rows, cols, tokens, workspace_bytes).kslices != 0;
+}
+
 hipError_t launch_gemm_rows(uint32_t dtype, int epilogue, const GemmRowsParams &p, hipStream_t stream) {
-  // more than kGemmMaxTokens rows: only in operand order and only where the kernel for wide blocks takes the shape
+  // more than kGemmMaxTokens rows: only in operand order
+  const uint64_t room = p.workspace != nullptr ? p.workspace_bytes : 0;
   const uint32_t wide_slices = p.tokens > kGemmMaxTokens && p.tokens <= kGemmWideMaxTokens && p.x_packed != 0
-                                   ? gemm_wide_slices(epilogue, p.rows, p.cols, p.tokens, p.workspace != nullptr ? p.workspace_bytes : 0)
+                                   ? gemm_wide_slices(epilogue, p.rows, p.cols, p.tokens, room)
                                    : 0u;
-  const uint32_t deep_slices = p.tokens > kGemmWideMaxTokens && p.x_packed != 0
-                                   ? gemm_deep_slices(epilogue, p.rows, p.cols, p.tokens, p.workspace != nullptr ? p.workspace_bytes : 0)
+  const uint32_t deep_slices = p.tokens > kGemmMaxTokens && wide_slices == 0 && p.x_packed != 0
+                                   ? gemm_deep_slices(epilogue, p.rows, p.cols, p.tokens, room)
                                    : 0u;
+  const bool streams = gemm_rows_supported(p.rows, p.cols, p.tokens);   // the kernels of this file and of gemm_block.hip
+  const GemmFlowPlan flow = p.x_packed != 0 && !streams ? gemm_flow_plan(epilogue, p.rows, p.cols, p.tokens, room) : GemmFlowPlan{};
   if (p.w == nullptr || p.x16 == nullptr) return hipErrorInvalidValue;
-  if (wide_slices == 0 && deep_slices == 0 && !gemm_rows_supported(p.rows, p.cols, p.tokens)) return hipErrorInvalidValue;
+  if (wide_slices == 0 && deep_slices == 0 && flow.kslices == 0 && !streams) return hipErrorInvalidValue;
   if (!aligned16(p.w) || !aligned16(p.x16)) return hipErrorInvalidValue;
   if ((epilogue == kGemmF32 || epilogue == kGemmResidual) && p.out_f32 == nullptr) return hipErrorInvalidValue;
   if (epilogue == kGemmResidual && p.residual == nullptr) return hipErrorInvalidValue;
@@ -344,6 +354,7 @@ hipError_t launch_gemm_rows(uint32_t dtype, int epilogue, const GemmRowsParams &
   if (p.x_packed != 0) {   // blocks in operand order: the kernel that shares X through LDS, where its plan takes the shape
     const GemmBlockPlan plan = gemm_block_plan(epilogue, p.rows, p.cols, p.tokens, p.workspace != nullptr ? p.workspace_bytes : 0);
     if (plan.kslices != 0) return launch_gemm_block(dtype, epilogue, p, plan, stream);
+    if (flow.kslices != 0) return launch_gemm_flow(dtype, epilogue, p, flow, stream);
   }
   if (dtype == kBF16) return launch_dt<kBF16>(epilogue, p, stream);
   return launch_dt<kF16>(epilogue, p, stream);

@@ -554,9 +554,22 @@ int nerva_hip_argmax(const NervaHipArgmaxRequest *r, void *stream, int32_t *hip_
   return finish(launch_argmax(r->logits, r->count, s, resolve_stream(stream)), hip_error);
 }
 
+// The shapes the operator is declared for (nerva_hip_api.h); sessions also launch it on others, in layouts of their own.
+namespace {
+bool gemm_rows_declared(const NervaHipGemmRowsRequest *r) {
+  const int epilogue = static_cast<int>(r->epilogue);
+  if (r->tokens <= kGemmMaxTokens) return gemm_rows_supported(r->rows, r->cols, r->tokens);
+  if (r->input_operand_order == 0) return false;
+  if (r->tokens <= kGemmWideMaxTokens) return gemm_wide_slices(epilogue, r->rows, r->cols, r->tokens, 0) != 0;
+  const uint32_t tile = epilogue == kGemmSwiglu ? 32u : 64u;
+  return r->tokens <= kGemmDeepMaxTokens && r->rows != 0 && r->cols != 0 && (r->rows % (3u * tile) == 0 || r->rows % (4u * tile) == 0) &&
+         r->cols % 128u == 0;
+}
+}  // namespace
+
 int nerva_hip_gemm_rows(const NervaHipGemmRowsRequest *r, void *stream, int32_t *hip_error) {
   if (hip_error) *hip_error = 0;
-  if (r == nullptr || r->epilogue > 2) return finish(hipErrorInvalidValue, hip_error);
+  if (r == nullptr || r->epilogue > 2 || !gemm_rows_declared(r)) return finish(hipErrorInvalidValue, hip_error);
   GemmRowsParams p{};
   p.w = r->weights;
   p.x16 = r->input16;

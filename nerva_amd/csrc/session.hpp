@@ -88,6 +88,7 @@ struct NervaHipHfDecodeSequenceSession {
   bool block_prefill = false;
   // the multi-row kernels take this model's shapes (prompt blocks and batch steps need it)
   bool rows_ready = false;
+  bool rows_plain = false;           // ... also for rows as they come, without matrix-operand order
   float *blogits = nullptr;          // [NERVA_HIP_BATCH_MAX_BLOCK_TOKENS][vocab] logits of a batch step
   nv::BatchTable *btable = nullptr, *host_btable = nullptr;
   nv::Slot *bslots = nullptr, *host_bslots = nullptr;   // a batch step's published slots, gathered for one copy

@@ -1,0 +1,128 @@
+"""Prompt blocks, batch steps and the decode attention at widths, head sizes and numbers of query heads a key head outside
+the power-of-two ones: against the oracle where an operator can be called alone, else against the same session walking
+token by token (whose kernels the other files hold to the oracle)."""
+import numpy as np
+import pytest
+
+import nerva_amd as N
+import oracle as O
+from nerva_amd.runtime import attention_workspace
+from test_gpu_ops import _attention_case, _attention_device, _attention_oracle, dev
+from test_gpu_session import BF16, E2E_REL_L2, F16, REL_L2, random_model, rel_l2, started
+
+pytestmark = pytest.mark.gpu
+
+# dtype, hidden, heads, kv, hd, inter, vocab, layers, theta, qk_norm, bias
+WIDTHS = [
+    (BF16, 416, 6, 2, 128, 608, 517, 2, 1e6, True, False),     # K an odd multiple of 32: blocks of 128 rows only; 3 heads a key head
+    (F16, 192, 10, 2, 64, 320, 301, 3, 1e4, False, True),      # heads of 64, 5 a key head; K of 3 and 5 blocks of 64
+    (BF16, 1344, 14, 2, 64, 2112, 1003, 2, 1e6, True, True),   # heads of 64, 7 a key head; 21 and 33 blocks of 64, ragged row groups
+    (BF16, 1536, 12, 2, 128, 2944, 801, 2, 1e6, False, True),  # 6 heads a key head; a gate/up pair that is no multiple of 128
+    (F16, 640, 5, 5, 128, 1728, 402, 2, 1e4, True, False),     # a key head each
+]
+
+
+@pytest.mark.parametrize("heads,kv_heads,hd,dtype,theta,qk_norm,bias", [
+    (6, 2, 128, BF16, 1e6, True, False), (20, 4, 128, F16, 1e4, False, True), (12, 2, 128, BF16, 0, True, True),
+    (28, 4, 128, BF16, 1e6, False, True), (8, 8, 64, F16, 1e4, True, False), (32, 8, 64, BF16, 5e5, False, False),
+    (14, 2, 64, BF16, 1e6, True, True), (16, 2, 64, F16, 0, False, False)])
+def test_step_attention_of_any_group_and_head(heads, kv_heads, hd, dtype, theta, qk_norm, bias):
+    """Edges of the 16-token tiles, one split and many, more tiles a wave than it requests ahead (few forced splits)."""
+    for tokens, splits in ((0, 0), (15, 0), (16, 0), (70, 0), (1000, 0), (2500, 2)):
+        c = _attention_case(dtype, heads, kv_heads, hd, tokens, theta, qk_norm, heads * 7 + tokens, bias=bias)
+        ref, k16, v16 = _attention_oracle(c)
+        if splits == 0:
+            got32, got16, k_new, v_new, _, _ = _attention_device(c)
+            assert np.max(np.abs(k_new.astype(np.int32) - k16.astype(np.int32))) <= 1
+            assert np.array_equal(v_new, v16)
+            assert np.array_equal(got16, O.encode16(dtype, got32))
+        else:
+            cache = N.PagedKvCache(c["layers"], c["n_blocks"], kv_heads, hd, c["table"])
+            cache.fill(c["layer"], c["k_rows"], c["v_rows"])
+            out16, out32 = N.DeviceBuffer(heads * hd * 2), N.DeviceBuffer(heads * hd * 4)
+            opt = lambda a: dev(a) if a is not None else None   # noqa: E731
+            qb, kb, vb = (opt(b) for b in c["biases"])
+            N.paged_attention(dtype, heads, kv_heads, hd, cache, c["layer"], tokens, dev(c["qkv"]), attention_workspace(heads, hd), out16,
+                              out_f32=out32, append=True, rope_theta=theta, q_norm=opt(c["qn"]), k_norm=opt(c["kn"]), q_bias=qb,
+                              k_bias=kb, v_bias=vb, splits=splits)
+            got32 = out32.numpy(np.float32)
+        assert rel_l2(got32, ref) <= REL_L2, (tokens, splits)
+
+
+def test_more_splits_than_stay_resident_still_run_where_they_did():
+    """Heads of 64 took any split factor (their kernel had no splits); they still do."""
+    c = _attention_case(BF16, 16, 8, 64, 1100, 1e6, True, 3)
+    ref, _, _ = _attention_oracle(c)
+    cache = N.PagedKvCache(c["layers"], c["n_blocks"], 8, 64, c["table"])
+    cache.fill(c["layer"], c["k_rows"], c["v_rows"])
+    out16, out32 = N.DeviceBuffer(16 * 64 * 2), N.DeviceBuffer(16 * 64 * 4)
+    N.paged_attention(BF16, 16, 8, 64, cache, c["layer"], 1100, dev(c["qkv"]), attention_workspace(16, 64), out16, out_f32=out32,
+                      append=True, rope_theta=1e6, q_norm=dev(c["qn"]), k_norm=dev(c["kn"]), splits=64)
+    assert rel_l2(out32.numpy(np.float32), ref) <= REL_L2
+
+
+def walked(weights, max_ctx):
+    N.Device.set_tuning("prefill_walk", 1)
+    try:
+        return N.DecodeSession.create(weights, max_ctx)
+    finally:
+        N.Device.set_tuning("prefill_walk", 0)
+
+
+@pytest.mark.parametrize("geom", WIDTHS)
+def test_prompt_blocks_match_the_token_walk(geom):
+    """Prompts that end in a block of 1 token, just past 32, 64, 128 and 256 rows, and in the second block of 512."""
+    dtype, hidden, heads, kv, hd, inter, vocab, layers, theta, qk_norm, bias = geom
+    weights, _ = random_model(dtype, hidden, heads, kv, hd, inter, vocab, layers, hidden, theta, qk_norm, bias)
+    s, walk = N.DecodeSession.create(weights, 704), walked(weights, 704)
+    assert s.create_result.prefill_chunk_tokens == (512 if hidden % 64 == 0 and inter % 64 == 0 else 128)
+    assert walk.create_result.prefill_chunk_tokens == 1
+    rng = np.random.default_rng(hidden)
+    for n in (2, 3, 34, 66, 130, 258, 300, 515, 640):
+        prompt = rng.integers(0, vocab, n).astype(np.uint32)
+        for session in (s, walk):
+            rc, res = session.start(prompt)
+            assert rc == 0 and res.hot_path_allocations == 0
+        assert rel_l2(s.logits(), walk.logits()) <= E2E_REL_L2, n
+        for layer in range(layers):
+            for got, want in zip(s.kv_range(layer, 0, n), walk.kv_range(layer, 0, n)):
+                tol = 2e-3 if layer == 0 else E2E_REL_L2
+                assert rel_l2(O.decode16(dtype, got), O.decode16(dtype, want)) <= tol, (n, layer)
+    for session in (s, walk):
+        session.destroy()
+
+
+@pytest.mark.parametrize("geom,count", [(WIDTHS[2], 2), (WIDTHS[2], 17), (WIDTHS[3], 5), (WIDTHS[3], 32), (WIDTHS[4], 3)])
+def test_batch_steps_match_sequences_alone(geom, count):
+    """The rows every sequence appends in batch steps are those it appends alone on the same history."""
+    dtype, hidden, heads, kv, hd, inter, vocab, layers, theta, qk_norm, bias = geom
+    weights, _ = random_model(dtype, hidden, heads, kv, hd, inter, vocab, layers, count, theta, qk_norm, bias)
+    parent = N.DecodeSession.create(weights, 96, plan=N.WeightPlan.from_weights(weights))
+    sessions = [parent] + [parent.fork_shared_weights() for _ in range(count - 1)]
+    assert parent.shares_weight_stream()
+    rng = np.random.default_rng(count)
+    prompts = [rng.integers(0, vocab, 1 + (11 * i) % 50).astype(np.uint32) for i in range(count)]
+    streams = [[started(s, p)] for s, p in zip(sessions, prompts)]
+    for _ in range(3):
+        rc, res, tokens = N.DecodeSession.batch_advance_one(sessions, 32, 2)
+        assert rc == 0 and res.block_tokens == count and res.hot_path_allocations == 0
+        for stream, token in zip(streams, tokens):
+            stream.append(int(token))
+    solo = parent.fork_shared_weights()
+    for i in sorted({0, 1, count // 2, count - 1}):
+        assert solo.release_sequence() == 0
+        rc, _, _, _ = solo.extend(prompts[i])
+        assert rc == 0
+        for token in streams[i][:-1]:       # the same history, one step at a time
+            rc, _, logits, _ = solo.extend([token], [0])
+            assert rc == 0
+        top = np.sort(logits[0])
+        assert streams[i][-1] == int(np.argmax(logits[0])) or top[-1] - top[-2] <= E2E_REL_L2 * np.max(np.abs(logits))
+        at = len(prompts[i])
+        for layer in range(layers):
+            for got, want in zip(sessions[i].kv_range(layer, at, 3), solo.kv_range(layer, at, 3)):
+                tol = 2e-3 if layer == 0 else E2E_REL_L2
+                assert rel_l2(O.decode16(dtype, got), O.decode16(dtype, want)) <= tol, (i, layer)
+    solo.destroy()
+    for s in sessions[::-1]:
+        s.destroy()
