@@ -228,6 +228,45 @@ void nv::destroy_session(Session *s) {
 
 namespace {
 
+// Sampling parameters of a session's own step: slot[position], cursor -> position + 1, the session's sampler.
+SamplerParams session_sampler(Session *s, const float *logits) {
+  SamplerParams sp{};
+  sp.logits = logits;
+  sp.vocab = s->vocab;
+  sp.config = s->sampler_dev;
+  sp.keys = s->sampler_keys;
+  sample_bind_workspace(sp.out, s->sample_ws);
+  sp.out.slots = s->slots;
+  sp.out.cursor_rw = s->state;
+  sp.out.fault = s->state + 3;
+  sp.cursor = s->state;
+  sp.max_steps = s->max_ctx;
+  return sp;
+}
+
+// The LM head of a step: final norm of the hidden row `x`, logits, one greedy candidate per workgroup.
+GemvParams head_launch(Session *s, const float *x) {
+  GemvParams p{};
+  p.w = s->lm_head;
+  p.xf = x;
+  p.gamma = s->final_norm;
+  p.out_f32 = s->logits;
+  p.rows = s->vocab;
+  p.cols = s->hidden;
+  p.eps = s->eps;
+  p.cursor = s->state;
+  p.max_steps = s->max_ctx;
+  p.sample = session_sampler(s, s->logits).out;
+  return p;
+}
+// The token of a step whose head has left its logits and `head_blocks` candidates.
+hipError_t head_sample(Session *s, const SampleParams &sample, uint32_t head_blocks) {
+  // greedy: one small workgroup reduces the per-workgroup candidates, writes slot[pos], bumps the cursor;
+  // else temperature sampling from the logits (two launches), then slot[pos] and the cursor likewise
+  if (s->sampler.mode == kSamplerGreedy) return launch_sample_finish(sample, head_blocks, s->state, s->max_ctx, s->stream);
+  return launch_sampler(session_sampler(s, s->logits), s->stream);
+}
+
 // Enqueue one step on the session stream (eagerly or under stream capture). With
 // `only` >= 0 just the per-layer launches of that kind are enqueued (profiling).
 hipError_t enqueue_step(Session *s, StepMode mode, StepProfiler *prof, int only = -1) {
@@ -386,39 +425,12 @@ hipError_t enqueue_step(Session *s, StepMode mode, StepProfiler *prof, int only 
     if (prof && err == hipSuccess) err = prof->after();
     return err;
   }
-  GemvParams p{};
-  p.w = s->lm_head;
-  p.xf = s->x;
-  p.gamma = s->final_norm;
-  p.out_f32 = s->logits;
-  p.rows = s->vocab;
-  p.cols = s->hidden;
-  p.eps = s->eps;
-  p.cursor = s->state;
-  p.max_steps = s->max_ctx;
-  sample_bind_workspace(p.sample, s->sample_ws);
-  p.sample.slots = s->slots;
-  p.sample.cursor_rw = s->state;
-  p.sample.fault = s->state + 3;
+  GemvParams p = head_launch(s, s->x);
   p.x16_dump = snap_slot(static_cast<uint64_t>(s->hidden) * sizeof(uint16_t));
   uint32_t head_blocks = 0;  // workgroups of the LM-head launch = candidates it leaves
   NV_STEP(kLHead, launch_gemv(s->dtype, kProRmsNorm, kEpiArgmax, p, st, nullptr, &head_blocks));
   snap(s->logits, static_cast<uint64_t>(s->vocab) * sizeof(float));
-  if (s->sampler.mode == kSamplerGreedy) {
-    // one small workgroup reduces the per-workgroup candidates, writes slot[pos], bumps the cursor
-    NV_STEP(kLAdvance, launch_sample_finish(p.sample, head_blocks, s->state, s->max_ctx, st));
-  } else {
-    // temperature sampling from the logits (two launches), then slot[pos] and the cursor as above
-    SamplerParams sp{};
-    sp.logits = s->logits;
-    sp.vocab = s->vocab;
-    sp.config = s->sampler_dev;
-    sp.keys = s->sampler_keys;
-    sp.out = p.sample;
-    sp.cursor = s->state;
-    sp.max_steps = s->max_ctx;
-    NV_STEP(kLAdvance, launch_sampler(sp, st));
-  }
+  NV_STEP(kLAdvance, head_sample(s, p.sample, head_blocks));
 #undef NV_STEP
   return hipSuccess;
 }
@@ -625,13 +637,48 @@ uint32_t block_operand_tiles(const Session *s, uint32_t tokens) {
   return operand || !s->rows_plain ? gemm_packed_tiles(tokens) : 0u;
 }
 
+// The final norm and the LM head on rows row .. row + count - 1 of the block whose layers have run: logits of all of
+// them, side by side in s->blogits (count <= NERVA_HIP_BATCH_MAX_BLOCK_TOKENS, through one stream of the head).
+hipError_t head_rows(Session *s, uint32_t row, uint32_t count, NervaHipHfDecodeSequenceResult *out) {
+  const float *x = s->px + static_cast<uint64_t>(row) * s->hidden;
+  out->kernel_launches += count == 1 ? 1 : 2;
+  if (count == 1) {
+    GemvParams p{};
+    p.w = s->lm_head;
+    p.xf = x;
+    p.gamma = s->final_norm;
+    p.out_f32 = s->blogits;
+    p.rows = s->vocab;
+    p.cols = s->hidden;
+    p.eps = s->eps;
+    return launch_gemv(s->dtype, kProRmsNorm, kEpiF32, p, s->stream);
+  }
+  const uint32_t tiles = block_operand_tiles(s, count);
+  hipError_t err = launch_rmsnorm_rows(s->dtype, x, s->final_norm, s->eps, count, s->hidden, s->pxn16, s->stream, tiles);
+  if (err != hipSuccess) return err;
+  GemmRowsParams g{};
+  g.tokens = count;
+  g.w = s->lm_head;
+  g.x16 = s->pxn16;
+  g.x_packed = tiles;
+  g.out_f32 = s->blogits;
+  g.rows = s->vocab;
+  g.cols = s->hidden;
+  g.workspace = s->pgemm_ws;
+  g.workspace_bytes = s->pgemm_ws_bytes;
+  return launch_gemm_rows(s->dtype, kGemmF32, g, s->stream);
+}
+
 // Prompt tokens begin .. count-1 through every layer in blocks of up to prefill_block_tokens tokens, with the
 // prompt staging (16-bit hidden state between layers, prefill_kernels.cu:494-508): per block and
 // layer one RMSNorm launch, the qkv projection as a multi-row GEMM, the K/V rows of the block into the
 // cache, the attention of all its tokens in one launch (token z attends to keys 0 .. first + z), and
-// the o / gate-up / down projections as multi-row GEMMs. Leaves the cursor at `count`. The reference
+// the o / gate-up / down projections as multi-row GEMMs. Leaves the device's cursor at `cursor`. The reference
 // prefills in chunks too (session_decode_prefill.inc.cu:1879-2243).
-hipError_t prefill_blocks(Session *s, uint32_t begin, uint32_t count, uint32_t prompt_count, NervaHipHfDecodeSequenceResult *out) {
+// `wanted`, optional: places (relative to `begin`, ascending) whose logits go to host rows of `logits` as their block is
+// done.
+hipError_t prefill_blocks(Session *s, uint32_t begin, uint32_t count, uint32_t cursor, uint32_t prompt_count, const uint32_t *wanted,
+                          uint32_t wanted_count, float *logits, NervaHipHfDecodeSequenceResult *out) {
   hipStream_t st = s->stream;
   const uint32_t H = s->hidden, A = s->heads * s->head_dim, KV = s->kv_heads * s->head_dim, I = s->intermediate;
   const float *rope_freq = s->theta > 0.0f ? s->rope_freq : nullptr;
@@ -769,9 +816,22 @@ hipError_t prefill_blocks(Session *s, uint32_t begin, uint32_t count, uint32_t p
       }
     }
     if (err == hipSuccess) out->kernel_launches += 1 + (rows_attention ? 9ull : 10ull) * s->layers;
+    while (err == hipSuccess && wanted_count != 0 && begin + *wanted < first + T) {
+      // a run of wanted places side by side
+      uint32_t run = 1;
+      while (run < wanted_count && run < NERVA_HIP_BATCH_MAX_BLOCK_TOKENS && wanted[run] == wanted[0] + run && begin + wanted[run] < first + T) ++run;
+      err = head_rows(s, begin + *wanted - first, run, out);
+      s->head_run = run;
+      if (err == hipSuccess)
+        err = hipMemcpyAsync(logits, s->blogits, static_cast<uint64_t>(run) * s->vocab * sizeof(float), hipMemcpyDeviceToHost, st);
+      out->d2h_bytes += static_cast<uint64_t>(run) * s->vocab * sizeof(float);
+      logits += static_cast<uint64_t>(run) * s->vocab;
+      wanted += run;
+      wanted_count -= run;
+    }
   }
   if (err == hipSuccess) {
-    hipLaunchKernelGGL(set_state_kernel, dim3(1), dim3(64), 0, st, s->state, count, prompt_count, 0u);
+    hipLaunchKernelGGL(set_state_kernel, dim3(1), dim3(64), 0, st, s->state, cursor, prompt_count, 0u);
     err = hipGetLastError();
     out->kernel_launches += 1;
   }
@@ -824,17 +884,56 @@ hipError_t set_device_position(Session *s, uint32_t cursor, uint32_t prompt_coun
 namespace {
 
 // Prompt tokens begin .. end-1 (already in s->prompt, the cursor at `begin`), the last one with the head and the
-// sampler: blocks where the model has them, else one captured prompt step per token.
-hipError_t prompt_tokens(Session *s, uint32_t begin, uint32_t end, NervaHipHfDecodeSequenceResult *out) {
+// sampler: blocks where the model has them, else one captured prompt step per token. `wanted`, `logits` as in
+// prefill_blocks; only with blocks, and all of them end up on the host in stream order.
+hipError_t prompt_tokens(Session *s, uint32_t begin, uint32_t end, const uint32_t *wanted, uint32_t wanted_count, float *logits,
+                         NervaHipHfDecodeSequenceResult *out) {
   if (s->stack != nullptr) return stack_prompt(s, begin, end, nullptr, 0, nullptr, nullptr, out);
   hipError_t err = hipSuccess;
-  if (s->block_prefill) {
-    if (end - begin > 1) err = prefill_blocks(s, begin, end - 1, end, out);
-  } else {
+  const uint32_t n = end - begin, last = n - 1;   // (place of the last token)
+  // (with the hook for the error path of the decode attention's merge on, the last token takes a decode step: it is there
+  // that the hook acts first)
+  if (!s->block_prefill) {
     for (uint32_t i = begin; err == hipSuccess && i + 1 < end; ++i) err = launch_step(s, 1, out);
+  } else if (n % s->prefill_block_tokens != 1 && tuning(kTuneAttnWithholdSplit) == 0) {
+    // every token in blocks; the head then reads the last one's row. With the place before it wanted too, its logits come
+    // with the others' through one stream of the head, and the sampler reads them there.
+    const bool with_others = wanted_count > 1 && wanted[wanted_count - 1] == last && wanted[wanted_count - 2] + 1 == last &&
+                             last % s->prefill_block_tokens != 0;
+    const uint32_t ahead = wanted_count != 0 && wanted[wanted_count - 1] == last && !with_others ? wanted_count - 1 : wanted_count;
+    err = prefill_blocks(s, begin, end, end - 1, end, wanted, ahead, logits, out);
+    if (err != hipSuccess) return err;
+    if (with_others) {
+      // (the last run of rows ends with it: prefill_blocks has just computed that run)
+      err = hipMemcpyAsync(s->logits, s->blogits + static_cast<uint64_t>(s->head_run - 1) * s->vocab, s->vocab * sizeof(float),
+                           hipMemcpyDeviceToDevice, s->stream);
+      if (err == hipSuccess) err = launch_sampler(session_sampler(s, s->logits), s->stream);
+      out->kernel_launches += 2;
+      return err;
+    }
+    const GemvParams p = head_launch(s, s->px + static_cast<uint64_t>(last % s->prefill_block_tokens) * s->hidden);
+    uint32_t head_blocks = 0;
+    err = launch_gemv(s->dtype, kProRmsNorm, kEpiArgmax, p, s->stream, nullptr, &head_blocks);
+    if (err == hipSuccess) err = head_sample(s, p.sample, head_blocks);
+    out->kernel_launches += s->sampler.mode == kSamplerGreedy ? 2 : 3;
+    if (err == hipSuccess && ahead != wanted_count) {
+      err = hipMemcpyAsync(logits + static_cast<uint64_t>(ahead) * s->vocab, s->logits, s->vocab * sizeof(float), hipMemcpyDeviceToHost,
+                           s->stream);
+      out->d2h_bytes += s->vocab * sizeof(float);
+    }
+    return err;
+  } else if (n > 1) {   // whole blocks and one token, which a step of its own serves at the cost of a weight stream either way
+    const uint32_t ahead = wanted_count != 0 && wanted[wanted_count - 1] == last ? wanted_count - 1 : wanted_count;
+    err = prefill_blocks(s, begin, end - 1, end - 1, end, wanted, ahead, logits, out);
+    logits += static_cast<uint64_t>(ahead) * s->vocab;
+    wanted_count -= ahead;
   }
   if (err == hipSuccess) err = enqueue_step(s, kPromptHeadStep, nullptr);
   if (err == hipSuccess) out->kernel_launches += step_launches(s, 0);
+  if (err == hipSuccess && wanted_count != 0) {
+    err = hipMemcpyAsync(logits, s->logits, s->vocab * sizeof(float), hipMemcpyDeviceToHost, s->stream);
+    out->d2h_bytes += s->vocab * sizeof(float);
+  }
   return err;
 }
 
@@ -906,10 +1005,10 @@ hipError_t setup_state(Session *s, int32_t *failure_stage, bool with_weights) {
                     gemm_rows_takes(kGemmSwiglu, s->intermediate, s->hidden, kGemmMaxTokens, 0) &&
                     gemm_rows_takes(kGemmResidual, s->hidden, s->intermediate, kGemmMaxTokens, 0);
   }
+  const bool head_block = s->rows_ready && gemm_rows_takes(kGemmF32, s->vocab, s->hidden, NERVA_HIP_BATCH_MAX_BLOCK_TOKENS, 0);
   // (a batch of sequences of a model with less than 6 MiB of weights a layer runs the sequences' own steps)
-  const bool batch_head = s->rows_ready && (A + KV) * H * 2 + 3 * H * I >= (3u << 20) &&
-                          gemm_rows_takes(kGemmF32, s->vocab, s->hidden, NERVA_HIP_BATCH_MAX_BLOCK_TOKENS, 0);
-  const uint64_t off_blogits = batch_head ? c.take(static_cast<uint64_t>(NERVA_HIP_BATCH_MAX_BLOCK_TOKENS) * V * 4) : 0;
+  s->batch_ready = head_block && (A + KV) * H * 2 + 3 * H * I >= (3u << 20);
+  const uint64_t off_blogits = head_block ? c.take(static_cast<uint64_t>(NERVA_HIP_BATCH_MAX_BLOCK_TOKENS) * V * 4) : 0;
   const uint64_t off_btable = c.take(sizeof(BatchTable));
   const uint64_t off_bslots = c.take(static_cast<uint64_t>(NERVA_HIP_BATCH_MAX_BLOCK_TOKENS) * sizeof(Slot));
   s->state_bytes = c.offset;
@@ -963,7 +1062,7 @@ hipError_t setup_state(Session *s, int32_t *failure_stage, bool with_weights) {
   const bool wide = block_cap != 128 && tuning(kTuneBlockLayout) != 1 && all_four(kGemmMaxTokens + 1) && all_four(kGemmWideMaxTokens);
   const bool deep = wide && block_cap != 256 && all_four(kGemmWideMaxTokens + 1) && all_four(kGemmDeepMaxTokens);
   s->prefill_block_tokens = deep ? kGemmDeepMaxTokens : wide ? kGemmWideMaxTokens : kGemmMaxTokens;
-  s->blogits = batch_head ? reinterpret_cast<float *>(s->arena + off_blogits) : nullptr;
+  s->blogits = head_block ? reinterpret_cast<float *>(s->arena + off_blogits) : nullptr;
   s->btable = reinterpret_cast<BatchTable *>(s->arena + off_btable);
   s->bslots = reinterpret_cast<Slot *>(s->arena + off_bslots);
   // ("prefill_walk" override = 1, read here: one prompt step per token where prompt blocks would be possible)
@@ -1689,7 +1788,7 @@ int nerva_hip_hf_decode_sequence_batch_advance_one(const NervaHipHfDecodeSequenc
     err = hipStreamSynchronize(seqs[t]->stream);
     out->sync_calls += 1;
   }
-  const bool shared = lead->rows_ready && lead->blogits != nullptr;
+  const bool shared = lead->batch_ready;
   if (err == hipSuccess && shared) {
     err = hipEventRecord(lead->ev0, lead->stream);
     if (err == hipSuccess) err = enqueue_batch_step(lead, seqs, T, out);
@@ -1830,7 +1929,7 @@ int nerva_hip_hf_decode_sequence_session_start(const NervaHipHfDecodeSequenceSes
   // else one captured prompt step per token), then one prompt step with the LM head and sampler
   if (err == hipSuccess && P > 1 && s->stack == nullptr && !s->block_prefill) err = ensure_graph(s, 1, out);
   if (err == hipSuccess) err = hipEventRecord(s->ev0, s->stream);
-  if (err == hipSuccess) err = prompt_tokens(s, 0, P, out);
+  if (err == hipSuccess) err = prompt_tokens(s, 0, P, nullptr, 0, nullptr, out);
   if (err == hipSuccess) err = hipEventRecord(s->ev1, s->stream);
   if (err != hipSuccess) {
     out->hip_error = static_cast<int32_t>(err);
@@ -1900,13 +1999,15 @@ int nerva_hip_session_extend(const NervaHipSessionExtendRequest *request, NervaH
   } else if (s->stack != nullptr) {
     if (err == hipSuccess)
       err = stack_prompt(s, begin, end, request->wanted, request->wanted_count, request->logits, request->residuals, out);
+  } else if (s->block_prefill && (request->wanted_count == 0 || s->blogits != nullptr)) {
+    if (err == hipSuccess) err = prompt_tokens(s, begin, end, request->wanted, request->wanted_count, request->logits, out);
   } else {
     if (err == hipSuccess && !s->block_prefill) err = ensure_graph(s, 1, out);
     // runs of tokens that end at a wanted place (or at the end), each with the head on its last token
     uint32_t at = 0;
     for (uint32_t i = 0; err == hipSuccess && at < n; ++i) {
       const uint32_t stop = i < request->wanted_count ? request->wanted[i] + 1 : n;
-      if (stop > at) err = prompt_tokens(s, begin + at, begin + stop, out);
+      if (stop > at) err = prompt_tokens(s, begin + at, begin + stop, nullptr, 0, nullptr, out);
       if (err == hipSuccess && stop < end - begin) err = set_device_position(s, begin + stop, end, 0);
       if (err == hipSuccess && i < request->wanted_count) logits_out(i);
       at = stop;
@@ -2271,7 +2372,7 @@ int nerva_hip_session_profile_step(NervaHipHfDecodeSequenceSession *s, uint32_t 
 
 int nerva_hip_session_shares_weight_stream(NervaHipHfDecodeSequenceSession *s) {
   if (s == nullptr) return -1;
-  return s->rows_ready && s->blogits != nullptr ? 1 : 0;
+  return s->batch_ready ? 1 : 0;
 }
 
 int nerva_hip_steps_are_eager(void) { return eager_steps() ? 1 : 0; }

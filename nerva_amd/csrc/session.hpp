@@ -89,7 +89,9 @@ struct NervaHipHfDecodeSequenceSession {
   // the multi-row kernels take this model's shapes (prompt blocks and batch steps need it)
   bool rows_ready = false;
   bool rows_plain = false;           // ... also for rows as they come, without matrix-operand order
-  float *blogits = nullptr;          // [NERVA_HIP_BATCH_MAX_BLOCK_TOKENS][vocab] logits of a batch step
+  bool batch_ready = false;          // batch steps stream the weights once for all sequences
+  float *blogits = nullptr;          // [NERVA_HIP_BATCH_MAX_BLOCK_TOKENS][vocab] logits of a batch step, or of rows of a prompt block
+  uint32_t head_run = 0;             // rows of the last of the latter
   nv::BatchTable *btable = nullptr, *host_btable = nullptr;
   nv::Slot *bslots = nullptr, *host_bslots = nullptr;   // a batch step's published slots, gathered for one copy
   float *px = nullptr, *pr = nullptr, *pqkv = nullptr, *prope = nullptr;
