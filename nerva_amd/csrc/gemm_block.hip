@@ -951,14 +951,30 @@ inline uint32_t deep_slices_for(int epilogue, uint32_t rows, uint32_t cols, int 
   while (slices > 1 && static_cast<uint64_t>(slices) * kDTokCap * wrows * sizeof(float) > workspace_bytes) slices /= 2u;
   return slices;
 }
+// Estimated times of a launch of these kernels and of the launch that adds its partial sums: rounds of 256 workgroups,
+// each 5 us and so much a K-block - 1.5 us for 64 columns of 256 rows x 256 tokens, 1.3 for 192 rows, 2.05 and 1.75 us
+// for 128 columns of the four and three wave pairs above - and for the partial sums 4 us and a read at 5 TB/s.
+inline double rounds_us(uint32_t workgroups, uint32_t blocks, double block_us) {
+  return ((workgroups + 255u) / 256u) * (5.0 + block_us * blocks);
+}
+inline double partials_us(uint32_t wrows, uint32_t tokens, uint32_t kslices) {
+  return kslices > 1 ? 4.0 + 4.0 * kslices * tokens * wrows / 5e6 : 0.0;
+}
+inline double deep_us(int epilogue, uint32_t rows, uint32_t cols, uint32_t tokens, const DeepPlan &plan) {
+  const uint32_t groups = (rows + deep_wg_rows(epilogue, plan.tpw) - 1) / deep_wg_rows(epilogue, plan.tpw);
+  return rounds_us(groups * ((tokens + 255u) / 256u) * plan.kslices, (cols / kDK + plan.kslices - 1) / plan.kslices,
+                   plan.tpw == 4 ? 1.5 : 1.3) +
+         partials_us(rows, tokens, plan.kslices);
+}
+
 // Shapes that divide (rows into workgroups, K into pairs of blocks) of more than 256 token rows: the tile height whose
-// busiest CU has the least to do - rounds of 256 workgroups x rows a workgroup x columns a slice. Other shapes, and blocks
-// of 129..256 rows that the kernel with wave pairs does not take: the tile height and the K slices (any number: a slice
-// is a run of whole K-blocks) of the shortest estimate - 1.5 us a CU for 256 rows x 256 tokens x 64 columns, and for
-// partial sums 4 us and their way to memory and back at 4 TB/s.
+// busiest CU has the least to do - rounds of 256 workgroups x rows a workgroup x columns a slice. Other shapes and smaller
+// blocks, and those where it is clearly ahead (512 rows of 3584 x 18944, whose K halves twice into pairs of blocks: 112
+// workgroups in 4 slices, 224 in 8): the tile height and the K slices - any number, a slice is a run of whole K-blocks - of
+// the shortest estimate.
 inline DeepPlan deep_plan(int epilogue, uint32_t rows, uint32_t cols, uint32_t tokens, uint64_t workspace_bytes) {
-  DeepPlan best{0, 0};
-  if (tokens <= kBTokCap || tokens > kDTokCap || cols % kDK != 0 || rows % 8u != 0) return best;
+  DeepPlan even{0, 0};
+  if (tokens <= kBTokCap || tokens > kDTokCap || cols % kDK != 0 || rows % 8u != 0) return even;
   if (tokens > kWTokCap && cols % (2u * kDK) == 0) {
     uint64_t best_cost = ~uint64_t{0};
     for (int tpw = 4; tpw >= 3; --tpw) {
@@ -968,26 +984,26 @@ inline DeepPlan deep_plan(int epilogue, uint32_t rows, uint32_t cols, uint32_t t
       const uint64_t cost = (wgs + 255u) / 256u * deep_wg_rows(epilogue, tpw) * (cols / slices);
       if (cost < best_cost) {
         best_cost = cost;
-        best = DeepPlan{tpw, slices};
+        even = DeepPlan{tpw, slices};
       }
     }
-    if (best.tpw != 0) return best;
+    if (even.tpw != 0 && tuning(kTuneGemmBlockSlices) > 0) return even;
   }
-  const uint32_t halves = (tokens + 255u) / 256u, blocks = cols / kDK;
-  double least = 0.0;
-  for (int tpw = 4; tpw >= 3; --tpw) {
-    const uint32_t groups = (rows + deep_wg_rows(epilogue, tpw) - 1) / deep_wg_rows(epilogue, tpw);
-    for (uint32_t slices = 1; slices <= 8u && slices * 2u <= blocks; ++slices) {
+  DeepPlan best{4, 1};
+  double least = deep_us(epilogue, rows, cols, tokens, best);
+  const auto consider = [&](const DeepPlan &plan) {
+    const double us = deep_us(epilogue, rows, cols, tokens, plan);
+    if (us < least) {
+      least = us;
+      best = plan;
+    }
+  };
+  for (int tpw = 4; tpw >= 3; --tpw)
+    for (uint32_t slices = 1; slices <= 8u && slices * 4u <= cols / kDK; ++slices) {
       if (slices > 1 && (epilogue == kGemmSwiglu || static_cast<uint64_t>(slices) * kDTokCap * rows * sizeof(float) > workspace_bytes)) break;
-      const double us = 0.375 * tpw * ((groups * halves * slices + 255u) / 256u) * ((blocks + slices - 1) / slices) +
-                        (slices > 1 ? 4.0 + 8.0 * slices * tokens * rows / 4e6 : 0.0);
-      if (best.tpw == 0 || us < least) {
-        least = us;
-        best = DeepPlan{tpw, slices};
-      }
+      consider(DeepPlan{tpw, slices});
     }
-  }
-  if (best.tpw == 0) best = DeepPlan{4, 1};   // a single K-block
+  if (even.tpw != 0 && deep_us(epilogue, rows, cols, tokens, even) * 0.9 <= least) return even;
   return best;
 }
 
@@ -1115,6 +1131,7 @@ GemmBlockPlan gemm_block_plan(int epilogue, uint32_t rows, uint32_t cols, uint32
   plan.row_tiles = tiles;
   plan.kslices = slices;
   plan.waves = waves;
+  plan.workgroups = groups * slices;
   return plan;
 }
 
@@ -1143,10 +1160,21 @@ uint32_t gemm_deep_slices(int epilogue, uint32_t rows, uint32_t cols, uint32_t t
   return deep_plan(epilogue, rows, cols, tokens, workspace_bytes).kslices;
 }
 
+double gemm_wide_us(int epilogue, uint32_t rows, uint32_t cols, uint32_t tokens, uint32_t kslices) {
+  const int pairs = wide_pairs(epilogue, rows);
+  const uint32_t wg_rows = wide_wg_rows(epilogue, pairs);
+  return rounds_us(rows / wg_rows * kslices, cols / kBK / kslices, pairs == 4 ? 2.05 : 1.75) +
+         partials_us(epilogue == kGemmSwiglu ? 2u * rows : rows, tokens, kslices);
+}
+
+double gemm_deep_us(int epilogue, uint32_t rows, uint32_t cols, uint32_t tokens, uint64_t workspace_bytes) {
+  return deep_us(epilogue, rows, cols, tokens, deep_plan(epilogue, rows, cols, tokens, workspace_bytes));
+}
+
 uint32_t gemm_rows_partial_slices(uint32_t rows, uint32_t cols, uint32_t tokens, uint32_t x_packed, uint64_t workspace_bytes,
                                   uint32_t *slice_stride) {
   if (x_packed == 0 || tokens > kBTokCap) return 0;
-  const uint32_t slices = gemm_block_plan(kGemmF32, rows, cols, tokens, workspace_bytes).kslices;
+  const uint32_t slices = gemm_rows_route(kGemmF32, rows, cols, tokens, workspace_bytes).kslices;   // (stride of either kernel's)
   if (slice_stride != nullptr) *slice_stride = kBTokCap * rows;
   return slices >= 2 && slices <= 4 ? slices : 0;
 }
@@ -1155,15 +1183,8 @@ bool gemm_rows_fuses_norm(int epilogue, uint32_t rows, uint32_t cols, uint32_t t
   if (epilogue != kGemmResidual || x_packed == 0 || rows % 4 != 0 ||
       rows > static_cast<uint32_t>(kFinNormThreads * kFinNormPerLane * 4))
     return false;
-  // wherever a launch of its own adds the K slices: the deep or the wide kernel's, or the shared-X kernel's for smaller blocks
-  if (tokens > kWTokCap) return gemm_deep_slices(epilogue, rows, cols, tokens, workspace_bytes) > 1;
-  if (tokens > kBTokCap) {
-    const uint32_t wide = gemm_wide_slices(epilogue, rows, cols, tokens, workspace_bytes);
-    return (wide != 0 ? wide : gemm_deep_slices(epilogue, rows, cols, tokens, workspace_bytes)) > 1;
-  }
-  const uint32_t block = gemm_block_plan(epilogue, rows, cols, tokens, workspace_bytes).kslices;
-  if (block != 0 || gemm_rows_supported(rows, cols, tokens)) return block > 1;
-  return gemm_flow_plan(epilogue, rows, cols, tokens, workspace_bytes).kslices > 1;
+  // wherever a launch of its own adds the K slices
+  return gemm_rows_route(epilogue, rows, cols, tokens, workspace_bytes).kslices > 1;
 }
 
 uint64_t gemm_block_workspace_bytes(uint32_t rows_max) {

@@ -1,6 +1,6 @@
 // Multi-row projection for token blocks of up to 128 rows (X in matrix-operand order) of any number of weight rows and
-// any K that is a multiple of 32: the shapes whose K does not divide into the rings of gemm_block.hip (a width of 2560,
-// 3584 or 5120, a feed-forward of 9728 or 18944, a vocabulary of any size).
+// any K that is a multiple of 32: the shapes whose K does not divide into the rings of gemm_block.hip (a width of 896 or
+// 1344, a vocabulary of any size), or not into enough slices of them (a feed-forward of 9728 or 18944).
 //
 // What bounds it is the weight stream, so a workgroup keeps as much of it in flight as LDS holds: the K-blocks of 64
 // columns - 64 RT weight rows of 128 bytes and the block's X pieces - go from global memory straight into a ring of
@@ -238,19 +238,23 @@ hipError_t launch_flow_dt(int epilogue, const GemmRowsParams &p, const GemmFlowP
 
 }  // namespace
 
-// Two row tiles a wave where that still gives most CUs two workgroups, K slices until the launch has about two a CU;
-// a slice keeps at least four K-blocks (its pipeline has to fill), and the partial sums fit the workspace.
+// K slices until every CU has a workgroup and no further (what is left over from a second round costs more than it
+// spreads: 2 rows of 5120 x 5120 in 3 / 4 / 6 slices of 80 row groups 15.0 / 18.4 / 15.9 us, of 2560 x 9728 in 4 / 6 / 8
+// slices of 40 17.2 / 14.5 / 18.1), each of at least eight K-blocks (its pipeline has to fill: 4096 x 1024 in 1 / 2 / 4
+// slices 7.0 / 7.3 / 6.8 us, 11 and 12 us at 128 rows), the partial sums within the workspace. Two row tiles a wave only
+// for a gate/up pair and for heads of so many rows that every CU still has three rounds of workgroups.
 GemmFlowPlan gemm_flow_plan(int epilogue, uint32_t rows, uint32_t cols, uint32_t tokens, uint64_t workspace_bytes) {
   GemmFlowPlan plan{};
   if (tokens == 0 || tokens > kFTokCap || cols == 0 || cols % 32u != 0 || rows == 0 || (epilogue != kGemmF32 && rows % 4u != 0)) return plan;
   const uint32_t wrows = epilogue == kGemmSwiglu ? 2u * rows : rows;
-  plan.row_tiles = epilogue == kGemmSwiglu || rows >= 128u * 384u ? 2u : 1u;
+  plan.row_tiles = epilogue == kGemmSwiglu || rows >= 128u * 768u ? 2u : 1u;
   const uint32_t wg_rows = epilogue == kGemmSwiglu ? 64u : 64u * plan.row_tiles;
   const uint32_t groups = (rows + wg_rows - 1) / wg_rows, blocks = (cols + kFK - 1) / kFK;
-  uint32_t slices = rows % 4u != 0 ? 1u : std::max(1u, std::min({512u / groups, blocks / 4u, 8u}));
+  uint32_t slices = rows % 4u != 0 ? 1u : std::max(1u, std::min({256u / groups, blocks / 8u, 8u}));
   const uint64_t one = static_cast<uint64_t>(kFTokCap) * wrows * sizeof(float);
   if (slices > 1 && slices * one > workspace_bytes) slices = std::max<uint32_t>(1u, static_cast<uint32_t>(workspace_bytes / one));
   plan.kslices = slices;
+  plan.workgroups = groups * slices;
   return plan;
 }
 
@@ -260,7 +264,7 @@ hipError_t launch_gemm_flow(uint32_t dtype, int epilogue, const GemmRowsParams &
   hipError_t err = dtype == kBF16  ? launch_flow_dt<kBF16>(epilogue, p, plan, stream)
                    : dtype == kF16 ? launch_flow_dt<kF16>(epilogue, p, plan, stream)
                                    : hipErrorInvalidValue;
-  if (err == hipSuccess && plan.kslices > 1)
+  if (err == hipSuccess && plan.kslices > 1 && !(epilogue == kGemmF32 && p.keep_partials != 0))
     err = launch_gemm_finish(dtype, epilogue, p, static_cast<const float *>(p.workspace), plan.kslices, kFTokCap, stream);
   return err;
 }

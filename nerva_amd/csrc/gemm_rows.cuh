@@ -77,9 +77,16 @@ struct GemmRowsParams {
 // multiple of 16 a residual must not be added in place), cols % 2048 == 0 (each of the 8 waves walks
 // whole 256-column blocks), 1 <= tokens <= kGemmMaxTokens, 16-byte aligned w and x16.
 bool gemm_rows_supported(uint32_t rows, uint32_t cols, uint32_t tokens);
-// Whether launch_gemm_rows takes a block of `tokens` rows in operand order (what gemm_rows_supported says, in any layout
-// with up to kGemmMaxTokens rows; else one of the kernels below).
-bool gemm_rows_takes(int epilogue, uint32_t rows, uint32_t cols, uint32_t tokens, uint64_t workspace_bytes);
+// The kernel a block of `tokens` rows in operand order goes to, and its K slices (kGemmNone: not taken).
+enum GemmKernel : int { kGemmNone = 0, kGemmWaves, kGemmBlock, kGemmFlow, kGemmWide, kGemmDeep };
+struct GemmRoute {
+  GemmKernel kernel;
+  uint32_t kslices;
+};
+GemmRoute gemm_rows_route(int epilogue, uint32_t rows, uint32_t cols, uint32_t tokens, uint64_t workspace_bytes);
+inline bool gemm_rows_takes(int epilogue, uint32_t rows, uint32_t cols, uint32_t tokens, uint64_t workspace_bytes) {
+  return gemm_rows_route(epilogue, rows, cols, tokens, workspace_bytes).kernel != kGemmNone;
+}
 hipError_t launch_gemm_rows(uint32_t dtype, int epilogue, const GemmRowsParams &p, hipStream_t stream);
 
 // Blocks of more than 64 token rows with X in operand order: the kernel that shares the X operand through
@@ -88,6 +95,7 @@ hipError_t launch_gemm_rows(uint32_t dtype, int epilogue, const GemmRowsParams &
 // itself where the plan allows.
 struct GemmBlockPlan {
   uint32_t row_tiles, kslices, waves;
+  uint32_t workgroups;
 };
 GemmBlockPlan gemm_block_plan(int epilogue, uint32_t rows, uint32_t cols, uint32_t tokens, uint64_t workspace_bytes);
 // K slices (2..4) whose partial sums a plain projection of this shape can leave to its reader (keep_partials), with
@@ -103,15 +111,18 @@ hipError_t launch_gemm_block(uint32_t dtype, int epilogue, const GemmRowsParams 
 // (rows a multiple of 128, gate/up pairs of 64; cols a multiple of 512 per slice). launch_gemm_rows uses it by itself.
 uint32_t gemm_wide_slices(int epilogue, uint32_t rows, uint32_t cols, uint32_t tokens, uint64_t workspace_bytes);
 hipError_t launch_gemm_wide(uint32_t dtype, int epilogue, const GemmRowsParams &p, uint32_t kslices, hipStream_t stream);
+// Estimated time of that launch (gemm_rows_route), and of the one below.
+double gemm_wide_us(int epilogue, uint32_t rows, uint32_t cols, uint32_t tokens, uint32_t kslices);
+double gemm_deep_us(int epilogue, uint32_t rows, uint32_t cols, uint32_t tokens, uint64_t workspace_bytes);
 // Blocks of 129..kGemmDeepMaxTokens rows in operand order: the same for the kernel that takes 256 or 192 rows x 256
-// tokens per workgroup (rows a multiple of 8, cols of 64). launch_gemm_rows uses it above kGemmWideMaxTokens rows, and
-// below where gemm_wide_slices does not take the shape.
+// tokens per workgroup (rows a multiple of 8, cols of 64).
 uint32_t gemm_deep_slices(int epilogue, uint32_t rows, uint32_t cols, uint32_t tokens, uint64_t workspace_bytes);
 hipError_t launch_gemm_deep(uint32_t dtype, int epilogue, const GemmRowsParams &p, uint32_t kslices, hipStream_t stream);
-// Blocks of up to kGemmMaxTokens rows in operand order whose shape neither kernel above takes (gemm_flow.hip): any number
+// Blocks of up to kGemmMaxTokens rows in operand order of any shape (gemm_flow.hip): any number
 // of rows (a multiple of 4 except for the plain epilogue), cols % 32 == 0. kslices 0: not taken.
 struct GemmFlowPlan {
   uint32_t row_tiles, kslices;
+  uint32_t workgroups;
 };
 GemmFlowPlan gemm_flow_plan(int epilogue, uint32_t rows, uint32_t cols, uint32_t tokens, uint64_t workspace_bytes);
 hipError_t launch_gemm_flow(uint32_t dtype, int epilogue, const GemmRowsParams &p, const GemmFlowPlan &plan, hipStream_t stream);

@@ -310,26 +310,42 @@ bool gemm_rows_supported(uint32_t rows, uint32_t cols, uint32_t tokens) {
   return rows >= 16 && cols != 0 && cols % (kGW * kKB) == 0 && tokens >= 1 && tokens <= kGemmMaxTokens;
 }
 
-bool gemm_rows_takes(int epilogue, uint32_t rows, uint32_t cols, uint32_t tokens, uint64_t workspace_bytes) {
-  if (tokens > kGemmMaxTokens)
-    return (tokens <= kGemmWideMaxTokens && gemm_wide_slices(epilogue, rows, cols, tokens, workspace_bytes) != 0) ||
-           gemm_deep_slices(epilogue, rows, cols, tokens, workspace_bytes) != 0;
-  return gemm_rows_supported(rows, cols, tokens) || gemm_flow_plan(epilogue, rows, cols, tokens, workspace_bytes).kslices != 0;
+// Up to kGemmMaxTokens rows: the kernel that shares X through LDS (gemm_block.hip) where its plan takes the shape, unless
+// its K slices - rings of 512 columns, a power of two of them - leave it well short of the workgroups that slices of any
+// length give (2 / 32 / 128 rows of 2560 x 9728: 39.2 / 39.5 / 59.4 us in 40 workgroups, 14.5 / 15.2 / 21.6 in 240;
+// of 5120 x 5120, 160 against 240: 15.8 / 16.7 / 24.0 against 15.0 / 15.5 / 22.4; at equal numbers the shared block is the
+// faster one: 7168 x 5120 17.1 / 17.7 / 25.6 against 18.6 / 19.2 / 28.8). A gate/up pair in slices writes and reads two
+// rows of partial sums per output and gains only up to 64 rows (8192 x 2048 pairs 16.7 / 16.6 / 25.6 against
+// 15.9 / 16.9 / 28.7).
+// More: the kernel with wave pairs or the one for 256-row tiles, whichever the estimate has clearly ahead.
+GemmRoute gemm_rows_route(int epilogue, uint32_t rows, uint32_t cols, uint32_t tokens, uint64_t workspace_bytes) {
+  if (tokens == 0) return GemmRoute{kGemmNone, 0};
+  if (tokens > kGemmMaxTokens) {
+    const uint32_t wide = tokens <= kGemmWideMaxTokens ? gemm_wide_slices(epilogue, rows, cols, tokens, workspace_bytes) : 0u;
+    const uint32_t deep = gemm_deep_slices(epilogue, rows, cols, tokens, workspace_bytes);
+    if (wide != 0 && (deep == 0 || gemm_deep_us(epilogue, rows, cols, tokens, workspace_bytes) >
+                                       0.9 * gemm_wide_us(epilogue, rows, cols, tokens, wide)))
+      return GemmRoute{kGemmWide, wide};
+    return deep != 0 ? GemmRoute{kGemmDeep, deep} : GemmRoute{kGemmNone, 0};
+  }
+  const GemmBlockPlan block = gemm_block_plan(epilogue, rows, cols, tokens, workspace_bytes);
+  const GemmFlowPlan flow = gemm_flow_plan(epilogue, rows, cols, tokens, workspace_bytes);
+  if (block.kslices == 0 && gemm_rows_supported(rows, cols, tokens)) return GemmRoute{kGemmWaves, 1};
+  const bool forced = tuning(kTuneGemmBlockSlices) != 0 || tuning(kTuneGemmBlockRowTiles) != 0;
+  const bool short_of = block.workgroups * 5u < flow.workgroups * 3u && !(epilogue == kGemmSwiglu && tokens > 64u) && !forced;
+  if (flow.kslices != 0 && (block.kslices == 0 || short_of)) return GemmRoute{kGemmFlow, flow.kslices};
+  if (block.kslices == 0) return GemmRoute{kGemmNone, 0};
+  return GemmRoute{kGemmBlock, block.kslices};
 }
 
 hipError_t launch_gemm_rows(uint32_t dtype, int epilogue, const GemmRowsParams &p, hipStream_t stream) {
-  // more than kGemmMaxTokens rows: only in operand order
+  // rows as they come: only the kernel of this file
   const uint64_t room = p.workspace != nullptr ? p.workspace_bytes : 0;
-  const uint32_t wide_slices = p.tokens > kGemmMaxTokens && p.tokens <= kGemmWideMaxTokens && p.x_packed != 0
-                                   ? gemm_wide_slices(epilogue, p.rows, p.cols, p.tokens, room)
-                                   : 0u;
-  const uint32_t deep_slices = p.tokens > kGemmMaxTokens && wide_slices == 0 && p.x_packed != 0
-                                   ? gemm_deep_slices(epilogue, p.rows, p.cols, p.tokens, room)
-                                   : 0u;
-  const bool streams = gemm_rows_supported(p.rows, p.cols, p.tokens);   // the kernels of this file and of gemm_block.hip
-  const GemmFlowPlan flow = p.x_packed != 0 && !streams ? gemm_flow_plan(epilogue, p.rows, p.cols, p.tokens, room) : GemmFlowPlan{};
+  GemmRoute route{kGemmNone, 0};
+  if (p.x_packed != 0) route = gemm_rows_route(epilogue, p.rows, p.cols, p.tokens, room);
+  else if (gemm_rows_supported(p.rows, p.cols, p.tokens)) route = GemmRoute{kGemmWaves, 1};
   if (p.w == nullptr || p.x16 == nullptr) return hipErrorInvalidValue;
-  if (wide_slices == 0 && deep_slices == 0 && flow.kslices == 0 && !streams) return hipErrorInvalidValue;
+  if (route.kernel == kGemmNone) return hipErrorInvalidValue;
   if (!aligned16(p.w) || !aligned16(p.x16)) return hipErrorInvalidValue;
   if ((epilogue == kGemmF32 || epilogue == kGemmResidual) && p.out_f32 == nullptr) return hipErrorInvalidValue;
   if (epilogue == kGemmResidual && p.residual == nullptr) return hipErrorInvalidValue;
@@ -349,12 +365,12 @@ hipError_t launch_gemm_rows(uint32_t dtype, int epilogue, const GemmRowsParams &
   if (p.norm_gamma != nullptr &&   // a fused norm only where the shape has one; never silently dropped
       (p.norm_out16 == nullptr || !gemm_rows_fuses_norm(epilogue, p.rows, p.cols, p.tokens, p.x_packed, p.workspace != nullptr ? p.workspace_bytes : 0)))
     return hipErrorInvalidValue;
-  if (deep_slices != 0) return launch_gemm_deep(dtype, epilogue, p, deep_slices, stream);
-  if (wide_slices != 0) return launch_gemm_wide(dtype, epilogue, p, wide_slices, stream);
-  if (p.x_packed != 0) {   // blocks in operand order: the kernel that shares X through LDS, where its plan takes the shape
-    const GemmBlockPlan plan = gemm_block_plan(epilogue, p.rows, p.cols, p.tokens, p.workspace != nullptr ? p.workspace_bytes : 0);
-    if (plan.kslices != 0) return launch_gemm_block(dtype, epilogue, p, plan, stream);
-    if (flow.kslices != 0) return launch_gemm_flow(dtype, epilogue, p, flow, stream);
+  switch (route.kernel) {
+    case kGemmDeep: return launch_gemm_deep(dtype, epilogue, p, route.kslices, stream);
+    case kGemmWide: return launch_gemm_wide(dtype, epilogue, p, route.kslices, stream);
+    case kGemmBlock: return launch_gemm_block(dtype, epilogue, p, gemm_block_plan(epilogue, p.rows, p.cols, p.tokens, room), stream);
+    case kGemmFlow: return launch_gemm_flow(dtype, epilogue, p, gemm_flow_plan(epilogue, p.rows, p.cols, p.tokens, room), stream);
+    default: break;
   }
   if (dtype == kBF16) return launch_dt<kBF16>(epilogue, p, stream);
   return launch_dt<kF16>(epilogue, p, stream);
