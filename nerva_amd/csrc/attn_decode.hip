@@ -122,15 +122,6 @@ __global__ __launch_bounds__(W *kWave, W / 2) void attn_block_kernel(AttnParams 
 // tokens that keeps 31 of 32 splits busy instead of 22 - and a wave without a tile simply contributes
 // nothing to the merge.
 // ---------------------------------------------------------------------------------------------
-// Loads through the scalar path (position, block-table entries: the same for every lane, and read-only
-// while the launch runs). The compiler takes the vector path for them - it cannot prove that the
-// launch does not write there - and a vector load would have to be awaited with everything requested
-// before it.
-__device__ __forceinline__ uint32_t sload(const uint32_t *ptr) {
-  uint32_t v;
-  asm volatile("s_load_dword %0, %1, 0x0\n\ts_waitcnt lgkmcnt(0)" : "=s"(v) : "s"(ptr) : "memory");
-  return v;
-}
 __device__ __forceinline__ void sload4(const uint32_t *p0, const uint32_t *p1, const uint32_t *p2, const uint32_t *p3,
                                        uint32_t (&v)[4]) {
   asm volatile(
@@ -362,7 +353,7 @@ __global__ __launch_bounds__(8 * kWave) void attn_step_kernel(AttnParams p) {
     phys[0] = mine[2], phys[1] = mine[3], phys[2] = mine[4], phys[3] = mine[5];
     if (pos >= p.max_steps) return;
   } else {
-    pos = p.cursor != nullptr ? sload(p.cursor) : p.position;
+    pos = p.cursor != nullptr ? scalar_load(p.cursor) : p.position;
     if (p.cursor != nullptr && pos >= p.max_steps) return;
     attn_split_geometry(pos, S, p.single_split_blocks, nblk, bps, active);
     first = split * bps + wave;
@@ -433,7 +424,7 @@ __global__ __launch_bounds__(8 * kWave) void attn_step_kernel(AttnParams p) {
   link_mark(tr, 9);
   if (owns_new && wave == W - 1) {
     // publish the rounded row to the cache in operand order
-    const uint64_t tile = kv_tile_offset(p.block_count, p.kv_heads, HD, p.layer, sload(p.table + new_block), kvh);
+    const uint64_t tile = kv_tile_offset(p.block_count, p.kv_heads, HD, p.layer, scalar_load(p.table + new_block), kvh);
     if (lane < HD / 8)  // K: pieces of 8 consecutive dims
       *reinterpret_cast<uint4 *>(p.k_cache + tile + kv_k_elem(HD, new_row, lane * 8)) =
           *reinterpret_cast<const uint4 *>(sh.knew + lane * 8);
@@ -474,7 +465,7 @@ __global__ __launch_bounds__(8 * kWave) void attn_step_kernel(AttnParams p) {
       const uint32_t bb = first + t_idx * W;                                                                       \
       attn_tile<DT, HD, G, false>(kk, vv, qx, nullptr, bb, n_keys, col, grp, owns_new && bb == new_block, new_row,     \
                               sh.knew, sh.vnew, m, l, acc);                                                        \
-      if (t_idx + 4u < nt) NV_AT_TILE_LOAD(F, sload(p.table + first + (t_idx + 4u) * W));                          \
+      if (t_idx + 4u < nt) NV_AT_TILE_LOAD(F, scalar_load(p.table + first + (t_idx + 4u) * W));                          \
     }                                                                                                              \
   } while (0)
   for (uint32_t done = 0; done < nt; done += 4) {

@@ -5,17 +5,24 @@
 // of the block itself are in the cache already (launch_kv_publish_rows), so token t simply attends to
 // keys 0 .. position + t.
 //
-// gfx950 mapping (head_dim 64 or 128, G = heads / kv_heads up to 8): the 16-column matrix-core tile
-// of the decode kernel holds the G query heads of ONE token as hi/lo column pairs and leaves the
-// rest of its columns empty; here a wave fills its 16 columns with (token, head) pairs - 16 / G tokens
-// of the kv head's G query heads - and the hi and lo halves of a query (and of a tile's probabilities) are
-// two products into the same accumulators (attn_tile_wide), with the causal limit n_keys chosen per column.
-// The 8 waves of a workgroup take 8 * 16 / G consecutive tokens and walk the SAME tiles: a tile (4 KiB of K,
-// 4 KiB of V) is requested once
-// by the workgroup - one 16-byte piece per lane - parked in LDS (two stages, one barrier per tile) and
-// read back by every wave as matrix operands. Grid (kv head, split of the prefix, token group); split
-// partials go to the per-token workspaces the decode kernel uses and a small second launch merges them.
+// gfx950 mapping (head_dim 64 or 128, G = heads / kv_heads up to 8): a wave fills two 16-column matrix-core tiles with
+// (token, head) pairs - 32 / G tokens of the kv head's G query heads - and the hi and lo halves of a query (and of a
+// step's probabilities) are two products into the same accumulators, with the causal limit n_keys chosen per column.
+// The 8 waves of a workgroup take 8 * 32 / G consecutive tokens and walk the SAME keys, 64 a step: the step's four K and
+// four V tiles (one each per wave) go from the cache straight into a ring of four LDS stages, two steps ahead.
+// What bounds it is the matrix cores and the exponentials beside them, so a step is laid out for both: 64 keys share one
+// running maximum, one rescale and one look at the mask (only steps that reach the diagonal have one), every K or V piece
+// read from LDS meets 32 columns, the product with V contracts over two tiles at once with the full-rate 32-deep
+// instruction - the operand order of the cache keeps a lane's four tokens of a tile side by side, so the pair's operand is
+// a choice of registers - and the two waves of a SIMD take turns: one multiplies while the other works on its
+// probabilities, kept half a step apart by two barriers a step. Against 16 keys a step, 16 columns a wave
+// and the 16-deep product, blocks of 512 tokens of 32 heads over contexts 512 to 8192: 111.8 -> 82.7 us a launch on
+// average (85.8 without the turns), 0.94 PFLOP/s with the hi and lo halves counted, where the products of the same block
+// reach 1.1.
+// Grid (kv head, split of the prefix, token group); split partials go to the per-token workspaces the decode kernel uses
+// and a small second launch merges them.
 #include <algorithm>
+#include <mutex>
 
 #include "attn_decode.cuh"
 #include "attn_tile.cuh"
@@ -26,23 +33,38 @@ namespace {
 
 using namespace attn;
 
-constexpr int kPW = 8;    // waves per workgroup
-constexpr int kVG = 16;   // (token, head) pairs per wave: one per column of the matrix-core tile
+constexpr int kPW = 8;                // waves per workgroup
+constexpr int kCols = 32;             // (token, head) pairs per wave: two column tiles
+constexpr uint32_t kStepBlocks = 4;   // cache blocks (16 keys) of a step
+constexpr int kStages = 4;
 
-// Split geometry of a token group, the same on both launches: tiles per split, active splits.
+// Split geometry of a token group, the same on both launches: blocks per split (whole steps), active splits.
 __device__ __forceinline__ void prompt_splits(uint32_t last_pos, uint32_t S, uint32_t &bps, uint32_t &active, uint32_t &nblk) {
   nblk = last_pos / kKvBlockTokens + 1;
-  bps = (nblk + S - 1) / S;
+  bps = ((nblk + S - 1) / S + kStepBlocks - 1) / kStepBlocks * kStepBlocks;
   active = (nblk + bps - 1) / bps;
 }
 
+constexpr uint32_t prompt_tile_bytes(int hd) { return kKvBlockTokens * hd * 2u; }
+constexpr uint32_t prompt_stage_bytes(int hd) { return 2u * kStepBlocks * prompt_tile_bytes(hd); }
+// (the f32 queries of sixteen columns a wave lie in the second and third stage until the walk begins)
+static_assert(kPW * 16 * 128 * sizeof(float) <= 2 * prompt_stage_bytes(128) && kPW * 16 * 64 * sizeof(float) <= 2 * prompt_stage_bytes(64),
+              "room for the queries");
+
+#define NV_PR_LDS(P) ((__attribute__((address_space(3))) void *)(P))
+
+// Operand reads, issued one group ahead of the products that use them and awaited by count: the awaited registers are
+// in/out operands of the wait, so that nothing that uses them can come before it.
+#define NV_PR_READ(DST, AT, OFF) asm volatile("ds_read_b128 %0, %1 offset:%2" : "=v"(DST) : "v"(AT), "n"(OFF) : "memory")
+#define NV_PR_AWAIT2(N_, A_, B_) asm volatile("s_waitcnt lgkmcnt(%2)" : "+v"(A_), "+v"(B_) : "n"(N_) : "memory")
+
 template <uint32_t DT, int HD, int G>
-__global__ __launch_bounds__(kPW *kWave) void attn_prompt_kernel(AttnParams p) {
-  constexpr int kTokensPerWave = kVG / G, kPairs = kTokensPerWave * G;   // (columns kPairs .. 15 repeat the last pair, unused)
+__global__ __launch_bounds__(kPW *kWave, 2) void attn_prompt_kernel(AttnParams p) {
+  constexpr int kTokensPerWave = kCols / G, kPairs = kTokensPerWave * G;   // (columns kPairs .. 31 repeat the last pair, unused)
   constexpr uint32_t kGroupTokens = kPW * kTokensPerWave;
-  constexpr int kPieces = HD / 32;               // 1 KiB pieces of a K tile, and of a V tile
-  __shared__ uint4 stage[2][2 * kPieces][kWave];   // K pieces, then V pieces of a tile, twice
-  __shared__ __align__(16) float q_s[kPW][kVG][HD];
+  constexpr int kPieces = HD / 32;               // 1 KiB pieces of a tile
+  constexpr uint32_t kTile = prompt_tile_bytes(HD), kStage = prompt_stage_bytes(HD);
+  extern __shared__ __align__(16) unsigned char smem[];
   const int lane = threadIdx.x & (kWave - 1);
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
   const uint32_t kvh = blockIdx.x, split = blockIdx.y, S = gridDim.y, T = p.tokens;
@@ -51,129 +73,270 @@ __global__ __launch_bounds__(kPW *kWave) void attn_prompt_kernel(AttnParams p) {
   uint32_t bps, active, nblk;
   prompt_splits(p.position + group_last, S, bps, active, nblk);
   if (split >= active) return;
-  const uint32_t b0 = split * bps, b1 = min(nblk, b0 + bps);
+  const uint32_t b0 = split * bps, steps = (min(nblk, b0 + bps) - b0 + kStepBlocks - 1) / kStepBlocks;
 
-  // the workgroup's first tile is on its way while the queries are prepared
-  // (at 64 dims four waves fetch a piece each; the others ask for the same ones and leave them)
-  const int my_piece = wave & (2 * kPieces - 1);
-  const uint16_t *cache = my_piece < kPieces ? p.k_cache : p.v_cache;
-  const uint32_t piece = (my_piece & (kPieces - 1)) * 512 + lane * 8;
-  auto tile_piece = [&](uint32_t b) {
-    return load_stream(cache + kv_tile_offset(p.block_count, p.kv_heads, HD, p.layer, p.table[b], kvh) + piece);
+  // this wave's tile of a step: K (even waves) or V of block wave / 2; blocks past the last are that one again, masked
+  const uint16_t *cache = (wave & 1) == 0 ? p.k_cache : p.v_cache;
+  auto request = [&](uint32_t step) {
+    const uint32_t block = min(b0 + step * kStepBlocks + (wave >> 1), nblk - 1);
+    const uint16_t *src = cache + kv_tile_offset(p.block_count, p.kv_heads, HD, p.layer, scalar_load(p.table + block), kvh) + lane * 8;
+    unsigned char *at = smem + (step % kStages) * kStage + wave * kTile;
+#pragma unroll
+    for (int i = 0; i < kPieces; ++i)
+      __builtin_amdgcn_global_load_lds(reinterpret_cast<const u32x4_t *>(src + i * 512), NV_PR_LDS(at + i * 1024), 16, 0, 0);
   };
-  uint4 inflight = tile_piece(b0);
+  request(0);   // on its way while the queries are prepared
 
-  // ---- this wave's eight (token, head) pairs: bias, norm, rotation -> f32 q in LDS
+  // ---- this wave's (token, head) pairs: bias, norm, rotation -> f32 q in LDS -> hi and lo operands
   const uint32_t wave_first = group_first + wave * kTokensPerWave;   // may lie past the block: clamped, never stored
-  // (every input of all eight requested first, unconditionally: one round trip instead of eight)
-  const bool has_bias = p.q_bias != nullptr, has_gamma = p.q_norm != nullptr, has_rope = p.rope_freq != nullptr;
-  const uint16_t *bias_base = has_bias ? p.q_bias : p.k_cache;    // any readable address when unused
-  const float *rope_base = has_rope ? p.rope_cs : p.qkv;
-  const uint32_t rope_stride = has_rope ? p.rope_token_stride : 0u;
-  const uint16_t *gamma_base = has_gamma ? p.q_norm : p.k_cache;
-  const int pl = pair_of<HD>(lane);
-  const float g0 = dec16<DT>(gamma_base[pl]), g1 = dec16<DT>(gamma_base[pl + HD / 2]);
-#pragma unroll
-  for (int part = 0; part < kVG / 8; ++part) {   // eight pairs at a time: their inputs in one round trip
-    float x0[8], x1[8], rc[8], rs[8];
-    uint16_t qb0[8], qb1[8];
-#pragma unroll
-    for (int i = 0; i < 8; ++i) {
-      const int vh = min(part * 8 + i, kPairs - 1);
-      const uint32_t tok = min(wave_first + vh / G, T - 1);
-      const uint32_t h = kvh * G + vh % G;
-      const float *src = p.qkv + static_cast<uint64_t>(tok) * p.qkv_token_stride + h * HD;
-      x0[i] = src[pl];
-      x1[i] = src[pl + HD / 2];
-      qb0[i] = bias_base[h * HD + pl];
-      qb1[i] = bias_base[h * HD + pl + HD / 2];
-      rc[i] = rope_base[static_cast<uint64_t>(tok) * rope_stride + pl];
-      rs[i] = rope_base[static_cast<uint64_t>(tok) * rope_stride + HD / 2 + pl];
-    }
-#pragma unroll
-    for (int i = 0; i < 8; ++i)
-      prep_head_core<DT, HD>(x0[i], x1[i], has_bias, dec16<DT>(qb0[i]), dec16<DT>(qb1[i]), has_gamma, g0, g1, has_rope,
-                            rc[i], rs[i], p.eps, lane, q_s[wave][part * 8 + i], nullptr);
-  }
-  __syncthreads();
-
   const int col = lane & 15, grp = lane >> 4;
-  const float scale = kLog2e / sqrtf(static_cast<float>(HD));
-  uint4 qhi[kPieces], qlo[kPieces];
+  u32x4_t qhi[2][kPieces], qlo[2][kPieces];
+  uint32_t n_keys[2];
+  {
+    float *q_s = reinterpret_cast<float *>(smem + kStage) + wave * 16 * HD;
+    // (every input of eight pairs requested first, unconditionally: one round trip instead of eight)
+    const bool has_bias = p.q_bias != nullptr, has_gamma = p.q_norm != nullptr, has_rope = p.rope_freq != nullptr;
+    const uint16_t *bias_base = has_bias ? p.q_bias : p.k_cache;    // any readable address when unused
+    const float *rope_base = has_rope ? p.rope_cs : p.qkv;
+    const uint32_t rope_stride = has_rope ? p.rope_token_stride : 0u;
+    const uint16_t *gamma_base = has_gamma ? p.q_norm : p.k_cache;
+    const int pl = pair_of<HD>(lane);
+    const float g0 = dec16<DT>(gamma_base[pl]), g1 = dec16<DT>(gamma_base[pl + HD / 2]);
+    const float scale = kLog2e / sqrtf(static_cast<float>(HD));
 #pragma unroll
-  for (int j = 0; j < kPieces; ++j) {
-    const float *src = &q_s[wave][col][j * 32 + grp * 8];
-    uint32_t wh[4], wl[4];
+    for (int c = 0; c < 2; ++c) {
 #pragma unroll
-    for (int e = 0; e < 4; ++e) {
-      uint16_t h0, l0, h1, l1;
-      split16<DT>(src[2 * e] * scale, h0, l0);
-      split16<DT>(src[2 * e + 1] * scale, h1, l1);
-      wh[e] = h0 | (static_cast<uint32_t>(h1) << 16);
-      wl[e] = l0 | (static_cast<uint32_t>(l1) << 16);
-    }
-    qhi[j] = make_uint4(wh[0], wh[1], wh[2], wh[3]);
-    qlo[j] = make_uint4(wl[0], wl[1], wl[2], wl[3]);
-  }
-  // causal limit of this lane's column, and the last tile any of the wave's tokens can see
-  const int pair = min(col, kPairs - 1);
-  const uint32_t my_tok = min(wave_first + pair / G, T - 1);
-  const uint32_t n_keys = p.position + my_tok + 1;
-  const uint32_t wave_last_tile = (p.position + min(wave_first + kTokensPerWave - 1, T - 1)) / kKvBlockTokens;
-  const bool wave_on = wave_first < T;
-
-  float m = -INFINITY, l = 0.0f;
-  f32x4_t acc[HD / 16];
+      for (int part = 0; part < 2; ++part) {   // eight pairs at a time: their inputs in one round trip
+        float x0[8], x1[8], rc[8], rs[8];
+        uint16_t qb0[8], qb1[8];
 #pragma unroll
-  for (int s2 = 0; s2 < HD / 16; ++s2) acc[s2] = f32x4_t{0.0f, 0.0f, 0.0f, 0.0f};
-
-  for (uint32_t b = b0; b < b1; ++b) {
-    const int st = (b - b0) & 1;
-    if (HD == 128 || wave < 2 * kPieces) stage[st][my_piece][lane] = inflight;
-    inflight = tile_piece(min(b + 1, b1 - 1));   // unconditional: a load under a branch would serialise
-    __syncthreads();                             // the tile is complete; the other stage is free again
-    if (wave_on && b <= wave_last_tile) {
-      uint4 kreg[kPieces], vreg[kPieces];
+        for (int i = 0; i < 8; ++i) {
+          const int vh = min(c * 16 + part * 8 + i, kPairs - 1);
+          const uint32_t tok = min(wave_first + vh / G, T - 1);
+          const uint32_t h = kvh * G + vh % G;
+          const float *src = p.qkv + static_cast<uint64_t>(tok) * p.qkv_token_stride + h * HD;
+          x0[i] = src[pl];
+          x1[i] = src[pl + HD / 2];
+          qb0[i] = bias_base[h * HD + pl];
+          qb1[i] = bias_base[h * HD + pl + HD / 2];
+          rc[i] = rope_base[static_cast<uint64_t>(tok) * rope_stride + pl];
+          rs[i] = rope_base[static_cast<uint64_t>(tok) * rope_stride + HD / 2 + pl];
+        }
+#pragma unroll
+        for (int i = 0; i < 8; ++i)
+          prep_head_core<DT, HD>(x0[i], x1[i], has_bias, dec16<DT>(qb0[i]), dec16<DT>(qb1[i]), has_gamma, g0, g1, has_rope, rc[i],
+                                 rs[i], p.eps, lane, q_s + (part * 8 + i) * HD, nullptr);
+      }
+      // (written and read by this wave alone, in order)
 #pragma unroll
       for (int j = 0; j < kPieces; ++j) {
-        kreg[j] = stage[st][j][lane];
-        vreg[j] = stage[st][kPieces + j][lane];
+        const float *src = q_s + col * HD + j * 32 + grp * 8;
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+          uint16_t h0, l0, h1, l1;
+          split16<DT>(src[2 * e] * scale, h0, l0);
+          split16<DT>(src[2 * e + 1] * scale, h1, l1);
+          qhi[c][j][e] = h0 | (static_cast<uint32_t>(h1) << 16);
+          qlo[c][j][e] = l0 | (static_cast<uint32_t>(l1) << 16);
+        }
       }
-      attn_tile_wide<DT, HD>(kreg, vreg, qhi, qlo, b, n_keys, grp, m, l, acc);
+      n_keys[c] = p.position + min(wave_first + min(c * 16 + col, kPairs - 1) / G, T - 1) + 1;   // causal limit of the column
+    }
+  }
+  const bool wave_on = wave_first < T;
+  const uint32_t least_keys = p.position + min(wave_first, T - 1) + 1;                            // of any column of the wave,
+  const uint32_t most_keys = p.position + min(wave_first + kTokensPerWave - 1, T - 1) + 1;        // and the most of any
+
+  float m[2], l[2];
+  f32x4_t acc[2][HD / 16];   // O^T[dims s*16 + grp*4 .. +3][column]
+#pragma unroll
+  for (int c = 0; c < 2; ++c) {
+    m[c] = -INFINITY;
+    l[c] = 0.0f;
+#pragma unroll
+    for (int s2 = 0; s2 < HD / 16; ++s2) acc[c][s2] = f32x4_t{0.0f, 0.0f, 0.0f, 0.0f};
+  }
+  __syncthreads();   // everyone has taken its queries: the second and third stage are free
+  if (steps > 1) request(1);
+  const uint32_t lds0 = static_cast<uint32_t>(reinterpret_cast<uintptr_t>(NV_PR_LDS(smem))) + lane * 16u;
+
+  // ---- the three parts of a step (skipped where no column of the wave sees it)
+  f32x4_t sc[2][kStepBlocks];   // scores of keys key0 + 16 t + 4 grp + r, then the bits of their probabilities: two words hi, two lo
+  auto sees = [&](uint32_t step) { return wave_on && (b0 + step * kStepBlocks) * kKvBlockTokens < most_keys; };
+  auto scores = [&](uint32_t step) {
+    if (!sees(step)) return;
+    const uint32_t at = lds0 + (step % kStages) * kStage;
+    u32x4_t k[2][kPieces];
+#pragma unroll
+    for (int j = 0; j < kPieces; ++j) NV_PR_READ(k[0][j], at, j * 1024);
+#pragma unroll
+    for (uint32_t t = 0; t < kStepBlocks; ++t) {
+      if (t + 1 < kStepBlocks) {
+#pragma unroll
+        for (int j = 0; j < kPieces; ++j) NV_PR_READ(k[(t + 1) & 1][j], at, (t + 1) * 2 * kTile + j * 1024);
+      }
+#pragma unroll
+      for (int j = 0; j < kPieces; j += 2) {
+        if (t + 1 < kStepBlocks) NV_PR_AWAIT2(kPieces, k[t & 1][j], k[t & 1][j + 1]);
+        else NV_PR_AWAIT2(0, k[t & 1][j], k[t & 1][j + 1]);
+      }
+      __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+      for (int c = 0; c < 2; ++c) sc[c][t] = f32x4_t{0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+      for (int j = 0; j < kPieces; ++j)
+#pragma unroll
+        for (int c = 0; c < 2; ++c) sc[c][t] = mfma_k32<DT>(k[t & 1][j], qhi[c][j], sc[c][t]);
+#pragma unroll
+      for (int j = 0; j < kPieces; ++j)
+#pragma unroll
+        for (int c = 0; c < 2; ++c) sc[c][t] = mfma_k32<DT>(k[t & 1][j], qlo[c][j], sc[c][t]);
+      __builtin_amdgcn_sched_barrier(0);
+    }
+  };
+  auto softmax = [&](uint32_t step) {
+    if (!sees(step)) return;
+    const uint32_t key0 = (b0 + step * kStepBlocks) * kKvBlockTokens;
+    if (key0 + kStepBlocks * kKvBlockTokens > least_keys) {   // some column ends inside this step (or before it)
+#pragma unroll
+      for (int c = 0; c < 2; ++c)
+#pragma unroll
+        for (uint32_t t = 0; t < kStepBlocks; ++t)
+#pragma unroll
+          for (uint32_t r = 0; r < 4; ++r) sc[c][t][r] = key0 + t * 16u + grp * 4u + r < n_keys[c] ? sc[c][t][r] : -INFINITY;
+    }
+#pragma unroll
+    for (int c = 0; c < 2; ++c) {
+      float mb = fmaxf(fmaxf(sc[c][0][0], sc[c][0][1]), fmaxf(sc[c][0][2], sc[c][0][3]));
+#pragma unroll
+      for (uint32_t t = 1; t < kStepBlocks; ++t) mb = fmaxf(fmaxf(mb, fmaxf(sc[c][t][0], sc[c][t][1])), fmaxf(sc[c][t][2], sc[c][t][3]));
+      mb = fmaxf(mb, __shfl_xor(mb, 16, kWave));
+      mb = fmaxf(mb, __shfl_xor(mb, 32, kWave));
+      const float m_new = fmaxf(m[c], mb);
+      const float m_ref = fmaxf(m_new, -3.0e38f);   // a column with nothing to see yet: exponentials against a finite stand-in
+      const float alpha = attn_exp2(m[c] - m_ref);
+      float psum = 0.0f;
+#pragma unroll
+      for (uint32_t t = 0; t < kStepBlocks; ++t) {
+        float e[4];
+#pragma unroll
+        for (int r = 0; r < 4; ++r) e[r] = attn_exp2(sc[c][t][r] - m_ref);
+        psum += (e[0] + e[1]) + (e[2] + e[3]);
+#pragma unroll
+        for (int r = 0; r < 4; r += 2) {
+          uint16_t h0, l0, h1, l1;
+          split16<DT>(e[r], h0, l0);
+          split16<DT>(e[r + 1], h1, l1);
+          sc[c][t][r / 2] = __uint_as_float(h0 | (static_cast<uint32_t>(h1) << 16));
+          sc[c][t][2 + r / 2] = __uint_as_float(l0 | (static_cast<uint32_t>(l1) << 16));
+        }
+      }
+      l[c] = l[c] * alpha + psum;
+      m[c] = m_new;
+      if (__any(alpha != 1.0f)) {
+#pragma unroll
+        for (int s2 = 0; s2 < HD / 16; ++s2) acc[c][s2] *= alpha;
+      }
+    }
+  };
+  // O^T += V^T . P, two tiles of keys at a time
+  auto values = [&](uint32_t step) {
+    if (!sees(step)) return;
+    const uint32_t at = lds0 + (step % kStages) * kStage + kTile;
+    u32x4_t v[2][2];   // a piece of each of the two tiles, this group's and the next one's
+    NV_PR_READ(v[0][0], at, 0);
+    NV_PR_READ(v[0][1], at, 2 * kTile);
+    constexpr int kGroups = 2 * kPieces;   // (pair of tiles, piece)
+#pragma unroll
+    for (int g = 0; g < kGroups; ++g) {
+      if (g + 1 < kGroups) {
+        NV_PR_READ(v[(g + 1) & 1][0], at, ((g + 1) / kPieces) * 4 * kTile + ((g + 1) % kPieces) * 1024);
+        NV_PR_READ(v[(g + 1) & 1][1], at, ((g + 1) / kPieces) * 4 * kTile + 2 * kTile + ((g + 1) % kPieces) * 1024);
+        NV_PR_AWAIT2(2, v[g & 1][0], v[g & 1][1]);
+      } else {
+        NV_PR_AWAIT2(0, v[g & 1][0], v[g & 1][1]);
+      }
+      __builtin_amdgcn_sched_barrier(0);
+      const int pair = g / kPieces, j = g % kPieces;
+      const u32x4_t &a = v[g & 1][0], &b = v[g & 1][1];
+      const u32x4_t lo_slab = {a[0], a[1], b[0], b[1]}, hi_slab = {a[2], a[3], b[2], b[3]};
+#pragma unroll
+      for (int c = 0; c < 2; ++c) {
+        const u32x4_t pa = __builtin_bit_cast(u32x4_t, sc[c][2 * pair]), pb = __builtin_bit_cast(u32x4_t, sc[c][2 * pair + 1]);
+        const u32x4_t bh = {pa[0], pa[1], pb[0], pb[1]};
+        acc[c][2 * j] = mfma_k32<DT>(lo_slab, bh, acc[c][2 * j]);
+        acc[c][2 * j + 1] = mfma_k32<DT>(hi_slab, bh, acc[c][2 * j + 1]);
+      }
+#pragma unroll
+      for (int c = 0; c < 2; ++c) {
+        const u32x4_t pa = __builtin_bit_cast(u32x4_t, sc[c][2 * pair]), pb = __builtin_bit_cast(u32x4_t, sc[c][2 * pair + 1]);
+        const u32x4_t bl = {pa[2], pa[3], pb[2], pb[3]};
+        acc[c][2 * j] = mfma_k32<DT>(lo_slab, bl, acc[c][2 * j]);
+        acc[c][2 * j + 1] = mfma_k32<DT>(hi_slab, bl, acc[c][2 * j + 1]);
+      }
+      __builtin_amdgcn_sched_barrier(0);
+    }
+  };
+
+  // ---- the walk, in two phases a step: while waves 0..3 (one a SIMD) multiply, waves 4..7 work on their probabilities, and
+  // the other way round. Phase 2k: first half V(k-1) and K(k), second half softmax(k-1); phase 2k+1: first half
+  // softmax(k), second half V(k-1) and K(k). A stage is free when the second half has left V of its step, two phases
+  // before it is filled again.
+  const bool first_half = wave < kPW / 2;
+  for (uint32_t k = 0; k <= steps; ++k) {
+    // this wave's part of step k has arrived (step k + 1 may be on its way)
+    if (k + 1 < steps) asm volatile("s_waitcnt vmcnt(%0)\n\ts_barrier" ::"n"(kPieces) : "memory");
+    else asm volatile("s_waitcnt vmcnt(0)\n\ts_barrier" ::: "memory");
+    if (k + 2 < steps) request(k + 2);
+    if (!first_half) {
+      if (k > 0) softmax(k - 1);
+      asm volatile("s_barrier" ::: "memory");
+    }
+    if (k > 0) values(k - 1);
+    if (k < steps) scores(k);
+    if (first_half) {
+      asm volatile("s_barrier" ::: "memory");
+      if (k < steps) softmax(k);
     }
   }
   if (!wave_on) return;
 
   // ---- results of the wave's pairs: token rows of the four lane groups
-  l += __shfl_xor(l, 16, kWave);
-  l += __shfl_xor(l, 32, kWave);
-  const uint32_t tok = min(wave_first + pair / G, T - 1);
-  const uint32_t h = kvh * G + pair % G;
-  const bool writer = wave_first + pair / G < T && col < kPairs;
-  const float inv = l > 0.0f && isfinite(l) ? 1.0f / l : 1.0f;
-  char *ws = reinterpret_cast<char *>(p.part_acc) + static_cast<uint64_t>(tok) * p.ws_token_stride;
   const uint64_t ml_off = reinterpret_cast<char *>(p.part_m) - reinterpret_cast<char *>(p.part_acc);
   const uint64_t l_off = reinterpret_cast<char *>(p.part_l) - reinterpret_cast<char *>(p.part_acc);
 #pragma unroll
-  for (int s2 = 0; s2 < HD / 16; ++s2) {
-    if (!writer) continue;
-    const float4 o = make_float4(acc[s2][0], acc[s2][1], acc[s2][2], acc[s2][3]);
-    const uint32_t d = s2 * 16 + grp * 4;
-    if (active == 1) {
-      // a single split holds every key: final
-      uint2 packed;
-      packed.x = enc16<DT>(o.x * inv) | (static_cast<uint32_t>(enc16<DT>(o.y * inv)) << 16);
-      packed.y = enc16<DT>(o.z * inv) | (static_cast<uint32_t>(enc16<DT>(o.w * inv)) << 16);
-      *reinterpret_cast<uint2 *>(p.out16 + attn_out_token(p, tok) + attn_out_elem(p, h * HD + d)) = packed;   // d % 4 == 0
-    } else {
-      *reinterpret_cast<float4 *>(reinterpret_cast<float *>(ws) + (static_cast<uint64_t>(h) * S + split) * HD + d) = o;
+  for (int c = 0; c < 2; ++c) {
+    float lc = l[c];
+    lc += __shfl_xor(lc, 16, kWave);
+    lc += __shfl_xor(lc, 32, kWave);
+    const int pair = c * 16 + col;
+    const uint32_t tok = wave_first + pair / G, h = kvh * G + pair % G;
+    if (pair >= kPairs || tok >= T) continue;
+    const float inv = lc > 0.0f && isfinite(lc) ? 1.0f / lc : 1.0f;
+    char *ws = reinterpret_cast<char *>(p.part_acc) + static_cast<uint64_t>(tok) * p.ws_token_stride;
+#pragma unroll
+    for (int s2 = 0; s2 < HD / 16; ++s2) {
+      const float4 o = make_float4(acc[c][s2][0], acc[c][s2][1], acc[c][s2][2], acc[c][s2][3]);
+      const uint32_t d = s2 * 16 + grp * 4;
+      if (active == 1) {
+        // a single split holds every key: final
+        uint2 packed;
+        packed.x = enc16<DT>(o.x * inv) | (static_cast<uint32_t>(enc16<DT>(o.y * inv)) << 16);
+        packed.y = enc16<DT>(o.z * inv) | (static_cast<uint32_t>(enc16<DT>(o.w * inv)) << 16);
+        *reinterpret_cast<uint2 *>(p.out16 + attn_out_token(p, tok) + attn_out_elem(p, h * HD + d)) = packed;   // d % 4 == 0
+      } else {
+        *reinterpret_cast<float4 *>(reinterpret_cast<float *>(ws) + (static_cast<uint64_t>(h) * S + split) * HD + d) = o;
+      }
+    }
+    if (active != 1 && grp == 0) {
+      reinterpret_cast<float *>(ws + ml_off)[h * S + split] = m[c];
+      reinterpret_cast<float *>(ws + l_off)[h * S + split] = lc;
     }
   }
-  if (active != 1 && writer && grp == 0) {
-    reinterpret_cast<float *>(ws + ml_off)[h * S + split] = m;
-    reinterpret_cast<float *>(ws + l_off)[h * S + split] = l;
-  }
 }
+#undef NV_PR_LDS
+#undef NV_PR_READ
+#undef NV_PR_AWAIT2
 
 // Second launch: grid (head, token), one lane per dim; splits in order, kRound of them requested at a time
 // (4 where the launch has no more splits than that: the same sums in the same order with a quarter of the loads).
@@ -224,22 +387,37 @@ __global__ __launch_bounds__(HD) void attn_prompt_merge_kernel(AttnParams p, uin
   p.out16[attn_out_token(p, tok) + attn_out_elem(p, h * HD + d)] = enc16<DT>(o);
 }
 
+template <uint32_t DT, int HD, int G>
+hipError_t launch_group(const AttnParams &p, uint32_t splits, hipStream_t stream) {
+  constexpr size_t lds = static_cast<size_t>(kStages) * prompt_stage_bytes(HD);
+  // more than the default dynamic LDS limit: raised once per kernel (never under stream capture)
+  static std::once_flag once;
+  static hipError_t raised = hipSuccess;
+  std::call_once(once, [] {
+    raised = hipFuncSetAttribute(reinterpret_cast<const void *>(&attn_prompt_kernel<DT, HD, G>),
+                                 hipFuncAttributeMaxDynamicSharedMemorySize, static_cast<int>(lds));
+  });
+  if (raised != hipSuccess) return raised;
+  constexpr uint32_t group_tokens = kPW * (kCols / G);
+  hipLaunchKernelGGL((attn_prompt_kernel<DT, HD, G>), dim3(p.kv_heads, splits, (p.tokens + group_tokens - 1) / group_tokens),
+                     dim3(kPW * kWave), lds, stream, p);
+  return hipGetLastError();
+}
+
 template <uint32_t DT, int HD>
 hipError_t launch_hd(const AttnParams &p, uint32_t splits, hipStream_t stream) {
-  const uint32_t group = p.heads / p.kv_heads;
-  const uint32_t group_tokens = kPW * (kVG / group);
-  const dim3 grid(p.kv_heads, splits, (p.tokens + group_tokens - 1) / group_tokens);
+  const uint32_t group = p.heads / p.kv_heads, group_tokens = kPW * (kCols / group);
+  hipError_t err = hipSuccess;
   switch (group) {
-    case 1: hipLaunchKernelGGL((attn_prompt_kernel<DT, HD, 1>), grid, dim3(kPW * kWave), 0, stream, p); break;
-    case 2: hipLaunchKernelGGL((attn_prompt_kernel<DT, HD, 2>), grid, dim3(kPW * kWave), 0, stream, p); break;
-    case 3: hipLaunchKernelGGL((attn_prompt_kernel<DT, HD, 3>), grid, dim3(kPW * kWave), 0, stream, p); break;
-    case 4: hipLaunchKernelGGL((attn_prompt_kernel<DT, HD, 4>), grid, dim3(kPW * kWave), 0, stream, p); break;
-    case 5: hipLaunchKernelGGL((attn_prompt_kernel<DT, HD, 5>), grid, dim3(kPW * kWave), 0, stream, p); break;
-    case 6: hipLaunchKernelGGL((attn_prompt_kernel<DT, HD, 6>), grid, dim3(kPW * kWave), 0, stream, p); break;
-    case 7: hipLaunchKernelGGL((attn_prompt_kernel<DT, HD, 7>), grid, dim3(kPW * kWave), 0, stream, p); break;
-    default: hipLaunchKernelGGL((attn_prompt_kernel<DT, HD, 8>), grid, dim3(kPW * kWave), 0, stream, p); break;
+    case 1: err = launch_group<DT, HD, 1>(p, splits, stream); break;
+    case 2: err = launch_group<DT, HD, 2>(p, splits, stream); break;
+    case 3: err = launch_group<DT, HD, 3>(p, splits, stream); break;
+    case 4: err = launch_group<DT, HD, 4>(p, splits, stream); break;
+    case 5: err = launch_group<DT, HD, 5>(p, splits, stream); break;
+    case 6: err = launch_group<DT, HD, 6>(p, splits, stream); break;
+    case 7: err = launch_group<DT, HD, 7>(p, splits, stream); break;
+    default: err = launch_group<DT, HD, 8>(p, splits, stream); break;
   }
-  hipError_t err = hipGetLastError();
   if (err != hipSuccess || splits == 1) return err;
   if (splits <= 4)
     hipLaunchKernelGGL((attn_prompt_merge_kernel<DT, HD, 4>), dim3(p.heads, p.tokens), dim3(HD), 0, stream, p, splits, group_tokens);
@@ -266,11 +444,11 @@ hipError_t launch_attn_prompt(uint32_t dtype, const AttnParams &p, hipStream_t s
     return hipErrorInvalidValue;
   if (p.rope_freq != nullptr && p.rope_cs == nullptr) return hipErrorInvalidValue;   // rotation tables per token row
   if (p.out_packed_tiles != 0 && p.out_packed_tiles * 16u < p.tokens) return hipErrorInvalidValue;
-  // enough splits of the prefix to spread the block over the chip, at least eight tiles each
-  const uint32_t group_tokens = kPW * (kVG / group);
+  // enough splits of the prefix to give every CU a workgroup, at least two steps each
+  const uint32_t group_tokens = kPW * (kCols / group);
   const uint32_t groups = (p.tokens + group_tokens - 1) / group_tokens;
   const uint32_t nblk = (p.position + p.tokens - 1) / kKvBlockTokens + 1;
-  uint32_t splits = p.splits != 0 ? p.splits : (512u + p.kv_heads * groups - 1) / (p.kv_heads * groups);
+  uint32_t splits = p.splits != 0 ? p.splits : (256u + p.kv_heads * groups - 1) / (p.kv_heads * groups);
   splits = std::min(splits, std::max(1u, nblk / 8));
   splits = std::max(1u, std::min<uint32_t>(splits, kAttnMaxSplits));
   if (dtype == kBF16) return launch_dt<kBF16>(p, splits, stream);

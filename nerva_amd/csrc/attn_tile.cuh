@@ -124,6 +124,10 @@ __device__ __forceinline__ f32x4_t mfma_k32(const uint4 &a, const uint4 &b, f32x
     return __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(f16x8_t, a),
                                                   __builtin_bit_cast(f16x8_t, b), c, 0, 0, 0);
 }
+template <uint32_t DT>
+__device__ __forceinline__ f32x4_t mfma_k32(const u32x4_t &a, const u32x4_t &b, f32x4_t c) {
+  return mfma_k32<DT>(__builtin_bit_cast(uint4, a), __builtin_bit_cast(uint4, b), c);
+}
 // D(16x16) += A(16x16) . B(16x16): four contraction elements per lane, 4*(l/16)..+3.
 template <uint32_t DT>
 __device__ __forceinline__ f32x4_t mfma_k16(const uint2 &a, const uint2 &b, f32x4_t c) {
@@ -181,6 +185,16 @@ __device__ __forceinline__ uint32_t load_coherent(const uint32_t *ptr) {
 }
 // Returns when every store this wave has issued has been performed.
 __device__ __forceinline__ void wait_stores_performed() { asm volatile("s_waitcnt vmcnt(0)" ::: "memory"); }
+
+// Loads through the scalar path (position, block-table entries: the same for every lane, and read-only
+// while the launch runs). The compiler takes the vector path for them - it cannot prove that the
+// launch does not write there - and a vector load would have to be awaited with everything requested
+// before it.
+__device__ __forceinline__ uint32_t scalar_load(const uint32_t *ptr) {
+  uint32_t v;
+  asm volatile("s_load_dword %0, %1, 0x0\n\ts_waitcnt lgkmcnt(0)" : "=s"(v) : "s"(ptr) : "memory");
+  return v;
+}
 
 // Requests one (physical block, kv head) tile: a 1 KiB load each of K and V for every 32 dims.
 template <int HD>
@@ -279,60 +293,6 @@ __device__ __forceinline__ void attn_tile(uint4 (&kreg)[HD / 32], uint4 (&vreg)[
     const uint4 &vr = vreg[s2 / 2];
     const uint2 va = (s2 & 1) ? make_uint2(vr.z, vr.w) : make_uint2(vr.x, vr.y);
     acc[s2] = mfma_k16<DT>(va, pb, acc[s2]);
-  }
-}
-
-// The same tile step for sixteen independent columns (prompt blocks: sixteen (token, head) pairs of a wave). The
-// hi and lo halves of a query, and of a tile's probabilities, are two operands of two products that accumulate in the
-// same registers instead of two columns that meet by a lane exchange: the same number of matrix instructions per
-// pair, but the softmax arithmetic of a lane - the maximum, five exponentials, four hi/lo splits - serves a pair of
-// its own instead of being done twice, and a K/V tile read from LDS meets twice as many pairs. Columns are masked
-// individually (n_keys by column; a column may find a whole tile masked) and the accumulators are rescaled only
-// in tiles where some running maximum moved.
-template <uint32_t DT, int HD>
-__device__ __forceinline__ void attn_tile_wide(const uint4 (&kreg)[HD / 32], const uint4 (&vreg)[HD / 32], const uint4 (&qhi)[HD / 32],
-                                               const uint4 (&qlo)[HD / 32], uint32_t b, uint32_t n_keys, int grp, float &m,
-                                               float &l, f32x4_t (&acc)[HD / 16]) {
-  // scores of tokens b*16 + grp*4 + r for this lane's column
-  f32x4_t c{0.0f, 0.0f, 0.0f, 0.0f};
-#pragma unroll
-  for (int j = 0; j < HD / 32; ++j) c = mfma_k32<DT>(kreg[j], qhi[j], c);
-#pragma unroll
-  for (int j = 0; j < HD / 32; ++j) c = mfma_k32<DT>(kreg[j], qlo[j], c);
-  float sc[4];
-#pragma unroll
-  for (int r = 0; r < 4; ++r) sc[r] = b * kKvBlockTokens + grp * 4 + r < n_keys ? c[r] : -INFINITY;
-  float mb = fmaxf(fmaxf(sc[0], sc[1]), fmaxf(sc[2], sc[3]));
-  mb = fmaxf(mb, __shfl_xor(mb, 16, kWave));
-  mb = fmaxf(mb, __shfl_xor(mb, 32, kWave));
-  const float m_new = fmaxf(m, mb);
-  const float m_ref = fmaxf(m_new, -3.0e38f);   // a column with nothing to see yet: exponentials against a finite stand-in
-  const float alpha = attn_exp2(m - m_ref);
-  uint32_t ph[2], pl[2];
-  float psum = 0.0f;
-#pragma unroll
-  for (int r = 0; r < 4; r += 2) {
-    const float p0 = attn_exp2(sc[r] - m_ref), p1 = attn_exp2(sc[r + 1] - m_ref);
-    psum += p0 + p1;
-    uint16_t h0, l0, h1, l1;
-    split16<DT>(p0, h0, l0);
-    split16<DT>(p1, h1, l1);
-    ph[r / 2] = h0 | (static_cast<uint32_t>(h1) << 16);
-    pl[r / 2] = l0 | (static_cast<uint32_t>(l1) << 16);
-  }
-  l = l * alpha + psum;
-  m = m_new;
-  const uint2 pbh = make_uint2(ph[0], ph[1]), pbl = make_uint2(pl[0], pl[1]);
-  if (__any(alpha != 1.0f)) {
-#pragma unroll
-    for (int s2 = 0; s2 < HD / 16; ++s2) acc[s2] *= alpha;
-  }
-#pragma unroll
-  for (int s2 = 0; s2 < HD / 16; ++s2) {
-    const uint4 &vr = vreg[s2 / 2];
-    const uint2 va = (s2 & 1) ? make_uint2(vr.z, vr.w) : make_uint2(vr.x, vr.y);
-    acc[s2] = mfma_k16<DT>(va, pbh, acc[s2]);
-    acc[s2] = mfma_k16<DT>(va, pbl, acc[s2]);
   }
 }
 
