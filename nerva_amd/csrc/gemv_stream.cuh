@@ -410,7 +410,7 @@ __global__ __launch_bounds__(kBlock) void gemv_kernel(GemvParams p) {
 }
 
 // ---------------------------------------------------------------------------
-// Production-shape kernel: cols % (512 * B) == 0, 16-byte aligned rows, cols <= 12288 (30720 with a 16-bit input).
+// Production-shape kernel: cols % (512 * B) == 0 (RAGGED: % 64), 16-byte aligned rows, cols <= 12288 (30720 with a 16-bit input).
 // Same contract as gemv_kernel, leaner register budget (about 64 VGPRs instead of
 // ~150) so that 6-8 workgroups stay resident per CU and a whole 4096-row matrix is
 // on the machine at once. A wave walks a flat list of request batches - (its 1st
@@ -455,10 +455,15 @@ constexpr int kFastMaxColsLoop = 30720;  // ... or, with a 16-bit input, copied 
 // products behind a batch's arrival do not wait for LDS reads (a wave gets one 1 KiB LDS read through every
 // ~30 cycles: eight of them a row were twice the time of the row's 32 dot instructions). Costs 32 registers:
 // one wave per SIMD less.
+// RAGGED: rows of any whole number of cache lines (cols % 64 == 0). The last batch of a row ends with it: lanes past the
+// end ask for the row's last piece again (one cache line for all of them) and leave it out of the sum. What the general
+// kernel, with its ~150 registers, took 11.8 / 43.5 / 24.6 / 176 us for at a width of 3584 (qkv, gate/up pairs of 18944,
+// down, a head of 152064 rows) takes 8.4 / 42.1 / 23.6 / 158; 20.4 us for pairs of 9728 x 2560 is 17.1.
 template <uint32_t DT, int PRO, int EPI, int NR, int B, bool EXACT = false, int WG = kWavesPerBlock, bool XREG = false,
-          bool ROT = false>
+          bool ROT = false, bool RAGGED = false>
 __global__ __launch_bounds__(WG *kWave, XREG ? 4 : PRO == kProJoin && WG == 8 ? 2 : fast_waves_per_simd(PRO)) void gemv_fast_kernel(GemvParams p) {
   static_assert(!(ROT && (XREG || EXACT)), "the rotated walk has no exact-start or register-input variant");
+  static_assert(!(RAGGED && (XREG || EXACT)), "nor have ragged rows");
   constexpr int TB = WG * kWave;
   constexpr uint32_t kXregBpr = 8 / B;   // batches per 4096-column row
   extern __shared__ __align__(16) uint16_t xs[];
@@ -473,7 +478,7 @@ __global__ __launch_bounds__(WG *kWave, XREG ? 4 : PRO == kProJoin && WG == 8 ? 
   // (kProJoin: consecutive units go to different workgroups - one per CU - so that every CU has the same share to a row)
   const uint32_t wave_global = PRO == kProJoin ? wave * gridDim.x + blockIdx.x : blockIdx.x * WG + wave;
   const uint32_t wave_stride = gridDim.x * WG;
-  const uint32_t bpr = cols / (kWave * 8 * B);  // request batches per row
+  const uint32_t bpr = RAGGED ? (cols + kWave * 8 * B - 1) / (kWave * 8 * B) : cols / (kWave * 8 * B);  // request batches per row
   const uint32_t my_units = wave_global < units ? (units - wave_global + wave_stride - 1) / wave_stride : 0u;
   const uint32_t total = my_units * bpr;
 
@@ -526,7 +531,7 @@ __global__ __launch_bounds__(WG *kWave, XREG ? 4 : PRO == kProJoin && WG == 8 ? 
     if (ib == 0) {                                                                                \
       if constexpr (ROT) ic = iu % bpr;                                                           \
       _Pragma("unroll") for (int k = 0; k < NR; ++k)                                              \
-        wp[k] = p.w + static_cast<uint64_t>(iu + k * p.rows) * cols + k * p.pair_gap + ic * kBatchElems + lane * 8; \
+        wp[k] = p.w + static_cast<uint64_t>(iu + k * p.rows) * cols + k * p.pair_gap + (RAGGED ? 0u : ic * kBatchElems + lane * 8); \
       if constexpr (EPI == kEpiResidual) {                                                        \
         if (EXACT || lane == 0) RES = p.residual[iu];                                             \
       }                                                                                           \
@@ -536,6 +541,15 @@ __global__ __launch_bounds__(WG *kWave, XREG ? 4 : PRO == kProJoin && WG == 8 ? 
         UB = p.bias2[iu];                                                                         \
       }                                                                                           \
     }                                                                                             \
+    if constexpr (RAGGED) {                                                                       \
+      _Pragma("unroll") for (int u = 0; u < B; ++u) {                                             \
+        const uint32_t at_ = min((ROT ? ic : ib) * kBatchElems + u * (kWave * 8) + lane * 8, cols - 8); \
+        _Pragma("unroll") for (int k = 0; k < NR; ++k) DST[k][u] = load_stream(wp[k] + at_);      \
+      }                                                                                           \
+      if constexpr (ROT) {                                                                        \
+        if (++ic == bpr) ic = 0;                                                                  \
+      }                                                                                           \
+    } else {                                                                                      \
     _Pragma("unroll") for (int u = 0; u < B; ++u)                                                 \
       _Pragma("unroll") for (int k = 0; k < NR; ++k) DST[k][u] = load_stream(wp[k] + u * (kWave * 8)); \
     _Pragma("unroll") for (int k = 0; k < NR; ++k) wp[k] += kBatchElems;                              \
@@ -544,6 +558,7 @@ __global__ __launch_bounds__(WG *kWave, XREG ? 4 : PRO == kProJoin && WG == 8 ? 
         ic = 0;                                                                                   \
         _Pragma("unroll") for (int k = 0; k < NR; ++k) wp[k] -= cols;                             \
       }                                                                                           \
+    }                                                                                             \
     }                                                                                             \
     if (++ib == bpr) {                                                                            \
       ib = 0;                                                                                     \
@@ -655,6 +670,9 @@ __global__ __launch_bounds__(WG *kWave, XREG ? 4 : PRO == kProJoin && WG == 8 ? 
     }                                                                                             \
     _Pragma("unroll") for (int u = 0; u < B; ++u) {                                               \
       uint4 xv;                                                                                   \
+      if constexpr (RAGGED) {                                                                     \
+        if (c0 + u * (kWave * 8) >= cols) break;                                                  \
+      }                                                                                           \
       if constexpr (XREG) xv = xr[cb * B + u]; /* cb is a constant at every use in this mode */   \
       else xv = *reinterpret_cast<const uint4 *>(xs + c0 + u * (kWave * 8));                      \
       _Pragma("unroll") for (int k = 0; k < NR; ++k) acc[k] = dot8<DT, true>(SRC[k][u], xv, acc[k]);  \
@@ -769,6 +787,7 @@ struct GemvPlan {
   uint32_t grid;    // workgroups launched: ceil(blocks * 4 / wg_waves)
   bool rotated;     // kFast: the rotated walk (see gemv_fast_kernel)
   int chunks;       // kFast: 1 KiB chunks per row and request batch
+  bool ragged;      // kFast: rows that are no whole number of batches
 };
 constexpr int kFast = 3;  // the lean production-shape kernel
 GemvPlan gemv_plan(int prologue, int epilogue, uint32_t rows, uint32_t cols, bool vec16,

@@ -98,6 +98,19 @@ hipError_t launch_one(const GemvParams &p, const GemvPlan &plan, size_t lds, hip
         if (plan.rotated) NV_GEMV_LAUNCH(2, false, 16, false, true);
         else NV_GEMV_LAUNCH(2, false, 16, false, false);
       }
+    } else if (plan.ragged) {
+#define NV_GEMV_RAGGED(BB, W) \
+  hipLaunchKernelGGL((gemv_fast_kernel<DT, PRO, EPI, NR, BB, false, W, false, true, true>), dim3((waves + W - 1) / W), dim3(W * kWave), lds, stream, p)
+      if constexpr (EPI == kEpiArgmax) {
+        if (wg == 16) NV_GEMV_RAGGED(2, 16);
+        else NV_GEMV_RAGGED(2, 4);
+      } else if constexpr (NR == 2) {
+        NV_GEMV_RAGGED(2, 4);
+      } else {
+        if (plan.chunks == 2) NV_GEMV_RAGGED(2, 4);
+        else NV_GEMV_RAGGED(4, 4);
+      }
+#undef NV_GEMV_RAGGED
     } else if (plan.rotated) {
       // (which launches walk rotated, and with how many chunks a batch, is the plan's choice)
       if constexpr (EPI == kEpiSwiglu) {
@@ -193,7 +206,7 @@ int fast_workgroup_waves(int prologue, int epilogue, uint32_t rows, uint32_t col
 
 }  // namespace
 
-// kFast needs cols % 1024 == 0 and cols <= kFastMaxCols (kFastMaxColsLoop with a 16-bit input).
+// kFast needs cols % 64 == 0 and cols <= kFastMaxCols (kFastMaxColsLoop with a 16-bit input).
 GemvPlan gemv_plan(int prologue, int epilogue, uint32_t rows, uint32_t cols, bool vec16,
                    const GemvTuning *tuning) {
   GemvPlan plan;
@@ -201,8 +214,17 @@ GemvPlan gemv_plan(int prologue, int epilogue, uint32_t rows, uint32_t cols, boo
   plan.mode = !vec ? kScalar : (cols % (kWave * 8) == 0 ? kVecFull : kVecGuarded);
   const uint32_t fast_cols = kWave * 8 * 2;
   const uint32_t max_cols = prologue == kProX16 ? kFastMaxColsLoop : kFastMaxCols;
-  if (plan.mode == kVecFull && cols % fast_cols == 0 && cols <= (prologue == kProJoin ? kJoinFastCols : max_cols) && !(tuning && tuning->force_generic))
-    plan.mode = kFast;
+  plan.ragged = false;
+  if (plan.mode != kScalar && cols <= (prologue == kProJoin ? kJoinFastCols : max_cols) && !(tuning && tuning->force_generic)) {
+    // Rows of whole cache lines; a seam's only where they are whole batches of 1024 columns too. Ragged rows of a matrix
+    // of less than 6 MiB stay with the general kernel, whose launch is all start-up either way (1152 x 1152 3.10 us
+    // against 3.27, 2304 x 1152 3.95 against 4.22; a little above it 1152 x 4416 5.62
+    // against 5.01) - but for a head, which loops.
+    plan.ragged = cols % fast_cols != 0;
+    const uint64_t elems = static_cast<uint64_t>(rows) * cols * (epilogue == kEpiSwiglu ? 2u : 1u);
+    const bool small = elems < (3u << 20) && epilogue != kEpiArgmax;
+    if (!plan.ragged || (cols % 64u == 0 && prologue != kProJoin && !small)) plan.mode = kFast;
+  }
   // one wave per unit (a row, or a gate/up pair)
   const uint32_t want = (rows + kWavesPerBlock - 1) / kWavesPerBlock;
   uint32_t blocks = want;
@@ -235,6 +257,23 @@ GemvPlan gemv_plan(int prologue, int epilogue, uint32_t rows, uint32_t cols, boo
     plan.wg_waves = nv::tuning(kTuneGemvWorkgroupWaves);
     if ((plan.wg_waves != 4 && plan.wg_waves != 16) || prologue == kProJoin) plan.wg_waves = fast_workgroup_waves(prologue, epilogue, rows, cols);
     if (epilogue != kEpiSwiglu && cols % (kWave * 8 * 4) != 0) plan.chunks = 2;
+    if (plan.ragged) {
+      // Two chunks of a row a batch, four where a launch has few rows to keep requests in flight with (2560 x 9728
+      // 11.06 -> 10.08 us, 3840 x 16064 22.4 -> 21.2; 5120 x 13824 24.1 -> 25.3) and for the step's qkv projection.
+      // The launches with the norm in front: four workgroups a CU at most where a workgroup holds the row (6144 x 2560
+      // 8.84 -> 7.59 us, pairs of 9728 x 2560 17.8 -> 17.1 and of 18944 x 3584 43.3 -> 41.8), a head that does not take
+      // 16-wave workgroups five (32000 x 1152 18.3 -> 15.7).
+      plan.rotated = true;
+      const bool few = epilogue != kEpiArgmax && epilogue != kEpiSwiglu && (prologue == kProRmsNorm || rows < 4096u) && cols > 1536u;
+      plan.chunks = few ? 4 : 2;
+      if (epilogue != kEpiArgmax) plan.wg_waves = kWavesPerBlock;
+      if (!(tuning && tuning->max_blocks > 0)) {
+        if (prologue == kProRmsNorm && epilogue != kEpiArgmax && cols <= 4096u) plan.blocks = std::min(plan.blocks, kCus * 4u);
+        if (epilogue == kEpiArgmax && plan.wg_waves == kWavesPerBlock) plan.blocks = std::min(plan.blocks, kCus * 5u);
+      }
+      plan.grid = (plan.blocks * kWavesPerBlock + plan.wg_waves - 1) / plan.wg_waves;
+      return plan;
+    }
     // The rotated walk (see the kernel), where it measured faster; "gemv_rotated_walk" = 2 keeps the plain walk.
     const bool auto_grid = !(tuning && tuning->max_blocks > 0);
     if (nv::tuning(kTuneGemvRotatedWalk) != 2) {

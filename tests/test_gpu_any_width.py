@@ -126,3 +126,60 @@ def test_batch_steps_match_sequences_alone(geom, count):
     solo.destroy()
     for s in sessions[::-1]:
         s.destroy()
+
+
+@pytest.mark.parametrize("dtype", [BF16, F16])
+@pytest.mark.parametrize("rows,cols", [(3073, 1088),     # one cache line into the second batch
+                                       (2050, 1984), (5003, 3584), (1027, 9728),
+                                       (50000, 64),      # rows shorter than one request
+                                       (700, 12224),     # the widest an f32 input is kept for
+                                       (133, 30656)])    # the widest a 16-bit one is
+def test_lean_gemv_of_ragged_rows(dtype, rows, cols):
+    """Rows that are no whole number of batches, in all forms: what lies behind a row's end is the next row (or, behind the
+    last, nothing), so a lane too many shows. The activations of the general kernel, whose oracle is the same."""
+    rng = np.random.default_rng(rows + cols)
+    seed = rows * 131 + cols
+    w = O.synth_16(dtype, seed, 1, rows * cols, 0.0, 0.02).reshape(rows, cols)
+    dw = dev(w)
+    x16 = O.encode16(dtype, rng.normal(0, 1, cols).astype(np.float32))
+    res = rng.normal(0, 1, rows).astype(np.float32)
+    bias = O.encode16(dtype, rng.normal(0, 1, rows).astype(np.float32))
+    y, y16 = N.DeviceBuffer(rows * 4), N.DeviceBuffer(rows * 2 + 16)
+    kernel = lambda prologue, epilogue, n: N.gemv_launch_shape(prologue, epilogue, n, cols)[0]   # noqa: E731
+    assert kernel(0, 1, rows) == 3
+    N.gemv(dtype, dw, rows, cols, input16=dev(x16), residual=dev(res), out_f32=y, epilogue=1)
+    assert rel_l2(y.numpy(np.float32), O.gemv_x16(dtype, w, x16) + res) <= REL_L2
+    if cols > 12288:
+        return
+    h = rng.normal(0, 1, cols).astype(np.float32)
+    gamma = O.encode16(dtype, rng.normal(1, 0.02, cols))
+    n16 = O.encode16(dtype, O.rms_norm(dtype, h, gamma, 1e-6))
+    ref = O.gemv_x16(dtype, w, n16)
+    N.gemv(dtype, dw, rows, cols, input_f32=dev(h), gamma=dev(gamma), eps=1e-6, bias=dev(bias), out_f32=y)
+    got = y.numpy(np.float32).copy()
+    assert rel_l2(got, ref + O.decode16(dtype, bias)) <= REL_L2
+    N.gemv(dtype, dw, rows, cols, input_f32=dev(h), gamma=dev(gamma), eps=1e-6, bias=dev(bias), out16=y16, epilogue=3)
+    assert np.array_equal(y16.numpy(np.uint16, rows), O.encode16(dtype, got))
+    pairs = rows // 2
+    if 2 * pairs * cols >= 3 << 20:
+        assert kernel(1, 2, pairs) == 3
+    g, u = ref[:pairs], ref[pairs:2 * pairs]
+    ff = (g / (1.0 + np.exp(-g.astype(np.float64)))).astype(np.float32) * u
+    N.gemv(dtype, dw, pairs, cols, input_f32=dev(h), gamma=dev(gamma), eps=1e-6, out16=y16, epilogue=2)
+    assert rel_l2(O.decode16(dtype, y16.numpy(np.uint16, pairs)), O.decode16(dtype, O.encode16(dtype, ff))) <= 4e-3   # one 16-bit rounding
+
+
+@pytest.mark.parametrize("hidden,vocab", [(576, 20011), (1344, 40001), (704, 517)])
+def test_ragged_head_takes_the_largest(hidden, vocab):
+    """The head of a width off the 1024 grid, in workgroups of 4 and of 16 waves: every logit is the oracle's (one layer, one
+    token: one bf16 flip, as in the single-layer test), the token is the first of the largest."""
+    weights, omodel = random_model(BF16, hidden, hidden // 64, hidden // 64, 64, 320, vocab, 1, hidden, 1e4, False, False)
+    s = N.DecodeSession.create(weights, 32)
+    ctx = O.Context(omodel, 32, staging=1)
+    ctx.forward_token(3, prompt_token=True, want_logits=True)
+    rc, _ = s.start([3])
+    assert rc == 0
+    logits = s.logits()
+    assert np.max(np.abs(logits - ctx.logits())) <= 6e-3 * np.max(np.abs(logits)) and rel_l2(logits, ctx.logits()) <= 6e-3
+    rc, _, tokens = s.advance(1)
+    assert rc == 0 and tokens[0] == np.argmax(logits)
