@@ -669,10 +669,10 @@ hipError_t head_rows(Session *s, uint32_t row, uint32_t count, NervaHipHfDecodeS
   return launch_gemm_rows(s->dtype, kGemmF32, g, s->stream);
 }
 
-// Prompt tokens begin .. count-1 through every layer in blocks of up to prefill_block_tokens tokens, with the
-// prompt staging (16-bit hidden state between layers, prefill_kernels.cu:494-508): per block and
-// layer one RMSNorm launch, the qkv projection as a multi-row GEMM, the K/V rows of the block into the
-// cache, the attention of all its tokens in one launch (token z attends to keys 0 .. first + z), and
+// Prompt tokens begin .. count-1 through every layer in passes of up to prefill_pass_tokens tokens, with the
+// prompt staging (16-bit hidden state between layers, prefill_kernels.cu:494-508): per pass and
+// layer one RMSNorm launch, the qkv projection as a multi-row GEMM, the K/V rows of the pass into the
+// cache, the attention of its tokens, a block of prefill_block_tokens a launch (token z attends to keys 0 .. first + z), and
 // the o / gate-up / down projections as multi-row GEMMs. Leaves the device's cursor at `cursor`. The reference
 // prefills in chunks too (session_decode_prefill.inc.cu:1879-2243).
 // `wanted`, optional: places (relative to `begin`, ascending) whose logits go to host rows of `logits` as their block is
@@ -690,8 +690,8 @@ hipError_t prefill_blocks(Session *s, uint32_t begin, uint32_t count, uint32_t c
   const uint32_t prompt_splits = want_prompt_splits >= 1 && want_prompt_splits <= static_cast<int>(kAttnMaxSplits)
                                      ? static_cast<uint32_t>(want_prompt_splits)
                                      : 0u;
-  for (uint32_t first = begin; err == hipSuccess && first < count; first += s->prefill_block_tokens) {
-    const uint32_t T = std::min<uint32_t>(s->prefill_block_tokens, count - first);
+  for (uint32_t first = begin; err == hipSuccess && first < count; first += s->prefill_pass_tokens) {
+    const uint32_t T = std::min<uint32_t>(s->prefill_pass_tokens, count - first);
     const uint32_t tiles = block_operand_tiles(s, T);
     if (s->dtype == kBF16)
       hipLaunchKernelGGL(embed_rows_kernel<kBF16>, dim3(T), dim3(kBlock), 0, st, s->emb, s->prompt, first, H, s->vocab,
@@ -748,13 +748,15 @@ hipError_t prefill_blocks(Session *s, uint32_t begin, uint32_t count, uint32_t c
       a.ws_token_stride = s->pattn_ws_stride;
       a.out_packed_tiles = tiles;
       if (err == hipSuccess) err = launch_kv_publish_rows(s->dtype, a, st);
-      if (err == hipSuccess) {
-        if (rows_attention) {
-          err = launch_attn_decode(s->dtype, a, st);   // every token streams the prefix itself
-        } else {
-          a.splits = prompt_splits;                    // K/V tiles shared by the tokens of the block (0: the launcher chooses)
-          err = launch_attn_prompt(s->dtype, a, st);
-        }
+      if (!rows_attention) a.splits = prompt_splits;   // (0: the launcher chooses)
+      for (uint32_t at = 0; err == hipSuccess && at < T; at += s->prefill_block_tokens) {   // attention block by block
+        a.tokens = std::min(s->prefill_block_tokens, T - at);
+        if (rows_attention) err = launch_attn_decode(s->dtype, a, st);   // every token streams the prefix itself
+        else err = launch_attn_prompt(s->dtype, a, st);                  // K/V tiles shared by the tokens of the block
+        a.position += a.tokens;
+        a.qkv += static_cast<uint64_t>(a.tokens) * a.qkv_token_stride;
+        a.rope_cs = a.rope_cs != nullptr ? a.rope_cs + static_cast<uint64_t>(a.tokens) * a.rope_token_stride : nullptr;
+        a.out16 += a.tokens / 16u * 512u;   // (past the first block the rows are in operand order, a whole number of tiles further)
       }
       if (err == hipSuccess) {
         g = GemmRowsParams{};
@@ -815,7 +817,7 @@ hipError_t prefill_blocks(Session *s, uint32_t begin, uint32_t count, uint32_t c
         err = launch_gemm_rows(s->dtype, kGemmResidual, g, st);
       }
     }
-    if (err == hipSuccess) out->kernel_launches += 1 + (rows_attention ? 9ull : 10ull) * s->layers;
+    if (err == hipSuccess) out->kernel_launches += 1 + ((rows_attention ? 9ull : 10ull) + (T - 1) / s->prefill_block_tokens) * s->layers;
     while (err == hipSuccess && wanted_count != 0 && begin + *wanted < first + T) {
       // a run of wanted places side by side
       uint32_t run = 1;
@@ -895,11 +897,11 @@ hipError_t prompt_tokens(Session *s, uint32_t begin, uint32_t end, const uint32_
   // that the hook acts first)
   if (!s->block_prefill) {
     for (uint32_t i = begin; err == hipSuccess && i + 1 < end; ++i) err = launch_step(s, 1, out);
-  } else if (n % s->prefill_block_tokens != 1 && tuning(kTuneAttnWithholdSplit) == 0) {
+  } else if (n % s->prefill_pass_tokens != 1 && tuning(kTuneAttnWithholdSplit) == 0) {
     // every token in blocks; the head then reads the last one's row. With the place before it wanted too, its logits come
     // with the others' through one stream of the head, and the sampler reads them there.
     const bool with_others = wanted_count > 1 && wanted[wanted_count - 1] == last && wanted[wanted_count - 2] + 1 == last &&
-                             last % s->prefill_block_tokens != 0;
+                             last % s->prefill_pass_tokens != 0;
     const uint32_t ahead = wanted_count != 0 && wanted[wanted_count - 1] == last && !with_others ? wanted_count - 1 : wanted_count;
     err = prefill_blocks(s, begin, end, end - 1, end, wanted, ahead, logits, out);
     if (err != hipSuccess) return err;
@@ -911,7 +913,7 @@ hipError_t prompt_tokens(Session *s, uint32_t begin, uint32_t end, const uint32_
       out->kernel_launches += 2;
       return err;
     }
-    const GemvParams p = head_launch(s, s->px + static_cast<uint64_t>(last % s->prefill_block_tokens) * s->hidden);
+    const GemvParams p = head_launch(s, s->px + static_cast<uint64_t>(last % s->prefill_pass_tokens) * s->hidden);
     uint32_t head_blocks = 0;
     err = launch_gemv(s->dtype, kProRmsNorm, kEpiArgmax, p, s->stream, nullptr, &head_blocks);
     if (err == hipSuccess) err = head_sample(s, p.sample, head_blocks);
@@ -978,7 +980,9 @@ hipError_t setup_state(Session *s, int32_t *failure_stage, bool with_weights) {
   const uint64_t off_attn_plan = c.take(attn_plan_bytes(kAttnMaxSplits));
   const uint64_t off_attn_tagged = c.take(attn_step_workspace_bytes(s->heads));
   const uint64_t off_sample_ws = c.take(sample_workspace_bytes());
-  const uint64_t pT = kGemmDeepMaxTokens;
+  // A prompt's pass: eight blocks, fewer where the context has no room for as many tokens
+  const uint64_t pB = kGemmDeepMaxTokens;
+  const uint64_t pT = std::max<uint64_t>(pB, std::min<uint64_t>(kGemmPassMaxTokens, (s->max_ctx + pB - 1) / pB * pB));
   const uint64_t off_px = c.take(pT * H * 4);
   const uint64_t off_pr = c.take(pT * H * 4);
   const uint64_t off_pqkv = c.take(pT * (A + 2 * KV) * 4);
@@ -987,8 +991,9 @@ hipError_t setup_state(Session *s, int32_t *failure_stage, bool with_weights) {
   const uint64_t off_pff16 = c.take(pT * I * 2);
   const uint64_t off_prope = c.take(pT * HD * 4);
   const uint64_t pattn_ws_stride = (attn_ws_bytes + 255u) & ~uint64_t{255};
-  const uint64_t off_pattn_ws = c.take(pT * pattn_ws_stride);
-  const uint64_t pgemm_ws_bytes = gemm_block_workspace_bytes(static_cast<uint32_t>(std::max<uint64_t>(H, A + 2 * KV)));
+  const uint64_t off_pattn_ws = c.take(pB * pattn_ws_stride);
+  const uint64_t widest = std::max<uint64_t>(H, A + 2 * KV);   // (a pass's partial sums: two slices of the widest)
+  const uint64_t pgemm_ws_bytes = std::max(gemm_block_workspace_bytes(static_cast<uint32_t>(widest)), 2 * pT * widest * sizeof(float));
   const uint64_t off_pgemm_ws = c.take(pgemm_ws_bytes);
   const uint64_t off_sampler_dev = c.take(sizeof(SamplerDev));
   const uint64_t off_sampler_keys = c.take(sampler_workspace_bytes(s->vocab));
@@ -1057,11 +1062,17 @@ hipError_t setup_state(Session *s, int32_t *failure_stage, bool with_weights) {
            gemm_rows_takes(kGemmSwiglu, s->intermediate, s->hidden, tokens, pgemm_ws_bytes) &&
            gemm_rows_takes(kGemmResidual, s->hidden, s->intermediate, tokens, pgemm_ws_bytes);
   };
+  // A pass of the layers takes up to eight blocks of 512 through the projections together: an 8192 token prompt and 64 steps
+  // of 36 layers of 4096 x 12288 take 382 ms with passes of 512 tokens, 356 / 336 / 332 with 1024 / 2048 / 4096 (a page of
+  // 900 tokens 3584 wide: 11.3 and 10.8).
   const int block_cap = tuning(kTunePrefillBlockTokens);
   // (a prompt's last block can have any size: larger blocks only where every smaller one has its kernel too)
   const bool wide = block_cap != 128 && tuning(kTuneBlockLayout) != 1 && all_four(kGemmMaxTokens + 1) && all_four(kGemmWideMaxTokens);
   const bool deep = wide && block_cap != 256 && all_four(kGemmWideMaxTokens + 1) && all_four(kGemmDeepMaxTokens);
   s->prefill_block_tokens = deep ? kGemmDeepMaxTokens : wide ? kGemmWideMaxTokens : kGemmMaxTokens;
+  s->prefill_pass_tokens = !deep ? s->prefill_block_tokens
+                           : block_cap >= 512 ? std::min(static_cast<uint32_t>(pT), static_cast<uint32_t>(block_cap) / 512u * 512u)
+                                              : static_cast<uint32_t>(pT);
   s->blogits = head_block ? reinterpret_cast<float *>(s->arena + off_blogits) : nullptr;
   s->btable = reinterpret_cast<BatchTable *>(s->arena + off_btable);
   s->bslots = reinterpret_cast<Slot *>(s->arena + off_bslots);
@@ -1093,7 +1104,7 @@ hipError_t setup_state(Session *s, int32_t *failure_stage, bool with_weights) {
   if (err == hipSuccess) err = hipMemsetAsync(s->arena + off_attn_plan, 0, attn_plan_bytes(kAttnMaxSplits), s->stream);
   if (err == hipSuccess) err = hipMemsetAsync(s->arena + off_attn_tagged, 0, attn_step_workspace_bytes(s->heads), s->stream);
   if (err == hipSuccess) err = hipMemsetAsync(s->arena + off_sample_ws, 0, sample_workspace_bytes(), s->stream);
-  if (err == hipSuccess) err = hipMemsetAsync(s->arena + off_pattn_ws, 0, pT * pattn_ws_stride, s->stream);
+  if (err == hipSuccess) err = hipMemsetAsync(s->arena + off_pattn_ws, 0, pB * pattn_ws_stride, s->stream);
   if (err == hipSuccess && L > 0) err = hipMemsetAsync(s->arena + off_attn_trace, 0, L * 32 * 8, s->stream);
   if (err == hipSuccess) err = hipMemsetAsync(s->arena + off_kc, 0, 2 * ((kv_half + 255) & ~uint64_t{255}), s->stream);
   if (err == hipSuccess) err = hipMemsetAsync(s->slots, 0, static_cast<uint64_t>(s->max_ctx) * sizeof(Slot), s->stream);

@@ -619,14 +619,17 @@ __global__ __launch_bounds__(PAIRS * 2 * kWave, 2) void gemm_wide_kernel(GemmRow
 }
 
 // ---------------------------------------------------------------------------------------------
-// Token blocks of 257..512 rows (X in operand order with 32 token tiles; blocks of 129..256 where the kernel above does
-// not take the shape). What bounds the kernel above is what a
+// Token blocks of 257..4096 rows (X in operand order, 16 token tiles per 256 rows; blocks of 129..256 where the kernel above
+// does not take the shape). What bounds the kernel above is what a
 // CU has to pull in, not its matrix cores: every workgroup of 128 weight rows fetches the whole X block from L2
 // (twice the weight bytes per launch), ten operand pieces cross the LDS port for every sixteen products, and every
 // X block is written to LDS through registers. A block of 512 tokens lets a workgroup take 256 weight rows (a
 // gate/up pair: 128 + 128) x 256 tokens - one half of the block - so that a byte of X is fetched by half as many
 // workgroups and a byte of W still by two (the two halves of a row group run on the same XCD, next to each other
-// in dispatch order: the second finds the rows in that L2):
+// in dispatch order: the second finds the rows in that L2). With several blocks in one launch there are more such
+// workgroups than CUs without K slices, the start and the end of a launch come once, and partial sums are written and
+// read by nobody: per 512 of 4096 rows 74 us instead of 92 for a gate/up pair of 12288 x 4096 (1.38 PFLOP/s), 38 instead
+// of 52 + 17 for 4096 x 12288 and 15 instead of 26 + 17 for 4096 x 4096:
 //   * grid: one dimension, workgroup L -> XCD L % 8 (the hardware deals them round robin), and within an XCD
 //     (unit, half) with the half running fastest; unit = (row group, K slice);
 //   * 8 waves = 4 row quarters x 2 token halves of 128, a wave holds 4 row tiles x 8 token tiles of accumulators
@@ -642,7 +645,8 @@ __global__ __launch_bounds__(PAIRS * 2 * kWave, 2) void gemm_wide_kernel(GemmRow
 //     in flight - and every LDS operand read is issued by hand with a counted wait (the compiler's own
 //     bookkeeping falls back to "everything" once direct-to-LDS requests are pending).
 // ---------------------------------------------------------------------------------------------
-constexpr uint32_t kDTokCap = 512;                      // token rows at most; the token stride of this kernel's partial sums
+constexpr uint32_t kDTokCap = 512;                      // token stride of this kernel's partial sums, of blocks of up to as many rows
+__host__ __device__ __forceinline__ uint32_t deep_token_stride(uint32_t tokens) { return tokens <= kDTokCap ? kDTokCap : (tokens + 255u) / 256u * 256u; }
 constexpr int kDK = 64;                                 // columns per K-block
 constexpr int kDXBuf = 2 * 16 * kWave * static_cast<int>(sizeof(u32x4_t));   // one X block of a half: 2 K-steps x 16 tiles = 32 KiB
 constexpr int kDWTile = 16 * kDK * static_cast<int>(sizeof(uint16_t));       // one W tile of a block: 2 KiB
@@ -896,7 +900,7 @@ __global__ __launch_bounds__(8 * kWave, 2) void gemm_deep_kernel(GemmRowsParams 
     }
   } else {
     const uint32_t wrows = EPI == kGemmSwiglu ? 2u * p.rows : p.rows;
-    float *part = partials + static_cast<uint64_t>(slice) * kDTokCap * wrows;
+    float *part = partials + static_cast<uint64_t>(slice) * deep_token_stride(T) * wrows;
 #pragma unroll
     for (int c = 0; c < 8; ++c) {
       const uint32_t t = half * 256u + (th * 8 + c) * 16u + n;
@@ -967,15 +971,15 @@ inline double deep_us(int epilogue, uint32_t rows, uint32_t cols, uint32_t token
          partials_us(rows, tokens, plan.kslices);
 }
 
-// Shapes that divide (rows into workgroups, K into pairs of blocks) of more than 256 token rows: the tile height whose
-// busiest CU has the least to do - rounds of 256 workgroups x rows a workgroup x columns a slice. Other shapes and smaller
-// blocks, and those where it is clearly ahead (512 rows of 3584 x 18944, whose K halves twice into pairs of blocks: 112
+// Shapes that divide (rows into workgroups, K into pairs of blocks) of 257 to 512 token rows: the tile height whose
+// busiest CU has the least to do - rounds of 256 workgroups x rows a workgroup x columns a slice. Other shapes, smaller
+// and larger blocks, and those where it is clearly ahead (512 rows of 3584 x 18944, whose K halves twice into pairs of blocks: 112
 // workgroups in 4 slices, 224 in 8): the tile height and the K slices - any number, a slice is a run of whole K-blocks - of
 // the shortest estimate.
 inline DeepPlan deep_plan(int epilogue, uint32_t rows, uint32_t cols, uint32_t tokens, uint64_t workspace_bytes) {
   DeepPlan even{0, 0};
-  if (tokens <= kBTokCap || tokens > kDTokCap || cols % kDK != 0 || rows % 8u != 0) return even;
-  if (tokens > kWTokCap && cols % (2u * kDK) == 0) {
+  if (tokens <= kBTokCap || tokens > kGemmPassMaxTokens || cols % kDK != 0 || rows % 8u != 0) return even;
+  if (tokens > kWTokCap && tokens <= kDTokCap && cols % (2u * kDK) == 0) {
     uint64_t best_cost = ~uint64_t{0};
     for (int tpw = 4; tpw >= 3; --tpw) {
       const uint32_t slices = deep_slices_for(epilogue, rows, cols, tpw, workspace_bytes);
@@ -1000,7 +1004,7 @@ inline DeepPlan deep_plan(int epilogue, uint32_t rows, uint32_t cols, uint32_t t
   };
   for (int tpw = 4; tpw >= 3; --tpw)
     for (uint32_t slices = 1; slices <= 8u && slices * 4u <= cols / kDK; ++slices) {
-      if (slices > 1 && (epilogue == kGemmSwiglu || static_cast<uint64_t>(slices) * kDTokCap * rows * sizeof(float) > workspace_bytes)) break;
+      if (slices > 1 && (epilogue == kGemmSwiglu || static_cast<uint64_t>(slices) * deep_token_stride(tokens) * rows * sizeof(float) > workspace_bytes)) break;
       consider(DeepPlan{tpw, slices});
     }
   if (even.tpw != 0 && deep_us(epilogue, rows, cols, tokens, even) * 0.9 <= least) return even;
@@ -1031,7 +1035,7 @@ hipError_t launch_deep(const GemmRowsParams &p, float *partials, const DeepPlan 
                                  : (ragged ? launch_deep_tpw<DT, EPI, 4, true>(p, partials, kslices, stream)
                                            : launch_deep_tpw<DT, EPI, 4, false>(p, partials, kslices, stream));
   if (err == hipSuccess && kslices > 1) {
-    err = launch_finish<DT, EPI>(p, partials, kslices, kDTokCap, stream);
+    err = launch_finish<DT, EPI>(p, partials, kslices, deep_token_stride(p.tokens), stream);
   }
   return err;
 }

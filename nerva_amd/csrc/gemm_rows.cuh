@@ -25,6 +25,7 @@ namespace nv {
 constexpr uint32_t kGemmMaxTokens = 128;       // token rows of a block in any layout
 constexpr uint32_t kGemmWideMaxTokens = 256;   // token rows of a block in operand order, where gemm_wide_slices takes the shape
 constexpr uint32_t kGemmDeepMaxTokens = 512;   // ... where gemm_deep_slices takes the shape
+constexpr uint32_t kGemmPassMaxTokens = 4096;  // the same kernel's limit (sessions' prompts; the operator and the stacks stay with 512)
 
 // Operand order of a block of token rows X[t][k] (16-bit), the layout the multi-row GEMM reads fastest:
 // for every K-step of 32 columns and every tile of 16 tokens the 64 lanes' 16-byte pieces in lane order,
@@ -40,7 +41,7 @@ __host__ __device__ __forceinline__ uint64_t gemm_x_block_index(uint32_t tiles, 
 }
 // Token tiles the GEMM works with for a block of `tokens` rows (its X buffer in operand order has as many).
 __host__ __device__ __forceinline__ uint32_t gemm_packed_tiles(uint32_t tokens) {
-  return tokens > 256u ? 32u : tokens > 128u ? 16u : tokens > 64u ? 8u : tokens > 32u ? 4u : 2u;
+  return tokens > 512u ? (tokens + 255u) / 256u * 16u : tokens > 256u ? 32u : tokens > 128u ? 16u : tokens > 64u ? 8u : tokens > 32u ? 4u : 2u;
 }
 // kGemmXielu: a plain projection whose outputs leave as round16(xielu(y)) (activations.cuh).
 enum : int { kGemmF32 = 0, kGemmResidual = 1, kGemmSwiglu = 2, kGemmXielu = 3 };
@@ -114,7 +115,7 @@ hipError_t launch_gemm_wide(uint32_t dtype, int epilogue, const GemmRowsParams &
 // Estimated time of that launch (gemm_rows_route), and of the one below.
 double gemm_wide_us(int epilogue, uint32_t rows, uint32_t cols, uint32_t tokens, uint32_t kslices);
 double gemm_deep_us(int epilogue, uint32_t rows, uint32_t cols, uint32_t tokens, uint64_t workspace_bytes);
-// Blocks of 129..kGemmDeepMaxTokens rows in operand order: the same for the kernel that takes 256 or 192 rows x 256
+// Blocks of 129..kGemmPassMaxTokens rows in operand order: the same for the kernel that takes 256 or 192 rows x 256
 // tokens per workgroup (rows a multiple of 8, cols of 64).
 uint32_t gemm_deep_slices(int epilogue, uint32_t rows, uint32_t cols, uint32_t tokens, uint64_t workspace_bytes);
 hipError_t launch_gemm_deep(uint32_t dtype, int epilogue, const GemmRowsParams &p, uint32_t kslices, hipStream_t stream);

@@ -83,8 +83,8 @@ struct NervaHipHfDecodeSequenceSession {
   hipGraph_t graph[3] = {nullptr, nullptr, nullptr};
   hipGraphExec_t exec[3] = {nullptr, nullptr, nullptr};
   uint64_t graph_nodes[3] = {0, 0, 0};
-  // prompt blocks: up to prefill_block_tokens prompt tokens per pass through the layers (weights streamed
-  // once per block on the matrix cores); false = one prompt step per token
+  // prompt blocks: up to prefill_pass_tokens prompt tokens per pass through the layers (weights streamed
+  // once per pass on the matrix cores); false = one prompt step per token
   bool block_prefill = false;
   // the multi-row kernels take this model's shapes (prompt blocks and batch steps need it)
   bool rows_ready = false;
@@ -100,6 +100,7 @@ struct NervaHipHfDecodeSequenceSession {
   uint64_t pattn_ws_stride = 0;
   char *pgemm_ws = nullptr;        // partial sums of the K-sliced projections of a prompt block
   uint64_t pgemm_ws_bytes = 0;
+  uint32_t prefill_pass_tokens = nv::kGemmMaxTokens;    // tokens a pass of the layers takes: a block, or several where the projections take them together
   uint32_t prefill_block_tokens = nv::kGemmMaxTokens;   // tokens per prompt block: 512 or 256 where every projection has the kernel for it
   nv::SamplerDev sampler{};            // normalised configuration of the active sequence
   nv::SamplerDev *sampler_dev = nullptr;

@@ -92,6 +92,43 @@ def test_prompt_blocks_match_the_token_walk(geom):
         session.destroy()
 
 
+@pytest.mark.parametrize("geom", [WIDTHS[2], WIDTHS[3], (F16, 2048, 16, 4, 128, 4096, 1000, 2, 1e6, True, False)])
+def test_passes_of_several_blocks_match_single_blocks(geom):
+    """A pass takes the projections of several blocks of 512 together: one row into the second, an edge of 256, the largest
+    pass (4096) and one row, and a block, past it; in a prompt that starts behind another (not at a block's edge)."""
+    dtype, hidden, heads, kv, hd, inter, vocab, layers, theta, qk_norm, bias = geom
+    weights, _ = random_model(dtype, hidden, heads, kv, hd, inter, vocab, layers, hidden, theta, qk_norm, bias)
+    s = N.DecodeSession.create(weights, 4800)
+    N.Device.set_tuning("prefill_block_tokens", 512)
+    try:
+        single = N.DecodeSession.create(weights, 4800)
+    finally:
+        N.Device.set_tuning("prefill_block_tokens", 0)
+    assert s.create_result.prefill_chunk_tokens == single.create_result.prefill_chunk_tokens == 512
+    rng = np.random.default_rng(hidden)
+    for n in (513, 769, 1024, 1500, 4097, 4650):
+        prompt = rng.integers(0, vocab, n).astype(np.uint32)
+        for session in (s, single):
+            rc, res = session.start(prompt)
+            assert rc == 0 and res.hot_path_allocations == 0
+        assert rel_l2(s.logits(), single.logits()) <= E2E_REL_L2, n
+        for layer in range(layers):
+            for got, want in zip(s.kv_range(layer, 0, n), single.kv_range(layer, 0, n)):
+                tol = 2e-3 if layer == 0 else E2E_REL_L2
+                assert rel_l2(O.decode16(dtype, got), O.decode16(dtype, want)) <= tol, (n, layer)
+    places = [0, 511, 600, 601, 602, 1088]
+    head, more = rng.integers(0, vocab, 77).astype(np.uint32), rng.integers(0, vocab, 1089).astype(np.uint32)
+    rows = []
+    for session in (s, single):
+        session.start(head)
+        rc, _, logits, _ = session.extend(more, places)
+        assert rc == 0
+        rows.append(logits)
+    assert rel_l2(rows[0], rows[1]) <= E2E_REL_L2
+    for session in (s, single):
+        session.destroy()
+
+
 @pytest.mark.parametrize("geom,count", [(WIDTHS[2], 2), (WIDTHS[2], 17), (WIDTHS[3], 5), (WIDTHS[3], 32), (WIDTHS[4], 3)])
 def test_batch_steps_match_sequences_alone(geom, count):
     """The rows every sequence appends in batch steps are those it appends alone on the same history."""
