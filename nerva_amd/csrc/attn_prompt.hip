@@ -19,7 +19,7 @@
 // and the 16-deep product, blocks of 512 tokens of 32 heads over contexts 512 to 8192: 111.8 -> 82.7 us a launch on
 // average (85.8 without the turns), 0.94 PFLOP/s with the hi and lo halves counted, where the products of the same block
 // reach 1.1.
-// Grid (kv head, split of the prefix, token group); split partials go to the per-token workspaces the decode kernel uses
+// Grid (kv head, split of the prefix, token group, the last one first); split partials go to the per-token workspaces the decode kernel uses
 // and a small second launch merges them.
 #include <algorithm>
 #include <mutex>
@@ -68,7 +68,7 @@ __global__ __launch_bounds__(kPW *kWave, 2) void attn_prompt_kernel(AttnParams p
   const int lane = threadIdx.x & (kWave - 1);
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
   const uint32_t kvh = blockIdx.x, split = blockIdx.y, S = gridDim.y, T = p.tokens;
-  const uint32_t group_first = blockIdx.z * kGroupTokens;
+  const uint32_t group_first = (gridDim.z - 1 - blockIdx.z) * kGroupTokens;   // the longest prefix first
   const uint32_t group_last = min(T, group_first + kGroupTokens) - 1;
   uint32_t bps, active, nblk;
   prompt_splits(p.position + group_last, S, bps, active, nblk);
@@ -432,6 +432,32 @@ hipError_t launch_dt(const AttnParams &p, uint32_t splits, hipStream_t stream) {
 }
 
 }  // namespace
+
+// Several blocks in one launch need no splits and no merge once their workgroups fill the chip: with two workgroups a CU,
+// the longest prefixes first, a long one is followed by a short one. Both sides in steps of 64 keys a workgroup; a
+// launch and its merge count as three. (Eight blocks of 32 heads in two passes over 8192 positions: 16 launches in four
+// splits 2.50 ms with the merges 2.88, two without splits 2.10.)
+uint32_t attn_prompt_launch_tokens(uint32_t heads, uint32_t kv_heads, uint32_t position, uint32_t tokens, uint32_t block) {
+  const uint32_t group_tokens = kPW * (kCols / (heads / kv_heads)), groups = (tokens + group_tokens - 1) / group_tokens;
+  const auto steps = [&](uint32_t last) { return (position + std::min(last, tokens)) / 64u + 1u; };   // of a token group that ends there
+  if (tokens <= block || kv_heads * groups < 192u) return std::min(tokens, block);
+  const auto nth = [&](uint32_t i) { return steps((groups - i / kv_heads) * group_tokens); };   // i: place in launch order
+  uint64_t together = steps(tokens);
+  if (kv_heads * groups > 512u) {
+    uint64_t all = 0;
+    for (uint32_t g = 1; g <= groups; ++g) all += static_cast<uint64_t>(kv_heads) * steps(g * group_tokens);
+    together = std::max<uint64_t>(together, all / 256u + steps(group_tokens) / 2u);
+  } else if (kv_heads * groups > 256u) {
+    together = std::max<uint64_t>(together, nth(255) + nth(256));
+  }
+  uint64_t apart = 0;
+  for (uint32_t at = 0; at < tokens; at += block) {
+    const uint32_t last = std::min(at + block, tokens), wgs = kv_heads * ((last - at + group_tokens - 1) / group_tokens);
+    const uint32_t splits = (256u + wgs - 1) / wgs;
+    apart += 3u + static_cast<uint64_t>(steps(last)) * ((wgs * splits + 255u) / 256u) / splits;
+  }
+  return together < apart ? tokens : block;
+}
 
 hipError_t launch_attn_prompt(uint32_t dtype, const AttnParams &p, hipStream_t stream) {
   const uint32_t group = p.kv_heads != 0 ? p.heads / p.kv_heads : 0;

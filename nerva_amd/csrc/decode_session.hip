@@ -672,7 +672,7 @@ hipError_t head_rows(Session *s, uint32_t row, uint32_t count, NervaHipHfDecodeS
 // Prompt tokens begin .. count-1 through every layer in passes of up to prefill_pass_tokens tokens, with the
 // prompt staging (16-bit hidden state between layers, prefill_kernels.cu:494-508): per pass and
 // layer one RMSNorm launch, the qkv projection as a multi-row GEMM, the K/V rows of the pass into the
-// cache, the attention of its tokens, a block of prefill_block_tokens a launch (token z attends to keys 0 .. first + z), and
+// cache, the attention of its tokens, block by block or all in one launch (token z attends to keys 0 .. first + z), and
 // the o / gate-up / down projections as multi-row GEMMs. Leaves the device's cursor at `cursor`. The reference
 // prefills in chunks too (session_decode_prefill.inc.cu:1879-2243).
 // `wanted`, optional: places (relative to `begin`, ascending) whose logits go to host rows of `logits` as their block is
@@ -700,6 +700,9 @@ hipError_t prefill_blocks(Session *s, uint32_t begin, uint32_t count, uint32_t c
       hipLaunchKernelGGL(embed_rows_kernel<kF16>, dim3(T), dim3(kBlock), 0, st, s->emb, s->prompt, first, H, s->vocab,
                          s->px, rope_freq, s->prope, s->head_dim / 2);
     err = hipGetLastError();
+    const uint32_t attn_tokens = rows_attention || prompt_splits != 0
+                                     ? s->prefill_block_tokens
+                                     : attn_prompt_launch_tokens(s->heads, s->kv_heads, first, T, s->prefill_block_tokens);
     // Where a projection's slice-adding launch can write the following RMSNorm too, it does (one launch less each)
     const bool o_norms = gemm_rows_fuses_norm(kGemmResidual, H, A, T, tiles, s->pgemm_ws_bytes);
     const bool down_norms = gemm_rows_fuses_norm(kGemmResidual, H, I, T, tiles, s->pgemm_ws_bytes);
@@ -748,9 +751,9 @@ hipError_t prefill_blocks(Session *s, uint32_t begin, uint32_t count, uint32_t c
       a.ws_token_stride = s->pattn_ws_stride;
       a.out_packed_tiles = tiles;
       if (err == hipSuccess) err = launch_kv_publish_rows(s->dtype, a, st);
-      if (!rows_attention) a.splits = prompt_splits;   // (0: the launcher chooses)
-      for (uint32_t at = 0; err == hipSuccess && at < T; at += s->prefill_block_tokens) {   // attention block by block
-        a.tokens = std::min(s->prefill_block_tokens, T - at);
+      if (!rows_attention) a.splits = attn_tokens > s->prefill_block_tokens ? 1u : prompt_splits;   // (0: the launcher chooses)
+      for (uint32_t at = 0; err == hipSuccess && at < T; at += attn_tokens) {
+        a.tokens = std::min(attn_tokens, T - at);
         if (rows_attention) err = launch_attn_decode(s->dtype, a, st);   // every token streams the prefix itself
         else err = launch_attn_prompt(s->dtype, a, st);                  // K/V tiles shared by the tokens of the block
         a.position += a.tokens;
@@ -817,7 +820,7 @@ hipError_t prefill_blocks(Session *s, uint32_t begin, uint32_t count, uint32_t c
         err = launch_gemm_rows(s->dtype, kGemmResidual, g, st);
       }
     }
-    if (err == hipSuccess) out->kernel_launches += 1 + ((rows_attention ? 9ull : 10ull) + (T - 1) / s->prefill_block_tokens) * s->layers;
+    if (err == hipSuccess) out->kernel_launches += 1 + ((rows_attention ? 9ull : 10ull) + (T - 1) / attn_tokens) * s->layers;
     while (err == hipSuccess && wanted_count != 0 && begin + *wanted < first + T) {
       // a run of wanted places side by side
       uint32_t run = 1;
