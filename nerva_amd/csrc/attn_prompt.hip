@@ -47,9 +47,6 @@ __device__ __forceinline__ void prompt_splits(uint32_t last_pos, uint32_t S, uin
 
 constexpr uint32_t prompt_tile_bytes(int hd) { return kKvBlockTokens * hd * 2u; }
 constexpr uint32_t prompt_stage_bytes(int hd) { return 2u * kStepBlocks * prompt_tile_bytes(hd); }
-// (the f32 queries of sixteen columns a wave lie in the second and third stage until the walk begins)
-static_assert(kPW * 16 * 128 * sizeof(float) <= 2 * prompt_stage_bytes(128) && kPW * 16 * 64 * sizeof(float) <= 2 * prompt_stage_bytes(64),
-              "room for the queries");
 
 #define NV_PR_LDS(P) ((__attribute__((address_space(3))) void *)(P))
 
@@ -85,62 +82,93 @@ __global__ __launch_bounds__(kPW *kWave, 2) void attn_prompt_kernel(AttnParams p
     for (int i = 0; i < kPieces; ++i)
       __builtin_amdgcn_global_load_lds(reinterpret_cast<const u32x4_t *>(src + i * 512), NV_PR_LDS(at + i * 1024), 16, 0, 0);
   };
-  request(0);   // on its way while the queries are prepared
 
-  // ---- this wave's (token, head) pairs: bias, norm, rotation -> f32 q in LDS -> hi and lo operands
+  // ---- this wave's (token, head) pairs: bias, norm, rotation -> hi and lo operands. A lane fetches what it will hold of
+  // its column's pair, eight dims of every 32: both ends of each rotation are among them, the sum of squares takes two
+  // exchanges, and every input of the wave's pairs is requested at once.
   const uint32_t wave_first = group_first + wave * kTokensPerWave;   // may lie past the block: clamped, never stored
   const int col = lane & 15, grp = lane >> 4;
   u32x4_t qhi[2][kPieces], qlo[2][kPieces];
   uint32_t n_keys[2];
   {
-    float *q_s = reinterpret_cast<float *>(smem + kStage) + wave * 16 * HD;
-    // (every input of eight pairs requested first, unconditionally: one round trip instead of eight)
+    constexpr int kHalf = kPieces / 2;   // pieces of a rotation's first ends
     const bool has_bias = p.q_bias != nullptr, has_gamma = p.q_norm != nullptr, has_rope = p.rope_freq != nullptr;
     const uint16_t *bias_base = has_bias ? p.q_bias : p.k_cache;    // any readable address when unused
     const float *rope_base = has_rope ? p.rope_cs : p.qkv;
     const uint32_t rope_stride = has_rope ? p.rope_token_stride : 0u;
     const uint16_t *gamma_base = has_gamma ? p.q_norm : p.k_cache;
-    const int pl = pair_of<HD>(lane);
-    const float g0 = dec16<DT>(gamma_base[pl]), g1 = dec16<DT>(gamma_base[pl + HD / 2]);
+    f32x4_t x[2][kPieces][2], rc[2][kHalf][2], rs[2][kHalf][2];
+    u32x4_t bias[2][kPieces], gamma[kPieces];
+#pragma unroll
+    for (int c = 0; c < 2; ++c) {
+      const int vh = min(c * 16 + col, kPairs - 1);
+      const uint32_t tok = min(wave_first + vh / G, T - 1);
+      const uint32_t h = kvh * G + vh % G;
+      const float *src = p.qkv + static_cast<uint64_t>(tok) * p.qkv_token_stride + h * HD + grp * 8;
+      const float *rope = rope_base + static_cast<uint64_t>(tok) * rope_stride + grp * 8;
+#pragma unroll
+      for (int j = 0; j < kPieces; ++j) {
+#pragma unroll
+        for (int i = 0; i < 2; ++i) x[c][j][i] = *reinterpret_cast<const f32x4_t *>(src + j * 32 + i * 4);
+        bias[c][j] = *reinterpret_cast<const u32x4_t *>(bias_base + h * HD + j * 32 + grp * 8);
+      }
+#pragma unroll
+      for (int j = 0; j < kHalf; ++j)
+#pragma unroll
+        for (int i = 0; i < 2; ++i) {
+          rc[c][j][i] = *reinterpret_cast<const f32x4_t *>(rope + j * 32 + i * 4);
+          rs[c][j][i] = *reinterpret_cast<const f32x4_t *>(rope + HD / 2 + j * 32 + i * 4);
+        }
+      n_keys[c] = p.position + tok + 1;   // causal limit of the column
+    }
+#pragma unroll
+    for (int j = 0; j < kPieces; ++j) gamma[j] = *reinterpret_cast<const u32x4_t *>(gamma_base + j * 32 + grp * 8);
+    __builtin_amdgcn_sched_barrier(0);
+    request(0);   // the first tiles behind the inputs, on their way while the queries are prepared
+    if (steps > 1) request(1);
+    __builtin_amdgcn_sched_barrier(0);
+    const auto elem16 = [](const u32x4_t &v, int e) { return dec16<DT>(static_cast<uint16_t>(v[e / 2] >> (16 * (e % 2)))); };
     const float scale = kLog2e / sqrtf(static_cast<float>(HD));
 #pragma unroll
     for (int c = 0; c < 2; ++c) {
+      float y[kPieces][8], ss = 0.0f;
 #pragma unroll
-      for (int part = 0; part < 2; ++part) {   // eight pairs at a time: their inputs in one round trip
-        float x0[8], x1[8], rc[8], rs[8];
-        uint16_t qb0[8], qb1[8];
+      for (int j = 0; j < kPieces; ++j)
 #pragma unroll
-        for (int i = 0; i < 8; ++i) {
-          const int vh = min(c * 16 + part * 8 + i, kPairs - 1);
-          const uint32_t tok = min(wave_first + vh / G, T - 1);
-          const uint32_t h = kvh * G + vh % G;
-          const float *src = p.qkv + static_cast<uint64_t>(tok) * p.qkv_token_stride + h * HD;
-          x0[i] = src[pl];
-          x1[i] = src[pl + HD / 2];
-          qb0[i] = bias_base[h * HD + pl];
-          qb1[i] = bias_base[h * HD + pl + HD / 2];
-          rc[i] = rope_base[static_cast<uint64_t>(tok) * rope_stride + pl];
-          rs[i] = rope_base[static_cast<uint64_t>(tok) * rope_stride + HD / 2 + pl];
+        for (int e = 0; e < 8; ++e) {
+          y[j][e] = x[c][j][e / 4][e % 4];
+          if (has_bias) y[j][e] += elem16(bias[c][j], e);
+          ss += y[j][e] * y[j][e];
         }
+      if (has_gamma) {
+        ss += __shfl_xor(ss, 16, kWave);
+        ss += __shfl_xor(ss, 32, kWave);
+        const float norm = 1.0f / sqrtf(ss / static_cast<float>(HD) + p.eps);
 #pragma unroll
-        for (int i = 0; i < 8; ++i)
-          prep_head_core<DT, HD>(x0[i], x1[i], has_bias, dec16<DT>(qb0[i]), dec16<DT>(qb1[i]), has_gamma, g0, g1, has_rope, rc[i],
-                                 rs[i], p.eps, lane, q_s + (part * 8 + i) * HD, nullptr);
+        for (int j = 0; j < kPieces; ++j)
+#pragma unroll
+          for (int e = 0; e < 8; ++e) y[j][e] *= norm * elem16(gamma[j], e);
       }
-      // (written and read by this wave alone, in order)
+      if (has_rope) {
 #pragma unroll
-      for (int j = 0; j < kPieces; ++j) {
-        const float *src = q_s + col * HD + j * 32 + grp * 8;
+        for (int j = 0; j < kHalf; ++j)
+#pragma unroll
+          for (int e = 0; e < 8; ++e) {
+            const float y0 = y[j][e], y1 = y[j + kHalf][e], co = rc[c][j][e / 4][e % 4], si = rs[c][j][e / 4][e % 4];
+            y[j][e] = y0 * co - y1 * si;
+            y[j + kHalf][e] = y1 * co + y0 * si;
+          }
+      }
+#pragma unroll
+      for (int j = 0; j < kPieces; ++j)
 #pragma unroll
         for (int e = 0; e < 4; ++e) {
           uint16_t h0, l0, h1, l1;
-          split16<DT>(src[2 * e] * scale, h0, l0);
-          split16<DT>(src[2 * e + 1] * scale, h1, l1);
+          split16<DT>(y[j][2 * e] * scale, h0, l0);
+          split16<DT>(y[j][2 * e + 1] * scale, h1, l1);
           qhi[c][j][e] = h0 | (static_cast<uint32_t>(h1) << 16);
           qlo[c][j][e] = l0 | (static_cast<uint32_t>(l1) << 16);
         }
-      }
-      n_keys[c] = p.position + min(wave_first + min(c * 16 + col, kPairs - 1) / G, T - 1) + 1;   // causal limit of the column
     }
   }
   const bool wave_on = wave_first < T;
@@ -156,8 +184,6 @@ __global__ __launch_bounds__(kPW *kWave, 2) void attn_prompt_kernel(AttnParams p
 #pragma unroll
     for (int s2 = 0; s2 < HD / 16; ++s2) acc[c][s2] = f32x4_t{0.0f, 0.0f, 0.0f, 0.0f};
   }
-  __syncthreads();   // everyone has taken its queries: the second and third stage are free
-  if (steps > 1) request(1);
   const uint32_t lds0 = static_cast<uint32_t>(reinterpret_cast<uintptr_t>(NV_PR_LDS(smem))) + lane * 16u;
 
   // ---- the three parts of a step (skipped where no column of the wave sees it)
