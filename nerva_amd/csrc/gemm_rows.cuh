@@ -25,7 +25,7 @@ namespace nv {
 constexpr uint32_t kGemmMaxTokens = 128;       // token rows of a block in any layout
 constexpr uint32_t kGemmWideMaxTokens = 256;   // token rows of a block in operand order, where gemm_wide_slices takes the shape
 constexpr uint32_t kGemmDeepMaxTokens = 512;   // ... where gemm_deep_slices takes the shape
-constexpr uint32_t kGemmPassMaxTokens = 4096;  // the same kernel's limit (sessions' prompts; the operator and the stacks stay with 512)
+constexpr uint32_t kGemmPassMaxTokens = 4096;  // the same kernel's limit (sessions' prompts; the operator stays with 512)
 
 // Operand order of a block of token rows X[t][k] (16-bit), the layout the multi-row GEMM reads fastest:
 // for every K-step of 32 columns and every tile of 16 tokens the 64 lanes' 16-byte pieces in lane order,
@@ -33,11 +33,6 @@ constexpr uint32_t kGemmPassMaxTokens = 4096;  // the same kernel's limit (sessi
 // K-step; a buffer holds tiles * 16 token slots (slots past the block's tokens are never looked at).
 __host__ __device__ __forceinline__ uint64_t gemm_x_packed_index(uint32_t tiles, uint32_t t, uint32_t k) {
   return (static_cast<uint64_t>(k / 32u) * tiles + t / 16u) * 512u + (((k % 32u) / 8u) * 16u + t % 16u) * 8u + k % 8u;
-}
-// The same for rows past kGemmDeepMaxTokens: pieces of that many token rows, one after the other, each in operand order.
-__host__ __device__ __forceinline__ uint64_t gemm_x_block_index(uint32_t tiles, uint32_t t, uint32_t k, uint32_t cols) {
-  constexpr uint32_t kPiece = 512;
-  return static_cast<uint64_t>(t / kPiece) * kPiece * cols + gemm_x_packed_index(tiles, t % kPiece, k);
 }
 // Token tiles the GEMM works with for a block of `tokens` rows (its X buffer in operand order has as many).
 __host__ __device__ __forceinline__ uint32_t gemm_packed_tiles(uint32_t tokens) {

@@ -381,14 +381,11 @@ hipError_t parallel_step_16(Session *s) {
 
 // ---- blocks of token rows --------------------------------------------------------------------
 
-// Token tiles of the matrix-operand order a projection's input takes, 0 where its shape goes through gemm_any.
+// Token tiles of the matrix-operand order a projection's input takes, 0 where its shape goes through gemm_any (columns that
+// are no multiple of 32, or of 64 past 128 token rows; rows that are no multiple of 8 there, of 4 for an activation).
 uint32_t operand_tiles(const Session *s, int epilogue, uint32_t rows, uint32_t cols, uint32_t tokens) {
   if (wide(s) || cols % 32 != 0) return 0;
-  tokens = std::min(tokens, kGemmDeepMaxTokens);   // (larger blocks go in pieces)
-  const bool taken = tokens <= kGemmMaxTokens       ? gemm_rows_supported(rows, cols, tokens)
-                     : tokens <= kGemmWideMaxTokens ? gemm_wide_slices(epilogue, rows, cols, tokens, s->pgemm_ws_bytes) != 0
-                                                    : gemm_deep_slices(epilogue, rows, cols, tokens, s->pgemm_ws_bytes) != 0;
-  return taken ? gemm_packed_tiles(tokens) : 0u;
+  return gemm_rows_route(epilogue, rows, cols, tokens, s->pgemm_ws_bytes).kernel != kGemmNone ? gemm_packed_tiles(tokens) : 0u;
 }
 
 struct Block {
@@ -427,20 +424,6 @@ struct Block {
                      uint32_t out_tiles, const uint16_t *act) {
     launches += 1;
     const bool narrow = epilogue == kGemmXielu && !wide(s);
-    if (tiles != 0 && tokens > kGemmDeepMaxTokens) {
-      // pieces of kGemmDeepMaxTokens rows; the last one has the others' layout, so enough rows for that are multiplied
-      hipError_t err = hipSuccess;
-      const uint32_t all = tokens;
-      for (uint32_t at = 0; err == hipSuccess && at < all; at += kGemmDeepMaxTokens) {
-        tokens = std::min(kGemmDeepMaxTokens, std::max(all - at, kGemmWideMaxTokens + 1));
-        const uint64_t done = static_cast<uint64_t>(at) * rows;
-        err = project(epilogue, w, rows, cols, static_cast<const uint16_t *>(x) + static_cast<uint64_t>(at) * cols, tiles,
-                      narrow ? static_cast<void *>(static_cast<uint16_t *>(out) + done) : static_cast<void *>(static_cast<float *>(out) + done),
-                      out_tiles, act);
-      }
-      tokens = all;
-      return err;
-    }
     if (tiles != 0) {
       GemmRowsParams g{};
       g.w = w;
@@ -552,13 +535,20 @@ struct Block {
       if (wide(s)) g.out32 = static_cast<float *>(s->pmix);
       else g.out16 = static_cast<uint16_t *>(s->pmix);
       g.packed_tiles = out_tiles;
-      g.tokens = tokens;
       g.width = w.spec.width;
       if (at_cursor) {
         g.cursor = s->state;
         g.max_steps = s->max_ctx;
       }
-      err = launch_mingru_rows(s->dtype, g, s->stream);
+      // (as many tokens a launch as keep their gates in registers between the scan's two walks)
+      for (uint32_t at = 0; err == hipSuccess && at < tokens; at += kStackBlockTokens) {
+        g.tokens = std::min(kStackBlockTokens, tokens - at);
+        err = launch_mingru_rows(s->dtype, g, s->stream);
+        g.zxg += static_cast<uint64_t>(g.tokens) * 3u * g.width;
+        if (g.out32 != nullptr) g.out32 += static_cast<uint64_t>(g.tokens) * g.width;
+        else g.out16 += out_tiles != 0 ? g.tokens / 16u * 512u : g.tokens * g.width;   // (a whole number of tiles further)
+      }
+      launches += (tokens - 1) / kStackBlockTokens;
     }
     launches += 1;
     if (err == hipSuccess) err = project(kGemmF32, w.w_out, s->hidden, w.out_cols, s->pmix, out_tiles, s->py, 0, nullptr);
@@ -675,7 +665,7 @@ struct Block {
   // a block of one token, into `logits`. Leaves the residual rows as they are where rows are picked.
   hipError_t logits_of(const uint32_t *pick, uint32_t count, float *logits) {
     const StackModel &m = *s->stack;
-    const uint32_t tiles = !wide(s) && s->hidden % 32 == 0 && gemm_rows_supported(s->vocab, s->hidden, count) ? gemm_packed_tiles(count) : 0u;
+    const uint32_t tiles = operand_tiles(s, kGemmF32, s->vocab, s->hidden, count);
     hipError_t err;
     if (parallel(s)) {
       RmsRows r = rms_rows();
@@ -995,7 +985,11 @@ int create_stack(const NervaHipStackSessionCreateRequest *rq, bool synthetic, ui
   s->intermediate = m.max_ff;
   bool experts = !sandwich;
   for (const StackLayer &w : m.layers) experts = experts && w.spec.mixer == NERVA_HIP_MIXER_LATENT && w.spec.ff == 0;
-  if (experts) m.block_tokens = kExpertBlockTokens;
+  bool routed = false;
+  for (const StackLayer &w : m.layers) routed = routed || w.spec.experts != 0;
+  if (experts) m.block_tokens = m.chunk_tokens = kExpertBlockTokens;
+  else if (!routed && rq->precision != NERVA_HIP_PRECISION_32)
+    m.block_tokens = std::max(kStackBlockTokens, std::min(kGemmPassMaxTokens, (s->max_ctx + kStackBlockTokens - 1) / kStackBlockTokens * kStackBlockTokens));
   for (const StackLayer &w : m.layers)
     if (w.spec.experts != 0)
       m.plan_bytes = std::max(m.plan_bytes, moe_plan_bytes(m.block_tokens, w.spec.experts_per_token, w.spec.experts));
@@ -1210,7 +1204,7 @@ int create_stack(const NervaHipStackSessionCreateRequest *rq, bool synthetic, ui
   }
   out->failure_stage = 0;
   fill_create_result(s, out);
-  out->prefill_chunk_tokens = m.block_tokens;
+  out->prefill_chunk_tokens = m.chunk_tokens;
   out->h2d_bytes = h2d;
   out->sync_calls = syncs;
   out->status = 0;

@@ -18,7 +18,10 @@
 namespace nv {
 
 // Token rows a block holds at most. Layers of latents and experts take larger ones: an expert sees a few of a block's
-// tokens, and its weights are read once a block whatever it sees.
+// tokens, and its weights are read once a block whatever it sees. Without experts a block is several of these, up to
+// kGemmPassMaxTokens where the context has room: the projections take them together, in launches that need no K slices (3000
+// tokens through six layers of 4096 x 12288, one attention layer in two, and 24 steps: 23.0 -> 19.9 ms), and experts' blocks
+// were always several launches a projection (1800 tokens, five layers 2048 wide: 11.9 -> 11.0).
 constexpr uint32_t kStackBlockTokens = kGemmDeepMaxTokens, kExpertBlockTokens = 2048;
 
 // Tensors of one layer in device memory. Row-concatenated: w_in is [q; k; v; gate] ([q; gate] where the keys are
@@ -49,7 +52,8 @@ struct StackLayer {
 struct StackModel {
   std::vector<StackLayer> layers;
   uint32_t precision = NERVA_HIP_PRECISION_16;
-  uint32_t block_tokens = kStackBlockTokens;
+  uint32_t block_tokens = kStackBlockTokens;      // token rows the layers take at a time
+  uint32_t chunk_tokens = kStackBlockTokens;      // what a session reports
   uint32_t arrangement = NERVA_HIP_STACK_SANDWICH;
   float embedding_scale = 1.0f, logit_scale = 1.0f;
   const uint16_t *final_w = nullptr, *final_b = nullptr;

@@ -220,3 +220,14 @@ def test_ragged_head_takes_the_largest(hidden, vocab):
     assert np.max(np.abs(logits - ctx.logits())) <= 6e-3 * np.max(np.abs(logits)) and rel_l2(logits, ctx.logits()) <= 6e-3
     rc, _, tokens = s.advance(1)
     assert rc == 0 and tokens[0] == np.argmax(logits)
+
+
+@pytest.mark.parametrize("sizes", [[1400], [513, 300, 1, 586]], ids=str)
+def test_stack_blocks_of_widths_off_the_power_of_two_grid(sizes):
+    """Projections of a mixed stack in operand order at K of 3, 5 and 32 blocks of 64, in blocks past 512 token rows (with a
+    scan in several launches), whole and in portions, as the oracle has them."""
+    import stack_models as M
+    import test_gpu_mixed_stack as T
+    cfg = M.config([M.attention(16, 4, 128, 128, rot=32, chunk=700, ff=320), M.mingru(width=320, ff=448), M.mingru(width=64, ff=0)],
+                   width=192, vocab=300)
+    T.check(cfg, M.weights(cfg, seed=31), T.tokens_of(cfg, 1400, seed=9), sizes, 0)
