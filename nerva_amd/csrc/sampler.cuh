@@ -55,7 +55,7 @@ struct SamplerParams {
   const float *logits;
   uint32_t vocab;
   const SamplerDev *config;   // device memory
-  uint64_t *keys;             // [chunks][kSamplerTopKMax] workspace (top-k: word 0 of a row the chunk's best key, word 1 its finite count)
+  uint64_t *keys;             // [chunks][kSamplerTopKMax] workspace (top-k: word 0 of a row the chunk's best key, word 1 its finite count, then the maxima of its runs of 64)
   SampleParams out;           // chunk candidates (greedy / Gumbel), slot / cursor / plain token output
   const uint32_t *cursor;     // device position (slot index and random-number counter), or null -> position
   uint32_t position, max_steps;

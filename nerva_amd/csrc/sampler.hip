@@ -47,6 +47,10 @@ __device__ __forceinline__ uint32_t wanted_candidates(uint32_t top_k, uint32_t v
   return requested < vocab ? requested : vocab;  // sampler.cu:169-174
 }
 
+// Runs of 64 logits of a chunk, and where their maxima lie in its workspace row (a word is 64 bits).
+constexpr uint32_t kRuns = kSamplerChunk / kWave, kRunMaxWord = 2;
+static_assert(kRunMaxWord + kRuns / 2 <= kSamplerTopKMax && kSelectThreads * kRuns <= 65536, "room for the maxima; a run's number in 16 bits");
+
 // `batch` (device memory) replaces `p` by its entry blockIdx.y: one launch for several sequences.
 __global__ __launch_bounds__(kChunkThreads) void sample_chunk_kernel(SamplerParams p, const SamplerParams *batch) {
   if (batch != nullptr) p = batch[blockIdx.y];
@@ -98,19 +102,24 @@ __global__ __launch_bounds__(kChunkThreads) void sample_chunk_kernel(SamplerPara
     return;
   }
 
-  // top-k: the chunk's best key and the number of its finite logits (words 0 and 1 of the chunk's workspace row)
+  // top-k: the chunk's best key, the number of its finite logits, and the largest of each run of 64 (words 0, 1 and 2 ..
+  // of the chunk's workspace row)
   uint64_t best = 0;
   uint32_t finite = 0;
-  for (uint32_t e = threadIdx.x; e < kSamplerChunk; e += kChunkThreads) {
-    const uint32_t i = base + e;
-    if (i < p.vocab) {
-      const float v = p.logits[i];
-      if (isfinite(v)) {
-        const uint64_t key = make_key(v, i);
-        best = key > best ? key : best;
-        ++finite;
-      }
+  float *run_max = reinterpret_cast<float *>(p.keys + static_cast<uint64_t>(blockIdx.x) * kSamplerTopKMax + kRunMaxWord);
+#pragma unroll
+  for (uint32_t e0 = 0; e0 < kSamplerChunk; e0 += kChunkThreads) {
+    const uint32_t e = e0 + threadIdx.x, i = base + e;
+    const float v = p.logits[min(i, p.vocab - 1)];
+    const bool in = i < p.vocab && isfinite(v);
+    float most = in ? v : -INFINITY;
+    if (in) {
+      const uint64_t key = make_key(v, i);
+      best = key > best ? key : best;
+      ++finite;
     }
+    for (int o = kWave / 2; o > 0; o >>= 1) most = fmaxf(most, __shfl_xor(most, o, kWave));
+    if (e % kWave == 0) run_max[e / kWave] = most;
   }
   for (int o = kWave / 2; o > 0; o >>= 1) {
     const uint64_t other = (static_cast<uint64_t>(__shfl_xor(static_cast<uint32_t>(best >> 32), o, kWave)) << 32) |
@@ -134,6 +143,24 @@ __global__ __launch_bounds__(kChunkThreads) void sample_chunk_kernel(SamplerPara
   }
 }
 
+// ranks[i] += number of keys[0 .. n) above keys[i]. The keys are zero from n to the next multiple of eight. A wave takes 64
+// keys and a run of those they are compared with, one LDS read for all its lanes each: as many runs as there are waves for.
+__device__ __forceinline__ void count_above(const uint64_t *keys, uint32_t n, uint32_t *ranks) {
+  constexpr uint32_t kWaves = kSelectThreads / kWave;
+  const uint32_t groups = (n + kWave - 1) / kWave, runs = kWaves / groups;
+  const uint32_t wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave), run = wave / groups;
+  if (run >= runs) return;
+  const uint32_t place = (wave % groups) * kWave + threadIdx.x % kWave;
+  const uint32_t len = ((n + runs - 1) / runs + 7u) / 8u * 8u, end = min((run + 1) * len, (n + 7u) / 8u * 8u);
+  const uint64_t key = keys[min(place, n - 1)];
+  uint32_t above = 0;
+  for (uint32_t c = run * len; c < end; c += 8) {
+#pragma unroll
+    for (uint32_t u = 0; u < 8; ++u) above += keys[c + u] > key ? 1u : 0u;
+  }
+  if (place < n) atomicAdd(&ranks[place], above);
+}
+
 __global__ __launch_bounds__(kSelectThreads) void sample_select_kernel(SamplerParams p, uint32_t chunks,
                                                                       const SamplerParams *batch) {
   if (batch != nullptr) p = batch[blockIdx.y];
@@ -141,6 +168,8 @@ __global__ __launch_bounds__(kSelectThreads) void sample_select_kernel(SamplerPa
   __shared__ uint32_t scan[kSelectThreads];
   __shared__ uint64_t top[kSamplerTopKMax];
   __shared__ uint64_t cand[kSelectThreads];
+  __shared__ uint32_t look[kSamplerTopKMax];
+  __shared__ uint16_t runs[kSamplerTopKMax * kRuns];
   __shared__ float ex[kSamplerTopKMax];
   __shared__ float red_v[kSelectThreads / kWave];
   __shared__ uint32_t red_i[kSelectThreads / kWave];
@@ -197,39 +226,54 @@ __global__ __launch_bounds__(kSelectThreads) void sample_select_kernel(SamplerPa
   }
 
   // ---- fast path: a bound from the chunk maxima. The selected-th largest of the chunks' best keys is no
-  // larger than the selected-th largest key overall, so only keys at or above it matter: with logits spread
-  // over the chunks that leaves a few hundred of the whole vocabulary, which one pass over the logits collects
-  // and a sort in LDS orders. (Keys are distinct, so the order they are collected in does not show.)
+  // larger than the selected-th largest key overall, so only keys at or above it matter, and only the `selected` chunks
+  // whose best keys are: with logits spread over the chunks that leaves a few hundred keys, which one pass over those
+  // chunks collects and a sort in LDS orders. (Keys are distinct, so the order they are collected in does not show.)
   bool fast = chunks <= static_cast<uint32_t>(kSelectThreads);
   if (fast) {
     cand[tid] = tid < chunks ? p.keys[static_cast<uint64_t>(tid) * kSamplerTopKMax] : 0ull;
+    scan[tid] = 0;
     if (tid == 0) {
       prefix_s = 0;   // the bound: 0 (everything) when fewer chunks than `selected` hold a finite logit
       count_s = 0;
+      need_s = 0;
     }
     __syncthreads();
-    const uint64_t mine_max = cand[tid];
-    if (mine_max != 0ull) {
-      uint32_t above = 0;
-      for (uint32_t c = 0; c < chunks; ++c) above += cand[c] > mine_max ? 1u : 0u;
-      if (above == selected - 1) prefix_s = mine_max;   // distinct keys: exactly one chunk has this rank
-    }
+    count_above(cand, chunks, scan);
     __syncthreads();
+    const uint64_t chunk_max = cand[tid];
+    const uint32_t chunk_rank = scan[tid];
+    scan[tid] = 0;
+    if (chunk_max != 0ull && chunk_rank < selected) {
+      if (chunk_rank == selected - 1) prefix_s = chunk_max;   // distinct keys: exactly one chunk has this rank
+      look[chunk_rank] = tid;
+    }
+    const uint32_t looks = min(selected, static_cast<uint32_t>(__syncthreads_count(chunk_max != 0ull)));
     const uint64_t bound = prefix_s;
-    __syncthreads();
-    // One workgroup looks at every logit, so the look is two comparisons (a float at or above the bound's value,
-    // and finite); the key is formed and compared exactly only for the few that pass (forming every key was 15
-    // instructions a logit: 17 of the kernel's 36 us). Eight logits are requested before the first is looked at.
+    // Of those chunks only runs of 64 logits whose largest reaches the bound: one compute unit gets 30 bytes a nanosecond
+    // from where the head left its logits, and half a megabyte of them was 17 us. (The launch, top 128 of 151936: 32.3 us
+    // with every logit of the vocabulary looked at, keys ranked by a lane each and one lane summing; 16.6 now, 10.0 -> 7.9
+    // for the top 20.)
     const float bound_value = bound != 0ull ? key_value(bound) : -INFINITY;
-    constexpr uint32_t kScan = 8;
-    for (uint32_t i0 = tid; i0 < p.vocab; i0 += kScan * kSelectThreads) {
+    const uint32_t lane = tid % kWave;
+    for (uint32_t e = tid; e < looks * kRuns; e += kSelectThreads) {
+      const uint32_t chunk = look[e / kRuns];
+      const float most = reinterpret_cast<const float *>(p.keys + static_cast<uint64_t>(chunk) * kSamplerTopKMax + kRunMaxWord)[e % kRuns];
+      if (most >= bound_value) runs[atomicAdd(&need_s, 1u)] = static_cast<uint16_t>(chunk * kRuns + e % kRuns);
+    }
+    __syncthreads();
+    const uint32_t run_count = need_s;
+    // A wave takes four runs at a time. The look is two comparisons (a float at or above the bound's value, and finite);
+    // the key is formed and compared exactly only for the few that pass.
+    constexpr uint32_t kScan = 4, kStride = kScan * (kSelectThreads / kWave);
+    for (uint32_t r = tid / kWave * kScan; r < run_count; r += kStride) {
       float v[kScan];
 #pragma unroll
-      for (uint32_t u = 0; u < kScan; ++u) v[u] = p.logits[min(i0 + u * kSelectThreads, p.vocab - 1)];
+      for (uint32_t u = 0; u < kScan; ++u) v[u] = p.logits[min(runs[min(r + u, run_count - 1)] * kWave + lane, p.vocab - 1)];
 #pragma unroll
       for (uint32_t u = 0; u < kScan; ++u) {
-        const uint32_t i = i0 + u * kSelectThreads;
-        if (v[u] >= bound_value && fabsf(v[u]) <= 3.402823466e+38f && i < p.vocab) {   // (finite: a NaN passes neither)
+        const uint32_t i = runs[min(r + u, run_count - 1)] * kWave + lane;
+        if (r + u < run_count && v[u] >= bound_value && fabsf(v[u]) <= 3.402823466e+38f && i < p.vocab) {   // (finite: a NaN passes neither)
           const uint64_t key = make_key(v[u], i);
           if (key >= bound) {
             const uint32_t slot = atomicAdd(&count_s, 1u);
@@ -244,13 +288,11 @@ __global__ __launch_bounds__(kSelectThreads) void sample_select_kernel(SamplerPa
     if (fast) {
       // order by counting: a key's place is the number of keys above it (distinct keys: no two share a place)
       if (tid < kSamplerTopKMax) top[tid] = 0ull;
+      if (tid >= total && tid < total + 8u) cand[tid] = 0ull;
       __syncthreads();
-      if (tid < total) {
-        const uint64_t key = cand[tid];
-        uint32_t above = 0;
-        for (uint32_t c = 0; c < total; ++c) above += cand[c] > key ? 1u : 0u;
-        if (above < kSamplerTopKMax) top[above] = key;
-      }
+      count_above(cand, total, scan);
+      __syncthreads();
+      if (tid < total && scan[tid] < kSamplerTopKMax) top[scan[tid]] = cand[tid];
       __syncthreads();
     }
   }
@@ -330,25 +372,29 @@ __global__ __launch_bounds__(kSelectThreads) void sample_select_kernel(SamplerPa
   if (tid < selected) ex[tid] = expf((key_value(top[tid]) - max_value) * inv_temperature);
   __syncthreads();
   // The rule's three sums (total, nucleus, draw) are one running sum over the candidates in order, read at
-  // three places: lane 0 forms it once - sequential float additions, the rule's order, eight LDS values
-  // requested per turn - and the two searches ("first candidate whose running share reaches top_p", "first whose
-  // running sum reaches the draw") test every candidate at once.
-  if (tid == 0) {
-    float run = 0.0f;
-    for (uint32_t i0 = 0; i0 < selected; i0 += 8) {
-      float e[8];
+  // three places: a lane of the first wave adds up those before and at its own, one by one - sequential float additions,
+  // the rule's order; those behind count as zero - and the two searches ("first candidate whose running share reaches
+  // top_p", "first whose running sum reaches the draw") test every candidate at once.
+  if (tid < kWave) {
+    float before = 0.0f;
+    for (uint32_t i0 = 0; i0 < selected; i0 += kWave) {
+      const uint32_t left = min(selected - i0, static_cast<uint32_t>(kWave));
+      const float e = tid < left ? ex[i0 + tid] : 0.0f;
+      float run = before;
+      for (uint32_t i = 0; i < left; i += 8) {
 #pragma unroll
-      for (uint32_t u = 0; u < 8; ++u) e[u] = ex[min(i0 + u, selected - 1)];
-#pragma unroll
-      for (uint32_t u = 0; u < 8; ++u) {
-        if (i0 + u < selected) {
-          run += e[u];
-          ex[i0 + u] = run;
+        for (uint32_t u = 0; u < 8; ++u) {   // (past the last: zeros)
+          const float term = __uint_as_float(__builtin_amdgcn_readlane(__float_as_uint(e), i + u));
+          run += tid >= i + u ? term : 0.0f;
         }
       }
+      if (tid < left) ex[i0 + tid] = run;
+      before = __uint_as_float(__builtin_amdgcn_readlane(__float_as_uint(run), kWave - 1));
     }
-    need_s = selected;   // kept: candidates inside the nucleus
-    count_s = selected;  // first candidate at or above the draw
+    if (tid == 0) {
+      need_s = selected;   // kept: candidates inside the nucleus
+      count_s = selected;  // first candidate at or above the draw
+    }
   }
   __syncthreads();
   const float total = ex[selected - 1];

@@ -231,3 +231,31 @@ def test_stack_blocks_of_widths_off_the_power_of_two_grid(sizes):
     cfg = M.config([M.attention(16, 4, 128, 128, rot=32, chunk=700, ff=320), M.mingru(width=320, ff=448), M.mingru(width=64, ff=0)],
                    width=192, vocab=300)
     T.check(cfg, M.weights(cfg, seed=31), T.tokens_of(cfg, 1400, seed=9), sizes, 0)
+
+
+@pytest.mark.parametrize("n,kind", [(151937, "sorted"), (65601, "one run"), (40000, "equal"), (2112, "lowest"), (151936, "spread")])
+def test_top_k_collects_from_the_runs_that_hold_candidates(n, kind):
+    """Logits placed so that all candidates share a chunk, a run of 64, the end of the vocabulary, or tie (more of them than
+    are collected: the general selection), and with the type's lowest number as a logit like any other."""
+    from nerva_amd import abi
+    rng = np.random.default_rng(n)
+    l = rng.standard_normal(n).astype(np.float32)
+    if kind == "sorted":
+        l.sort()
+    elif kind == "one run":
+        l[n - 70:] += 50.0
+    elif kind == "equal":
+        l[:] = 1.5
+    elif kind == "lowest":
+        l[:] = -np.finfo(np.float32).max
+        l[[3, 64, n - 1]] = [1.0, 2.0, 3.0]
+    buf, ws = dev(l), N.DeviceBuffer.zeros(abi.load().nerva_hip_sample_workspace_bytes(n))
+    close = 0
+    for top_k in (1, 2, 40, 127, 128, 0):
+        for position in range(4):
+            want, margin = O.sample(l, 0.9, 0.97, top_k, 11, position)
+            got = N.sample(buf, n, 0.9, 0.97, top_k, 11, position, ws)
+            if got != want:   # (a draw within rounding of a boundary, as in the rule's own test)
+                assert margin < 1e-5, (top_k, position, got, want, margin)
+                close += 1
+    assert close <= 1
