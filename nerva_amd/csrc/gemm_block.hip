@@ -293,7 +293,7 @@ template <uint32_t DT>
 __global__ __launch_bounds__(kFinNormThreads) void gemm_finish_norm_kernel(GemmRowsParams p, const float *partials, uint32_t kslices,
                                                                          uint32_t tokcap) {
   __shared__ float red[kFinNormThreads / kWave];
-  const uint32_t t = blockIdx.x, rows = p.rows;
+  const uint32_t t = tile_row_of(blockIdx.x, gridDim.x), rows = p.rows;
   float4 v[kFinNormPerLane];
   float ss = 0.0f;
 #pragma unroll

@@ -34,6 +34,12 @@ constexpr uint32_t kGemmPassMaxTokens = 4096;  // the same kernel's limit (sessi
 __host__ __device__ __forceinline__ uint64_t gemm_x_packed_index(uint32_t tiles, uint32_t t, uint32_t k) {
   return (static_cast<uint64_t>(k / 32u) * tiles + t / 16u) * 512u + (((k % 32u) / 8u) * 16u + t % 16u) * 8u + k % 8u;
 }
+// Token row of workgroup `b` in a launch of one workgroup a row that writes operand order: the sixteen rows of a tile share
+// its cache lines, so they go to one XCD (workgroups are dealt out round robin), whose L2 puts the lines together (4096
+// normalised rows of 4096: 42.5 -> 31.8 us, with a seam's sum in front 43.8 -> 38.1).
+__device__ __forceinline__ uint32_t tile_row_of(uint32_t b, uint32_t rows) {
+  return b < rows / 128u * 128u ? b / 128u * 128u + b % 8u * 16u + b % 128u / 8u : b;
+}
 // Token tiles the GEMM works with for a block of `tokens` rows (its X buffer in operand order has as many).
 __host__ __device__ __forceinline__ uint32_t gemm_packed_tiles(uint32_t tokens) {
   return tokens > 512u ? (tokens + 255u) / 256u * 16u : tokens > 256u ? 32u : tokens > 128u ? 16u : tokens > 64u ? 8u : tokens > 32u ? 4u : 2u;

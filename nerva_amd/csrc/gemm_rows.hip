@@ -203,7 +203,8 @@ template <uint32_t DT>
 __global__ __launch_bounds__(kNormThreads) void rmsnorm_rows_kernel(const float *x, const uint16_t *gamma, float eps,
                                                                     uint32_t cols, uint16_t *out16, uint32_t packed_tiles) {
   __shared__ float red[kNormThreads / kWave];
-  const float *row = x + static_cast<uint64_t>(blockIdx.x) * cols;
+  const uint32_t t = tile_row_of(blockIdx.x, gridDim.x);
+  const float *row = x + static_cast<uint64_t>(t) * cols;
   float4 v[kNormPerLane];
   float ss = 0.0f;
 #pragma unroll
@@ -220,7 +221,7 @@ __global__ __launch_bounds__(kNormThreads) void rmsnorm_rows_kernel(const float 
 #pragma unroll
   for (int w = 0; w < kNormThreads / kWave; ++w) total += red[w];
   const float scale = 1.0f / sqrtf(total / static_cast<float>(cols) + eps);
-  uint16_t *out = out16 + static_cast<uint64_t>(blockIdx.x) * cols;
+  uint16_t *out = out16 + static_cast<uint64_t>(t) * cols;
 #pragma unroll
   for (int i = 0; i < kNormPerLane; ++i) {
     const uint32_t c = (i * kNormThreads + threadIdx.x) * 4;
@@ -233,7 +234,7 @@ __global__ __launch_bounds__(kNormThreads) void rmsnorm_rows_kernel(const float 
       o.x = enc16<DT>(v[i].x * scale * g0) | (static_cast<uint32_t>(enc16<DT>(v[i].y * scale * g1)) << 16);
       o.y = enc16<DT>(v[i].z * scale * g2) | (static_cast<uint32_t>(enc16<DT>(v[i].w * scale * g3)) << 16);
       // four consecutive columns stay together in operand order too (c % 8 is 0 or 4)
-      if (packed_tiles != 0) *reinterpret_cast<uint2 *>(out16 + gemm_x_packed_index(packed_tiles, blockIdx.x, c)) = o;
+      if (packed_tiles != 0) *reinterpret_cast<uint2 *>(out16 + gemm_x_packed_index(packed_tiles, t, c)) = o;
       else *reinterpret_cast<uint2 *>(out + c) = o;
     }
   }

@@ -10,7 +10,7 @@ namespace {
 template <uint32_t DT, int WG>
 __global__ __launch_bounds__(WG *kWave) void join_rows_kernel(JoinRows p) {
   __shared__ float red[WG * 3];
-  const uint32_t row = blockIdx.x, src = p.pick != nullptr ? p.pick[row] : row, cols = p.cols;
+  const uint32_t row = tile_row_of(blockIdx.x, gridDim.x), src = p.pick != nullptr ? p.pick[row] : row, cols = p.cols;
   JoinNorm j;
   float *x = p.x + static_cast<uint64_t>(src) * cols;
   j.x = x;
@@ -34,7 +34,7 @@ __global__ __launch_bounds__(WG *kWave) void join_rows_vec_kernel(JoinRows p) {
   extern __shared__ __align__(16) uint16_t h[];
   __shared__ float red[WG * 3];
   constexpr uint32_t TB = WG * kWave;
-  const uint32_t row = blockIdx.x, src = p.pick != nullptr ? p.pick[row] : row, cols = p.cols;
+  const uint32_t row = tile_row_of(blockIdx.x, gridDim.x), src = p.pick != nullptr ? p.pick[row] : row, cols = p.cols;
   JoinNorm j;
   float *x = p.x + static_cast<uint64_t>(src) * cols;
   j.x = x;

@@ -40,7 +40,7 @@ template <uint32_t DT, int WG, int V>
 __global__ __launch_bounds__(WG *kWave) void rms_rows_kernel(RmsRows p) {
   __shared__ float red[WG];
   constexpr uint32_t TB = WG * kWave;
-  const uint32_t row = blockIdx.x, src = p.pick != nullptr ? p.pick[row] : row, cols = p.cols;
+  const uint32_t row = tile_row_of(blockIdx.x, gridDim.x), src = p.pick != nullptr ? p.pick[row] : row, cols = p.cols;
   const uint64_t base = static_cast<uint64_t>(src) * cols;
   const float *weights = p.slot_rows != nullptr ? p.slot_weights + static_cast<uint64_t>(src) * p.slots : nullptr;
   const bool add = p.y[0] != nullptr || p.y[1] != nullptr || p.slot_rows != nullptr;

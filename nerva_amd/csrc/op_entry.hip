@@ -591,7 +591,7 @@ int nerva_hip_gemm_rows(const NervaHipGemmRowsRequest *r, void *stream, int32_t 
 uint64_t nerva_hip_gemm_rows_workspace_bytes(uint32_t rows) { return gemm_block_workspace_bytes(rows); }
 
 uint64_t nerva_hip_gemm_operand_index(uint32_t tokens, uint32_t token, uint32_t column) {
-  return gemm_x_packed_index(gemm_packed_tiles(tokens), token, column);
+  return gemm_x_packed_index(gemm_packed_tiles(std::min(tokens, kGemmDeepMaxTokens)), token, column);
 }
 
 int nerva_hip_rmsnorm_rows(uint32_t dtype, const float *x, const uint16_t *gamma, float eps, uint32_t tokens,
