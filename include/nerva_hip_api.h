@@ -583,7 +583,7 @@ int nerva_hip_gemv(const NervaHipGemvRequest *request, void *stream, int32_t *hi
 
 /* The launch shape nerva_hip_gemv (and the session's step) chooses for a request of these sizes with
  * 16-byte-aligned pointers: *kernel, low four bits = 0 scalar, 1 guarded vector, 2 full vector, 3 the lean
- * production-shape kernel; bit 4 = the lean kernel walks its rows from a rotated start; bits 8 and up = 1 KiB
+ * kernel (rows of whole cache lines); bit 4 = the lean kernel walks its rows from a rotated start; bits 8 and up = 1 KiB
  * chunks of a row per request batch; *workgroups = the grid. Host arithmetic only (no device is touched):
  * measurements taken for one launch shape (counter profiles) are keyed to it. No counterpart. */
 int nerva_hip_gemv_launch_shape(uint32_t prologue, uint32_t epilogue, uint32_t rows, uint32_t cols,
@@ -645,7 +645,7 @@ int nerva_hip_paged_attention_status(void *workspace, uint32_t heads, uint32_t h
 /* Element offset of (layer, physical block, kv_head, token-in-block, dim) in the K (is_value 0)
  * or V (is_value 1) cache array. A (block, kv_head) tile of 16 tokens x head_dim elements is
  * contiguous; inside it the order is the library's own (matrix-core operand order at head_dim
- * 128, row-major otherwise), so hosts that fill or read a cache go through this function. */
+ * 64 and 128, row-major otherwise), so hosts that fill or read a cache go through this function. */
 uint64_t nerva_hip_kv_cache_offset(uint32_t block_count, uint32_t kv_heads, uint32_t head_dim,
                                    uint32_t layer, uint32_t physical_block, uint32_t kv_head,
                                    uint32_t token_in_block, uint32_t dim, uint32_t is_value);
@@ -875,8 +875,8 @@ int nerva_hip_steps_are_eager(void);
 /* Reads back the f32 logits of the last sampled position (vocab_size floats) and
  * one KV row (kv_heads*head_dim 16-bit values each for K and V) for parity tests. */
 /* 1 when a batch step led by this session streams the weights once for all its sequences (the
- * model's shapes fit the multi-row kernels: head_dim 128, GQA factor 1/2/4/8, K dimensions multiples
- * of 2048), 0 when every sequence of such a step runs its own decode step; -1 for a null session. */
+ * model's shapes fit the multi-row kernels: head_dim 64 or 128, up to 8 query heads a key head, widths multiples of 32,
+ * at least 4.5 MiB of weights a layer), 0 when every sequence of such a step runs its own decode step; -1 for a null session. */
 int nerva_hip_session_shares_weight_stream(NervaHipHfDecodeSequenceSession *session);
 int nerva_hip_session_read_logits(NervaHipHfDecodeSequenceSession *session, float *host_logits);
 /* Test hook (no counterpart): copies `count` token slots, from slot `first`, out of the session's device memory

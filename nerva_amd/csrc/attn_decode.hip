@@ -99,7 +99,7 @@ __global__ __launch_bounds__(W *kWave, W / 2) void attn_block_kernel(AttnParams 
 }
 
 // ---------------------------------------------------------------------------------------------
-// The decode step's launch: one token, grid (kv_heads, splits), 8 waves, G = 1, 2, 4 or 8 query heads per
+// The decode step's launch: one token, grid (kv_heads, splits), 8 waves, G = 1 to 8 query heads per
 // kv head. Same arithmetic as attn_fast_body (same tile step, same merges); what differs is the order
 // in which a wave asks for things, because at decode sizes - a wave owns two or three 8 KiB tiles of an
 // 8k-token context - the launch is one burst of requests and a chain of latencies, not a stream:
