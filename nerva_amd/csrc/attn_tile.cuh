@@ -244,6 +244,19 @@ __device__ __forceinline__ void attn_tile(uint4 (&kreg)[HD / 32], uint4 (&vreg)[
       }
     }
   }
+  if (!COLUMN_MASKS && (b + 1) * kKvBlockTokens > n_keys) {
+    // The last tile's rows past the position hold whatever was there: their probabilities are 0, and so are the values
+    // they meet (0 x NaN or infinity would not be)
+    const uint32_t at = b * kKvBlockTokens + grp * 4, rows = n_keys > at ? n_keys - at : 0u;   // of this lane's four
+    const uint32_t first = rows == 0 ? 0u : rows == 1 ? 0xffffu : ~0u, second = rows <= 2 ? 0u : rows == 3 ? 0xffffu : ~0u;
+#pragma unroll
+    for (int j = 0; j < HD / 32; ++j) {
+      vreg[j].x &= first;
+      vreg[j].y &= second;
+      vreg[j].z &= first;
+      vreg[j].w &= second;
+    }
+  }
   // scores of tokens b*16 + grp*4 + r for column col
   f32x4_t c{0.0f, 0.0f, 0.0f, 0.0f};
 #pragma unroll
