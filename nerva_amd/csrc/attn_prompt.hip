@@ -55,6 +55,9 @@ constexpr uint32_t prompt_stage_bytes(int hd) { return 2u * kStepBlocks * prompt
 #define NV_PR_READ(DST, AT, OFF) asm volatile("ds_read_b128 %0, %1 offset:%2" : "=v"(DST) : "v"(AT), "n"(OFF) : "memory")
 #define NV_PR_AWAIT2(N_, A_, B_) asm volatile("s_waitcnt lgkmcnt(%2)" : "+v"(A_), "+v"(B_) : "n"(N_) : "memory")
 
+template <uint32_t DT>
+__device__ __forceinline__ bool finite16(uint16_t bits) { return (bits & 0x7fffu) < (DT == kBF16 ? 0x7f80u : 0x7c00u); }
+
 template <uint32_t DT, int HD, int G>
 __global__ __launch_bounds__(kPW *kWave, 2) void attn_prompt_kernel(AttnParams p) {
   constexpr int kTokensPerWave = kCols / G, kPairs = kTokensPerWave * G;   // (columns kPairs .. 31 repeat the last pair, unused)
@@ -330,33 +333,108 @@ __global__ __launch_bounds__(kPW *kWave, 2) void attn_prompt_kernel(AttnParams p
   // ---- results of the wave's pairs: token rows of the four lane groups
   const uint64_t ml_off = reinterpret_cast<char *>(p.part_m) - reinterpret_cast<char *>(p.part_acc);
   const uint64_t l_off = reinterpret_cast<char *>(p.part_l) - reinterpret_cast<char *>(p.part_acc);
+  uint32_t spoilt[2];   // columns with a sum that is not finite
+#pragma unroll
+  for (int c = 0; c < 2; ++c) {
+    float zero = 0.0f;
+#pragma unroll
+    for (int s2 = 0; s2 < HD / 16; ++s2)
+#pragma unroll
+      for (int r = 0; r < 4; ++r) zero = fmaf(acc[c][s2][r], 0.0f, zero);
+    const uint64_t lanes = __ballot(zero != 0.0f);   // (NaN)
+    spoilt[c] = static_cast<uint32_t>(lanes | (lanes >> 16) | (lanes >> 32) | (lanes >> 48)) & 0xffffu;
+  }
+  if ((spoilt[0] | spoilt[1]) != 0) {
+    // 0 x NaN or infinity is NaN: a value that is not finite may have come in by a key that the column does not see - of a
+    // later token of its step, or a row not written yet. Where there is such a value behind the least limit of the wave's
+    // columns, their sums are formed once more below, over the keys they see.
+    uint32_t found = 0;
+    for (uint32_t b = max(b0, least_keys / kKvBlockTokens); b < nblk; ++b) {
+      const uint16_t *tile = p.v_cache + kv_tile_offset(p.block_count, p.kv_heads, HD, p.layer, p.table[b], kvh) + lane * 8;
+#pragma unroll
+      for (int i = 0; i < kPieces * 8; ++i) found |= finite16<DT>(tile[i / 8 * 512 + i % 8]) ? 0u : 1u;
+    }
+    if (!__any(found != 0)) spoilt[0] = spoilt[1] = 0;
+  }
 #pragma unroll
   for (int c = 0; c < 2; ++c) {
     float lc = l[c];
     lc += __shfl_xor(lc, 16, kWave);
     lc += __shfl_xor(lc, 32, kWave);
+    l[c] = lc;
     const int pair = c * 16 + col;
     const uint32_t tok = wave_first + pair / G, h = kvh * G + pair % G;
     if (pair >= kPairs || tok >= T) continue;
     const float inv = lc > 0.0f && isfinite(lc) ? 1.0f / lc : 1.0f;
     char *ws = reinterpret_cast<char *>(p.part_acc) + static_cast<uint64_t>(tok) * p.ws_token_stride;
+    if (((spoilt[c] >> col) & 1u) == 0) {
 #pragma unroll
-    for (int s2 = 0; s2 < HD / 16; ++s2) {
-      const float4 o = make_float4(acc[c][s2][0], acc[c][s2][1], acc[c][s2][2], acc[c][s2][3]);
-      const uint32_t d = s2 * 16 + grp * 4;
-      if (active == 1) {
-        // a single split holds every key: final
-        uint2 packed;
-        packed.x = enc16<DT>(o.x * inv) | (static_cast<uint32_t>(enc16<DT>(o.y * inv)) << 16);
-        packed.y = enc16<DT>(o.z * inv) | (static_cast<uint32_t>(enc16<DT>(o.w * inv)) << 16);
-        *reinterpret_cast<uint2 *>(p.out16 + attn_out_token(p, tok) + attn_out_elem(p, h * HD + d)) = packed;   // d % 4 == 0
-      } else {
-        *reinterpret_cast<float4 *>(reinterpret_cast<float *>(ws) + (static_cast<uint64_t>(h) * S + split) * HD + d) = o;
+      for (int s2 = 0; s2 < HD / 16; ++s2) {
+        const float4 o = make_float4(acc[c][s2][0], acc[c][s2][1], acc[c][s2][2], acc[c][s2][3]);
+        const uint32_t d = s2 * 16 + grp * 4;
+        if (active == 1) {
+          // a single split holds every key: final
+          uint2 packed;
+          packed.x = enc16<DT>(o.x * inv) | (static_cast<uint32_t>(enc16<DT>(o.y * inv)) << 16);
+          packed.y = enc16<DT>(o.z * inv) | (static_cast<uint32_t>(enc16<DT>(o.w * inv)) << 16);
+          *reinterpret_cast<uint2 *>(p.out16 + attn_out_token(p, tok) + attn_out_elem(p, h * HD + d)) = packed;   // d % 4 == 0
+        } else {
+          *reinterpret_cast<float4 *>(reinterpret_cast<float *>(ws) + (static_cast<uint64_t>(h) * S + split) * HD + d) = o;
+        }
       }
     }
     if (active != 1 && grp == 0) {
       reinterpret_cast<float *>(ws + ml_off)[h * S + split] = m[c];
       reinterpret_cast<float *>(ws + l_off)[h * S + split] = lc;
+    }
+  }
+  // ---- the sums of spoilt columns, one after the other: the query again (a lane has a rotation's two ends), scores of 64
+  // keys at a time (a lane a key), then their values in key order (a lane its two dims)
+  if (__builtin_expect((spoilt[0] | spoilt[1]) == 0, 1)) return;
+  for (int pair = 0; pair < kPairs; ++pair) {
+    const uint32_t tok = wave_first + pair / G, h = kvh * G + pair % G;
+    if (((spoilt[pair / 16] >> (pair % 16)) & 1u) == 0 || tok >= T) continue;
+    const int at = pair_of<HD>(lane);
+    const float *src = p.qkv + static_cast<uint64_t>(tok) * p.qkv_token_stride + h * HD;
+    const float *rope = p.rope_freq != nullptr ? p.rope_cs + static_cast<uint64_t>(tok) * p.rope_token_stride : p.qkv;
+    const bool has_bias = p.q_bias != nullptr, has_gamma = p.q_norm != nullptr;
+    float q0 = src[at], q1 = src[at + HD / 2];
+    head_values<DT, HD>(q0, q1, has_bias, has_bias ? dec16<DT>(p.q_bias[h * HD + at]) : 0.0f,
+                        has_bias ? dec16<DT>(p.q_bias[h * HD + at + HD / 2]) : 0.0f, has_gamma, has_gamma ? dec16<DT>(p.q_norm[at]) : 0.0f,
+                        has_gamma ? dec16<DT>(p.q_norm[at + HD / 2]) : 0.0f, p.rope_freq != nullptr, rope[at], rope[HD / 2 + at], p.eps);
+    const float scale = kLog2e / sqrtf(static_cast<float>(HD));
+    q0 *= scale;
+    q1 *= scale;
+    const float most = __shfl(pair < 16 ? m[0] : m[1], pair % 16, kWave), sum = __shfl(pair < 16 ? l[0] : l[1], pair % 16, kWave);
+    const uint32_t end = min((b0 + steps * kStepBlocks) * kKvBlockTokens, p.position + tok + 1);
+    float o0 = 0.0f, o1 = 0.0f;
+    for (uint32_t k0 = b0 * kKvBlockTokens; k0 < end; k0 += kWave) {
+      const uint32_t key = min(k0 + lane, end - 1);
+      const uint64_t tile = kv_tile_offset(p.block_count, p.kv_heads, HD, p.layer, p.table[key / kKvBlockTokens], kvh);
+      float score = 0.0f;
+      for (uint32_t d = 0; d < HD / 2; ++d) {
+        score = fmaf(__shfl(q0, d, kWave), dec16<DT>(p.k_cache[tile + kv_k_elem(HD, key % kKvBlockTokens, d)]), score);
+        score = fmaf(__shfl(q1, d, kWave), dec16<DT>(p.k_cache[tile + kv_k_elem(HD, key % kKvBlockTokens, d + HD / 2)]), score);
+      }
+      const float weight = attn_exp2(score - most);
+      for (uint32_t i = 0; i < min(end - k0, static_cast<uint32_t>(kWave)); ++i) {
+        const uint64_t row = kv_tile_offset(p.block_count, p.kv_heads, HD, p.layer, p.table[(k0 + i) / kKvBlockTokens], kvh);
+        const float w = __shfl(weight, i, kWave);
+        o0 = fmaf(w, dec16<DT>(p.v_cache[row + kv_v_elem(HD, (k0 + i) % kKvBlockTokens, at)]), o0);
+        o1 = fmaf(w, dec16<DT>(p.v_cache[row + kv_v_elem(HD, (k0 + i) % kKvBlockTokens, at + HD / 2)]), o1);
+      }
+    }
+    if (lane >= HD / 2) continue;
+    if (active == 1) {
+      const float inv = sum > 0.0f && isfinite(sum) ? 1.0f / sum : 1.0f;
+      uint16_t *out = p.out16 + attn_out_token(p, tok);
+      out[attn_out_elem(p, h * HD + at)] = enc16<DT>(o0 * inv);
+      out[attn_out_elem(p, h * HD + at + HD / 2)] = enc16<DT>(o1 * inv);
+    } else {
+      float *part = reinterpret_cast<float *>(reinterpret_cast<char *>(p.part_acc) + static_cast<uint64_t>(tok) * p.ws_token_stride) +
+                    (static_cast<uint64_t>(h) * S + split) * HD;
+      part[at] = o0;
+      part[at + HD / 2] = o1;
     }
   }
 }

@@ -6,8 +6,9 @@ import pytest
 import nerva_amd as N
 import oracle as O
 from nerva_amd.runtime import attention_workspace
+from test_gpu_any_width import walked
 from test_gpu_ops import _attention_case, _attention_oracle, dev
-from test_gpu_session import BF16, F16, REL_L2, rel_l2
+from test_gpu_session import BF16, E2E_REL_L2, F16, REL_L2, random_model, rel_l2
 
 pytestmark = pytest.mark.gpu
 
@@ -32,3 +33,77 @@ def test_rows_behind_the_position_may_hold_anything(heads, kv_heads, hd, dtype):
                           out_f32=out32, append=True, rope_theta=1e4)
         assert rel_l2(out32.numpy(np.float32), ref) <= REL_L2, tokens
 
+
+# hidden, heads, kv, hd, inter, vocab, layers; half precision, whose largest number is in reach
+OVERFLOWING = [(192, 10, 2, 64, 320, 301, 2), (896, 14, 2, 64, 1728, 300, 2), (768, 6, 2, 128, 1536, 300, 2), (2048, 16, 4, 128, 4096, 300, 2)]
+
+
+def overflowing_model(geom):
+    """A model one of whose tokens (0) has a value past the largest number in dims 5 and 40 of its first layer's key head 1:
+    its embedding is constant, the other tokens' have no constant part, and those dims sum the embedding up."""
+    hidden, heads, kv, hd, inter, vocab, layers = geom
+    weights, _ = random_model(F16, hidden, heads, kv, hd, inter, vocab, layers, hidden, 1e4, False, False)
+    rng = np.random.default_rng(hidden)
+    table = rng.normal(0, 1, (vocab, hidden))
+    table -= table.mean(axis=1, keepdims=True)
+    table[0] = 1.0
+    weights.embeddings[:] = O.encode16(F16, table).reshape(weights.embeddings.shape)
+    weights.layers[0]["rms_attn"][:] = O.encode16(F16, np.ones(hidden))
+    w_v = weights.layers[0]["w_v"].reshape(kv * hd, hidden)
+    w_v[[hd + 5, hd + 40]] = O.encode16(F16, np.full(hidden, 1e5 / hidden))
+    return weights
+
+
+@pytest.mark.parametrize("geom", OVERFLOWING, ids=str)
+def test_a_later_tokens_infinity_does_not_reach_earlier_tokens(geom):
+    """A prompt with the overflowing token in it: at its start, inside and at the edges of a step of 64 keys, and behind a
+    prefix long enough for splits. The tokens before it have the logits that a walk token by token gives them; those that see
+    it have none that are finite, as there."""
+    weights = overflowing_model(geom)
+    s, walk = N.DecodeSession.create(weights, 900), walked(weights, 900)
+    assert s.create_result.prefill_chunk_tokens > 1 and walk.create_result.prefill_chunk_tokens == 1
+    rng = np.random.default_rng(7)
+    for prefix, tokens, at in ((0, 3, 1), (0, 70, 9), (0, 70, 63), (0, 130, 64), (650, 40, 20), (650, 150, 149)):
+        prompt = rng.integers(1, weights.vocab, prefix + tokens).astype(np.uint32)
+        prompt[prefix + at] = 0
+        places = sorted({0, at // 2, max(0, at - 3), at - 1, min(at + 2, tokens - 1)})
+        rows = []
+        for session in (s, walk):
+            assert session.release_sequence() == 0
+            if prefix:
+                rc, _, _, _ = session.extend(prompt[:prefix])
+                assert rc == 0
+            rows.append(session.extend(prompt[prefix:], places)[2])
+        for place, got, want in zip(places, *rows):
+            assert np.all(np.isfinite(want)) == (place < at), (prefix, at, place)
+            if place < at:
+                assert rel_l2(got, want) <= E2E_REL_L2, (prefix, at, place)
+            else:
+                assert not np.any(np.isfinite(got)), (prefix, at, place)
+    for session in (s, walk):
+        session.destroy()
+
+
+@pytest.mark.parametrize("geom", OVERFLOWING, ids=str)
+def test_an_earlier_sequences_rows_do_not_reach_the_next(geom):
+    """A session whose cache holds infinities of the sequence before, up to behind the next one's end: prompt, steps and
+    logits are those of a session that has held nothing else."""
+    weights = overflowing_model(geom)
+    used, fresh = N.DecodeSession.create(weights, 128), N.DecodeSession.create(weights, 128)
+    used.extend(np.zeros(100, np.uint32))
+    assert used.release_sequence() == 0
+    for length in (1, 2, 21, 64, 70):
+        prompt = np.random.default_rng(length).integers(1, weights.vocab, length).astype(np.uint32)
+        results = []
+        for session in (used, fresh):
+            rc, _ = session.start(prompt)
+            assert rc == 0
+            rc, _, tokens = session.advance(4)
+            assert rc == 0
+            results.append((tokens.tolist(), session.logits().copy()))
+            assert session.release_sequence() == 0
+        assert np.all(np.isfinite(results[1][1])) and rel_l2(results[0][1], results[1][1]) <= E2E_REL_L2, length
+        top = np.sort(results[1][1])
+        assert results[0][0][:1] == results[1][0][:1] or top[-1] - top[-2] <= E2E_REL_L2 * np.max(np.abs(top)), length
+    for session in (used, fresh):
+        session.destroy()
