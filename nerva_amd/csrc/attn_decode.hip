@@ -242,10 +242,18 @@ __device__ __forceinline__ void sload8x2(const uint32_t *a, const uint32_t *b, u
                : "memory");
 }
 
+// The shapes of attn_f32_shape keep an f32's 24 bits of queries and probabilities here, in three 16-bit parts: the third ones
+// have operands of their own (with G up to 8 there is no room in the sixteen columns), twelve matrix instructions a tile
+// more (28 heads on 4, keys in cache: 7.8 -> 7.9 us a launch at 900 keys, 8.5 -> 8.8 at 8000; 32 heads of 64 on 8: 8.2 -> 8.4). Error of the f32 output against 64 bits, 28 heads on 4, 75 / 900 / 4000 keys, bf16: the
+// general kernel 1.6 / 3.1 / 6.2e-7, two parts 2.9 / 2.7 / 2.9e-6, three 1.9 / 2.4 / 2.5e-7.
+// The kernels of prompts and batches have two: they leave 16-bit outputs only, which a third part does not move (1.68375e-3,
+// 1.63985e-3 and 1.69469e-3 from 64 bits with three and with f32; with two 1.63986e-3 for the second and the others the same).
 template <int HD, int G>
 struct StepShared {
   static constexpr int kRow = HD + 8;      // 272-byte rows (HD = 64: 144): the operand reads of a lane group spread over the banks
-  alignas(16) uint16_t qhl[2 * G][kRow];   // Qx columns: rows 0..G-1 the hi halves of the scaled query heads, G..2G-1 the lo halves
+  static constexpr int kParts = attn_f32_shape(HD, G) ? 3 : 2;
+  alignas(16) uint16_t qhl[kParts * G][kRow];   // Qx columns: rows 0..G-1 the hi parts of the scaled query heads, G..2G-1 the next, 2G..3G-1 the third
+  float qdown[G];                          // attn_scaled: 1 / the power of two the head was multiplied with
   alignas(16) uint16_t knew[HD];
   alignas(16) uint16_t vnew[HD];
   float wm[8][G], wl[8][G];
@@ -301,6 +309,7 @@ template <uint32_t DT, int HD, int G>
 __global__ __launch_bounds__(8 * kWave) void attn_step_kernel(AttnParams p) {
   constexpr int W = 8;
   constexpr int kThreads = W * kWave;
+  constexpr bool kF32Parts = attn_f32_shape(HD, G);
   __shared__ StepShared<HD, G> sh;
   const int lane = threadIdx.x & (kWave - 1);
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
@@ -398,8 +407,24 @@ __global__ __launch_bounds__(8 * kWave) void attn_step_kernel(AttnParams p) {
     // softmax runs in base 2 on scores scaled by 1/sqrt(d): both folded into the query
     const float scale = kLog2e / sqrtf(static_cast<float>(HD));
     uint16_t h0, l0, h1, l1;
-    split16<DT>(x0 * scale, h0, l0);
-    split16<DT>(x1 * scale, h1, l1);
+    if constexpr (kF32Parts) {
+      uint16_t t0, t1;
+      x0 *= scale;
+      x1 *= scale;
+      if constexpr (attn_scaled<DT, HD, G>()) {
+        const int up = attn_query_exponent(wave_max(fmaxf(fabsf(x0), fabsf(x1))));
+        x0 = ldexpf(x0, up);
+        x1 = ldexpf(x1, up);
+        if (lane == 0) sh.qdown[wave] = ldexpf(1.0f, -up);
+      }
+      split16<DT>(x0, h0, l0, t0);
+      split16<DT>(x1, h1, l1, t1);
+      sh.qhl[2 * G + wave][pl] = t0;
+      sh.qhl[2 * G + wave][pl + HD / 2] = t1;
+    } else {
+      split16<DT>(x0 * scale, h0, l0);
+      split16<DT>(x1 * scale, h1, l1);
+    }
     sh.qhl[wave][pl] = h0;
     sh.qhl[wave][pl + HD / 2] = h1;
     sh.qhl[G + wave][pl] = l0;
@@ -443,6 +468,16 @@ __global__ __launch_bounds__(8 * kWave) void attn_step_kernel(AttnParams p) {
     const uint4 v = *reinterpret_cast<const uint4 *>(&sh.qhl[col < 2 * G ? col : 0][j * 32 + grp * 8]);
     qx[j] = col < 2 * G ? v : make_uint4(0u, 0u, 0u, 0u);
   }
+  uint4 third[kF32Parts ? HD / 32 : 1];
+  float down = 1.0f;
+  if constexpr (kF32Parts) {
+#pragma unroll
+    for (int j = 0; j < HD / 32; ++j) {
+      const uint4 v = *reinterpret_cast<const uint4 *>(&sh.qhl[2 * G + (col < G ? col : 0)][j * 32 + grp * 8]);
+      third[j] = col < G ? v : make_uint4(0u, 0u, 0u, 0u);
+    }
+    if constexpr (attn_scaled<DT, HD, G>()) down = sh.qdown[col < G ? col : col < 2 * G ? col - G : 0];
+  }
   link_mark(tr, 10);
 
   // ---- 6. tiles in request order
@@ -463,8 +498,8 @@ __global__ __launch_bounds__(8 * kWave) void attn_step_kernel(AttnParams p) {
         vv[j] = NV_AT_U4(vr[F][j]);                                                                                \
       }                                                                                                            \
       const uint32_t bb = first + t_idx * W;                                                                       \
-      attn_tile<DT, HD, G, false>(kk, vv, qx, nullptr, bb, n_keys, col, grp, owns_new && bb == new_block, new_row,     \
-                              sh.knew, sh.vnew, m, l, acc);                                                        \
+      attn_tile<DT, HD, G, false, kF32Parts>(kk, vv, qx, nullptr, bb, n_keys, col, grp, owns_new && bb == new_block,   \
+                                             new_row, sh.knew, sh.vnew, m, l, acc, down, third);                      \
       if (t_idx + 4u < nt) NV_AT_TILE_LOAD(F, scalar_load(p.table + first + (t_idx + 4u) * W));                          \
     }                                                                                                              \
   } while (0)

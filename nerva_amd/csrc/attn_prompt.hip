@@ -93,6 +93,8 @@ __global__ __launch_bounds__(kPW *kWave, 2) void attn_prompt_kernel(AttnParams p
   const int col = lane & 15, grp = lane >> 4;
   u32x4_t qhi[2][kPieces], qlo[2][kPieces];
   uint32_t n_keys[2];
+  constexpr bool kScaled = attn_scaled<DT, HD, G>();
+  float down[2] = {1.0f, 1.0f};   // undoes the scale of the column's query
   {
     constexpr int kHalf = kPieces / 2;   // pieces of a rotation's first ends
     const bool has_bias = p.q_bias != nullptr, has_gamma = p.q_norm != nullptr, has_rope = p.rope_freq != nullptr;
@@ -162,13 +164,26 @@ __global__ __launch_bounds__(kPW *kWave, 2) void attn_prompt_kernel(AttnParams p
             y[j + kHalf][e] = y1 * co + y0 * si;
           }
       }
+      float up = scale;
+      if constexpr (kScaled) {
+        float largest = 0.0f;
+#pragma unroll
+        for (int j = 0; j < kPieces; ++j)
+#pragma unroll
+          for (int e = 0; e < 8; ++e) largest = fmaxf(largest, fabsf(y[j][e]));
+        largest = fmaxf(largest, __shfl_xor(largest, 16, kWave));
+        largest = fmaxf(largest, __shfl_xor(largest, 32, kWave));
+        const int shift = attn_query_exponent(largest * scale);
+        up = ldexpf(scale, shift);
+        down[c] = ldexpf(1.0f, -shift);
+      }
 #pragma unroll
       for (int j = 0; j < kPieces; ++j)
 #pragma unroll
         for (int e = 0; e < 4; ++e) {
           uint16_t h0, l0, h1, l1;
-          split16<DT>(y[j][2 * e] * scale, h0, l0);
-          split16<DT>(y[j][2 * e + 1] * scale, h1, l1);
+          split16<DT>(y[j][2 * e] * up, h0, l0);
+          split16<DT>(y[j][2 * e + 1] * up, h1, l1);
           qhi[c][j][e] = h0 | (static_cast<uint32_t>(h1) << 16);
           qlo[c][j][e] = l0 | (static_cast<uint32_t>(l1) << 16);
         }
@@ -241,15 +256,17 @@ __global__ __launch_bounds__(kPW *kWave, 2) void attn_prompt_kernel(AttnParams p
       for (uint32_t t = 1; t < kStepBlocks; ++t) mb = fmaxf(fmaxf(mb, fmaxf(sc[c][t][0], sc[c][t][1])), fmaxf(sc[c][t][2], sc[c][t][3]));
       mb = fmaxf(mb, __shfl_xor(mb, 16, kWave));
       mb = fmaxf(mb, __shfl_xor(mb, 32, kWave));
+      if constexpr (kScaled) mb *= down[c];
       const float m_new = fmaxf(m[c], mb);
       const float m_ref = fmaxf(m_new, -3.0e38f);   // a column with nothing to see yet: exponentials against a finite stand-in
       const float alpha = attn_exp2(m[c] - m_ref);
+      const float m_low = kScaled ? m_ref - kAttnWeightShift : m_ref;
       float psum = 0.0f;
 #pragma unroll
       for (uint32_t t = 0; t < kStepBlocks; ++t) {
         float e[4];
 #pragma unroll
-        for (int r = 0; r < 4; ++r) e[r] = attn_exp2(sc[c][t][r] - m_ref);
+        for (int r = 0; r < 4; ++r) e[r] = attn_exp2(kScaled ? fmaf(sc[c][t][r], down[c], -m_low) : sc[c][t][r] - m_low);
         psum += (e[0] + e[1]) + (e[2] + e[3]);
 #pragma unroll
         for (int r = 0; r < 4; r += 2) {
@@ -416,7 +433,7 @@ __global__ __launch_bounds__(kPW *kWave, 2) void attn_prompt_kernel(AttnParams p
         score = fmaf(__shfl(q0, d, kWave), dec16<DT>(p.k_cache[tile + kv_k_elem(HD, key % kKvBlockTokens, d)]), score);
         score = fmaf(__shfl(q1, d, kWave), dec16<DT>(p.k_cache[tile + kv_k_elem(HD, key % kKvBlockTokens, d + HD / 2)]), score);
       }
-      const float weight = attn_exp2(score - most);
+      const float weight = attn_exp2(score - (kScaled ? most - kAttnWeightShift : most));
       for (uint32_t i = 0; i < min(end - k0, static_cast<uint32_t>(kWave)); ++i) {
         const uint64_t row = kv_tile_offset(p.block_count, p.kv_heads, HD, p.layer, p.table[(k0 + i) / kKvBlockTokens], kvh);
         const float w = __shfl(weight, i, kWave);

@@ -163,6 +163,26 @@ __device__ __forceinline__ void split16(float v, uint16_t &hi, uint16_t &lo) {
   hi = enc16_finite<DT>(v);
   lo = enc16_finite<DT>(v - dec16<DT>(hi));
 }
+// v = hi + mid + lo: 24 bits or more of it, as an f32 has them.
+template <uint32_t DT>
+__device__ __forceinline__ void split16(float v, uint16_t &hi, uint16_t &mid, uint16_t &lo) {
+  hi = enc16_finite<DT>(v);
+  const float rest = v - dec16<DT>(hi);
+  mid = enc16_finite<DT>(rest);
+  lo = enc16_finite<DT>(rest - dec16<DT>(mid));
+}
+// Heads of 64, and 3, 5, 6 or 7 query heads a kv head: the shapes whose queries and probabilities were f32 in the general
+// kernel before the matrix cores took them. (Heads of 128 with 1, 2, 4 or 8 query heads always had two parts in their own
+// units.)
+constexpr bool attn_f32_shape(int head_dim, int group) { return head_dim != 128 || (group & (group - 1)) != 0; }
+// In f16 the parts of small numbers fall below its smallest: there a query of those shapes is multiplied with a power of two
+// that brings its head's largest element to 2^14 .. 2^15 (the scores are multiplied back), and probabilities go up to
+// 2^kAttnWeightShift, in the sums l and in the accumulators alike. (Queries of 1e-4 against keys of 1e4: the output was 1e-3
+// off in the step kernel, 2.5e-7 with both.)
+template <uint32_t DT, int HD, int G>
+constexpr bool attn_scaled() { return DT == kF16 && attn_f32_shape(HD, G); }
+constexpr float kAttnWeightShift = 15.0f;
+__device__ __forceinline__ int attn_query_exponent(float largest) { return max(-126, min(126, 15 - __builtin_amdgcn_frexp_expf(largest))); }
 // Softmax arithmetic runs in base 2: the query is pre-scaled by log2(e) / sqrt(d), so scores, the
 // running maxima m and every exchanged partial maximum are log2-domain numbers and
 // exp(s - m) is one v_exp_f32. exp2(-inf) = 0.
@@ -208,7 +228,9 @@ __device__ __forceinline__ void attn_load_tile(const AttnParams &p, uint32_t phy
   }
 }
 
-// One 16-token tile against the G query heads of the kv head (see attn_fast_body).
+// One 16-token tile against the G query heads of the kv head (see attn_fast_body). F32_PARTS (see attn_step_kernel): queries
+// and probabilities in three parts, the third ones in operands of their own (columns 0 .. G-1). `down` (attn_scaled) undoes
+// the scale of the query of this lane's column.
 // n_keys may differ from lane to lane (by column: the prompt kernel's columns belong to tokens at
 // different positions). COLUMN_MASKS = a column may find a whole tile masked, even its first one: the
 // running maximum then stays at minus infinity, and the exponentials are taken against a finite stand-in
@@ -216,12 +238,12 @@ __device__ __forceinline__ void attn_load_tile(const AttnParams &p, uint32_t phy
 // LAZY_RESCALE = the accumulators are multiplied by alpha only in tiles where some lane's alpha is not 1 (a
 // running maximum that did not move gives exp2(0) = 1 exactly, so the result is the same bits): worth a branch
 // where a wave walks many tiles and the vector ALU is what it waits for (prompt blocks).
-template <uint32_t DT, int HD, int G, bool QX_LDS, bool COLUMN_MASKS = false, bool LAZY_RESCALE = false>
+template <uint32_t DT, int HD, int G, bool QX_LDS, bool F32_PARTS = false, bool COLUMN_MASKS = false, bool LAZY_RESCALE = false>
 __device__ __forceinline__ void attn_tile(uint4 (&kreg)[HD / 32], uint4 (&vreg)[HD / 32], const uint4 (&qx)[HD / 32],
                                           const uint4 *qx_lds, uint32_t b,
                                           uint32_t n_keys, int col, int grp, bool splice, uint32_t new_row,
                                           const uint16_t *knew, const uint16_t *vnew, float &m, float &l,
-                                          f32x4_t (&acc)[HD / 16]) {
+                                          f32x4_t (&acc)[HD / 16], float down, const uint4 *qx_third = nullptr) {
   if (splice) {
     // the row published by this workgroup may not be visible to its own loads yet: take it from LDS
     if (static_cast<uint32_t>(col) == new_row) {  // K operand: lane = (token col, dims grp*8..)
@@ -263,7 +285,9 @@ __device__ __forceinline__ void attn_tile(uint4 (&kreg)[HD / 32], uint4 (&vreg)[
   for (int j = 0; j < HD / 32; ++j) {
     if constexpr (QX_LDS) c = mfma_k32<DT>(kreg[j], qx_lds[j * kWave], c);  // qx_lds: this lane's first operand
     else c = mfma_k32<DT>(kreg[j], qx[j], c);
+    if constexpr (F32_PARTS) c = mfma_k32<DT>(kreg[j], qx_third[j], c);
   }
+  constexpr bool kScaled = attn_scaled<DT, HD, G>();
   float sc[4];
 #pragma unroll
   for (int r = 0; r < 4; ++r) {
@@ -272,7 +296,8 @@ __device__ __forceinline__ void attn_tile(uint4 (&kreg)[HD / 32], uint4 (&vreg)[
     const float from_up = row_shl<G>(c[r]), from_down = row_shr<G>(c[r]);
     const float other = col < G ? from_up : from_down;
     const bool valid = b * kKvBlockTokens + grp * 4 + r < n_keys;
-    sc[r] = valid ? c[r] + other : -INFINITY;
+    const float score = kScaled ? (c[r] + other) * down : c[r] + other;
+    sc[r] = valid ? score : -INFINITY;
   }
   float mb = fmaxf(fmaxf(sc[0], sc[1]), fmaxf(sc[2], sc[3]));
   mb = fmaxf(mb, __shfl_xor(mb, 16, kWave));
@@ -280,15 +305,23 @@ __device__ __forceinline__ void attn_tile(uint4 (&kreg)[HD / 32], uint4 (&vreg)[
   const float m_new = fmaxf(m, mb);   // finite: every processed tile has a valid token (without column masks)
   const float m_ref = COLUMN_MASKS ? fmaxf(m_new, -3.0e38f) : m_new;
   const float alpha = attn_exp2(m - m_ref);
-  uint32_t px[2];
+  const float m_low = kScaled ? m_ref - kAttnWeightShift : m_ref;
+  uint32_t px[2], third[2];
   float psum = 0.0f;
 #pragma unroll
   for (int r = 0; r < 4; r += 2) {
-    const float p0 = attn_exp2(sc[r] - m_ref), p1 = attn_exp2(sc[r + 1] - m_ref);
+    const float p0 = attn_exp2(sc[r] - m_low), p1 = attn_exp2(sc[r + 1] - m_low);
     psum += p0 + p1;
     uint16_t h0, l0, h1, l1;
-    split16<DT>(p0, h0, l0);
-    split16<DT>(p1, h1, l1);
+    if constexpr (F32_PARTS) {
+      uint16_t t0, t1;
+      split16<DT>(p0, h0, l0, t0);
+      split16<DT>(p1, h1, l1, t1);
+      third[r / 2] = col < G ? (t0 | (static_cast<uint32_t>(t1) << 16)) : 0u;
+    } else {
+      split16<DT>(p0, h0, l0);
+      split16<DT>(p1, h1, l1);
+    }
     px[r / 2] = col < G ? (h0 | (static_cast<uint32_t>(h1) << 16)) : (l0 | (static_cast<uint32_t>(l1) << 16));
   }
   l = l * alpha + psum;
@@ -306,6 +339,7 @@ __device__ __forceinline__ void attn_tile(uint4 (&kreg)[HD / 32], uint4 (&vreg)[
     const uint4 &vr = vreg[s2 / 2];
     const uint2 va = (s2 & 1) ? make_uint2(vr.z, vr.w) : make_uint2(vr.x, vr.y);
     acc[s2] = mfma_k16<DT>(va, pb, acc[s2]);
+    if constexpr (F32_PARTS) acc[s2] = mfma_k16<DT>(va, make_uint2(third[0], third[1]), acc[s2]);
   }
 }
 
@@ -529,6 +563,19 @@ __device__ __forceinline__ void attn_fast_body(const AttnParams &p, const uint32
 
   // B operand of the first product: column `col` of Qx for dims j*32 + grp*8 .. +7
   uint4 qx[HD / 32];
+  float up = scale, down = 1.0f;
+  if constexpr (attn_scaled<DT, HD, G>()) {
+    float largest = 0.0f;
+#pragma unroll
+    for (int j = 0; j < HD / 32; ++j)
+#pragma unroll
+      for (int e = 0; e < 8; ++e) largest = fmaxf(largest, fabsf(q_s[col < G ? col : col < 2 * G ? col - G : 0][j * 32 + grp * 8 + e]));
+    largest = fmaxf(largest, __shfl_xor(largest, 16, kWave));
+    largest = fmaxf(largest, __shfl_xor(largest, 32, kWave));
+    const int shift = attn_query_exponent(largest * scale);
+    up = ldexpf(scale, shift);
+    down = ldexpf(1.0f, -shift);
+  }
 #pragma unroll
   for (int j = 0; j < HD / 32; ++j) {
     uint32_t w[4] = {0u, 0u, 0u, 0u};
@@ -537,8 +584,8 @@ __device__ __forceinline__ void attn_fast_body(const AttnParams &p, const uint32
 #pragma unroll
       for (int e = 0; e < 4; ++e) {
         uint16_t h0, l0, h1, l1;
-        split16<DT>(src[2 * e] * scale, h0, l0);
-        split16<DT>(src[2 * e + 1] * scale, h1, l1);
+        split16<DT>(src[2 * e] * up, h0, l0);
+        split16<DT>(src[2 * e + 1] * up, h1, l1);
         w[e] = col < G ? (h0 | (static_cast<uint32_t>(h1) << 16)) : (l0 | (static_cast<uint32_t>(l1) << 16));
       }
     }
@@ -565,7 +612,7 @@ __device__ __forceinline__ void attn_fast_body(const AttnParams &p, const uint32
       const uint32_t bb = b + f * W;
       if (bb < b1) {
         attn_tile<DT, HD, G, kLean>(kreg[f], vreg[f], qx, qx_lds, bb, n_keys, col, grp, owns_new && bb == new_block, new_row,
-                                 knew, vnew, m, l, acc);
+                                 knew, vnew, m, l, acc, down);
         if (bb + kInFlight * W < b1) attn_load_tile<HD>(p, p.table[bb + kInFlight * W], kvh, lane, kreg[f], vreg[f]);
       }
     }

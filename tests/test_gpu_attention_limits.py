@@ -8,7 +8,7 @@ import oracle as O
 from nerva_amd.runtime import attention_workspace
 from test_gpu_any_width import walked
 from test_gpu_ops import _attention_case, _attention_oracle, dev
-from test_gpu_session import BF16, E2E_REL_L2, F16, REL_L2, random_model, rel_l2
+from test_gpu_session import BF16, E2E_REL_L2, F16, REL_L2, oracle_follow, random_model, rel_l2, started
 
 pytestmark = pytest.mark.gpu
 
@@ -107,3 +107,65 @@ def test_an_earlier_sequences_rows_do_not_reach_the_next(geom):
         assert results[0][0][:1] == results[1][0][:1] or top[-1] - top[-2] <= E2E_REL_L2 * np.max(np.abs(top)), length
     for session in (used, fresh):
         session.destroy()
+
+
+@pytest.mark.parametrize("scale", [1.0, 1e-4, 3e3])
+@pytest.mark.parametrize("heads,kv_heads,hd", [(28, 4, 128), (5, 1, 128), (6, 2, 128), (48, 8, 128), (14, 2, 64), (8, 8, 64), (32, 4, 64)])
+@pytest.mark.parametrize("dtype", [BF16, F16])
+def test_step_attention_keeps_the_bits_of_f32(dtype, heads, kv_heads, hd, scale):
+    """Heads of 64, and of 128 with 3, 5, 6 or 7 query heads a key head, against 64 bits: queries and probabilities that had
+    16 bits (bf16) or fell below half precision's smallest numbers were 3e-6 off, whatever the number of keys. 24 bits of each
+    and sums in f32 leave 2^-23 from the query and the probability and less than that again from sums in pieces of 16 and 64
+    (bound: four times 2^-23). Queries of 1e-4 and keys of as many times more, and the other way round: the size of either alone does not matter."""
+    for n in (75, 600):
+        rng = np.random.default_rng(heads * n)
+        table = rng.permutation(n // 16 + 2).astype(np.uint32)
+        k = O.encode16(dtype, rng.normal(0, 1 / scale, (n, kv_heads * hd)))
+        v = O.encode16(dtype, rng.normal(0, 1, (n, kv_heads * hd)))
+        q = rng.normal(0, scale, (heads + 2 * kv_heads) * hd).astype(np.float32)
+        cache = N.PagedKvCache(1, table.size, kv_heads, hd, table)
+        cache.fill(0, k, v)
+        out16, out32 = N.DeviceBuffer(heads * hd * 2), N.DeviceBuffer(heads * hd * 4)
+        N.paged_attention(dtype, heads, kv_heads, hd, cache, 0, n - 1, dev(q), attention_workspace(heads, hd), out16, out_f32=out32,
+                          append=False)
+        keys, values = (O.decode16(dtype, a).astype(np.float64).reshape(n, kv_heads, 1, hd) for a in (k, v))
+        score = (keys * q[:heads * hd].astype(np.float64).reshape(1, kv_heads, -1, hd)).sum(3) / np.sqrt(hd)
+        weight = np.exp(score - score.max(0))
+        want = (weight[..., None] * values).sum(0) / weight.sum(0)[..., None]
+        assert rel_l2(out32.numpy(np.float32), want.reshape(-1)) <= 4 * 2.0 ** -23, n
+
+
+@pytest.mark.parametrize("geom", [(896, 14, 2, 64, 1728, 300, 2), (1536, 12, 2, 128, 2944, 301, 2)], ids=str)
+def test_queries_below_half_precisions_smallest(geom):
+    """Query weights of 1e-4 and key weights of 1e4: scores as large as any, of query elements that half precision rounds to
+    some 1e-3 in their own units. Prompt blocks and batch steps against the oracle, in a model whose second layer sees little
+    but the first one's attention. Rounding to 16 bits is 2^-12 of an element, in three stages up to there (embedding and
+    normalised row, attention, row of the second layer): a bound of 8e-4 (scores off by 3e-3 had left up to 9.6e-4)."""
+    hidden, heads, kv, hd, inter, vocab, layers = geom
+    weights, _ = random_model(F16, hidden, heads, kv, hd, inter, vocab, layers, hidden, 1e4, True, False)
+    weights.embeddings[:] = O.encode16(F16, 0.01 * O.decode16(F16, weights.embeddings))
+    for layer in weights.layers:
+        layer["q_norm"][:] = O.encode16(F16, np.full(hd, 1e-4))
+        layer["k_norm"][:] = O.encode16(F16, np.full(hd, 1e4))
+    weights.layers[0]["w_down"][:] = 0
+    omodel = O.Model(F16, hidden, heads, kv, hd, inter, vocab, 1e-6, 1e4, weights.embeddings, weights.layers, weights.final_norm,
+                     weights.lm_head)
+    parent = N.DecodeSession.create(weights, 256, plan=N.WeightPlan.from_weights(weights))
+    sessions = [parent, parent.fork_shared_weights(), parent.fork_shared_weights()]
+    assert parent.shares_weight_stream()
+    rng = np.random.default_rng(3)
+    prompts = [rng.integers(0, vocab, n).astype(np.uint32) for n in (5, 70, 200)]
+    streams = [[started(s, p)] for s, p in zip(sessions, prompts)]
+    for _ in range(3):
+        rc, _, tokens = N.DecodeSession.batch_advance_one(sessions, 3, 2)
+        assert rc == 0
+        for stream, token in zip(streams, tokens):
+            stream.append(int(token))
+    for session, prompt, stream in zip(sessions, prompts, streams):
+        ctx, _ = oracle_follow(omodel, 256, prompt, stream[:-1])
+        for token in (*range(2, prompt.size, 7), *range(prompt.size, prompt.size + 3)):
+            for got, want in zip(session.kv_row(1, token), ctx.read_kv16(1, token)):
+                assert rel_l2(O.decode16(F16, got), O.decode16(F16, want)) <= 8e-4, (prompt.size, token)
+        ctx.close()
+    for s in sessions[::-1]:
+        s.destroy()
