@@ -114,6 +114,18 @@ __host__ __device__ __forceinline__ uint32_t attn_launch_tag(uint32_t seq, uint3
 // holds its CU while it polls), one 8-wave workgroup per CU: the largest split factor a launch may use there.
 uint32_t attn_resident_splits(uint32_t kv_heads);
 
+// Heads of 64, and 3, 5, 6 or 7 query heads a kv head: the shapes whose queries and probabilities were f32 in the general
+// kernel before the matrix cores took them, and whose launches waited for nobody. (Heads of 128 with 1, 2, 4 or 8 query heads
+// always had two 16-bit parts of them and a merge by every split.)
+constexpr bool attn_f32_shape(uint32_t head_dim, uint32_t group) { return head_dim != 128 || (group & (group - 1)) != 0; }
+// At those shapes no more than this many workgroups of a launch merge, and wait: sessions on streams of their own run
+// their launches side by side, a workgroup has a CU to itself, and 28 heads on 4 (or 40 on 8) were 112 (160) that poll on
+// 256 CUs - two launches could hold each other's CUs until the waits gave up. Consecutive workgroups go round the eight
+// XCDs, so that is seven of an XCD's 32 CUs: four launches at once, one a hardware queue, leave it four that nobody waits on. A merging workgroup then
+// has up to four parts at a time (28 heads on 4 at 900 / 8000 keys: 7.9 / 8.8 -> 8.8 / 10.0 us a launch, one part after the other
+// 9.2 / 10.0; 40 on 8 at 4000: 8.7 -> 10.1, 11.1; 32 heads of 64 on 8 at 8000: 8.4 -> 8.6, 9.2).
+constexpr uint32_t kAttnWaitingWorkgroups = 56;
+
 // ---- per-step split plan of the decode attention ---------------------------------------------
 // words [0..7]: position, blocks, blocks per split, active splits, step number (the caller's), 3 spare;
 // then one 8-word entry per (split, wave): tiles of the wave, its first block, the physical blocks
@@ -177,6 +189,11 @@ inline uint32_t attn_default_splits(uint32_t kv_heads, uint32_t block_count) {
   if (splits > kAttnMaxSplits) splits = kAttnMaxSplits;
   if (splits > block_count) splits = block_count;
   return splits == 0 ? 1 : splits;
+}
+// The same for the step kernel of a model: one split where a workgroup a kv head would be more than may wait.
+inline uint32_t attn_step_splits(uint32_t heads, uint32_t kv_heads, uint32_t head_dim) {
+  const bool few_wait = attn_f32_shape(head_dim, heads / kv_heads);
+  return few_wait && kv_heads > kAttnWaitingWorkgroups ? 1u : attn_resident_splits(kv_heads);
 }
 uint64_t attn_workspace_bytes(uint32_t heads, uint32_t head_dim);
 // Bytes of AttnParams::part_tagged (head_dim up to 128), zero-initialised once.

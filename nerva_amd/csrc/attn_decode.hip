@@ -137,7 +137,7 @@ __device__ __forceinline__ void sload4(const uint32_t *p0, const uint32_t *p1, c
 // is read - and its tags cleared - by exactly one merging workgroup.
 constexpr uint32_t kStepPartDims = 32, kStepPartWords = kStepPartDims + 2;
 constexpr uint32_t step_record(uint32_t head_dim) { return head_dim / kStepPartDims * kStepPartWords; }
-// One part (32 dims of one head) merged by one workgroup of 512 threads. Thread (dl = t % 32,
+// Parts (32 dims of one head each) merged by one workgroup of 512 threads. Thread (dl = t % 32,
 // q = t / 32) takes the splits q, q + 16, q + 32, q + 48: it polls their accumulator word and their m
 // and l words until every tag is up and folds them in split order; the two groups of a wave meet by a lane
 // exchange and the eight waves in LDS, in wave order - a fixed order, whatever the arrival order was. A CU sustains only a few hundred
@@ -148,85 +148,95 @@ constexpr uint32_t step_record(uint32_t head_dim) { return head_dim / kStepPartD
 // fault word is set - the session hands it out with the token, the operator entry point through its status call -
 // and the outputs it feeds become NaN. A word counts only with this launch's tag, so a partial that lands after
 // its merge gave up is never taken for a later launch's.
-template <uint32_t DT, int HD, int G>
-__device__ __forceinline__ void merge_part_tagged(const AttnParams &p, uint32_t kvh, uint32_t g, uint32_t part, uint32_t S,
-                                                  uint32_t active, float *lds_o, float *lds_m, float *lds_l, bool first_part,
-                                                  uint32_t tag) {
+// N parts at a time, j, j + step, ...: their words are asked for together.
+template <uint32_t DT, int HD, int G, int N>
+__device__ __forceinline__ void merge_parts_tagged(const AttnParams &p, uint32_t kvh, uint32_t j, uint32_t step, uint32_t S, uint32_t active,
+                                                   float *lds_o, float *lds_m, float *lds_l, bool first_part, uint32_t tag) {
   const uint32_t spin_limit = p.merge_spin_limit != 0 ? p.merge_spin_limit : kAttnMergeSpinLimit;
   constexpr uint32_t kGroups = 16, kPer = kAttnMaxSplits / kGroups;  // 4 splits per thread at most
-  const uint32_t h = kvh * G + g;
-  uint64_t *rec = p.part_tagged + static_cast<uint64_t>(h) * S * step_record(HD) + part * kStepPartWords;
-  const uint32_t dl = threadIdx.x % kStepPartDims, q = threadIdx.x / kStepPartDims;
-  uint64_t av[kPer], mv[kPer], lv[kPer];
+  constexpr uint32_t kWaves = kGroups / 2;
+  const uint32_t dl = threadIdx.x % kStepPartDims, q = threadIdx.x / kStepPartDims, w = q / 2;
+  const auto head = [&](uint32_t n) { return kvh * G + (j + n * step) % G; };
+  const auto part = [&](uint32_t n) { return (j + n * step) / G; };
+  const uint64_t *rec[N];
+#pragma unroll
+  for (uint32_t n = 0; n < N; ++n) rec[n] = p.part_tagged + static_cast<uint64_t>(head(n)) * S * step_record(HD) + part(n) * kStepPartWords;
+  uint64_t av[N][kPer], mv[N][kPer], lv[N][kPer];
   uint32_t spins = 0;
   for (;;) {
     bool ok = true;
 #pragma unroll
-    for (uint32_t i = 0; i < kPer; ++i) {
-      // unconditional loads (index clamped): a load under a branch would serialise the round
-      const uint64_t *r = rec + static_cast<uint64_t>(min(q + i * kGroups, active - 1)) * step_record(HD);
-      av[i] = load_tagged(r + dl);
-      mv[i] = load_tagged(r + kStepPartDims);
-      lv[i] = load_tagged(r + kStepPartDims + 1);
-    }
+    for (uint32_t n = 0; n < N; ++n)
 #pragma unroll
-    for (uint32_t i = 0; i < kPer; ++i)  // (a clamped repeat of the last split belongs to another thread: not awaited)
-      if (q + i * kGroups < active) ok = ok && tag_is(av[i], tag) && tag_is(mv[i], tag) && tag_is(lv[i], tag);
+      for (uint32_t i = 0; i < kPer; ++i) {
+        // unconditional loads (index clamped): a load under a branch would serialise the round
+        const uint64_t *r = rec[n] + static_cast<uint64_t>(min(q + i * kGroups, active - 1)) * step_record(HD);
+        av[n][i] = load_tagged(r + dl);
+        mv[n][i] = load_tagged(r + kStepPartDims);
+        lv[n][i] = load_tagged(r + kStepPartDims + 1);
+      }
+#pragma unroll
+    for (uint32_t n = 0; n < N; ++n)
+#pragma unroll
+      for (uint32_t i = 0; i < kPer; ++i)  // (a clamped repeat of the last split belongs to another thread: not awaited)
+        if (q + i * kGroups < active) ok = ok && tag_is(av[n][i], tag) && tag_is(mv[n][i], tag) && tag_is(lv[n][i], tag);
     if (__all(ok) || ++spins > spin_limit) break;
   }
   const bool gave_up = spins > spin_limit;  // per wave; poisons the outputs this wave contributes to
   if (gave_up && p.fault != nullptr && (threadIdx.x & (kWave - 1)) == 0)
     __hip_atomic_store(p.fault, tag, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-  float M = -INFINITY, L = 0.0f, o = 0.0f;
+  if (!first_part) __syncthreads();   // the previous parts' last reads
 #pragma unroll
-  for (uint32_t i = 0; i < kPer; ++i)
-    if (q + i * kGroups < active) M = fmaxf(M, tag_value(mv[i]));
+  for (uint32_t n = 0; n < N; ++n) {
+    float M = -INFINITY, L = 0.0f, o = 0.0f;
 #pragma unroll
-  for (uint32_t i = 0; i < kPer; ++i) {
-    if (q + i * kGroups < active) {
-      const float f = attn_exp2(tag_value(mv[i]) - M);  // every active split saw a key: its m is finite
-      L = fmaf(tag_value(lv[i]), f, L);
-      o = fmaf(tag_value(av[i]), f, o);
+    for (uint32_t i = 0; i < kPer; ++i)
+      if (q + i * kGroups < active) M = fmaxf(M, tag_value(mv[n][i]));
+#pragma unroll
+    for (uint32_t i = 0; i < kPer; ++i) {
+      if (q + i * kGroups < active) {
+        const float f = attn_exp2(tag_value(mv[n][i]) - M);  // every active split saw a key: its m is finite
+        L = fmaf(tag_value(lv[n][i]), f, L);
+        o = fmaf(tag_value(av[n][i]), f, o);
+      }
     }
-  }
-  // the two groups of a wave (its lanes 0-31 and 32-63) meet by a lane exchange, the even group's sum first;
-  // the eight waves meet in LDS (arrays of their own: no barrier before they are written, except between parts)
-  {
-    const float Mo = __shfl_xor(M, static_cast<int>(kStepPartDims), kWave), Lo = __shfl_xor(L, static_cast<int>(kStepPartDims), kWave),
-                oo = __shfl_xor(o, static_cast<int>(kStepPartDims), kWave);
-    const bool even = (q & 1u) == 0;
-    const float Ma = even ? M : Mo, La = even ? L : Lo, oa = even ? o : oo;
-    const float Mb = even ? Mo : M, Lb = even ? Lo : L, ob = even ? oo : o;
-    const float Mw = fmaxf(Ma, Mb);
-    const float fa = Ma > -INFINITY ? attn_exp2(Ma - Mw) : 0.0f, fb = Mb > -INFINITY ? attn_exp2(Mb - Mw) : 0.0f;   // a group without a split
-    M = Mw;
-    L = fmaf(Lb, fb, La * fa);
-    o = fmaf(ob, fb, oa * fa);
-  }
-  constexpr uint32_t kWaves = kGroups / 2;
-  const uint32_t w = q / 2;
-  if (!first_part) __syncthreads();   // the previous part's last reads
-  if ((q & 1u) == 0) {
-    lds_o[w * kStepPartDims + dl] = gave_up ? NAN : o;
-    if (dl == 0) {
-      lds_m[w] = M;
-      lds_l[w] = L;
+    // the two groups of a wave (its lanes 0-31 and 32-63) meet by a lane exchange, the even group's sum first;
+    // the eight waves meet in LDS (arrays of their own: no barrier before they are written, except between parts)
+    {
+      const float Mo = __shfl_xor(M, static_cast<int>(kStepPartDims), kWave), Lo = __shfl_xor(L, static_cast<int>(kStepPartDims), kWave),
+                  oo = __shfl_xor(o, static_cast<int>(kStepPartDims), kWave);
+      const bool even = (q & 1u) == 0;
+      const float Ma = even ? M : Mo, La = even ? L : Lo, oa = even ? o : oo;
+      const float Mb = even ? Mo : M, Lb = even ? Lo : L, ob = even ? oo : o;
+      const float Mw = fmaxf(Ma, Mb);
+      const float fa = Ma > -INFINITY ? attn_exp2(Ma - Mw) : 0.0f, fb = Mb > -INFINITY ? attn_exp2(Mb - Mw) : 0.0f;   // a group without a split
+      M = Mw;
+      L = fmaf(Lb, fb, La * fa);
+      o = fmaf(ob, fb, oa * fa);
+    }
+    if ((q & 1u) == 0) {
+      lds_o[(n * kWaves + w) * kStepPartDims + dl] = gave_up ? NAN : o;
+      if (dl == 0) {
+        lds_m[n * kWaves + w] = M;
+        lds_l[n * kWaves + w] = L;
+      }
     }
   }
   __syncthreads();
-  if (q == 0) {
+  if (q < N) {   // (a group of 32 threads a part)
+    const uint32_t n = q;
     float Mt = -INFINITY;
 #pragma unroll
-    for (uint32_t k = 0; k < kWaves; ++k) Mt = fmaxf(Mt, lds_m[k]);
+    for (uint32_t k = 0; k < kWaves; ++k) Mt = fmaxf(Mt, lds_m[n * kWaves + k]);
     float Lt = 0.0f, ot = 0.0f;
 #pragma unroll
     for (uint32_t k = 0; k < kWaves; ++k) {
-      const float f = lds_m[k] > -INFINITY ? attn_exp2(lds_m[k] - Mt) : 0.0f;  // a wave without a split
-      Lt = fmaf(lds_l[k], f, Lt);
-      ot = fmaf(lds_o[k * kStepPartDims + dl], f, ot);
+      const float mk = lds_m[n * kWaves + k], f = mk > -INFINITY ? attn_exp2(mk - Mt) : 0.0f;  // a wave without a split
+      Lt = fmaf(lds_l[n * kWaves + k], f, Lt);
+      ot = fmaf(lds_o[(n * kWaves + k) * kStepPartDims + dl], f, ot);
     }
     if (Lt > 0.0f && isfinite(Lt)) ot /= Lt;
-    const uint32_t e = h * HD + part * kStepPartDims + dl;
+    const uint32_t e = head(n) * HD + part(n) * kStepPartDims + dl;
     if (p.out_f32 != nullptr) p.out_f32[e] = ot;
     p.out16[attn_out_elem(p, e)] = enc16<DT>(ot);
   }
@@ -258,7 +268,8 @@ struct StepShared {
   alignas(16) uint16_t vnew[HD];
   float wm[8][G], wl[8][G];
   alignas(16) float wacc[8][G][HD];
-  float merge_o[8][32], merge_m[8], merge_l[8];   // the splits' merge: one entry per wave
+  static constexpr int kMerged = attn_f32_shape(HD, G) ? 4 : 1;   // parts merged together
+  float merge_o[kMerged][8][32], merge_m[kMerged][8], merge_l[kMerged][8];   // the splits' merge: one entry per wave
   uint32_t is_last;
 };
 
@@ -567,12 +578,22 @@ __global__ __launch_bounds__(8 * kWave) void attn_step_kernel(AttnParams p) {
   if (active == 1) return;
   link_mark(tr, 12);
   // ---- 8. the splits' merge: part j = (head g, 32 dims) of this kv head is merged by split j (mod the
-  // active splits), which polls the other splits' words until every tag is up - two memory round
+  // active splits, or fewer: kAttnWaitingWorkgroups), which polls the other splits' words until every tag is up - two memory round
   // trips after the slowest split's tiles (store, then the poll that finds it), where a ticket taken
   // after the stores have been performed and a merge by the last arriver needed four.
-  for (uint32_t j = split; j < G * (HD / kStepPartDims); j += active) {
+  const uint32_t mergers = kF32Parts ? min(active, kAttnWaitingWorkgroups / gridDim.x) : active;
+  if (split >= mergers) return;
+  constexpr uint32_t kParts = G * (HD / kStepPartDims);
+  constexpr int kMerged = StepShared<HD, G>::kMerged;
+  for (uint32_t j = split; j < kParts; j += kMerged * mergers) {
     link_mark(trm, 16);
-    merge_part_tagged<DT, HD, G>(p, kvh, j % G, j / G, S, active, sh.merge_o[0], sh.merge_m, sh.merge_l, j == split, tag);
+#define NV_AT_MERGE(N) merge_parts_tagged<DT, HD, G, N>(p, kvh, j, mergers, S, active, sh.merge_o[0][0], sh.merge_m[0], sh.merge_l[0], j == split, tag)
+    const uint32_t left = (kParts - j + mergers - 1) / mergers;
+    if (kMerged == 1 || left == 1) NV_AT_MERGE(1);
+    else if (left == 2) NV_AT_MERGE(kMerged == 1 ? 1 : 2);
+    else if (left == 3) NV_AT_MERGE(kMerged == 1 ? 1 : 3);
+    else NV_AT_MERGE(kMerged);
+#undef NV_AT_MERGE
     link_mark(trm, 17);
   }
 }
@@ -759,8 +780,8 @@ hipError_t launch_dt(const AttnParams &p, hipStream_t stream) {
   bool fast = attn_matrix_cores(p.heads, p.kv_heads, p.head_dim) && p.part_acc != nullptr && p.splits >= 1;
   // every active split of a kv head has to be resident while the merges poll: a larger split factor is refused at the
   // shapes the split factor is declared for, and left to the general kernel, which has no splits, at the others
-  if (fast && !block && p.splits > 1 && p.splits > attn_resident_splits(p.kv_heads)) {
-    if (p.head_dim == 128 && (group & (group - 1)) == 0) return hipErrorInvalidValue;
+  if (fast && !block && p.splits > 1 && p.splits > attn_step_splits(p.heads, p.kv_heads, p.head_dim)) {
+    if (!attn_f32_shape(p.head_dim, group)) return hipErrorInvalidValue;
     fast = false;
   }
   if (fast) {

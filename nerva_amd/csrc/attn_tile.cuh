@@ -171,11 +171,7 @@ __device__ __forceinline__ void split16(float v, uint16_t &hi, uint16_t &mid, ui
   mid = enc16_finite<DT>(rest);
   lo = enc16_finite<DT>(rest - dec16<DT>(mid));
 }
-// Heads of 64, and 3, 5, 6 or 7 query heads a kv head: the shapes whose queries and probabilities were f32 in the general
-// kernel before the matrix cores took them. (Heads of 128 with 1, 2, 4 or 8 query heads always had two parts in their own
-// units.)
-constexpr bool attn_f32_shape(int head_dim, int group) { return head_dim != 128 || (group & (group - 1)) != 0; }
-// In f16 the parts of small numbers fall below its smallest: there a query of those shapes is multiplied with a power of two
+// In f16 the parts of small numbers fall below its smallest: there a query of the shapes of attn_f32_shape is multiplied with a power of two
 // that brings its head's largest element to 2^14 .. 2^15 (the scores are multiplied back), and probabilities go up to
 // 2^kAttnWeightShift, in the sums l and in the accumulators alike. (Queries of 1e-4 against keys of 1e4: the output was 1e-3
 // off in the step kernel, 2.5e-7 with both.)

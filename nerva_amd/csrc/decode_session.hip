@@ -953,11 +953,12 @@ hipError_t setup_state(Session *s, int32_t *failure_stage, bool with_weights) {
                  L = s->layers, HD = s->head_dim;
   const uint32_t block_count = (s->max_ctx + kKvBlockTokens - 1) / kKvBlockTokens;
   s->block_count = block_count;
-  s->attn_splits = attn_default_splits(s->kv_heads, block_count);
+  const uint32_t most_splits = attn_step_splits(s->heads, s->kv_heads, s->head_dim);
+  s->attn_splits = std::min(attn_default_splits(s->kv_heads, block_count), most_splits);
   s->attn_single_blocks = kAttnSingleSplitBlocks;
   if (const int want = tuning(kTuneAttnSplits); want >= 1 && want <= static_cast<int>(kAttnMaxSplits)) {
     // (never more than stay resident together: the merges of the step kernel poll)
-    s->attn_splits = std::min({static_cast<uint32_t>(want), block_count, attn_resident_splits(s->kv_heads)});
+    s->attn_splits = std::min({static_cast<uint32_t>(want), block_count, most_splits});
     s->attn_single_blocks = 0;  // a forced factor holds at every context length
   }
 

@@ -524,6 +524,7 @@ int nerva_hip_paged_gqa_decode(const NervaHipPagedAttentionRequest *r, void *str
   p.layer = r->layer;
   p.block_count = r->block_count;
   p.splits = attn_default_splits(r->kv_heads, r->block_count);
+  if (r->kv_heads != 0) p.splits = std::min(p.splits, attn_step_splits(r->heads, r->kv_heads, r->head_dim));
   p.single_split_blocks = kAttnSingleSplitBlocks;
   if (r->splits != 0) {
     if (r->splits > kAttnMaxSplits || r->splits > r->block_count) return finish(hipErrorInvalidValue, hip_error);

@@ -1,5 +1,7 @@
 """What a token does not see has no part in its attention: keys behind its position - rows of its last block that nobody has
 written, rows of an earlier sequence, later tokens of its prompt - may hold anything, numbers that are not finite too."""
+import threading
+
 import numpy as np
 import pytest
 
@@ -169,3 +171,51 @@ def test_queries_below_half_precisions_smallest(geom):
         ctx.close()
     for s in sessions[::-1]:
         s.destroy()
+
+
+@pytest.mark.parametrize("geom", [(1280, 40, 8, 128, 1280, 301, 2), (896, 28, 4, 128, 896, 301, 2), (1024, 48, 8, 64, 1024, 301, 2)], ids=str)
+def test_sessions_on_streams_of_their_own_do_not_hold_each_other_up(geom):
+    """Four sessions decode at once, a thread and a stream each, at contexts whose splits merge inside the launch: every step
+    ends without a merge that gave up, and the tokens are those of the sessions one after the other."""
+    hidden, heads, kv, hd, inter, vocab, layers = geom
+    weights, _ = random_model(BF16, hidden, heads, kv, hd, inter, vocab, layers, hidden, 1e4, False, False)
+    sessions = [N.DecodeSession.create(weights, 1400) for _ in range(4)]
+    prompts = [np.random.default_rng(i).integers(0, vocab, 1000 + 50 * i).astype(np.uint32) for i in range(4)]
+
+    def advance(session, results, at):
+        results[at] = [session.advance(25) for _ in range(6)]
+
+    results = {}
+    for how in ("alone", "together"):
+        results[how] = [None] * 4
+        for session, prompt in zip(sessions, prompts):
+            assert session.start(prompt)[0] == 0
+        threads = [threading.Thread(target=advance, args=(s, results[how], i)) for i, s in enumerate(sessions)]
+        for thread in threads:
+            thread.start()
+            if how == "alone":
+                thread.join()
+        for thread in threads:
+            thread.join()
+    for alone, together in zip(results["alone"], results["together"]):
+        for (rc, res, tokens), (rc2, res2, tokens2) in zip(alone, together):
+            assert rc == rc2 == 0 and res2.hip_error == 0
+            assert tokens.tolist() == tokens2.tolist()
+    for session in sessions:
+        session.destroy()
+
+
+@pytest.mark.parametrize("heads,kv_heads,hd", [(60, 60, 64), (65, 65, 64), (171, 57, 128), (56, 56, 64), (40, 8, 128), (5, 1, 128), (96, 16, 64)])
+def test_merges_by_few_workgroups(heads, kv_heads, hd):
+    """Numbers of kv heads around the one from which no split may wait, and where a workgroup merges several parts."""
+    c = _attention_case(BF16, heads, kv_heads, hd, 1500, 1e4, False, heads)
+    ref, _, _ = _attention_oracle(c)
+    cache = N.PagedKvCache(c["layers"], c["n_blocks"], kv_heads, hd, c["table"])
+    cache.fill(c["layer"], c["k_rows"], c["v_rows"])
+    out16, out32, ws = N.DeviceBuffer(heads * hd * 2), N.DeviceBuffer(heads * hd * 4), attention_workspace(heads, hd)
+    qkv = dev(c["qkv"])
+    for splits in (0, 0, 2, 4, 64):
+        N.paged_attention(BF16, heads, kv_heads, hd, cache, c["layer"], 1500, qkv, ws, out16, out_f32=out32, append=True, rope_theta=1e4,
+                          splits=splits)
+        assert rel_l2(out32.numpy(np.float32), ref) <= REL_L2, splits
+    assert N.paged_attention_status(ws, heads, hd) == (0, 0)
