@@ -218,6 +218,7 @@ void nv::destroy_session(Session *s) {
   if (s->ev1) (void)hipEventDestroy(s->ev1);
   if (s->arena && !s->arena_in_weights) (void)hipFree(s->arena);
   if (s->weights != nullptr && s->weights->refs.fetch_sub(1) == 1) {
+    if (s->weights->pass_done) (void)hipEventDestroy(s->weights->pass_done);
     if (s->weights->origin) (void)hipFree(s->weights->origin);
     delete s->weights;
   }
@@ -894,7 +895,9 @@ namespace {
 hipError_t prompt_tokens(Session *s, uint32_t begin, uint32_t end, const uint32_t *wanted, uint32_t wanted_count, float *logits,
                          NervaHipHfDecodeSequenceResult *out) {
   if (s->stack != nullptr) return stack_prompt(s, begin, end, nullptr, 0, nullptr, nullptr, out);
-  hipError_t err = hipSuccess;
+  const PassTurn rows(s, s->block_prefill ? end - begin : 0);
+  hipError_t err = rows.error;
+  if (err != hipSuccess) return err;
   const uint32_t n = end - begin, last = n - 1;   // (place of the last token)
   // (with the hook for the error path of the decode attention's merge on, the last token takes a decode step: it is there
   // that the hook acts first)
@@ -984,21 +987,27 @@ hipError_t setup_state(Session *s, int32_t *failure_stage, bool with_weights) {
   const uint64_t off_attn_plan = c.take(attn_plan_bytes(kAttnMaxSplits));
   const uint64_t off_attn_tagged = c.take(attn_step_workspace_bytes(s->heads));
   const uint64_t off_sample_ws = c.take(sample_workspace_bytes());
-  // A prompt's pass: eight blocks, fewer where the context has no room for as many tokens
-  const uint64_t pB = kGemmDeepMaxTokens;
-  const uint64_t pT = std::max<uint64_t>(pB, std::min<uint64_t>(kGemmPassMaxTokens, (s->max_ctx + pB - 1) / pB * pB));
-  const uint64_t off_px = c.take(pT * H * 4);
-  const uint64_t off_pr = c.take(pT * H * 4);
-  const uint64_t off_pqkv = c.take(pT * (A + 2 * KV) * 4);
-  const uint64_t off_pxn16 = c.take(pT * H * 2);
-  const uint64_t off_pattn16 = c.take(pT * A * 2);
-  const uint64_t off_pff16 = c.take(pT * I * 2);
-  const uint64_t off_prope = c.take(pT * HD * 4);
+  // Rows of a prompt block (or a batch step)
+  const uint64_t pB = kGemmDeepMaxTokens, widest = std::max<uint64_t>(H, A + 2 * KV);
+  struct RowOffsets {
+    uint64_t px, pr, pqkv, pxn16, pattn16, pff16, prope, pgemm_ws;
+  };
+  const auto take_rows = [&](uint64_t rows, uint64_t gemm_bytes) {
+    RowOffsets o;
+    o.px = c.take(rows * H * 4);
+    o.pr = c.take(rows * H * 4);
+    o.pqkv = c.take(rows * (A + 2 * KV) * 4);
+    o.pxn16 = c.take(rows * H * 2);
+    o.pattn16 = c.take(rows * A * 2);
+    o.pff16 = c.take(rows * I * 2);
+    o.prope = c.take(rows * HD * 4);
+    o.pgemm_ws = c.take(gemm_bytes);
+    return o;
+  };
+  const uint64_t pgemm_ws_bytes = gemm_block_workspace_bytes(static_cast<uint32_t>(widest));
+  const RowOffsets off_rows = take_rows(pB, pgemm_ws_bytes);
   const uint64_t pattn_ws_stride = (attn_ws_bytes + 255u) & ~uint64_t{255};
   const uint64_t off_pattn_ws = c.take(pB * pattn_ws_stride);
-  const uint64_t widest = std::max<uint64_t>(H, A + 2 * KV);   // (a pass's partial sums: two slices of the widest)
-  const uint64_t pgemm_ws_bytes = std::max(gemm_block_workspace_bytes(static_cast<uint32_t>(widest)), 2 * pT * widest * sizeof(float));
-  const uint64_t off_pgemm_ws = c.take(pgemm_ws_bytes);
   const uint64_t off_sampler_dev = c.take(sizeof(SamplerDev));
   const uint64_t off_sampler_keys = c.take(sampler_workspace_bytes(s->vocab));
   const uint64_t off_attn_trace = c.take(L * 32 * 8);
@@ -1022,9 +1031,38 @@ hipError_t setup_state(Session *s, int32_t *failure_stage, bool with_weights) {
   const uint64_t off_blogits = head_block ? c.take(static_cast<uint64_t>(NERVA_HIP_BATCH_MAX_BLOCK_TOKENS) * V * 4) : 0;
   const uint64_t off_btable = c.take(sizeof(BatchTable));
   const uint64_t off_bslots = c.take(static_cast<uint64_t>(NERVA_HIP_BATCH_MAX_BLOCK_TOKENS) * sizeof(Slot));
+  // ("prefill_walk" override = 1, read here: one prompt step per token where prompt blocks would be possible)
+  s->block_prefill = s->rows_ready && tuning(kTunePrefillWalk) != 1;
+  // Prompt blocks of 512 tokens where all four projections of a layer have the kernel for them (256 weight rows x
+  // 256 tokens a workgroup: half the X bytes per product of the 256-token kernel), else of 256 tokens where they
+  // have that kernel (twice the tokens per weight byte of the 128-token one): every width that is a multiple of 64
+  // qualifies for both; other widths keep 128-token blocks. The "prefill_block_tokens" override caps the choice.
+  const auto all_four = [&](uint32_t tokens) {
+    return gemm_rows_takes(kGemmF32, static_cast<uint32_t>(A + 2 * KV), s->hidden, tokens, pgemm_ws_bytes) &&
+           gemm_rows_takes(kGemmResidual, s->hidden, static_cast<uint32_t>(A), tokens, pgemm_ws_bytes) &&
+           gemm_rows_takes(kGemmSwiglu, s->intermediate, s->hidden, tokens, pgemm_ws_bytes) &&
+           gemm_rows_takes(kGemmResidual, s->hidden, s->intermediate, tokens, pgemm_ws_bytes);
+  };
+  const int block_cap = tuning(kTunePrefillBlockTokens);
+  // (a prompt's last block can have any size: larger blocks only where every smaller one has its kernel too)
+  const bool wide = block_cap != 128 && tuning(kTuneBlockLayout) != 1 && all_four(kGemmMaxTokens + 1) && all_four(kGemmWideMaxTokens);
+  const bool deep = wide && block_cap != 256 && all_four(kGemmWideMaxTokens + 1) && all_four(kGemmDeepMaxTokens);
+  s->prefill_block_tokens = deep ? kGemmDeepMaxTokens : wide ? kGemmWideMaxTokens : kGemmMaxTokens;
+  s->prefill_pass_tokens = s->prefill_block_tokens;
+  // A pass of the layers takes up to eight blocks of 512 through the projections together: an 8192 token prompt and 64 steps
+  // of 36 layers of 4096 x 12288 take 382 ms with passes of 512 tokens, 356 / 336 / 332 with 1024 / 2048 / 4096 (a page of
+  // 900 tokens 3584 wide: 11.3 and 10.8). The rows for that are there once, with the weights, and only where the
+  // context has room for more than a block.
+  uint64_t pT = std::min<uint64_t>(kGemmPassMaxTokens, (s->max_ctx + pB - 1) / pB * pB);
+  if (block_cap >= 512) pT = std::min<uint64_t>(pT, static_cast<uint64_t>(block_cap) / 512u * 512u);
+  const bool passes = s->block_prefill && deep && pT > pB;
+  RowOffsets off_pass{};
+  const uint64_t pass_ws_bytes = std::max(pgemm_ws_bytes, 2 * pT * widest * sizeof(float));   // (partial sums: two slices of the widest)
+  if (passes && with_weights) off_pass = take_rows(pT, pass_ws_bytes);
   s->state_bytes = c.offset;
 
   hipError_t err = allocate_session(s, failure_stage, with_weights);
+  if (err == hipSuccess && with_weights) err = hipEventCreateWithFlags(&s->weights->pass_done, hipEventDisableTiming);
   if (err != hipSuccess) return err;
 
   auto dev16 = [&](uint64_t off) { return reinterpret_cast<uint16_t *>(s->arena + off); };
@@ -1047,43 +1085,30 @@ hipError_t setup_state(Session *s, int32_t *failure_stage, bool with_weights) {
   if (attn_matrix_cores(s->heads, s->kv_heads, s->head_dim))   // the plan serves the step kernel
     s->attn_plan = reinterpret_cast<uint32_t *>(s->arena + off_attn_plan);
   s->sample_ws = s->arena + off_sample_ws;
-  s->px = reinterpret_cast<float *>(s->arena + off_px);
-  s->pr = reinterpret_cast<float *>(s->arena + off_pr);
-  s->pqkv = reinterpret_cast<float *>(s->arena + off_pqkv);
-  s->pxn16 = dev16(off_pxn16);
-  s->pattn16 = dev16(off_pattn16);
-  s->pff16 = dev16(off_pff16);
-  s->prope = reinterpret_cast<float *>(s->arena + off_prope);
+  const auto bind_rows = [&](RowScratch &rows, const RowOffsets &o, uint64_t gemm_bytes) {
+    rows.px = reinterpret_cast<float *>(s->arena + o.px);
+    rows.pr = reinterpret_cast<float *>(s->arena + o.pr);
+    rows.pqkv = reinterpret_cast<float *>(s->arena + o.pqkv);
+    rows.pxn16 = dev16(o.pxn16);
+    rows.pattn16 = dev16(o.pattn16);
+    rows.pff16 = dev16(o.pff16);
+    rows.prope = reinterpret_cast<float *>(s->arena + o.prope);
+    rows.pgemm_ws = s->arena + o.pgemm_ws;
+    rows.pgemm_ws_bytes = gemm_bytes;
+  };
+  bind_rows(*s, off_rows, pgemm_ws_bytes);
+  if (passes && with_weights) {
+    bind_rows(s->weights->pass, off_pass, pass_ws_bytes);
+    s->weights->pass.prefill_pass_tokens = static_cast<uint32_t>(pT);
+  }
+  // (a session made with other overrides than the one that made the weights: as far as their rows go)
+  if (passes && s->weights->pass.px != nullptr)
+    s->prefill_long_tokens = std::min(static_cast<uint32_t>(pT), s->weights->pass.prefill_pass_tokens);
   s->pattn_ws = s->arena + off_pattn_ws;
   s->pattn_ws_stride = pattn_ws_stride;
-  s->pgemm_ws = s->arena + off_pgemm_ws;
-  s->pgemm_ws_bytes = pgemm_ws_bytes;
-  // Prompt blocks of 512 tokens where all four projections of a layer have the kernel for them (256 weight rows x
-  // 256 tokens a workgroup: half the X bytes per product of the 256-token kernel), else of 256 tokens where they
-  // have that kernel (twice the tokens per weight byte of the 128-token one): every width that is a multiple of 64
-  // qualifies for both; other widths keep 128-token blocks. The "prefill_block_tokens" override caps the choice.
-  const auto all_four = [&](uint32_t tokens) {
-    return gemm_rows_takes(kGemmF32, static_cast<uint32_t>(A + 2 * KV), s->hidden, tokens, pgemm_ws_bytes) &&
-           gemm_rows_takes(kGemmResidual, s->hidden, static_cast<uint32_t>(A), tokens, pgemm_ws_bytes) &&
-           gemm_rows_takes(kGemmSwiglu, s->intermediate, s->hidden, tokens, pgemm_ws_bytes) &&
-           gemm_rows_takes(kGemmResidual, s->hidden, s->intermediate, tokens, pgemm_ws_bytes);
-  };
-  // A pass of the layers takes up to eight blocks of 512 through the projections together: an 8192 token prompt and 64 steps
-  // of 36 layers of 4096 x 12288 take 382 ms with passes of 512 tokens, 356 / 336 / 332 with 1024 / 2048 / 4096 (a page of
-  // 900 tokens 3584 wide: 11.3 and 10.8).
-  const int block_cap = tuning(kTunePrefillBlockTokens);
-  // (a prompt's last block can have any size: larger blocks only where every smaller one has its kernel too)
-  const bool wide = block_cap != 128 && tuning(kTuneBlockLayout) != 1 && all_four(kGemmMaxTokens + 1) && all_four(kGemmWideMaxTokens);
-  const bool deep = wide && block_cap != 256 && all_four(kGemmWideMaxTokens + 1) && all_four(kGemmDeepMaxTokens);
-  s->prefill_block_tokens = deep ? kGemmDeepMaxTokens : wide ? kGemmWideMaxTokens : kGemmMaxTokens;
-  s->prefill_pass_tokens = !deep ? s->prefill_block_tokens
-                           : block_cap >= 512 ? std::min(static_cast<uint32_t>(pT), static_cast<uint32_t>(block_cap) / 512u * 512u)
-                                              : static_cast<uint32_t>(pT);
   s->blogits = head_block ? reinterpret_cast<float *>(s->arena + off_blogits) : nullptr;
   s->btable = reinterpret_cast<BatchTable *>(s->arena + off_btable);
   s->bslots = reinterpret_cast<Slot *>(s->arena + off_bslots);
-  // ("prefill_walk" override = 1, read here: one prompt step per token where prompt blocks would be possible)
-  s->block_prefill = s->rows_ready && tuning(kTunePrefillWalk) != 1;
   s->sampler_dev = reinterpret_cast<SamplerDev *>(s->arena + off_sampler_dev);
   s->sampler_keys = reinterpret_cast<uint64_t *>(s->arena + off_sampler_keys);
   {

@@ -148,7 +148,7 @@ MixedAttnParams attention_params(Session *s, const StackLayer &layer, const floa
   a.scale = layer.spec.score_scale;
   a.cache32 = wide(s) ? 1u : 0u;
   a.max_steps = s->max_ctx;
-  a.workspace = s->attn_ws;
+  a.workspace = s->stack_attn_ws;
   a.last_block = m.logical_blocks - 1;
   return a;
 }
@@ -196,7 +196,7 @@ LatentAttnParams latent_params(Session *s, const StackLayer &w, const float *pro
   a.scale = w.spec.score_scale;
   a.cache32 = wide(s) ? 1u : 0u;
   a.max_steps = s->max_ctx;
-  a.workspace = s->attn_ws;
+  a.workspace = s->stack_attn_ws;
   a.last_block = m.logical_blocks - 1;
   return a;
 }
@@ -742,10 +742,11 @@ uint64_t nv::stack_step_launches(const Session *s) {
 
 hipError_t nv::stack_prompt(Session *s, uint32_t begin, uint32_t end, const uint32_t *wanted, uint32_t wanted_count, float *logits,
                             float *residuals, NervaHipHfDecodeSequenceResult *out) {
-  hipError_t err = hipSuccess;
+  const PassTurn rows(s, end - begin);
+  hipError_t err = rows.error;
   uint32_t next_wanted = 0;
   const uint64_t H = s->hidden;
-  const uint32_t most = s->stack->block_tokens;
+  const uint32_t most = s->prefill_pass_tokens;
   for (uint32_t first = begin; err == hipSuccess && first < end; first += most) {
     Block b{s, std::min(most, end - first), first, false, Seam{}, 0};
     err = b.layers(residuals != nullptr ? residuals + static_cast<uint64_t>(first - begin) * H : nullptr,
@@ -987,12 +988,13 @@ int create_stack(const NervaHipStackSessionCreateRequest *rq, bool synthetic, ui
   for (const StackLayer &w : m.layers) experts = experts && w.spec.mixer == NERVA_HIP_MIXER_LATENT && w.spec.ff == 0;
   bool routed = false;
   for (const StackLayer &w : m.layers) routed = routed || w.spec.experts != 0;
-  if (experts) m.block_tokens = m.chunk_tokens = kExpertBlockTokens;
-  else if (!routed && rq->precision != NERVA_HIP_PRECISION_32)
+  if (experts) m.chunk_tokens = kExpertBlockTokens;
+  m.block_tokens = m.chunk_tokens;
+  if (!experts && !routed && rq->precision != NERVA_HIP_PRECISION_32)
     m.block_tokens = std::max(kStackBlockTokens, std::min(kGemmPassMaxTokens, (s->max_ctx + kStackBlockTokens - 1) / kStackBlockTokens * kStackBlockTokens));
   for (const StackLayer &w : m.layers)
     if (w.spec.experts != 0)
-      m.plan_bytes = std::max(m.plan_bytes, moe_plan_bytes(m.block_tokens, w.spec.experts_per_token, w.spec.experts));
+      m.plan_bytes = std::max(m.plan_bytes, moe_plan_bytes(m.chunk_tokens, w.spec.experts_per_token, w.spec.experts));
   for (uint32_t l = 0; l < L; ++l) {
     StackLayer &w = m.layers[l];
     if (!w.own_cache()) continue;
@@ -1216,7 +1218,7 @@ int create_stack(const NervaHipStackSessionCreateRequest *rq, bool synthetic, ui
 
 hipError_t nv::stack_setup_state(Session *s, int32_t *failure_stage, bool with_weights) {
   const StackModel &m = *s->stack;
-  const uint64_t H = s->hidden, V = s->vocab, T = m.block_tokens, es = wide(s) ? 4 : 2;
+  const uint64_t H = s->hidden, V = s->vocab, T = m.chunk_tokens, es = wide(s) ? 4 : 2;
   s->block_count = m.logical_blocks;
   s->kv_bytes = m.cache_bytes;
   s->stack_state_bytes = m.state_floats * sizeof(float);
@@ -1231,26 +1233,47 @@ hipError_t nv::stack_setup_state(Session *s, int32_t *failure_stage, bool with_w
   const uint64_t off_angles = c.take(angles * 12 + 4);
   const uint64_t off_sample_ws = c.take(sample_workspace_bytes()), off_sampler_dev = c.take(sizeof(SamplerDev)),
                  off_sampler_keys = c.take(sampler_workspace_bytes(s->vocab));
-  const uint64_t off_px = c.take(T * H * 4), off_py = c.take(T * H * 4), off_pin = c.take(T * m.max_in * 4),
-                 off_pxn = c.take(T * H * es), off_pmix = c.take(T * m.max_mix * es), off_pff = c.take(T * m.max_ff * es),
-                 off_prope = c.take(T * m.rotation_columns * 4ull + 4), off_pgemm = c.take(s->pgemm_ws_bytes);
-  uint64_t attn_ws_bytes = 0;
-  for (const StackLayer &w : m.layers)
-    if (w.spec.mixer == NERVA_HIP_MIXER_ATTENTION && !wide(s) &&
-        mixed_attention_wide(w.spec.heads, w.spec.kv_heads, w.spec.key_dim, w.spec.value_dim))
-      attn_ws_bytes = std::max(attn_ws_bytes, mixed_attention_workspace_bytes(w.spec.heads, m.block_tokens));
-    else if (w.spec.mixer == NERVA_HIP_MIXER_LATENT && !wide(s) &&
-             latent_attention_wide(w.spec.heads, w.spec.key_dim, w.spec.rotary_key_dim, w.spec.value_dim, w.spec.kv_rank))
-      attn_ws_bytes = std::max(attn_ws_bytes, latent_workspace_bytes(w.spec.heads, w.spec.rotary_key_dim, w.spec.kv_rank, m.block_tokens));
-  const uint64_t off_attn_ws = c.take(attn_ws_bytes);
+  // rows of a block of T token rows, and of a pass with the weights' own
+  struct RowOffsets {
+    uint64_t px, py, pin, pxn, pmix, pff, prope, pgemm, attn_ws, pxn2, pz, pql, pq;
+  };
+  const auto take_rows = [&](uint64_t rows) {
+    uint64_t attn_ws_bytes = 0;
+    for (const StackLayer &w : m.layers)
+      if (w.spec.mixer == NERVA_HIP_MIXER_ATTENTION && !wide(s) &&
+          mixed_attention_wide(w.spec.heads, w.spec.kv_heads, w.spec.key_dim, w.spec.value_dim))
+        attn_ws_bytes = std::max(attn_ws_bytes, mixed_attention_workspace_bytes(w.spec.heads, static_cast<uint32_t>(rows)));
+      else if (w.spec.mixer == NERVA_HIP_MIXER_LATENT && !wide(s) &&
+               latent_attention_wide(w.spec.heads, w.spec.key_dim, w.spec.rotary_key_dim, w.spec.value_dim, w.spec.kv_rank))
+        attn_ws_bytes = std::max(attn_ws_bytes,
+                                 latent_workspace_bytes(w.spec.heads, w.spec.rotary_key_dim, w.spec.kv_rank, static_cast<uint32_t>(rows)));
+    const uint64_t both = parallel(s) ? rows * H : 0;   // layers whose sublayers read the same row
+    RowOffsets o;
+    o.px = c.take(rows * H * 4);
+    o.py = c.take(rows * H * 4);
+    o.pin = c.take(rows * m.max_in * 4);
+    o.pxn = c.take(rows * H * es);
+    o.pmix = c.take(rows * m.max_mix * es);
+    o.pff = c.take(rows * m.max_ff * es);
+    o.prope = c.take(rows * m.rotation_columns * 4ull + 4);
+    o.pgemm = c.take(s->pgemm_ws_bytes);
+    o.attn_ws = c.take(attn_ws_bytes);
+    o.pxn2 = c.take(both * es);
+    o.pz = c.take(both * 4);
+    o.pql = c.take(rows * m.max_q_rank * es);
+    o.pq = c.take(rows * m.max_q * 4ull);
+    return o;
+  };
+  const RowOffsets off_rows = take_rows(T);
   const uint64_t off_want = c.take(kStackWantedRows * H * es), off_want_rows = c.take(kStackWantedRows * 4ull),
                  off_want_logits = c.take(kStackWantedRows * V * 4ull);
-  const uint64_t both = parallel(s) ? T * H : 0;   // layers whose sublayers read the same row
-  const uint64_t off_pxn2 = c.take(both * es), off_pz = c.take(both * 4), off_pql = c.take(T * m.max_q_rank * es),
-                 off_pq = c.take(T * m.max_q * 4ull), off_router = c.take(T * m.max_experts * 4ull),
-                 off_slots_rows = c.take(T * m.max_top * H * 4), off_plan = c.take(m.plan_bytes);
+  const uint64_t off_router = c.take(T * m.max_experts * 4ull), off_slots_rows = c.take(T * m.max_top * H * 4), off_plan = c.take(m.plan_bytes);
+  const bool passes = m.block_tokens > m.chunk_tokens;
+  RowOffsets off_pass{};
+  if (passes && with_weights) off_pass = take_rows(m.block_tokens);
   s->state_bytes = c.offset;
   hipError_t err = allocate_session(s, failure_stage, with_weights);
+  if (err == hipSuccess && with_weights) err = hipEventCreateWithFlags(&s->weights->pass_done, hipEventDisableTiming);
   if (err != hipSuccess) return err;
   *failure_stage = 5;
   const auto f32 = [&](uint64_t off) { return reinterpret_cast<float *>(s->arena + off); };
@@ -1271,19 +1294,26 @@ hipError_t nv::stack_setup_state(Session *s, int32_t *failure_stage, bool with_w
   s->sample_ws = s->arena + off_sample_ws;
   s->sampler_dev = reinterpret_cast<SamplerDev *>(s->arena + off_sampler_dev);
   s->sampler_keys = reinterpret_cast<uint64_t *>(s->arena + off_sampler_keys);
-  s->px = f32(off_px);
-  s->py = f32(off_py);
-  s->pqkv = f32(off_pin);
-  s->pxn = s->arena + off_pxn;
-  s->pmix = s->arena + off_pmix;
-  s->pff = s->arena + off_pff;
-  s->prope = f32(off_prope);
-  s->pgemm_ws = s->arena + off_pgemm;
-  s->attn_ws = s->arena + off_attn_ws;
-  s->pxn2 = s->arena + off_pxn2;
-  s->pz = f32(off_pz);
-  s->pql = s->arena + off_pql;
-  s->pq = f32(off_pq);
+  const auto bind_rows = [&](RowScratch &rows, const RowOffsets &o, uint32_t tokens) {
+    rows.px = f32(o.px);
+    rows.py = f32(o.py);
+    rows.pqkv = f32(o.pin);
+    rows.pxn = s->arena + o.pxn;
+    rows.pmix = s->arena + o.pmix;
+    rows.pff = s->arena + o.pff;
+    rows.prope = f32(o.prope);
+    rows.pgemm_ws = s->arena + o.pgemm;
+    rows.pgemm_ws_bytes = s->pgemm_ws_bytes;
+    rows.stack_attn_ws = s->arena + o.attn_ws;
+    rows.pxn2 = s->arena + o.pxn2;
+    rows.pz = f32(o.pz);
+    rows.pql = s->arena + o.pql;
+    rows.pq = f32(o.pq);
+    rows.prefill_pass_tokens = tokens;
+  };
+  bind_rows(*s, off_rows, m.chunk_tokens);
+  if (passes && with_weights) bind_rows(s->weights->pass, off_pass, m.block_tokens);
+  s->prefill_long_tokens = passes ? m.block_tokens : 0u;
   s->prouter = f32(off_router);
   s->pslots = f32(off_slots_rows);
   s->pplan = s->arena + off_plan;

@@ -52,8 +52,8 @@ struct StackLayer {
 struct StackModel {
   std::vector<StackLayer> layers;
   uint32_t precision = NERVA_HIP_PRECISION_16;
-  uint32_t block_tokens = kStackBlockTokens;      // token rows the layers take at a time
-  uint32_t chunk_tokens = kStackBlockTokens;      // what a session reports
+  uint32_t chunk_tokens = kStackBlockTokens;      // token rows a session has rows of its own for
+  uint32_t block_tokens = kStackBlockTokens;      // ... and a pass of a longer prompt takes, on the rows of its weights (RowScratch)
   uint32_t arrangement = NERVA_HIP_STACK_SANDWICH;
   float embedding_scale = 1.0f, logit_scale = 1.0f;
   const uint16_t *final_w = nullptr, *final_b = nullptr;

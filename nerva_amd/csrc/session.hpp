@@ -3,6 +3,7 @@
 
 #include <atomic>
 #include <memory>
+#include <mutex>
 #include <vector>
 
 #include "argmax.cuh"
@@ -24,9 +25,33 @@ struct LayerDev {
 enum StepMode { kDecodeStep = 0, kPromptStep = 1, kPromptHeadStep = 2 };
 enum LaunchKind { kLEmbed = 0, kLQkv, kLAttn, kLO, kLGateUp, kLDown, kLHead, kLAdvance, kLKinds };
 
+// Token rows of a prompt block or a batch step between the launches of the layers. Uniform decoder layers (16-bit rows by
+// type) and mixed stacks (untyped rows of the session's precision) each use their part.
+struct RowScratch {
+  float *px = nullptr, *pr = nullptr, *pqkv = nullptr, *prope = nullptr;
+  uint16_t *pxn16 = nullptr, *pattn16 = nullptr, *pff16 = nullptr;
+  char *pgemm_ws = nullptr;        // partial sums of the K-sliced projections
+  uint64_t pgemm_ws_bytes = 0;
+  float *py = nullptr;               // output of the sublayer under way, before its norm
+  void *pxn = nullptr, *pmix = nullptr, *pff = nullptr;   // 16-bit or f32 token rows (the session's precision)
+  // layers whose sublayers read the same row: the feed-forward's normalised rows and output
+  void *pxn2 = nullptr;
+  float *pz = nullptr;
+  void *pql = nullptr;               // latent attention: normalised query latents, queries
+  float *pq = nullptr;
+  void *stack_attn_ws = nullptr;     // split partials of the attention kernels
+  uint32_t prefill_pass_tokens = kGemmMaxTokens;   // token rows there is room for: what a pass of the layers takes
+};
+
 // The weight arena of a session and of every session forked from it (one stream of the weights can
 // then serve a token row of each of them); freed by the last of them to go.
 struct SharedWeights {
+  // Rows for passes of more than a block of a prompt, of the creating session and all its forks: at 4096 x 12288 another
+  // 435 MB, which 32 forks would hold once each and hardly use at the same time. Sessions take turns (PassTurn), in
+  // the order in which they enqueue: the event says when the turn before has left the device.
+  RowScratch pass;
+  std::mutex pass_turn;
+  hipEvent_t pass_done = nullptr;
   char *origin = nullptr;  // what the allocator returned (and takes back)
   char *base = nullptr;    // the first kMatrixAlign boundary in it: offsets of the weight layout count from here
   uint64_t bytes = 0;
@@ -45,7 +70,7 @@ struct StackModel;   // layer_stack.hpp
 
 }  // namespace nv
 
-struct NervaHipHfDecodeSequenceSession {
+struct NervaHipHfDecodeSequenceSession : nv::RowScratch {
   uint32_t dtype = 0, hidden = 0, heads = 0, kv_heads = 0, head_dim = 0, intermediate = 0, vocab = 0,
            layers = 0, max_ctx = 0;
   float eps = 0.0f, theta = 0.0f;
@@ -84,7 +109,7 @@ struct NervaHipHfDecodeSequenceSession {
   hipGraphExec_t exec[3] = {nullptr, nullptr, nullptr};
   uint64_t graph_nodes[3] = {0, 0, 0};
   // prompt blocks: up to prefill_pass_tokens prompt tokens per pass through the layers (weights streamed
-  // once per pass on the matrix cores); false = one prompt step per token
+  // once per pass on the matrix cores), in a long prompt prefill_long_tokens; false = one prompt step per token
   bool block_prefill = false;
   // the multi-row kernels take this model's shapes (prompt blocks and batch steps need it)
   bool rows_ready = false;
@@ -94,13 +119,9 @@ struct NervaHipHfDecodeSequenceSession {
   uint32_t head_run = 0;             // rows of the last of the latter
   nv::BatchTable *btable = nullptr, *host_btable = nullptr;
   nv::Slot *bslots = nullptr, *host_bslots = nullptr;   // a batch step's published slots, gathered for one copy
-  float *px = nullptr, *pr = nullptr, *pqkv = nullptr, *prope = nullptr;
-  uint16_t *pxn16 = nullptr, *pattn16 = nullptr, *pff16 = nullptr;
   char *pattn_ws = nullptr;
   uint64_t pattn_ws_stride = 0;
-  char *pgemm_ws = nullptr;        // partial sums of the K-sliced projections of a prompt block
-  uint64_t pgemm_ws_bytes = 0;
-  uint32_t prefill_pass_tokens = nv::kGemmMaxTokens;    // tokens a pass of the layers takes: a block, or several where the projections take them together
+  uint32_t prefill_long_tokens = 0;   // tokens a pass of a prompt of more than prefill_pass_tokens takes, with the rows of all sessions on these weights (0: no such passes)
   uint32_t prefill_block_tokens = nv::kGemmMaxTokens;   // tokens per prompt block: 512 or 256 where every projection has the kernel for it
   nv::SamplerDev sampler{};            // normalised configuration of the active sequence
   nv::SamplerDev *sampler_dev = nullptr;
@@ -125,19 +146,13 @@ struct NervaHipHfDecodeSequenceSession {
   uint32_t *stack_tables = nullptr;  // logical block -> block of the layer's ring, per caching layer
   float *stack_state = nullptr;      // recurrent state, f32, all recurrent layers
   uint64_t stack_state_bytes = 0;
-  float *y = nullptr, *py = nullptr; // output of the sublayer under way, before its norm: decode row, token rows
+  float *y = nullptr;                // output of the sublayer under way, before its norm: decode row
   uint64_t stack_launches = 0;       // kernel launches of the step enqueued last (where the layers do not tell)
-  // layers whose sublayers read the same row: the feed-forward's normalised rows and output
-  void *pxn2 = nullptr;
-  float *pz = nullptr;
-  void *pql = nullptr;               // latent attention: normalised query latents, queries
-  float *pq = nullptr;
   float *prouter = nullptr, *pslots = nullptr;   // experts: router logits, one output row per (token, choice)
   void *pplan = nullptr;             // ... and the block's routing (MoePlan)
   void *pwant = nullptr;             // normalised rows whose logits are asked for, with their row numbers and logits
   uint32_t *pwant_rows = nullptr;
   float *pwant_logits = nullptr;
-  void *pxn = nullptr, *pmix = nullptr, *pff = nullptr;   // 16-bit or f32 token rows (the session's precision)
   // active sequence
   bool started = false, finished = false;
   uint32_t prompt_count = 0, observed = 0, cursor = 0, seed_token = 0, has_eos = 0, eos = 0;
@@ -161,6 +176,34 @@ struct Carver {
 // with the rotated walk 31.0 us at 0 modulo 8 MiB, 31.4 at 2 and 6 MiB, 31.8 at 4 MiB, 32.1 at an odd KiB (the
 // plain walk: 33.0 / 31.7 / 31.3 / 31.8 / 31.7). At most 8 MiB a matrix is left unused: under 1.2 GB for 36 layers.
 constexpr uint64_t kMatrixAlign = 8u << 20;
+
+// A prompt of `tokens` tokens: while this lives its session works on the shared rows of its weights, if it has more tokens
+// than the session's own rows take. Everything that reads rows has to be enqueued before it ends.
+class PassTurn {
+ public:
+  PassTurn(Session *session, uint32_t tokens) : s(session) {
+    if (tokens <= s->prefill_pass_tokens || s->prefill_long_tokens <= s->prefill_pass_tokens) return;
+    turn = std::unique_lock<std::mutex>(s->weights->pass_turn);
+    own = *s;
+    static_cast<RowScratch &>(*s) = s->weights->pass;
+    s->prefill_pass_tokens = s->prefill_long_tokens;
+    error = hipStreamWaitEvent(s->stream, s->weights->pass_done, 0);   // (nothing to wait for before its first record)
+  }
+  ~PassTurn() {
+    if (!turn.owns_lock()) return;
+    static_cast<RowScratch &>(*s) = own;
+    // whoever comes next waits on the device; where that cannot be arranged, here
+    if (hipEventRecord(s->weights->pass_done, s->stream) != hipSuccess) (void)hipStreamSynchronize(s->stream);
+  }
+  PassTurn(const PassTurn &) = delete;
+  PassTurn &operator=(const PassTurn &) = delete;
+  hipError_t error = hipSuccess;
+
+ private:
+  Session *s;
+  RowScratch own;
+  std::unique_lock<std::mutex> turn;
+};
 
 // Moves the sequence's device-side position words (decode_session.hip).
 hipError_t set_device_position(Session *s, uint32_t cursor, uint32_t prompt_count, uint32_t clear_fault);

@@ -1,0 +1,122 @@
+"""Rows of long prompts: there once for all sessions on the same weights, which take turns on them."""
+import threading
+
+import numpy as np
+import pytest
+
+import nerva_amd as N
+import stack_models as M
+from test_gpu_any_width import walked
+from test_gpu_session import BF16, E2E_REL_L2, F16, random_model, rel_l2
+
+pytestmark = pytest.mark.gpu
+
+# dtype, hidden, heads, kv, hd, inter, vocab, layers
+DENSE = (BF16, 1536, 12, 2, 128, 2944, 801, 2)
+
+
+def dense(geom=DENSE):
+    dtype, hidden, heads, kv, hd, inter, vocab, layers = geom
+    return random_model(dtype, hidden, heads, kv, hd, inter, vocab, layers, hidden, 1e6, False, False)[0]
+
+
+def decoder_session(max_context):
+    return N.DecodeSession.create(dense(), max_context)
+
+
+def stack_session(max_context):
+    cfg = M.config([M.attention(16, 4, 128, 128, rot=32, chunk=700, ff=320), M.mingru(width=320, ff=448), M.mingru(width=64, ff=0)],
+                   width=192, vocab=300)
+    return M.session(cfg, M.weights(cfg, seed=31), max_context)
+
+
+def without_cache(session):
+    return session.create_result.device_arena_bytes - session.create_result.resident_kv_bytes
+
+
+def test_only_the_weights_hold_rows_for_passes():
+    """A fork has rows for a block of 512, the creating session those for passes of 4096 besides; sessions that take no
+    passes (128-row blocks, a walk token by token, a head size without blocks) have neither, whatever their context."""
+    dtype, hidden, heads, kv, hd, inter, vocab, layers = DENSE
+    row = 10 * hidden + 4 * (heads + 2 * kv) * hd + 2 * heads * hd + 2 * inter
+    parent = decoder_session(4800)
+    fork = parent.fork_shared_weights()
+    assert without_cache(parent) - without_cache(fork) >= 4096 * row
+    for s in (fork, parent):
+        s.destroy()
+    odd, eighty = dense((BF16, 416, 6, 2, 128, 608, 517, 2)), dense((F16, 320, 4, 2, 80, 640, 301, 2))
+    for create in (lambda ctx: walked(dense(), ctx), lambda ctx: N.DecodeSession.create(odd, ctx), lambda ctx: N.DecodeSession.create(eighty, ctx)):
+        small, large = create(512), create(4800)
+        assert without_cache(large) - without_cache(small) <= (4800 - 512) * 64
+        for s in (small, large):
+            s.destroy()
+    parent = stack_session(4800)
+    fork = parent.fork_shared_weights()
+    assert without_cache(parent) - without_cache(fork) >= 4096 * 192 * 10
+    for s in (fork, parent):
+        s.destroy()
+
+
+@pytest.mark.parametrize("create", [decoder_session, stack_session])
+def test_long_prompts_of_sessions_on_the_same_weights(create):
+    """Three sessions on one set of weights, a thread each: long prompts, short ones and steps between them, twice over, as
+    each has them alone; and the forks go on when the creating session is gone."""
+    parent = create(2600)
+    sessions = [parent, parent.fork_shared_weights(), parent.fork_shared_weights()]
+    prompts = [[np.random.default_rng(10 * i + k).integers(0, parent.vocab, n).astype(np.uint32) for k, n in enumerate(lengths)]
+               for i, lengths in enumerate(((1700, 40, 900), (513, 2100, 300), (600, 601, 1025)))]
+
+    def work(session, own, results, at):
+        out = []
+        for prompt in own + own:
+            rc, _, logits, _ = session.extend(prompt, [0, prompt.size - 1])
+            assert rc == 0
+            rc, _, tokens = session.advance(3)
+            assert rc == 0 and session.release_sequence() == 0
+            out.append((logits, tokens.tolist()))
+        results[at] = out
+
+    def run(who, together):
+        results = [None] * 3
+        threads = [threading.Thread(target=work, args=(sessions[i], prompts[i], results, i)) for i in who]
+        for thread in threads:
+            thread.start()
+            if not together:
+                thread.join()
+        for thread in threads:
+            thread.join()
+        return results
+
+    alone, together = run((0, 1, 2), False), run((0, 1, 2), True)
+    parent.destroy()
+    orphaned = run((1, 2), True)
+    for i in range(3):
+        for got in (together, orphaned):
+            if got is orphaned and i == 0:
+                continue
+            for (logits, tokens), (want, want_tokens) in zip(got[i], alone[i]):
+                assert np.array_equal(logits, want) and tokens == want_tokens, i      # the same launches on the same rows
+    for s in sessions[1:]:
+        s.destroy()
+
+
+def test_a_fork_made_under_other_overrides():
+    """A fork that takes passes where the creating session did not has no rows for them; one that does not, where it did,
+    takes none: both have the prompt's logits."""
+    prompt = np.random.default_rng(5).integers(0, DENSE[6], 1500).astype(np.uint32)
+    logits = []
+    for first, second in ((0, 512), (512, 0), (1024, 0), (0, 1024)):
+        sessions = []
+        for cap in (first, second):
+            N.Device.set_tuning("prefill_block_tokens", cap)
+            try:
+                sessions.append(sessions[0].fork_shared_weights() if sessions else N.DecodeSession.create(dense(), 1600))
+            finally:
+                N.Device.set_tuning("prefill_block_tokens", 0)
+        for s in sessions:
+            assert s.start(prompt)[0] == 0
+            logits.append(s.logits().copy())
+        for s in sessions[::-1]:
+            s.destroy()
+    for got in logits[1:]:
+        assert rel_l2(got, logits[0]) <= E2E_REL_L2
