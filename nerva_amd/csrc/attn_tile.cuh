@@ -227,14 +227,7 @@ __device__ __forceinline__ void attn_load_tile(const AttnParams &p, uint32_t phy
 // One 16-token tile against the G query heads of the kv head (see attn_fast_body). F32_PARTS (see attn_step_kernel): queries
 // and probabilities in three parts, the third ones in operands of their own (columns 0 .. G-1). `down` (attn_scaled) undoes
 // the scale of the query of this lane's column.
-// n_keys may differ from lane to lane (by column: the prompt kernel's columns belong to tokens at
-// different positions). COLUMN_MASKS = a column may find a whole tile masked, even its first one: the
-// running maximum then stays at minus infinity, and the exponentials are taken against a finite stand-in
-// so that they come out as 0 instead of NaN.
-// LAZY_RESCALE = the accumulators are multiplied by alpha only in tiles where some lane's alpha is not 1 (a
-// running maximum that did not move gives exp2(0) = 1 exactly, so the result is the same bits): worth a branch
-// where a wave walks many tiles and the vector ALU is what it waits for (prompt blocks).
-template <uint32_t DT, int HD, int G, bool QX_LDS, bool F32_PARTS = false, bool COLUMN_MASKS = false, bool LAZY_RESCALE = false>
+template <uint32_t DT, int HD, int G, bool QX_LDS, bool F32_PARTS = false>
 __device__ __forceinline__ void attn_tile(uint4 (&kreg)[HD / 32], uint4 (&vreg)[HD / 32], const uint4 (&qx)[HD / 32],
                                           const uint4 *qx_lds, uint32_t b,
                                           uint32_t n_keys, int col, int grp, bool splice, uint32_t new_row,
@@ -262,7 +255,7 @@ __device__ __forceinline__ void attn_tile(uint4 (&kreg)[HD / 32], uint4 (&vreg)[
       }
     }
   }
-  if (!COLUMN_MASKS && (b + 1) * kKvBlockTokens > n_keys) {
+  if ((b + 1) * kKvBlockTokens > n_keys) {
     // The last tile's rows past the position hold whatever was there: their probabilities are 0, and so are the values
     // they meet (0 x NaN or infinity would not be)
     const uint32_t at = b * kKvBlockTokens + grp * 4, rows = n_keys > at ? n_keys - at : 0u;   // of this lane's four
@@ -298,10 +291,9 @@ __device__ __forceinline__ void attn_tile(uint4 (&kreg)[HD / 32], uint4 (&vreg)[
   float mb = fmaxf(fmaxf(sc[0], sc[1]), fmaxf(sc[2], sc[3]));
   mb = fmaxf(mb, __shfl_xor(mb, 16, kWave));
   mb = fmaxf(mb, __shfl_xor(mb, 32, kWave));
-  const float m_new = fmaxf(m, mb);   // finite: every processed tile has a valid token (without column masks)
-  const float m_ref = COLUMN_MASKS ? fmaxf(m_new, -3.0e38f) : m_new;
-  const float alpha = attn_exp2(m - m_ref);
-  const float m_low = kScaled ? m_ref - kAttnWeightShift : m_ref;
+  const float m_new = fmaxf(m, mb);   // finite: every processed tile has a valid token
+  const float alpha = attn_exp2(m - m_new);
+  const float m_low = kScaled ? m_new - kAttnWeightShift : m_new;
   uint32_t px[2], third[2];
   float psum = 0.0f;
 #pragma unroll
@@ -323,15 +315,9 @@ __device__ __forceinline__ void attn_tile(uint4 (&kreg)[HD / 32], uint4 (&vreg)[
   l = l * alpha + psum;
   m = m_new;
   const uint2 pb = make_uint2(px[0], px[1]);
-  if constexpr (LAZY_RESCALE) {
-    if (__any(alpha != 1.0f)) {
-#pragma unroll
-      for (int s2 = 0; s2 < HD / 16; ++s2) acc[s2] *= alpha;
-    }
-  }
 #pragma unroll
   for (int s2 = 0; s2 < HD / 16; ++s2) {
-    if constexpr (!LAZY_RESCALE) acc[s2] *= alpha;
+    acc[s2] *= alpha;
     const uint4 &vr = vreg[s2 / 2];
     const uint2 va = (s2 & 1) ? make_uint2(vr.z, vr.w) : make_uint2(vr.x, vr.y);
     acc[s2] = mfma_k16<DT>(va, pb, acc[s2]);
