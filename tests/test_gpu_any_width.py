@@ -259,3 +259,83 @@ def test_top_k_collects_from_the_runs_that_hold_candidates(n, kind):
                 assert margin < 1e-5, (top_k, position, got, want, margin)
                 close += 1
     assert close <= 1
+
+
+@pytest.mark.parametrize("geom,lengths", [
+    ((BF16, 512, 40, 8, 64, 512, 301, 2), (1601, 3333)),    # 272 and 560 workgroups
+    ((F16, 512, 48, 16, 64, 512, 301, 2), (1600, 2903)),    # 320 and 592
+    ((F16, 512, 32, 8, 128, 512, 301, 2), (2501, 4096)),    # 320 and 512
+    ((BF16, 512, 28, 4, 128, 512, 301, 2), (1999, 3001)),   # 252 and 376
+])
+def test_passes_through_one_attention_launch(geom, lengths):
+    """Passes whose attention takes all its blocks in one launch without splits - in each branch of the rule that says so - with
+    a ragged last group of tokens, from the start and behind 77 tokens, against passes of one block. That the launch is taken
+    shows in their number: the same as for a prompt of one block."""
+    dtype, hidden, heads, kv, hd, inter, vocab, layers = geom
+    weights, _ = random_model(dtype, hidden, heads, kv, hd, inter, vocab, layers, hidden, 1e5, True, False)
+    s = N.DecodeSession.create(weights, 4200)
+    N.Device.set_tuning("prefill_block_tokens", 512)
+    try:
+        single = N.DecodeSession.create(weights, 4200)
+    finally:
+        N.Device.set_tuning("prefill_block_tokens", 0)
+    rng = np.random.default_rng(hidden)
+    for prefix in (0, 77):
+        for n in lengths:
+            tokens = rng.integers(0, vocab, prefix + n).astype(np.uint32)
+
+            def prompt(session, count):
+                assert session.release_sequence() == 0
+                if prefix:
+                    assert session.extend(tokens[:prefix])[0] == 0
+                rc, res, _, _ = session.extend(tokens[prefix:prefix + count])
+                assert rc == 0
+                return res.kernel_launches
+
+            assert prompt(s, n) == prompt(s, 500) < prompt(single, n)
+            prompt(s, n)
+            assert rel_l2(s.logits(), single.logits()) <= E2E_REL_L2, (prefix, n)
+            for layer in range(layers):
+                for got, want in zip(s.kv_range(layer, 0, prefix + n), single.kv_range(layer, 0, prefix + n)):
+                    tol = 2e-3 if layer == 0 else E2E_REL_L2
+                    assert rel_l2(O.decode16(dtype, got), O.decode16(dtype, want)) <= tol, (prefix, n, layer)
+    for session in (s, single):
+        session.destroy()
+
+
+@pytest.mark.parametrize("vocab", [98305, 98306, 100003])
+def test_wanted_logits_of_a_large_vocabulary_of_any_size(vocab):
+    """From 98304 rows on a head takes two row tiles a wave; a vocabulary that is no multiple of 4 stores its logits one by
+    one. Rows side by side against each of them alone, through the head of a step."""
+    weights, _ = random_model(BF16, 192, 6, 2, 64, 320, vocab, 1, 5, 1e4, False, False)
+    s = N.DecodeSession.create(weights, 64)
+    tokens = np.random.default_rng(vocab).integers(0, vocab, 40).astype(np.uint32)
+    rc, _, rows, _ = s.extend(tokens, range(40))
+    assert rc == 0
+    for place in (0, 1, 31, 32, 38, 39):
+        assert s.release_sequence() == 0
+        rc, _, alone, _ = s.extend(tokens[:place + 1], [place])
+        assert rc == 0
+        assert rel_l2(rows[place], alone[0]) <= E2E_REL_L2 and np.max(np.abs(rows[place] - alone[0])) <= E2E_REL_L2 * np.max(np.abs(alone[0]))
+    s.destroy()
+
+
+def test_a_merge_that_gives_up_behind_a_prompt_in_blocks():
+    """The step-fault hook set once the prompt is in: its last token came with its block, so the first step that fails is the
+    one behind it - of heads of 64, five a key head, where few workgroups merge."""
+    weights, _ = random_model(F16, 640, 10, 2, 64, 1280, 301, 2, 9, 1e4, False, False)
+    s = N.DecodeSession.create(weights, 720)
+    prompt = np.random.default_rng(9).integers(0, 301, 700).astype(np.uint32)
+    assert s.start(prompt)[0] == 0
+    N.Device.set_tuning("attn_merge_spin_limit", 4)
+    N.Device.set_tuning("attn_withhold_split", 1 + 3)
+    try:
+        rc, res, tokens = s.advance(6)
+    finally:
+        N.Device.set_tuning("attn_merge_spin_limit", 0)
+        N.Device.set_tuning("attn_withhold_split", 0)
+    from nerva_amd import abi
+    assert rc == -1 and res.hip_error == abi.NERVA_HIP_ERROR_STEP_FAULT
+    slots = s.slots(len(prompt) - 1, 2).view(np.uint32).reshape(2, -1)
+    assert slots[0, 8] != abi.NERVA_HIP_SLOT_DEVICE_FAULT and slots[1, 8] == abi.NERVA_HIP_SLOT_DEVICE_FAULT
+    s.destroy()
