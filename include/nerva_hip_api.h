@@ -198,7 +198,10 @@ typedef struct NervaHipHfDecodeSequenceSessionCreateRequest {
       experimental_rt_sink_tokens;
 } NervaHipHfDecodeSequenceSessionCreateRequest;
 
-/* mirrors NervaCudaHfDecodeSequenceSessionCreateResult (nerva_cuda_api.h:640-687) */
+/* mirrors NervaCudaHfDecodeSequenceSessionCreateResult (nerva_cuda_api.h:640-687). prefill_chunk_tokens: prompt tokens
+ * that a session takes through the layers together on rows of its own (1: token by token). Prompts of more than 512 go in
+ * passes of up to 4096 where that is 512, on rows that lie once with the weights: device_arena_bytes has them in the creating
+ * session's figure, a fork's has not, and sessions on the same weights take turns on them. */
 typedef struct NervaHipHfDecodeSequenceSessionCreateResult {
   int32_t status, hip_error, failure_stage, device_count;
   uint32_t dtype, hidden, heads, kv_heads, head_dim, intermediate, vocab_size, layer_count,
@@ -622,18 +625,22 @@ typedef struct NervaHipPagedAttentionRequest {
   float *output_f32;            /* optional [heads*hd] */
   uint16_t *output16;           /* [heads*hd] rounded */
   uint32_t splits;              /* 0: the library's split-KV factor; 1..64: this one (tests). Refused with
-                                   hipErrorInvalidValue, and nothing launched, when it exceeds block_count or when
-                                   kv_heads * splits exceeds the device's compute units: the splits of a kv head
-                                   merge inside the launch and have to be resident together */
+                                   hipErrorInvalidValue, and nothing launched, when it exceeds block_count, or, at
+                                   head_dim 128 with 1, 2, 4 or 8 query heads a kv head, when kv_heads * splits
+                                   exceeds the device's compute units: the splits of a kv head merge inside the
+                                   launch and have to be resident together. At other shapes such a factor (and
+                                   any above 1 with more than 56 kv heads) runs without splits */
 } NervaHipPagedAttentionRequest;
 
 /* Fused per-head RMSNorm + RoPE + KV append + paged GQA split-KV decode attention
  * (kernels.cu:287-555, attention_kernels.cu:263-760; exact_blockwise_attention_into,
- * attention/exact/run.rs:13-127). */
+ * attention/exact/run.rs:13-127). Cache rows behind the position are not part of it, whatever they hold. A key or
+ * value of rows 0..position that is not finite leaves outputs that are not. output_f32 has the accuracy of f32
+ * sums, but for bf16 at head_dim 128 with 1, 2, 4 or 8 query heads a kv head: 3e-6 (queries and probabilities in 16 bits). */
 int nerva_hip_paged_gqa_decode(const NervaHipPagedAttentionRequest *request, void *stream,
                                int32_t *hip_error);
 uint64_t nerva_hip_paged_attention_workspace_bytes(uint32_t heads, uint32_t head_dim);
-/* The largest split factor nerva_hip_paged_gqa_decode accepts for this many kv heads on the current device. */
+/* The largest split factor nerva_hip_paged_gqa_decode splits a launch into for this many kv heads on the current device. */
 uint64_t nerva_hip_paged_attention_max_splits(uint32_t kv_heads);
 /* No counterpart in the reference (its attention reduces in a second launch and has no in-launch wait).
  * Synchronises `stream` and reports whether a launch of nerva_hip_paged_gqa_decode on this workspace gave up

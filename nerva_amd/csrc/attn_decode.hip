@@ -11,10 +11,11 @@
 //   grid (kv_heads, splits), 8 waves per workgroup; a wave owns whole 16-token KV
 //   tiles of its workgroup's token range and runs q.K^T and P.V on the matrix cores
 //   (details at attn_fast_body). The cache keeps each tile in matrix-operand order,
-//   so a tile is eight (HD = 64: four) coalesced 1 KiB loads straight into operand registers; two tiles
-//   are in flight per wave. LDS only carries q, the new K/V row and the cross-wave
-//   merge. The last workgroup to finish a kv head merges its split partials (arrival
-//   counter; nobody waits), so a layer needs no separate reduce launch.
+//   so a tile is eight (HD = 64: four) coalesced 1 KiB loads straight into operand registers. LDS
+//   only carries q, the new K/V row and the cross-wave merge. The splits of a kv head merge inside
+//   the launch, so a layer needs no separate reduce launch: of one token (attn_step_kernel) by workgroups
+//   that poll for each other's partials, of a block or a batch (attn_block_kernel) by the last one
+//   to finish (arrival counter; nobody waits).
 #include <stdlib.h>
 
 #include "attn_decode.cuh"

@@ -899,8 +899,8 @@ hipError_t prompt_tokens(Session *s, uint32_t begin, uint32_t end, const uint32_
   hipError_t err = rows.error;
   if (err != hipSuccess) return err;
   const uint32_t n = end - begin, last = n - 1;   // (place of the last token)
-  // (with the hook for the error path of the decode attention's merge on, the last token takes a decode step: it is there
-  // that the hook acts first)
+  // (with the hook for the error path of the decode attention's merge on, the last token takes a decode step, as a prompt's
+  // does that would leave it alone in a pass: so the hook acts on a start too)
   if (!s->block_prefill) {
     for (uint32_t i = begin; err == hipSuccess && i + 1 < end; ++i) err = launch_step(s, 1, out);
   } else if (n % s->prefill_pass_tokens != 1 && tuning(kTuneAttnWithholdSplit) == 0) {
@@ -1024,9 +1024,10 @@ hipError_t setup_state(Session *s, int32_t *failure_stage, bool with_weights) {
                     gemm_rows_takes(kGemmResidual, s->hidden, s->intermediate, kGemmMaxTokens, 0);
   }
   const bool head_block = s->rows_ready && gemm_rows_takes(kGemmF32, s->vocab, s->hidden, NERVA_HIP_BATCH_MAX_BLOCK_TOKENS, 0);
-  // A batch of sequences of a model with less than 4.5 MiB of weights a layer keeps the sequences' own steps, bit for bit
-  // what each computes alone, as such models always had it; from there on sharing pays at any number (eight layers 512 wide,
-  // steps of 2 / 6 / 32 sequences: their own 355 / 1240 / 7420 us at an MLP of 1024, shared 320 / 320 / 365 at 1536).
+  // Sequences of a model with less than 4.5 MiB of weights a layer advance by their own steps, bit for bit what each computes
+  // alone: what such models always had, and a promise (512 wide with an MLP of 1024, 4.25 MiB, is held to it). It is not where
+  // sharing begins to pay, which it does at any size and number (eight layers 512 wide, steps of 2 / 6 / 32 sequences: their
+  // own 355 / 1240 / 7420 us at an MLP of 1024, shared 320 / 320 / 365 at 1536).
   s->batch_ready = head_block && (A + KV) * H * 2 + 3 * H * I >= (9u << 18);
   const uint64_t off_blogits = head_block ? c.take(static_cast<uint64_t>(NERVA_HIP_BATCH_MAX_BLOCK_TOKENS) * V * 4) : 0;
   const uint64_t off_btable = c.take(sizeof(BatchTable));

@@ -712,7 +712,7 @@ __global__ __launch_bounds__(8 * kWave, 2) void gemm_deep_kernel(GemmRowsParams 
   }
   const uint32_t wlane = ((lane >> 3) * cols) * static_cast<uint32_t>(sizeof(uint16_t)) + (((lane & 7) ^ (lane >> 3)) << 4);
   // X requests of this wave: four consecutive token tiles of one K-step of the half's block
-  const uint32_t xtiles = p.x_packed;   // token tiles of the whole block per K-step (32 above 256 tokens)
+  const uint32_t xtiles = p.x_packed;   // token tiles of the whole block per K-step (16 for every 256 tokens)
   const char *xsrc = reinterpret_cast<const char *>(p.x16) +
                      ((static_cast<uint64_t>(k0 / 32u + (wave >> 2)) * xtiles + half * 16u + (wave & 3) * 4u) * kWave + lane) * sizeof(u32x4_t);
   const uint64_t xstep = static_cast<uint64_t>(2u * xtiles) * kWave * sizeof(u32x4_t);   // one K-block further
@@ -932,8 +932,8 @@ hipError_t launch_wide_pairs(const GemmRowsParams &p, float *partials, uint32_t 
   return hipGetLastError();
 }
 
-// Blocks of 257..512 rows (gemm_deep_kernel): workgroups of 256 rows (a gate/up pair: 128 + 128) x 256 tokens, or
-// of 192 rows (96 + 96) where the rows divide that way and the launch then fills the chip better.
+// gemm_deep_kernel (blocks of 129..4096 rows): workgroups of 256 weight rows (a gate/up pair: 128 + 128) x 256 tokens, or
+// of 192 (96 + 96) where the launch then fills the chip better.
 inline uint32_t deep_wg_rows(int epilogue, int tpw) { return (epilogue == kGemmSwiglu ? 32u : 64u) * static_cast<uint32_t>(tpw); }
 
 struct DeepPlan {
@@ -1159,7 +1159,7 @@ uint32_t gemm_wide_slices(int epilogue, uint32_t rows, uint32_t cols, uint32_t t
   return slices;
 }
 
-// Blocks of 129..512 rows: K slices of gemm_deep_kernel, or 0 where it does not take the shape (rows % 8, cols % 64).
+// Blocks of 129..kGemmPassMaxTokens rows: K slices of gemm_deep_kernel, or 0 where it does not take the shape (rows % 8, cols % 64).
 uint32_t gemm_deep_slices(int epilogue, uint32_t rows, uint32_t cols, uint32_t tokens, uint64_t workspace_bytes) {
   return deep_plan(epilogue, rows, cols, tokens, workspace_bytes).kslices;
 }
