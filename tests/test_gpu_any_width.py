@@ -339,3 +339,19 @@ def test_a_merge_that_gives_up_behind_a_prompt_in_blocks():
     slots = s.slots(len(prompt) - 1, 2).view(np.uint32).reshape(2, -1)
     assert slots[0, 8] != abi.NERVA_HIP_SLOT_DEVICE_FAULT and slots[1, 8] == abi.NERVA_HIP_SLOT_DEVICE_FAULT
     s.destroy()
+
+
+def test_stack_passes_past_4096_tokens():
+    """The largest pass of a mixed stack and some tokens behind it, through chunks of keys that start inside the pass and a
+    layer that sees everything, against the same tokens in portions of a block (which the tests of stacks hold to the oracle)."""
+    import stack_models as M
+    cfg = M.config([M.attention(16, 4, 128, 128, rot=32, chunk=700, ff=320), M.mingru(width=320, ff=448), M.attention(8, 2, 64, 64, rot=16, chunk=5000, ff=0)],
+                   width=192, vocab=300)
+    tensors, tokens = M.weights(cfg, seed=33), np.random.default_rng(4).integers(0, 300, 4500).astype(np.uint32)
+    rows = []
+    for sizes in ([4500], [512]):
+        s = M.session(cfg, tensors, 4600)
+        rows.append(M.feed(s, tokens, sizes))
+        s.destroy()
+    worst = M.errors(rows[0], rows[1])
+    assert worst.max() < 0.05, "position %d: %.2e" % (int(worst.argmax()), worst.max())   # (the bound of 16-bit stacks)
