@@ -582,7 +582,7 @@ __global__ __launch_bounds__(8 * kWave) void attn_step_kernel(AttnParams p) {
   // active splits, or fewer: kAttnWaitingWorkgroups), which polls the other splits' words until every tag is up - two memory round
   // trips after the slowest split's tiles (store, then the poll that finds it), where a ticket taken
   // after the stores have been performed and a merge by the last arriver needed four.
-  const uint32_t mergers = kF32Parts ? min(active, kAttnWaitingWorkgroups / gridDim.x) : active;
+  const uint32_t mergers = kF32Parts ? min(active, max(1u, kAttnWaitingWorkgroups / gridDim.x)) : active;
   if (split >= mergers) return;
   constexpr uint32_t kParts = G * (HD / kStepPartDims);
   constexpr int kMerged = StepShared<HD, G>::kMerged;
