@@ -779,6 +779,12 @@ hipError_t launch_dt(const AttnParams &p, hipStream_t stream) {
   const uint32_t group = p.heads / p.kv_heads;
   const bool block = p.tokens > 1 || p.seqs != nullptr;
   bool fast = attn_matrix_cores(p.heads, p.kv_heads, p.head_dim) && p.part_acc != nullptr && p.splits >= 1;
+  // The matrix-core kernels read the caches in pieces of 16 bytes and exchange words of 8. Shapes that came to them from the
+  // general kernel, which reads elements, go back to it where the caller's addresses are not made for that.
+  const auto at_multiple = [](const void *ptr, uintptr_t of) { return reinterpret_cast<uintptr_t>(ptr) % of == 0; };
+  if (fast && !block && attn_f32_shape(p.head_dim, group) &&
+      !(at_multiple(p.k_cache, 16) && at_multiple(p.v_cache, 16) && at_multiple(p.part_tagged, 8)))
+    fast = false;
   // every active split of a kv head has to be resident while the merges poll: a larger split factor is refused at the
   // shapes the split factor is declared for, and left to the general kernel, which has no splits, at the others
   if (fast && !block && p.splits > 1 && p.splits > attn_step_splits(p.heads, p.kv_heads, p.head_dim)) {

@@ -1,6 +1,7 @@
 """What a token does not see has no part in its attention: keys behind its position - rows of its last block that nobody has
 written, rows of an earlier sequence, later tokens of its prompt - may hold anything, numbers that are not finite too."""
 import threading
+from types import SimpleNamespace
 
 import numpy as np
 import pytest
@@ -219,3 +220,23 @@ def test_merges_by_few_workgroups(heads, kv_heads, hd):
                           splits=splits)
         assert rel_l2(out32.numpy(np.float32), ref) <= REL_L2, splits
     assert N.paged_attention_status(ws, heads, hd) == (0, 0)
+
+
+@pytest.mark.parametrize("heads,kv_heads,hd,dtype", [(28, 4, 128, BF16), (14, 2, 64, F16), (4, 2, 80, BF16)])
+def test_caches_and_workspaces_at_any_address_of_their_elements(heads, kv_heads, hd, dtype):
+    """Caches from an odd 16-bit element on, a workspace from an odd 32-bit one on, where element by element always did."""
+    for tokens, shift, ws_shift in ((70, 2, 0), (1000, 14, 0), (1000, 0, 4), (1000, 6, 12)):
+        c = _attention_case(dtype, heads, kv_heads, hd, tokens, 1e4, False, heads + tokens)
+        ref, _, _ = _attention_oracle(c)
+        cache = N.PagedKvCache(c["layers"], c["n_blocks"], kv_heads, hd, c["table"])
+        images = cache.host_layout(c["layer"], c["k_rows"], c["v_rows"])
+        buffers = [N.DeviceBuffer(image.nbytes + 16) for image in images]
+        for buf, image in zip(buffers, images):
+            buf.upload(image, shift)
+        views = [SimpleNamespace(ptr=buf.ptr + shift) for buf in buffers]
+        shifted = SimpleNamespace(k=views[0], v=views[1], table=cache.table, block_count=cache.block_count)
+        room = N.DeviceBuffer.zeros(N.abi.load().nerva_hip_paged_attention_workspace_bytes(heads, hd) + 16)
+        out16, out32 = N.DeviceBuffer(heads * hd * 2), N.DeviceBuffer(heads * hd * 4)
+        N.paged_attention(dtype, heads, kv_heads, hd, shifted, c["layer"], tokens, dev(c["qkv"]), room.ptr + ws_shift, out16,
+                          out_f32=out32, append=True, rope_theta=1e4)
+        assert rel_l2(out32.numpy(np.float32), ref) <= REL_L2, (tokens, shift, ws_shift)
