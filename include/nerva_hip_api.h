@@ -634,7 +634,9 @@ typedef struct NervaHipPagedAttentionRequest {
 
 /* Fused per-head RMSNorm + RoPE + KV append + paged GQA split-KV decode attention
  * (kernels.cu:287-555, attention_kernels.cu:263-760; exact_blockwise_attention_into,
- * attention/exact/run.rs:13-127). Cache rows behind the position are not part of it, whatever they hold. A key or
+ * attention/exact/run.rs:13-127). A call may be captured
+ * into a graph and replayed (with rope_theta > 0 after a first call on the workspace, which makes its table).
+ * Cache rows behind the position are not part of it, whatever they hold. A key or
  * value of rows 0..position that is not finite leaves outputs that are not. output_f32 has the accuracy of f32
  * sums, but for bf16 at head_dim 128 with 1, 2, 4 or 8 query heads a kv head: 3e-6 (queries and probabilities in 16 bits). */
 int nerva_hip_paged_gqa_decode(const NervaHipPagedAttentionRequest *request, void *stream,

@@ -93,9 +93,14 @@ struct AttnParams {
   // Decode step only: up to this many blocks in use, one split takes them all (attn_split_geometry). 0: never.
   uint32_t single_split_blocks;
   // Decode step only, the splits' merge. A partial is valid for the launch whose tag it carries: the tag is made
-  // of the launch's sequence number on this workspace - the plan's step number, or `launch_seq` without a plan -
+  // of the launch's sequence number on this workspace - the plan's step number, or `launches` without a plan -
   // and the layer, so a word that a late or earlier launch left behind can never be taken for this launch's.
-  uint32_t launch_seq;
+  // `launches`, a word for each kv head: kAttnLaunchQuantum for every launch on this workspace whose splits merged, added up
+  // by the workgroups themselves: a host's number would come back with every replay of a captured launch, and with it the
+  // words of the replay before. A workgroup adds its share behind its own look, so all of a kv head see the same number of
+  // whole quanta. (28 heads on 4, 900 keys: 8.8 -> 8.9 us; with one word for all
+  // kv heads and a look of its own 10.2.)
+  uint64_t *launches;
   // A merge gives up after this many polls of the words it waits for (0 = kAttnMergeSpinLimit), sets *fault
   // (optional device word, never cleared by a kernel) and leaves NaN in the outputs it feeds.
   uint32_t merge_spin_limit;
@@ -105,8 +110,10 @@ struct AttnParams {
   uint32_t withhold_split;
 };
 constexpr uint32_t kAttnMergeSpinLimit = 1u << 20;
+constexpr uint64_t kAttnLaunchQuantum = 65536;   // more than a kv head has splits
+constexpr uint32_t kAttnLaunchStride = 8;        // 64-bit words between kv heads': a cache line's part each
 // Tag of the partials of launch `seq` (never 0, the cleared state): distinct for 2^23 consecutive steps of up
-// to 256 layers; the words are cleared after every merge and when a sequence starts as well.
+// to 256 layers; a session's words are cleared when a sequence starts as well.
 __host__ __device__ __forceinline__ uint32_t attn_launch_tag(uint32_t seq, uint32_t layer) {
   return ((seq * 256u + (layer & 255u)) << 1) | 1u;
 }

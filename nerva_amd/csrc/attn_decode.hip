@@ -124,12 +124,12 @@ __global__ __launch_bounds__(W *kWave, W / 2) void attn_block_kernel(AttnParams 
 // nothing to the merge.
 // ---------------------------------------------------------------------------------------------
 __device__ __forceinline__ void sload4(const uint32_t *p0, const uint32_t *p1, const uint32_t *p2, const uint32_t *p3,
-                                       uint32_t (&v)[4]) {
+                                       const uint64_t *p4, uint32_t (&v)[4], uint64_t &w) {
   asm volatile(
-      "s_load_dword %0, %4, 0x0\n\ts_load_dword %1, %5, 0x0\n\ts_load_dword %2, %6, 0x0\n\ts_load_dword %3, %7, 0x0\n\t"
-      "s_waitcnt lgkmcnt(0)"
-      : "=&s"(v[0]), "=&s"(v[1]), "=&s"(v[2]), "=&s"(v[3])
-      : "s"(p0), "s"(p1), "s"(p2), "s"(p3)
+      "s_load_dword %0, %5, 0x0\n\ts_load_dword %1, %6, 0x0\n\ts_load_dword %2, %7, 0x0\n\t"
+      "s_load_dword %3, %8, 0x0\n\ts_load_dwordx2 %4, %9, 0x0\n\ts_waitcnt lgkmcnt(0)"
+      : "=&s"(v[0]), "=&s"(v[1]), "=&s"(v[2]), "=&s"(v[3]), "=&s"(w)
+      : "s"(p0), "s"(p1), "s"(p2), "s"(p3), "s"(p4)
       : "memory");
 }
 
@@ -364,7 +364,7 @@ __global__ __launch_bounds__(8 * kWave) void attn_step_kernel(AttnParams p) {
   NV_AT_LD32(rb, rbp, 0);
 
   // ---- 2. position, this split's blocks, this wave's tiles (scalar path)
-  uint32_t pos, nblk, bps, active, first, nt, phys[4], launch_seq = p.launch_seq;
+  uint32_t pos, nblk, bps, active, first, nt, phys[4], launch_seq;
   if (p.plan != nullptr) {
     // this step's plan: everything above in one round trip
     u32x8_t head, mine;
@@ -380,9 +380,11 @@ __global__ __launch_bounds__(8 * kWave) void attn_step_kernel(AttnParams p) {
     first = split * bps + wave;
     const uint32_t end = min(nblk, split * bps + bps);
     nt = first < end ? (end - first + W - 1) / W : 0u;  // tiles first, first + W, ...
+    uint64_t launches = 0;
     if (split < active)
       sload4(p.table + min(first, nblk - 1), p.table + min(first + W, nblk - 1), p.table + min(first + 2 * W, nblk - 1),
-             p.table + min(first + 3 * W, nblk - 1), phys);
+             p.table + min(first + 3 * W, nblk - 1), p.launches + kvh * kAttnLaunchStride, phys, launches);
+    launch_seq = static_cast<uint32_t>(launches / kAttnLaunchQuantum);
   }
   if (split >= active) return;  // idle splits neither store a partial nor take a ticket
   const uint32_t n_keys = pos + 1;
@@ -459,6 +461,11 @@ __global__ __launch_bounds__(8 * kWave) void attn_step_kernel(AttnParams p) {
   link_mark(tr, 15);
   __syncthreads();
   link_mark(tr, 9);
+  // this workgroup's share of the launch's quantum - the first split has what the others leave of it -, now that all its
+  // waves have had their look; nobody waits for it
+  if (p.plan == nullptr && active > 1 && threadIdx.x == kThreads - kWave)
+    __hip_atomic_fetch_add(p.launches + kvh * kAttnLaunchStride, split == 0 ? kAttnLaunchQuantum - (active - 1u) : uint64_t{1}, __ATOMIC_RELAXED,
+                           __HIP_MEMORY_SCOPE_AGENT);
   if (owns_new && wave == W - 1) {
     // publish the rounded row to the cache in operand order
     const uint64_t tile = kv_tile_offset(p.block_count, p.kv_heads, HD, p.layer, scalar_load(p.table + new_block), kvh);
@@ -779,11 +786,13 @@ hipError_t launch_dt(const AttnParams &p, hipStream_t stream) {
   const uint32_t group = p.heads / p.kv_heads;
   const bool block = p.tokens > 1 || p.seqs != nullptr;
   bool fast = attn_matrix_cores(p.heads, p.kv_heads, p.head_dim) && p.part_acc != nullptr && p.splits >= 1;
-  // The matrix-core kernels read the caches in pieces of 16 bytes and exchange words of 8. Shapes that came to them from the
-  // general kernel, which reads elements, go back to it where the caller's addresses are not made for that.
+  // The matrix-core kernels read the caches in pieces of 16 bytes, the step kernel exchanges and counts in words of 8. Calls
+  // whose workspace is not made for that go to the general kernel, which reads elements, and at the shapes that came from
+  // there those whose caches are not.
   const auto at_multiple = [](const void *ptr, uintptr_t of) { return reinterpret_cast<uintptr_t>(ptr) % of == 0; };
-  if (fast && !block && attn_f32_shape(p.head_dim, group) &&
-      !(at_multiple(p.k_cache, 16) && at_multiple(p.v_cache, 16) && at_multiple(p.part_tagged, 8)))
+  if (fast && !block &&
+      (!at_multiple(p.part_tagged, 8) ||
+       (attn_f32_shape(p.head_dim, group) && !(at_multiple(p.k_cache, 16) && at_multiple(p.v_cache, 16)))))
     fast = false;
   // every active split of a kv head has to be resident while the merges poll: a larger split factor is refused at the
   // shapes the split factor is declared for, and left to the general kernel, which has no splits, at the others
@@ -792,7 +801,7 @@ hipError_t launch_dt(const AttnParams &p, hipStream_t stream) {
     fast = false;
   }
   if (fast) {
-    if (!block && p.part_tagged == nullptr) return hipErrorInvalidValue;
+    if (!block && (p.part_tagged == nullptr || (p.plan == nullptr && p.launches == nullptr))) return hipErrorInvalidValue;
     return p.head_dim == 64 ? launch_fast_hd<DT, 64>(p, stream) : launch_fast_hd<DT, 128>(p, stream);
   }
   if (p.head_dim > 512) return hipErrorInvalidValue;

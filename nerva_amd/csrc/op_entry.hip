@@ -444,7 +444,6 @@ uint64_t paged_attention_fault_offset(uint32_t heads, uint32_t head_dim) {
   return attn_workspace_bytes(heads, head_dim) + ((static_cast<uint64_t>(head_dim) * sizeof(float) + 255u) & ~uint64_t{255}) +
          attn_step_workspace_bytes(heads);
 }
-std::atomic<uint32_t> g_attention_calls{0};   // the launch sequence number that tags a call's split partials
 }  // namespace
 
 uint64_t nerva_hip_paged_attention_workspace_bytes(uint32_t heads, uint32_t head_dim) {
@@ -536,7 +535,7 @@ int nerva_hip_paged_gqa_decode(const NervaHipPagedAttentionRequest *r, void *str
   p.position = r->position;
   p.max_steps = 0;
   p.append = r->append;
-  p.launch_seq = g_attention_calls.fetch_add(1, std::memory_order_relaxed) + 1u;
+  p.launches = static_cast<uint64_t *>(r->workspace);   // (in front of split partials that one token's launches do not use)
   p.fault = reinterpret_cast<uint32_t *>(static_cast<char *>(r->workspace) + paged_attention_fault_offset(r->heads, r->head_dim));
   p.merge_spin_limit = static_cast<uint32_t>(std::max(tuning(kTuneAttnMergeSpinLimit), 0));
   p.withhold_split = static_cast<uint32_t>(std::max(tuning(kTuneAttnWithholdSplit), 0));

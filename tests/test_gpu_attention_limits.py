@@ -240,3 +240,55 @@ def test_caches_and_workspaces_at_any_address_of_their_elements(heads, kv_heads,
         N.paged_attention(dtype, heads, kv_heads, hd, shifted, c["layer"], tokens, dev(c["qkv"]), room.ptr + ws_shift, out16,
                           out_f32=out32, append=True, rope_theta=1e4)
         assert rel_l2(out32.numpy(np.float32), ref) <= REL_L2, (tokens, shift, ws_shift)
+
+
+def test_a_workspace_at_an_odd_word_at_the_shapes_of_the_step_kernel():
+    c = _attention_case(BF16, 32, 8, 128, 1000, 1e4, False, 5)
+    ref, _, _ = _attention_oracle(c)
+    cache = N.PagedKvCache(c["layers"], c["n_blocks"], 8, 128, c["table"])
+    cache.fill(c["layer"], c["k_rows"], c["v_rows"])
+    room = N.DeviceBuffer.zeros(N.abi.load().nerva_hip_paged_attention_workspace_bytes(32, 128) + 16)
+    out16, out32 = N.DeviceBuffer(32 * 128 * 2), N.DeviceBuffer(32 * 128 * 4)
+    N.paged_attention(BF16, 32, 8, 128, cache, c["layer"], 1000, dev(c["qkv"]), room.ptr + 4, out16, out_f32=out32, append=True, rope_theta=1e4)
+    assert rel_l2(out32.numpy(np.float32), ref) <= REL_L2
+
+
+@pytest.mark.parametrize("heads,kv_heads,hd", [(28, 4, 128), (14, 2, 64), (32, 8, 128)])
+def test_a_captured_call_replayed_on_other_inputs(heads, kv_heads, hd):
+    """One call on its workspace in a graph, replayed with new projections (and so a new key and value) each time, with eager
+    calls on the same workspace and synchronizations between: no partial of the replay before is taken for this one's."""
+    import ctypes as C
+    c = _attention_case(BF16, heads, kv_heads, hd, 1500, 1e4, False, heads)
+    cache = N.PagedKvCache(c["layers"], c["n_blocks"], kv_heads, hd, c["table"])
+    cache.fill(c["layer"], c["k_rows"], c["v_rows"])
+    qkv, ws = dev(c["qkv"]), attention_workspace(heads, hd)
+    out16, out32 = N.DeviceBuffer(heads * hd * 2), N.DeviceBuffer(heads * hd * 4)
+    req = N.abi.NervaHipPagedAttentionRequest()
+    req.dtype, req.heads, req.kv_heads, req.head_dim = BF16, heads, kv_heads, hd
+    req.layer, req.block_count, req.position, req.append = c["layer"], c["n_blocks"], 1500, 1
+    req.rms_eps, req.rope_theta = 1e-6, 1e4
+    req.qkv_f32, req.k_cache, req.v_cache, req.block_table = qkv.ptr, cache.k.ptr, cache.v.ptr, cache.table.ptr
+    req.workspace, req.output_f32, req.output16 = ws.ptr, out32.ptr, out16.ptr
+    lib = N.abi.load()
+    call, err = lib.nerva_hip_paged_gqa_decode, C.c_int32(0)
+    assert call(C.byref(req), None, C.byref(err)) == 0     # (the rotation table is made by a first call)
+    N.Device.synchronize()
+    hip = C.CDLL(lib._name)                                # (the runtime that the library is linked with)
+    stream, graph, replayable = C.c_void_p(), C.c_void_p(), C.c_void_p()
+    assert hip.hipStreamCreateWithFlags(C.byref(stream), 1) == 0
+    assert hip.hipStreamBeginCapture(stream, 1) == 0
+    captured = call(C.byref(req), stream, C.byref(err))
+    assert hip.hipStreamEndCapture(stream, C.byref(graph)) == 0 and captured == 0
+    assert hip.hipGraphInstantiate(C.byref(replayable), graph, None, None, C.c_size_t(0)) == 0
+    rng = np.random.default_rng(heads)
+    for replay in range(12):
+        c["qkv"] = (rng.normal(0, 1, c["qkv"].size) * (1 + replay)).astype(np.float32)
+        ref, _, _ = _attention_oracle(c)
+        qkv.upload(c["qkv"])
+        if replay % 4 == 3:
+            assert call(C.byref(req), None, C.byref(err)) == 0
+            N.Device.synchronize()
+        assert hip.hipGraphLaunch(replayable, stream) == 0 and hip.hipStreamSynchronize(stream) == 0
+        assert rel_l2(out32.numpy(np.float32), ref) <= REL_L2, replay
+    assert N.paged_attention_status(ws, heads, hd) == (0, 0)
+    assert hip.hipGraphExecDestroy(replayable) == 0 and hip.hipGraphDestroy(graph) == 0 and hip.hipStreamDestroy(stream) == 0
