@@ -224,6 +224,6 @@ hipError_t launch_kv_publish_rows(uint32_t dtype, const AttnParams &p, hipStream
 hipError_t launch_attn_prompt(uint32_t dtype, const AttnParams &p, hipStream_t stream);
 // Tokens a launch should take of a pass of `tokens` from `position` on: a block (of at most `block` tokens, which is what the
 // splits' workspace is for), or all of them, without splits.
-uint32_t attn_prompt_launch_tokens(uint32_t heads, uint32_t kv_heads, uint32_t position, uint32_t tokens, uint32_t block);
+uint32_t attn_prompt_launch_tokens(uint32_t heads, uint32_t kv_heads, uint32_t head_dim, uint32_t position, uint32_t tokens, uint32_t block);
 
 }  // namespace nv

@@ -8,7 +8,7 @@
 // gfx950 mapping (head_dim 64 or 128, G = heads / kv_heads up to 8): a wave fills two 16-column matrix-core tiles with
 // (token, head) pairs - 32 / G tokens of the kv head's G query heads - and the hi and lo halves of a query (and of a
 // step's probabilities) are two products into the same accumulators, with the causal limit n_keys chosen per column.
-// The 8 waves of a workgroup take 8 * 32 / G consecutive tokens and walk the SAME keys, 64 a step: the step's four K and
+// The 8 waves of a (wide) workgroup take 8 * 32 / G consecutive tokens and walk the SAME keys, 64 a step: the step's four K and
 // four V tiles (one each per wave) go from the cache straight into a ring of four LDS stages, two steps ahead.
 // What bounds it is the matrix cores and the exponentials beside them, so a step is laid out for both: 64 keys share one
 // running maximum, one rescale and one look at the mask (only steps that reach the diagonal have one), every K or V piece
@@ -19,6 +19,11 @@
 // and the 16-deep product, blocks of 512 tokens of 32 heads over contexts 512 to 8192: 111.8 -> 82.7 us a launch on
 // average (85.8 without the turns), 0.94 PFLOP/s with the hi and lo halves counted, where the products of the same block
 // reach 1.1.
+// Prompts of less than some 3000 tokens do not fill the chip with such workgroups, and each of them is long: queries of 256
+// pairs prepared by four SIMDs (half of a short launch), then 3.3 to 4 us a step. The narrow workgroup has four waves of one
+// column tile: a quarter of the work for each SIMD, two workgroups a CU with two LDS stages each, and no
+// turns - the other workgroup's wave fills in. The same sums in the same order (32 heads on 8, 146 tokens 20.8 -> 11.4 us, 512 tokens in four splits 38 ->
+// 18.7 in one, 1024 tokens 64.7 -> 34.2; prompt_shape has the line between the two).
 // Grid (kv head, split of the prefix, token group, the last one first); split partials go to the per-token workspaces the decode kernel uses
 // and a small second launch merges them.
 #include <algorithm>
@@ -33,10 +38,14 @@ namespace {
 
 using namespace attn;
 
-constexpr int kPW = 8;                // waves per workgroup
-constexpr int kCols = 32;             // (token, head) pairs per wave: two column tiles
+// A workgroup's waves and the 16-column tiles of (token, head) pairs each of them has.
+constexpr int kWideWaves = 8, kWideTiles = 2;
+constexpr int kNarrowWaves = 4, kNarrowTiles = 1;
 constexpr uint32_t kStepBlocks = 4;   // cache blocks (16 keys) of a step
-constexpr int kStages = 4;
+constexpr int stages_of(int waves) { return waves == kWideWaves ? 4 : 2; }
+constexpr uint32_t group_tokens_of(bool wide, uint32_t group) {
+  return wide ? kWideWaves * (kWideTiles * 16u / group) : kNarrowWaves * (kNarrowTiles * 16u / group);
+}
 
 // Split geometry of a token group, the same on both launches: blocks per split (whole steps), active splits.
 __device__ __forceinline__ void prompt_splits(uint32_t last_pos, uint32_t S, uint32_t &bps, uint32_t &active, uint32_t &nblk) {
@@ -58,10 +67,12 @@ constexpr uint32_t prompt_stage_bytes(int hd) { return 2u * kStepBlocks * prompt
 template <uint32_t DT>
 __device__ __forceinline__ bool finite16(uint16_t bits) { return (bits & 0x7fffu) < (DT == kBF16 ? 0x7f80u : 0x7c00u); }
 
-template <uint32_t DT, int HD, int G>
-__global__ __launch_bounds__(kPW *kWave, 2) void attn_prompt_kernel(AttnParams p) {
-  constexpr int kTokensPerWave = kCols / G, kPairs = kTokensPerWave * G;   // (columns kPairs .. 31 repeat the last pair, unused)
-  constexpr uint32_t kGroupTokens = kPW * kTokensPerWave;
+template <uint32_t DT, int HD, int G, int PW, int NC>
+__global__ __launch_bounds__(PW *kWave, 2) void attn_prompt_kernel(AttnParams p) {
+  constexpr int kCols = 16 * NC, kStages = stages_of(PW);
+  constexpr int kTokensPerWave = kCols / G, kPairs = kTokensPerWave * G;   // (columns kPairs .. kCols - 1 repeat the last pair, unused)
+  constexpr uint32_t kGroupTokens = PW * kTokensPerWave;
+  constexpr int kWaveTiles = 2 * kStepBlocks / PW;   // K/V tiles of a step that a wave fetches
   constexpr int kPieces = HD / 32;               // 1 KiB pieces of a tile
   constexpr uint32_t kTile = prompt_tile_bytes(HD), kStage = prompt_stage_bytes(HD);
   extern __shared__ __align__(16) unsigned char smem[];
@@ -75,15 +86,20 @@ __global__ __launch_bounds__(kPW *kWave, 2) void attn_prompt_kernel(AttnParams p
   if (split >= active) return;
   const uint32_t b0 = split * bps, steps = (min(nblk, b0 + bps) - b0 + kStepBlocks - 1) / kStepBlocks;
 
-  // this wave's tile of a step: K (even waves) or V of block wave / 2; blocks past the last are that one again, masked
+  // this wave's tiles of a step, wave, wave + PW, ...: K (even ones) or V of block tile / 2; blocks past the last are that one
+  // again, masked
   const uint16_t *cache = (wave & 1) == 0 ? p.k_cache : p.v_cache;
   auto request = [&](uint32_t step) {
-    const uint32_t block = min(b0 + step * kStepBlocks + (wave >> 1), nblk - 1);
-    const uint16_t *src = cache + kv_tile_offset(p.block_count, p.kv_heads, HD, p.layer, scalar_load(p.table + block), kvh) + lane * 8;
-    unsigned char *at = smem + (step % kStages) * kStage + wave * kTile;
 #pragma unroll
-    for (int i = 0; i < kPieces; ++i)
-      __builtin_amdgcn_global_load_lds(reinterpret_cast<const u32x4_t *>(src + i * 512), NV_PR_LDS(at + i * 1024), 16, 0, 0);
+    for (int n = 0; n < kWaveTiles; ++n) {
+      const uint32_t tile = wave + n * PW;
+      const uint32_t block = min(b0 + step * kStepBlocks + (tile >> 1), nblk - 1);
+      const uint16_t *src = cache + kv_tile_offset(p.block_count, p.kv_heads, HD, p.layer, scalar_load(p.table + block), kvh) + lane * 8;
+      unsigned char *at = smem + (step % kStages) * kStage + tile * kTile;
+#pragma unroll
+      for (int i = 0; i < kPieces; ++i)
+        __builtin_amdgcn_global_load_lds(reinterpret_cast<const u32x4_t *>(src + i * 512), NV_PR_LDS(at + i * 1024), 16, 0, 0);
+    }
   };
 
   // ---- this wave's (token, head) pairs: bias, norm, rotation -> hi and lo operands. A lane fetches what it will hold of
@@ -91,10 +107,10 @@ __global__ __launch_bounds__(kPW *kWave, 2) void attn_prompt_kernel(AttnParams p
   // exchanges, and every input of the wave's pairs is requested at once.
   const uint32_t wave_first = group_first + wave * kTokensPerWave;   // may lie past the block: clamped, never stored
   const int col = lane & 15, grp = lane >> 4;
-  u32x4_t qhi[2][kPieces], qlo[2][kPieces];
-  uint32_t n_keys[2];
+  u32x4_t qhi[NC][kPieces], qlo[NC][kPieces];
+  uint32_t n_keys[NC];
   constexpr bool kScaled = attn_scaled<DT, HD, G>();
-  float down[2] = {1.0f, 1.0f};   // undoes the scale of the column's query
+  float down[NC];   // undoes the scale of the column's query
   {
     constexpr int kHalf = kPieces / 2;   // pieces of a rotation's first ends
     const bool has_bias = p.q_bias != nullptr, has_gamma = p.q_norm != nullptr, has_rope = p.rope_freq != nullptr;
@@ -102,10 +118,10 @@ __global__ __launch_bounds__(kPW *kWave, 2) void attn_prompt_kernel(AttnParams p
     const float *rope_base = has_rope ? p.rope_cs : p.qkv;
     const uint32_t rope_stride = has_rope ? p.rope_token_stride : 0u;
     const uint16_t *gamma_base = has_gamma ? p.q_norm : p.k_cache;
-    f32x4_t x[2][kPieces][2], rc[2][kHalf][2], rs[2][kHalf][2];
-    u32x4_t bias[2][kPieces], gamma[kPieces];
+    f32x4_t x[NC][kPieces][2], rc[NC][kHalf][2], rs[NC][kHalf][2];
+    u32x4_t bias[NC][kPieces], gamma[kPieces];
 #pragma unroll
-    for (int c = 0; c < 2; ++c) {
+    for (int c = 0; c < NC; ++c) {
       const int vh = min(c * 16 + col, kPairs - 1);
       const uint32_t tok = min(wave_first + vh / G, T - 1);
       const uint32_t h = kvh * G + vh % G;
@@ -135,7 +151,7 @@ __global__ __launch_bounds__(kPW *kWave, 2) void attn_prompt_kernel(AttnParams p
     const auto elem16 = [](const u32x4_t &v, int e) { return dec16<DT>(static_cast<uint16_t>(v[e / 2] >> (16 * (e % 2)))); };
     const float scale = kLog2e / sqrtf(static_cast<float>(HD));
 #pragma unroll
-    for (int c = 0; c < 2; ++c) {
+    for (int c = 0; c < NC; ++c) {
       float y[kPieces][8], ss = 0.0f;
 #pragma unroll
       for (int j = 0; j < kPieces; ++j)
@@ -165,6 +181,7 @@ __global__ __launch_bounds__(kPW *kWave, 2) void attn_prompt_kernel(AttnParams p
           }
       }
       float up = scale;
+      down[c] = 1.0f;
       if constexpr (kScaled) {
         float largest = 0.0f;
 #pragma unroll
@@ -193,10 +210,10 @@ __global__ __launch_bounds__(kPW *kWave, 2) void attn_prompt_kernel(AttnParams p
   const uint32_t least_keys = p.position + min(wave_first, T - 1) + 1;                            // of any column of the wave,
   const uint32_t most_keys = p.position + min(wave_first + kTokensPerWave - 1, T - 1) + 1;        // and the most of any
 
-  float m[2], l[2];
-  f32x4_t acc[2][HD / 16];   // O^T[dims s*16 + grp*4 .. +3][column]
+  float m[NC], l[NC];
+  f32x4_t acc[NC][HD / 16];   // O^T[dims s*16 + grp*4 .. +3][column]
 #pragma unroll
-  for (int c = 0; c < 2; ++c) {
+  for (int c = 0; c < NC; ++c) {
     m[c] = -INFINITY;
     l[c] = 0.0f;
 #pragma unroll
@@ -205,7 +222,7 @@ __global__ __launch_bounds__(kPW *kWave, 2) void attn_prompt_kernel(AttnParams p
   const uint32_t lds0 = static_cast<uint32_t>(reinterpret_cast<uintptr_t>(NV_PR_LDS(smem))) + lane * 16u;
 
   // ---- the three parts of a step (skipped where no column of the wave sees it)
-  f32x4_t sc[2][kStepBlocks];   // scores of keys key0 + 16 t + 4 grp + r, then the bits of their probabilities: two words hi, two lo
+  f32x4_t sc[NC][kStepBlocks];   // scores of keys key0 + 16 t + 4 grp + r, then the bits of their probabilities: two words hi, two lo
   auto sees = [&](uint32_t step) { return wave_on && (b0 + step * kStepBlocks) * kKvBlockTokens < most_keys; };
   auto scores = [&](uint32_t step) {
     if (!sees(step)) return;
@@ -226,15 +243,15 @@ __global__ __launch_bounds__(kPW *kWave, 2) void attn_prompt_kernel(AttnParams p
       }
       __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-      for (int c = 0; c < 2; ++c) sc[c][t] = f32x4_t{0.0f, 0.0f, 0.0f, 0.0f};
+      for (int c = 0; c < NC; ++c) sc[c][t] = f32x4_t{0.0f, 0.0f, 0.0f, 0.0f};
 #pragma unroll
       for (int j = 0; j < kPieces; ++j)
 #pragma unroll
-        for (int c = 0; c < 2; ++c) sc[c][t] = mfma_k32<DT>(k[t & 1][j], qhi[c][j], sc[c][t]);
+        for (int c = 0; c < NC; ++c) sc[c][t] = mfma_k32<DT>(k[t & 1][j], qhi[c][j], sc[c][t]);
 #pragma unroll
       for (int j = 0; j < kPieces; ++j)
 #pragma unroll
-        for (int c = 0; c < 2; ++c) sc[c][t] = mfma_k32<DT>(k[t & 1][j], qlo[c][j], sc[c][t]);
+        for (int c = 0; c < NC; ++c) sc[c][t] = mfma_k32<DT>(k[t & 1][j], qlo[c][j], sc[c][t]);
       __builtin_amdgcn_sched_barrier(0);
     }
   };
@@ -243,14 +260,14 @@ __global__ __launch_bounds__(kPW *kWave, 2) void attn_prompt_kernel(AttnParams p
     const uint32_t key0 = (b0 + step * kStepBlocks) * kKvBlockTokens;
     if (key0 + kStepBlocks * kKvBlockTokens > least_keys) {   // some column ends inside this step (or before it)
 #pragma unroll
-      for (int c = 0; c < 2; ++c)
+      for (int c = 0; c < NC; ++c)
 #pragma unroll
         for (uint32_t t = 0; t < kStepBlocks; ++t)
 #pragma unroll
           for (uint32_t r = 0; r < 4; ++r) sc[c][t][r] = key0 + t * 16u + grp * 4u + r < n_keys[c] ? sc[c][t][r] : -INFINITY;
     }
 #pragma unroll
-    for (int c = 0; c < 2; ++c) {
+    for (int c = 0; c < NC; ++c) {
       float mb = fmaxf(fmaxf(sc[c][0][0], sc[c][0][1]), fmaxf(sc[c][0][2], sc[c][0][3]));
 #pragma unroll
       for (uint32_t t = 1; t < kStepBlocks; ++t) mb = fmaxf(fmaxf(mb, fmaxf(sc[c][t][0], sc[c][t][1])), fmaxf(sc[c][t][2], sc[c][t][3]));
@@ -307,14 +324,14 @@ __global__ __launch_bounds__(kPW *kWave, 2) void attn_prompt_kernel(AttnParams p
       const u32x4_t &a = v[g & 1][0], &b = v[g & 1][1];
       const u32x4_t lo_slab = {a[0], a[1], b[0], b[1]}, hi_slab = {a[2], a[3], b[2], b[3]};
 #pragma unroll
-      for (int c = 0; c < 2; ++c) {
+      for (int c = 0; c < NC; ++c) {
         const u32x4_t pa = __builtin_bit_cast(u32x4_t, sc[c][2 * pair]), pb = __builtin_bit_cast(u32x4_t, sc[c][2 * pair + 1]);
         const u32x4_t bh = {pa[0], pa[1], pb[0], pb[1]};
         acc[c][2 * j] = mfma_k32<DT>(lo_slab, bh, acc[c][2 * j]);
         acc[c][2 * j + 1] = mfma_k32<DT>(hi_slab, bh, acc[c][2 * j + 1]);
       }
 #pragma unroll
-      for (int c = 0; c < 2; ++c) {
+      for (int c = 0; c < NC; ++c) {
         const u32x4_t pa = __builtin_bit_cast(u32x4_t, sc[c][2 * pair]), pb = __builtin_bit_cast(u32x4_t, sc[c][2 * pair + 1]);
         const u32x4_t bl = {pa[2], pa[3], pb[2], pb[3]};
         acc[c][2 * j] = mfma_k32<DT>(lo_slab, bl, acc[c][2 * j]);
@@ -328,7 +345,19 @@ __global__ __launch_bounds__(kPW *kWave, 2) void attn_prompt_kernel(AttnParams p
   // the other way round. Phase 2k: first half V(k-1) and K(k), second half softmax(k-1); phase 2k+1: first half
   // softmax(k), second half V(k-1) and K(k). A stage is free when the second half has left V of its step, two phases
   // before it is filled again.
-  const bool first_half = wave < kPW / 2;
+  // With one wave a SIMD nobody takes turns: a step's three parts follow one another, behind one barrier - which also says
+  // that the stage of the step before is free.
+  const bool first_half = wave < PW / 2;
+  if constexpr (PW != kWideWaves) {
+    for (uint32_t k = 0; k < steps; ++k) {
+      if (k == 0 && steps > 1) asm volatile("s_waitcnt vmcnt(%0)\n\ts_barrier" ::"n"(kPieces * kWaveTiles) : "memory");
+      else asm volatile("s_waitcnt vmcnt(0)\n\ts_barrier" ::: "memory");
+      if (k > 0 && k + 1 < steps) request(k + 1);
+      scores(k);
+      softmax(k);
+      values(k);
+    }
+  } else
   for (uint32_t k = 0; k <= steps; ++k) {
     // this wave's part of step k has arrived (step k + 1 may be on its way)
     if (k + 1 < steps) asm volatile("s_waitcnt vmcnt(%0)\n\ts_barrier" ::"n"(kPieces) : "memory");
@@ -350,9 +379,9 @@ __global__ __launch_bounds__(kPW *kWave, 2) void attn_prompt_kernel(AttnParams p
   // ---- results of the wave's pairs: token rows of the four lane groups
   const uint64_t ml_off = reinterpret_cast<char *>(p.part_m) - reinterpret_cast<char *>(p.part_acc);
   const uint64_t l_off = reinterpret_cast<char *>(p.part_l) - reinterpret_cast<char *>(p.part_acc);
-  uint32_t spoilt[2];   // columns with a sum that is not finite
+  uint32_t spoilt[NC];   // columns with a sum that is not finite
 #pragma unroll
-  for (int c = 0; c < 2; ++c) {
+  for (int c = 0; c < NC; ++c) {
     float zero = 0.0f;
 #pragma unroll
     for (int s2 = 0; s2 < HD / 16; ++s2)
@@ -361,7 +390,8 @@ __global__ __launch_bounds__(kPW *kWave, 2) void attn_prompt_kernel(AttnParams p
     const uint64_t lanes = __ballot(zero != 0.0f);   // (NaN)
     spoilt[c] = static_cast<uint32_t>(lanes | (lanes >> 16) | (lanes >> 32) | (lanes >> 48)) & 0xffffu;
   }
-  if ((spoilt[0] | spoilt[1]) != 0) {
+  const auto any_spoilt = [&] { return (spoilt[0] | spoilt[NC - 1]) != 0; };
+  if (any_spoilt()) {
     // 0 x NaN or infinity is NaN: a value that is not finite may have come in by a key that the column does not see - of a
     // later token of its step, or a row not written yet. Where there is such a value behind the least limit of the wave's
     // columns, their sums are formed once more below, over the keys they see.
@@ -371,10 +401,10 @@ __global__ __launch_bounds__(kPW *kWave, 2) void attn_prompt_kernel(AttnParams p
 #pragma unroll
       for (int i = 0; i < kPieces * 8; ++i) found |= finite16<DT>(tile[i / 8 * 512 + i % 8]) ? 0u : 1u;
     }
-    if (!__any(found != 0)) spoilt[0] = spoilt[1] = 0;
+    if (!__any(found != 0)) spoilt[0] = spoilt[NC - 1] = 0;
   }
 #pragma unroll
-  for (int c = 0; c < 2; ++c) {
+  for (int c = 0; c < NC; ++c) {
     float lc = l[c];
     lc += __shfl_xor(lc, 16, kWave);
     lc += __shfl_xor(lc, 32, kWave);
@@ -407,10 +437,10 @@ __global__ __launch_bounds__(kPW *kWave, 2) void attn_prompt_kernel(AttnParams p
   }
   // ---- the sums of spoilt columns, one after the other: the query again (a lane has a rotation's two ends), scores of 64
   // keys at a time (a lane a key), then their values in key order (a lane its two dims)
-  if (__builtin_expect((spoilt[0] | spoilt[1]) == 0, 1)) return;
+  if (__builtin_expect(!any_spoilt(), 1)) return;
   for (int pair = 0; pair < kPairs; ++pair) {
     const uint32_t tok = wave_first + pair / G, h = kvh * G + pair % G;
-    if (((spoilt[pair / 16] >> (pair % 16)) & 1u) == 0 || tok >= T) continue;
+    if ((((pair < 16 ? spoilt[0] : spoilt[NC - 1]) >> (pair % 16)) & 1u) == 0 || tok >= T) continue;
     const int at = pair_of<HD>(lane);
     const float *src = p.qkv + static_cast<uint64_t>(tok) * p.qkv_token_stride + h * HD;
     const float *rope = p.rope_freq != nullptr ? p.rope_cs + static_cast<uint64_t>(tok) * p.rope_token_stride : p.qkv;
@@ -422,7 +452,7 @@ __global__ __launch_bounds__(kPW *kWave, 2) void attn_prompt_kernel(AttnParams p
     const float scale = kLog2e / sqrtf(static_cast<float>(HD));
     q0 *= scale;
     q1 *= scale;
-    const float most = __shfl(pair < 16 ? m[0] : m[1], pair % 16, kWave), sum = __shfl(pair < 16 ? l[0] : l[1], pair % 16, kWave);
+    const float most = __shfl(pair < 16 ? m[0] : m[NC - 1], pair % 16, kWave), sum = __shfl(pair < 16 ? l[0] : l[NC - 1], pair % 16, kWave);
     const uint32_t end = min((b0 + steps * kStepBlocks) * kKvBlockTokens, p.position + tok + 1);
     float o0 = 0.0f, o1 = 0.0f;
     for (uint32_t k0 = b0 * kKvBlockTokens; k0 < end; k0 += kWave) {
@@ -508,36 +538,40 @@ __global__ __launch_bounds__(HD) void attn_prompt_merge_kernel(AttnParams p, uin
   p.out16[attn_out_token(p, tok) + attn_out_elem(p, h * HD + d)] = enc16<DT>(o);
 }
 
-template <uint32_t DT, int HD, int G>
-hipError_t launch_group(const AttnParams &p, uint32_t splits, hipStream_t stream) {
-  constexpr size_t lds = static_cast<size_t>(kStages) * prompt_stage_bytes(HD);
+template <uint32_t DT, int HD, int G, int PW, int NC>
+hipError_t launch_shape(const AttnParams &p, uint32_t splits, hipStream_t stream) {
+  constexpr size_t lds = static_cast<size_t>(stages_of(PW)) * prompt_stage_bytes(HD);
   // more than the default dynamic LDS limit: raised once per kernel (never under stream capture)
   static std::once_flag once;
   static hipError_t raised = hipSuccess;
   std::call_once(once, [] {
-    raised = hipFuncSetAttribute(reinterpret_cast<const void *>(&attn_prompt_kernel<DT, HD, G>),
+    raised = hipFuncSetAttribute(reinterpret_cast<const void *>(&attn_prompt_kernel<DT, HD, G, PW, NC>),
                                  hipFuncAttributeMaxDynamicSharedMemorySize, static_cast<int>(lds));
   });
   if (raised != hipSuccess) return raised;
-  constexpr uint32_t group_tokens = kPW * (kCols / G);
-  hipLaunchKernelGGL((attn_prompt_kernel<DT, HD, G>), dim3(p.kv_heads, splits, (p.tokens + group_tokens - 1) / group_tokens),
-                     dim3(kPW * kWave), lds, stream, p);
+  constexpr uint32_t group_tokens = PW * (16 * NC / G);
+  hipLaunchKernelGGL((attn_prompt_kernel<DT, HD, G, PW, NC>), dim3(p.kv_heads, splits, (p.tokens + group_tokens - 1) / group_tokens),
+                     dim3(PW * kWave), lds, stream, p);
   return hipGetLastError();
+}
+template <uint32_t DT, int HD, int G>
+hipError_t launch_group(const AttnParams &p, bool wide, uint32_t splits, hipStream_t stream) {
+  return wide ? launch_shape<DT, HD, G, kWideWaves, kWideTiles>(p, splits, stream) : launch_shape<DT, HD, G, kNarrowWaves, kNarrowTiles>(p, splits, stream);
 }
 
 template <uint32_t DT, int HD>
-hipError_t launch_hd(const AttnParams &p, uint32_t splits, hipStream_t stream) {
-  const uint32_t group = p.heads / p.kv_heads, group_tokens = kPW * (kCols / group);
+hipError_t launch_hd(const AttnParams &p, bool wide, uint32_t splits, hipStream_t stream) {
+  const uint32_t group = p.heads / p.kv_heads, group_tokens = group_tokens_of(wide, group);
   hipError_t err = hipSuccess;
   switch (group) {
-    case 1: err = launch_group<DT, HD, 1>(p, splits, stream); break;
-    case 2: err = launch_group<DT, HD, 2>(p, splits, stream); break;
-    case 3: err = launch_group<DT, HD, 3>(p, splits, stream); break;
-    case 4: err = launch_group<DT, HD, 4>(p, splits, stream); break;
-    case 5: err = launch_group<DT, HD, 5>(p, splits, stream); break;
-    case 6: err = launch_group<DT, HD, 6>(p, splits, stream); break;
-    case 7: err = launch_group<DT, HD, 7>(p, splits, stream); break;
-    default: err = launch_group<DT, HD, 8>(p, splits, stream); break;
+    case 1: err = launch_group<DT, HD, 1>(p, wide, splits, stream); break;
+    case 2: err = launch_group<DT, HD, 2>(p, wide, splits, stream); break;
+    case 3: err = launch_group<DT, HD, 3>(p, wide, splits, stream); break;
+    case 4: err = launch_group<DT, HD, 4>(p, wide, splits, stream); break;
+    case 5: err = launch_group<DT, HD, 5>(p, wide, splits, stream); break;
+    case 6: err = launch_group<DT, HD, 6>(p, wide, splits, stream); break;
+    case 7: err = launch_group<DT, HD, 7>(p, wide, splits, stream); break;
+    default: err = launch_group<DT, HD, 8>(p, wide, splits, stream); break;
   }
   if (err != hipSuccess || splits == 1) return err;
   if (splits <= 4)
@@ -548,40 +582,66 @@ hipError_t launch_hd(const AttnParams &p, uint32_t splits, hipStream_t stream) {
 }
 
 template <uint32_t DT>
-hipError_t launch_dt(const AttnParams &p, uint32_t splits, hipStream_t stream) {
-  return p.head_dim == 64 ? launch_hd<DT, 64>(p, splits, stream) : launch_hd<DT, 128>(p, splits, stream);
+hipError_t launch_dt(const AttnParams &p, bool wide, uint32_t splits, hipStream_t stream) {
+  return p.head_dim == 64 ? launch_hd<DT, 64>(p, wide, splits, stream) : launch_hd<DT, 128>(p, wide, splits, stream);
 }
 
 }  // namespace
 
-// Several blocks in one launch need no splits and no merge once their workgroups fill the chip: with two workgroups a CU,
-// the longest prefixes first, a long one is followed by a short one. Both sides in steps of 64 keys a workgroup; a
-// launch and its merge count as three. (Eight blocks of 32 heads in two passes over 8192 positions: 16 launches in four
-// splits 2.50 ms with the merges 2.88, two without splits 2.10.)
-uint32_t attn_prompt_launch_tokens(uint32_t heads, uint32_t kv_heads, uint32_t position, uint32_t tokens, uint32_t block) {
-  const uint32_t group_tokens = kPW * (kCols / (heads / kv_heads)), groups = (tokens + group_tokens - 1) / group_tokens;
-  const auto steps = [&](uint32_t last) { return (position + std::min(last, tokens)) / 64u + 1u; };   // of a token group that ends there
-  if (tokens <= block || kv_heads * groups < 192u) return std::min(tokens, block);
-  const auto nth = [&](uint32_t i) { return steps((groups - i / kv_heads) * group_tokens); };   // i: place in launch order
-  uint64_t together = steps(tokens);
-  if (kv_heads * groups > 512u) {
-    uint64_t all = 0;
-    for (uint32_t g = 1; g <= groups; ++g) all += static_cast<uint64_t>(kv_heads) * steps(g * group_tokens);
-    together = std::max<uint64_t>(together, all / 256u + steps(group_tokens) / 2u);
-  } else if (kv_heads * groups > 256u) {
-    together = std::max<uint64_t>(together, nth(255) + nth(256));
+namespace {
+
+struct PromptShape {
+  bool wide;
+  uint32_t splits;
+  double us;   // of the launch and its merge
+};
+// A launch's time: its start (queries, first tiles), and the longest workgroup's steps or, past the workgroups the chip holds
+// at once (one wide one a CU, two narrow ones, the longest first), all of them and a share of the longest's. A merge costs a
+// launch, and the partial sums' way to memory and back. Fitted on heads of 128 (32 on 8, tokens x first position, us):
+//                  146 x 0   512 x 0   88 x 512   512 x 512   1024 x 0   2048 x 0   4096 x 0   4096 x 4096   8 x 4096
+//   wide             20.8      38.6       29.3        44.5       64.7        116        241          607        23.5
+//   narrow           11.4      18.7       19.2        31.3       34.2         89        267          723        13
+// (wide in four or more splits where that is better, as it was before there were narrow ones; 64-wide heads go the same way.)
+PromptShape shape_at(bool wide, uint32_t splits, uint32_t heads, uint32_t kv_heads, uint32_t head_dim, uint32_t position, uint32_t tokens) {
+  const uint32_t group_tokens = group_tokens_of(wide, heads / kv_heads), groups = (tokens + group_tokens - 1) / group_tokens;
+  constexpr uint32_t kKeys = kStepBlocks * kKvBlockTokens;
+  const double longest = ((position + tokens - 1) / kKeys + splits) / splits;
+  const double workgroups = static_cast<double>(kv_heads) * groups * splits;
+  const double all = static_cast<double>(kv_heads) * groups * ((position + std::min(tokens, (tokens + group_tokens) / 2)) / kKeys + 1.0);
+  const double path = wide ? 3.3 : workgroups <= 256 ? 1.45 : 1.7;
+  const double steps = std::max(path * longest, wide ? 3.0 * all / 256 + 0.3 * longest : 1.7 * all / 512 + 0.6 * longest);
+  const double merge = splits == 1 ? 0.0 : 3.0 + static_cast<double>(tokens) * heads * head_dim * splits * 4 / 1.4e6;
+  return PromptShape{wide, splits, (wide ? 12.0 : 7.0) + steps + merge};
+}
+// The best of both shapes and of splits 1, 2, 4, ... (splits != 0: that many).
+PromptShape prompt_shape(uint32_t heads, uint32_t kv_heads, uint32_t head_dim, uint32_t position, uint32_t tokens, uint32_t splits) {
+  const int forced = tuning(kTunePromptWaves);
+  const uint32_t most = std::min(kAttnMaxSplits, (position + tokens - 1) / (kStepBlocks * kKvBlockTokens) + 1);
+  PromptShape best{true, 1, 1e30};
+  for (const bool wide : {true, false}) {
+    if (forced == (wide ? kNarrowWaves : kWideWaves)) continue;
+    for (uint32_t s = splits != 0 ? std::min(splits, most) : 1u; s <= most; s *= 2) {
+      const PromptShape shape = shape_at(wide, s, heads, kv_heads, head_dim, position, tokens);
+      if (shape.us < best.us) best = shape;
+      if (splits != 0) break;
+    }
   }
-  uint64_t apart = 0;
-  for (uint32_t at = 0; at < tokens; at += block) {
-    const uint32_t last = std::min(at + block, tokens), wgs = kv_heads * ((last - at + group_tokens - 1) / group_tokens);
-    const uint32_t splits = (256u + wgs - 1) / wgs;
-    apart += 3u + static_cast<uint64_t>(steps(last)) * ((wgs * splits + 255u) / 256u) / splits;
-  }
-  return together < apart ? tokens : block;
+  return best;
+}
+
+}  // namespace
+
+// Several blocks in one launch have no splits: that, or a launch a block with as many as are best for it.
+uint32_t attn_prompt_launch_tokens(uint32_t heads, uint32_t kv_heads, uint32_t head_dim, uint32_t position, uint32_t tokens, uint32_t block) {
+  if (tokens <= block) return tokens;
+  const double together = prompt_shape(heads, kv_heads, head_dim, position, tokens, 1).us;
+  double apart = 0.0;
+  for (uint32_t at = 0; at < tokens && apart < together; at += block)
+    apart += prompt_shape(heads, kv_heads, head_dim, position + at, std::min(block, tokens - at), 0).us;
+  return together <= apart ? tokens : block;
 }
 
 hipError_t launch_attn_prompt(uint32_t dtype, const AttnParams &p, hipStream_t stream) {
-  const uint32_t group = p.kv_heads != 0 ? p.heads / p.kv_heads : 0;
   if (p.qkv == nullptr || p.k_cache == nullptr || p.v_cache == nullptr || p.table == nullptr || p.out16 == nullptr ||
       p.part_acc == nullptr || p.part_m == nullptr || p.part_l == nullptr)
     return hipErrorInvalidValue;
@@ -591,15 +651,9 @@ hipError_t launch_attn_prompt(uint32_t dtype, const AttnParams &p, hipStream_t s
     return hipErrorInvalidValue;
   if (p.rope_freq != nullptr && p.rope_cs == nullptr) return hipErrorInvalidValue;   // rotation tables per token row
   if (p.out_packed_tiles != 0 && p.out_packed_tiles * 16u < p.tokens) return hipErrorInvalidValue;
-  // enough splits of the prefix to give every CU a workgroup, at least two steps each
-  const uint32_t group_tokens = kPW * (kCols / group);
-  const uint32_t groups = (p.tokens + group_tokens - 1) / group_tokens;
-  const uint32_t nblk = (p.position + p.tokens - 1) / kKvBlockTokens + 1;
-  uint32_t splits = p.splits != 0 ? p.splits : (256u + p.kv_heads * groups - 1) / (p.kv_heads * groups);
-  splits = std::min(splits, std::max(1u, nblk / 8));
-  splits = std::max(1u, std::min<uint32_t>(splits, kAttnMaxSplits));
-  if (dtype == kBF16) return launch_dt<kBF16>(p, splits, stream);
-  if (dtype == kF16) return launch_dt<kF16>(p, splits, stream);
+  const PromptShape shape = prompt_shape(p.heads, p.kv_heads, p.head_dim, p.position, p.tokens, std::min<uint32_t>(p.splits, kAttnMaxSplits));
+  if (dtype == kBF16) return launch_dt<kBF16>(p, shape.wide, shape.splits, stream);
+  if (dtype == kF16) return launch_dt<kF16>(p, shape.wide, shape.splits, stream);
   return hipErrorInvalidValue;
 }
 

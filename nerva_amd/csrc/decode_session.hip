@@ -703,7 +703,7 @@ hipError_t prefill_blocks(Session *s, uint32_t begin, uint32_t count, uint32_t c
     err = hipGetLastError();
     const uint32_t attn_tokens = rows_attention || prompt_splits != 0
                                      ? s->prefill_block_tokens
-                                     : attn_prompt_launch_tokens(s->heads, s->kv_heads, first, T, s->prefill_block_tokens);
+                                     : attn_prompt_launch_tokens(s->heads, s->kv_heads, s->head_dim, first, T, s->prefill_block_tokens);
     // Where a projection's slice-adding launch can write the following RMSNorm too, it does (one launch less each)
     const bool o_norms = gemm_rows_fuses_norm(kGemmResidual, H, A, T, tiles, s->pgemm_ws_bytes);
     const bool down_norms = gemm_rows_fuses_norm(kGemmResidual, H, I, T, tiles, s->pgemm_ws_bytes);

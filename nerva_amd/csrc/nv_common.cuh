@@ -150,6 +150,7 @@ enum TuningKnob : int {
   kTuneAttnSplits = 0,       // split-KV factor of a session's decode attention (read at session create)
   kTuneBatchSplits,          // split factor of the batch step's attention
   kTunePromptSplits,         // split factor of the prompt-block attention
+  kTunePromptWaves,          // prompt-block attention: waves per workgroup (4 or 8) whatever the launch
   kTuneGemmRowTiles,         // multi-row GEMM: 1 or 2 row tiles per wave for every plain projection
   kTuneGemmKWaves,           // multi-row GEMM: 8 or 4 waves along K
   kTuneGemmBlockSlices,      // shared-X GEMM: K slices for every projection

@@ -28,7 +28,7 @@ std::once_flag g_stream_once;
 hipStream_t g_stream = nullptr;
 std::atomic<bool> g_stream_ready{false};
 std::atomic<int> g_tuning[kTuneKnobs];
-constexpr const char *kTuningNames[kTuneKnobs] = {"attn_splits",       "batch_splits",       "prompt_splits",
+constexpr const char *kTuningNames[kTuneKnobs] = {"attn_splits",       "batch_splits",       "prompt_splits", "prompt_waves",
                                                   "gemm_row_tiles",    "gemm_k_waves",       "gemm_block_slices",
                                                   "gemm_block_row_tiles", "gemm_block_min_tokens", "gemv_exact_start",
                                                   "moe_down_shared_first", "gemv_workgroup_waves",
