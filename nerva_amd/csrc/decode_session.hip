@@ -707,9 +707,12 @@ hipError_t prefill_blocks(Session *s, uint32_t begin, uint32_t count, uint32_t c
     // Where a projection's slice-adding launch can write the following RMSNorm too, it does (one launch less each)
     const bool o_norms = gemm_rows_fuses_norm(kGemmResidual, H, A, T, tiles, s->pgemm_ws_bytes);
     const bool down_norms = gemm_rows_fuses_norm(kGemmResidual, H, I, T, tiles, s->pgemm_ws_bytes);
+    // ... or the projection behind it reads the rows themselves
+    const bool qkv_norms = tiles != 0 && gemm_rows_norms_input(kGemmF32, A + 2 * KV, H, T, s->pgemm_ws_bytes);
+    const bool gu_norms = !o_norms && tiles != 0 && gemm_rows_norms_input(kGemmSwiglu, I, H, T, s->pgemm_ws_bytes);
     for (uint32_t l = 0; err == hipSuccess && l < s->layers; ++l) {
       const LayerDev &w = s->layer[l];
-      if (l == 0 || !down_norms) err = launch_rmsnorm_rows(s->dtype, s->px, w.rms_attn, s->eps, T, H, s->pxn16, st, tiles);
+      if ((l == 0 || !down_norms) && !qkv_norms) err = launch_rmsnorm_rows(s->dtype, s->px, w.rms_attn, s->eps, T, H, s->pxn16, st, tiles);
       GemmRowsParams g{};
       g.tokens = T;
       if (err == hipSuccess) {
@@ -721,6 +724,11 @@ hipError_t prefill_blocks(Session *s, uint32_t begin, uint32_t count, uint32_t c
         g.cols = H;
         g.workspace = s->pgemm_ws;
         g.workspace_bytes = s->pgemm_ws_bytes;
+        if (qkv_norms && (l == 0 || !down_norms)) {
+          g.norm_in = s->px;
+          g.norm_in_gamma = w.rms_attn;
+          g.norm_eps = s->eps;
+        }
         err = launch_gemm_rows(s->dtype, kGemmF32, g, st);
       }
       AttnParams a{};
@@ -783,7 +791,7 @@ hipError_t prefill_blocks(Session *s, uint32_t begin, uint32_t count, uint32_t c
         }
         err = launch_gemm_rows(s->dtype, kGemmResidual, g, st);
       }
-      if (err == hipSuccess && !o_norms) err = launch_rmsnorm_rows(s->dtype, s->pr, w.rms_mlp, s->eps, T, H, s->pxn16, st, tiles);
+      if (err == hipSuccess && !o_norms && !gu_norms) err = launch_rmsnorm_rows(s->dtype, s->pr, w.rms_mlp, s->eps, T, H, s->pxn16, st, tiles);
       if (err == hipSuccess) {
         g = GemmRowsParams{};
         g.tokens = T;
@@ -797,6 +805,11 @@ hipError_t prefill_blocks(Session *s, uint32_t begin, uint32_t count, uint32_t c
         g.cols = H;
         g.workspace = s->pgemm_ws;
         g.workspace_bytes = s->pgemm_ws_bytes;
+        if (gu_norms) {
+          g.norm_in = s->pr;
+          g.norm_in_gamma = w.rms_mlp;
+          g.norm_eps = s->eps;
+        }
         err = launch_gemm_rows(s->dtype, kGemmSwiglu, g, st);
       }
       if (err == hipSuccess) {
@@ -1502,13 +1515,16 @@ hipError_t enqueue_batch_step(Session *lead, Session *const *seqs, uint32_t T,
   // follows as well (the next layer's attention norm, or the final norm): one launch less per layer
   const bool down_norms = gemm_rows_fuses_norm(kGemmResidual, H, I, T, tiles, lead->pgemm_ws_bytes);
   const bool o_norms = gemm_rows_fuses_norm(kGemmResidual, H, A, T, tiles, lead->pgemm_ws_bytes);   // likewise the MLP norm
+  // ... or the projection behind it reads the rows themselves
+  const bool qkv_norms = tiles != 0 && gemm_rows_norms_input(kGemmF32, A + 2 * KV, H, T, lead->pgemm_ws_bytes);
+  const bool gu_norms = !o_norms && tiles != 0 && gemm_rows_norms_input(kGemmSwiglu, I, H, T, lead->pgemm_ws_bytes);
   // where the q/k/v projection runs in a few K slices the attention adds them as it reads its inputs: no launch of
   // its own for that
   uint32_t qkv_slice_stride = 0;
   const uint32_t qkv_slices = gemm_rows_partial_slices(A + 2 * KV, H, T, tiles, lead->pgemm_ws_bytes, &qkv_slice_stride);
   for (uint32_t l = 0; err == hipSuccess && l < lead->layers; ++l) {
     const LayerDev &w = lead->layer[l];
-    if (l == 0 || !down_norms) err = launch_rmsnorm_rows(lead->dtype, lead->px, w.rms_attn, lead->eps, T, H, lead->pxn16, st, tiles);
+    if ((l == 0 || !down_norms) && !qkv_norms) err = launch_rmsnorm_rows(lead->dtype, lead->px, w.rms_attn, lead->eps, T, H, lead->pxn16, st, tiles);
     GemmRowsParams g{};
     if (err == hipSuccess) {
       g.tokens = T;
@@ -1521,6 +1537,11 @@ hipError_t enqueue_batch_step(Session *lead, Session *const *seqs, uint32_t T,
       g.workspace = lead->pgemm_ws;
       g.workspace_bytes = lead->pgemm_ws_bytes;
       g.keep_partials = qkv_slices != 0;
+      if (qkv_norms && (l == 0 || !down_norms)) {
+        g.norm_in = lead->px;
+        g.norm_in_gamma = w.rms_attn;
+        g.norm_eps = lead->eps;
+      }
       err = launch_gemm_rows(lead->dtype, kGemmF32, g, st);
     }
     AttnParams a{};
@@ -1572,7 +1593,7 @@ hipError_t enqueue_batch_step(Session *lead, Session *const *seqs, uint32_t T,
       }
       err = launch_gemm_rows(lead->dtype, kGemmResidual, g, st);
     }
-    if (err == hipSuccess && !o_norms)
+    if (err == hipSuccess && !o_norms && !gu_norms)
       err = launch_rmsnorm_rows(lead->dtype, lead->pr, w.rms_mlp, lead->eps, T, H, lead->pxn16, st, tiles);
     if (err == hipSuccess) {
       g = GemmRowsParams{};
@@ -1587,6 +1608,11 @@ hipError_t enqueue_batch_step(Session *lead, Session *const *seqs, uint32_t T,
       g.cols = H;
       g.workspace = lead->pgemm_ws;
       g.workspace_bytes = lead->pgemm_ws_bytes;
+      if (gu_norms) {
+        g.norm_in = lead->pr;
+        g.norm_in_gamma = w.rms_mlp;
+        g.norm_eps = lead->eps;
+      }
       err = launch_gemm_rows(lead->dtype, kGemmSwiglu, g, st);
     }
     if (err == hipSuccess) {
@@ -1609,7 +1635,7 @@ hipError_t enqueue_batch_step(Session *lead, Session *const *seqs, uint32_t T,
       }
       err = launch_gemm_rows(lead->dtype, kGemmResidual, g, st);
     }
-    out->pack_kernel_launches += (down_norms && l != 0 ? 0 : 1) + (o_norms ? 0 : 1);
+    out->pack_kernel_launches += ((down_norms && l != 0) || qkv_norms ? 0 : 1) + (o_norms || gu_norms ? 0 : 1);
     out->projection_kernel_launches += 4;
     out->dependency_kernel_launches += 1;
   }

@@ -73,6 +73,10 @@ struct GemmRowsParams {
   uint16_t *norm_out16;
   float norm_eps;
   uint32_t norm_packed_tiles;
+  // Optional, only where gemm_rows_norms_input() says so: the f32 rows [tokens][cols] and the weight of the RMSNorm whose result is
+  // the input - x[t] = round16(norm_in[t] * rsqrt(mean(norm_in[t]^2) + norm_eps) * norm_in_gamma) - instead of x16.
+  const float *norm_in;
+  const uint16_t *norm_in_gamma;
 };
 
 // rows >= 16 (any count: the last workgroup overlaps its neighbour, so with a row count that is no
@@ -80,7 +84,7 @@ struct GemmRowsParams {
 // whole 256-column blocks), 1 <= tokens <= kGemmMaxTokens, 16-byte aligned w and x16.
 bool gemm_rows_supported(uint32_t rows, uint32_t cols, uint32_t tokens);
 // The kernel a block of `tokens` rows in operand order goes to, and its K slices (kGemmNone: not taken).
-enum GemmKernel : int { kGemmNone = 0, kGemmWaves, kGemmBlock, kGemmFlow, kGemmWide, kGemmDeep };
+enum GemmKernel : int { kGemmNone = 0, kGemmWaves, kGemmFew, kGemmBlock, kGemmFlow, kGemmWide, kGemmDeep };
 struct GemmRoute {
   GemmKernel kernel;
   uint32_t kslices;
@@ -128,6 +132,15 @@ struct GemmFlowPlan {
 };
 GemmFlowPlan gemm_flow_plan(int epilogue, uint32_t rows, uint32_t cols, uint32_t tokens, uint64_t workspace_bytes);
 hipError_t launch_gemm_flow(uint32_t dtype, int epilogue, const GemmRowsParams &p, const GemmFlowPlan &plan, hipStream_t stream);
+// Blocks of up to kGemmFewMaxTokens rows in operand order, or of up to 16 f32 rows still to be normalised (gemm_few.hip): rows a
+// multiple of 4, cols of 64, no K slices. 0 workgroups: not taken.
+constexpr uint32_t kGemmFewMaxTokens = 32;
+uint32_t gemm_few_workgroups(int epilogue, uint32_t rows, uint32_t cols, uint32_t tokens);
+double gemm_few_us(int epilogue, uint32_t rows, uint32_t cols, uint32_t tokens);   // estimated time (gemm_rows_route)
+hipError_t launch_gemm_few(uint32_t dtype, int epilogue, const GemmRowsParams &p, hipStream_t stream);
+constexpr uint32_t kGemmNormInputCols = 1024;
+// Whether launch_gemm_rows honours GemmRowsParams::norm_in for this shape (X would be in operand order).
+bool gemm_rows_norms_input(int epilogue, uint32_t rows, uint32_t cols, uint32_t tokens, uint64_t workspace_bytes);
 // Whether launch_gemm_rows honours GemmRowsParams::norm_gamma for this shape (a K-sliced residual projection of a
 // wide block, rows a multiple of 4 and at most 16384); otherwise the caller normalises with launch_rmsnorm_rows.
 bool gemm_rows_fuses_norm(int epilogue, uint32_t rows, uint32_t cols, uint32_t tokens, uint32_t x_packed, uint64_t workspace_bytes);

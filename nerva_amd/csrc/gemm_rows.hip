@@ -319,7 +319,8 @@ bool gemm_rows_supported(uint32_t rows, uint32_t cols, uint32_t tokens) {
 // rows of partial sums per output and gains only up to 64 rows (8192 x 2048 pairs 16.7 / 16.6 / 25.6 against
 // 15.9 / 16.9 / 28.7).
 // More: the kernel with wave pairs or the one for 256-row tiles, whichever the estimate has clearly ahead.
-GemmRoute gemm_rows_route(int epilogue, uint32_t rows, uint32_t cols, uint32_t tokens, uint64_t workspace_bytes) {
+namespace {
+GemmRoute long_route(int epilogue, uint32_t rows, uint32_t cols, uint32_t tokens, uint64_t workspace_bytes) {
   if (tokens == 0) return GemmRoute{kGemmNone, 0};
   if (tokens > kGemmMaxTokens) {
     const uint32_t wide = tokens <= kGemmWideMaxTokens ? gemm_wide_slices(epilogue, rows, cols, tokens, workspace_bytes) : 0u;
@@ -338,6 +339,30 @@ GemmRoute gemm_rows_route(int epilogue, uint32_t rows, uint32_t cols, uint32_t t
   if (block.kslices == 0) return GemmRoute{kGemmNone, 0};
   return GemmRoute{kGemmBlock, block.kslices};
 }
+}  // namespace
+
+// Up to 32 rows: the kernel without K slices where its estimate is ahead of the others', which stream W at 6.9 MB a us behind 4 us,
+// 7 with the launch that adds the slices. That launch also writes the norm behind a residual projection: half a us for that where
+// the kernel here can norm its own input, else the 3.5 of a launch. A plain projection's slices are often added by its reader, for
+// 1 us. (us, the others with that launch -> here, 6 rows: 6144 x 4096 15.5 -> 11.9 and without it 11.3, 4096 x 4096 12.1 -> 8.6,
+// 2048 x 8192 11.7 -> 12.4, 4096 x 12288 21.8 -> 18.0, 8192 x 2048 pairs 15.8 -> 12.3, 12288 x 4096 pairs 31.7 -> 32.9, 13824 x 5120
+// pairs 45 -> 50; 32 rows: 4096 x 1024 6.8 -> 4.1, 3072 x 1024 pairs 7.9 -> 5.6, 6144 x 4096 16.0 -> 18.2.)
+GemmRoute gemm_rows_route(int epilogue, uint32_t rows, uint32_t cols, uint32_t tokens, uint64_t workspace_bytes) {
+  const GemmRoute route = long_route(epilogue, rows, cols, tokens, workspace_bytes);
+  const int mode = tuning(kTuneGemmFew);
+  if (route.kernel == kGemmNone || mode == 2 || gemm_few_workgroups(epilogue, rows, cols, tokens) == 0 || tuning(kTuneGemmBlockSlices) != 0 ||
+      tuning(kTuneGemmBlockRowTiles) != 0 || tuning(kTuneGemmBlockOff) == 1)
+    return route;
+  double others = (epilogue == kGemmSwiglu ? 2.0 : 1.0) * rows * cols * 2.0 / 6.9e6 + 4.0;
+  if (route.kslices > 1) others += epilogue == kGemmF32 ? 1.0 : epilogue == kGemmResidual ? (rows <= kGemmNormInputCols && tokens <= 16 ? 2.5 : -0.5) : 3.0;
+  return mode == 1 || gemm_few_us(epilogue, rows, cols, tokens) < others ? GemmRoute{kGemmFew, 1} : route;
+}
+
+bool gemm_rows_norms_input(int epilogue, uint32_t rows, uint32_t cols, uint32_t tokens, uint64_t workspace_bytes) {
+  // the rows in one pass of sixteen waves' registers, and a workgroup a CU: 3072 x 2048 7.6 us, with a norm of its own in front 7.4
+  return cols <= kGemmNormInputCols && tokens <= 16 && gemm_rows_route(epilogue, rows, cols, tokens, workspace_bytes).kernel == kGemmFew &&
+         gemm_few_workgroups(epilogue, rows, cols, tokens) <= 256u;
+}
 
 hipError_t launch_gemm_rows(uint32_t dtype, int epilogue, const GemmRowsParams &p, hipStream_t stream) {
   // rows as they come: only the kernel of this file
@@ -345,9 +370,13 @@ hipError_t launch_gemm_rows(uint32_t dtype, int epilogue, const GemmRowsParams &
   GemmRoute route{kGemmNone, 0};
   if (p.x_packed != 0) route = gemm_rows_route(epilogue, p.rows, p.cols, p.tokens, room);
   else if (gemm_rows_supported(p.rows, p.cols, p.tokens)) route = GemmRoute{kGemmWaves, 1};
-  if (p.w == nullptr || p.x16 == nullptr) return hipErrorInvalidValue;
+  if (p.w == nullptr || (p.x16 == nullptr && p.norm_in == nullptr)) return hipErrorInvalidValue;
   if (route.kernel == kGemmNone) return hipErrorInvalidValue;
   if (!aligned16(p.w) || !aligned16(p.x16)) return hipErrorInvalidValue;
+  if (p.norm_in != nullptr &&   // rows to be normalised only where the launch does that
+      (p.norm_in_gamma == nullptr || p.x_packed == 0 || !aligned16(p.norm_in) || !aligned16(p.norm_in_gamma) || p.norm_gamma != nullptr ||
+       !gemm_rows_norms_input(epilogue, p.rows, p.cols, p.tokens, room)))
+    return hipErrorInvalidValue;
   if ((epilogue == kGemmF32 || epilogue == kGemmResidual) && p.out_f32 == nullptr) return hipErrorInvalidValue;
   if (epilogue == kGemmResidual && p.residual == nullptr) return hipErrorInvalidValue;
   // rows shared by the last two workgroups are written twice: an in-place residual would be added twice
@@ -367,6 +396,7 @@ hipError_t launch_gemm_rows(uint32_t dtype, int epilogue, const GemmRowsParams &
       (p.norm_out16 == nullptr || !gemm_rows_fuses_norm(epilogue, p.rows, p.cols, p.tokens, p.x_packed, p.workspace != nullptr ? p.workspace_bytes : 0)))
     return hipErrorInvalidValue;
   switch (route.kernel) {
+    case kGemmFew: return launch_gemm_few(dtype, epilogue, p, stream);
     case kGemmDeep: return launch_gemm_deep(dtype, epilogue, p, route.kslices, stream);
     case kGemmWide: return launch_gemm_wide(dtype, epilogue, p, route.kslices, stream);
     case kGemmBlock: return launch_gemm_block(dtype, epilogue, p, gemm_block_plan(epilogue, p.rows, p.cols, p.tokens, room), stream);

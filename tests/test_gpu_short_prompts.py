@@ -1,9 +1,11 @@
-"""Kernels of short prompts, against the kernels of long ones and the token walk."""
+"""Kernels of short prompts, of few token rows and of batch steps, against the oracle and against the kernels they stand in for."""
 import numpy as np
 import pytest
 
 import nerva_amd as N
-from test_gpu_session import BF16, F16, random_model
+import oracle as O
+from test_gpu_ops import dev
+from test_gpu_session import BF16, E2E_REL_L2, F16, random_model, rel_l2, started
 
 pytestmark = pytest.mark.gpu
 
@@ -42,3 +44,100 @@ def test_narrow_and_wide_prompt_attention_give_the_same_bits(dtype, heads, kv, h
         for got, want in zip(results[0][1], results[1][1]):
             assert np.array_equal(got, want), (prefix, n)
     s.destroy()
+
+
+@pytest.fixture
+def tuned():
+    yield N.Device.set_tuning
+    N.Device.reset_tuning()
+
+
+@pytest.mark.parametrize("dtype", [BF16, F16])
+@pytest.mark.parametrize("rows,cols,tokens", [(16, 2048, 1), (20, 2048, 5), (48, 4096, 16), (4100, 2048, 17), (36, 6144, 32), (64, 10240, 15),
+                                              (32, 14336, 31)])
+def test_few_rows_without_slices_match_the_oracle(tuned, dtype, rows, cols, tokens):
+    """Row counts off the grid of 16, 4 to 28 blocks a wave (all requested at once; a remainder; several rounds), one and two
+    token tiles: plain, with bias, residual and rounding, and gate/up pairs in operand order."""
+    tuned("gemm_few", 1)
+    rng = np.random.default_rng(rows + cols + tokens)
+    w = O.encode16(dtype, rng.normal(0, 0.02, (2 * rows, cols)))
+    x = O.encode16(dtype, rng.normal(0, 1, (tokens, cols)))
+    bias, res = O.encode16(dtype, rng.normal(0, 0.1, rows)), rng.normal(0, 1, (tokens, rows)).astype(np.float32)
+    packed, _ = N.gemm_operand_order(x)
+    exact = O.decode16(dtype, x).astype(np.float64) @ O.decode16(dtype, w).astype(np.float64).T
+    y, dw, dx = N.DeviceBuffer(tokens * rows * 4), dev(w), dev(packed)
+    N.gemm_rows(dtype, dw, rows, cols, tokens, dx, epilogue=0, out_f32=y, input_operand_order=True)
+    got = y.numpy(np.float32).reshape(tokens, rows)
+    assert max(rel_l2(g, e) for g, e in zip(got, exact[:, :rows])) <= 2e-6      # sums of f32 over at most 14336 columns
+    N.gemm_rows(dtype, dw, rows, cols, tokens, dx, epilogue=1, bias=dev(bias), residual=dev(res), out_f32=y, round_output=True,
+                input_operand_order=True)
+    got = y.numpy(np.float32).reshape(tokens, rows)
+    assert rel_l2(got, O.decode16(dtype, O.encode16(dtype, (exact[:, :rows] + O.decode16(dtype, bias) + res).astype(np.float32)))) <= 4e-3
+    if rows % 32 == 0:
+        out = N.DeviceBuffer(32 * rows * 2)
+        N.gemm_rows(dtype, dw, rows, cols, tokens, dx, epilogue=2, out16=out, input_operand_order=True, output16_operand_order=True)
+        _, at = N.gemm_operand_order(np.zeros((tokens, rows), np.uint16))
+        gate, up = exact[:, :rows], exact[:, rows:]
+        got = O.decode16(dtype, out.numpy(np.uint16, 32 * rows)[at])
+        assert rel_l2(got, O.decode16(dtype, O.encode16(dtype, (gate / (1 + np.exp(-gate)) * up).astype(np.float32)))) <= 4e-3
+
+
+# dtype, hidden, heads, kv, hd, inter: the first normed projection reads fewer blocks of 64 columns than it has waves, an odd number, all
+NORMED = [(BF16, 512, 4, 2, 128, 1024), (F16, 960, 10, 2, 64, 2560), (BF16, 1024, 8, 4, 128, 3072)]
+
+
+@pytest.mark.parametrize("geom", NORMED, ids=str)
+def test_projections_that_norm_their_input(tuned, geom):
+    """2 to 16 tokens of a sequence, and 17, whose projections have a norm in front, with the kernel and without it."""
+    dtype, hidden, heads, kv, hd, inter = geom
+    weights, _ = random_model(dtype, hidden, heads, kv, hd, inter, 301, 3, hidden, 1e6, True, False)
+    s = N.DecodeSession.create(weights, 64)
+    rng = np.random.default_rng(hidden)
+    for n in (2, 3, 15, 16, 17):
+        tokens, rows = rng.integers(0, 301, 20 + n).astype(np.uint32), []
+        for mode in (0, 2):
+            tuned("gemm_few", mode)
+            assert s.release_sequence() == 0
+            assert s.extend(tokens[:20])[0] == 0
+            rc, _, logits, _ = s.extend(tokens[20:], range(n))
+            assert rc == 0
+            rows.append((logits.copy(), s.kv_range(0, 20, n)))
+        assert rel_l2(rows[0][0], rows[1][0]) <= E2E_REL_L2, n
+        for got, want in zip(rows[0][1], rows[1][1]):    # of the first layer: the sums' order alone
+            assert rel_l2(O.decode16(dtype, got), O.decode16(dtype, want)) <= 2e-3, n
+    s.destroy()
+
+
+# the batch step's attention: partial sums of q, k, v as they come (2048 wide, many sequences) or added; 1 to 8 query heads a key head
+@pytest.mark.parametrize("dtype,hidden,heads,kv,hd,count,length", [
+    (BF16, 1024, 16, 8, 128, 6, 764),    # from one split a sequence to several
+    (BF16, 2048, 16, 8, 128, 32, 30), (F16, 512, 8, 4, 64, 9, 250), (BF16, 512, 14, 2, 64, 3, 129), (F16, 768, 10, 2, 128, 2, 513),
+    (BF16, 512, 16, 2, 128, 5, 63), (BF16, 512, 16, 16, 64, 20, 15)])    # (the last: more workgroups than CUs)
+def test_batch_attention_matches_sequences_alone(dtype, hidden, heads, kv, hd, count, length):
+    """Contexts of a key, around a wave's four requested tiles, and across the lengths where the split factor changes."""
+    vocab, layers, steps = 301, 2, 6
+    weights, _ = random_model(dtype, hidden, heads, kv, hd, 1024, vocab, layers, count, 1e6, True, True)
+    parent = N.DecodeSession.create(weights, length + 16, plan=N.WeightPlan.from_weights(weights))
+    sessions = [parent] + [parent.fork_shared_weights() for _ in range(count - 1)]
+    assert parent.shares_weight_stream() or hidden < 1024
+    rng = np.random.default_rng(count)
+    prompts = [rng.integers(0, vocab, length if i % 3 == 0 else 1 + (length * i) // count).astype(np.uint32) for i in range(count)]
+    streams = [[started(s, p)] for s, p in zip(sessions, prompts)]
+    for _ in range(steps):
+        rc, _, tokens = N.DecodeSession.batch_advance_one(sessions, 32, 2)
+        assert rc == 0
+        for stream, token in zip(streams, tokens):
+            stream.append(int(token))
+    solo = parent.fork_shared_weights()
+    for i in sorted({0, 1, count - 1}):
+        assert solo.release_sequence() == 0
+        assert solo.extend(prompts[i])[0] == 0
+        for token in streams[i][:-1]:
+            assert solo.extend([token], [0])[0] == 0
+        for layer in range(layers):
+            for got, want in zip(sessions[i].kv_range(layer, len(prompts[i]), steps), solo.kv_range(layer, len(prompts[i]), steps)):
+                tol = 2e-3 if layer == 0 else E2E_REL_L2
+                assert rel_l2(O.decode16(dtype, got), O.decode16(dtype, want)) <= tol, (i, layer)
+    solo.destroy()
+    for s in sessions[::-1]:
+        s.destroy()
