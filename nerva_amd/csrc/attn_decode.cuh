@@ -152,6 +152,10 @@ __host__ __device__ __forceinline__ bool attn_matrix_cores(uint32_t heads, uint3
 // (measured on the Qwen3-8B head shape: 64 keys 4.8 us against 12.7, 256 keys 6.5 against 8.2, 512 keys 10.0
 // against 8.0).
 constexpr uint32_t kAttnSingleSplitBlocks = 20;
+// The same for a batch step, whose splits merge behind a ticket (16 heads on 8, 6 sequences of 100 / 300 / 620 / 1000 keys: one split
+// 5.7 / 8.2 / 11.0 / 14.2 us, six 6.9 / 11.3 / 12.5 / 14.2; 32 on 8, 16 sequences of 200 / 600 / 1000: 7.3 / 10.8 / 14.2 and 11.0 /
+// 13.8 / 15.6 in two).
+constexpr uint32_t kAttnBatchSingleSplitBlocks = 48;
 __host__ __device__ __forceinline__ void attn_split_geometry(uint32_t pos, uint32_t splits, uint32_t single_blocks,
                                                              uint32_t &nblk, uint32_t &bps, uint32_t &active) {
   nblk = (pos + 1 + kKvBlockTokens - 1) / kKvBlockTokens;

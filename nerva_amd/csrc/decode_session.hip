@@ -1474,7 +1474,7 @@ hipError_t enqueue_batch_step(Session *lead, Session *const *seqs, uint32_t T,
   const float *rope_freq = lead->theta > 0.0f ? lead->rope_freq : nullptr;
   const uint32_t tiles = block_operand_tiles(lead, T);
   BatchTable *host = lead->host_btable;
-  uint32_t min_blocks = ~0u;
+  uint32_t min_blocks = ~0u, used_blocks = 0;
   for (uint32_t t = 0; t < T; ++t) {
     const Session *q = seqs[t];
     host->seq[t] = AttnSeq{q->kc, q->vc, q->table, q->block_count, q->cursor};
@@ -1493,12 +1493,15 @@ hipError_t enqueue_batch_step(Session *lead, Session *const *seqs, uint32_t T,
     sp.cursor = q->state;
     sp.max_steps = q->max_ctx;
     min_blocks = std::min(min_blocks, q->block_count);
+    used_blocks = std::max(used_blocks, q->cursor / kKvBlockTokens + 1u);
   }
   // kv_heads x T workgroups per split already fill the chip at T = 32; measured on MI355X (Qwen3-8B
   // shapes, contexts 128 .. 8192) further splits only add merge work, so: as many as it takes to reach
   // one workgroup per CU
   uint32_t batch_splits = std::max<uint32_t>(1u, std::min<uint32_t>(attn_default_splits(lead->kv_heads, min_blocks),
                                                                    (256u + lead->kv_heads * T - 1) / (lead->kv_heads * T)));
+  // ... while the longest context is more than one workgroup reads in the time that splits take to hand over
+  if (used_blocks <= kAttnBatchSingleSplitBlocks) batch_splits = 1;
   if (const int want = tuning(kTuneBatchSplits); want >= 1 && want <= static_cast<int>(kAttnMaxSplits))
     batch_splits = std::min<uint32_t>(static_cast<uint32_t>(want), min_blocks);
   hipError_t err = hipMemcpyAsync(lead->btable, host, sizeof(BatchTable), hipMemcpyHostToDevice, st);
