@@ -44,12 +44,15 @@ constexpr int kBWTile = 16 * kBRowStride;    // one 16-row block of W in LDS
 // BW: waves per workgroup. With three, the X block is not a whole number of rounds of the workgroup's threads: the
 // last round wraps and fetches pieces of the first again (same bytes to the same place), so that no request sits
 // under a branch.
-template <uint32_t DT, int EPI, int NR, int TT, int BW>
+// USED: token tiles that hold tokens (the layout has TT): the others are neither fetched nor multiplied (12288 x 4096 pairs of 65 / 81 / 97
+// rows 55 / 49 / 49 us with all eight -> 50 / 43 / 46, 4096 x 12288 29.8 / 30.0 / 30.4 -> 25.6 / 26.7 / 28.4).
+template <uint32_t DT, int EPI, int NR, int TT, int BW, int USED = TT>
 __global__ __launch_bounds__(BW * kWave, NR == 1 ? 2 : 1) void gemm_block_kernel(GemmRowsParams p, float *partials, uint32_t rotate) {
   constexpr int kBThreads = BW * kWave;
-  constexpr int kTiles = TT;                              // 16-token tiles of the block (X in operand order with TT tiles)
+  constexpr int kTiles = USED;                            // 16-token tiles of the block (X in operand order with TT tiles)
   constexpr int kStageVec = kBSteps * kTiles * kWave;     // 16-byte pieces of one X block (TT = 8: 2048 = 32 KiB)
   constexpr int kFill = (kStageVec + kBThreads - 1) / kBThreads;   // pieces per thread and block
+  static_assert(USED == TT || kStageVec % kBThreads == 0, "a wave's requests are whole pieces of 1 KiB");
   static_assert(kFill <= 8, "the X requests of a block go out in the first four half K-steps, two at a time");
   extern __shared__ __align__(16) unsigned char smem[];
   u32x4_t *stage = reinterpret_cast<u32x4_t *>(smem);   // [kStageVec]: the X block, shared by the four waves
@@ -84,7 +87,7 @@ __global__ __launch_bounds__(BW * kWave, NR == 1 ? 2 : 1) void gemm_block_kernel
   uint16_t *park_at = wtile + q * kBRowStride + n * 8;
   const uint16_t *a_read = wtile + n * kBRowStride + q * 8;
   // X block b of this slice: kStageVec pieces in a row
-  const char *xbase = reinterpret_cast<const char *>(p.x16) + static_cast<uint64_t>(k0 / 32u) * (kTiles * kWave) * sizeof(u32x4_t);
+  const char *xbase = reinterpret_cast<const char *>(p.x16) + static_cast<uint64_t>(k0 / 32u) * (TT * kWave) * sizeof(u32x4_t);
 
   constexpr int kRing = NR == 1 ? 2 : kBRing;   // W blocks requested ahead: what the register budget holds
   u32x4_t areg[kRing][NR][4];
@@ -102,11 +105,19 @@ __global__ __launch_bounds__(BW * kWave, NR == 1 ? 2 : 1) void gemm_block_kernel
 #define NV_BLK_WPARK(BUF)                                                                           \
   _Pragma("unroll") for (int j = 0; j < NR; ++j) _Pragma("unroll") for (int i = 0; i < 4; ++i)       \
       *reinterpret_cast<u32x4_t *>(park_at + j * kBWTile + 4 * i * kBRowStride) = areg[BUF][j][i]
-#define NV_BLK_XPIECE(I) ((static_cast<uint32_t>(I) * kBThreads + threadIdx.x) & static_cast<uint32_t>(kStageVec - 1))
+#define NV_BLK_XPIECE(I) (USED == TT ? ((static_cast<uint32_t>(I) * kBThreads + threadIdx.x) & static_cast<uint32_t>(kStageVec - 1)) \
+                                     : static_cast<uint32_t>(I) * kBThreads + threadIdx.x)
+  // where that piece lies in the layout's block
+  const auto x_source = [&](int i) {
+    if constexpr (USED == TT) return (static_cast<uint32_t>(i) * kBThreads + threadIdx.x) & static_cast<uint32_t>(kStageVec - 1);
+    const uint32_t piece = static_cast<uint32_t>(i) * BW + wave;
+    return (piece / USED * TT + piece % USED) * kWave + lane;
+  };
+  constexpr uint32_t kBlockVec = kBSteps * TT * kWave;
 #define NV_BLK_X(XB, BLK)                                                                           \
   _Pragma("unroll") for (int i = 0; i < kFill; ++i)                                                 \
       xreg[XB][i] = *reinterpret_cast<const u32x4_t *>(                                              \
-          xbase + (static_cast<uint64_t>(NV_BLK_AT(BLK)) * kStageVec + NV_BLK_XPIECE(i)) * sizeof(u32x4_t))
+          xbase + (static_cast<uint64_t>(NV_BLK_AT(BLK)) * kBlockVec + x_source(i)) * sizeof(u32x4_t))
 #define NV_BLK_XPARK(XB)                                                                            \
   _Pragma("unroll") for (int i = 0; i < kFill; ++i) stage[NV_BLK_XPIECE(i)] = xreg[XB][i]
   // LDS operand reads run one half K-step ahead of the products that use them: once the products of token
@@ -117,9 +128,9 @@ __global__ __launch_bounds__(BW * kWave, NR == 1 ? 2 : 1) void gemm_block_kernel
   _Pragma("unroll") for (int j = 0; j < NR; ++j)                                                     \
       A[j] = *reinterpret_cast<const u32x4_t *>(a_read + j * kBWTile + (S) * 32)
 #define NV_BLK_READ_B(S, C0)                                                                        \
-  _Pragma("unroll") for (int c = C0; c < C0 + kTiles / 2; ++c) b[c] = stage[((S) * kTiles + c) * kWave + lane]
+  _Pragma("unroll") for (int c = C0; c < ((C0) == 0 ? kTiles / 2 : kTiles); ++c) b[c] = stage[((S) * kTiles + c) * kWave + lane]
 #define NV_BLK_PRODUCTS(A, C0)                                                                      \
-  _Pragma("unroll") for (int c = C0; c < C0 + kTiles / 2; ++c)                                      \
+  _Pragma("unroll") for (int c = C0; c < ((C0) == 0 ? kTiles / 2 : kTiles); ++c)                    \
       _Pragma("unroll") for (int j = 0; j < NR; ++j) acc[j][c] = mfma_k32<DT>(A[j], b[c], acc[j][c])
   // The requests for the blocks ahead go out between the products, two per half K-step (first the X pieces,
   // then the W rows: the order they are awaited in): the CU's vector-memory path takes 64 bytes a cycle, and
@@ -130,7 +141,7 @@ __global__ __launch_bounds__(BW * kWave, NR == 1 ? 2 : 1) void gemm_block_kernel
 #define NV_BLK_X1(XB, BLK, I)                                                                       \
   if constexpr ((I) < kFill)                                                                        \
     xreg[XB][I] = *reinterpret_cast<const u32x4_t *>(                                                \
-        xbase + (static_cast<uint64_t>(NV_BLK_AT(BLK)) * kStageVec + NV_BLK_XPIECE(I)) * sizeof(u32x4_t))
+        xbase + (static_cast<uint64_t>(NV_BLK_AT(BLK)) * kBlockVec + x_source(I)) * sizeof(u32x4_t))
 #define NV_BLK_SLOT(K, BUF, XB, XEN, XBLK, WEN, WBLK)                                               \
   if constexpr ((K) < 4) {                                                                          \
     if constexpr (XEN && 2 * (K) < kFill) {                                                         \
@@ -379,21 +390,21 @@ constexpr size_t block_lds_bytes() {
   return static_cast<size_t>(kBSteps) * TT * kWave * sizeof(u32x4_t) + static_cast<size_t>(BW) * NR * kBWTile * sizeof(uint16_t);
 }
 
-template <uint32_t DT, int EPI, int NR, int TT, int BW = kBW>
+template <uint32_t DT, int EPI, int NR, int TT, int BW = kBW, int USED = TT>
 hipError_t launch_block_tt(const GemmRowsParams &p, float *partials, uint32_t kslices, hipStream_t stream) {
   const uint32_t wg_rows = EPI == kGemmSwiglu ? 16u * BW : 16u * BW * NR;
-  constexpr size_t lds = block_lds_bytes<NR, TT, BW>();
+  constexpr size_t lds = block_lds_bytes<NR, USED, BW>();
   if (lds > 64 * 1024) {
     // more than the default dynamic LDS limit: raise it once per kernel (never under stream capture)
     static std::once_flag once;
     static hipError_t raised = hipSuccess;
     std::call_once(once, [] {
-      raised = hipFuncSetAttribute(reinterpret_cast<const void *>(&gemm_block_kernel<DT, EPI, NR, TT, BW>),
+      raised = hipFuncSetAttribute(reinterpret_cast<const void *>(&gemm_block_kernel<DT, EPI, NR, TT, BW, USED>),
                                    hipFuncAttributeMaxDynamicSharedMemorySize, static_cast<int>(lds));
     });
     if (raised != hipSuccess) return raised;
   }
-  hipLaunchKernelGGL((gemm_block_kernel<DT, EPI, NR, TT, BW>), dim3(p.rows / wg_rows, kslices), dim3(BW * kWave), lds, stream,
+  hipLaunchKernelGGL((gemm_block_kernel<DT, EPI, NR, TT, BW, USED>), dim3(p.rows / wg_rows, kslices), dim3(BW * kWave), lds, stream,
                      p, partials, block_rotation());
   hipError_t err = hipGetLastError();
   if (err == hipSuccess && kslices > 1 && !(EPI == kGemmF32 && p.keep_partials != 0)) {
@@ -417,7 +428,13 @@ hipError_t launch_block_nr(const GemmRowsParams &p, float *partials, uint32_t ks
   switch (p.x_packed) {   // token tiles of the block = tiles of its operand-order layout
     case 2: return launch_block_tt<DT, EPI, NR, 2>(p, partials, kslices, stream);
     case 4: return launch_block_tt<DT, EPI, NR, 4>(p, partials, kslices, stream);
-    case 8: return launch_block_tt<DT, EPI, NR, 8>(p, partials, kslices, stream);
+    case 8:
+      if constexpr (EPI != kGemmXielu) {
+        if (p.tokens <= 80) return launch_block_tt<DT, EPI, NR, 8, kBW, 5>(p, partials, kslices, stream);
+        if (p.tokens <= 96) return launch_block_tt<DT, EPI, NR, 8, kBW, 6>(p, partials, kslices, stream);
+        if (p.tokens <= 112) return launch_block_tt<DT, EPI, NR, 8, kBW, 7>(p, partials, kslices, stream);
+      }
+      return launch_block_tt<DT, EPI, NR, 8>(p, partials, kslices, stream);
     default: return hipErrorInvalidValue;
   }
 }
@@ -441,24 +458,28 @@ hipError_t launch_block_nr(const GemmRowsParams &p, float *partials, uint32_t ks
 // workgroup fetches the whole X block, whatever its rows).
 constexpr int kWTiles = 16;                  // token tiles of the block's operand-order layout
 constexpr uint32_t kWTokCap = 256;           // token rows at most; the token stride of this kernel's partial sums
-constexpr size_t wide_lds_bytes(int pairs) {
-  return static_cast<size_t>(kBSteps) * kWTiles * kWave * sizeof(u32x4_t) + static_cast<size_t>(pairs) * 2 * kBWTile * sizeof(uint16_t);
+constexpr size_t wide_lds_bytes(int pairs, int tiles) {
+  return static_cast<size_t>(kBSteps) * tiles * kWave * sizeof(u32x4_t) + static_cast<size_t>(pairs) * 2 * kBWTile * sizeof(uint16_t);
 }
 constexpr uint32_t wide_wg_rows(int epilogue, int pairs) { return (epilogue == kGemmSwiglu ? 16u : 32u) * pairs; }
+constexpr int wide_tiles(uint32_t tokens) { return static_cast<int>((tokens + 31u) / 32u * 2u); }   // 10 .. 16
 inline int wide_pairs(int epilogue, uint32_t rows) {
   const int first = epilogue == kGemmSwiglu ? 4 : 3, second = 7 - first;
   return rows % wide_wg_rows(epilogue, first) == 0 ? first : rows % wide_wg_rows(epilogue, second) == 0 ? second : 0;
 }
 
-template <uint32_t DT, int EPI, int PAIRS>
+// TILES: token tiles that are fetched and multiplied, an even number; the layout's other tiles hold no tokens. What a CU pulls in is
+// mostly X: 12288 x 4096 pairs of 130 / 162 / 195 / 250 rows
+// 73 / 81 / 76 / 79 us with all sixteen -> 53 / 59 / 70 / 79, 4096 x 12288 39 / 40 / 41 / 44 -> 32 / 35 / 38 / 44.
+template <uint32_t DT, int EPI, int PAIRS, int TILES>
 __global__ __launch_bounds__(PAIRS * 2 * kWave, 2) void gemm_wide_kernel(GemmRowsParams p, float *partials) {
   constexpr int kWPairs = PAIRS;
   constexpr int kWThreads = kWPairs * 2 * kWave;
-  constexpr int kStageVec = kBSteps * kWTiles * kWave;   // 16-byte pieces of one X block: 4096 = 64 KiB
+  constexpr int kStageVec = kBSteps * TILES * kWave;   // 16-byte pieces of one X block: 4096 = 64 KiB with all tiles
   constexpr int kFill = (kStageVec + kWThreads - 1) / kWThreads;   // pieces per thread and block (the last one only
   constexpr bool kFillRagged = kStageVec % kWThreads != 0;         // for the first threads when the count does not divide)
   constexpr int kXPer = (kFill + 3) / 4;                 // X requests per slot
-  constexpr int kHalf = kWTiles / 2;                     // token tiles per wave
+  constexpr int kHalf = TILES / 2;                       // token tiles per wave
   extern __shared__ __align__(16) unsigned char smem[];
   u32x4_t *stage = reinterpret_cast<u32x4_t *>(smem);
   const int lane = threadIdx.x & (kWave - 1);
@@ -481,7 +502,12 @@ __global__ __launch_bounds__(PAIRS * 2 * kWave, 2) void gemm_wide_kernel(GemmRow
   uint16_t *park_at = wtile + half * kBWTile + q * kBRowStride + n * 8;
   const uint16_t *a_read = wtile + n * kBRowStride + q * 8;
   const char *xbase = reinterpret_cast<const char *>(p.x16) + static_cast<uint64_t>(k0 / 32u) * (kWTiles * kWave) * sizeof(u32x4_t);
-  const uint32_t xlane = threadIdx.x * static_cast<uint32_t>(sizeof(u32x4_t));
+  const uint32_t xlane = lane * static_cast<uint32_t>(sizeof(u32x4_t));
+  // piece of 1 KiB that this wave's request i asks for: (K-step, tile) = piece / TILES, piece % TILES
+  const auto x_at = [&](int i) {
+    const uint32_t piece = static_cast<uint32_t>(i) * (kWPairs * 2) + wave;
+    return (piece / TILES * kWTiles + piece % TILES) * static_cast<uint32_t>(kWave * sizeof(u32x4_t));
+  };
   const u32x4_t *b_read = stage + half * kHalf * kWave + lane;
 
   constexpr int kRing = 2;   // W blocks requested ahead (a block is about two microseconds of products)
@@ -503,16 +529,16 @@ __global__ __launch_bounds__(PAIRS * 2 * kWave, 2) void gemm_wide_kernel(GemmRow
 #define NV_WD_X1(BLK, I)                                                                            \
   if (NV_WD_XLIVE(I))                                                                               \
   xreg[I] = *reinterpret_cast<const u32x4_t *>(                                                      \
-      xbase + (static_cast<uint64_t>(BLK) * kStageVec + (I) * kWThreads) * sizeof(u32x4_t) + xlane)
+      xbase + static_cast<uint64_t>(BLK) * (kBSteps * kWTiles * kWave * sizeof(u32x4_t)) + x_at(I) + xlane)
 #define NV_WD_X(BLK) _Pragma("unroll") for (int i = 0; i < kFill; ++i) { NV_WD_X1(BLK, i); }
 #define NV_WD_XPARK() \
   _Pragma("unroll") for (int i = 0; i < kFill; ++i) { if (NV_WD_XLIVE(i)) stage[i * kWThreads + threadIdx.x] = xreg[i]; }
 #define NV_WD_READ_A(S, A) \
   _Pragma("unroll") for (int j = 0; j < 2; ++j) A[j] = *reinterpret_cast<const u32x4_t *>(a_read + j * kBWTile + (S) * 32)
 #define NV_WD_READ_B(S, B) \
-  _Pragma("unroll") for (int c = 0; c < kHalf; ++c) B[c] = b_read[((S) * kWTiles + c) * kWave]
+  _Pragma("unroll") for (int c = 0; c < kHalf; ++c) B[c] = b_read[((S) * TILES + c) * kWave]
 #define NV_WD_PRODUCTS(A, B, C0)                                                                    \
-  _Pragma("unroll") for (int c = C0; c < C0 + kHalf / 2; ++c)                                       \
+  _Pragma("unroll") for (int c = C0; c < ((C0) == 0 ? kHalf / 2 : kHalf); ++c)                      \
       _Pragma("unroll") for (int j = 0; j < 2; ++j) acc[j][c] = mfma_k32<DT>(A[j], B[c], acc[j][c])
   // request slots between the products: slots 0..3 the next X block's pieces (two or three each), slots
   // 4 and 5 the four rows-of-four of the W block kRing ahead, two each (the order they are awaited in)
@@ -915,21 +941,35 @@ __global__ __launch_bounds__(8 * kWave, 2) void gemm_deep_kernel(GemmRowsParams 
   }
 }
 
-template <uint32_t DT, int EPI, int PAIRS>
-hipError_t launch_wide_pairs(const GemmRowsParams &p, float *partials, uint32_t kslices, hipStream_t stream) {
+template <uint32_t DT, int EPI, int PAIRS, int TILES>
+hipError_t launch_wide_tiles(const GemmRowsParams &p, float *partials, uint32_t kslices, hipStream_t stream) {
   constexpr uint32_t wg_rows = wide_wg_rows(EPI, PAIRS);
-  constexpr size_t lds = wide_lds_bytes(PAIRS);
+  constexpr size_t lds = wide_lds_bytes(PAIRS, TILES);
   // more than the default dynamic LDS limit: raised once per kernel (never under stream capture)
   static std::once_flag once;
   static hipError_t raised = hipSuccess;
   std::call_once(once, [] {
-    raised = hipFuncSetAttribute(reinterpret_cast<const void *>(&gemm_wide_kernel<DT, EPI, PAIRS>),
+    raised = hipFuncSetAttribute(reinterpret_cast<const void *>(&gemm_wide_kernel<DT, EPI, PAIRS, TILES>),
                                  hipFuncAttributeMaxDynamicSharedMemorySize, static_cast<int>(lds));
   });
   if (raised != hipSuccess) return raised;
-  hipLaunchKernelGGL((gemm_wide_kernel<DT, EPI, PAIRS>), dim3(p.rows / wg_rows, kslices), dim3(PAIRS * 2 * kWave), lds, stream, p,
+  hipLaunchKernelGGL((gemm_wide_kernel<DT, EPI, PAIRS, TILES>), dim3(p.rows / wg_rows, kslices), dim3(PAIRS * 2 * kWave), lds, stream, p,
                      partials);
   return hipGetLastError();
+}
+
+// (the activation of mixed stacks: all tiles)
+template <uint32_t DT, int EPI, int PAIRS>
+hipError_t launch_wide_pairs(const GemmRowsParams &p, float *partials, uint32_t kslices, hipStream_t stream) {
+  if constexpr (EPI != kGemmXielu) {
+    switch (wide_tiles(p.tokens)) {
+      case 10: return launch_wide_tiles<DT, EPI, PAIRS, 10>(p, partials, kslices, stream);
+      case 12: return launch_wide_tiles<DT, EPI, PAIRS, 12>(p, partials, kslices, stream);
+      case 14: return launch_wide_tiles<DT, EPI, PAIRS, 14>(p, partials, kslices, stream);
+      default: break;
+    }
+  }
+  return launch_wide_tiles<DT, EPI, PAIRS, kWTiles>(p, partials, kslices, stream);
 }
 
 // gemm_deep_kernel (blocks of 129..4096 rows): workgroups of 256 weight rows (a gate/up pair: 128 + 128) x 256 tokens, or
@@ -957,7 +997,7 @@ inline uint32_t deep_slices_for(int epilogue, uint32_t rows, uint32_t cols, int 
 }
 // Estimated times of a launch of these kernels and of the launch that adds its partial sums: rounds of 256 workgroups,
 // each 5 us and so much a K-block - 1.5 us for 64 columns of 256 rows x 256 tokens, 1.3 for 192 rows, 2.05 and 1.75 us
-// for 128 columns of the four and three wave pairs above - and for the partial sums 4 us and a read at 5 TB/s.
+// for 128 columns of the four and three wave pairs above with sixteen token tiles - and for the partial sums 4 us and a read at 5 TB/s.
 inline double rounds_us(uint32_t workgroups, uint32_t blocks, double block_us) {
   return ((workgroups + 255u) / 256u) * (5.0 + block_us * blocks);
 }
@@ -1167,7 +1207,7 @@ uint32_t gemm_deep_slices(int epilogue, uint32_t rows, uint32_t cols, uint32_t t
 double gemm_wide_us(int epilogue, uint32_t rows, uint32_t cols, uint32_t tokens, uint32_t kslices) {
   const int pairs = wide_pairs(epilogue, rows);
   const uint32_t wg_rows = wide_wg_rows(epilogue, pairs);
-  return rounds_us(rows / wg_rows * kslices, cols / kBK / kslices, pairs == 4 ? 2.05 : 1.75) +
+  return rounds_us(rows / wg_rows * kslices, cols / kBK / kslices, (pairs == 4 ? 2.05 : 1.75) * (0.05 + 0.95 * wide_tiles(tokens) / kWTiles)) +
          partials_us(epilogue == kGemmSwiglu ? 2u * rows : rows, tokens, kslices);
 }
 

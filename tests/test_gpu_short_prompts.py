@@ -141,3 +141,28 @@ def test_batch_attention_matches_sequences_alone(dtype, hidden, heads, kv, hd, c
     solo.destroy()
     for s in sessions[::-1]:
         s.destroy()
+
+
+@pytest.mark.parametrize("dtype", [BF16, F16])
+@pytest.mark.parametrize("tokens", [65, 80, 81, 96, 97, 112, 113, 129, 160, 161, 192, 193, 224, 225])
+def test_blocks_of_fewer_tiles_than_their_layout(dtype, tokens):
+    """Both ends of every number of token tiles between 5 and 16, in workgroups of three and of four wave pairs and of one and two
+    row tiles; token slots without a token hold NaN, which must not get anywhere."""
+    rng = np.random.default_rng(tokens)
+    for rows, cols in ((192, 2048), (256, 2048), (12288, 2048)):
+        pairs = rows == 256
+        w = O.encode16(dtype, rng.normal(0, 0.02, ((2 if pairs else 1) * rows, cols)))
+        x = O.encode16(dtype, rng.normal(0, 1, (tokens, cols)))
+        packed, at = N.gemm_operand_order(x)
+        packed[:] = 0x7fff
+        packed[at] = x
+        exact = O.decode16(dtype, x).astype(np.float32) @ O.decode16(dtype, w).astype(np.float32).T
+        ws, y = N.DeviceBuffer(N.gemm_rows_workspace_bytes(2 * rows)), N.DeviceBuffer(tokens * rows * 4)
+        N.gemm_rows(dtype, dev(w[:rows]), rows, cols, tokens, dev(packed), out_f32=y, input_operand_order=True, workspace=ws)
+        assert rel_l2(y.numpy(np.float32).reshape(tokens, rows), exact[:, :rows]) <= 4e-6     # f32 sums of 2048 on both sides
+        if pairs:
+            out = N.DeviceBuffer(tokens * rows * 2)
+            N.gemm_rows(dtype, dev(w), rows, cols, tokens, dev(packed), epilogue=2, out16=out, input_operand_order=True, workspace=ws)
+            gate, up = exact[:, :rows], exact[:, rows:]
+            got = O.decode16(dtype, out.numpy(np.uint16, tokens * rows)).reshape(tokens, rows)
+            assert rel_l2(got, O.decode16(dtype, O.encode16(dtype, gate / (1 + np.exp(-gate)) * up))) <= 4e-3
