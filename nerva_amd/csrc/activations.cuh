@@ -8,6 +8,48 @@ namespace nv {
 __device__ __forceinline__ float sigmoid(float v) { return 1.0f / (1.0f + expf(-v)); }
 __device__ __forceinline__ float softplus(float v) { return v > 20.0f ? v : log1pf(expf(v)); }
 
+// e^x for |x| <= 89 (infinity from 88.73 on): a whole power of two and the hardware's power of the fraction, which keeps the bits that the product by log2(e)
+// would lose. (expf takes some more instructions for ranges that its callers here do not need.)
+__device__ __forceinline__ float exp_bounded(float x) {
+  constexpr float kLog2e = 1.44269504f, kRest = 1.92596299e-8f;   // log2(e) and what its f32 leaves of it
+  const float whole = rintf(x * kLog2e);
+  const float fraction = fmaf(x, kRest, fmaf(x, kLog2e, -whole));
+  return ldexpf(__builtin_amdgcn_exp2f(fraction), static_cast<int>(whole));
+}
+// v / (1 + e^(-slope v)), the quotient by a reciprocal and one correction of it: as far from 64 bits as with expf and a division
+// (over -8 .. 8 at most 1.5e-7 and 3.2e-8 on average, both), in less than half the instructions. Infinities, NaN and gates whose
+// exponential overflows come out as there, by the plain product: the correction would be NaN.
+__device__ __forceinline__ float gated(float v, float slope) {
+  const float d = 1.0f + exp_bounded(-fminf(fmaxf(slope * v, -89.0f), 89.0f));
+  const float r = __builtin_amdgcn_rcpf(d);
+  const float q = v * r, exact = fmaf(fmaf(-q, d, v), r, q);
+  return fmaxf(v, d) < INFINITY ? exact : q;
+}
+// Two results as one word, rounded by the hardware's conversions (a NaN stays one; its bits may differ from enc16's).
+template <uint32_t DT>
+__device__ __forceinline__ uint32_t enc16_pair(float lo, float hi) {
+  if constexpr (DT == kBF16) {
+    typedef __bf16 pair_t __attribute__((ext_vector_type(2)));
+    return __builtin_bit_cast(uint32_t, pair_t{static_cast<__bf16>(lo), static_cast<__bf16>(hi)});
+  } else {
+    return enc16<DT>(lo) | (static_cast<uint32_t>(enc16<DT>(hi)) << 16);
+  }
+}
+
+// e^z - 1 - z for z <= 0: the power series where the difference would cancel, else the difference.
+__device__ __forceinline__ float exp_remainder(float z) {
+  float s = fmaf(z, 1.0f / 3628800.0f, 1.0f / 362880.0f);
+  s = fmaf(z, s, 1.0f / 40320.0f);
+  s = fmaf(z, s, 1.0f / 5040.0f);
+  s = fmaf(z, s, 1.0f / 720.0f);
+  s = fmaf(z, s, 1.0f / 120.0f);
+  s = fmaf(z, s, 1.0f / 24.0f);
+  s = fmaf(z, s, 1.0f / 6.0f);
+  s = fmaf(z, s, 0.5f);
+  const float far = (exp_bounded(fmaxf(z, -87.0f)) - 1.0f) - z;
+  return z > -1.0f ? z * z * s : far;
+}
+
 // xIELU: with two learned numbers (p, q), above zero softplus(p) z^2 + z / 2, at and below it
 // (softplus(q) + 1/2) (e^z - 1 - z) + z / 2.
 struct XieluParams {
@@ -19,14 +61,14 @@ __device__ __forceinline__ XieluParams xielu_params(const uint16_t *pq) {
 }
 __device__ __forceinline__ float xielu(float z, const XieluParams &a) {
   const float low = fminf(z, 0.0f);
-  return (z > 0.0f ? a.above * z * z : a.below * (expm1f(low) - low)) + 0.5f * z;
+  return (z > 0.0f ? a.above * z * z : a.below * exp_remainder(low)) + 0.5f * z;
 }
 
 // Gated linear unit with bounds: the gate from above, the linear part on both sides and moved up by one.
 __device__ __forceinline__ float clamped_glu(float g, float u, float limit) {
   g = fminf(g, limit);
   u = fminf(fmaxf(u, -limit), limit);
-  return g * sigmoid(1.702f * g) * (u + 1.0f);
+  return gated(g, 1.702f) * (u + 1.0f);
 }
 
 // minGRU: gate and candidate from the current token alone (pre-activations with their biases added).

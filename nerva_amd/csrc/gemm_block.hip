@@ -239,16 +239,17 @@ __global__ __launch_bounds__(BW * kWave, NR == 1 ? 2 : 1) void gemm_block_kernel
 #undef NV_BLK_ITER
 
   // D layout: lane (n, q) holds rows q*4 .. q*4+3 of a row tile for token n of a token tile
+  const XieluParams act = epilogue_act<DT, EPI>(p);
   if (kslices == 1) {
 #pragma unroll
     for (int c = 0; c < kTiles; ++c) {
       const uint32_t t = c * 16u + n;
       if (t < T) {
         if constexpr (EPI == kGemmSwiglu) {
-          block_epilogue<DT, EPI>(p, t, trow[0] + q * 4u, acc[0][c], acc[NR - 1][c]);
+          block_epilogue<DT, EPI>(p, t, trow[0] + q * 4u, acc[0][c], acc[NR - 1][c], act);
         } else {
 #pragma unroll
-          for (int j = 0; j < NR; ++j) block_epilogue<DT, EPI>(p, t, trow[j] + q * 4u, acc[j][c], acc[j][c]);
+          for (int j = 0; j < NR; ++j) block_epilogue<DT, EPI>(p, t, trow[j] + q * 4u, acc[j][c], acc[j][c], act);
         }
       }
     }
@@ -293,7 +294,7 @@ __global__ __launch_bounds__(256) void gemm_block_finish_kernel(GemmRowsParams p
       up[3] += b.w;
     }
   }
-  block_epilogue<DT, EPI>(p, t, row, y, up);
+  block_epilogue<DT, EPI>(p, t, row, y, up, epilogue_act<DT, EPI>(p));
 }
 
 // The slice-adding launch of a residual projection with the RMSNorm of the result in the same pass: one workgroup
@@ -615,16 +616,17 @@ __global__ __launch_bounds__(PAIRS * 2 * kWave, 2) void gemm_wide_kernel(GemmRow
 #undef NV_WD_ITER
 
   // D layout: lane (n, q) holds rows q*4 .. q*4+3 of a row tile for token n of a token tile
+  const XieluParams act = epilogue_act<DT, EPI>(p);
   if (kslices == 1) {
 #pragma unroll
     for (int c = 0; c < kHalf; ++c) {
       const uint32_t t = (half * kHalf + c) * 16u + n;
       if (t < T) {
         if constexpr (EPI == kGemmSwiglu) {
-          block_epilogue<DT, EPI>(p, t, trow[0] + q * 4u, acc[0][c], acc[1][c]);
+          block_epilogue<DT, EPI>(p, t, trow[0] + q * 4u, acc[0][c], acc[1][c], act);
         } else {
 #pragma unroll
-          for (int j = 0; j < 2; ++j) block_epilogue<DT, EPI>(p, t, trow[j] + q * 4u, acc[j][c], acc[j][c]);
+          for (int j = 0; j < 2; ++j) block_epilogue<DT, EPI>(p, t, trow[j] + q * 4u, acc[j][c], acc[j][c], act);
         }
       }
     }
@@ -885,6 +887,7 @@ __global__ __launch_bounds__(8 * kWave, 2) void gemm_deep_kernel(GemmRowsParams 
 #undef NV_DP_BLOCK
 
   // D layout: lane (n, q) holds rows q*4 .. q*4+3 of a row tile for token n of a token tile
+  const XieluParams act = epilogue_act<DT, EPI>(p);
   if constexpr (EPI == kGemmSwiglu && TPW == 3) {
     // the up sums (row parts 2, 3) cross to the waves that hold their gate tiles (parts 0, 1, same token half)
     // through LDS, which everyone has finished with
@@ -905,7 +908,7 @@ __global__ __launch_bounds__(8 * kWave, 2) void gemm_deep_kernel(GemmRowsParams 
 #pragma unroll
         for (int j = 0; j < TPW; ++j)
           if (const uint32_t row = slot_row(TPW * rq + j) + q * 4u; kept(row))
-            block_epilogue<DT, EPI>(p, t, row, acc[j][c], meet[(j * 8 + c) * kWave]);
+            block_epilogue<DT, EPI>(p, t, row, acc[j][c], meet[(j * 8 + c) * kWave], act);
       }
     }
   } else if (kslices == 1) {
@@ -916,11 +919,11 @@ __global__ __launch_bounds__(8 * kWave, 2) void gemm_deep_kernel(GemmRowsParams 
         if constexpr (EPI == kGemmSwiglu) {
 #pragma unroll
           for (int j = 0; j < 2; ++j)
-            if (const uint32_t row = slot_row(4 * rq + j) + q * 4u; kept(row)) block_epilogue<DT, EPI>(p, t, row, acc[j][c], acc[j + 2][c]);
+            if (const uint32_t row = slot_row(4 * rq + j) + q * 4u; kept(row)) block_epilogue<DT, EPI>(p, t, row, acc[j][c], acc[j + 2][c], act);
         } else {
 #pragma unroll
           for (int j = 0; j < TPW; ++j)
-            if (const uint32_t row = slot_row(TPW * rq + j) + q * 4u; kept(row)) block_epilogue<DT, EPI>(p, t, row, acc[j][c], acc[j][c]);
+            if (const uint32_t row = slot_row(TPW * rq + j) + q * 4u; kept(row)) block_epilogue<DT, EPI>(p, t, row, acc[j][c], acc[j][c], act);
         }
       }
     }

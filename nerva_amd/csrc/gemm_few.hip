@@ -25,8 +25,7 @@ constexpr int kFewK = 64;        // columns of a block: one cache line a row
 constexpr int kFewRow = 20;      // floats between the tokens of a 16-row tile of sums in LDS (16 and padding)
 enum : int { kFewOperand = 0, kFewNorm = 1 };
 
-// Eight normalised values, rounded by the hardware's conversion (a NaN stays one, its bits may differ from enc16's): in every
-// workgroup all rows are rounded once more, and with enc16's integer steps that took 1.5 us of a launch.
+// Eight normalised values: in every workgroup all rows are rounded once more, and with enc16's integer steps that took 1.5 us of a launch.
 template <uint32_t DT>
 __device__ __forceinline__ u32x4_t few_norm8(const f32x4_t &a, const f32x4_t &b, float scale, const u32x4_t &gamma) {
   u32x4_t out;
@@ -36,12 +35,7 @@ __device__ __forceinline__ u32x4_t few_norm8(const f32x4_t &a, const f32x4_t &b,
     unpack2<DT>(gamma[i], g0, g1);
     const f32x4_t &v = i < 2 ? a : b;
     const float y0 = v[i % 2 * 2] * scale * g0, y1 = v[i % 2 * 2 + 1] * scale * g1;
-    if constexpr (DT == kBF16) {
-      typedef __bf16 pair_t __attribute__((ext_vector_type(2)));
-      out[i] = __builtin_bit_cast(uint32_t, pair_t{static_cast<__bf16>(y0), static_cast<__bf16>(y1)});
-    } else {
-      out[i] = enc16<DT>(y0) | (static_cast<uint32_t>(enc16<DT>(y1)) << 16);
-    }
+    out[i] = enc16_pair<DT>(y0, y1);
   }
   return out;
 }
@@ -207,7 +201,7 @@ __global__ __launch_bounds__(NW *kWave, NW / 4) void gemm_few_kernel(GemmRowsPar
     if constexpr (EPI == kGemmSwiglu) up += *reinterpret_cast<const f32x4_t *>(&red[w][1][out % TT][n][q * 4]);
   }
   const uint32_t row = row0 + j * 16u + q * 4u;
-  if (row < rows) block_epilogue<DT, EPI>(p, t, row, y, up);
+  if (row < rows) block_epilogue<DT, EPI>(p, t, row, y, up, epilogue_act<DT, EPI>(p));
 }
 
 // Waves: sixteen for the normalising launch (a block each), eight otherwise (a wave has its whole DEPTH in flight: 4096 x 1024

@@ -165,6 +165,7 @@ __global__ __launch_bounds__(kFW *kWave, TT == 8 && RT == 2 ? 1 : 2) void gemm_f
   }
 
   // D layout: lane (n, q) holds rows q*4 .. q*4+3 of a row tile for token n of a token tile
+  const XieluParams act = epilogue_act<DT, EPI>(p);
   const uint32_t wrows = EPI == kGemmSwiglu ? 2u * rows : rows;
   float *part = partials + static_cast<uint64_t>(blockIdx.y) * kFTokCap * wrows;
 #pragma unroll
@@ -183,9 +184,9 @@ __global__ __launch_bounds__(kFW *kWave, TT == 8 && RT == 2 ? 1 : 2) void gemm_f
         for (uint32_t r = 0; r < 4 && row + r < rows; ++r)
           p.out_f32[static_cast<uint64_t>(t) * rows + row + r] = acc[j][c][r] + (p.bias != nullptr ? dec16<DT>(p.bias[row + r]) : 0.0f);
       } else if constexpr (EPI == kGemmSwiglu) {
-        if (j == 0) block_epilogue<DT, EPI>(p, t, row, acc[0][c], acc[RT - 1][c]);
+        if (j == 0) block_epilogue<DT, EPI>(p, t, row, acc[0][c], acc[RT - 1][c], act);
       } else {
-        block_epilogue<DT, EPI>(p, t, row, acc[j][c], acc[j][c]);
+        block_epilogue<DT, EPI>(p, t, row, acc[j][c], acc[j][c], act);
       }
     }
   }

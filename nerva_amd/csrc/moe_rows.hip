@@ -347,8 +347,8 @@ __global__ __launch_bounds__(8 * kWave, 2) void expert_deep_kernel(Products p, u
         uint32_t o[2];
 #pragma unroll
         for (int r = 0; r < 2; ++r)
-          o[r] = enc16<DT>(clamped_glu(acc[i][j][2 * r], acc[i + 2][j][2 * r], p.limit)) |
-                 (static_cast<uint32_t>(enc16<DT>(clamped_glu(acc[i][j][2 * r + 1], acc[i + 2][j][2 * r + 1], p.limit))) << 16);
+          o[r] = enc16_pair<DT>(clamped_glu(acc[i][j][2 * r], acc[i + 2][j][2 * r], p.limit),
+                                clamped_glu(acc[i][j][2 * r + 1], acc[i + 2][j][2 * r + 1], p.limit));
         *reinterpret_cast<uint2 *>(p.act16 + to + row) = make_uint2(o[0], o[1]);
       } else {
         *reinterpret_cast<float4 *>(p.out + to + row) = make_float4(acc[i][j][0], acc[i][j][1], acc[i][j][2], acc[i][j][3]);

@@ -166,3 +166,27 @@ def test_blocks_of_fewer_tiles_than_their_layout(dtype, tokens):
             gate, up = exact[:, :rows], exact[:, rows:]
             got = O.decode16(dtype, out.numpy(np.uint16, tokens * rows)).reshape(tokens, rows)
             assert rel_l2(got, O.decode16(dtype, O.encode16(dtype, gate / (1 + np.exp(-gate)) * up))) <= 4e-3
+
+
+@pytest.mark.parametrize("tokens", [3, 70, 130, 300])
+def test_gates_of_any_size(tokens):
+    """A gate/up pair whose gates are small, large, past where e^-g is finite in 32 bits, infinite and NaN."""
+    rows, cols = 128, 2048
+    values = np.array([0.0, -0.0, 1e-20, -1e-20, 0.5, -0.5, 9.0, -9.0, 80.0, -80.0, 87.0, -88.0, 90.0, -104.0, 300.0, -300.0, 3e38, -3e38, np.inf,
+                       -np.inf, np.nan], np.float32)
+    gates = O.decode16(BF16, O.encode16(BF16, np.resize(values, rows)))
+    w = np.zeros((2 * rows, cols), np.float32)
+    w[:rows, 0], w[rows:, 0] = gates, 1.5
+    x = np.zeros((tokens, cols), np.float32)
+    x[:, 0] = 1.0
+    packed, _ = N.gemm_operand_order(O.encode16(BF16, x))
+    out, ws = N.DeviceBuffer(tokens * rows * 2), N.DeviceBuffer(N.gemm_rows_workspace_bytes(2 * rows))
+    N.gemm_rows(BF16, dev(O.encode16(BF16, w)), rows, cols, tokens, dev(packed), epilogue=2, out16=out, input_operand_order=True, workspace=ws)
+    got = O.decode16(BF16, out.numpy(np.uint16, tokens * rows)).reshape(tokens, rows)
+    with np.errstate(all="ignore"):
+        g = gates.astype(np.float64)
+        want = np.where(np.isfinite(g), g / (1 + np.exp(-np.clip(g, -700, 700))) * 1.5, np.where(g > 0, np.inf, np.nan))
+    for row in got:
+        assert np.array_equal(np.isnan(row), np.isnan(want)) and np.array_equal(np.isinf(row), np.abs(want) > 3.39e38)
+        fine = np.isfinite(want) & (np.abs(want) <= 3.39e38)
+        assert np.all(np.abs(row[fine] - want[fine]) <= 2.0 ** -8 * np.abs(want[fine]) + 2e-36)    # a rounding; results whose divisor is past 2^126 are 0
