@@ -190,3 +190,30 @@ def test_gates_of_any_size(tokens):
         assert np.array_equal(np.isnan(row), np.isnan(want)) and np.array_equal(np.isinf(row), np.abs(want) > 3.39e38)
         fine = np.isfinite(want) & (np.abs(want) <= 3.39e38)
         assert np.all(np.abs(row[fine] - want[fine]) <= 2.0 ** -8 * np.abs(want[fine]) + 2e-36)    # a rounding; results whose divisor is past 2^126 are 0
+
+
+@pytest.mark.parametrize("experts", [1, 3, 48, 64, 65, 129, 255, 256, 257])
+def test_routes_of_any_number_of_experts(experts):
+    """Both kernels of the route: ties, experts without a share, logits that are not finite, all experts chosen."""
+    rng = np.random.default_rng(experts)
+    for kind in range(5):
+        logits = rng.normal(0, 2, experts).astype(np.float32)
+        if kind == 1:
+            logits = np.round(logits)                     # ties
+        if kind == 2:
+            logits[:] = 0.5
+        if kind == 3:
+            logits[rng.random(experts) < 0.5] = -200.0    # probabilities of 0, the rest ahead of them
+        if kind == 4:
+            logits[rng.random(experts) < 0.3] = -np.inf
+            logits[0] = 1.0
+        for top in sorted({1, min(8, experts), min(64, experts)}):
+            for norm in (True, False):
+                ids, weights, _, _ = N.moe_route_softmax(logits, top, norm)
+                want_ids, want = O.moe_route_softmax(np.maximum(logits, -1e30), top, norm)    # (the oracle takes finite logits: e^-1e30 is 0 too)
+                assert ids.tolist() == want_ids.tolist(), (kind, top)
+                assert np.allclose(weights, want, rtol=2e-6, atol=1e-38), (kind, top)
+    logits = rng.normal(0, 2, experts).astype(np.float32)
+    logits[experts // 2] = np.nan     # no expert with a NaN has a share; places that nobody takes hold expert 0 with weight 0
+    ids, weights, _, _ = N.moe_route_softmax(logits, min(4, experts), False)
+    assert np.all(np.isfinite(weights)) and not np.any((ids == experts // 2) & (weights > 0))
