@@ -127,6 +127,9 @@ struct NervaHipHfDecodeSequenceSession : nv::RowScratch {
   nv::SamplerDev *sampler_dev = nullptr;
   uint64_t *sampler_keys = nullptr;
   hipEvent_t ev0 = nullptr, ev1 = nullptr;
+  char *stage = nullptr;          // two halves of pinned memory that results leave through (copy_out), and their events
+  uint64_t stage_half = 0;
+  hipEvent_t staged[2] = {nullptr, nullptr};
   // test hook: the next decode step is launched kernel by kernel and every intermediate vector is
   // copied behind the previous one into this caller-owned device buffer (step_trace_bytes)
   char *trace_buf = nullptr;
@@ -209,6 +212,8 @@ class PassTurn {
 hipError_t set_device_position(Session *s, uint32_t cursor, uint32_t prompt_count, uint32_t clear_fault);
 void destroy_session(Session *s);
 void fill_create_result(const Session *s, NervaHipHfDecodeSequenceSessionCreateResult *out);
+// `bytes` from device memory to the caller's memory, behind what the session's stream holds; there when the call returns.
+hipError_t copy_out(Session *s, void *dst, const void *src, uint64_t bytes);
 // Stream, the arena of s->weights->bytes (with_weights) + s->state_bytes, the pinned mirrors and the events.
 hipError_t allocate_session(Session *s, int32_t *failure_stage, bool with_weights);
 
