@@ -239,7 +239,7 @@ __global__ __launch_bounds__(BW * kWave, NR == 1 ? 2 : 1) void gemm_block_kernel
 #undef NV_BLK_ITER
 
   // D layout: lane (n, q) holds rows q*4 .. q*4+3 of a row tile for token n of a token tile
-  const XieluParams act = epilogue_act<DT, EPI>(p);
+  const XieluParams act = kslices == 1 ? epilogue_act<DT, EPI>(p) : XieluParams{};
   if (kslices == 1) {
 #pragma unroll
     for (int c = 0; c < kTiles; ++c) {
@@ -616,7 +616,7 @@ __global__ __launch_bounds__(PAIRS * 2 * kWave, 2) void gemm_wide_kernel(GemmRow
 #undef NV_WD_ITER
 
   // D layout: lane (n, q) holds rows q*4 .. q*4+3 of a row tile for token n of a token tile
-  const XieluParams act = epilogue_act<DT, EPI>(p);
+  const XieluParams act = kslices == 1 ? epilogue_act<DT, EPI>(p) : XieluParams{};
   if (kslices == 1) {
 #pragma unroll
     for (int c = 0; c < kHalf; ++c) {
@@ -887,7 +887,7 @@ __global__ __launch_bounds__(8 * kWave, 2) void gemm_deep_kernel(GemmRowsParams 
 #undef NV_DP_BLOCK
 
   // D layout: lane (n, q) holds rows q*4 .. q*4+3 of a row tile for token n of a token tile
-  const XieluParams act = epilogue_act<DT, EPI>(p);
+  const XieluParams act = kslices == 1 ? epilogue_act<DT, EPI>(p) : XieluParams{};
   if constexpr (EPI == kGemmSwiglu && TPW == 3) {
     // the up sums (row parts 2, 3) cross to the waves that hold their gate tiles (parts 0, 1, same token half)
     // through LDS, which everyone has finished with

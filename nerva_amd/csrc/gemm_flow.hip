@@ -165,7 +165,7 @@ __global__ __launch_bounds__(kFW *kWave, TT == 8 && RT == 2 ? 1 : 2) void gemm_f
   }
 
   // D layout: lane (n, q) holds rows q*4 .. q*4+3 of a row tile for token n of a token tile
-  const XieluParams act = epilogue_act<DT, EPI>(p);
+  const XieluParams act = slices == 1 ? epilogue_act<DT, EPI>(p) : XieluParams{};
   const uint32_t wrows = EPI == kGemmSwiglu ? 2u * rows : rows;
   float *part = partials + static_cast<uint64_t>(blockIdx.y) * kFTokCap * wrows;
 #pragma unroll
