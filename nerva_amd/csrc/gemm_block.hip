@@ -463,7 +463,11 @@ constexpr size_t wide_lds_bytes(int pairs, int tiles) {
   return static_cast<size_t>(kBSteps) * tiles * kWave * sizeof(u32x4_t) + static_cast<size_t>(pairs) * 2 * kBWTile * sizeof(uint16_t);
 }
 constexpr uint32_t wide_wg_rows(int epilogue, int pairs) { return (epilogue == kGemmSwiglu ? 16u : 32u) * pairs; }
-constexpr int wide_tiles(uint32_t tokens) { return static_cast<int>((tokens + 31u) / 32u * 2u); }   // 10 .. 16
+// Token tiles a launch fetches and multiplies, for it and for its estimate: 10 .. 16. xIELU's, of mixed stacks alone, has no variants
+// for fewer than all (at most of their widths blocks of up to 224 rows go to the kernel of 256-row tiles).
+constexpr int wide_tiles(int epilogue, uint32_t tokens) {
+  return epilogue == kGemmXielu ? kWTiles : static_cast<int>((tokens + 31u) / 32u * 2u);
+}
 inline int wide_pairs(int epilogue, uint32_t rows) {
   const int first = epilogue == kGemmSwiglu ? 4 : 3, second = 7 - first;
   return rows % wide_wg_rows(epilogue, first) == 0 ? first : rows % wide_wg_rows(epilogue, second) == 0 ? second : 0;
@@ -961,11 +965,10 @@ hipError_t launch_wide_tiles(const GemmRowsParams &p, float *partials, uint32_t 
   return hipGetLastError();
 }
 
-// (the activation of mixed stacks: all tiles)
 template <uint32_t DT, int EPI, int PAIRS>
 hipError_t launch_wide_pairs(const GemmRowsParams &p, float *partials, uint32_t kslices, hipStream_t stream) {
-  if constexpr (EPI != kGemmXielu) {
-    switch (wide_tiles(p.tokens)) {
+  if constexpr (wide_tiles(EPI, 1) != kWTiles) {
+    switch (wide_tiles(EPI, p.tokens)) {
       case 10: return launch_wide_tiles<DT, EPI, PAIRS, 10>(p, partials, kslices, stream);
       case 12: return launch_wide_tiles<DT, EPI, PAIRS, 12>(p, partials, kslices, stream);
       case 14: return launch_wide_tiles<DT, EPI, PAIRS, 14>(p, partials, kslices, stream);
@@ -1210,7 +1213,7 @@ uint32_t gemm_deep_slices(int epilogue, uint32_t rows, uint32_t cols, uint32_t t
 double gemm_wide_us(int epilogue, uint32_t rows, uint32_t cols, uint32_t tokens, uint32_t kslices) {
   const int pairs = wide_pairs(epilogue, rows);
   const uint32_t wg_rows = wide_wg_rows(epilogue, pairs);
-  return rounds_us(rows / wg_rows * kslices, cols / kBK / kslices, (pairs == 4 ? 2.05 : 1.75) * (0.05 + 0.95 * wide_tiles(tokens) / kWTiles)) +
+  return rounds_us(rows / wg_rows * kslices, cols / kBK / kslices, (pairs == 4 ? 2.05 : 1.75) * (0.05 + 0.95 * wide_tiles(epilogue, tokens) / kWTiles)) +
          partials_us(epilogue == kGemmSwiglu ? 2u * rows : rows, tokens, kslices);
 }
 

@@ -268,6 +268,13 @@ def test_wide_layers_take_the_streaming_kernels():
     s.destroy()
 
 
+@pytest.mark.parametrize("tokens", [129, 160, 200, 225])
+@pytest.mark.parametrize("width,ff", [(512, 1536), (768, 2304), (1024, 2048), (1536, 4608)])    # wave pairs; 256-row tiles
+def test_feed_forward_of_blocks_between_128_and_256_rows(width, ff, tokens):
+    cfg = M.config([M.mingru(width=64, ff=ff)], width=width)
+    check(cfg, M.weights(cfg, seed=width), tokens_of(cfg, tokens), [tokens], 0)
+
+
 def test_greedy_generation_through_the_session_loop():
     """start / advance / run in a 32-bit session: every token is the plain statement's choice, or within rounding of it."""
     cfg = M.config(EVERYTHING)
