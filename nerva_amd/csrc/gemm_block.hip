@@ -507,9 +507,13 @@ __global__ __launch_bounds__(PAIRS * 2 * kWave, 2) void gemm_wide_kernel(GemmRow
   uint16_t *park_at = wtile + half * kBWTile + q * kBRowStride + n * 8;
   const uint16_t *a_read = wtile + n * kBRowStride + q * 8;
   const char *xbase = reinterpret_cast<const char *>(p.x16) + static_cast<uint64_t>(k0 / 32u) * (kWTiles * kWave) * sizeof(u32x4_t);
-  const uint32_t xlane = lane * static_cast<uint32_t>(sizeof(u32x4_t));
-  // piece of 1 KiB that this wave's request i asks for: (K-step, tile) = piece / TILES, piece % TILES
+  // With all tiles the X block is one run, and a thread's requests lie a constant apart (as a sum of the wave's and the lane's part the
+  // offsets took twelve registers more, which spilled with three pairs: 240 rows of 6144 x 4096 31.7 us, so 36.5)
+  constexpr bool kRun = TILES == kWTiles;
+  const uint32_t xlane = (kRun ? threadIdx.x : lane) * static_cast<uint32_t>(sizeof(u32x4_t));
+  // else the piece of 1 KiB that this wave's request i asks for: (K-step, tile) = piece / TILES, piece % TILES
   const auto x_at = [&](int i) {
+    if constexpr (kRun) return static_cast<uint32_t>(i * kWThreads * sizeof(u32x4_t));
     const uint32_t piece = static_cast<uint32_t>(i) * (kWPairs * 2) + wave;
     return (piece / TILES * kWTiles + piece % TILES) * static_cast<uint32_t>(kWave * sizeof(u32x4_t));
   };

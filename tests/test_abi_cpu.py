@@ -330,6 +330,17 @@ def test_launch_shape_and_tuning_hooks_are_host_arithmetic():
     N.Device.reset_tuning()                     # a null name switches every override off
 
 
+def test_build_refuses_register_spills_in_kernels_of_large_tiles():
+    """A spill in the loop of a kernel that lives on its register tiles costs a fifth of it and shows in no result."""
+    from nerva_amd import build
+    remark = "gemm_block.hip:1:1: remark: Function Name: %s [-Rpass-analysis=kernel-resource-usage]\n" \
+             "gemm_block.hip:1:1: remark:     ScratchSize [bytes/lane]: %d [-Rpass-analysis=kernel-resource-usage]"
+    wide, other = "_ZN2nv12_GLOBAL__N_116gemm_wide_kernelILj1ELi0ELi3ELi16EEEvNS_14GemmRowsParamsEPf", "_ZN2nv16gemv_fast_kernelILj1EEEvNS_10GemvParamsE"
+    assert build._refused_kernels(remark % (wide, 0)) == []
+    assert build._refused_kernels(remark % (other, 52)) == []
+    assert len(build._refused_kernels(remark % (wide, 52))) == 1
+
+
 def test_build_refuses_register_spills_in_kernels_that_issue_loads_by_hand():
     """The build reads hipcc's resource-usage remarks: a kernel that requests data with inline-assembly loads
     must not use scratch memory (a spilled register may still be receiving its data)."""

@@ -133,6 +133,6 @@ def test_safe_wrapper_checks_every_tensor_before_the_pointer_cast():
     assert not re.search(r"\b(len\(\)|steps|self\.\w+) as u32", session), "unchecked size conversion"
     from nerva_amd import build
     script = open(os.path.join(CRATE, "build.rs")).read()
-    for kernel in build.HAND_ISSUED_LOADS:
+    for kernel in build.HAND_ISSUED_LOADS + build.REGISTER_TILES:
         assert '"%s"' % kernel in script
     assert "kernel-resource-usage" in script and "ScratchSize" in script and 'SUPPORTED_ARCH: &str = "gfx950"' in script
