@@ -1214,10 +1214,10 @@ uint32_t gemm_deep_slices(int epilogue, uint32_t rows, uint32_t cols, uint32_t t
   return deep_plan(epilogue, rows, cols, tokens, workspace_bytes).kslices;
 }
 
-double gemm_wide_us(int epilogue, uint32_t rows, uint32_t cols, uint32_t tokens, uint32_t kslices) {
-  const int pairs = wide_pairs(epilogue, rows);
+double gemm_wide_us(int epilogue, uint32_t rows, uint32_t cols, uint32_t tokens, uint32_t kslices, bool all_tiles) {
+  const int pairs = wide_pairs(epilogue, rows), tiles = all_tiles ? kWTiles : wide_tiles(epilogue, tokens);
   const uint32_t wg_rows = wide_wg_rows(epilogue, pairs);
-  return rounds_us(rows / wg_rows * kslices, cols / kBK / kslices, (pairs == 4 ? 2.05 : 1.75) * (0.05 + 0.95 * wide_tiles(epilogue, tokens) / kWTiles)) +
+  return rounds_us(rows / wg_rows * kslices, cols / kBK / kslices, (pairs == 4 ? 2.05 : 1.75) * (0.05 + 0.95 * tiles / kWTiles)) +
          partials_us(epilogue == kGemmSwiglu ? 2u * rows : rows, tokens, kslices);
 }
 

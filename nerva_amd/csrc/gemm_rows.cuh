@@ -117,8 +117,8 @@ hipError_t launch_gemm_block(uint32_t dtype, int epilogue, const GemmRowsParams 
 // (rows a multiple of 128, gate/up pairs of 64; cols a multiple of 512 per slice). launch_gemm_rows uses it by itself.
 uint32_t gemm_wide_slices(int epilogue, uint32_t rows, uint32_t cols, uint32_t tokens, uint64_t workspace_bytes);
 hipError_t launch_gemm_wide(uint32_t dtype, int epilogue, const GemmRowsParams &p, uint32_t kslices, hipStream_t stream);
-// Estimated time of that launch (gemm_rows_route), and of the one below.
-double gemm_wide_us(int epilogue, uint32_t rows, uint32_t cols, uint32_t tokens, uint32_t kslices);
+// Estimated time of that launch (gemm_rows_route) with the token tiles it takes or with all sixteen, and of the one below.
+double gemm_wide_us(int epilogue, uint32_t rows, uint32_t cols, uint32_t tokens, uint32_t kslices, bool all_tiles);
 double gemm_deep_us(int epilogue, uint32_t rows, uint32_t cols, uint32_t tokens, uint64_t workspace_bytes);
 // Blocks of 129..kGemmPassMaxTokens rows in operand order: the same for the kernel that takes 256 or 192 rows x 256
 // tokens per workgroup (rows a multiple of 8, cols of 64).

@@ -318,16 +318,22 @@ bool gemm_rows_supported(uint32_t rows, uint32_t cols, uint32_t tokens) {
 // faster one: 7168 x 5120 17.1 / 17.7 / 25.6 against 18.6 / 19.2 / 28.8). A gate/up pair in slices writes and reads two
 // rows of partial sums per output and gains only up to 64 rows (8192 x 2048 pairs 16.7 / 16.6 / 25.6 against
 // 15.9 / 16.9 / 28.7).
-// More: the kernel with wave pairs or the one for 256-row tiles, whichever the estimate has clearly ahead.
+// More: the kernel for 256-row tiles where its estimate is clearly ahead of the one with wave pairs in sixteen token tiles - and
+// does not fall 5 % behind it in the tiles that it takes: its own does not count that a CU of few workgroups is served faster (189
+// rows of 3584 x 14336 with the norm behind 46.9 us, in wave pairs 52.0, estimated 49.7 and 54.9; 194 of 4608 x 18432 58.9 and 69.8; 208 of 9216 x
+// 3072 31.5 and 32.9). Of 736 measured projections of 129 to 256 rows none is slower for it by 2 % than the choice
+// between the two with sixteen tiles always; by the estimates alone 26 were, up to 1.19 times.
 namespace {
 GemmRoute long_route(int epilogue, uint32_t rows, uint32_t cols, uint32_t tokens, uint64_t workspace_bytes) {
   if (tokens == 0) return GemmRoute{kGemmNone, 0};
   if (tokens > kGemmMaxTokens) {
     const uint32_t wide = tokens <= kGemmWideMaxTokens ? gemm_wide_slices(epilogue, rows, cols, tokens, workspace_bytes) : 0u;
     const uint32_t deep = gemm_deep_slices(epilogue, rows, cols, tokens, workspace_bytes);
-    if (wide != 0 && (deep == 0 || gemm_deep_us(epilogue, rows, cols, tokens, workspace_bytes) >
-                                       0.9 * gemm_wide_us(epilogue, rows, cols, tokens, wide)))
-      return GemmRoute{kGemmWide, wide};
+    if (wide != 0) {
+      const double deep_us = deep != 0 ? gemm_deep_us(epilogue, rows, cols, tokens, workspace_bytes) : 1e30;
+      if (deep_us > 0.9 * gemm_wide_us(epilogue, rows, cols, tokens, wide, true) || deep_us > 1.05 * gemm_wide_us(epilogue, rows, cols, tokens, wide, false))
+        return GemmRoute{kGemmWide, wide};
+    }
     return deep != 0 ? GemmRoute{kGemmDeep, deep} : GemmRoute{kGemmNone, 0};
   }
   const GemmBlockPlan block = gemm_block_plan(epilogue, rows, cols, tokens, workspace_bytes);
