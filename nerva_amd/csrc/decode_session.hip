@@ -1558,13 +1558,13 @@ hipError_t enqueue_batch_step(Session *lead, Session *const *seqs, uint32_t T,
   // follows as well (the next layer's attention norm, or the final norm): one launch less per layer
   const bool down_norms = gemm_rows_fuses_norm(kGemmResidual, H, I, T, tiles, lead->pgemm_ws_bytes);
   const bool o_norms = gemm_rows_fuses_norm(kGemmResidual, H, A, T, tiles, lead->pgemm_ws_bytes);   // likewise the MLP norm
-  // ... or the projection behind it reads the rows themselves
-  const bool qkv_norms = tiles != 0 && gemm_rows_norms_input(kGemmF32, A + 2 * KV, H, T, lead->pgemm_ws_bytes);
-  const bool gu_norms = !o_norms && tiles != 0 && gemm_rows_norms_input(kGemmSwiglu, I, H, T, lead->pgemm_ws_bytes);
   // where the q/k/v projection runs in a few K slices the attention adds them as it reads its inputs: no launch of
   // its own for that
   uint32_t qkv_slice_stride = 0;
   const uint32_t qkv_slices = gemm_rows_partial_slices(A + 2 * KV, H, T, tiles, lead->pgemm_ws_bytes, &qkv_slice_stride);
+  // ... or the projection behind it reads the rows themselves
+  const bool qkv_norms = tiles != 0 && qkv_slices == 0 && gemm_rows_norms_input(kGemmF32, A + 2 * KV, H, T, lead->pgemm_ws_bytes);
+  const bool gu_norms = !o_norms && tiles != 0 && gemm_rows_norms_input(kGemmSwiglu, I, H, T, lead->pgemm_ws_bytes);
   for (uint32_t l = 0; err == hipSuccess && l < lead->layers; ++l) {
     const LayerDev &w = lead->layer[l];
     if ((l == 0 || !down_norms) && !qkv_norms) err = launch_rmsnorm_rows(lead->dtype, lead->px, w.rms_attn, lead->eps, T, H, lead->pxn16, st, tiles);

@@ -1228,7 +1228,7 @@ double gemm_deep_us(int epilogue, uint32_t rows, uint32_t cols, uint32_t tokens,
 uint32_t gemm_rows_partial_slices(uint32_t rows, uint32_t cols, uint32_t tokens, uint32_t x_packed, uint64_t workspace_bytes,
                                   uint32_t *slice_stride) {
   if (x_packed == 0 || tokens > kBTokCap) return 0;
-  const uint32_t slices = gemm_rows_route(kGemmF32, rows, cols, tokens, workspace_bytes).kslices;   // (stride of either kernel's)
+  const uint32_t slices = gemm_rows_route(kGemmF32, rows, cols, tokens, workspace_bytes, true).kslices;   // (stride of either kernel's)
   if (slice_stride != nullptr) *slice_stride = kBTokCap * rows;
   return slices >= 2 && slices <= 4 ? slices : 0;
 }

@@ -232,11 +232,15 @@ uint32_t gemm_few_workgroups(int epilogue, uint32_t rows, uint32_t cols, uint32_
   return (rows + 15u) / 16u;
 }
 
-// What a CU fetches of W and X at the rate one is served at (54 KiB a us; with two token tiles 40), or W at the rate of memory.
+// What a CU fetches of W and X at the rate one is served at (52 KiB a us up to 8 tokens, 46 to 16, 44 with two token tiles) and 2.5 us
+// for the start of the second workgroup where there are more than CUs, or W at the rate of memory. (Plain projections and pairs of 2 to 32 rows
+// as measured: 0.73 to 1.04 times this for nine in ten. One rate of 54 up to 16 tokens and no second start fell short of 7168 x 5120 by a
+// fourth and of pairs of 5120 x 2048 by a third, at 9 to 16 tokens.)
 double gemm_few_us(int epilogue, uint32_t rows, uint32_t cols, uint32_t tokens) {
   const double pair = epilogue == kGemmSwiglu ? 2.0 : 1.0, tiles = tokens > 16 ? 2.0 : 1.0;
-  const double a_cu = ((rows + 15u) / 16u + 255u) / 256u * (pair + tiles) * 16.0 * cols * 2.0 / 1024.0;
-  return 3.0 + std::max(a_cu / (tokens > 16 ? 40.0 : 54.0), pair * rows * cols * 2.0 / 6.3e6);
+  const uint32_t rounds = ((rows + 15u) / 16u + 255u) / 256u;
+  const double a_cu = rounds * (pair + tiles) * 16.0 * cols * 2.0 / 1024.0;
+  return 3.0 + (rounds > 1 ? 2.5 : 0.0) + std::max(a_cu / (tokens > 16 ? 44.0 : tokens > 8 ? 46.0 : 52.0), pair * rows * cols * 2.0 / 6.3e6);
 }
 
 hipError_t launch_gemm_few(uint32_t dtype, int epilogue, const GemmRowsParams &p, hipStream_t stream) {

@@ -83,13 +83,14 @@ struct GemmRowsParams {
 // multiple of 16 a residual must not be added in place), cols % 2048 == 0 (each of the 8 waves walks
 // whole 256-column blocks), 1 <= tokens <= kGemmMaxTokens, 16-byte aligned w and x16.
 bool gemm_rows_supported(uint32_t rows, uint32_t cols, uint32_t tokens);
-// The kernel a block of `tokens` rows in operand order goes to, and its K slices (kGemmNone: not taken).
+// The kernel a block of `tokens` rows in operand order goes to, and its K slices (kGemmNone: not taken). reader_adds: a plain projection whose
+// slices' sums stay for their reader (GemmRowsParams::keep_partials), as far as they are few.
 enum GemmKernel : int { kGemmNone = 0, kGemmWaves, kGemmFew, kGemmBlock, kGemmFlow, kGemmWide, kGemmDeep };
 struct GemmRoute {
   GemmKernel kernel;
   uint32_t kslices;
 };
-GemmRoute gemm_rows_route(int epilogue, uint32_t rows, uint32_t cols, uint32_t tokens, uint64_t workspace_bytes);
+GemmRoute gemm_rows_route(int epilogue, uint32_t rows, uint32_t cols, uint32_t tokens, uint64_t workspace_bytes, bool reader_adds = false);
 inline bool gemm_rows_takes(int epilogue, uint32_t rows, uint32_t cols, uint32_t tokens, uint64_t workspace_bytes) {
   return gemm_rows_route(epilogue, rows, cols, tokens, workspace_bytes).kernel != kGemmNone;
 }

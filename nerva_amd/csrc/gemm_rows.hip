@@ -347,20 +347,26 @@ GemmRoute long_route(int epilogue, uint32_t rows, uint32_t cols, uint32_t tokens
 }
 }  // namespace
 
-// Up to 32 rows: the kernel without K slices where its estimate is ahead of the others', which stream W at 6.9 MB a us behind 4 us,
-// 7 with the launch that adds the slices. That launch also writes the norm behind a residual projection: half a us for that where
-// the kernel here can norm its own input, else the 3.5 of a launch. A plain projection's slices are often added by its reader, for
-// 1 us. (us, the others with that launch -> here, 6 rows: 6144 x 4096 15.5 -> 11.9 and without it 11.3, 4096 x 4096 12.1 -> 8.6,
-// 2048 x 8192 11.7 -> 12.4, 4096 x 12288 21.8 -> 18.0, 8192 x 2048 pairs 15.8 -> 12.3, 12288 x 4096 pairs 31.7 -> 32.9, 13824 x 5120
-// pairs 45 -> 50; 32 rows: 4096 x 1024 6.8 -> 4.1, 3072 x 1024 pairs 7.9 -> 5.6, 6144 x 4096 16.0 -> 18.2.)
-GemmRoute gemm_rows_route(int epilogue, uint32_t rows, uint32_t cols, uint32_t tokens, uint64_t workspace_bytes) {
+// Up to 32 rows: the kernel without K slices where its estimate is ahead of the others', which stream W at 6.9 MB a us behind 4 us (5
+// in slices of any length), 2.5 to 3 more with the launch that adds the slices. That launch also writes the norm behind a residual projection: 3/4
+// of a us for that where the kernel here can norm its own input, else the 3.5 of a launch. A plain projection's slices are added by its reader
+// where that is a batch step's attention, for 1 us (reader_adds). (us, the others with that launch -> here, 6 rows: 4096 x 1024 6.8 -> 3.7,
+// 2688 x 3328 9.3 -> 6.3, 1024 x 3072 with its norm 8.7 -> 8.3 and a launch less behind it, 3072 x 1024 pairs 8.0 -> 4.9; 32 rows: pairs of 2560 x 512 6.3 ->
+// 4.0. They stay at 16 rows of 7168 x 5120 17.5 (here 20.1), of 6144 x 4096 14.1 (15.0), of 4096 x 4096 with its norm 12.5 (13.4), of pairs of
+// 5120 x 2048 13.0 (13.7). 1220 projections of 2 to 32 rows take 19.29 ms together, without this kernel 20.24, with the better of the two
+// each time 18.80; one is 2 % slower than without it, none 3.)
+GemmRoute gemm_rows_route(int epilogue, uint32_t rows, uint32_t cols, uint32_t tokens, uint64_t workspace_bytes, bool reader_adds) {
   const GemmRoute route = long_route(epilogue, rows, cols, tokens, workspace_bytes);
   const int mode = tuning(kTuneGemmFew);
   if (route.kernel == kGemmNone || mode == 2 || gemm_few_workgroups(epilogue, rows, cols, tokens) == 0 || tuning(kTuneGemmBlockSlices) != 0 ||
       tuning(kTuneGemmBlockRowTiles) != 0 || tuning(kTuneGemmBlockOff) == 1)
     return route;
-  double others = (epilogue == kGemmSwiglu ? 2.0 : 1.0) * rows * cols * 2.0 / 6.9e6 + 4.0;
-  if (route.kslices > 1) others += epilogue == kGemmF32 ? 1.0 : epilogue == kGemmResidual ? (rows <= kGemmNormInputCols && tokens <= 16 ? 2.5 : -0.5) : 3.0;
+  double others = (epilogue == kGemmSwiglu ? 2.0 : 1.0) * rows * cols * 2.0 / 6.9e6 + (route.kernel == kGemmFlow ? 4.9 : 4.0);
+  if (route.kslices > 1) {
+    if (epilogue == kGemmF32) others += reader_adds ? 1.0 : 3.0;
+    else if (epilogue == kGemmResidual) others += rows <= kGemmNormInputCols && tokens <= 16 ? 2.5 : -0.75;
+    else others += 2.5;
+  }
   return mode == 1 || gemm_few_us(epilogue, rows, cols, tokens) < others ? GemmRoute{kGemmFew, 1} : route;
 }
 
@@ -374,13 +380,13 @@ hipError_t launch_gemm_rows(uint32_t dtype, int epilogue, const GemmRowsParams &
   // rows as they come: only the kernel of this file
   const uint64_t room = p.workspace != nullptr ? p.workspace_bytes : 0;
   GemmRoute route{kGemmNone, 0};
-  if (p.x_packed != 0) route = gemm_rows_route(epilogue, p.rows, p.cols, p.tokens, room);
+  if (p.x_packed != 0) route = gemm_rows_route(epilogue, p.rows, p.cols, p.tokens, room, p.keep_partials != 0);
   else if (gemm_rows_supported(p.rows, p.cols, p.tokens)) route = GemmRoute{kGemmWaves, 1};
   if (p.w == nullptr || (p.x16 == nullptr && p.norm_in == nullptr)) return hipErrorInvalidValue;
   if (route.kernel == kGemmNone) return hipErrorInvalidValue;
   if (!aligned16(p.w) || !aligned16(p.x16)) return hipErrorInvalidValue;
   if (p.norm_in != nullptr &&   // rows to be normalised only where the launch does that
-      (p.norm_in_gamma == nullptr || p.x_packed == 0 || !aligned16(p.norm_in) || !aligned16(p.norm_in_gamma) || p.norm_gamma != nullptr ||
+      (p.norm_in_gamma == nullptr || p.x_packed == 0 || !aligned16(p.norm_in) || !aligned16(p.norm_in_gamma) || p.norm_gamma != nullptr || p.keep_partials != 0 ||
        !gemm_rows_norms_input(epilogue, p.rows, p.cols, p.tokens, room)))
     return hipErrorInvalidValue;
   if ((epilogue == kGemmF32 || epilogue == kGemmResidual) && p.out_f32 == nullptr) return hipErrorInvalidValue;
