@@ -82,6 +82,7 @@ struct AttnParams {
   // Applies to z = 0 as well, and to a block of one token. With append = 1 every sequence's new row
   // is written to its cache by the launch itself.
   const AttnSeq *seqs;
+  uint32_t seq_blocks;         // with seqs: cache blocks of the longest of them (0: not known), which the kernel is chosen by
   // Block launches only: != 0 writes out16 in the multi-row GEMM's operand order (gemm_x_packed_index)
   // with this many token tiles, instead of [token][heads * head_dim] rows.
   uint32_t out_packed_tiles;
@@ -156,6 +157,9 @@ constexpr uint32_t kAttnSingleSplitBlocks = 20;
 // 5.7 / 8.2 / 11.0 / 14.2 us, six 6.9 / 11.3 / 12.5 / 14.2; 32 on 8, 16 sequences of 200 / 600 / 1000: 7.3 / 10.8 / 14.2 and 11.0 /
 // 13.8 / 15.6 in two).
 constexpr uint32_t kAttnBatchSingleSplitBlocks = 48;
+// Whether a batch step's launch takes the step kernel (attn_decode.hip), the longest sequence in `longest_blocks` cache blocks.
+constexpr uint32_t kAttnBatchStepBlocks = 128;
+bool attn_batch_in_step(uint32_t heads, uint32_t kv_heads, uint32_t head_dim, uint32_t sequences, uint32_t splits, uint32_t longest_blocks);
 __host__ __device__ __forceinline__ void attn_split_geometry(uint32_t pos, uint32_t splits, uint32_t single_blocks,
                                                              uint32_t &nblk, uint32_t &bps, uint32_t &active) {
   nblk = (pos + 1 + kKvBlockTokens - 1) / kKvBlockTokens;

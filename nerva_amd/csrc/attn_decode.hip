@@ -808,17 +808,11 @@ __global__ __launch_bounds__(kBlock) void attn_generic_kernel(AttnParams p) {
   }
 }
 
-// A batch step's sequences in one split each go to the step kernel while a CU has no more than one workgroup: its requests are on
-// their way in one burst where the block kernel, made for launches of thousands of workgroups (two a CU), takes one tile after the
-// other (32 sequences of 200 keys, 32 heads on 8: 9.2 -> 6.9 us).
-bool attn_batch_in_step(const AttnParams &p) {
-  return p.seqs != nullptr && p.append != 0 && p.splits == 1 && p.out_f32 == nullptr && static_cast<uint64_t>(p.kv_heads) * p.tokens <= 256u;
-}
-
 template <uint32_t DT, int HD, int G>
 hipError_t launch_fast(const AttnParams &p, hipStream_t stream) {
   const dim3 grid(p.kv_heads, p.splits, p.tokens > 1 ? p.tokens : 1);
-  if (attn_batch_in_step(p)) {
+  if (p.seqs != nullptr && p.append != 0 && p.out_f32 == nullptr &&
+      attn_batch_in_step(p.heads, p.kv_heads, p.head_dim, p.tokens, p.splits, p.seq_blocks)) {
     const dim3 seqs(p.kv_heads, 1, p.tokens);
     if (p.qkv_slices > 1) hipLaunchKernelGGL((attn_step_kernel<DT, HD, G, 2>), seqs, dim3(8 * kWave), 0, stream, p);
     else hipLaunchKernelGGL((attn_step_kernel<DT, HD, G, 1>), seqs, dim3(8 * kWave), 0, stream, p);
@@ -875,6 +869,19 @@ hipError_t launch_dt(const AttnParams &p, hipStream_t stream) {
 }
 
 }  // namespace
+
+// A batch step's sequences in one split each go to the step kernel while a CU has no more than one workgroup: its requests are on
+// their way in one burst where the block kernel, made for launches of thousands of workgroups (two a CU), takes one tile after the
+// other. Where they are as many as CUs and read heads of 128, that lasts while the burst is most of a launch: 32 sequences, 32 heads on 8, of 200 / 767 /
+// 2000 / 3000 / 8250 keys 9.2 / 20.8 / 45.9 / 65.0 / 167 us in the block kernel, 7.6 / 18.1 / 44.9 / 66.1 / 180 here (16, 40 and 56 heads on 8
+// the same within 3 %). With eight query heads a key head (its waves are half as many there; 64 on 8: 194 -> 179 at 8250 keys), heads of 64 (24 on
+// 8: 99 -> 89) and fewer workgroups (32 on 8, 24 sequences: 143 -> 128, 20: 137 -> 106, 8: 124 -> 82; 28 would be even) it is the faster one
+// at every length.
+bool attn_batch_in_step(uint32_t heads, uint32_t kv_heads, uint32_t head_dim, uint32_t sequences, uint32_t splits, uint32_t longest_blocks) {
+  const uint64_t workgroups = static_cast<uint64_t>(kv_heads) * sequences;
+  if (splits != 1 || workgroups > 256u || longest_blocks == 0) return false;
+  return longest_blocks <= kAttnBatchStepBlocks || workgroups <= 208u || head_dim == 64 || heads / kv_heads == 8;
+}
 
 uint32_t attn_resident_splits(uint32_t kv_heads) {
   static const uint32_t cus = [] {

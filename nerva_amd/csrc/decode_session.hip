@@ -1612,6 +1612,7 @@ hipError_t enqueue_batch_step(Session *lead, Session *const *seqs, uint32_t T,
     a.rope_token_stride = lead->head_dim;
     a.ws_token_stride = lead->pattn_ws_stride;
     a.seqs = lead->btable->seq;
+    a.seq_blocks = used_blocks;
     a.out_packed_tiles = tiles;
     a.append = 1;  // each sequence's K/V row goes into its own cache inside the attention launch
     if (err == hipSuccess) err = launch_attn_decode(lead->dtype, a, st);

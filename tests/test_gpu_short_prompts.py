@@ -111,10 +111,12 @@ def test_projections_that_norm_their_input(tuned, geom):
 # the batch step's attention: partial sums of q, k, v as they come (2048 wide, many sequences) or added; 1 to 8 query heads a key head
 @pytest.mark.parametrize("dtype,hidden,heads,kv,hd,count,length", [
     (BF16, 1024, 16, 8, 128, 6, 764),    # from one split a sequence to several
+    (BF16, 1024, 16, 8, 128, 32, 2046),  # a workgroup a CU and up to 16 tiles a wave in the step kernel, then the block kernel
+    (F16, 1024, 16, 8, 64, 32, 1100),    # the same in one split, heads of 64
     (BF16, 2048, 16, 8, 128, 32, 30), (F16, 512, 8, 4, 64, 9, 250), (BF16, 512, 14, 2, 64, 3, 129), (F16, 768, 10, 2, 128, 2, 513),
     (BF16, 512, 16, 2, 128, 5, 63), (BF16, 512, 16, 16, 64, 20, 15)])    # (the last: more workgroups than CUs)
 def test_batch_attention_matches_sequences_alone(dtype, hidden, heads, kv, hd, count, length):
-    """Contexts of a key, around a wave's four requested tiles, and across the lengths where the split factor changes."""
+    """Contexts of a key, around a wave's four requested tiles, and across the lengths where the split factor or the kernel changes."""
     vocab, layers, steps = 301, 2, 6
     weights, _ = random_model(dtype, hidden, heads, kv, hd, 1024, vocab, layers, count, 1e6, True, True)
     parent = N.DecodeSession.create(weights, length + 16, plan=N.WeightPlan.from_weights(weights))

@@ -58,3 +58,19 @@ def test_slices_that_their_reader_adds_cost_less():
     assert route(PLAIN, 6144, 2560, 4)[0] == FEW
     assert route(PLAIN, 6144, 2560, 4, reader_adds=True)[0] != FEW and route(PLAIN, 6144, 2560, 4, reader_adds=True)[1] > 1
     assert route(PLAIN, 4096, 1024, 6, reader_adds=True)[0] == FEW
+
+
+def test_long_batches_that_fill_the_chip_stay_with_the_block_kernel():
+    """32 sequences, 32 heads of 128 on 8, one split each: the step kernel is the faster one up to about 2500 keys (18.1 against 20.8
+    us at 767, 180 against 167 at 8250); with fewer workgroups, heads of 64 or eight query heads a key head it is at every length."""
+    rule = getattr(abi.load(), "_ZN2nv18attn_batch_in_stepEjjjjjj")
+    rule.restype, rule.argtypes = C.c_bool, [C.c_uint32] * 6
+
+    def step(heads, kv_heads, head_dim, sequences, keys, splits=1):
+        return rule(heads, kv_heads, head_dim, sequences, splits, (keys + 15) // 16)
+    for heads in (8, 16, 32, 40, 56):
+        assert step(heads, 8, 128, 32, 1) and step(heads, 8, 128, 32, 2048)
+        assert not step(heads, 8, 128, 32, 2049) and not step(heads, 8, 128, 32, 8264)
+    assert step(64, 8, 128, 32, 8264) and step(24, 8, 64, 32, 8264) and step(32, 8, 128, 24, 8264) and step(32, 4, 128, 32, 8264)
+    assert not step(32, 8, 128, 33, 100) and not step(32, 8, 128, 16, 100, splits=2)
+    assert not rule(32, 8, 128, 32, 1, 0)    # a launch that does not say how long its sequences are
