@@ -153,10 +153,14 @@ __host__ __device__ __forceinline__ bool attn_matrix_cores(uint32_t heads, uint3
 // (measured on the Qwen3-8B head shape: 64 keys 4.8 us against 12.7, 256 keys 6.5 against 8.2, 512 keys 10.0
 // against 8.0).
 constexpr uint32_t kAttnSingleSplitBlocks = 20;
-// The same for a batch step, whose splits merge behind a ticket (16 heads on 8, 6 sequences of 100 / 300 / 620 / 1000 keys: one split
-// 5.7 / 8.2 / 11.0 / 14.2 us, six 6.9 / 11.3 / 12.5 / 14.2; 32 on 8, 16 sequences of 200 / 600 / 1000: 7.3 / 10.8 / 14.2 and 11.0 /
-// 13.8 / 15.6 in two).
-constexpr uint32_t kAttnBatchSingleSplitBlocks = 48;
+// The same for a batch step, whose splits merge behind a ticket. us in a running session, 6 sequences, 16 heads on 8, 158 / 338 / 548 / 753 keys: in
+// six splits 12.6 / 14.4 / 14.9 / 15.6, in one 6.4 / 8.9 / 12.4 / 13.8; 8 heads of 64 on 2, 9 sequences: 9.8 / 10.2 / 10.1 / 10.4 and 5.2 / 6.8 /
+// 8.3 / 9.6. With up to three query heads of 128 a key head the merge is so short that few workgroups lose by one split before that: 4
+// sequences, 16 on 8, 548 / 628 / 708 / 753 keys 12.7 / 12.8 / 13.1 / 12.9 in eight splits, 11.8 / 13.0 / 13.4 / 13.6 in one; 2 sequences
+// 12.2 / 12.1 / 12.1 / 12.4 and 11.4 / 12.9 / 13.2 / 13.8.
+constexpr uint32_t kAttnBatchSingleSplitBlocks = 48, kAttnBatchSingleSplitFew = 36;
+// Cache blocks up to which the longest of a batch step's sequences gets one split.
+uint32_t attn_batch_single_split(uint32_t heads, uint32_t kv_heads, uint32_t head_dim, uint32_t sequences);
 // Whether a batch step's launch takes the step kernel (attn_decode.hip), the longest sequence in `longest_blocks` cache blocks.
 constexpr uint32_t kAttnBatchStepBlocks = 128;
 bool attn_batch_in_step(uint32_t heads, uint32_t kv_heads, uint32_t head_dim, uint32_t sequences, uint32_t splits, uint32_t longest_blocks);

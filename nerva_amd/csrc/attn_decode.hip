@@ -883,6 +883,10 @@ bool attn_batch_in_step(uint32_t heads, uint32_t kv_heads, uint32_t head_dim, ui
   return longest_blocks <= kAttnBatchStepBlocks || workgroups <= 208u || head_dim == 64 || heads / kv_heads == 8;
 }
 
+uint32_t attn_batch_single_split(uint32_t heads, uint32_t kv_heads, uint32_t head_dim, uint32_t sequences) {
+  return head_dim == 128 && heads / kv_heads <= 3 && static_cast<uint64_t>(kv_heads) * sequences <= 32u ? kAttnBatchSingleSplitFew : kAttnBatchSingleSplitBlocks;
+}
+
 uint32_t attn_resident_splits(uint32_t kv_heads) {
   static const uint32_t cus = [] {
     int device = 0, count = 0;

@@ -1541,7 +1541,7 @@ hipError_t enqueue_batch_step(Session *lead, Session *const *seqs, uint32_t T,
   uint32_t batch_splits = std::max<uint32_t>(1u, std::min<uint32_t>(attn_default_splits(lead->kv_heads, min_blocks),
                                                                    (256u + lead->kv_heads * T - 1) / (lead->kv_heads * T)));
   // ... while the longest context is more than one workgroup reads in the time that splits take to hand over
-  if (used_blocks <= kAttnBatchSingleSplitBlocks) batch_splits = 1;
+  if (used_blocks <= attn_batch_single_split(lead->heads, lead->kv_heads, lead->head_dim, T)) batch_splits = 1;
   if (const int want = tuning(kTuneBatchSplits); want >= 1 && want <= static_cast<int>(kAttnMaxSplits))
     batch_splits = std::min<uint32_t>(static_cast<uint32_t>(want), min_blocks);
   hipError_t err = hipMemcpyAsync(lead->btable, host, sizeof(BatchTable), hipMemcpyHostToDevice, st);

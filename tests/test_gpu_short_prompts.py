@@ -111,6 +111,7 @@ def test_projections_that_norm_their_input(tuned, geom):
 # the batch step's attention: partial sums of q, k, v as they come (2048 wide, many sequences) or added; 1 to 8 query heads a key head
 @pytest.mark.parametrize("dtype,hidden,heads,kv,hd,count,length", [
     (BF16, 1024, 16, 8, 128, 6, 764),    # from one split a sequence to several
+    (F16, 1024, 16, 8, 128, 4, 573),     # the same where splits come earlier
     (BF16, 1024, 16, 8, 128, 32, 2046),  # a workgroup a CU and up to 16 tiles a wave in the step kernel, then the block kernel
     (F16, 1024, 16, 8, 64, 32, 1100),    # the same in one split, heads of 64
     (BF16, 2048, 16, 8, 128, 32, 30), (F16, 512, 8, 4, 64, 9, 250), (BF16, 512, 14, 2, 64, 3, 129), (F16, 768, 10, 2, 128, 2, 513),
