@@ -844,7 +844,7 @@ hipError_t prefill_blocks(Session *s, uint32_t begin, uint32_t count, uint32_t c
       err = head_rows(s, begin + *wanted - first, run, out);
       s->head_run = run;
       if (err == hipSuccess)
-        err = copy_out(s, logits, s->blogits, static_cast<uint64_t>(run) * s->vocab * sizeof(float));
+        err = copy_out(s, logits, s->blogits, static_cast<uint64_t>(run) * s->vocab * sizeof(float), &out->sync_calls, false);
       out->d2h_bytes += static_cast<uint64_t>(run) * s->vocab * sizeof(float);
       logits += static_cast<uint64_t>(run) * s->vocab;
       wanted += run;
@@ -905,15 +905,18 @@ hipError_t allocate_session(Session *s, int32_t *failure_stage, bool with_weight
 // The runtime's own copy into memory that is not pinned takes 260 to 290 us for the 600 KB of a vocabulary's logits and a
 // millisecond for 3 MB; a copy into pinned memory 19 and 64, and from there to the caller's 15 and 105. So: pieces through two
 // pinned halves, one on its way while the other is copied on - the session's own, no larger than 512 KiB each. Where the caller's
-// memory is pinned (or managed) itself the copy goes straight there.
-hipError_t copy_out(Session *s, void *dst, const void *src, uint64_t bytes) {
+// memory is pinned (or managed) itself the copy goes straight there, and the host goes on with the next launches.
+hipError_t copy_out(Session *s, void *dst, const void *src, uint64_t bytes, uint64_t *waits, bool now) {
   hipPointerAttribute_t attr{};
   const bool direct = hipPointerGetAttributes(&attr, dst) == hipSuccess && attr.type != hipMemoryTypeUnregistered;
   (void)hipGetLastError();
   if (direct) {
     const hipError_t err = hipMemcpyAsync(dst, src, bytes, hipMemcpyDeviceToHost, s->stream);
-    return err == hipSuccess ? hipStreamSynchronize(s->stream) : err;
+    if (err != hipSuccess || !now) return err;
+    *waits += 1;
+    return hipStreamSynchronize(s->stream);
   }
+  *waits += 1;
   const uint64_t piece = std::min(s->stage_half, std::max<uint64_t>(kStageLeast, (bytes / 2 + 4095u) & ~uint64_t{4095}));
   uint64_t asked = 0, done = 0;
   hipError_t err = hipSuccess;
@@ -979,7 +982,7 @@ hipError_t prompt_tokens(Session *s, uint32_t begin, uint32_t end, const uint32_
     if (err == hipSuccess) err = head_sample(s, p.sample, head_blocks);
     out->kernel_launches += s->sampler.mode == kSamplerGreedy ? 2 : 3;
     if (err == hipSuccess && ahead != wanted_count) {
-      err = copy_out(s, logits + static_cast<uint64_t>(ahead) * s->vocab, s->logits, s->vocab * sizeof(float));
+      err = copy_out(s, logits + static_cast<uint64_t>(ahead) * s->vocab, s->logits, s->vocab * sizeof(float), &out->sync_calls, false);
       out->d2h_bytes += s->vocab * sizeof(float);
     }
     return err;
@@ -992,7 +995,7 @@ hipError_t prompt_tokens(Session *s, uint32_t begin, uint32_t end, const uint32_
   if (err == hipSuccess) err = enqueue_step(s, kPromptHeadStep, nullptr);
   if (err == hipSuccess) out->kernel_launches += step_launches(s, 0);
   if (err == hipSuccess && wanted_count != 0) {
-    err = copy_out(s, logits, s->logits, s->vocab * sizeof(float));
+    err = copy_out(s, logits, s->logits, s->vocab * sizeof(float), &out->sync_calls, false);
     out->d2h_bytes += s->vocab * sizeof(float);
   }
   return err;
@@ -2099,9 +2102,8 @@ int nerva_hip_session_extend(const NervaHipSessionExtendRequest *request, NervaH
     out->h2d_bytes = static_cast<uint64_t>(n) * sizeof(uint32_t);
   }
   const auto logits_out = [&](uint32_t i) {   // the last step's logits are wanted row i
-    err = copy_out(s, request->logits + static_cast<uint64_t>(i) * s->vocab, s->logits, s->vocab * sizeof(float));
+    err = copy_out(s, request->logits + static_cast<uint64_t>(i) * s->vocab, s->logits, s->vocab * sizeof(float), &out->sync_calls, false);
     out->d2h_bytes += s->vocab * sizeof(float);
-    out->sync_calls += 1;
   };
   if (n == 1 && request->residuals == nullptr) {
     if (err == hipSuccess) err = ensure_graph(s, decode_graph(s), out);
@@ -2512,7 +2514,8 @@ int nerva_hip_session_trace_next_step(NervaHipHfDecodeSequenceSession *s, void *
 
 int nerva_hip_session_read_logits(NervaHipHfDecodeSequenceSession *s, float *host_logits) {
   if (s == nullptr || host_logits == nullptr) return -1;
-  return copy_out(s, host_logits, s->logits, static_cast<uint64_t>(s->vocab) * 4) == hipSuccess ? 0 : -1;
+  uint64_t waits = 0;
+  return copy_out(s, host_logits, s->logits, static_cast<uint64_t>(s->vocab) * 4, &waits, true) == hipSuccess ? 0 : -1;
 }
 
 int nerva_hip_session_read_slots(NervaHipHfDecodeSequenceSession *s, uint32_t first, uint32_t count,

@@ -760,9 +760,9 @@ hipError_t nv::stack_prompt(Session *s, uint32_t begin, uint32_t end, const uint
       err = hipMemcpyAsync(s->pwant_rows, rows, count * sizeof(uint32_t), hipMemcpyHostToDevice, s->stream);
       if (err == hipSuccess) err = b.logits_of(s->pwant_rows, count, s->pwant_logits);
       if (err == hipSuccess)
-        err = copy_out(s, logits + static_cast<uint64_t>(next_wanted) * s->vocab, s->pwant_logits, static_cast<uint64_t>(count) * s->vocab * sizeof(float));
+        err = copy_out(s, logits + static_cast<uint64_t>(next_wanted) * s->vocab, s->pwant_logits, static_cast<uint64_t>(count) * s->vocab * sizeof(float),
+                       &out->sync_calls, true);
       out->d2h_bytes += static_cast<uint64_t>(count) * s->vocab * sizeof(float);
-      out->sync_calls += 1;
       next_wanted += count;
     }
     if (err == hipSuccess && first + b.tokens == end) {

@@ -1085,3 +1085,36 @@ def test_batch_step_of_sessions_with_their_own_steps_at_long_context():
     solo.destroy()
     for s in sessions[::-1]:
         s.destroy()
+
+
+@pytest.mark.parametrize("vocab", [301, 40001])    # a piece of the session's pinned memory each, and several
+def test_wanted_logits_in_ordinary_and_in_pinned_memory(vocab):
+    """Rows side by side, apart and the last one: each run waits once on its way to ordinary memory (and the call at its end); to
+    pinned memory nobody waits before the end. The same bits, with the last logits read back into either too."""
+    import ctypes as C
+    weights, _ = random_model(BF16, 512, 4, 2, 128, 1024, vocab, 2, 7)
+    s = N.DecodeSession.create(weights, 128)
+    tokens = np.random.default_rng(vocab).integers(0, vocab, 70).astype(np.uint32)
+    lib = N.abi.load()
+    hip = C.CDLL(lib._name)                                # (the runtime that the library is linked with)
+    for wanted, runs in ((list(range(10)) + [12] + list(range(20, 50)) + [69], 4), ([69], 1), ([67, 68, 69], 1), (range(0, 70, 7), 10)):
+        wanted = np.ascontiguousarray(list(wanted), np.uint32)
+        size = wanted.size * vocab * 4
+        pinned = C.c_void_p()
+        assert hip.hipHostMalloc(C.byref(pinned), C.c_size_t(size), 0) == 0
+        C.memset(pinned, 0xff, size)
+        assert s.release_sequence() == 0
+        rc, res, plain, _ = s.extend(tokens, wanted)
+        assert rc == 0 and res.sync_calls == runs + 1 and res.d2h_bytes >= size
+        assert s.release_sequence() == 0
+        req, res = N.abi.NervaHipSessionExtendRequest(), N.abi.NervaHipHfDecodeSequenceResult()
+        req.session, req.tokens, req.token_count = s.handle, tokens.ctypes.data, tokens.size
+        req.wanted, req.wanted_count, req.logits = wanted.ctypes.data, wanted.size, pinned.value
+        assert lib.nerva_hip_session_extend(C.byref(req), C.byref(res)) == 0 and res.sync_calls == 1
+        direct = np.frombuffer((C.c_char * size).from_address(pinned.value), np.float32).reshape(plain.shape)
+        assert np.all(np.isfinite(plain)) and np.array_equal(plain, direct)
+        C.memset(pinned, 0xff, vocab * 4)
+        assert lib.nerva_hip_session_read_logits(s.handle, pinned) == 0
+        assert np.array_equal(direct[0], s.logits())
+        assert hip.hipHostFree(pinned) == 0
+    s.destroy()
