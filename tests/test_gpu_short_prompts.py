@@ -56,8 +56,8 @@ def tuned():
 @pytest.mark.parametrize("rows,cols,tokens", [(16, 2048, 1), (20, 2048, 5), (48, 4096, 16), (4100, 2048, 17), (36, 6144, 32), (64, 10240, 15),
                                               (32, 14336, 31)])
 def test_few_rows_without_slices_match_the_oracle(tuned, dtype, rows, cols, tokens):
-    """Row counts off the grid of 16, 4 to 28 blocks a wave (all requested at once; a remainder; several rounds), one and two
-    token tiles: plain, with bias, residual and rounding, and gate/up pairs in operand order."""
+    """Row counts off the grid of 16, 4 to 28 blocks a wave in whole rounds of four (the operator takes no other widths: those are in
+    the next test), one and two token tiles: plain, with bias, residual and rounding, and gate/up pairs in rows and in operand order."""
     tuned("gemm_few", 1)
     rng = np.random.default_rng(rows + cols + tokens)
     w = O.encode16(dtype, rng.normal(0, 0.02, (2 * rows, cols)))
@@ -73,6 +73,11 @@ def test_few_rows_without_slices_match_the_oracle(tuned, dtype, rows, cols, toke
                 input_operand_order=True)
     got = y.numpy(np.float32).reshape(tokens, rows)
     assert rel_l2(got, O.decode16(dtype, O.encode16(dtype, (exact[:, :rows] + O.decode16(dtype, bias) + res).astype(np.float32)))) <= 4e-3
+    gate, up = exact[:, :rows], exact[:, rows:]
+    pairs = O.decode16(dtype, O.encode16(dtype, (gate / (1 + np.exp(-gate)) * up).astype(np.float32)))
+    out = N.DeviceBuffer(tokens * rows * 2)
+    N.gemm_rows(dtype, dw, rows, cols, tokens, dx, epilogue=2, out16=out, input_operand_order=True)
+    assert rel_l2(O.decode16(dtype, out.numpy(np.uint16, tokens * rows)).reshape(tokens, rows), pairs) <= 4e-3
     if rows % 32 == 0:
         out = N.DeviceBuffer(32 * rows * 2)
         N.gemm_rows(dtype, dw, rows, cols, tokens, dx, epilogue=2, out16=out, input_operand_order=True, output16_operand_order=True)
@@ -105,6 +110,40 @@ def test_projections_that_norm_their_input(tuned, geom):
         assert rel_l2(rows[0][0], rows[1][0]) <= E2E_REL_L2, n
         for got, want in zip(rows[0][1], rows[1][1]):    # of the first layer: the sums' order alone
             assert rel_l2(O.decode16(dtype, got), O.decode16(dtype, want)) <= 2e-3, n
+    s.destroy()
+
+
+# dtype, hidden, heads, kv, hd, inter: eight waves, four blocks of 64 columns of each in flight - of inter's 1 a wave or none, 6, 5 or 6, 6 or 7,
+# 10 or 11 (whole rounds of four and a remainder, unequal waves); of hidden's 1 or none, 2, 1 or 2, 1 or none, 2 or 3
+FEW = [(F16, 64, 2, 1, 64, 448), (BF16, 1024, 8, 4, 128, 3072), (BF16, 704, 6, 2, 64, 2624), (F16, 320, 4, 4, 64, 3520), (BF16, 1088, 6, 2, 128, 5248)]
+
+
+@pytest.mark.parametrize("geom", FEW, ids=str)
+def test_few_rows_of_any_width_match_the_oracle(tuned, geom):
+    """2 to 16 tokens of a sequence, 17 and 31, behind 20 others, through the kernel without K slices wherever it can run and as the
+    estimate has it: logits, and every layer's keys and values, against the oracle's token by token."""
+    dtype, hidden, heads, kv, hd, inter = geom
+    weights, model = random_model(dtype, hidden, heads, kv, hd, inter, 301, 2, hidden, 1e6, True, False)
+    tokens = np.random.default_rng(hidden).integers(0, 301, 51).astype(np.uint32)
+    oracle, want, rows = O.Context(model, 64), [], []
+    for i, token in enumerate(tokens):
+        oracle.forward_token(int(token), prompt_token=True)
+        want.append(oracle.logits())
+        rows.append([oracle.read_kv16(layer, i) for layer in range(2)])
+    s = N.DecodeSession.create(weights, 64)
+    for mode in (1, 0):
+        tuned("gemm_few", mode)
+        for n in (2, 3, 15, 16, 17, 31):
+            assert s.release_sequence() == 0
+            assert s.extend(tokens[:20])[0] == 0
+            rc, _, logits, _ = s.extend(tokens[20:20 + n], range(n))
+            assert rc == 0
+            assert max(rel_l2(g, w) for g, w in zip(logits, want[20:20 + n])) <= E2E_REL_L2, (mode, n)
+            for layer in range(2):
+                for which, got in enumerate(s.kv_range(layer, 0, 20 + n)):
+                    ref = np.stack([r[layer][which] for r in rows[:20 + n]])
+                    got = O.decode16(dtype, got).reshape(ref.shape)
+                    assert rel_l2(got, O.decode16(dtype, ref)) <= (2e-3 if layer == 0 else E2E_REL_L2), (mode, n, layer)
     s.destroy()
 
 
