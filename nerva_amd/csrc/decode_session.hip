@@ -863,7 +863,7 @@ hipError_t prefill_blocks(Session *s, uint32_t begin, uint32_t count, uint32_t c
 
 namespace nv {
 
-constexpr uint64_t kStageLeast = 64u << 10, kStageMost = 512u << 10;
+constexpr uint64_t kStageLeast = 16u << 10, kStageMost = 512u << 10, kStageFrom = 1u << 20;   // halves; bytes from which both are used (copy_out)
 
 hipError_t allocate_session(Session *s, int32_t *failure_stage, bool with_weights) {
   s->arena_bytes = s->weights->bytes + s->state_bytes;
@@ -885,7 +885,7 @@ hipError_t allocate_session(Session *s, int32_t *failure_stage, bool with_weight
   const uint64_t pinned_seq = (static_cast<uint64_t>(s->max_ctx) * (sizeof(Slot) + 4) + 256 + 255u) & ~uint64_t{255};
   const uint64_t pinned_table = (sizeof(BatchTable) + 255u) & ~uint64_t{255};
   const uint64_t pinned_slots = (static_cast<uint64_t>(NERVA_HIP_BATCH_MAX_BLOCK_TOKENS) * sizeof(Slot) + 255u) & ~uint64_t{255};
-  s->stage_half = std::min<uint64_t>(kStageMost, std::max<uint64_t>(kStageLeast, (static_cast<uint64_t>(s->vocab) * sizeof(float) + 4095u) & ~uint64_t{4095}));
+  s->stage_half = s->vocab * sizeof(float) >= kStageMost ? kStageMost : kStageLeast;
   s->pinned_bytes = pinned_seq + pinned_table + pinned_slots + 2 * s->stage_half;
   err = counted_host_malloc(reinterpret_cast<void **>(&s->pinned), s->pinned_bytes);
   if (err == hipSuccess) err = hipEventCreate(&s->ev0);
@@ -902,22 +902,27 @@ hipError_t allocate_session(Session *s, int32_t *failure_stage, bool with_weight
   return hipSuccess;
 }
 
-// The runtime's own copy into memory that is not pinned takes 260 to 290 us for the 600 KB of a vocabulary's logits and a
-// millisecond for 3 MB; a copy into pinned memory 19 and 64, and from there to the caller's 15 and 105. So: pieces through two
-// pinned halves, one on its way while the other is copied on - the session's own, no larger than 512 KiB each. Where the caller's
-// memory is pinned (or managed) itself the copy goes straight there, and the host goes on with the next launches.
+// The runtime's own copy into memory that is not pinned is the faster one between 16 KiB and 1 MiB: a call of 64 tokens with 8 rows of logits
+// apart, 32 KB / 128 KB / 608 KB a row, 371 / 453 / 920 us, through pinned memory 421 / 591 / 983. Smaller pieces arrive in pinned memory
+// by a kernel: 8 rows of 16 KB 298 us, with the runtime's copies 341. For larger ones the runtime pins the caller's pages (us behind a kernel into memory written
+// before / fresh: 1.2 MB 91 / 289, 3 MB 174 / 628, 4.9 MB 277 / 1064): those leave in pieces of 512 KiB through two pinned halves, the session's own,
+// one on its way while the other is copied on (78 / 219, 157 / 479, 244 / 770) - where a few rows are as much. Where the caller's memory is
+// pinned (or managed) itself the copy goes straight there, and the host goes on with the next launches.
 hipError_t copy_out(Session *s, void *dst, const void *src, uint64_t bytes, uint64_t *waits, bool now) {
-  hipPointerAttribute_t attr{};
-  const bool direct = hipPointerGetAttributes(&attr, dst) == hipSuccess && attr.type != hipMemoryTypeUnregistered;
-  (void)hipGetLastError();
-  if (direct) {
+  bool staged = bytes <= kStageLeast || (bytes >= kStageFrom && s->stage_half == kStageMost);
+  if (staged) {
+    hipPointerAttribute_t attr{};
+    staged = hipPointerGetAttributes(&attr, dst) != hipSuccess || attr.type == hipMemoryTypeUnregistered;
+    (void)hipGetLastError();
+  }
+  if (!staged) {
     const hipError_t err = hipMemcpyAsync(dst, src, bytes, hipMemcpyDeviceToHost, s->stream);
     if (err != hipSuccess || !now) return err;
     *waits += 1;
     return hipStreamSynchronize(s->stream);
   }
   *waits += 1;
-  const uint64_t piece = std::min(s->stage_half, std::max<uint64_t>(kStageLeast, (bytes / 2 + 4095u) & ~uint64_t{4095}));
+  const uint64_t piece = s->stage_half;
   uint64_t asked = 0, done = 0;
   hipError_t err = hipSuccess;
   for (uint32_t sent = 0, taken = 0; err == hipSuccess && done < bytes; ++taken) {
@@ -2514,8 +2519,8 @@ int nerva_hip_session_trace_next_step(NervaHipHfDecodeSequenceSession *s, void *
 
 int nerva_hip_session_read_logits(NervaHipHfDecodeSequenceSession *s, float *host_logits) {
   if (s == nullptr || host_logits == nullptr) return -1;
-  uint64_t waits = 0;
-  return copy_out(s, host_logits, s->logits, static_cast<uint64_t>(s->vocab) * 4, &waits, true) == hipSuccess ? 0 : -1;
+  if (hipStreamSynchronize(s->stream) != hipSuccess) return -1;
+  return hipMemcpy(host_logits, s->logits, static_cast<uint64_t>(s->vocab) * 4, hipMemcpyDeviceToHost) == hipSuccess ? 0 : -1;
 }
 
 int nerva_hip_session_read_slots(NervaHipHfDecodeSequenceSession *s, uint32_t first, uint32_t count,

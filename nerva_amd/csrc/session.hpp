@@ -213,7 +213,7 @@ hipError_t set_device_position(Session *s, uint32_t cursor, uint32_t prompt_coun
 void destroy_session(Session *s);
 void fill_create_result(const Session *s, NervaHipHfDecodeSequenceSessionCreateResult *out);
 // `bytes` from device memory to the caller's memory, behind what the session's stream holds; there when the call returns, for which it
-// waits (one more in *waits) - or, where that memory is pinned and `now` not asked for, when the stream gets there.
+// waits (one more in *waits) - or, where it enqueues a copy by the runtime and `now` is not asked for, when the stream gets there.
 hipError_t copy_out(Session *s, void *dst, const void *src, uint64_t bytes, uint64_t *waits, bool now);
 // Stream, the arena of s->weights->bytes (with_weights) + s->state_bytes, the pinned mirrors and the events.
 hipError_t allocate_session(Session *s, int32_t *failure_stage, bool with_weights);

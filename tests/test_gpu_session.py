@@ -1087,25 +1087,27 @@ def test_batch_step_of_sessions_with_their_own_steps_at_long_context():
         s.destroy()
 
 
-@pytest.mark.parametrize("vocab", [301, 40001])    # a piece of the session's pinned memory each, and several
-def test_wanted_logits_in_ordinary_and_in_pinned_memory(vocab):
-    """Rows side by side, apart and the last one: each run waits once on its way to ordinary memory (and the call at its end); to
-    pinned memory nobody waits before the end. The same bits, with the last logits read back into either too."""
+# rows through the session's pinned memory in one piece each, through the runtime's own copies, through both halves in up to 33 pieces
+@pytest.mark.parametrize("vocab,hidden,heads", [(301, 512, 4), (40001, 512, 4), (140001, 64, 2)])
+def test_wanted_logits_in_ordinary_and_in_pinned_memory(vocab, hidden, heads):
+    """Rows side by side, apart and the last one: a run that leaves through the session's memory waits once (and the call at its end); the
+    others, and all into pinned memory, wait for nobody before the end. The same bits, with the last logits read back into either too."""
     import ctypes as C
-    weights, _ = random_model(BF16, 512, 4, 2, 128, 1024, vocab, 2, 7)
+    weights, _ = random_model(BF16, hidden, heads, 1, 64, 448, vocab, 2, 7)
     s = N.DecodeSession.create(weights, 128)
     tokens = np.random.default_rng(vocab).integers(0, vocab, 70).astype(np.uint32)
     lib = N.abi.load()
     hip = C.CDLL(lib._name)                                # (the runtime that the library is linked with)
-    for wanted, runs in ((list(range(10)) + [12] + list(range(20, 50)) + [69], 4), ([69], 1), ([67, 68, 69], 1), (range(0, 70, 7), 10)):
-        wanted = np.ascontiguousarray(list(wanted), np.uint32)
+    for runs in ([range(10), [12], range(20, 50), [69]], [[69]], [[67, 68, 69]], [[i] for i in range(0, 70, 7)]):
+        wanted = np.concatenate([np.asarray(run, np.uint32) for run in runs])
+        waits = sum(len(run) * vocab * 4 <= 16384 or (len(run) * vocab * 4 >= 1 << 20 and vocab * 4 >= 524288) for run in runs)
         size = wanted.size * vocab * 4
         pinned = C.c_void_p()
         assert hip.hipHostMalloc(C.byref(pinned), C.c_size_t(size), 0) == 0
         C.memset(pinned, 0xff, size)
         assert s.release_sequence() == 0
         rc, res, plain, _ = s.extend(tokens, wanted)
-        assert rc == 0 and res.sync_calls == runs + 1 and res.d2h_bytes >= size
+        assert rc == 0 and res.sync_calls == waits + 1 and res.d2h_bytes >= size
         assert s.release_sequence() == 0
         req, res = N.abi.NervaHipSessionExtendRequest(), N.abi.NervaHipHfDecodeSequenceResult()
         req.session, req.tokens, req.token_count = s.handle, tokens.ctypes.data, tokens.size
