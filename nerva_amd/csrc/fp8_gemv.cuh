@@ -38,6 +38,7 @@ struct MoeRouteParams {
 
 hipError_t launch_fp8_gemv(const Fp8GemvParams &p, hipStream_t stream);
 hipError_t launch_moe_fp8(const MoeFp8Params &p, hipStream_t stream);
+bool moe_route_ranked(uint32_t experts, uint32_t top);   // whether it takes the kernel that counts instead of rounds of an argmax
 hipError_t launch_moe_route(const MoeRouteParams &p, hipStream_t stream);
 
 }  // namespace nv

@@ -866,10 +866,11 @@ __global__ __launch_bounds__(kBlock) void moe_route_kernel(MoeRouteParams p) {
   }
 }
 
-// The same for up to 256 experts, where rounds of an argmax over a workgroup - two barriers and a chain of exchanges each - are most of
-// the time: an expert's place among the chosen is the number of experts ahead of it, counted for all at once (an expert a lane, the
+// The same for up to 256 experts without rounds of an argmax over a workgroup - two barriers and a chain of exchanges each:
+// an expert's place among the chosen is the number of experts ahead of it, counted for all at once (an expert a lane, the
 // probabilities read from LDS four at a time by every lane alike). Maximum, exponentials and sum are worked out by every wave for
-// itself. The same sums in the same order, so the same bits (8 of 48: 10.6 -> 4.2 us).
+// itself. The same sums in the same order, so the same bits. What it takes grows with the experts, what the rounds take with the chosen
+// (moe_route_ranked has the line; 8 of 48: 10.7 -> 4.5 us).
 constexpr uint32_t kRankedExperts = 256;
 __global__ __launch_bounds__(kRankedExperts) void moe_route_ranked_kernel(MoeRouteParams p) {
   __shared__ __align__(16) float probs[kRankedExperts / kWave][kRankedExperts];
@@ -1088,13 +1089,20 @@ hipError_t launch_moe_fp8(const MoeFp8Params &p, hipStream_t stream) {
   return hipGetLastError();
 }
 
+// Rounds: 2.9 us, 8 ns an expert and 1.05 us for every chosen one behind the first; ranked: 2 us and 52 ns an expert (measured, rounds and ranked:
+// 1 of 16 3.0 / 2.8 us, 1 of 32 3.2 / 3.6, 2 of 32 4.3 / 3.6, 2 of 64 4.5 / 5.3, 4 of 64 6.7 / 5.4, 4 of 128 7.4 / 8.7, 8 of 128 11.7 / 8.6,
+// 8 of 192 12.7 / 12.0, 8 of 256 13.7 / 15.4, 64 of 256 84 / 16).
+bool moe_route_ranked(uint32_t experts, uint32_t top) {
+  return experts <= kRankedExperts && 0.044 * experts < 0.92 + (1.04 + 0.0008 * experts) * (top - 1u);
+}
+
 hipError_t launch_moe_route(const MoeRouteParams &p, hipStream_t stream) {
   if (p.logits == nullptr || p.expert_ids == nullptr || p.expert_weights == nullptr)
     return hipErrorInvalidValue;
   if (p.num_experts == 0 || p.num_experts > 1024 || p.top_k == 0 || p.top_k > p.num_experts ||
       p.top_k > 64)
     return hipErrorInvalidValue;
-  if (p.num_experts <= kRankedExperts)   // (a wave for every 64 experts; the work grows with their square)
+  if (moe_route_ranked(p.num_experts, p.top_k))   // (a wave for every 64 experts)
     hipLaunchKernelGGL(moe_route_ranked_kernel, dim3(1), dim3((p.num_experts + kWave - 1) / kWave * kWave), 0, stream, p);
   else
     hipLaunchKernelGGL(moe_route_kernel, dim3(1), dim3(kBlock), 0, stream, p);

@@ -85,3 +85,14 @@ def test_few_sequences_of_short_merges_split_earlier():
         assert rule(heads, 8, 128, sequences) == 36
     for heads, kv_heads, head_dim, sequences in ((16, 8, 128, 6), (32, 8, 128, 4), (28, 4, 128, 4), (16, 8, 64, 4), (8, 2, 64, 9)):
         assert rule(heads, kv_heads, head_dim, sequences) == 48
+
+
+def test_expert_routes_count_only_where_rounds_take_longer():
+    """Counting who is ahead grows with the experts, rounds of an argmax with the chosen: measured 3.6 us against 3.2 for 1 of 32, 8.6
+    and 5.1 for 2 of 128, 15.4 and 13.7 for 8 of 256; 4.5 and 10.7 for 8 of 48, 8.6 and 11.7 for 8 of 128."""
+    rule = getattr(abi.load(), "_ZN2nv16moe_route_rankedEjj")
+    rule.restype, rule.argtypes = C.c_bool, [C.c_uint32] * 2
+    for experts, top in ((32, 1), (48, 2), (64, 2), (128, 1), (128, 2), (128, 4), (256, 1), (256, 8), (257, 64), (1024, 64)):
+        assert not rule(experts, top), (experts, top)
+    for experts, top in ((1, 1), (8, 1), (8, 2), (16, 1), (16, 4), (32, 2), (48, 8), (64, 4), (64, 8), (128, 8), (192, 8), (256, 64)):
+        assert rule(experts, top), (experts, top)
