@@ -601,7 +601,10 @@ struct PromptShape {
 //                  146 x 0   512 x 0   88 x 512   512 x 512   1024 x 0   2048 x 0   4096 x 0   4096 x 4096   8 x 4096
 //   wide             20.8      38.6       29.3        44.5       64.7        116        241          607        23.5
 //   narrow           11.4      18.7       19.2        31.3       34.2         89        267          723        13
-// (wide in four or more splits where that is better, as it was before there were narrow ones; 64-wide heads go the same way.)
+// (wide in four or more splits where that is better, as it was before there were narrow ones.) Heads of 64, and of 128 with any number of query heads a
+// key head, go by the same constants, too high for heads of 64 on both sides: of 260 launches drawn over both, 1 to 8 query heads a key head, 2 to 4096
+// tokens behind 0 to 8000, none is slower than with wide workgroups alone, and all take 7.3 ms instead of 13.4 (64 wide, 4 of a key head: 18 tokens
+// 10.2 -> 5.9 us, 267 tokens 18.7 -> 9.8; 128 wide, 7 of a key head: 140 tokens 21.3 -> 11.2, 2902 tokens 152 -> 119).
 PromptShape shape_at(bool wide, uint32_t splits, uint32_t heads, uint32_t kv_heads, uint32_t head_dim, uint32_t position, uint32_t tokens) {
   const uint32_t group_tokens = group_tokens_of(wide, heads / kv_heads), groups = (tokens + group_tokens - 1) / group_tokens;
   constexpr uint32_t kKeys = kStepBlocks * kKvBlockTokens;
