@@ -24,6 +24,7 @@
 #include <algorithm>
 #include <string>
 #include <atomic>
+#include <utility>
 #include <vector>
 
 #include "layer_stack.hpp"
@@ -491,7 +492,10 @@ hipError_t ensure_graph(Session *s, int which, NervaHipHfDecodeSequenceResult *o
   hipGraph_t graph = nullptr;
   hipError_t err = hipStreamBeginCapture(s->stream, hipStreamCaptureModeThreadLocal);
   if (err != hipSuccess) return err;
+  // (a trace that is armed is the next step's: its copies would stay in the graph, and write to the caller's buffer ever after)
+  char *const trace = std::exchange(s->trace_buf, nullptr);
   hipError_t step_err = enqueue_step(s, which == 1 ? kPromptStep : kDecodeStep, nullptr);
+  s->trace_buf = trace;
   err = hipStreamEndCapture(s->stream, &graph);
   if (step_err != hipSuccess) err = step_err;
   size_t nodes = 0;

@@ -40,6 +40,21 @@ def test_every_link_of_every_step_matches_the_oracle(geom):
           % (steps - 1, ", ".join("%s %.1e" % kv_ for kv_ in sorted(worst.items())), e2e, chain_budget(layers)), flush=True)
 
 
+def test_a_step_captured_behind_an_armed_trace_holds_no_copies():
+    """The step's graph is captured by the first call that replays one, with a trace armed too: the replays after it are the
+    step's launches, without the trace's copies into a buffer that is gone by then."""
+    dtype, hidden, heads, kv, hd, inter, vocab, layers, theta, qk_norm, bias = GEOMETRIES[0]
+    weights, _ = random_model(dtype, hidden, heads, kv, hd, inter, vocab, layers, hidden, theta, qk_norm, bias)
+    s = N.DecodeSession.create(weights, 64)
+    assert s.start(np.arange(9, dtype=np.uint32))[0] == 0
+    assert s.advance(1)[0] == 0
+    rc, _, _, trace = s.traced_advance()
+    assert rc == 0 and trace is not None
+    rc, res, _ = s.advance(2)
+    assert rc == 0 and res.graph_replays == 2 and res.graph_nodes == 3 + 5 * layers
+    s.destroy()
+
+
 def test_links_at_qwen3_8b_widths_two_layers_full_vocabulary():
     """hidden 4096, 32 q / 8 kv heads x 128, MLP 12288, vocabulary 151936 (the real launch shapes of
     every GEMV, the LM head's looping launch with its candidates, 32 heads of attention), 2 layers,
