@@ -177,6 +177,7 @@ __device__ __forceinline__ void split16(float v, uint16_t &hi, uint16_t &mid, ui
 // off in the step kernel, 2.5e-7 with both.)
 template <uint32_t DT, int HD, int G>
 constexpr bool attn_scaled() { return DT == kF16 && attn_f32_shape(HD, G); }
+// (G may be rounded up to a power of two, with columns that no head has: SCALED then says what the real number asks for.)
 constexpr float kAttnWeightShift = 15.0f;
 __device__ __forceinline__ int attn_query_exponent(float largest) { return max(-126, min(126, 15 - __builtin_amdgcn_frexp_expf(largest))); }
 // Softmax arithmetic runs in base 2: the query is pre-scaled by log2(e) / sqrt(d), so scores, the
@@ -227,7 +228,7 @@ __device__ __forceinline__ void attn_load_tile(const AttnParams &p, uint32_t phy
 // One 16-token tile against the G query heads of the kv head (see attn_fast_body). F32_PARTS (see attn_step_kernel): queries
 // and probabilities in three parts, the third ones in operands of their own (columns 0 .. G-1). `down` (attn_scaled) undoes
 // the scale of the query of this lane's column.
-template <uint32_t DT, int HD, int G, bool QX_LDS, bool F32_PARTS = false>
+template <uint32_t DT, int HD, int G, bool QX_LDS, bool F32_PARTS = false, bool SCALED = attn_scaled<DT, HD, G>()>
 __device__ __forceinline__ void attn_tile(uint4 (&kreg)[HD / 32], uint4 (&vreg)[HD / 32], const uint4 (&qx)[HD / 32],
                                           const uint4 *qx_lds, uint32_t b,
                                           uint32_t n_keys, int col, int grp, bool splice, uint32_t new_row,
@@ -276,7 +277,7 @@ __device__ __forceinline__ void attn_tile(uint4 (&kreg)[HD / 32], uint4 (&vreg)[
     else c = mfma_k32<DT>(kreg[j], qx[j], c);
     if constexpr (F32_PARTS) c = mfma_k32<DT>(kreg[j], qx_third[j], c);
   }
-  constexpr bool kScaled = attn_scaled<DT, HD, G>();
+  constexpr bool kScaled = SCALED;
   float sc[4];
 #pragma unroll
   for (int r = 0; r < 4; ++r) {

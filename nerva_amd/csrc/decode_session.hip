@@ -211,7 +211,7 @@ bool layer_has_weights(const NervaHipHfDecodeChainLayer &l) {
 void nv::destroy_session(Session *s) {
   if (s == nullptr) return;
   if (s->stream) (void)hipStreamSynchronize(s->stream);
-  for (int i = 0; i < 3; ++i) {
+  for (int i = 0; i < 5; ++i) {
     if (s->exec[i]) (void)hipGraphExecDestroy(s->exec[i]);
     if (s->graph[i]) (void)hipGraphDestroy(s->graph[i]);
   }
@@ -243,6 +243,7 @@ SamplerParams session_sampler(Session *s, const float *logits) {
   sp.out.slots = s->slots;
   sp.out.cursor_rw = s->state;
   sp.out.fault = s->state + 3;
+  sp.out.step_rw = s->chain_context != 0 ? s->state + 2 : nullptr;
   sp.cursor = s->state;
   sp.max_steps = s->max_ctx;
   return sp;
@@ -439,6 +440,32 @@ hipError_t enqueue_step(Session *s, StepMode mode, StepProfiler *prof, int only 
   return hipSuccess;
 }
 
+// The same for a narrow model: its layers in one launch.
+hipError_t enqueue_chain_step(Session *s) {
+  const int spins = tuning(kTuneAttnMergeSpinLimit);
+  ChainLaunch c{};
+  c.model = s->chain_model_dev;
+  c.trace = s->trace_buf;
+  c.spin_limit = spins > 0 ? static_cast<uint32_t>(spins) : kAttnMergeSpinLimit;
+  hipError_t err = launch_step_chain(s->dtype, s->head_dim, s->chain_model, c, s->stream);
+  GemvParams p = head_launch(s, s->x);
+  const auto slot = [](uint64_t bytes) { return (bytes + 255u) & ~uint64_t{255}; };
+  char *trace = s->trace_buf;
+  if (trace != nullptr) {   // the launch has left every layer's vectors; the head's two are the last
+    s->trace_used = nerva_hip_session_step_trace_bytes(s);
+    trace += s->trace_used - slot(s->vocab * 4ull);
+    p.x16_dump = reinterpret_cast<uint16_t *>(trace - slot(s->hidden * 2ull));
+  }
+  uint32_t head_blocks = 0;
+  if (err == hipSuccess) err = launch_gemv(s->dtype, kProRmsNorm, kEpiArgmax, p, s->stream, nullptr, &head_blocks);
+  if (err == hipSuccess && trace != nullptr)
+    err = hipMemcpyAsync(trace, s->logits, s->vocab * sizeof(float), hipMemcpyDeviceToDevice, s->stream);
+  return err == hipSuccess ? head_sample(s, p.sample, head_blocks) : err;
+}
+hipError_t enqueue_graph_step(Session *s, int which) {
+  return which >= 3 ? enqueue_chain_step(s) : enqueue_step(s, which == 1 ? kPromptStep : kDecodeStep, nullptr);
+}
+
 // Steps are launched kernel by kernel instead of as graph replays when NERVA_HIP_EAGER_STEPS=1 is
 // set, or when the process runs under the ROCm profiler: with ROCm 7.2 a process traced by
 // rocprofv3 --kernel-trace died inside the HIP runtime at its first hipGraphLaunch (no message of its
@@ -465,9 +492,10 @@ bool eager_steps() {
   return eager;
 }
 
-// Kernel launches of one step (which = 0: decode step, 1: prompt step).
+// Kernel launches of one step (which = 0: decode step, 1: prompt step, 3 and 4: a decode step as a chain).
 uint64_t step_launches(const Session *s, int which) {
   if (s->stack != nullptr) return stack_step_launches(s);
+  if (which >= 3) return s->sampler.mode == kSamplerGreedy ? 3 : 4;
   // embed + (lm head + greedy finish | lm head + two sampler launches | cursor advance)
   const uint64_t fixed = which == 1 ? 2 : (s->sampler.mode == kSamplerGreedy ? 3 : 4);
   return fixed + 5ull * s->layers;
@@ -476,10 +504,14 @@ uint64_t step_launches(const Session *s, int which) {
 // Launch one step: graph replay, or the same kernels eagerly (tracing mode).
 hipError_t launch_step(Session *s, int which, NervaHipHfDecodeSequenceResult *out);
 
-// Index of the captured decode step for the active sampler.
-int decode_graph(const Session *s) { return s->sampler.mode == kSamplerGreedy ? 0 : 2; }
+// Index of the captured decode step for the active sampler, at a position.
+int decode_graph(const Session *s, uint32_t position) {
+  const bool greedy = s->sampler.mode == kSamplerGreedy;
+  if (position < s->chain_context) return greedy ? 3 : 4;
+  return greedy ? 0 : 2;
+}
 
-// graph index 0 / 2: decode step (greedy finish / sampler), 1: prompt step
+// graph index 0 / 2: decode step (greedy finish / sampler), 1: prompt step, 3 / 4: decode step as a chain
 hipError_t ensure_graph(Session *s, int which, NervaHipHfDecodeSequenceResult *out) {
   if (eager_steps()) return hipSuccess;
   if (s->exec[which] != nullptr) {
@@ -494,7 +526,7 @@ hipError_t ensure_graph(Session *s, int which, NervaHipHfDecodeSequenceResult *o
   if (err != hipSuccess) return err;
   // (a trace that is armed is the next step's: its copies would stay in the graph, and write to the caller's buffer ever after)
   char *const trace = std::exchange(s->trace_buf, nullptr);
-  hipError_t step_err = enqueue_step(s, which == 1 ? kPromptStep : kDecodeStep, nullptr);
+  hipError_t step_err = enqueue_graph_step(s, which);
   s->trace_buf = trace;
   err = hipStreamEndCapture(s->stream, &graph);
   if (step_err != hipSuccess) err = step_err;
@@ -516,17 +548,25 @@ hipError_t ensure_graph(Session *s, int which, NervaHipHfDecodeSequenceResult *o
   return hipSuccess;
 }
 
+// Those of `steps` decode steps from a position on.
+hipError_t ensure_graphs(Session *s, uint32_t position, uint32_t steps, NervaHipHfDecodeSequenceResult *out) {
+  const int first = decode_graph(s, position), last = decode_graph(s, position + steps - 1);
+  hipError_t err = ensure_graph(s, first, out);
+  if (err == hipSuccess && last != first) err = ensure_graph(s, last, out);
+  return err;
+}
+
 hipError_t launch_step(Session *s, int which, NervaHipHfDecodeSequenceResult *out) {
   if (s->trace_buf != nullptr && which != 1) {
     // armed by nerva_hip_session_trace_next_step: this one step runs kernel by kernel with copies
     s->trace_used = 0;
-    hipError_t err = enqueue_step(s, kDecodeStep, nullptr);
+    hipError_t err = enqueue_graph_step(s, which);
     s->trace_buf = nullptr;
     if (err == hipSuccess) out->kernel_launches += step_launches(s, which);
     return err;
   }
   if (eager_steps()) {
-    hipError_t err = enqueue_step(s, which == 1 ? kPromptStep : kDecodeStep, nullptr);
+    hipError_t err = enqueue_graph_step(s, which);
     if (err == hipSuccess)
       out->kernel_launches += step_launches(s, which);
     return err;
@@ -620,6 +660,7 @@ hipError_t reset_sequence(Session *s, const uint32_t *prompt_tokens, uint32_t pr
   // the words cleared here none of an earlier sequence's can ever match
   if (err == hipSuccess && s->attn_tagged != nullptr)
     err = hipMemsetAsync(s->attn_tagged, 0, attn_step_workspace_bytes(s->heads), s->stream);
+  if (err == hipSuccess && s->chain_word_bytes != 0) err = hipMemsetAsync(s->chain_model.words, 0, s->chain_word_bytes, s->stream);
   if (err == hipSuccess && s->stack_state_bytes != 0)   // a new sequence's recurrent state
     err = hipMemsetAsync(s->stack_state, 0, s->stack_state_bytes, s->stream);
   if (err == hipSuccess) {
@@ -1015,6 +1056,33 @@ hipError_t prompt_tokens(Session *s, uint32_t begin, uint32_t end, const uint32_
 // workspaces), the pinned host mirrors, the step modes. Shared by create and fork.
 // with_weights: one allocation holds the weights (s->weights->bytes, not allocated yet) and, behind
 // them, this session's state; it lives as long as any session uses the weights.
+// What a chain's launch reads of the model, once its weights have their places.
+hipError_t upload_chain(Session *s) {
+  if (s->chain_model_dev == nullptr) return hipSuccess;
+  ChainModel &m = s->chain_model;
+  m.emb = s->emb;
+  m.prompt = s->prompt;
+  m.slots = s->slots;
+  m.state = s->state;
+  m.fault = s->state + 3;
+  m.k_cache = s->kc;
+  m.v_cache = s->vc;
+  m.table = s->table;
+  m.rope_freq = s->theta > 0.0f ? s->rope_freq : nullptr;
+  m.x = s->x;
+  m.vocab = s->vocab;
+  m.max_steps = s->max_ctx;
+  m.block_count = s->block_count;
+  m.pair_gap = s->pair_gap;
+  m.eps = s->eps;
+  m.inv_hidden = 1.0f / static_cast<float>(s->hidden);
+  std::vector<ChainStage> stages(4 * s->layer.size());
+  for (size_t l = 0; l < s->layer.size(); ++l) chain_stages(m, s->head_dim, s->layer[l], reinterpret_cast<ChainStage(&)[4]>(stages[4 * l]));
+  hipError_t err = hipMemcpy(const_cast<LayerDev *>(m.layer), s->layer.data(), s->layer.size() * sizeof(LayerDev), hipMemcpyHostToDevice);
+  if (err == hipSuccess) err = hipMemcpy(const_cast<ChainStage *>(m.stage), stages.data(), stages.size() * sizeof(ChainStage), hipMemcpyHostToDevice);
+  return err == hipSuccess ? hipMemcpy(s->chain_model_dev, &m, sizeof(m), hipMemcpyHostToDevice) : err;
+}
+
 hipError_t setup_state(Session *s, int32_t *failure_stage, bool with_weights) {
   const uint64_t H = s->hidden, A = static_cast<uint64_t>(s->heads) * s->head_dim,
                  KV = static_cast<uint64_t>(s->kv_heads) * s->head_dim, I = s->intermediate, V = s->vocab,
@@ -1052,6 +1120,19 @@ hipError_t setup_state(Session *s, int32_t *failure_stage, bool with_weights) {
   const uint64_t off_attn_plan = c.take(attn_plan_bytes(kAttnMaxSplits));
   const uint64_t off_attn_tagged = c.take(attn_step_workspace_bytes(s->heads));
   const uint64_t off_sample_ws = c.take(sample_workspace_bytes());
+  const bool chain = tuning(kTuneStepChain) != 2 && tuning(kTuneAttnSplits) == 0 && chain_takes(s->layers, s->hidden, s->heads, s->kv_heads, s->head_dim, s->intermediate);
+  if (chain) {
+    ChainModel &m = s->chain_model;
+    m.layers = s->layers;
+    m.hidden = s->hidden;
+    m.heads = s->heads;
+    m.kv_heads = s->kv_heads;
+    m.ff = s->intermediate;
+    s->chain_word_bytes = chain_place(m, s->head_dim) * sizeof(uint64_t);
+  }
+  const uint64_t off_chain_words = c.take(s->chain_word_bytes);
+  const uint64_t off_chain_layers = c.take(chain ? L * sizeof(LayerDev) : 0), off_chain_model = c.take(chain ? sizeof(ChainModel) : 0),
+                 off_chain_stages = c.take(chain ? 4 * L * sizeof(ChainStage) : 0);
   // Rows of a prompt block (or a batch step)
   const uint64_t pB = kGemmDeepMaxTokens, widest = std::max<uint64_t>(H, A + 2 * KV);
   struct RowOffsets {
@@ -1151,6 +1232,13 @@ hipError_t setup_state(Session *s, int32_t *failure_stage, bool with_weights) {
   if (attn_matrix_cores(s->heads, s->kv_heads, s->head_dim))   // the plan serves the step kernel
     s->attn_plan = reinterpret_cast<uint32_t *>(s->arena + off_attn_plan);
   s->sample_ws = s->arena + off_sample_ws;
+  if (chain) {
+    s->chain_context = kChainContext;
+    s->chain_model.words = reinterpret_cast<uint64_t *>(s->arena + off_chain_words);
+    s->chain_model.layer = reinterpret_cast<LayerDev *>(s->arena + off_chain_layers);
+    s->chain_model.stage = reinterpret_cast<ChainStage *>(s->arena + off_chain_stages);
+    s->chain_model_dev = reinterpret_cast<ChainModel *>(s->arena + off_chain_model);
+  }
   const auto bind_rows = [&](RowScratch &rows, const RowOffsets &o, uint64_t gemm_bytes) {
     rows.px = reinterpret_cast<float *>(s->arena + o.px);
     rows.pr = reinterpret_cast<float *>(s->arena + o.pr);
@@ -1201,6 +1289,7 @@ hipError_t setup_state(Session *s, int32_t *failure_stage, bool with_weights) {
   if (err == hipSuccess) err = hipMemsetAsync(s->arena + off_attn_plan, 0, attn_plan_bytes(kAttnMaxSplits), s->stream);
   if (err == hipSuccess) err = hipMemsetAsync(s->arena + off_attn_tagged, 0, attn_step_workspace_bytes(s->heads), s->stream);
   if (err == hipSuccess) err = hipMemsetAsync(s->arena + off_sample_ws, 0, sample_workspace_bytes(), s->stream);
+  if (err == hipSuccess && chain) err = hipMemsetAsync(s->chain_model.words, 0, s->chain_word_bytes, s->stream);
   if (err == hipSuccess) err = hipMemsetAsync(s->arena + off_pattn_ws, 0, pB * pattn_ws_stride, s->stream);
   if (err == hipSuccess && L > 0) err = hipMemsetAsync(s->arena + off_attn_trace, 0, L * 32 * 8, s->stream);
   if (err == hipSuccess) err = hipMemsetAsync(s->arena + off_kc, 0, 2 * ((kv_half + 255) & ~uint64_t{255}), s->stream);
@@ -1408,6 +1497,7 @@ int create_impl(const NervaHipHfDecodeSequenceSessionCreateRequest *rq, bool syn
                            w16(lo[l].k_bias),   w16(lo[l].v_bias),  w16(lo[l].wo),
                            w16(lo[l].o_bias),   w16(lo[l].wgu),     w16(lo[l].wdown)};
   }
+  err = upload_chain(s);
 
   // ---- weights -------------------------------------------------------------
   out->failure_stage = 4;
@@ -1769,6 +1859,7 @@ int nerva_hip_hf_decode_sequence_session_fork_shared_weights(
   s->stack = parent->stack;
   hipError_t err = s->stack != nullptr ? stack_setup_state(s, &out->failure_stage, false) : setup_state(s, &out->failure_stage, false);
   uint64_t syncs = 1;
+  if (err == hipSuccess) err = upload_chain(s);
   if (err == hipSuccess && clone) {
     err = hipStreamSynchronize(parent->stream);
     syncs += 1;
@@ -1945,9 +2036,9 @@ int nerva_hip_hf_decode_sequence_batch_advance_one(const NervaHipHfDecodeSequenc
     Session *before = nullptr;
     for (uint32_t t = 0; err == hipSuccess && t < T; ++t) {
       Session *q = seqs[t];
-      err = ensure_graph(q, decode_graph(q), &scratch);
+      err = ensure_graph(q, decode_graph(q, q->cursor), &scratch);
       if (err == hipSuccess && before != nullptr) err = hipStreamWaitEvent(q->stream, before->ev1, 0);
-      if (err == hipSuccess) err = launch_step(q, decode_graph(q), &scratch);
+      if (err == hipSuccess) err = launch_step(q, decode_graph(q, q->cursor), &scratch);
       if (err == hipSuccess) err = hipEventRecord(q->ev1, q->stream);
       before = q;
       if (err == hipSuccess)
@@ -2115,8 +2206,8 @@ int nerva_hip_session_extend(const NervaHipSessionExtendRequest *request, NervaH
     out->d2h_bytes += s->vocab * sizeof(float);
   };
   if (n == 1 && request->residuals == nullptr) {
-    if (err == hipSuccess) err = ensure_graph(s, decode_graph(s), out);
-    if (err == hipSuccess) err = launch_step(s, decode_graph(s), out);
+    if (err == hipSuccess) err = ensure_graph(s, decode_graph(s, begin), out);
+    if (err == hipSuccess) err = launch_step(s, decode_graph(s, begin), out);
     if (err == hipSuccess && request->wanted_count != 0) logits_out(0);
   } else if (s->stack != nullptr) {
     if (err == hipSuccess)
@@ -2182,11 +2273,11 @@ int nerva_hip_hf_decode_sequence_session_advance(const NervaHipHfDecodeSequenceS
   fill_header(s, out, request->steps, seed);
 
   hipError_t err = hipSuccess;
-  if (run_count != 0) err = ensure_graph(s, decode_graph(s), out);
+  if (run_count != 0) err = ensure_graphs(s, s->cursor, run_count, out);
   const uint64_t allocs_before = allocation_count();
   if (err == hipSuccess && run_count != 0) err = hipEventRecord(s->ev0, s->stream);
   for (uint32_t step = 0; err == hipSuccess && step < run_count; ++step) {
-    err = launch_step(s, decode_graph(s), out);
+    err = launch_step(s, decode_graph(s, s->cursor + step), out);
     // With a stop token the host looks at each token so that it can stop launching
     // (session_api_lifecycle.inc.cu:1206-1234); without one the loop never syncs.
     if (err == hipSuccess && s->has_eos != 0) {
@@ -2270,11 +2361,11 @@ int nerva_hip_hf_decode_sequence_session_run(const NervaHipHfDecodeSequenceSessi
   hipError_t err = set_sampler(s, request->sampler);   // session_api_lifecycle.inc.cu:770
   if (err == hipSuccess) err = reset_sequence(s, request->prompt_tokens, P, out);
   // the decode-step graph walks every position, prompt included (session_api_lifecycle.inc.cu:748-990)
-  if (err == hipSuccess) err = ensure_graph(s, decode_graph(s), out);
+  if (err == hipSuccess) err = ensure_graphs(s, 0, context_steps, out);
   const uint64_t allocs_before = allocation_count();
   if (err == hipSuccess) err = hipEventRecord(s->ev0, s->stream);
   for (uint32_t step = 0; err == hipSuccess && step < context_steps; ++step) {
-    err = launch_step(s, decode_graph(s), out);
+    err = launch_step(s, decode_graph(s, step), out);
   }
   if (err == hipSuccess) err = hipEventRecord(s->ev1, s->stream);
   const uint64_t slots_bytes = static_cast<uint64_t>(context_steps) * sizeof(Slot);

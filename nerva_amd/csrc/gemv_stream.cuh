@@ -51,6 +51,7 @@ struct SampleParams {
   uint32_t *cursor_rw;
   uint32_t *token_out;     // optional: plain token output (operator entry point)
   const uint32_t *fault;   // optional: a word that a kernel of this step sets when a bounded wait of its gave up
+  uint32_t *step_rw;       // optional: the step number, which the next step's launches derive their tags from
 };
 
 // One lane: hands the step's token out - plain output word and/or slot[pos] in the reference's
@@ -70,6 +71,7 @@ __device__ __forceinline__ void publish_token(const SampleParams &s, uint32_t to
     slot.host_copied = 0;
     s.slots[pos] = slot;
     *s.cursor_rw = pos + 1u;
+    if (s.step_rw != nullptr) *s.step_rw += 1u;
   }
 }
 

@@ -173,6 +173,7 @@ enum TuningKnob : int {
   kTuneGemmFew,              // multi-row GEMM of up to 32 rows: 1 = the kernel without K slices wherever it can run, 2 = nowhere
   kTuneMixedAttentionWide,   // mixed stacks: 2 = every attention layer through the general kernel
   kTuneLatentAttentionWide,  // mixed stacks: 2 = every layer of attention over latents through the general kernel
+  kTuneStepChain,            // narrow models: 2 = a step's layers never in one launch (read at session create)
   kTuneKnobs
 };
 int tuning(TuningKnob knob);

@@ -12,15 +12,11 @@
 #include "gemv_stream.cuh"
 #include "runtime_state.hpp"
 #include "sampler.cuh"
+#include "step_chain.cuh"
 
 namespace nv {
 
 using Slot = NervaHipSyntheticTokenSlot;
-
-struct LayerDev {
-  const uint16_t *rms_attn, *rms_mlp, *wqkv, *q_norm, *k_norm, *q_bias, *k_bias, *v_bias, *wo, *o_bias,
-      *wgu, *wdown;
-};
 
 enum StepMode { kDecodeStep = 0, kPromptStep = 1, kPromptHeadStep = 2 };
 enum LaunchKind { kLEmbed = 0, kLQkv, kLAttn, kLO, kLGateUp, kLDown, kLHead, kLAdvance, kLKinds };
@@ -104,10 +100,15 @@ struct NervaHipHfDecodeSequenceSession : nv::RowScratch {
   uint32_t *host_state = nullptr;    // 64 words
   // captured steps: 0 decode step with the greedy finish, 1 prompt step, 2 decode step with the
   // temperature / top-k / top-p sampler (its parameters live in device memory, so one capture
-  // serves every such configuration)
-  hipGraph_t graph[3] = {nullptr, nullptr, nullptr};
-  hipGraphExec_t exec[3] = {nullptr, nullptr, nullptr};
-  uint64_t graph_nodes[3] = {0, 0, 0};
+  // serves every such configuration), 3 and 4 the two decode steps with their layers in one launch
+  hipGraph_t graph[5] = {};
+  hipGraphExec_t exec[5] = {};
+  uint64_t graph_nodes[5] = {};
+  // narrow models: positions below chain_context step with their layers in one launch (step_chain.cuh); 0: never
+  uint32_t chain_context = 0;
+  nv::ChainModel chain_model{};      // ... what that launch works on, and its copy on the device
+  nv::ChainModel *chain_model_dev = nullptr;
+  uint64_t chain_word_bytes = 0;
   // prompt blocks: up to prefill_pass_tokens prompt tokens per pass through the layers (weights streamed
   // once per pass on the matrix cores), in a long prompt prefill_long_tokens; false = one prompt step per token
   bool block_prefill = false;

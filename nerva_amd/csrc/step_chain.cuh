@@ -1,0 +1,64 @@
+// A decode step's layers in one launch, for narrow models (step_chain.hip).
+#pragma once
+
+#include "nv_common.cuh"
+#include "nerva_hip_api.h"
+
+namespace nv {
+
+// One decoder layer's weights in device memory.
+struct LayerDev {
+  const uint16_t *rms_attn, *rms_mlp, *wqkv, *q_norm, *k_norm, *q_bias, *k_bias, *v_bias, *wo, *o_bias,
+      *wgu, *wdown;
+};
+
+// One projection of one layer, as a launch's workgroups walk it: one read through the scalar path.
+struct alignas(64) ChainStage {
+  const uint16_t *w;
+  const uint16_t *vec;         // the norm's weights in front of it, or the o projection's bias, or null
+  uint32_t cols, chunks, groups, units;
+  uint32_t unit_bytes, row_bytes, up_bytes;   // from unit to unit, from a unit's first row to its second, from its first two to its last two
+  uint32_t in_at, in_words, out_at;           // 8-byte words of ChainModel::words
+  uint32_t whole, spare;                      // every request of a row is a whole one, and every group has four
+};
+// What a model's chain works on, in device memory (a session's, written once).
+struct ChainModel {
+  const LayerDev *layer;       // device memory, [layers]
+  const ChainStage *stage;     // ..., [layers][4]
+  const uint16_t *emb;
+  const uint32_t *prompt;
+  const NervaHipSyntheticTokenSlot *slots;
+  const uint32_t *state;       // position, prompt tokens, step number (the words' tags derive from it)
+  uint32_t *fault;
+  uint16_t *k_cache, *v_cache;
+  const uint32_t *table;
+  const float *rope_freq;      // null: no rotation
+  float *x;                    // [hidden]: the last layer's output
+  uint64_t *words;             // what the workgroups hand to each other, cleared when a sequence starts
+  uint32_t layers, hidden, heads, kv_heads, ff, vocab, max_steps, block_count, pair_gap;
+  uint32_t at_x, at_qkv, at_attn, at_part, at_r, at_ff;   // places in `words` (chain_place)
+  float eps, inv_hidden;
+};
+
+// Cache blocks up to which a key head's attention stays with one workgroup: 61 / 101 / 151 keys in one 65.5 / 66 / 68 us a step, in several
+// 67.9 / 68.3 / 68.6; 201 keys 73 and 68.6.
+constexpr uint32_t kChainSingleBlocks = 8;
+constexpr uint32_t kChainMaxHidden = 1024, kChainMaxIn = 4096, kChainMaxSplits = 16;
+// Tokens of context up to which steps run as a chain: with 4000 keys, sixteen splits of sixteen blocks, it is 0.87 to 0.99 of the launches' time.
+constexpr uint32_t kChainContext = 4096;
+// Whether a model's steps can run as a chain.
+bool chain_takes(uint32_t layers, uint32_t hidden, uint32_t heads, uint32_t kv_heads, uint32_t head_dim, uint32_t ff);
+uint32_t chain_workgroups(uint32_t hidden, uint32_t heads, uint32_t kv_heads, uint32_t head_dim, uint32_t ff);
+// 8-byte words of ChainModel::words, whose places it fills in.
+uint64_t chain_place(ChainModel &model, uint32_t head_dim);
+// The walks of a layer's four projections.
+void chain_stages(const ChainModel &model, uint32_t head_dim, const LayerDev &layer, ChainStage (&stage)[4]);
+struct ChainLaunch {
+  const ChainModel *model;     // device memory
+  char *trace;                 // test hook: every link's vector, 256 bytes apart (step_trace_bytes), or null
+  uint32_t spin_limit;         // polls after which a wait gives up
+};
+// `model`: the same on the host.
+hipError_t launch_step_chain(uint32_t dtype, uint32_t head_dim, const ChainModel &model, const ChainLaunch &p, hipStream_t stream);
+
+}  // namespace nv

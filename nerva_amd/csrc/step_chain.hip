@@ -1,0 +1,781 @@
+// A decode step's layers in one launch, for narrow models.
+//
+// What bounds a step of a narrow model is neither its bytes (5.8 MB a layer at 512 x 1376: a microsecond) nor its arithmetic but the
+// five launches a layer, 3.4 to 4.2 us each, of which a boundary and the first accesses behind it are most. Here the workgroups stay for the
+// whole step and hand vectors to each other as words of (value, tag), which a reader polls until the tag is its own, and the
+// weights of the next projection are requested before the wait for its input begins: 12 us a layer instead of 19. us a step, 12 / 100 / 260 / 1000
+// / 4000 keys, launches and chain, head and sampler (10 us) included:
+//   4 layers  512 x 1376,  8 heads of  64 on 4:   81 /  85 /  88 /  92 /  92     61 /  66 /  68 /  69 /  79
+//   8 layers  512 x 1792,  4 heads of 128 on 2:  158 / 163 / 178 / 173 / 176    116 / 125 / 130 / 132 / 156
+//   6 layers  640 x 1600,  5 heads of 128 on 5:  131 / 135 / 147 / 142 / 149    115 / 122 / 127 / 129 / 147
+//   8 layers  768 x 2304, 12 heads of  64 on 4:  175 / 178 / 188 / 191 / -      188 / 197 / 207 / 208 / -      (not taken)
+// (in a stack of 13.8 MB a layer the requests, which a launch of 128 workgroups has too few of in flight, cost what the boundaries did).
+//
+// A layer is five hand-overs: x -> qkv -> attention -> r = x + o -> activation -> x = r + down. Every workgroup reads the whole of x, of
+// the attention's output, of r and of the activation (the residual rows and the norms come with them); a key head's q, k
+// and v go to the workgroups of its attention alone. Contexts of more than kChainSingleBlocks blocks are split over workgroups, whose partial
+// sums others merge: a sixth hand-over. What a layer costs beyond them is instructions, one wave's at a time - requests 0.4 to 0.8 us a
+// projection, its products 0.6 to 1.0, a norm 0.4, the attention 2.8 -, so everything about a projection that can be known before is in
+// one table entry (ChainStage).
+//
+// The workgroups wait for each other, so all of a launch have to be resident: 128 of four waves at most, with registers and
+// LDS for two a CU, of which four launches at once - one a hardware queue - fit the chip together. A wait that runs out is
+// an error as in the decode attention: the fault word is set and the rest of the launch waits for nothing.
+//
+// No word is written before all its readers have read what it held. Every workgroup has rows of o, of gate and up and of down, and writes
+// them behind its own reads of what came before; so when x is whole, everyone has read the activation and the r of that layer, and the
+// attention's output and the x before it.
+#include <algorithm>
+#include <type_traits>
+
+#include "attn_tile.cuh"
+#include "gemv_stream.cuh"
+#include "step_chain.cuh"
+
+namespace nv {
+
+namespace {
+
+using namespace attn;
+
+constexpr int kThreads = 256, kWaves = 4;
+constexpr uint32_t kMaxWorkgroups = 128;
+constexpr int kRing = 4, kGroup = 4;          // request groups in flight a wave, 16-byte requests of a lane in each
+constexpr uint32_t kSplitTiles = 4;           // cache blocks of a split: one a wave (two a wave: 600 keys 72 us a step instead of 69)
+
+// The model through the scalar path. `fresh` forgets what has been read of it, so that a stage holds what it uses and no more: held over the
+// whole loop, the model's and the layer's words and the addresses made of them take more registers than there are.
+typedef const __attribute__((address_space(4))) ChainModel *Model;
+__device__ __forceinline__ void fresh(Model &m) { asm volatile("" : "+s"(m)); }
+__device__ __forceinline__ uint32_t fresh_thread() {
+  uint32_t t = threadIdx.x;
+  asm volatile("" : "+v"(t));
+  return t;
+}
+// Member number `which` of a layer's weights.
+enum : int { kRmsAttn = 0, kRmsMlp, kWqkv, kQNorm, kKNorm, kQBias, kKBias, kVBias, kWo, kOBias, kWgu, kWdown };
+static_assert(sizeof(LayerDev) == 12 * sizeof(void *), "twelve pointers");
+__device__ __forceinline__ const uint16_t *weight(Model m, uint32_t layer, int which) {
+  typedef const uint16_t *Pointer;
+  typedef const __attribute__((address_space(4))) Pointer *Constant;
+  return ((Constant)(reinterpret_cast<uint64_t>(m->layer)))[layer * 12 + which];
+}
+
+// Elements through a uniform base and a 32-bit offset in bytes: one address instruction each.
+template <typename T>
+__device__ __forceinline__ T *at_bytes(T *base, uint32_t bytes) {
+  typedef typename std::conditional<std::is_const<T>::value, const char, char>::type Byte;
+  return reinterpret_cast<T *>(reinterpret_cast<Byte *>(base) + bytes);
+}
+__device__ __forceinline__ void store_word(uint64_t *at, uint32_t payload, uint32_t tag) {
+  __hip_atomic_store(at, (static_cast<uint64_t>(tag) << 32) | payload, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+
+// The wave's share of n words that lie together, i * 256 + thread, until every tag is this launch's.
+struct Waiter {
+  uint32_t limit;     // 0: a wait has run out, nothing is waited for any more
+  uint32_t *fault;
+  __device__ __forceinline__ bool again(bool ok, uint32_t &spins, uint32_t tag) {
+    if (__all(ok) || limit == 0) return false;
+    if (++spins <= limit) return true;
+    limit = 0;
+    if ((threadIdx.x & (kWave - 1)) == 0) __hip_atomic_store(fault, tag, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    return false;
+  }
+};
+template <int N>
+__device__ __forceinline__ void poll_words(const uint64_t *src, uint32_t n, uint32_t tag, Waiter &wait, uint64_t (&v)[N]) {
+  uint32_t spins = 0;
+  bool ok;
+  const uint32_t thread = fresh_thread();
+  do {
+#pragma unroll
+    for (int i = 0; i < N; ++i) v[i] = load_tagged(at_bytes(src, min(thread + i * kThreads, n - 1) * 8u));
+    ok = true;
+#pragma unroll
+    for (int i = 0; i < N; ++i) ok = ok && tag_is(v[i], tag);
+  } while (wait.again(ok, spins, tag));
+}
+// Packed 16-bit pairs into LDS.
+template <int N>
+__device__ __forceinline__ void take_pairs_n(const uint64_t *src, uint32_t n, uint32_t tag, Waiter &wait, uint16_t *dst) {
+  uint64_t v[N];
+  poll_words<N>(src, n, tag, wait, v);
+  const uint32_t thread = fresh_thread();
+#pragma unroll
+  for (int i = 0; i < N; ++i)
+    if (thread + i * kThreads < n) reinterpret_cast<uint32_t *>(dst)[thread + i * kThreads] = static_cast<uint32_t>(v[i]);
+}
+__device__ __forceinline__ void take_pairs(const uint64_t *src, uint32_t n, uint32_t tag, Waiter &wait, uint16_t *dst) {
+  if (n <= 3u * kThreads) take_pairs_n<3>(src, n, tag, wait, dst);
+  else take_pairs_n<kChainMaxIn / 2 / kThreads>(src, n, tag, wait, dst);
+}
+
+// A projection as a wave walks it. A workgroup's units lie together - every workgroup has some - and go round its waves. A unit is four
+// rows, sixteen lanes each (128 columns a request) - of a gate/up pair of matrices two gate rows and their two up rows -, or one row
+// (512 columns a request) where rows are few. It takes `groups` request groups; four are in flight. One walk, and one piece of code, for all
+// four projections: a kernel with a copy for each (60 KB, a layer's loop through nearly all of it) spent most of its time on fetching instructions.
+enum : uint32_t { kQkv = 0, kO = 1, kGateUp = 2, kDown = 3, kStages = 4 };
+typedef const __attribute__((address_space(4))) ChainStage *StageAt;
+__device__ __forceinline__ ChainStage read_stage(Model m, uint32_t at) {
+  const StageAt s = (StageAt)(reinterpret_cast<uint64_t>(m->stage)) + at;
+  return ChainStage{s->w,          s->vec,       s->cols,     s->chunks, s->groups,   s->units,  s->unit_bytes,
+                    s->row_bytes, s->up_bytes, s->in_at, s->in_words, s->out_at, s->whole,  0u};
+}
+struct Walk {
+  uint32_t total;
+  uint32_t first;         // the wave's first unit; the others are kWaves apart
+  uint32_t unit, group;   // requested next: unit, place in it
+  uint32_t row;           // of the lane: bytes from the unit's first row
+  uint32_t col, last;     // ... of its piece of a request, in bytes, and of a row's last piece
+  // The request that the lane's row begins with: rows begin at different ones and wrap, so that what the chip asks for at any one time
+  // lies on all memory channels (rows are a multiple of their interleave apart: without it 1024 wide requests took 2.5 times as long).
+  uint32_t turn;
+  uint32_t shift;         // log2 of a request's bytes of a row
+};
+__device__ __forceinline__ void request_group(Walk &k, const ChainStage &d, uint4 (&dst)[kGroup]) {
+  const char *const base = reinterpret_cast<const char *>(d.w) + static_cast<uint64_t>(k.unit) * d.unit_bytes;
+  uint32_t c = k.turn + k.group * kGroup;
+#pragma unroll
+  for (int u = 0; u < kGroup; ++u) {   // (requests that the row does not have: its last pieces once more)
+    c = min(c, c - d.chunks);
+    // (kept in the caches: a small model's weights are still there when the next step asks for them, 62.5 -> 60.8 us at 512 x 1376)
+    dst[u] = *reinterpret_cast<const uint4 *>(base + (k.row + min((c << k.shift) + k.col, k.last)));
+    ++c;
+  }
+  if (++k.group == d.groups) {
+    k.group = 0;
+    k.unit += kWaves;
+  }
+}
+__device__ __forceinline__ void walk_begin(Walk &k, const ChainStage &d, bool rows, uint32_t log_grid, uint4 (&ring)[kRing][kGroup]) {
+  const uint32_t lane = fresh_thread() & (kWave - 1), wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
+  const uint32_t begin = blockIdx.x * d.units >> log_grid, end = (blockIdx.x + 1) * d.units >> log_grid;
+  k.first = k.unit = begin + wave;
+  k.total = k.first < end ? (end - k.first + kWaves - 1) / kWaves * d.groups : 0u;
+  k.group = 0;
+  k.row = rows ? 0u : (lane / 16 & 1u) * d.row_bytes + (lane / 32) * d.up_bytes;
+  k.col = (rows ? lane : lane % 16) * 16;
+  k.last = d.cols * 2 - 16;
+  k.shift = rows ? 10 : 8;
+  k.turn = wave + (rows ? 0u : lane / 16 * (d.chunks / 4));
+  k.turn = min(k.turn, k.turn - d.chunks);
+  k.turn = min(k.turn, k.turn - d.chunks);
+  k.turn = min(k.turn, k.turn - d.chunks);
+  k.turn = min(k.turn, k.turn - d.chunks);
+  // (what the ring held is over: without this, requests under a condition would keep it alive from one walk to the next, through the attention)
+#pragma unroll
+  for (int f = 0; f < kRing; ++f)
+#pragma unroll
+    for (int u = 0; u < kGroup; ++u) asm volatile("" : "=v"(ring[f][u].x), "=v"(ring[f][u].y), "=v"(ring[f][u].z), "=v"(ring[f][u].w));
+#pragma unroll
+  for (int f = 0; f < kRing; ++f)
+    if (static_cast<uint32_t>(f) < k.total) request_group(k, d, ring[f]);
+}
+// done(unit, sum): the sum of a lane's row, in every lane of its sixteen (of the wave, where a unit is a row).
+template <uint32_t DT, typename Done>
+__device__ __forceinline__ void walk(Walk &k, const ChainStage &d, bool rows, const uint16_t *x, uint4 (&ring)[kRing][kGroup], Done done) {
+  const uint32_t lane = fresh_thread() & (kWave - 1);
+  const char *const in = reinterpret_cast<const char *>(x);
+  uint32_t unit = k.first, group = 0, c = k.turn;
+  float open = 0.0f;   // of the unit under way
+#pragma unroll 1
+  for (uint32_t t = 0; t < k.total; t += kRing) {
+    float ends[kRing];
+    uint32_t ended = 0;
+#pragma unroll
+    for (int f = 0; f < kRing; ++f) {
+      ends[f] = 0.0f;
+      if (t + f < k.total) {
+        uint4 xv[kGroup];
+        uint32_t at[kGroup];
+        float acc[kGroup];
+#pragma unroll
+        for (int u = 0; u < kGroup; ++u) {
+          at[u] = (c << k.shift) + k.col;
+          xv[u] = *reinterpret_cast<const uint4 *>(in + min(at[u], k.last));
+          ++c;
+          c = min(c, c - d.chunks);
+        }
+#pragma unroll
+        for (int u = 0; u < kGroup; ++u) acc[u] = dot8<DT, true>(ring[f][u], xv[u], 0.0f);
+        if (!d.whole) {
+#pragma unroll
+          for (int u = 0; u < kGroup; ++u) acc[u] = at[u] <= k.last && group * kGroup + u < d.chunks ? acc[u] : 0.0f;
+        }
+        if (t + f + kRing < k.total) request_group(k, d, ring[f]);
+        float sum = (acc[0] + acc[1]) + (acc[2] + acc[3]);
+        sum += dpp_move<kDppQuadSwap1>(sum);
+        sum += dpp_move<kDppQuadSwap2>(sum);
+        sum += dpp_move<kDppRowHalfMirror>(sum);
+        sum += dpp_move<kDppRowMirror>(sum);
+        ends[f] = open = open + sum;
+        if (++group == d.groups) {
+          ended |= 1u << f;
+          group = 0;
+          c = k.turn;
+          open = 0.0f;
+        }
+      }
+    }
+#pragma unroll 1
+    for (int f = 0; f < kRing && ended >> f != 0; ++f) {
+      if ((ended >> f & 1u) == 0) continue;
+      float sum = f == 0 ? ends[0] : f == 1 ? ends[1] : f == 2 ? ends[2] : ends[3];
+      if (rows) sum = (lane_value(sum, 0) + lane_value(sum, 16)) + (lane_value(sum, 32) + lane_value(sum, 48));
+      done(unit, sum, lane);
+      unit += kWaves;
+    }
+  }
+}
+
+template <int HD, int G, bool PARTS>
+struct ChainAttnShared {
+  static constexpr int kRow = HD + 8;
+  alignas(16) uint16_t qhl[(PARTS ? 3 : 2) * G][kRow];   // as in the step kernel (StepShared)
+  float qdown[G];
+  alignas(16) uint16_t knew[HD];
+  alignas(16) uint16_t vnew[HD];
+  float wm[kWaves][G], wl[kWaves][G];
+  alignas(16) float wacc[kWaves][G][HD];
+};
+struct ChainMergeShared {
+  alignas(16) float o[4][128];
+  float m[4], l[4];
+};
+template <int HD, int G, bool PARTS>
+struct ChainShared {
+  alignas(16) float xf[kChainMaxHidden];
+  alignas(16) float rf[kChainMaxHidden];
+  alignas(16) uint16_t x16[kChainMaxHidden];
+  float red[2][kWaves];
+  float cs[HD];
+  union {
+    alignas(16) uint16_t in16[kChainMaxIn];
+    ChainAttnShared<HD, G, PARTS> attn;
+    ChainMergeShared merge;
+  };
+};
+
+// Split geometry of a step: blocks a split, splits.
+__device__ __forceinline__ void chain_splits(uint32_t kv_heads, uint32_t pos, uint32_t workgroups, uint32_t &nblk, uint32_t &bps, uint32_t &active) {
+  nblk = pos / kKvBlockTokens + 1;
+  uint32_t splits = 1;
+  if (nblk > kChainSingleBlocks) splits = max(1u, min(min(kChainMaxSplits, workgroups / kv_heads), (nblk + kSplitTiles - 1) / kSplitTiles));
+  bps = (nblk + splits - 1) / splits;
+  active = (nblk + bps - 1) / bps;
+}
+
+// The attention of one (key head, split): its q, k and v as they arrive, the cache's tiles through the matrix cores (attn_tile), and the 16-bit
+// output or, of several splits, the partial sums.
+template <uint32_t DT, int HD, int G, bool PARTS>
+__device__ __forceinline__ void chain_attention(Model m_, uint32_t layer, uint32_t pos, uint32_t kvh, uint32_t split, uint32_t nblk, uint32_t bps,
+                                                uint32_t active, uint32_t tag, Waiter &wait, ChainShared<HD, G, PARTS> &shared) {
+  Model p = m_;
+  fresh(p);
+  auto &sh = shared.attn;
+  const int lane = fresh_thread() & (kWave - 1);
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
+  const uint32_t A = p->heads * HD, KV = p->kv_heads * HD, n_keys = pos + 1, group = p->heads / p->kv_heads;
+  const uint16_t *const q_norm = weight(p, layer, kQNorm), *const k_norm = weight(p, layer, kKNorm);
+  const uint16_t *const q_bias = weight(p, layer, kQBias), *const k_bias = weight(p, layer, kKBias), *const v_bias = weight(p, layer, kVBias);
+  const bool rotates = p->rope_freq != nullptr;
+  const float eps = p->eps;
+  const uint32_t b0 = split * bps, b1 = min(nblk, b0 + bps);
+  const uint32_t new_block = pos / kKvBlockTokens, new_row = pos % kKvBlockTokens;
+  const bool owns_new = new_block >= b0 && new_block < b1;
+  const int pl = pair_of<HD>(lane);
+
+  // the wave's first tile is on its way before anything is waited for
+  uint4 kreg[HD / 32], vreg[HD / 32];
+  const auto load_tile = [&](uint32_t block) {
+    const uint64_t tile = kv_tile_offset(p->block_count, p->kv_heads, HD, layer, scalar_load(p->table + block), kvh);
+#pragma unroll
+    for (int i = 0; i < HD / 32; ++i) {
+      kreg[i] = load_stream(p->k_cache + tile + i * 512 + lane * 8);
+      vreg[i] = load_stream(p->v_cache + tile + i * 512 + lane * 8);
+    }
+  };
+  uint32_t b = b0 + wave;
+  if (b < b1) load_tile(b);
+
+  // heads of this wave, of the group's queries, the key and the value
+  constexpr int kMine = (G + 2 + kWaves - 1) / kWaves;
+  uint32_t head[kMine];
+  float b_0[kMine], b_1[kMine], g_0[kMine], g_1[kMine];
+  const uint64_t *src[kMine];
+#pragma unroll
+  for (int i = 0; i < kMine; ++i) {
+    head[i] = wave + i * kWaves;
+    const uint32_t h = min(head[i], group + 1);
+    const uint32_t off = h < group ? (kvh * group + h) * HD : (h == group ? A : A + KV) + kvh * HD;
+    src[i] = p->words + p->at_qkv + off + pl;
+    const uint16_t *bias = h < group ? q_bias : h == group ? k_bias : v_bias;
+    const uint16_t *gamma = h < group ? q_norm : h == group ? k_norm : nullptr;
+    const uint32_t boff = (h < group ? kvh * group + h : kvh) * HD + pl;
+    b_0[i] = bias != nullptr ? dec16<DT>(bias[boff]) : 0.0f;
+    b_1[i] = bias != nullptr ? dec16<DT>(bias[boff + HD / 2]) : 0.0f;
+    g_0[i] = gamma != nullptr ? dec16<DT>(gamma[pl]) : 1.0f;
+    g_1[i] = gamma != nullptr ? dec16<DT>(gamma[pl + HD / 2]) : 1.0f;
+  }
+  const float rc = shared.cs[pl], rs = shared.cs[HD / 2 + pl];
+  uint64_t v0[kMine], v1[kMine];
+  {
+    uint32_t spins = 0;
+    bool ok;
+    do {
+#pragma unroll
+      for (int i = 0; i < kMine; ++i) {
+        v0[i] = load_tagged(src[i]);
+        v1[i] = load_tagged(src[i] + HD / 2);
+      }
+      ok = true;
+#pragma unroll
+      for (int i = 0; i < kMine; ++i) ok = ok && tag_is(v0[i], tag) && tag_is(v1[i], tag);
+    } while (wait.again(ok, spins, tag));
+  }
+#pragma unroll
+  for (int i = 0; i < kMine; ++i) {
+    float x0 = tag_value(v0[i]), x1 = tag_value(v1[i]);
+    const bool query = head[i] < group, key = head[i] == group;
+    const bool norm = query ? q_norm != nullptr : key && k_norm != nullptr;
+    const bool bias = query ? q_bias != nullptr : key ? k_bias != nullptr : v_bias != nullptr;
+    if (head[i] < group + 2) {
+      head_values<DT, HD>(x0, x1, bias, b_0[i], b_1[i], norm, g_0[i], g_1[i], rotates && (query || key), rc, rs, eps);
+      if (query) {
+        const float scale = kLog2e / sqrtf(static_cast<float>(HD));
+        const uint32_t g = head[i];
+        uint16_t h0, l0, h1, l1;
+        x0 *= scale;
+        x1 *= scale;
+        if constexpr (PARTS) {
+          uint16_t t0, t1;
+          if constexpr (DT == kF16) {
+            const int up = attn_query_exponent(wave_max(fmaxf(fabsf(x0), fabsf(x1))));
+            x0 = ldexpf(x0, up);
+            x1 = ldexpf(x1, up);
+            if (lane == 0) sh.qdown[g] = ldexpf(1.0f, -up);
+          }
+          split16<DT>(x0, h0, l0, t0);
+          split16<DT>(x1, h1, l1, t1);
+          sh.qhl[2 * G + g][pl] = t0;
+          sh.qhl[2 * G + g][pl + HD / 2] = t1;
+        } else {
+          split16<DT>(x0, h0, l0);
+          split16<DT>(x1, h1, l1);
+        }
+        sh.qhl[g][pl] = h0;
+        sh.qhl[g][pl + HD / 2] = h1;
+        sh.qhl[G + g][pl] = l0;
+        sh.qhl[G + g][pl + HD / 2] = l1;
+      } else {
+        uint16_t *row = key ? sh.knew : sh.vnew;
+        row[pl] = enc16<DT>(x0);
+        row[pl + HD / 2] = enc16<DT>(x1);
+      }
+    }
+  }
+  __syncthreads();
+  if (owns_new && wave == kWaves - 1) {   // the new row, in operand order
+    const uint64_t tile = kv_tile_offset(p->block_count, p->kv_heads, HD, layer, scalar_load(p->table + new_block), kvh);
+    if (lane < HD / 8)
+      *reinterpret_cast<uint4 *>(p->k_cache + tile + kv_k_elem(HD, new_row, lane * 8)) = *reinterpret_cast<const uint4 *>(sh.knew + lane * 8);
+#pragma unroll
+    for (int i = 0; i < HD / kWave; ++i) {
+      const uint32_t d = lane + i * kWave;
+      p->v_cache[tile + kv_v_elem(HD, new_row, d)] = sh.vnew[d];
+    }
+  }
+  // columns of heads that the group does not have are zero
+  const int col = lane & 15, grp = lane >> 4;
+  const bool has = col < G ? static_cast<uint32_t>(col) < group : col < 2 * G && static_cast<uint32_t>(col - G) < group;
+  const uint4 zero = make_uint4(0u, 0u, 0u, 0u);
+  uint4 qx[HD / 32], third[PARTS ? HD / 32 : 1];
+  float down = 1.0f;
+#pragma unroll
+  for (int j = 0; j < HD / 32; ++j) {
+    const uint4 q = *reinterpret_cast<const uint4 *>(&sh.qhl[has ? col : 0][j * 32 + grp * 8]);
+    qx[j] = has ? q : zero;
+    if constexpr (PARTS) {
+      const bool own = has && col < G;
+      const uint4 t = *reinterpret_cast<const uint4 *>(&sh.qhl[2 * G + (own ? col : 0)][j * 32 + grp * 8]);
+      third[j] = own ? t : zero;
+    }
+  }
+  if constexpr (PARTS && DT == kF16) down = has ? sh.qdown[col < G ? col : col - G] : 1.0f;
+
+  float m = -INFINITY, l = 0.0f;
+  f32x4_t acc[HD / 16];
+#pragma unroll
+  for (int s = 0; s < HD / 16; ++s) acc[s] = f32x4_t{0.0f, 0.0f, 0.0f, 0.0f};
+  for (; b < b1; b += kWaves) {
+    attn_tile<DT, HD, G, false, PARTS, PARTS && DT == kF16>(kreg, vreg, qx, nullptr, b, n_keys, col, grp, owns_new && b == new_block, new_row, sh.knew, sh.vnew, m, l, acc,
+                                       down, third);
+    if (b + kWaves < b1) load_tile(b + kWaves);
+  }
+  l += __shfl_xor(l, 16, kWave);
+  l += __shfl_xor(l, 32, kWave);
+#pragma unroll
+  for (int s = 0; s < HD / 16; ++s) {
+    float4 o;
+    o.x = acc[s][0] + row_shl<G>(acc[s][0]);
+    o.y = acc[s][1] + row_shl<G>(acc[s][1]);
+    o.z = acc[s][2] + row_shl<G>(acc[s][2]);
+    o.w = acc[s][3] + row_shl<G>(acc[s][3]);
+    if (col < G) *reinterpret_cast<float4 *>(&sh.wacc[wave][col][s * 16 + grp * 4]) = o;
+  }
+  if (lane < G) {
+    sh.wm[wave][lane] = m;
+    sh.wl[wave][lane] = l;
+  }
+  __syncthreads();
+  for (uint32_t e = threadIdx.x; e < group * (HD / 2); e += kThreads) {
+    const uint32_t g = e / (HD / 2), d = e % (HD / 2) * 2;
+    float M = -INFINITY;
+#pragma unroll
+    for (int i = 0; i < kWaves; ++i) M = fmaxf(M, sh.wm[i][g]);
+    float L = 0.0f, o0 = 0.0f, o1 = 0.0f;
+#pragma unroll
+    for (int i = 0; i < kWaves; ++i) {
+      const float mw = sh.wm[i][g], f = mw > -INFINITY ? attn_exp2(mw - M) : 0.0f;   // a wave without a tile
+      L = fmaf(sh.wl[i][g], f, L);
+      o0 = fmaf(sh.wacc[i][g][d], f, o0);
+      o1 = fmaf(sh.wacc[i][g][d + 1], f, o1);
+    }
+    const uint32_t h = kvh * group + g;
+    if (active == 1) {
+      if (L > 0.0f && isfinite(L)) {
+        o0 /= L;
+        o1 /= L;
+      }
+      store_word(p->words + p->at_attn + (h * HD + d) / 2, enc16<DT>(o0) | (static_cast<uint32_t>(enc16<DT>(o1)) << 16), tag);
+    } else {
+      uint64_t *rec = p->words + p->at_part + (static_cast<uint64_t>(h) * kChainMaxSplits + split) * (HD + 2);
+      store_tagged(rec + d, o0, tag);
+      store_tagged(rec + d + 1, o1, tag);
+      if (d == 0) {
+        store_tagged(rec + HD, M, tag);
+        store_tagged(rec + HD + 1, L, tag);
+      }
+    }
+  }
+  __syncthreads();   // (the scratch is the next input's place)
+}
+
+// One head's splits: the threads of a dimension take every (256 / HD)-th of them, in order, and meet in LDS.
+template <uint32_t DT, int HD>
+__device__ __forceinline__ void chain_merge(Model m_, uint32_t h, uint32_t active, uint32_t tag, Waiter &wait, ChainMergeShared &sh) {
+  Model p = m_;
+  fresh(p);
+  constexpr uint32_t kSets = kThreads / HD, kPer = kChainMaxSplits / kSets;
+  const uint32_t thread = fresh_thread(), d = thread % HD, q = thread / HD;
+  const uint64_t *rec = p->words + p->at_part + static_cast<uint64_t>(h) * kChainMaxSplits * (HD + 2);
+  uint64_t av[kPer], mv[kPer], lv[kPer];
+  uint32_t spins = 0;
+  bool ok;
+  do {
+#pragma unroll
+    for (uint32_t i = 0; i < kPer; ++i) {
+      const uint32_t r = min(q + i * kSets, active - 1) * ((HD + 2) * 8u);
+      av[i] = load_tagged(at_bytes(rec, r + d * 8u));
+      mv[i] = load_tagged(at_bytes(rec, r + HD * 8u));
+      lv[i] = load_tagged(at_bytes(rec, r + HD * 8u + 8u));
+    }
+    ok = true;
+#pragma unroll
+    for (uint32_t i = 0; i < kPer; ++i)
+      if (q + i * kSets < active) ok = ok && tag_is(av[i], tag) && tag_is(mv[i], tag) && tag_is(lv[i], tag);
+  } while (wait.again(ok, spins, tag));
+  float M = -INFINITY, L = 0.0f, o = 0.0f;
+#pragma unroll
+  for (uint32_t i = 0; i < kPer; ++i)
+    if (q + i * kSets < active) M = fmaxf(M, tag_value(mv[i]));
+#pragma unroll
+  for (uint32_t i = 0; i < kPer; ++i) {
+    if (q + i * kSets < active) {
+      const float f = attn_exp2(tag_value(mv[i]) - M);
+      L = fmaf(tag_value(lv[i]), f, L);
+      o = fmaf(tag_value(av[i]), f, o);
+    }
+  }
+  sh.o[q][d] = o;
+  if (d == 0) {
+    sh.m[q] = M;
+    sh.l[q] = L;
+  }
+  __syncthreads();
+  if (threadIdx.x < HD / 2) {
+    float Mt = -INFINITY, Lt = 0.0f, o0 = 0.0f, o1 = 0.0f;
+#pragma unroll
+    for (uint32_t i = 0; i < kSets; ++i) Mt = fmaxf(Mt, sh.m[i]);
+#pragma unroll
+    for (uint32_t i = 0; i < kSets; ++i) {
+      const float f = sh.m[i] > -INFINITY ? attn_exp2(sh.m[i] - Mt) : 0.0f;
+      Lt = fmaf(sh.l[i], f, Lt);
+      o0 = fmaf(sh.o[i][2 * threadIdx.x], f, o0);
+      o1 = fmaf(sh.o[i][2 * threadIdx.x + 1], f, o1);
+    }
+    if (Lt > 0.0f && isfinite(Lt)) {
+      o0 /= Lt;
+      o1 /= Lt;
+    }
+    store_word(p->words + p->at_attn + (h * HD) / 2 + threadIdx.x, enc16<DT>(o0) | (static_cast<uint32_t>(enc16<DT>(o1)) << 16), tag);
+  }
+  __syncthreads();
+}
+
+template <uint32_t DT, int HD, int G, bool PARTS>
+__global__ __launch_bounds__(kThreads, 2) void step_chain_kernel(ChainLaunch p) {
+  __shared__ ChainShared<HD, G, PARTS> sh;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
+  Model m = (Model)(reinterpret_cast<uint64_t>(p.model));
+  const uint32_t pos = scalar_load(m->state), step = scalar_load(m->state + 2);
+  if (pos >= m->max_steps) return;
+  constexpr int kX = kChainMaxHidden / kThreads;
+  uint4 ring[kRing][kGroup];
+  Walk k;
+  const uint32_t log_grid = 31 - __builtin_clz(gridDim.x);   // (chain_workgroups: a power of two)
+  ChainStage d = read_stage(m, 0);
+  walk_begin(k, d, false, log_grid, ring);
+
+  uint32_t nblk, bps, active;
+  chain_splits(m->kv_heads, pos, gridDim.x, nblk, bps, active);
+  const bool attends = blockIdx.x < m->kv_heads * active;
+  const uint32_t kvh = blockIdx.x % m->kv_heads, split = blockIdx.x / m->kv_heads;
+  if (attends && m->rope_freq != nullptr) {
+    for (int i = threadIdx.x; i < HD / 2; i += kThreads) {
+      float sn, cs;
+      sincosf(static_cast<float>(pos) / m->rope_freq[i], &sn, &cs);
+      sh.cs[i] = cs;
+      sh.cs[HD / 2 + i] = sn;
+    }
+  }
+  Waiter wait{p.spin_limit, m->fault};
+  // test hook: where a layer's vectors go. Workgroup 0 reads all of them but the raw heads, which their producers write
+  const auto slot = [](uint32_t bytes) { return (bytes + 255u) & ~255u; };
+  const bool traces = p.trace != nullptr;
+  const auto trace_at = [&](uint32_t layer, int link) {
+    const uint32_t H = m->hidden, h16 = slot(H * 2), h32 = slot(H * 4), qkv = slot((m->heads + 2 * m->kv_heads) * HD * 4), a16 = slot(m->heads * HD * 2), f16 = slot(m->ff * 2);
+    uint64_t at = h32 + static_cast<uint64_t>(layer) * (2 * h16 + qkv + a16 + 2 * h32 + f16);
+    if (link > 0) at += h16;
+    if (link > 1) at += qkv;
+    if (link > 2) at += a16;
+    if (link > 3) at += h32;
+    if (link > 4) at += h16;
+    if (link > 5) at += f16;
+    return p.trace + at;
+  };
+  const auto dump16 = [&](uint32_t layer, int link, const uint16_t *from, uint32_t n) {
+    if (traces && blockIdx.x == 0)
+      for (uint32_t i = fresh_thread(); i < n; i += kThreads) reinterpret_cast<uint16_t *>(trace_at(layer, link))[i] = from[i];
+  };
+
+  // A row of x or r: its elements as they come, in f32 and normalised.
+  uint32_t turn = 0;
+  const auto take_row = [&](float (&v)[kX], const uint16_t (&g)[kX], float *raw) {
+    const uint32_t H = m->hidden, thread = fresh_thread();
+    float ss = 0.0f;
+#pragma unroll
+    for (int i = 0; i < kX; ++i) {
+      const uint32_t c = thread + i * kThreads;
+      if (c < H) ss = fmaf(v[i], v[i], ss);
+    }
+    ss = wave_sum(ss);
+    if (thread % kWave == 0) sh.red[turn][wave] = ss;
+    __syncthreads();
+    // 1 / sqrt by the hardware's (an ulp) and a step of Newton's: what a square root and a division leave of it, in a tenth of the time
+    const float mean = fmaf((sh.red[turn][0] + sh.red[turn][1]) + (sh.red[turn][2] + sh.red[turn][3]), m->inv_hidden, m->eps);
+    const float rough = __builtin_amdgcn_rsqf(mean), scale = fmaf(rough * 0.5f, fmaf(-mean * rough, rough, 1.0f), rough);
+    turn ^= 1u;
+#pragma unroll
+    for (int i = 0; i < kX; ++i) {
+      const uint32_t c = thread + i * kThreads;
+      if (c < H) {
+        raw[c] = v[i];
+        sh.x16[c] = enc16<DT>(v[i] * scale * dec16<DT>(g[i]));
+      }
+    }
+    __syncthreads();
+  };
+  const auto poll_row = [&](const uint64_t *src, uint32_t tag, float (&v)[kX]) {
+    const uint32_t H = m->hidden;
+    uint64_t words[kX];
+    if (H <= 2u * kThreads) {
+      uint64_t few[2];
+      poll_words<2>(src, H, tag, wait, few);
+      words[0] = few[0];
+      words[1] = few[1];
+#pragma unroll
+      for (int i = 2; i < kX; ++i) words[i] = 0;
+    } else {
+      poll_words<kX>(src, H, tag, wait, words);
+    }
+#pragma unroll
+    for (int i = 0; i < kX; ++i) v[i] = tag_value(words[i]);
+  };
+
+  const uint32_t stages = m->layers * kStages;
+#pragma unroll 1
+  for (uint32_t at = 0; at < stages; ++at) {
+    const uint32_t layer = at / kStages, stage = at % kStages;
+    const bool rows = (stage & 1u) != 0;
+    const uint32_t tag = step * 256u + layer + 1u;   // (never that of another step until 2^24 of them)
+    fresh(m);
+    const ChainStage next = read_stage(m, min(at + 1, stages - 1));
+    uint64_t *const words = m->words;
+    if (!rows) {
+      float v[kX];
+      uint16_t g[kX];
+      const uint32_t thread = fresh_thread();
+#pragma unroll
+      for (int i = 0; i < kX; ++i) g[i] = *at_bytes(d.vec, min(thread + i * kThreads, m->hidden - 1) * 2u);   // (requested before the wait for the row)
+      if (at == 0) {
+        uint32_t token = pos < scalar_load(m->state + 1) ? m->prompt[pos] : m->slots[pos - 1].token;
+        if (token >= m->vocab) token = 0;   // prompts are validated on the host; sampled ids are < vocab
+        const uint16_t *row = m->emb + static_cast<uint64_t>(token) * m->hidden;
+#pragma unroll
+        for (int i = 0; i < kX; ++i) v[i] = dec16<DT>(row[min(thread + i * kThreads, m->hidden - 1)]);
+        if (traces && blockIdx.x == 0)
+          for (int i = 0; i < kX; ++i)
+            if (thread + i * kThreads < m->hidden) reinterpret_cast<float *>(p.trace)[thread + i * kThreads] = v[i];
+      } else {
+        poll_row(words + d.in_at, tag, v);
+      }
+      float *raw = stage == kQkv ? sh.xf : sh.rf;
+      take_row(v, g, raw);
+      if (traces && stage == kGateUp && blockIdx.x == 0)
+        for (uint32_t i = fresh_thread(); i < m->hidden; i += kThreads) reinterpret_cast<float *>(trace_at(layer, 3))[i] = raw[i];
+    } else {
+      take_pairs(words + d.in_at, d.in_words, tag, wait, sh.in16);
+      __syncthreads();
+    }
+    const uint16_t *const in = rows ? sh.in16 : sh.x16;
+    if (traces) dump16(layer, stage == kQkv ? 0 : stage == kO ? 2 : stage == kGateUp ? 4 : 5, in, d.cols);
+    uint64_t *const out = words + d.out_at;
+    const bool last = at + 1 == stages;
+    walk<DT>(k, d, rows, in, ring, [&](uint32_t unit, float sum, uint32_t lane) {
+      if (stage == kQkv) {
+        if (lane % 16 == 0) {
+          store_tagged(at_bytes(out, unit * 32 + lane / 2), sum, tag);
+          if (traces) reinterpret_cast<float *>(trace_at(layer, 1))[unit * 4 + lane / 16] = sum;
+        }
+      } else if (stage == kGateUp) {
+        const float other = lane_value(sum, 32), own = lane_value(sum, 48);
+        const float g = sum, u = lane < 16 ? other : own;   // (lanes 0 to 31: the two gate rows)
+        const uint32_t half = enc16<DT>(gated(g, 1.0f) * u);
+        const uint32_t pair = half | (static_cast<uint32_t>(__builtin_amdgcn_readlane(half, 16)) << 16);
+        if (lane == 0) store_word(at_bytes(out, unit * 8), pair, tag);
+      } else if (lane == 0) {
+        float y = sum;
+        if (d.vec != nullptr) y += dec16<DT>(d.vec[unit]);
+        y += stage == kO ? sh.xf[unit] : sh.rf[unit];
+        if (last) m->x[unit] = y;
+        else store_tagged(at_bytes(out, unit * 8), y, stage == kO ? tag : tag + 1u);
+        if (traces && stage == kDown) reinterpret_cast<float *>(trace_at(layer, 6))[unit] = y;
+      }
+    });
+    if (stage == kQkv) {
+      fresh(m);
+      if (attends) chain_attention<DT, HD, G, PARTS>(m, layer, pos, kvh, split, nblk, bps, active, tag, wait, sh);
+      if (active > 1) {   // (heads from the other end of the grid)
+        for (uint32_t h = gridDim.x - 1 - blockIdx.x; h < m->heads; h += gridDim.x) chain_merge<DT, HD>(m, h, active, tag, wait, sh.merge);
+      }
+    }
+    d = next;
+    if (!last) walk_begin(k, d, !rows, log_grid, ring);
+  }
+}
+
+}  // namespace
+
+bool chain_takes(uint32_t layers, uint32_t hidden, uint32_t heads, uint32_t kv_heads, uint32_t head_dim, uint32_t ff) {
+  if (!attn_matrix_cores(heads, kv_heads, head_dim) || heads > 512 || hidden > kChainMaxHidden || ff > kChainMaxIn || heads * head_dim > kChainMaxIn) return false;
+  // At least as many units of every projection as workgroups, whole 16-byte pieces, and a table of layers that the tags can tell
+  // apart. Stacks of one to three layers keep their launches: callers look at those piece by piece.
+  if (layers < 4 || layers >= 255 || hidden < kMaxWorkgroups || hidden % 8 != 0 || ff < 2 * kMaxWorkgroups || ff % 8 != 0 || kv_heads > 32) return false;
+  // Up to 10 MB of weights a layer (see above: 9.4 MB 1.14 to 1.10 times as fast, 13.8 MB 0.93)
+  return hidden * (2 * heads + 2 * kv_heads) * head_dim + 3 * hidden * ff <= 5000000u;
+}
+
+// A unit or two for a wave (512 x 1376: 64 / 128 / 256 workgroups 76 / 65 / 74 us a step), a power of two.
+uint32_t chain_workgroups(uint32_t hidden, uint32_t heads, uint32_t kv_heads, uint32_t head_dim, uint32_t ff) {
+  const uint32_t units = std::max(ff / 2, (heads + 2 * kv_heads) * head_dim / 4) * ((hidden + 511) / 512);
+  const uint32_t want = std::max({(units + 2 * kWaves - 1) / (2 * kWaves), 32u, kv_heads});
+  uint32_t grid = 32;
+  while (grid < want && grid < kMaxWorkgroups) grid *= 2;
+  return grid;
+}
+
+uint64_t chain_place(ChainModel &m, uint32_t head_dim) {
+  uint64_t end = 0;
+  const auto take = [&](uint32_t &at, uint64_t words) {   // on cache lines
+    at = static_cast<uint32_t>(end);
+    end += (words + 15u) & ~uint64_t{15};
+  };
+  take(m.at_x, m.hidden);
+  take(m.at_qkv, static_cast<uint64_t>(m.heads + 2 * m.kv_heads) * head_dim);
+  take(m.at_attn, static_cast<uint64_t>(m.heads) * head_dim / 2);
+  take(m.at_part, static_cast<uint64_t>(m.heads) * kChainMaxSplits * (head_dim + 2));
+  take(m.at_r, m.hidden);
+  take(m.at_ff, m.ff / 2);
+  return end;
+}
+
+void chain_stages(const ChainModel &m, uint32_t head_dim, const LayerDev &w, ChainStage (&stage)[4]) {
+  const uint32_t A = m.heads * head_dim;
+  const uint16_t *const matrix[4] = {w.wqkv, w.wo, w.wgu, w.wdown}, *const vec[4] = {w.rms_attn, w.o_bias, w.rms_mlp, nullptr};
+  const uint32_t cols[4] = {m.hidden, A, m.hidden, m.ff}, units[4] = {(m.heads + 2 * m.kv_heads) * head_dim / 4, m.hidden, m.ff / 2, m.hidden};
+  const uint32_t in_at[4] = {m.at_x, m.at_attn, m.at_r, m.at_ff}, out_at[4] = {m.at_qkv, m.at_r, m.at_ff, m.at_x};
+  for (uint32_t i = 0; i < 4; ++i) {
+    const bool rows = i % 2 != 0;
+    ChainStage &s = stage[i];
+    s = ChainStage{};
+    s.w = matrix[i];
+    s.vec = vec[i];
+    s.cols = cols[i];
+    s.chunks = (cols[i] + (rows ? 511 : 127)) / (rows ? 512 : 128);
+    s.groups = (s.chunks + kGroup - 1) / kGroup;
+    s.units = units[i];
+    s.row_bytes = cols[i] * 2;
+    s.unit_bytes = s.row_bytes * (rows ? 1 : i == kQkv ? 4 : 2);
+    s.up_bytes = i == kGateUp ? m.ff * s.row_bytes + m.pair_gap * 2 : s.row_bytes * 2;
+    s.in_at = in_at[i];
+    s.in_words = rows ? cols[i] / 2 : cols[i];
+    s.out_at = out_at[i];
+    s.whole = cols[i] % (rows ? 512 : 128) == 0 && s.chunks % kGroup == 0;
+  }
+}
+
+namespace {
+template <uint32_t DT, int HD, int G, bool PARTS>
+hipError_t launch_one(const ChainModel &m, const ChainLaunch &p, hipStream_t stream) {
+  hipLaunchKernelGGL((step_chain_kernel<DT, HD, G, PARTS>), dim3(chain_workgroups(m.hidden, m.heads, m.kv_heads, HD, m.ff)), dim3(kThreads), 0, stream, p);
+  return hipGetLastError();
+}
+template <uint32_t DT>
+hipError_t launch_shape(uint32_t head_dim, const ChainModel &m, const ChainLaunch &p, hipStream_t stream) {
+  const uint32_t group = m.heads / m.kv_heads;
+  if (head_dim == 64) {
+    if (group == 1) return launch_one<DT, 64, 1, true>(m, p, stream);
+    if (group == 2) return launch_one<DT, 64, 2, true>(m, p, stream);
+    if (group <= 4) return launch_one<DT, 64, 4, true>(m, p, stream);
+    return launch_one<DT, 64, 8, true>(m, p, stream);
+  }
+  if (group == 1) return launch_one<DT, 128, 1, false>(m, p, stream);
+  if (group == 2) return launch_one<DT, 128, 2, false>(m, p, stream);
+  if (group == 3) return launch_one<DT, 128, 4, true>(m, p, stream);
+  if (group == 4) return launch_one<DT, 128, 4, false>(m, p, stream);
+  if (group < 8) return launch_one<DT, 128, 8, true>(m, p, stream);
+  return launch_one<DT, 128, 8, false>(m, p, stream);
+}
+}  // namespace
+
+hipError_t launch_step_chain(uint32_t dtype, uint32_t head_dim, const ChainModel &m, const ChainLaunch &p, hipStream_t stream) {
+  if (!chain_takes(m.layers, m.hidden, m.heads, m.kv_heads, head_dim, m.ff) || p.model == nullptr || m.words == nullptr || p.spin_limit == 0)
+    return hipErrorInvalidValue;
+  if (dtype == kBF16) return launch_shape<kBF16>(head_dim, m, p, stream);
+  if (dtype == kF16) return launch_shape<kF16>(head_dim, m, p, stream);
+  return hipErrorInvalidValue;
+}
+
+}  // namespace nv

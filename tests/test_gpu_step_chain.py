@@ -1,0 +1,120 @@
+"""Decode steps of narrow models whose layers run in one launch, against the oracle and against the launches they stand in for."""
+import numpy as np
+import pytest
+
+import nerva_amd as N
+import oracle as O
+from nerva_amd import abi
+from oracle.links import chain_budget, run_traced_stream
+from test_gpu_session import BF16, F16, random_model, rel_l2
+
+pytestmark = pytest.mark.gpu
+
+# dtype, hidden, heads, kv, hd, inter, vocab, layers, theta, qk_norm, bias: widths of whole and of part columns a request, one to
+# eight query heads a key head (three, five and seven among them) of both sizes, units that do not go round evenly, the largest of everything
+SHAPES = [
+    (F16, 512, 8, 4, 64, 1376, 803, 4, 1e4, False, False),
+    (BF16, 256, 2, 2, 128, 512, 301, 4, 1e6, True, True),
+    (BF16, 520, 3, 1, 128, 1000, 301, 4, 0, True, False),
+    (F16, 640, 10, 2, 64, 2056, 301, 5, 1e4, False, True),
+    (BF16, 1024, 4, 2, 128, 1024, 511, 4, 1e6, True, False),
+    (F16, 1016, 7, 1, 128, 776, 301, 4, 1e6, False, False),
+    (BF16, 256, 32, 4, 128, 3000, 301, 4, 1e6, True, True),
+    (F16, 264, 20, 20, 64, 4096, 301, 4, 1e4, True, False),
+]
+
+
+@pytest.mark.parametrize("shape", SHAPES)
+def test_every_link_of_a_chained_step_matches_the_oracle(shape):
+    """Each vector that a layer hands on, at 1e-3 of the oracle's operator on the device's own input, and the stream's logits within the
+    budget of the chain; the same stream from one call. Positions cross a cache block."""
+    dtype, hidden, heads, kv, hd, inter, vocab, layers, theta, qk_norm, bias = shape
+    weights, model = random_model(dtype, hidden, heads, kv, hd, inter, vocab, layers, hidden, theta, qk_norm, bias)
+    prompt = np.random.default_rng(1).integers(0, vocab, 11).astype(np.uint32)
+    s = N.DecodeSession.create(weights, 64)
+    tokens, worst, e2e = run_traced_stream(s, model, prompt, 12, 64)
+    assert s.start(prompt)[0] == 0
+    rc, res, again = s.advance(12)
+    assert rc == 0 and res.graph_nodes == 3 and res.graph_replays == 11 and again.tolist() == tokens
+    s.destroy()
+    print(sorted(worst.items()), e2e, flush=True)
+
+
+@pytest.mark.parametrize("shape", [SHAPES[0], SHAPES[4], SHAPES[5], SHAPES[6], SHAPES[7]])
+def test_a_chain_over_longer_contexts_gives_what_launches_give(shape):
+    """Contexts of one split, of the first several and of as many as there are, behind prompts that both kinds of session have
+    read alike: logits and cache rows of the steps. Only roundings of 16-bit values that lie on a boundary may fall differently."""
+    dtype, hidden, heads, kv, hd, inter, vocab, layers, theta, qk_norm, bias = shape
+    weights, _ = random_model(dtype, hidden, heads, kv, hd, inter, vocab, layers, 7, theta, qk_norm, bias)
+    rng = np.random.default_rng(3)
+    results = []
+    lengths = (30, 125, 130, 255, 700, 1100)
+    prompts = [rng.integers(0, vocab, n).astype(np.uint32) for n in lengths]
+    try:
+        for mode in (2, 0):
+            N.Device.set_tuning("step_chain", mode)
+            s = N.DecodeSession.create(weights, 1200)
+            out = []
+            for prompt in prompts:
+                assert s.start(prompt)[0] == 0
+                assert s.advance(1)[0] == 0
+                for step in range(3):
+                    rc, res = s.extend(prompt[step:step + 1])[:2]     # the same tokens whatever the logits say
+                    assert rc == 0 and res.kernel_launches == (3 if mode == 0 else 3 + 5 * layers)
+                out.append((s.logits(), s.kv_range(layers - 1, len(prompt), 3)))
+            results.append(out)
+            s.destroy()
+    finally:
+        N.Device.reset_tuning()
+    for n, (want, want_rows), (got, got_rows) in zip(lengths, *results):
+        assert np.all(np.isfinite(got)) and rel_l2(got, want) <= chain_budget(layers), (n, rel_l2(got, want))
+        for a, b in zip(want_rows, got_rows):
+            assert rel_l2(O.decode16(dtype, b), O.decode16(dtype, a)) <= chain_budget(layers), n
+
+
+def test_sampled_and_stopped_chains_and_forks():
+    """The sampler behind a chain, a stop token, a fork of a running sequence and a second sequence on the same words."""
+    dtype, hidden, heads, kv, hd, inter, vocab, layers, theta, qk_norm, bias = SHAPES[0]
+    weights, _ = random_model(dtype, hidden, heads, kv, hd, inter, vocab, layers, 5, theta, qk_norm, bias)
+    prompt = np.random.default_rng(2).integers(0, vocab, 9).astype(np.uint32)
+    sampler = abi.NervaHipHfDecodeSamplerConfig()
+    sampler.temperature, sampler.top_p, sampler.top_k, sampler.seed = 0.9, 0.95, 0, 11
+    s = N.DecodeSession.create(weights, 64)
+    assert s.start(prompt, sampler=sampler)[0] == 0
+    rc, res, drawn = s.advance(16)
+    assert rc == 0 and res.graph_nodes == 4
+    assert s.start(prompt)[0] == 0
+    rc, res, greedy = s.advance(6)
+    assert rc == 0 and res.graph_nodes == 3
+    fork = s.fork_shared_weights()
+    rest = s.advance(8)[2].tolist()
+    assert fork.advance(8)[2].tolist() == rest
+    assert s.start(prompt, sampler=sampler)[0] == 0
+    assert s.advance(16)[2].tolist() == drawn.tolist()
+    rc, res, walked = s.run(prompt, 14)
+    assert rc == 0 and len(walked) == 14
+    fork.destroy()
+    s.destroy()
+
+
+def test_a_wait_that_runs_out_ends_the_sequence():
+    """With a limit of one poll a chain's waits run out: every wait ends, the slot says so, advance returns the step fault; a
+    sequence started afterwards is the healthy one."""
+    dtype, hidden, heads, kv, hd, inter, vocab, layers, theta, qk_norm, bias = SHAPES[4]
+    weights, _ = random_model(dtype, hidden, heads, kv, hd, inter, vocab, layers, 5, theta, qk_norm, bias)
+    prompt = np.random.default_rng(2).integers(0, vocab, 9).astype(np.uint32)
+    s = N.DecodeSession.create(weights, 64)
+    assert s.start(prompt)[0] == 0
+    want = s.advance(12)[2].tolist()
+    fork = s.fork_shared_weights()
+    N.Device.set_tuning("attn_merge_spin_limit", 1)
+    try:
+        assert fork.start(prompt)[0] == 0
+        rc, res, tokens = fork.advance(3)         # (captured with the limit)
+    finally:
+        N.Device.reset_tuning()
+    assert rc == -1 and res.hip_error == abi.NERVA_HIP_ERROR_STEP_FAULT
+    fork.destroy()
+    assert s.start(prompt)[0] == 0
+    assert s.advance(12)[2].tolist() == want
+    s.destroy()
