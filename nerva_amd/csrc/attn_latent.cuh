@@ -13,6 +13,7 @@
 #pragma once
 
 #include "attn_decode.cuh"
+#include "gemv_layer.cuh"
 
 namespace nv {
 
@@ -68,7 +69,9 @@ hipError_t launch_latent_attention(uint32_t dtype, const LatentAttnParams &p, hi
 bool latent_attention_wide(uint32_t heads, uint32_t key_dim, uint32_t rot_dim, uint32_t value_dim, uint32_t kv_rank);
 uint64_t latent_workspace_bytes(uint32_t heads, uint32_t rot_dim, uint32_t kv_rank, uint32_t max_tokens);
 hipError_t latent_wide_setup();   // once per process, outside stream capture
+// What of a layer's feed-forward rides with a decode step's launches: `riders` (of which none, with empty ranges and no y). Their LDS has to fit.
+bool latent_riders_fit(uint32_t kv_rank, uint32_t hidden, uint32_t top, uint32_t ff, uint32_t shared_ff);
 // (launches: counted up)
-hipError_t launch_latent_attention_wide(uint32_t dtype, const LatentAttnParams &p, hipStream_t stream, uint64_t *launches);
+hipError_t launch_latent_attention_wide(uint32_t dtype, const LatentAttnParams &p, const LayerRiders &riders, hipStream_t stream, uint64_t *launches);
 
 }  // namespace nv

@@ -24,6 +24,7 @@
 #include "attn_mixed.cuh"
 #include "attn_tile.cuh"
 #include "gemm_rows.cuh"
+#include "gemv_layer_walk.cuh"
 
 namespace nv {
 
@@ -65,13 +66,61 @@ typedef uint32_t u32x2_t __attribute__((ext_vector_type(2)));
 
 // ---- absorb ----------------------------------------------------------------------------------
 
+// 32 contraction rows of a workgroup's columns of W_uk, and a lane's queries of them.
+template <int RT>
+struct AbsorbStep {
+  static constexpr uint32_t kCols = RT * 16, kPieces = 32u * kCols / (kBlock * 8u);
+  static_assert(kPieces * kBlock * 8u == 32u * kCols && kPieces <= 2, "whole pieces");
+  u32x4_t w0, w1;
+  f32x4_t a, b;
+};
+template <int RT>
+__device__ __forceinline__ void absorb_request(AbsorbStep<RT> &s, const uint16_t *w, const float *q, uint32_t rank, uint32_t d, uint32_t q4) {
+  constexpr uint32_t kCols = AbsorbStep<RT>::kCols;
+  const uint32_t i = threadIdx.x * 8u;
+  const uint16_t *const src = w + static_cast<uint64_t>(d + i / kCols) * rank + i % kCols;
+  s.w0 = *reinterpret_cast<const u32x4_t *>(src);
+  if constexpr (AbsorbStep<RT>::kPieces == 2) s.w1 = *reinterpret_cast<const u32x4_t *>(src + kBlock * 8u / kCols * rank);
+  s.a = *reinterpret_cast<const f32x4_t *>(q + d + 4u * q4);
+  s.b = *reinterpret_cast<const f32x4_t *>(q + d + 16u + 4u * q4);
+}
+template <int RT>
+__device__ __forceinline__ void absorb_step(const AbsorbStep<RT> &s, uint16_t *w_s, uint32_t at, f32x4_t (&acc)[RT]) {
+  constexpr uint32_t kCols = AbsorbStep<RT>::kCols;
+  __syncthreads();
+  *reinterpret_cast<u32x4_t *>(w_s + threadIdx.x * 8u) = s.w0;
+  if constexpr (AbsorbStep<RT>::kPieces == 2) *reinterpret_cast<u32x4_t *>(w_s + (threadIdx.x + kBlock) * 8u) = s.w1;
+  const uint4 x = make_uint4(pack16(s.a.x, s.a.y), pack16(s.a.z, s.a.w), pack16(s.b.x, s.b.y), pack16(s.b.z, s.b.w));
+  __syncthreads();
+#pragma unroll
+  for (int i = 0; i < RT; i += 2) {
+    u32x2_t lo[2], hi[2];
+    asm volatile("ds_read_b64_tr_b16 %0, %4 offset:%5\n\tds_read_b64_tr_b16 %1, %4 offset:%6\n\t"
+                 "ds_read_b64_tr_b16 %2, %4 offset:%7\n\tds_read_b64_tr_b16 %3, %4 offset:%8\n\ts_waitcnt lgkmcnt(0)"
+                 : "=&v"(lo[0]), "=&v"(hi[0]), "=&v"(lo[1]), "=&v"(hi[1])
+                 : "v"(at), "n"(i * 32), "n"(i * 32 + 16 * kCols * 2), "n"((i + 1) * 32), "n"((i + 1) * 32 + 16 * kCols * 2)
+                 : "memory");
+#pragma unroll
+    for (int j = 0; j < 2; ++j) acc[i + j] = mfma_k32<kBF16>(make_uint4(lo[j].x, lo[j].y, hi[j].x, hi[j].y), x, acc[i + j]);
+  }
+}
+
 // A workgroup: one head, RT x 16 latent columns, 64 tokens (16 a wave); the column group past the last one prepares the
 // rotated elements (and a decode step's cache row, head 0).
-template <int RT>
-__global__ __launch_bounds__(kBlock) void latent_absorb_kernel(LatentAttnParams p, uint16_t *q16) {
+// RIDES (a decode step): the grid's other layers (z) are the riders'.
+template <int RT, bool RIDES>
+__global__ __launch_bounds__(kBlock, RIDES ? 4 : 1) void latent_absorb_kernel(LatentAttnParams p, uint16_t *q16, RiderPairs riders) {
   constexpr uint32_t DT = kBF16, kCols = RT * 16;
   __shared__ __align__(16) uint16_t w_s[32 * kCols];
   __shared__ float red[kWavesPerBlock];
+  if constexpr (RIDES) {
+    extern __shared__ __align__(16) uint16_t rider_s[];
+    if (blockIdx.z != 0) {
+      const uint32_t plane = gridDim.x * gridDim.y;
+      layer::ride_pairs<DT, kWavesPerBlock>(riders, p.cursor, p.max_steps, rider_s, (blockIdx.z - 1) * plane + blockIdx.y * gridDim.x + blockIdx.x, (gridDim.z - 1) * plane);
+      return;
+    }
+  }
   const uint32_t pos0 = p.cursor != nullptr ? *p.cursor : p.position;
   if (p.cursor != nullptr && pos0 >= p.max_steps) return;
   const uint32_t R = p.kv_rank, width = R + p.rot_dim, head = p.key_dim + p.rot_dim, h = blockIdx.y;
@@ -106,25 +155,18 @@ __global__ __launch_bounds__(kBlock) void latent_absorb_kernel(LatentAttnParams 
   f32x4_t acc[RT];
 #pragma unroll
   for (int i = 0; i < RT; ++i) acc[i] = f32x4_t{0.0f, 0.0f, 0.0f, 0.0f};
-  for (uint32_t d0 = 0; d0 < p.key_dim; d0 += 32) {
-    __syncthreads();
-#pragma unroll
-    for (uint32_t i = threadIdx.x * 8u; i < 32u * kCols; i += kBlock * 8u)
-      *reinterpret_cast<uint4 *>(w_s + i) = *reinterpret_cast<const uint4 *>(w + static_cast<uint64_t>(d0 + i / kCols) * R + i % kCols);
-    const float4 a = *reinterpret_cast<const float4 *>(q + d0 + 4u * q4), b = *reinterpret_cast<const float4 *>(q + d0 + 16u + 4u * q4);
-    const uint4 x = make_uint4(pack16(a.x, a.y), pack16(a.z, a.w), pack16(b.x, b.y), pack16(b.z, b.w));
-    __syncthreads();
-#pragma unroll
-    for (int i = 0; i < RT; i += 2) {
-      u32x2_t lo[2], hi[2];
-      asm volatile("ds_read_b64_tr_b16 %0, %4 offset:%5\n\tds_read_b64_tr_b16 %1, %4 offset:%6\n\t"
-                   "ds_read_b64_tr_b16 %2, %4 offset:%7\n\tds_read_b64_tr_b16 %3, %4 offset:%8\n\ts_waitcnt lgkmcnt(0)"
-                   : "=&v"(lo[0]), "=&v"(hi[0]), "=&v"(lo[1]), "=&v"(hi[1])
-                   : "v"(at), "n"(i * 32), "n"(i * 32 + 16 * kCols * 2), "n"((i + 1) * 32), "n"((i + 1) * 32 + 16 * kCols * 2)
-                   : "memory");
-#pragma unroll
-      for (int j = 0; j < 2; ++j) acc[i + j] = mfma_k32<DT>(make_uint4(lo[j].x, lo[j].y, hi[j].x, hi[j].y), x, acc[i + j]);
-    }
+  // The weights and queries of four steps are asked for together: four round trips one behind the other were most of a decode step's launch.
+  for (uint32_t d = 0; d < p.key_dim; d += 128) {
+    AbsorbStep<RT> s0, s1, s2, s3;
+    const uint32_t last = p.key_dim - 32u;
+    absorb_request(s0, w, q, R, d, q4);
+    absorb_request(s1, w, q, R, min(d + 32u, last), q4);
+    absorb_request(s2, w, q, R, min(d + 64u, last), q4);
+    absorb_request(s3, w, q, R, min(d + 96u, last), q4);
+    absorb_step(s0, w_s, at, acc);
+    if (d + 32 < p.key_dim) absorb_step(s1, w_s, at, acc);
+    if (d + 64 < p.key_dim) absorb_step(s2, w_s, at, acc);
+    if (d + 96 < p.key_dim) absorb_step(s3, w_s, at, acc);
   }
   if (t >= p.tokens) return;
   uint16_t *out = q16 + (static_cast<uint64_t>(t) * p.heads + h) * width + c0 + 4u * q4;
@@ -152,13 +194,17 @@ constexpr size_t latent_rows_lds() {
 }
 
 template <int R, int RD, int PAIRS>
-__global__ __launch_bounds__(2 * PAIRS * kWave, 2) void latent_rows_kernel(LatentAttnParams p, uint32_t splits) {
+__global__ __launch_bounds__(2 * PAIRS * kWave, 2) void latent_rows_kernel(LatentAttnParams p, uint32_t splits, uint32_t own, RiderPairs riders) {
   constexpr uint32_t DT = kBF16;
   constexpr int D = R + RD, KS = D / 32, DTL = R / 32;        // K-steps of the scores, tiles of 16 latent columns a wave
   constexpr int kTileBytes = 16 * D * 2, kBuf = 2 * kTileBytes, kPieces = kBuf / 1024, kWaves = 2 * PAIRS;
   constexpr int KH = KS / 2;                                  // ... of a wave
   static_assert(KS % 2 == 0 && KH > 2 && DTL % 2 == 0 && D % 32 == 0, "whole groups");
   extern __shared__ __align__(16) unsigned char smem[];
+  if (blockIdx.x >= own) {   // (a decode step's riders, behind the workgroups of the rows)
+    layer::ride_pairs<DT, kWaves>(riders, p.cursor, p.max_steps, reinterpret_cast<uint16_t *>(smem), blockIdx.x - own, gridDim.x - own);
+    return;
+  }
   const uint32_t rows = p.tokens * p.heads;
   const uint32_t split = blockIdx.x % splits, row0 = blockIdx.x / splits * (PAIRS * kPairRows);
   const uint32_t lane = threadIdx.x & (kWave - 1), wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
@@ -508,10 +554,19 @@ __global__ __launch_bounds__(kBlock) void latent_merge_step_kernel(LatentAttnPar
 
 // Decode step: merges the splits of one head where that has not been done, then a wave a value column at a time.
 constexpr uint32_t kStepColumns = 16;   // value columns of a workgroup
-__global__ __launch_bounds__(kBlock) void latent_value_step_kernel(LatentAttnParams p, uint32_t splits, bool merged) {
+constexpr uint32_t kValueMaxRank = 512;  // (latent_attention_wide)
+__global__ __launch_bounds__(kBlock, 4) void latent_value_step_kernel(LatentAttnParams p, uint32_t splits, bool merged, LayerBack riders) {
   constexpr uint32_t DT = kBF16;
-  __shared__ __align__(16) float o_s[kLatentMaxRank];
+  __shared__ __align__(16) float o_s[kValueMaxRank], part_s[kWavesPerBlock * kValueMaxRank];
   __shared__ float f_s[kMostSplits], red[kWavesPerBlock];
+  if (blockIdx.z != 0) {   // (the grid's other layers are the riders')
+    extern __shared__ __align__(16) uint16_t rider_s[];
+    const uint32_t plane = gridDim.x * gridDim.y;
+    const uint32_t columns = layer::back_columns(0, riders.top, riders.ff, riders.shared_ff);
+    layer::walk_back<DT, kWavesPerBlock>(riders, rider_s, reinterpret_cast<layer::Chunk *>(rider_s + columns), (blockIdx.z - 1) * plane + blockIdx.y * gridDim.x + blockIdx.x,
+                                         (gridDim.z - 1) * plane);
+    return;
+  }
   const uint32_t pos = *p.cursor;
   if (pos >= p.max_steps) return;
   const uint32_t R = p.kv_rank, h = blockIdx.y, tid = threadIdx.x, lane = tid & (kWave - 1), wave = tid / kWave;
@@ -524,22 +579,46 @@ __global__ __launch_bounds__(kBlock) void latent_value_step_kernel(LatentAttnPar
     const uint32_t c = min(blockIdx.x * kStepColumns + wave + i * kWavesPerBlock, p.value_dim - 1);
     w[i] = *reinterpret_cast<const uint4 *>(p.w_uv + (static_cast<uint64_t>(h) * p.value_dim + c) * R + (lane * 8u < R ? lane * 8u : 0u));
   }
+  float gate[kStepColumns / kWavesPerBlock];
+#pragma unroll
+  for (uint32_t i = 0; i < kStepColumns / kWavesPerBlock; ++i)
+    gate[i] = p.proj[p.gate_col + h * p.value_dim + min(blockIdx.x * kStepColumns + wave + i * kWavesPerBlock, p.value_dim - 1)];
   if (merged) {
     for (uint32_t c = tid * 2u; c < R; c += kBlock * 2u) *reinterpret_cast<float2 *>(o_s + c) = *reinterpret_cast<const float2 *>(ws.sum + base * R + c);
   } else {
-    const float inv = step_factors(tid < splits ? ws.m[base + tid] : -INFINITY, tid < splits ? ws.l[base + tid] : 0.0f, splits, f_s, red);
+    // A wave takes every fourth split, four columns a lane (and 256 columns on); what it sums of the first eight is asked for before the splits'
+    // factors are known. The waves meet in LDS, in their order.
+    constexpr uint32_t kAhead = 8;
     const uint32_t used = used_splits(p, pos, splits);
-    for (uint32_t c = tid * 2u; c < R; c += kBlock * 2u) {
-      float2 o = make_float2(0.0f, 0.0f);
-#pragma unroll 16
-      for (uint32_t i = 0; i < used; ++i) {
-        const float2 v = *reinterpret_cast<const float2 *>(ws.sum + (base + i) * R + c);
-        o.x = fmaf(v.x, f_s[i], o.x);
-        o.y = fmaf(v.y, f_s[i], o.y);
-      }
-      o_s[c] = o.x * inv;
-      o_s[c + 1] = o.y * inv;
+    const float ms = tid < splits ? ws.m[base + tid] : -INFINITY, ls = tid < splits ? ws.l[base + tid] : 0.0f;
+    constexpr uint32_t kRuns = kValueMaxRank / (kWave * 4u);
+    float4 v[kRuns][kAhead];
+#pragma unroll
+    for (uint32_t j = 0; j < kRuns; ++j)
+#pragma unroll
+      for (uint32_t i = 0; i < kAhead; ++i)
+        v[j][i] = *reinterpret_cast<const float4 *>(ws.sum + (base + min(wave + i * kWavesPerBlock, used - 1)) * R + min((j * kWave + lane) * 4u, R - 4u));
+    const float inv = step_factors(ms, ls, splits, f_s, red);
+#pragma unroll
+    for (uint32_t j = 0; j < kRuns; ++j) {
+      const uint32_t c = (j * kWave + lane) * 4u;
+      if (c >= R) break;
+      float4 o = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+      const auto add = [&](const float4 &a, float f) {
+        o.x = fmaf(a.x, f, o.x);
+        o.y = fmaf(a.y, f, o.y);
+        o.z = fmaf(a.z, f, o.z);
+        o.w = fmaf(a.w, f, o.w);
+      };
+#pragma unroll
+      for (uint32_t i = 0; i < kAhead; ++i)
+        if (wave + i * kWavesPerBlock < used) add(v[j][i], f_s[wave + i * kWavesPerBlock]);
+      for (uint32_t i = wave + kAhead * kWavesPerBlock; i < used; i += kWavesPerBlock) add(*reinterpret_cast<const float4 *>(ws.sum + (base + i) * R + c), f_s[i]);
+      *reinterpret_cast<float4 *>(part_s + wave * R + c) = o;
     }
+    __syncthreads();
+    for (uint32_t c = tid; c < R; c += kBlock)
+      o_s[c] = ((part_s[c] + part_s[R + c]) + (part_s[2 * R + c] + part_s[3 * R + c])) * inv;
   }
   __syncthreads();
 #pragma unroll
@@ -560,7 +639,7 @@ __global__ __launch_bounds__(kBlock) void latent_value_step_kernel(LatentAttnPar
     }
     sum = wave_sum(sum);
     const uint32_t e = h * p.value_dim + c;
-    if (lane == 0) p.out16[p.packed_tiles != 0 ? gemm_x_packed_index(p.packed_tiles, 0, e) : e] = enc16<DT>(sum * sigmoid(p.proj[p.gate_col + e]));
+    if (lane == 0) p.out16[p.packed_tiles != 0 ? gemm_x_packed_index(p.packed_tiles, 0, e) : e] = enc16<DT>(sum * sigmoid(gate[i]));
   }
 }
 
@@ -575,25 +654,36 @@ uint32_t block_splits(uint32_t rows) {
   return std::max(1u, std::min(kBlockSplits, kWorkgroups / groups));
 }
 
+constexpr uint32_t kRiderBlocks = 768;   // of four waves: three a CU
+uint32_t rider_blocks(uint32_t units, uint32_t waves, uint32_t most) { return std::min(most, (units + waves - 1) / waves); }
+
 template <int R, int RD, int PAIRS>
-hipError_t launch_rows(const LatentAttnParams &p, uint32_t splits, hipStream_t stream) {
+hipError_t launch_rows(const LatentAttnParams &p, uint32_t splits, const RiderPairs &riders, hipStream_t stream) {
   constexpr size_t lds = latent_rows_lds<R, RD, PAIRS>();
   const uint32_t rows = p.tokens * p.heads, groups = (rows + PAIRS * kPairRows - 1) / (PAIRS * kPairRows);
-  hipLaunchKernelGGL((latent_rows_kernel<R, RD, PAIRS>), dim3(groups * splits), dim3(2 * PAIRS * kWave), lds, stream, p, splits);
+  // two workgroups a CU: those that the rows leave
+  const uint32_t own = groups * splits, ride = rider_blocks(riders.end - riders.begin, 2 * PAIRS, kWorkgroups > own + kWorkgroups / 2 ? kWorkgroups - own : kWorkgroups / 2);
+  hipLaunchKernelGGL((latent_rows_kernel<R, RD, PAIRS>), dim3(own + ride), dim3(2 * PAIRS * kWave), lds, stream, p, splits, own, riders);
   return hipGetLastError();
 }
 
 template <int R, int RD>
-hipError_t launch_shape(const LatentAttnParams &p, hipStream_t stream, uint64_t *launches) {
+hipError_t launch_shape(const LatentAttnParams &p, const LayerRiders &riders, hipStream_t stream, uint64_t *launches) {
   const bool step = p.cursor != nullptr;
   const uint32_t rows = p.tokens * p.heads, splits = step ? step_splits(p) : block_splits(rows);
   const Work ws = work_at(p.workspace, rows, R, R + RD, splits);
   const uint32_t token_tiles = (p.tokens + 63) / 64;
-  if (step) hipLaunchKernelGGL((latent_absorb_kernel<4>), dim3(R / 64 + 1, p.heads, 1), dim3(kBlock), 0, stream, p, ws.q16);
-  else hipLaunchKernelGGL((latent_absorb_kernel<8>), dim3(R / 128 + 1, p.heads, token_tiles), dim3(kBlock), 0, stream, p, ws.q16);
+  const auto planes = [](uint32_t blocks, uint32_t plane) { return (blocks + plane - 1) / plane; };
+  if (step) {
+    const RiderPairs &r = riders.absorb;
+    const uint32_t z = 1 + planes(rider_blocks(r.end - r.begin, kWavesPerBlock, kRiderBlocks), (R / 64 + 1) * p.heads);
+    hipLaunchKernelGGL((latent_absorb_kernel<4, true>), dim3(R / 64 + 1, p.heads, z), dim3(kBlock), z > 1 ? 2u * layer::padded(r.hidden) : 0u, stream, p, ws.q16, r);
+  } else {
+    hipLaunchKernelGGL((latent_absorb_kernel<8, false>), dim3(R / 128 + 1, p.heads, token_tiles), dim3(kBlock), 0, stream, p, ws.q16, RiderPairs{});
+  }
   hipError_t err = hipGetLastError();
   if (err != hipSuccess) return err;
-  err = rows > kPairRows ? launch_rows<R, RD, 2>(p, splits, stream) : launch_rows<R, RD, 1>(p, splits, stream);
+  err = rows > kPairRows ? launch_rows<R, RD, 2>(p, splits, riders.rows, stream) : launch_rows<R, RD, 1>(p, splits, riders.rows, stream);
   if (err != hipSuccess) return err;
   if (step) {
     const bool merged = splits > kStepMergeSplits;
@@ -603,8 +693,11 @@ hipError_t launch_shape(const LatentAttnParams &p, hipStream_t stream, uint64_t 
       err = hipGetLastError();
       if (err != hipSuccess) return err;
     }
-    hipLaunchKernelGGL(latent_value_step_kernel, dim3((p.value_dim + kStepColumns - 1) / kStepColumns, p.heads), dim3(kBlock), 0, stream, p, splits,
-                       merged);
+    const LayerBack &b = riders.back;
+    const uint32_t x = (p.value_dim + kStepColumns - 1) / kStepColumns, columns = b.y != nullptr ? layer::back_columns(0, b.top, b.ff, b.shared_ff) : 0u;
+    const uint32_t z = 1 + planes(b.y != nullptr ? rider_blocks(b.hidden, kWavesPerBlock, kRiderBlocks) : 0u, x * p.heads);
+    const size_t lds = z > 1 ? 2u * columns + (columns / layer::kChunk + layer::kBackBatch) * sizeof(layer::Chunk) : 0u;
+    hipLaunchKernelGGL(latent_value_step_kernel, dim3(x, p.heads, z), dim3(kBlock), lds, stream, p, splits, merged, b);
     return hipGetLastError();
   }
   *launches += splits > 1 ? 4 : 3;
@@ -636,6 +729,11 @@ bool latent_attention_wide(uint32_t heads, uint32_t key_dim, uint32_t rot_dim, u
   return shape && heads != 0 && key_dim % 32 == 0 && value_dim % 16 == 0 && (key_dim + rot_dim) % 4 == 0;
 }
 
+bool latent_riders_fit(uint32_t kv_rank, uint32_t hidden, uint32_t top, uint32_t ff, uint32_t shared_ff) {
+  const uint32_t rows = 2u * kUnitKeys * (kv_rank + 64u) * 2u, columns = layer::back_columns(0, top, ff, shared_ff);
+  return 2u * layer::padded(hidden) <= std::min<uint32_t>(rows, 32u * 1024u) && 2u * columns <= 36u * 1024u;   // (beside the launches' own LDS, four workgroups a CU)
+}
+
 uint64_t latent_workspace_bytes(uint32_t heads, uint32_t rot_dim, uint32_t kv_rank, uint32_t max_tokens) {
   const uint64_t width = kv_rank + rot_dim, partial = (kv_rank + 2ull) * sizeof(float);
   const auto total = [&](uint64_t rows, uint64_t splits) {
@@ -657,7 +755,7 @@ hipError_t latent_wide_setup() {
   return raised;
 }
 
-hipError_t launch_latent_attention_wide(uint32_t dtype, const LatentAttnParams &p, hipStream_t stream, uint64_t *launches) {
+hipError_t launch_latent_attention_wide(uint32_t dtype, const LatentAttnParams &p, const LayerRiders &riders, hipStream_t stream, uint64_t *launches) {
   const auto aligned = [](const void *q, uintptr_t n) { return (reinterpret_cast<uintptr_t>(q) & (n - 1)) == 0; };
   if (dtype != kBF16 || !latent_attention_wide(p.heads, p.key_dim, p.rot_dim, p.value_dim, p.kv_rank) || p.cache32 != 0 || p.out16 == nullptr ||
       p.workspace == nullptr || p.proj == nullptr || p.q == nullptr || p.w_uk == nullptr || p.w_uv == nullptr || p.cache == nullptr ||
@@ -666,10 +764,14 @@ hipError_t launch_latent_attention_wide(uint32_t dtype, const LatentAttnParams &
     return hipErrorInvalidValue;
   if (!aligned(p.workspace, 256) || !aligned(p.cache, 16) || !aligned(p.w_uk, 16) || !aligned(p.w_uv, 16) || !aligned(p.q, 16) || !aligned(p.out16, 16))
     return hipErrorInvalidValue;
+  const bool rides = riders.absorb.begin != riders.absorb.end || riders.rows.begin != riders.rows.end || riders.back.y != nullptr;
+  if (rides && (p.cursor == nullptr || !latent_riders_fit(p.kv_rank, riders.back.hidden, riders.back.top, riders.back.ff, riders.back.shared_ff) ||
+                riders.absorb.begin > riders.absorb.end || riders.rows.begin > riders.rows.end || riders.back.mix_cols != 0))
+    return hipErrorInvalidValue;
   if (p.cursor != nullptr ? p.tokens != 1 : (p.position + p.tokens - 1) / kKvBlockTokens > p.last_block) return hipErrorInvalidValue;
-  if (p.kv_rank == 512) return launch_shape<512, 64>(p, stream, launches);
-  if (p.kv_rank == 256) return launch_shape<256, 64>(p, stream, launches);
-  return launch_shape<128, 64>(p, stream, launches);
+  if (p.kv_rank == 512) return launch_shape<512, 64>(p, riders, stream, launches);
+  if (p.kv_rank == 256) return launch_shape<256, 64>(p, riders, stream, launches);
+  return launch_shape<128, 64>(p, riders, stream, launches);
 }
 
 }  // namespace nv

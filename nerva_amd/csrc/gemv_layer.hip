@@ -3,25 +3,17 @@
 
 #include <algorithm>
 
-#include "activations.cuh"
-#include "gemv_stream.cuh"
+#include "gemv_layer_walk.cuh"
 #include "moe_rows.cuh"
 
 namespace nv {
 
 namespace {
 
+using namespace layer;
+
 constexpr int kWaves = 8, kThreads = kWaves * kWave;
-constexpr uint32_t kChunk = kWave * 8;       // columns of a load instruction
 constexpr uint32_t kMaxWorkgroups = 512;     // two a CU
-constexpr size_t kMaxLds = 56 * 1024;
-__host__ __device__ __forceinline__ uint32_t padded(uint32_t cols) { return (cols + kChunk - 1) / kChunk * kChunk; }
-
-// Zeros behind a staged vector, up to a whole chunk (the weights there are taken as zero as well).
-__device__ __forceinline__ void clear_tail(uint16_t *xs, uint32_t cols) {
-  for (uint32_t c = cols + threadIdx.x; c < padded(cols); c += kThreads) xs[c] = 0;
-}
-
 // round16(x * rsqrt(mean(x^2) + eps) * gamma) of a row, for one or two gammas. cols % 8 == 0.
 template <uint32_t DT>
 __device__ __forceinline__ void rms_stage(const float *x, uint32_t cols, float eps, const uint16_t *g0, uint16_t *xs0, const uint16_t *g1,
@@ -48,105 +40,11 @@ __device__ __forceinline__ void rms_stage(const float *x, uint32_t cols, float e
     put(g0, xs0);
     if (g1 != nullptr) put(g1, xs1);
   }
-  clear_tail(xs0, cols);
-  if (g1 != nullptr) clear_tail(xs1, cols);
+  clear_tail<kThreads>(xs0, cols);
+  if (g1 != nullptr) clear_tail<kThreads>(xs1, cols);
 }
 
 // ---- front, middle ---------------------------------------------------------------------------
-
-// Two rows of weights that a wave walks together, and what becomes of their sums.
-struct Unit {
-  const uint16_t *w0, *w1;
-  uint32_t at;             // the staged input's place in LDS
-  uint32_t cols;
-  float *out0, *out1;      // plain rows (out1 null: there is no second one)
-  uint16_t *act;           // gate and up row: one activation
-  float limit;
-};
-
-constexpr int kBatch = 4;   // chunks of a request batch: 4 KiB of each row
-
-// A wave's walk over its units first, first + stride, .. < units; unit_at(i) -> Unit (i is wave-uniform). The first two
-// batches of weights are requested by start(), which does not need the staged inputs.
-template <uint32_t DT, typename At>
-struct PairWalk {
-  At unit_at;
-  uint32_t units, stride, lane;
-  uint4 b0[2][kBatch], b1[2][kBatch];
-  uint32_t iu, ic;      // next batch to request: unit, first column
-  Unit in;
-  uint32_t cu, cc;      // next batch to multiply
-  Unit cur;
-  float acc0, acc1;
-
-  __device__ __forceinline__ PairWalk(At at, uint32_t n, uint32_t first, uint32_t step)
-      : unit_at(at), units(n), stride(step), lane(threadIdx.x & (kWave - 1)), iu(first), ic(0), in{}, cu(first), cc(0), cur{}, acc0(0.0f), acc1(0.0f) {}
-  __device__ __forceinline__ void issue(uint4 (&to)[2][kBatch]) {
-    if (iu >= units) return;
-#pragma unroll
-    for (int u = 0; u < kBatch; ++u) {
-      const uint32_t c = ic + u * kChunk + lane * 8u;
-      const bool on = c < in.cols;
-      to[0][u] = on ? load_stream(in.w0 + c) : make_uint4(0u, 0u, 0u, 0u);
-      to[1][u] = on ? load_stream(in.w1 + c) : make_uint4(0u, 0u, 0u, 0u);
-    }
-    ic += kBatch * kChunk;
-    if (ic >= in.cols) {
-      ic = 0;
-      iu += stride;
-      if (iu < units) in = unit_at(iu);
-    }
-  }
-  __device__ __forceinline__ void consume(const uint4 (&from)[2][kBatch], const uint16_t *xs) {
-#pragma unroll
-    for (int u = 0; u < kBatch; ++u) {
-      if (cc + u * kChunk < cur.cols) {
-        const uint4 x = *reinterpret_cast<const uint4 *>(xs + cur.at + cc + u * kChunk + lane * 8u);
-        acc0 = dot8<DT, true>(from[0][u], x, acc0);
-        acc1 = dot8<DT, true>(from[1][u], x, acc1);
-      }
-    }
-    cc += kBatch * kChunk;
-    if (cc < cur.cols) return;
-    acc0 = wave_sum(acc0);
-    acc1 = wave_sum(acc1);
-    if (lane == 0) {
-      if (cur.act != nullptr) {
-        *cur.act = enc16<DT>(clamped_glu(acc0, acc1, cur.limit));
-      } else {
-        *cur.out0 = acc0;
-        if (cur.out1 != nullptr) *cur.out1 = acc1;
-      }
-    }
-    acc0 = acc1 = 0.0f;
-    cc = 0;
-    cu += stride;
-    if (cu < units) cur = unit_at(cu);
-  }
-  __device__ __forceinline__ void start() {
-    if (iu < units) in = cur = unit_at(iu);
-    issue(b0);
-    issue(b1);
-  }
-  __device__ __forceinline__ void run(const uint16_t *xs) {
-    while (cu < units) {
-      consume(b0, xs);
-      issue(b0);
-      if (cu >= units) break;
-      consume(b1, xs);
-      issue(b1);
-    }
-  }
-};
-
-__device__ __forceinline__ Unit two_rows(const uint16_t *w, uint32_t cols, uint32_t rows, uint32_t i, uint32_t at, float *out) {
-  const uint32_t r0 = 2u * i, r1 = min(r0 + 1u, rows - 1u);
-  return Unit{w + static_cast<uint64_t>(r0) * cols, w + static_cast<uint64_t>(r1) * cols, at, cols, out + r0, r0 + 1u < rows ? out + r1 : nullptr,
-              nullptr, 0.0f};
-}
-__device__ __forceinline__ Unit gate_and_up(const uint16_t *w, uint32_t cols, uint32_t ff, uint32_t i, uint32_t at, uint16_t *act, float limit) {
-  return Unit{w + static_cast<uint64_t>(i) * cols, w + static_cast<uint64_t>(ff + i) * cols, at, cols, nullptr, nullptr, act + i, limit};
-}
 
 template <uint32_t DT>
 __global__ __launch_bounds__(kThreads, 4) void layer_front_kernel(LayerFront p) {
@@ -172,154 +70,82 @@ __global__ __launch_bounds__(kThreads, 4) void layer_front_kernel(LayerFront p) 
   walk.run(xs);
 }
 
-template <uint32_t DT>
+template <uint32_t DT, bool RIDES>
 __global__ __launch_bounds__(kThreads, 4) void layer_middle_kernel(LayerMiddle p) {
   extern __shared__ __align__(16) uint16_t xs[];   // the query latent, the feed-forward's row
   __shared__ float red[kWaves];
   __shared__ float score[kMaxExperts];
   __shared__ uint32_t id_s[kMaxTop];
   __shared__ float s_s[kMaxTop];
-  if (*p.cursor >= p.max_steps) return;
   uint16_t *xs2 = xs + padded(p.q_rank);
   const uint32_t tid = threadIdx.x;
-  for (uint32_t e = tid; e < p.experts; e += kThreads) score[e] = 1.0f / (1.0f + expf(-p.logits[e]));
-  if (tid < kMaxTop) {   // (scores that are no numbers choose nothing: some expert that exists)
-    id_s[tid] = 0u;
-    s_s[tid] = 0.0f;
-  }
-  __syncthreads();
-  // an expert's place is the number of experts ahead of it
-  for (uint32_t e = tid; e < p.experts; e += kThreads) {
-    const float s = score[e];
-    uint32_t ahead = 0;
-#pragma unroll 8
-    for (uint32_t j = 0; j < p.experts; ++j) ahead += score[j] > s || (score[j] == s && j < e) ? 1u : 0u;
-    if (ahead < p.top) {
-      id_s[ahead] = e;
-      s_s[ahead] = s;
+  const auto choose = [&] {
+    for (uint32_t e = tid; e < p.experts; e += kThreads) score[e] = 1.0f / (1.0f + expf(-p.logits[e]));
+    if (tid < kMaxTop) {   // (scores that are no numbers choose nothing: some expert that exists)
+      id_s[tid] = 0u;
+      s_s[tid] = 0.0f;
     }
+    __syncthreads();
+    // an expert's place is the number of experts ahead of it
+    for (uint32_t e = tid; e < p.experts; e += kThreads) {
+      const float s = score[e];
+      uint32_t ahead = 0;
+#pragma unroll 8
+      for (uint32_t j = 0; j < p.experts; ++j) ahead += score[j] > s || (score[j] == s && j < e) ? 1u : 0u;
+      if (ahead < p.top) {
+        id_s[ahead] = e;
+        s_s[ahead] = s;
+      }
+    }
+    __syncthreads();
+  };
+  const auto publish = [&] {
+    if (tid >= p.top) return;
+    float sum = 0.0f;
+    for (uint32_t k = 0; k < p.top; ++k) sum += s_s[k];
+    p.ids[tid] = id_s[tid];
+    p.weights[tid] = s_s[tid] / (sum + 1e-20f);
+  };
+  if constexpr (RIDES) {
+    if (blockIdx.x == gridDim.x - 1) {   // a workgroup of its own: who is chosen is wanted by the next launch
+      if (*p.cursor >= p.max_steps) return;
+      choose();
+      publish();
+      return;
+    }
+  } else if (p.experts != 0) {
+    choose();   // (whose rows this launch walks, everyone has to know)
   }
-  __syncthreads();
+  const uint32_t blocks = gridDim.x - (RIDES ? 1u : 0u);
   const uint32_t wave = __builtin_amdgcn_readfirstlane(tid / kWave);
-  const uint32_t n_experts = p.experts != 0 ? p.top * p.ff : 0u, units = n_experts + (p.q_rows + 1) / 2;
+  const uint32_t pairs = RIDES ? p.shared_ff : p.experts != 0 ? p.top * p.ff : 0u, units = pairs + (p.q_rows + 1) / 2;
   const auto unit_at = [&](uint32_t i) {
-    if (i >= n_experts) return two_rows(p.w_uq, p.q_rank, p.q_rows, i - n_experts, 0u, p.q);
+    if (i >= pairs) return two_rows(p.w_uq, p.q_rank, p.q_rows, i - pairs, 0u, p.q);
+    if (RIDES) return gate_and_up(p.shared_in, p.hidden, p.shared_ff, i, padded(p.q_rank), p.shared_act, p.shared_limit);
     const uint32_t k = i / p.ff, e = __builtin_amdgcn_readfirstlane(id_s[k]);
     return gate_and_up(p.e_in + static_cast<uint64_t>(e) * 2u * p.ff * p.hidden, p.hidden, p.ff, i - k * p.ff, padded(p.q_rank), p.act + k * p.ff,
                        p.limit);
   };
-  PairWalk<DT, decltype(unit_at)> walk(unit_at, units, wave * gridDim.x + blockIdx.x, gridDim.x * kWaves);
+  PairWalk<DT, decltype(unit_at)> walk(unit_at, units, wave * blocks + blockIdx.x, blocks * kWaves);
   walk.start();
-  if (p.experts != 0) {
-    for (uint32_t c = tid * 8u; c < p.hidden; c += kThreads * 8u) *reinterpret_cast<uint4 *>(xs2 + c) = *reinterpret_cast<const uint4 *>(p.h16 + c);
-    clear_tail(xs2, p.hidden);
-    if (blockIdx.x == 0 && tid < p.top) {
-      float sum = 0.0f;
-      for (uint32_t k = 0; k < p.top; ++k) sum += s_s[k];
-      p.ids[tid] = id_s[tid];
-      p.weights[tid] = s_s[tid] / (sum + 1e-20f);
-    }
-  }
+  if (*p.cursor >= p.max_steps) return;   // (after the requests, which do not depend on it)
+  if (pairs != 0) stage_vector<kThreads>(xs2, p.h16, p.hidden);
   rms_stage<DT>(p.latent, p.q_rank, p.eps, p.latent_norm, xs, nullptr, nullptr, red);
   __syncthreads();
+  if (!RIDES && p.experts != 0 && blockIdx.x == 0) publish();
   walk.run(xs);
 }
 
 // ---- back ------------------------------------------------------------------------------------
 
-// A row's columns are the pieces' columns one after the other, each piece padded to whole chunks, as their inputs lie in
-// LDS. A chunk: where it starts in row 0, bytes from row to row, lanes that have columns, what its products are worth.
-struct Chunk {
-  uint64_t base;
-  uint16_t stride, lanes;
-  float factor;
-};
-static_assert(sizeof(Chunk) == 16, "one LDS read");
-constexpr uint32_t kMaxChunks = kMaxLds / (2 * kChunk);
-constexpr int kBackBatch = 8;   // chunks of a request batch
-
 template <uint32_t DT>
 __global__ __launch_bounds__(kThreads, 4) void layer_back_kernel(LayerBack p) {
   extern __shared__ __align__(16) uint16_t xs[];   // the pieces' inputs
   __shared__ __align__(16) Chunk table[kMaxChunks + kBackBatch];
-  if (*p.cursor >= p.max_steps) return;
-  const uint32_t tid = threadIdx.x, lane = tid & (kWave - 1), wave = __builtin_amdgcn_readfirstlane(tid / kWave);
-  const uint32_t expert_at = padded(p.mix_cols), shared_at = expert_at + p.top * padded(p.ff);
-  const uint32_t chunks = (shared_at + padded(p.shared_ff)) / kChunk, batches = (chunks + kBackBatch - 1) / kBackBatch;
-  if (tid < batches * kBackBatch) {
-    const uint32_t at = tid * kChunk;
-    const uint16_t *base = p.w_o;
-    uint32_t cols = p.mix_cols, c = at;
-    float factor = 1.0f;
-    if (at >= shared_at) {
-      base = p.shared_out;
-      cols = p.shared_ff;
-      c = at - shared_at;
-    } else if (at >= expert_at) {
-      const uint32_t k = (at - expert_at) / padded(p.ff);
-      base = p.e_out + static_cast<uint64_t>(p.ids[k]) * p.hidden * p.ff;
-      cols = p.ff;
-      c = at - expert_at - k * padded(p.ff);
-      factor = p.weights[k];
-    }
-    const uint32_t lanes = tid < chunks ? min((cols - c) / 8u, static_cast<uint32_t>(kWave)) : 0u;   // (the last batch's chunks past the end)
-    table[tid] = Chunk{reinterpret_cast<uint64_t>(base) + 2u * (lanes != 0 ? c : 0u), static_cast<uint16_t>(2u * cols), static_cast<uint16_t>(lanes), factor};
-  }
-  __syncthreads();
-  const uint32_t stride = gridDim.x * kWaves;
-  uint4 b0[kBackBatch], b1[kBackBatch];
-  uint32_t irow = wave * gridDim.x + blockIdx.x, ib = 0, crow = irow, cb = 0;
-  float total = 0.0f;
-  const auto issue = [&](uint4 (&to)[kBackBatch]) {
-    if (irow >= p.hidden) return;
-#pragma unroll
-    for (int u = 0; u < kBackBatch; ++u) {
-      const Chunk k = table[ib * kBackBatch + u];
-      to[u] = make_uint4(0u, 0u, 0u, 0u);
-      if (lane < k.lanes) to[u] = load_stream(reinterpret_cast<const char *>(k.base) + static_cast<uint64_t>(irow) * k.stride + lane * 16u);
-    }
-    if (++ib == batches) {
-      ib = 0;
-      irow += stride;
-    }
-  };
-  const auto consume = [&](const uint4 (&from)[kBackBatch]) {
-#pragma unroll
-    for (int u = 0; u < kBackBatch; ++u) {
-      const uint32_t i = cb * kBackBatch + u;
-      if (i < chunks) total = fmaf(table[i].factor, dot8<DT, true>(from[u], *reinterpret_cast<const uint4 *>(xs + i * kChunk + lane * 8u), 0.0f), total);
-    }
-    if (++cb < batches) return;
-    total = wave_sum(total);
-    if (lane == 0) p.x[crow] += total;
-    total = 0.0f;
-    cb = 0;
-    crow += stride;
-  };
-  issue(b0);
-  issue(b1);
-  // the inputs, under the first requests
-  const auto stage = [&](const uint16_t *src, uint32_t cols, uint32_t at) {
-    for (uint32_t c = tid * 8u; c < cols; c += kThreads * 8u) *reinterpret_cast<uint4 *>(xs + at + c) = *reinterpret_cast<const uint4 *>(src + c);
-    clear_tail(xs + at, cols);
-  };
-  stage(p.mixed, p.mix_cols, 0);
-  for (uint32_t k = 0; k < p.top; ++k) stage(p.act + k * p.ff, p.ff, expert_at + k * padded(p.ff));
-  if (p.shared_ff != 0) stage(p.shared_act, p.shared_ff, shared_at);
-  __syncthreads();
-  while (crow < p.hidden) {
-    consume(b0);
-    issue(b0);
-    if (crow >= p.hidden) break;
-    consume(b1);
-    issue(b1);
-  }
+  walk_back<DT, kWaves>(p, xs, table, blockIdx.x, gridDim.x);
 }
 
 uint32_t workgroups(uint32_t units) { return std::max(1u, std::min(kMaxWorkgroups, (units + kWaves - 1) / kWaves)); }
-size_t back_columns(uint32_t mix_cols, uint32_t top, uint32_t ff, uint32_t shared_ff) {
-  return static_cast<size_t>(padded(mix_cols)) + static_cast<size_t>(top) * padded(ff) + padded(shared_ff);
-}
 bool whole(const void *p) { return (reinterpret_cast<uintptr_t>(p) & 15u) == 0; }
 
 }  // namespace
@@ -349,14 +175,16 @@ hipError_t launch_layer_middle(uint32_t dtype, const LayerMiddle &p, hipStream_t
                           p.ff == 0 || p.act == nullptr || p.ids == nullptr || p.weights == nullptr)) ||
       !whole(p.latent) || !whole(p.latent_norm) || !whole(p.w_uq) || !whole(p.h16) || !whole(p.e_in))
     return hipErrorInvalidValue;
-  const uint32_t units = (p.q_rows + 1) / 2 + (p.experts != 0 ? p.top * p.ff : 0u);
+  if (p.rides != 0 && (p.experts == 0 || (p.shared_ff != 0 && (p.shared_in == nullptr || p.shared_act == nullptr || !whole(p.shared_in))))) return hipErrorInvalidValue;
+  const uint32_t units = (p.q_rows + 1) / 2 + (p.rides != 0 ? p.shared_ff : p.experts != 0 ? p.top * p.ff : 0u);
   const size_t lds = 2u * (padded(p.q_rank) + (p.experts != 0 ? padded(p.hidden) : 0u));
-  hipLaunchKernelGGL(layer_middle_kernel<kBF16>, dim3(workgroups(units)), dim3(kThreads), lds, stream, p);
+  if (p.rides != 0) hipLaunchKernelGGL((layer_middle_kernel<kBF16, true>), dim3(workgroups(units) + 1), dim3(kThreads), lds, stream, p);
+  else hipLaunchKernelGGL((layer_middle_kernel<kBF16, false>), dim3(workgroups(units)), dim3(kThreads), lds, stream, p);
   return hipGetLastError();
 }
 
 hipError_t launch_layer_back(uint32_t dtype, const LayerBack &p, hipStream_t stream) {
-  if (dtype != kBF16 || p.x == nullptr || p.w_o == nullptr || p.mixed == nullptr || p.hidden == 0 || p.mix_cols == 0 || p.cursor == nullptr ||
+  if (dtype != kBF16 || p.x == nullptr || p.w_o == nullptr || p.mixed == nullptr || p.hidden == 0 || p.mix_cols == 0 || p.y != nullptr || p.cursor == nullptr ||
       !layer_gemv_takes(8, 8, p.mix_cols, 0, p.top, p.top != 0 ? p.ff : 0, p.shared_ff) ||
       (p.top != 0 && (p.e_out == nullptr || p.act == nullptr || p.ids == nullptr || p.weights == nullptr || p.ff == 0)) ||
       (p.shared_ff != 0 && (p.shared_out == nullptr || p.shared_act == nullptr)) || !whole(p.w_o) || !whole(p.mixed) || !whole(p.e_out) ||

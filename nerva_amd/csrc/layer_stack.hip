@@ -304,6 +304,10 @@ hipError_t parallel_step_16(Session *s) {
     const StackLayer &w = m.layers[l];
     const NervaHipStackLayer &d = w.spec;
     const MoePlan plan = moe_plan_at(s->pplan, 1, d.experts_per_token, d.experts, true);
+    const bool fast = takes_latent_wide(s, d);
+    // Most of the feed-forward rides with the attention's three launches, which are latency and leave most of the chip idle: the experts'
+    // gate and up rows with the first two, the way back with the third.
+    const bool rides = fast && d.experts != 0 && latent_riders_fit(d.kv_rank, s->hidden, d.experts_per_token, d.expert_ff, d.shared_ff);
     LayerFront f{};
     f.x = s->x;
     f.mixer_norm = w.norm[0];
@@ -317,7 +321,7 @@ hipError_t parallel_step_16(Session *s) {
     f.experts = d.experts;
     f.logits = s->prouter;
     f.shared_in = w.shared_in;
-    f.shared_ff = d.shared_ff;
+    f.shared_ff = rides ? 0u : d.shared_ff;
     f.shared_limit = d.shared_limit;
     f.shared_act = s->ff16;
     f.h16 = static_cast<uint16_t *>(s->pxn2);
@@ -339,6 +343,11 @@ hipError_t parallel_step_16(Session *s) {
     g.top = d.experts_per_token;
     g.e_in = w.e_in;
     g.ff = d.expert_ff;
+    g.rides = rides;
+    g.shared_in = w.shared_in;
+    g.shared_ff = d.shared_ff;
+    g.shared_limit = d.shared_limit;
+    g.shared_act = s->ff16;
     g.limit = d.expert_limit;
     g.act = static_cast<uint16_t *>(s->pff);
     g.ids = plan.ids;
@@ -350,10 +359,8 @@ hipError_t parallel_step_16(Session *s) {
     a.cursor = s->state;
     a.tokens = 1;
     a.out16 = s->attn16;
-    const bool fast = takes_latent_wide(s, d);
     if (!fast) a.q_latent16 = static_cast<uint16_t *>(s->pql);   // (the middle launch has its own)
     if (err == hipSuccess && !fast) err = launch_latent_prepare(s->dtype, a, st);
-    if (err == hipSuccess) err = fast ? launch_latent_attention_wide(s->dtype, a, st, &launches) : launch_latent_attention(s->dtype, a, st);
     LayerBack b{};
     b.x = s->x;
     b.hidden = s->hidden;
@@ -371,6 +378,20 @@ hipError_t parallel_step_16(Session *s) {
     b.shared_ff = d.shared_ff;
     b.cursor = s->state;
     b.max_steps = s->max_ctx;
+    LayerRiders riders{};
+    if (rides) {
+      const uint32_t pairs = d.experts_per_token * d.expert_ff;
+      riders.absorb = RiderPairs{f.h16, w.e_in, plan.ids, s->hidden, d.expert_ff, 0u, pairs / 2, d.expert_limit, g.act};
+      riders.rows = riders.absorb;
+      riders.rows.begin = riders.absorb.end;
+      riders.rows.end = pairs;
+      riders.back = b;
+      riders.back.mix_cols = 0;
+      riders.back.y = s->y;
+      b.top = b.shared_ff = 0;
+      b.add = s->y;
+    }
+    if (err == hipSuccess) err = fast ? launch_latent_attention_wide(s->dtype, a, riders, st, &launches) : launch_latent_attention(s->dtype, a, st);
     if (err == hipSuccess) err = launch_layer_back(s->dtype, b, st);
     launches += 3 + (fast ? 0 : 2);
   }
@@ -514,7 +535,7 @@ struct Block {
       err = launch_latent_prepare(s->dtype, a, s->stream);
       if (err == hipSuccess) err = project(kGemmF32, w.w_uq, w.q_rows(), w.spec.q_rank, s->pql, q_tiles, s->pq, 0, nullptr);
       const bool fast = takes_latent_wide(s, w.spec);
-      if (err == hipSuccess) err = fast ? launch_latent_attention_wide(s->dtype, a, s->stream, &launches) : launch_latent_attention(s->dtype, a, s->stream);
+      if (err == hipSuccess) err = fast ? launch_latent_attention_wide(s->dtype, a, LayerRiders{}, s->stream, &launches) : launch_latent_attention(s->dtype, a, s->stream);
       launches += fast ? 0 : 1;
     } else if (w.spec.mixer == NERVA_HIP_MIXER_ATTENTION) {
       MixedAttnParams a = attention_params(s, w, s->pqkv, s->prope);

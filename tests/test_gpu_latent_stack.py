@@ -274,6 +274,27 @@ def test_wide_layers_take_the_streaming_kernels():
     s.destroy()
 
 
+@pytest.mark.parametrize("change", [dict(experts=3, top=1, ff=8), dict(experts=7, top=3, ff=24, shared=0), dict(experts=5, top=5, ff=1032, shared=520),
+                                    dict(heads=34, experts=4, top=3, ff=136, shared=8), dict(kv_rank=256, vdim=48, experts=9, top=4, ff=72, shared=136),
+                                    dict(experts=20, top=20, ff=1024, shared=64), dict(experts=0, top=0, ff=0, shared=0)], ids=str)
+def test_feed_forwards_beside_a_steps_attention(change):
+    """Decode steps whose feed-forward rides with the attention's launches: one pair a workgroup, halves that are not even, part chunks, no shared
+    expert, more rows than a pair of waves has, as many experts as there are; one whose way back is too wide to ride, and none at all. Contexts
+    of one split, of more than a wave asks for ahead, and of more than the step merges by itself."""
+    shape = dict(heads=5, dim=32, rot_dim=64, vdim=32, q_rank=40, kv_rank=128, window=4000, limit=1.2, shared=24, shared_limit=1.1)
+    shape.update(change)
+    cfg = M.parallel_config([M.latent(**shape)] * 2, width=136, vocab=64)
+    tensors = M.weights(cfg, seed=21)
+    if shape["experts"]:
+        tensors = M.clear_routes(cfg, tensors)
+    tokens = tokens_of(cfg, 1720, seed=3)
+    want, _ = M.oracle_model(cfg, tensors).run(tokens)
+    s = M.session(cfg, tensors, 1730)
+    got = M.feed(s, tokens, [1, 1, 14, 1, 1, 1100, 1, 1, 590, 1, 1, 7, 1])
+    assert M.errors(got, want).max() < HALF
+    s.destroy()
+
+
 @pytest.mark.parametrize("sizes", [[700], [400, 90, 80, 2, 1, 127]], ids=str)
 def test_experts_with_many_tokens(sizes):
     """Blocks in which an expert has enough tokens for the large tiles: whole steps, rows past the last tile, uneven experts."""
