@@ -435,11 +435,17 @@ constexpr int fast_waves_per_simd(int prologue) { return prologue == kProJoin ? 
 constexpr int kFastMaxCols = 12288;  // x staged through at most 6 x 16 B per lane in registers ...
 constexpr int kFastMaxColsLoop = 30720;  // ... or, with a 16-bit input, copied into LDS behind the first weight requests
 
-// EXACT (short launches: a wave's whole share is the two batches requested up front, so the start-up is
-// the launch): the first two batches and the residual element are requested unconditionally - a wave
-// without a row asks for the last row's data and drops it - so that the compiler can count the requests
-// behind the activation loads and waits for exactly those before the prologue, which then runs under
-// the weights' latency. With the requests under `if (total > n)` it waits for everything.
+// The requests run free of the waits: the first two batches, with the residual element, are asked for unconditionally behind the
+// activations - a wave without a row asks for the last one's data, one without a second batch (kWalkOne aside) for its row's again - and in
+// the loop the batch after next is, so that the compiler can count what is on its way behind what it needs: with the requests under
+// `if (total > n)`, or through pointers that it takes for flat ones (global_u16), it waits for everything - the prologue for the first weights, every batch
+// for the next one's. us before -> after: gate/up pairs 8192 x 2048 13.5 -> 12.1, 2560 wide qkv 8.4 -> 7.3, o 6.4 -> 5.5, down 10.5 -> 9.9, 3584 wide o 7.5 -> 6.4,
+// down 25.4 -> 24.1, behind a join at 4096 columns 19.5 -> 19.0, 19.8 -> 18.9 (minGRU), 15.9 -> 14.8 (qkv); decode steps 2048 wide 2.6 % less in all, 2560 wide
+// 1.6 %. Launches with many batches a wave and enough waves on their way gain nothing (pairs of 12288 x 4096 31.0, down 16.8), and two lose, which keep the waits (kLoose): the head
+// (256 workgroups of 16 waves 82.6 -> 84.3) and the rotated qkv projection (9.67 -> 9.89).
+// WALK: kWalkOne where a wave's share is one batch - the second request, which is not used, made those launches 10 % longer -; kWalkLoops where the norm's
+// row does not fit the registers (its loops would be on the way to every wait, too).
+// EXACT: the shape in which everything about that is a constant (two batches a row, the input in registers): o at 4096 columns 7.5 -> 7.2 us.
 // WG: waves per workgroup (4 or 16; 8 with the join prologue). Every workgroup fetches the whole input vector (and for the RMSNorm
 // prologue the norm weights) for itself, so fewer, larger workgroups move that much less through the L2s ahead of
 // the weights; the waves' work is the same whatever the size (wave_global = workgroup x WG + wave).
@@ -461,12 +467,14 @@ constexpr int kFastMaxColsLoop = 30720;  // ... or, with a 16-bit input, copied 
 // end ask for the row's last piece again (one cache line for all of them) and leave it out of the sum. What the general
 // kernel, with its ~150 registers, took 11.8 / 43.5 / 24.6 / 176 us for at a width of 3584 (qkv, gate/up pairs of 18944,
 // down, a head of 152064 rows) takes 8.4 / 42.1 / 23.6 / 158; 20.4 us for pairs of 9728 x 2560 is 17.1.
+enum : int { kWalkRegs = 0, kWalkLoops = 1, kWalkOne = 2 };
 template <uint32_t DT, int PRO, int EPI, int NR, int B, bool EXACT = false, int WG = kWavesPerBlock, bool XREG = false,
-          bool ROT = false, bool RAGGED = false>
+          bool ROT = false, bool RAGGED = false, int WALK = kWalkRegs>
 __global__ __launch_bounds__(WG *kWave, XREG ? 4 : PRO == kProJoin && WG == 8 ? 2 : fast_waves_per_simd(PRO)) void gemv_fast_kernel(GemvParams p) {
   static_assert(!(ROT && (XREG || EXACT)), "the rotated walk has no exact-start or register-input variant");
   static_assert(!(RAGGED && (XREG || EXACT)), "nor have ragged rows");
   constexpr int TB = WG * kWave;
+  constexpr bool kLoose = EPI == kEpiArgmax || (PRO == kProRmsNorm && EPI == kEpiF32 && ROT && !RAGGED);
   constexpr uint32_t kXregBpr = 8 / B;   // batches per 4096-column row
   extern __shared__ __align__(16) uint16_t xs[];
   __shared__ float red[PRO == kProJoin ? WG * 3 : WG];
@@ -489,7 +497,7 @@ __global__ __launch_bounds__(WG *kWave, XREG ? 4 : PRO == kProJoin && WG == 8 ? 
   uint4 xraw[PRO == kProX16 ? kXV : 1];
   float4 xa[PRO == kProRmsNorm ? 2 : 1], xb[PRO == kProRmsNorm ? 2 : 1];
   uint4 gw[PRO == kProRmsNorm ? 2 : 1];
-  const bool norm_in_regs = cols <= TB * 16;
+  constexpr bool norm_in_regs = WALK != kWalkLoops;   // (the launcher: cols <= TB * 16)
   JoinRegs join[1];   // (kProJoin: the launcher keeps cols <= TB * 8)
   // (the same for every wave of the launch; a constant in the variant with exact start-up waits, which only
   // runs at 4096 columns, so its request counts stay countable)
@@ -519,11 +527,17 @@ __global__ __launch_bounds__(WG *kWave, XREG ? 4 : PRO == kProJoin && WG == 8 ? 
     }
   }
 
+  uint16_t act_raw[2] = {0, 0};
+  if constexpr (EPI == kEpiXielu) {
+    act_raw[0] = p.act[0];
+    act_raw[1] = p.act[1];
+  }
+
   // ---- 2. weight request state + the first two batches
-  uint32_t iu = EXACT ? min(wave_global, units - 1) : wave_global, ib = 0;  // next batch to request: unit, batch within the row
+  uint32_t iu = min(wave_global, units - 1), ib = 0;  // next batch to request: unit, batch within the row
   uint32_t ic = 0, cc = 0;            // ROT: column batch being requested / consumed (ic stays 0 otherwise)
   constexpr uint32_t kBatchElems = B * kWave * 8;
-  const uint16_t *wp[NR];
+  global_u16 wp[NR];
   uint4 buf0[NR][B], buf1[NR][B];
   float res0 = 0.0f, res1 = 0.0f;     // residual element (recurrent state) requested with a row's first batch
   uint16_t zb0 = 0, zb1 = 0, ub0 = 0, ub1 = 0;   // kEpiMinGru: the row's two biases, likewise (widened where they are used:
@@ -533,9 +547,9 @@ __global__ __launch_bounds__(WG *kWave, XREG ? 4 : PRO == kProJoin && WG == 8 ? 
     if (ib == 0) {                                                                                \
       if constexpr (ROT) ic = iu % bpr;                                                           \
       _Pragma("unroll") for (int k = 0; k < NR; ++k)                                              \
-        wp[k] = p.w + static_cast<uint64_t>(iu + k * p.rows) * cols + k * p.pair_gap + (RAGGED ? 0u : ic * kBatchElems + lane * 8); \
+        wp[k] = (global_u16)p.w + static_cast<uint64_t>(iu + k * p.rows) * cols + k * p.pair_gap + (RAGGED ? 0u : ic * kBatchElems + lane * 8); \
       if constexpr (EPI == kEpiResidual) {                                                        \
-        if (EXACT || lane == 0) RES = p.residual[iu];                                             \
+        RES = p.residual[iu];                                             \
       }                                                                                           \
       if constexpr (EPI == kEpiMinGru) {                                                          \
         RES = p.state[iu];                                                                        \
@@ -564,15 +578,15 @@ __global__ __launch_bounds__(WG *kWave, XREG ? 4 : PRO == kProJoin && WG == 8 ? 
     }                                                                                             \
     if (++ib == bpr) {                                                                            \
       ib = 0;                                                                                     \
-      iu += wave_stride;                                                                          \
+      if (iu + wave_stride < units) iu += wave_stride;   /* (else its last one again, not used) */ \
     }                                                                                             \
   } while (0)
-  if constexpr (EXACT) {  // the launcher guarantees two batches per row at least
-    NV_FAST_ISSUE(buf0, res0, zb0, ub0);
-    NV_FAST_ISSUE(buf1, res1, zb1, ub1);
-  } else {
+  if constexpr (kLoose) {
     if (total > 0) NV_FAST_ISSUE(buf0, res0, zb0, ub0);
     if (total > 1) NV_FAST_ISSUE(buf1, res1, zb1, ub1);
+  } else {
+    NV_FAST_ISSUE(buf0, res0, zb0, ub0);
+    if constexpr (WALK != kWalkOne) NV_FAST_ISSUE(buf1, res1, zb1, ub1);
   }
 
   // ---- 3. step guard (after the requests: they do not depend on it and are always in bounds)
@@ -656,7 +670,7 @@ __global__ __launch_bounds__(WG *kWave, XREG ? 4 : PRO == kProJoin && WG == 8 ? 
   float res_cur = 0.0f;
   uint16_t zb_cur = 0, ub_cur = 0;
   XieluParams act{};
-  if constexpr (EPI == kEpiXielu) act = xielu_params<DT>(p.act);
+  if constexpr (EPI == kEpiXielu) act = xielu_params<DT>(act_raw);
 #define NV_FAST_CONSUME(SRC, RES, ZB, UB)                                                               \
   do {                                                                                            \
     if (cb == 0) {                                                                                \
@@ -737,7 +751,9 @@ __global__ __launch_bounds__(WG *kWave, XREG ? 4 : PRO == kProJoin && WG == 8 ? 
         if (t + 5 < total) NV_FAST_ISSUE(buf1, res1, zb1, ub1);
       }
     }
-  } else {
+  } else if constexpr (WALK == kWalkOne) {
+    if (total != 0) NV_FAST_CONSUME(buf0, res0, zb0, ub0);
+  } else if constexpr (kLoose) {
     for (uint32_t t = 0; t < total; t += 2) {
       NV_FAST_CONSUME(buf0, res0, zb0, ub0);
       if (t + 2 < total) NV_FAST_ISSUE(buf0, res0, zb0, ub0);
@@ -745,6 +761,23 @@ __global__ __launch_bounds__(WG *kWave, XREG ? 4 : PRO == kProJoin && WG == 8 ? 
         NV_FAST_CONSUME(buf1, res1, zb1, ub1);
         if (t + 3 < total) NV_FAST_ISSUE(buf1, res1, zb1, ub1);
       }
+    }
+  } else {
+    uint32_t left = total;
+    for (; left >= 4; left -= 2) {
+      NV_FAST_CONSUME(buf0, res0, zb0, ub0);
+      NV_FAST_ISSUE(buf0, res0, zb0, ub0);
+      NV_FAST_CONSUME(buf1, res1, zb1, ub1);
+      NV_FAST_ISSUE(buf1, res1, zb1, ub1);
+    }
+    if (left == 3) {
+      NV_FAST_CONSUME(buf0, res0, zb0, ub0);
+      NV_FAST_ISSUE(buf0, res0, zb0, ub0);
+      NV_FAST_CONSUME(buf1, res1, zb1, ub1);
+      NV_FAST_CONSUME(buf0, res0, zb0, ub0);
+    } else if (left != 0) {
+      NV_FAST_CONSUME(buf0, res0, zb0, ub0);
+      if (left == 2) NV_FAST_CONSUME(buf1, res1, zb1, ub1);
     }
   }
 #undef NV_FAST_ISSUE

@@ -74,9 +74,25 @@ hipError_t launch_one(const GemvParams &p, const GemvPlan &plan, size_t lds, hip
     // 31.8 -> 33.5 us, LM head 187 -> 189 us (one wave per SIMD less) - so only the short launches with a
     // 16-bit input take it.
     const bool xreg = PRO == kProX16 && p.cols == 4096u && tuning(kTuneGemvXRegisters) != 2;
-#define NV_GEMV_LAUNCH(BB, EX, W, XR, RT)                                                                      \
-  hipLaunchKernelGGL((gemv_fast_kernel<DT, PRO, EPI, NR, BB, EX, W, XR, RT>), dim3((waves + W - 1) / W),        \
-                     dim3(W * kWave), lds, stream, p)
+#define NV_GEMV_WALK(BB, EX, W, XR, RT, RG, WALK) \
+  hipLaunchKernelGGL((gemv_fast_kernel<DT, PRO, EPI, NR, BB, EX, W, XR, RT, RG, WALK>), dim3((waves + W - 1) / W), dim3(W * kWave), lds, stream, p)
+#define NV_GEMV_LAUNCH_AS(BB, EX, W, XR, RT, RG)                                                             \
+  do {                                                                                                       \
+    if constexpr (PRO != kProJoin && EPI != kEpiArgmax && !EX && !XR) {                                       \
+      if (p.cols <= BB * kWave * 8u && p.rows <= (waves + W - 1) / W * W) {                                   \
+        NV_GEMV_WALK(BB, EX, W, XR, RT, RG, kWalkOne);                                                       \
+        break;                                                                                               \
+      }                                                                                                      \
+    }                                                                                                        \
+    if constexpr (PRO == kProRmsNorm && !EX && !XR) {                                                        \
+      if (p.cols > W * kWave * 16u) {                                                                        \
+        NV_GEMV_WALK(BB, EX, W, XR, RT, RG, kWalkLoops);                                                     \
+        break;                                                                                               \
+      }                                                                                                      \
+    }                                                                                                        \
+    NV_GEMV_WALK(BB, EX, W, XR, RT, RG, kWalkRegs);                                                          \
+  } while (0)
+#define NV_GEMV_LAUNCH(BB, EX, W, XR, RT) NV_GEMV_LAUNCH_AS(BB, EX, W, XR, RT, false)
     if constexpr (PRO == kProJoin) {   // one workgroup a CU (the plan)
       if ((wg != 16 && wg != 8) || p.cols > static_cast<uint32_t>(wg) * kWave * 8u) return hipErrorInvalidValue;
       if (wg == 8) {
@@ -99,8 +115,7 @@ hipError_t launch_one(const GemvParams &p, const GemvPlan &plan, size_t lds, hip
         else NV_GEMV_LAUNCH(2, false, 16, false, false);
       }
     } else if (plan.ragged) {
-#define NV_GEMV_RAGGED(BB, W) \
-  hipLaunchKernelGGL((gemv_fast_kernel<DT, PRO, EPI, NR, BB, false, W, false, true, true>), dim3((waves + W - 1) / W), dim3(W * kWave), lds, stream, p)
+#define NV_GEMV_RAGGED(BB, W) NV_GEMV_LAUNCH_AS(BB, false, W, false, true, true)
       if constexpr (EPI == kEpiArgmax) {
         if (wg == 16) NV_GEMV_RAGGED(2, 16);
         else NV_GEMV_RAGGED(2, 4);
@@ -140,6 +155,8 @@ hipError_t launch_one(const GemvParams &p, const GemvPlan &plan, size_t lds, hip
       else NV_GEMV_LAUNCH(4 / NR, false, 4, false, false);
     }
 #undef NV_GEMV_LAUNCH
+#undef NV_GEMV_LAUNCH_AS
+#undef NV_GEMV_WALK
   } else if constexpr (MODE == kVecFull) {
     hipLaunchKernelGGL((gemv_kernel<DT, PRO, EPI, NR, kDefaultU / NR, kVecFull, kDefaultDot2>),
                        dim3(plan.blocks), dim3(kBlock), lds, stream, p);

@@ -184,5 +184,12 @@ __device__ __forceinline__ uint4 load_stream(const void *p) {
   const u32x4_t v = __builtin_nontemporal_load(reinterpret_cast<const u32x4_t *>(p));
   return make_uint4(v.x, v.y, v.z, v.w);
 }
+// The same through a pointer that says it is one into global memory: where the compiler loses that - an array of pointers which a loop moves on -
+// it loads by flat instructions, which count as LDS accesses too and are waited for with them, all at once.
+typedef const __attribute__((address_space(1))) uint16_t *global_u16;
+__device__ __forceinline__ uint4 load_stream(global_u16 p) {
+  const u32x4_t v = __builtin_nontemporal_load(reinterpret_cast<const __attribute__((address_space(1))) u32x4_t *>(p));
+  return make_uint4(v.x, v.y, v.z, v.w);
+}
 
 }  // namespace nv
