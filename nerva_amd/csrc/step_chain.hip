@@ -5,9 +5,9 @@
 // whole step and hand vectors to each other as words of (value, tag), which a reader polls until the tag is its own, and the
 // weights of the next projection are requested before the wait for its input begins: 12 us a layer instead of 19. us a step, 12 / 100 / 260 / 1000
 // / 4000 keys, launches and chain, head and sampler (10 us) included:
-//   4 layers  512 x 1376,  8 heads of  64 on 4:   81 /  85 /  88 /  92 /  92     61 /  66 /  68 /  69 /  79
-//   8 layers  512 x 1792,  4 heads of 128 on 2:  158 / 163 / 178 / 173 / 176    116 / 125 / 130 / 132 / 156
-//   6 layers  640 x 1600,  5 heads of 128 on 5:  131 / 135 / 147 / 142 / 149    115 / 122 / 127 / 129 / 147
+//   4 layers  512 x 1376,  8 heads of  64 on 4:   81 /  84 /  88 /  91 /  92     59 /  64 /  64 /  67 /  76
+//   8 layers  512 x 1792,  4 heads of 128 on 2:  151 / 158 / 173 / 168 / 171    112 / 124 / 127 / 131 / 154
+//   6 layers  640 x 1600,  5 heads of 128 on 5:  125 / 130 / 142 / 137 / 143    107 / 116 / 118 / 121 / 140
 //   8 layers  768 x 2304, 12 heads of  64 on 4:  175 / 178 / 188 / 191 / -      188 / 197 / 207 / 208 / -      (not taken)
 // (in a stack of 13.8 MB a layer the requests, which a launch of 128 workgroups has too few of in flight, cost what the boundaries did).
 //
