@@ -158,7 +158,7 @@ __global__ void set_state_kernel(uint32_t *state, uint32_t cursor, uint32_t prom
   if (threadIdx.x == 0 && blockIdx.x == 0) {
     state[0] = cursor;
     state[1] = prompt_count;
-    if (clear_fault) state[3] = 0u;
+    if (clear_fault) state[3] = state[4] = state[5] = 0u;
   }
 }
 
@@ -244,6 +244,7 @@ SamplerParams session_sampler(Session *s, const float *logits) {
   sp.out.cursor_rw = s->state;
   sp.out.fault = s->state + 3;
   sp.out.step_rw = s->chain_context != 0 ? s->state + 2 : nullptr;
+  sp.out.host_given_up = s->given_up;
   sp.cursor = s->state;
   sp.max_steps = s->max_ctx;
   return sp;
@@ -446,7 +447,8 @@ hipError_t enqueue_chain_step(Session *s) {
   ChainLaunch c{};
   c.model = s->chain_model_dev;
   c.trace = s->trace_buf;
-  c.spin_limit = spins > 0 ? static_cast<uint32_t>(spins) : kAttnMergeSpinLimit;
+  c.spin_limit = spins > 0 ? static_cast<uint32_t>(spins) : kChainSpinLimit;
+  c.withhold = static_cast<uint32_t>(std::max(tuning(kTuneStepChainWithhold), 0));
   hipError_t err = launch_step_chain(s->dtype, s->head_dim, s->chain_model, c, s->stream);
   GemvParams p = head_launch(s, s->x);
   const auto slot = [](uint64_t bytes) { return (bytes + 255u) & ~uint64_t{255}; };
@@ -556,13 +558,35 @@ hipError_t ensure_graphs(Session *s, uint32_t position, uint32_t steps, NervaHip
   return err;
 }
 
+// Steps that have given up since the last look, of work that is done: the next step was the same one again, and as many are still to come. (One that
+// ends the sequence with a fault counts as done; the bit stays until another begins.)
+uint32_t take_given_up(Session *s) {
+  if (s->given_up == nullptr) return 0;
+  const uint32_t told = *static_cast<volatile uint32_t *>(s->given_up), count = told & ~kHostFault;
+  if (count != 0) *static_cast<volatile uint32_t *>(s->given_up) = told & kHostFault;
+  return count;
+}
+// `count` steps more, up to a position.
+hipError_t launch_steps_again(Session *s, uint32_t end, uint32_t count, NervaHipHfDecodeSequenceResult *out) {
+  hipError_t err = hipSuccess;
+  for (uint32_t i = 0; err == hipSuccess && i < count; ++i) err = launch_step(s, decode_graph(s, end - count + i), out);
+  return err;
+}
+
 hipError_t launch_step(Session *s, int which, NervaHipHfDecodeSequenceResult *out) {
   if (s->trace_buf != nullptr && which != 1) {
     // armed by nerva_hip_session_trace_next_step: this one step runs kernel by kernel with copies
     s->trace_used = 0;
     hipError_t err = enqueue_graph_step(s, which);
-    s->trace_buf = nullptr;
     if (err == hipSuccess) out->kernel_launches += step_launches(s, which);
+    // (one that gave up is traced once more, now: its replays would be the caller's steps without a trace)
+    while (err == hipSuccess && which >= 3) {
+      err = hipStreamSynchronize(s->stream);
+      if (err != hipSuccess || take_given_up(s) == 0) break;
+      err = enqueue_graph_step(s, which);
+      if (err == hipSuccess) out->kernel_launches += step_launches(s, which);
+    }
+    s->trace_buf = nullptr;
     return err;
   }
   if (eager_steps()) {
@@ -660,6 +684,7 @@ hipError_t reset_sequence(Session *s, const uint32_t *prompt_tokens, uint32_t pr
   // the words cleared here none of an earlier sequence's can ever match
   if (err == hipSuccess && s->attn_tagged != nullptr)
     err = hipMemsetAsync(s->attn_tagged, 0, attn_step_workspace_bytes(s->heads), s->stream);
+  if (s->given_up != nullptr) *s->given_up = 0;
   if (err == hipSuccess && s->chain_word_bytes != 0) err = hipMemsetAsync(s->chain_model.words, 0, s->chain_word_bytes, s->stream);
   if (err == hipSuccess && s->stack_state_bytes != 0)   // a new sequence's recurrent state
     err = hipMemsetAsync(s->stack_state, 0, s->stack_state_bytes, s->stream);
@@ -1064,7 +1089,7 @@ hipError_t upload_chain(Session *s) {
   m.prompt = s->prompt;
   m.slots = s->slots;
   m.state = s->state;
-  m.fault = s->state + 3;
+  m.gave_up = s->state + 4;
   m.k_cache = s->kc;
   m.v_cache = s->vc;
   m.table = s->table;
@@ -1120,7 +1145,9 @@ hipError_t setup_state(Session *s, int32_t *failure_stage, bool with_weights) {
   const uint64_t off_attn_plan = c.take(attn_plan_bytes(kAttnMaxSplits));
   const uint64_t off_attn_tagged = c.take(attn_step_workspace_bytes(s->heads));
   const uint64_t off_sample_ws = c.take(sample_workspace_bytes());
-  const bool chain = tuning(kTuneStepChain) != 2 && tuning(kTuneAttnSplits) == 0 && chain_takes(s->layers, s->hidden, s->heads, s->kv_heads, s->head_dim, s->intermediate);
+  const bool chain = tuning(kTuneStepChain) != 2 && tuning(kTuneAttnSplits) == 0 &&
+                     chain_takes(s->layers, s->hidden, s->heads, s->kv_heads, s->head_dim, s->intermediate) &&
+                     chain_resident(s->dtype, s->hidden, s->heads, s->kv_heads, s->head_dim, s->intermediate);
   if (chain) {
     ChainModel &m = s->chain_model;
     m.layers = s->layers;
@@ -1234,6 +1261,8 @@ hipError_t setup_state(Session *s, int32_t *failure_stage, bool with_weights) {
   s->sample_ws = s->arena + off_sample_ws;
   if (chain) {
     s->chain_context = kChainContext;
+    s->given_up = s->host_state;
+    *s->given_up = 0;
     s->chain_model.words = reinterpret_cast<uint64_t *>(s->arena + off_chain_words);
     s->chain_model.layer = reinterpret_cast<LayerDev *>(s->arena + off_chain_layers);
     s->chain_model.stage = reinterpret_cast<ChainStage *>(s->arena + off_chain_stages);
@@ -2051,8 +2080,17 @@ int nerva_hip_hf_decode_sequence_batch_advance_one(const NervaHipHfDecodeSequenc
       out->sampling_kernel_launches += q->sampler.mode == kSamplerGreedy ? 1 : 2;
     }
     for (uint32_t t = 0; err == hipSuccess && t < T; ++t) {
-      err = hipStreamSynchronize(seqs[t]->stream);
+      Session *q = seqs[t];
+      err = hipStreamSynchronize(q->stream);
       out->sync_calls += 1;
+      while (err == hipSuccess && take_given_up(q) != 0) {
+        err = launch_step(q, decode_graph(q, q->cursor), &scratch);
+        if (err == hipSuccess)
+          err = hipMemcpyAsync(&q->host_slots[q->cursor], &q->slots[q->cursor], sizeof(Slot), hipMemcpyDeviceToHost, q->stream);
+        if (err == hipSuccess) err = hipStreamSynchronize(q->stream);
+        out->d2h_bytes += sizeof(Slot);
+        out->sync_calls += 1;
+      }
     }
   }
   out->hot_path_allocations = allocation_count() - allocs_before;
@@ -2201,14 +2239,20 @@ int nerva_hip_session_extend(const NervaHipSessionExtendRequest *request, NervaH
     if (err == hipSuccess) err = set_device_position(s, begin, end, 0);
     out->h2d_bytes = static_cast<uint64_t>(n) * sizeof(uint32_t);
   }
+  bool idle = false;
   const auto logits_out = [&](uint32_t i) {   // the last step's logits are wanted row i
     err = copy_out(s, request->logits + static_cast<uint64_t>(i) * s->vocab, s->logits, s->vocab * sizeof(float), &out->sync_calls, false);
     out->d2h_bytes += s->vocab * sizeof(float);
   };
   if (n == 1 && request->residuals == nullptr) {
     if (err == hipSuccess) err = ensure_graph(s, decode_graph(s, begin), out);
-    if (err == hipSuccess) err = launch_step(s, decode_graph(s, begin), out);
-    if (err == hipSuccess && request->wanted_count != 0) logits_out(0);
+    for (uint32_t again = 1; err == hipSuccess && again != 0;) {
+      err = launch_step(s, decode_graph(s, begin), out);
+      if (err == hipSuccess && request->wanted_count != 0) logits_out(0);
+      if (err == hipSuccess) err = hipStreamSynchronize(s->stream);
+      idle = true;
+      again = take_given_up(s);
+    }
   } else if (s->stack != nullptr) {
     if (err == hipSuccess)
       err = stack_prompt(s, begin, end, request->wanted, request->wanted_count, request->logits, request->residuals, out);
@@ -2226,10 +2270,11 @@ int nerva_hip_session_extend(const NervaHipSessionExtendRequest *request, NervaH
       at = stop;
     }
   }
-  if (err == hipSuccess) err = hipStreamSynchronize(s->stream);
+  if (err == hipSuccess && !idle) err = hipStreamSynchronize(s->stream);
   out->sync_calls += 1;
-  if (err != hipSuccess) {
-    out->hip_error = static_cast<int32_t>(err);
+  const bool fault = s->given_up != nullptr && (*s->given_up & kHostFault) != 0;
+  if (err != hipSuccess || fault) {
+    out->hip_error = err != hipSuccess ? static_cast<int32_t>(err) : NERVA_HIP_ERROR_STEP_FAULT;
     s->finished = true;
     return -1;
   }
@@ -2286,21 +2331,30 @@ int nerva_hip_hf_decode_sequence_session_advance(const NervaHipHfDecodeSequenceS
       if (err == hipSuccess) err = hipStreamSynchronize(s->stream);
       out->sync_calls += 1;
       out->d2h_bytes += sizeof(Slot);
+      if (err == hipSuccess && take_given_up(s) != 0) {
+        step -= 1;
+        continue;
+      }
       if (err == hipSuccess && s->host_slots[pos].completion == NERVA_HIP_SLOT_DEVICE_COMPLETE &&
           s->host_slots[pos].token == s->eos)
         break;
     }
   }
-  if (err == hipSuccess && run_count != 0) err = hipEventRecord(s->ev1, s->stream);
   const uint64_t slots_bytes = static_cast<uint64_t>(request->steps) * sizeof(Slot);
-  if (err == hipSuccess) {
-    err = hipMemcpyAsync(s->host_slots + slot_start, s->slots + slot_start, slots_bytes,
-                         hipMemcpyDeviceToHost, s->stream);
-    out->d2h_bytes += slots_bytes;
-  }
-  if (err == hipSuccess) {
-    err = hipStreamSynchronize(s->stream);
-    out->sync_calls += 1;
+  for (uint32_t again = 0; err == hipSuccess;) {
+    err = launch_steps_again(s, target, again, out);
+    if (err == hipSuccess && run_count != 0) err = hipEventRecord(s->ev1, s->stream);
+    if (err == hipSuccess) {
+      err = hipMemcpyAsync(s->host_slots + slot_start, s->slots + slot_start, slots_bytes,
+                           hipMemcpyDeviceToHost, s->stream);
+      out->d2h_bytes += slots_bytes;
+    }
+    if (err == hipSuccess) {
+      err = hipStreamSynchronize(s->stream);
+      out->sync_calls += 1;
+    }
+    again = take_given_up(s);
+    if (again == 0) break;
   }
   out->hot_path_allocations = allocation_count() - allocs_before;
   if (err == hipSuccess && run_count != 0) {
@@ -2367,15 +2421,20 @@ int nerva_hip_hf_decode_sequence_session_run(const NervaHipHfDecodeSequenceSessi
   for (uint32_t step = 0; err == hipSuccess && step < context_steps; ++step) {
     err = launch_step(s, decode_graph(s, step), out);
   }
-  if (err == hipSuccess) err = hipEventRecord(s->ev1, s->stream);
   const uint64_t slots_bytes = static_cast<uint64_t>(context_steps) * sizeof(Slot);
-  if (err == hipSuccess) {
-    err = hipMemcpyAsync(s->host_slots, s->slots, slots_bytes, hipMemcpyDeviceToHost, s->stream);
-    out->d2h_bytes = slots_bytes;
-  }
-  if (err == hipSuccess) {
-    err = hipStreamSynchronize(s->stream);
-    out->sync_calls += 1;
+  for (uint32_t again = 0; err == hipSuccess;) {
+    err = launch_steps_again(s, context_steps, again, out);
+    if (err == hipSuccess) err = hipEventRecord(s->ev1, s->stream);
+    if (err == hipSuccess) {
+      err = hipMemcpyAsync(s->host_slots, s->slots, slots_bytes, hipMemcpyDeviceToHost, s->stream);
+      out->d2h_bytes += slots_bytes;
+    }
+    if (err == hipSuccess) {
+      err = hipStreamSynchronize(s->stream);
+      out->sync_calls += 1;
+    }
+    again = take_given_up(s);
+    if (again == 0) break;
   }
   out->hot_path_allocations = allocation_count() - allocs_before;
   if (err == hipSuccess) {

@@ -51,12 +51,36 @@ struct SampleParams {
   uint32_t *cursor_rw;
   uint32_t *token_out;     // optional: plain token output (operator entry point)
   const uint32_t *fault;   // optional: a word that a kernel of this step sets when a bounded wait of its gave up
-  uint32_t *step_rw;       // optional: the step number, which the next step's launches derive their tags from
+  // optional (narrow models): the step's words - its number, which the next step's launches derive their tags from, the fault word, whether its
+  // layers' launch gave up (step_chain.cuh), and how often in a row they have - and a word of the host's
+  uint32_t *step_rw;
+  uint32_t *host_given_up;
 };
+
+// Steps that give up one after the other at the same position (0.8 s of them) until the sequence ends with a fault, and the bit that says so to the host
+constexpr uint32_t kMostGivenUp = 256, kHostFault = 1u << 31;
+
+// One lane: whether the step that ends here gave up. Its token is not handed out and the cursor stays, so that the next step is the same one again.
+__device__ __forceinline__ bool step_given_up(const SampleParams &s) {
+  const uint32_t gave_up = s.step_rw[2], in_a_row = s.step_rw[3];
+  *s.step_rw += 1u;
+  s.step_rw[2] = s.step_rw[3] = 0u;
+  if (gave_up == 0 || s.step_rw[1] != 0u) return false;
+  const uint32_t told = __hip_atomic_load(s.host_given_up, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+  if (in_a_row + 1u < kMostGivenUp) {
+    s.step_rw[3] = in_a_row + 1u;
+    __hip_atomic_store(s.host_given_up, told + 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+    return true;
+  }
+  s.step_rw[1] = 1u;
+  __hip_atomic_store(s.host_given_up, told | kHostFault, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+  return false;
+}
 
 // One lane: hands the step's token out - plain output word and/or slot[pos] in the reference's
 // slot format (nerva_cuda_api.h:29-37, sampler.cu:394-407) plus the cursor bump.
 __device__ __forceinline__ void publish_token(const SampleParams &s, uint32_t token) {
+  if (s.step_rw != nullptr && step_given_up(s)) return;
   if (s.token_out != nullptr) *s.token_out = token;
   if (s.slots != nullptr) {
     const uint32_t pos = *s.cursor_rw;
@@ -71,7 +95,6 @@ __device__ __forceinline__ void publish_token(const SampleParams &s, uint32_t to
     slot.host_copied = 0;
     s.slots[pos] = slot;
     *s.cursor_rw = pos + 1u;
-    if (s.step_rw != nullptr) *s.step_rw += 1u;
   }
 }
 

@@ -174,6 +174,7 @@ enum TuningKnob : int {
   kTuneMixedAttentionWide,   // mixed stacks: 2 = every attention layer through the general kernel
   kTuneLatentAttentionWide,  // mixed stacks: 2 = every layer of attention over latents through the general kernel
   kTuneStepChain,            // narrow models: 2 = a step's layers never in one launch (read at session create)
+  kTuneStepChainWithhold,    // test hook: a workgroup of a step's chain stays away so often in a row
   kTuneKnobs
 };
 int tuning(TuningKnob knob);

@@ -85,7 +85,8 @@ struct NervaHipHfDecodeSequenceSession : nv::RowScratch {
   uint32_t block_count = 0;
   uint32_t *table = nullptr, *prompt = nullptr;
   uint32_t *state = nullptr;  // state[0] cursor, state[1] prompt count, state[2] steps executed so far,
-                              // state[3] fault word (set by a kernel whose bounded wait gave up; cleared by start)
+                              // state[3] fault word (set by a kernel whose bounded wait gave up; cleared by start),
+                              // state[4] the step's chain gave up, state[5] how many in a row have (step_given_up)
   nv::Slot *slots = nullptr;
   float *x = nullptr, *r = nullptr, *qkv = nullptr, *logits = nullptr, *rope_freq = nullptr, *rope_cs = nullptr;
   uint16_t *attn16 = nullptr, *ff16 = nullptr;
@@ -109,6 +110,7 @@ struct NervaHipHfDecodeSequenceSession : nv::RowScratch {
   nv::ChainModel chain_model{};      // ... what that launch works on, and its copy on the device
   nv::ChainModel *chain_model_dev = nullptr;
   uint64_t chain_word_bytes = 0;
+  uint32_t *given_up = nullptr;      // host_state[0]: steps that gave up since the host looked (step_given_up writes it)
   // prompt blocks: up to prefill_pass_tokens prompt tokens per pass through the layers (weights streamed
   // once per pass on the matrix cores), in a long prompt prefill_long_tokens; false = one prompt step per token
   bool block_prefill = false;

@@ -28,8 +28,8 @@ struct ChainModel {
   const uint16_t *emb;
   const uint32_t *prompt;
   const NervaHipSyntheticTokenSlot *slots;
-  const uint32_t *state;       // position, prompt tokens, step number (the words' tags derive from it)
-  uint32_t *fault;
+  const uint32_t *state;       // position, prompt tokens, step number (the words' tags derive from it), -, -, steps that gave up in a row
+  uint32_t *gave_up;           // set by a launch whose waits ran out
   uint16_t *k_cache, *v_cache;
   const uint32_t *table;
   const float *rope_freq;      // null: no rotation
@@ -46,9 +46,13 @@ constexpr uint32_t kChainSingleBlocks = 8;
 constexpr uint32_t kChainMaxHidden = 1024, kChainMaxIn = 4096, kChainMaxSplits = 16;
 // Tokens of context up to which steps run as a chain: with 4000 keys, sixteen splits of sixteen blocks, it is 0.87 to 0.99 of the launches' time.
 constexpr uint32_t kChainContext = 4096;
+// Polls after which a wait gives up: 3.1 ms (a step whose workgroup 0 stays away), where the longest wait of a healthy launch is some 20 us.
+constexpr uint32_t kChainSpinLimit = 1u << 14;
 // Whether a model's steps can run as a chain.
 bool chain_takes(uint32_t layers, uint32_t hidden, uint32_t heads, uint32_t kv_heads, uint32_t head_dim, uint32_t ff);
 uint32_t chain_workgroups(uint32_t hidden, uint32_t heads, uint32_t kv_heads, uint32_t head_dim, uint32_t ff);
+// ... and whether the device holds all of them at once.
+bool chain_resident(uint32_t dtype, uint32_t hidden, uint32_t heads, uint32_t kv_heads, uint32_t head_dim, uint32_t ff);
 // 8-byte words of ChainModel::words, whose places it fills in.
 uint64_t chain_place(ChainModel &model, uint32_t head_dim);
 // The walks of a layer's four projections.
@@ -57,6 +61,7 @@ struct ChainLaunch {
   const ChainModel *model;     // device memory
   char *trace;                 // test hook: every link's vector, 256 bytes apart (step_trace_bytes), or null
   uint32_t spin_limit;         // polls after which a wait gives up
+  uint32_t withhold;           // test hook: so often in a row a workgroup is missing
 };
 // `model`: the same on the host.
 hipError_t launch_step_chain(uint32_t dtype, uint32_t head_dim, const ChainModel &model, const ChainLaunch &p, hipStream_t stream);

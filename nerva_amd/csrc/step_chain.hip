@@ -18,9 +18,12 @@
 // projection, its products 0.6 to 1.0, a norm 0.4, the attention 2.8 -, so everything about a projection that can be known before is in
 // one table entry (ChainStage).
 //
-// The workgroups wait for each other, so all of a launch have to be resident: 128 of four waves at most, with registers and
-// LDS for two a CU, of which four launches at once - one a hardware queue - fit the chip together. A wait that runs out is
-// an error as in the decode attention: the fault word is set and the rest of the launch waits for nothing.
+// The workgroups wait for each other, so all of a launch have to be resident: 128 of four waves at most, with registers and LDS for two or three
+// a CU. A device that does not hold them never runs a chain (chain_resident). One that does may still be shared, with other sessions' chains on more
+// hardware queues than there is room for, with an attention launch that wants every CU for itself and waits too, with another process: launches that
+// are each partly resident would then hold each other's places. So a chain's waits are short (kChainSpinLimit): when one runs out the launch says so, waits for
+// nothing any more and leaves the chip, and the step is void - its token is not handed out, the cursor stays (step_given_up), whatever it wrote is written
+// again - and taken once more. Only kMostGivenUp of them in a row are the step fault that a wait of the decode attention's is.
 //
 // No word is written before all its readers have read what it held. Every workgroup has rows of o, of gate and up and of down, and writes
 // them behind its own reads of what came before; so when x is whole, everyone has read the activation and the r of that layer, and the
@@ -74,12 +77,12 @@ __device__ __forceinline__ void store_word(uint64_t *at, uint32_t payload, uint3
 // The wave's share of n words that lie together, i * 256 + thread, until every tag is this launch's.
 struct Waiter {
   uint32_t limit;     // 0: a wait has run out, nothing is waited for any more
-  uint32_t *fault;
-  __device__ __forceinline__ bool again(bool ok, uint32_t &spins, uint32_t tag) {
+  uint32_t *gave_up;
+  __device__ __forceinline__ bool again(bool ok, uint32_t &spins) {
     if (__all(ok) || limit == 0) return false;
     if (++spins <= limit) return true;
     limit = 0;
-    if ((threadIdx.x & (kWave - 1)) == 0) __hip_atomic_store(fault, tag, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    if ((threadIdx.x & (kWave - 1)) == 0) __hip_atomic_store(gave_up, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     return false;
   }
 };
@@ -94,7 +97,7 @@ __device__ __forceinline__ void poll_words(const uint64_t *src, uint32_t n, uint
     ok = true;
 #pragma unroll
     for (int i = 0; i < N; ++i) ok = ok && tag_is(v[i], tag);
-  } while (wait.again(ok, spins, tag));
+  } while (wait.again(ok, spins));
 }
 // Packed 16-bit pairs into LDS.
 template <int N>
@@ -332,7 +335,7 @@ __device__ __forceinline__ void chain_attention(Model m_, uint32_t layer, uint32
       ok = true;
 #pragma unroll
       for (int i = 0; i < kMine; ++i) ok = ok && tag_is(v0[i], tag) && tag_is(v1[i], tag);
-    } while (wait.again(ok, spins, tag));
+    } while (wait.again(ok, spins));
   }
 #pragma unroll
   for (int i = 0; i < kMine; ++i) {
@@ -485,7 +488,7 @@ __device__ __forceinline__ void chain_merge(Model m_, uint32_t h, uint32_t activ
 #pragma unroll
     for (uint32_t i = 0; i < kPer; ++i)
       if (q + i * kSets < active) ok = ok && tag_is(av[i], tag) && tag_is(mv[i], tag) && tag_is(lv[i], tag);
-  } while (wait.again(ok, spins, tag));
+  } while (wait.again(ok, spins));
   float M = -INFINITY, L = 0.0f, o = 0.0f;
 #pragma unroll
   for (uint32_t i = 0; i < kPer; ++i)
@@ -531,6 +534,7 @@ __global__ __launch_bounds__(kThreads, 2) void step_chain_kernel(ChainLaunch p) 
   Model m = (Model)(reinterpret_cast<uint64_t>(p.model));
   const uint32_t pos = scalar_load(m->state), step = scalar_load(m->state + 2);
   if (pos >= m->max_steps) return;
+  if (p.withhold != 0 && blockIdx.x == 0 && scalar_load(m->state + 5) < p.withhold) return;
   constexpr int kX = kChainMaxHidden / kThreads;
   uint4 ring[kRing][kGroup];
   Walk k;
@@ -550,7 +554,7 @@ __global__ __launch_bounds__(kThreads, 2) void step_chain_kernel(ChainLaunch p) 
       sh.cs[HD / 2 + i] = sn;
     }
   }
-  Waiter wait{p.spin_limit, m->fault};
+  Waiter wait{p.spin_limit, m->gave_up};
   // test hook: where a layer's vectors go. Workgroup 0 reads all of them but the raw heads, which their producers write
   const auto slot = [](uint32_t bytes) { return (bytes + 255u) & ~255u; };
   const bool traces = p.trace != nullptr;
@@ -747,35 +751,45 @@ void chain_stages(const ChainModel &m, uint32_t head_dim, const LayerDev &w, Cha
 }
 
 namespace {
-template <uint32_t DT, int HD, int G, bool PARTS>
-hipError_t launch_one(const ChainModel &m, const ChainLaunch &p, hipStream_t stream) {
-  hipLaunchKernelGGL((step_chain_kernel<DT, HD, G, PARTS>), dim3(chain_workgroups(m.hidden, m.heads, m.kv_heads, HD, m.ff)), dim3(kThreads), 0, stream, p);
-  return hipGetLastError();
-}
+using Kernel = void (*)(ChainLaunch);
 template <uint32_t DT>
-hipError_t launch_shape(uint32_t head_dim, const ChainModel &m, const ChainLaunch &p, hipStream_t stream) {
-  const uint32_t group = m.heads / m.kv_heads;
+Kernel kernel_of(uint32_t head_dim, uint32_t group) {
   if (head_dim == 64) {
-    if (group == 1) return launch_one<DT, 64, 1, true>(m, p, stream);
-    if (group == 2) return launch_one<DT, 64, 2, true>(m, p, stream);
-    if (group <= 4) return launch_one<DT, 64, 4, true>(m, p, stream);
-    return launch_one<DT, 64, 8, true>(m, p, stream);
+    if (group == 1) return step_chain_kernel<DT, 64, 1, true>;
+    if (group == 2) return step_chain_kernel<DT, 64, 2, true>;
+    if (group <= 4) return step_chain_kernel<DT, 64, 4, true>;
+    return step_chain_kernel<DT, 64, 8, true>;
   }
-  if (group == 1) return launch_one<DT, 128, 1, false>(m, p, stream);
-  if (group == 2) return launch_one<DT, 128, 2, false>(m, p, stream);
-  if (group == 3) return launch_one<DT, 128, 4, true>(m, p, stream);
-  if (group == 4) return launch_one<DT, 128, 4, false>(m, p, stream);
-  if (group < 8) return launch_one<DT, 128, 8, true>(m, p, stream);
-  return launch_one<DT, 128, 8, false>(m, p, stream);
+  if (group == 1) return step_chain_kernel<DT, 128, 1, false>;
+  if (group == 2) return step_chain_kernel<DT, 128, 2, false>;
+  if (group == 3) return step_chain_kernel<DT, 128, 4, true>;
+  if (group == 4) return step_chain_kernel<DT, 128, 4, false>;
+  if (group < 8) return step_chain_kernel<DT, 128, 8, true>;
+  return step_chain_kernel<DT, 128, 8, false>;
+}
+Kernel kernel_of(uint32_t dtype, uint32_t head_dim, uint32_t group) {
+  return dtype == kBF16 ? kernel_of<kBF16>(head_dim, group) : dtype == kF16 ? kernel_of<kF16>(head_dim, group) : nullptr;
 }
 }  // namespace
+
+bool chain_resident(uint32_t dtype, uint32_t hidden, uint32_t heads, uint32_t kv_heads, uint32_t head_dim, uint32_t ff) {
+  const Kernel kernel = kernel_of(dtype, head_dim, heads / kv_heads);
+  int device = 0, cus = 0, each = 0;
+  if (kernel == nullptr || hipGetDevice(&device) != hipSuccess || hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, device) != hipSuccess ||
+      hipOccupancyMaxActiveBlocksPerMultiprocessor(&each, reinterpret_cast<const void *>(kernel), kThreads, 0) != hipSuccess) {
+    (void)hipGetLastError();
+    return false;
+  }
+  return static_cast<uint64_t>(cus) * static_cast<uint64_t>(each) >= chain_workgroups(hidden, heads, kv_heads, head_dim, ff);
+}
 
 hipError_t launch_step_chain(uint32_t dtype, uint32_t head_dim, const ChainModel &m, const ChainLaunch &p, hipStream_t stream) {
   if (!chain_takes(m.layers, m.hidden, m.heads, m.kv_heads, head_dim, m.ff) || p.model == nullptr || m.words == nullptr || p.spin_limit == 0)
     return hipErrorInvalidValue;
-  if (dtype == kBF16) return launch_shape<kBF16>(head_dim, m, p, stream);
-  if (dtype == kF16) return launch_shape<kF16>(head_dim, m, p, stream);
-  return hipErrorInvalidValue;
+  const Kernel kernel = kernel_of(dtype, head_dim, m.heads / m.kv_heads);
+  if (kernel == nullptr) return hipErrorInvalidValue;
+  hipLaunchKernelGGL(kernel, dim3(chain_workgroups(m.hidden, m.heads, m.kv_heads, head_dim, m.ff)), dim3(kThreads), 0, stream, p);
+  return hipGetLastError();
 }
 
 }  // namespace nv

@@ -1,4 +1,6 @@
 """Decode steps of narrow models whose layers run in one launch, against the oracle and against the launches they stand in for."""
+import threading
+
 import numpy as np
 import pytest
 
@@ -118,3 +120,130 @@ def test_a_wait_that_runs_out_ends_the_sequence():
     assert s.start(prompt)[0] == 0
     assert s.advance(12)[2].tolist() == want
     s.destroy()
+
+
+# Polls that a wait is given where a test has many run out: an eighth of what it has, and far more than a healthy one takes
+SHORT_WAIT = 2000
+
+
+def test_steps_that_give_up_are_taken_again():
+    """A workgroup that stays away twice at every position, as one that finds no place on a shared chip: the other waits end, the step is void and
+    taken again, and every call gives what it gives without - advance, with a stop token too, run, extend with its logits, a traced step, a batch of
+    sequences that step one by one, and the sampler."""
+    dtype, hidden, heads, kv, hd, inter, vocab, layers, theta, qk_norm, bias = SHAPES[1]
+    cfg = dict(dtype=dtype, hidden=hidden, heads=heads, kv_heads=kv, head_dim=hd, intermediate=inter, vocab=vocab, layers=layers, rms_eps=1e-6, rope_theta=theta)
+    prompt = np.random.default_rng(2).integers(0, vocab, 9).astype(np.uint32)
+    sampler = abi.NervaHipHfDecodeSamplerConfig()
+    sampler.temperature, sampler.top_p, sampler.top_k, sampler.seed = 0.9, 0.95, 0, 11
+    s = N.DecodeSession.create_synthetic(cfg, 64, weight_hash=7, weight_std=0.05)
+
+    def calls(s):
+        out = []
+        assert s.start(prompt)[0] == 0
+        rc, res, tokens = s.advance(6)
+        assert rc == 0
+        out += [tokens, s.logits()]
+        replays = res.graph_replays
+        assert s.start(prompt, eos=int(tokens[3]))[0] == 0
+        rc, res, stopped = s.advance(12)
+        assert rc == 0 and len(stopped) <= 4
+        out.append(stopped)
+        rc, res, walked = s.run(prompt, 5)
+        assert rc == 0
+        out.append(walked)
+        s.release_sequence()
+        assert s.extend(prompt)[0] == 0
+        for t in prompt[:3]:
+            rc, res, rows, _ = s.extend([t], [0])
+            assert rc == 0
+            out.append(rows)
+        assert s.start(prompt)[0] == 0
+        assert s.advance(2)[0] == 0
+        rc, res, token, trace = s.traced_advance()
+        assert rc == 0
+        out += [token, trace["x0"], trace["logits"]] + [layer[k] for layer in trace["layers"] for k in sorted(layer)]
+        assert s.start(prompt, sampler=sampler)[0] == 0
+        rc, res, drawn = s.advance(8)
+        assert rc == 0
+        out.append(drawn)
+        others = [s.fork_shared_weights() for _ in range(2)]
+        for i, q in enumerate([s] + others):
+            assert q.start(prompt[:5 + i])[0] == 0 and q.advance(1)[0] == 0
+        for _ in range(3):
+            rc, res, tokens = N.DecodeSession.batch_advance_one([s] + others, 3, 3)
+            assert rc == 0
+            out.append(tokens)
+        for q in others:
+            q.destroy()
+        return out, replays
+
+    want, replays = calls(s)
+    assert replays == 5 and not s.shares_weight_stream()
+    fork = s.fork_shared_weights()
+    N.Device.set_tuning("attn_merge_spin_limit", SHORT_WAIT)
+    N.Device.set_tuning("step_chain_withhold", 2)
+    try:
+        got, replays = calls(fork)
+    finally:
+        N.Device.reset_tuning()
+    assert replays == 3 * 5
+    for i, (a, b) in enumerate(zip(want, got)):
+        assert np.array_equal(a, b), i
+    fork.destroy()
+    s.destroy()
+
+
+def test_a_chain_that_never_runs_is_a_step_fault():
+    """Steps that give up again and again end the sequence: advance says so in the slot, a one-token extend in its result."""
+    dtype, hidden, heads, kv, hd, inter, vocab, layers, theta, qk_norm, bias = SHAPES[1]
+    weights, _ = random_model(dtype, hidden, heads, kv, hd, inter, vocab, layers, 5, theta, qk_norm, bias)
+    prompt = np.arange(9, dtype=np.uint32)
+    N.Device.set_tuning("attn_merge_spin_limit", 50)
+    N.Device.set_tuning("step_chain_withhold", 100000)
+    try:
+        s = N.DecodeSession.create(weights, 64)
+        assert s.start(prompt)[0] == 0
+        rc, res, tokens = s.advance(3)
+        assert rc == -1 and res.hip_error == abi.NERVA_HIP_ERROR_STEP_FAULT
+        s.release_sequence()
+        assert s.extend(prompt)[0] == 0
+        rc, res = s.extend([3], [0])[:2]
+        assert rc == -1 and res.hip_error == abi.NERVA_HIP_ERROR_STEP_FAULT
+        s.destroy()
+    finally:
+        N.Device.reset_tuning()
+
+
+def test_many_chains_and_a_wide_attention_at_once():
+    """Six sessions of the largest chains, and one whose attention wants every CU, from threads of their own: whatever of it is resident at a
+    time, each gives what it gives alone."""
+    narrow = (BF16, 1024, 8, 4, 128, 1024, 301, 6, 1e6, True, False)
+    wide = (BF16, 2048, 16, 8, 128, 2048, 301, 2, 1e6, True, False)
+    rng = np.random.default_rng(8)
+    prompts = [rng.integers(0, 301, n).astype(np.uint32) for n in (1800, 20, 150, 300, 40, 700, 9)]
+    weights = [random_model(*g[:8], 3, *g[8:])[0] for g in (narrow, wide)]
+    first, broad = N.DecodeSession.create(weights[0], 1024), N.DecodeSession.create(weights[1], 2048)
+    sessions = [broad, first] + [first.fork_shared_weights() for _ in range(5)]
+
+    def all_steps(i, out):
+        s = sessions[i]
+        rc = s.start(prompts[i])[0]
+        for _ in range(20):
+            if rc == 0:
+                rc, res, tokens = s.advance(10)
+                out.append((rc, tokens.tolist()))
+        out.append(rc)
+
+    alone = [[] for _ in sessions]
+    for i in range(len(sessions)):
+        all_steps(i, alone[i])
+    together = [[] for _ in sessions]
+    threads = [threading.Thread(target=all_steps, args=(i, together[i])) for i in range(len(sessions))]
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join()
+    assert all(out[-1] == 0 for out in alone + together)
+    assert together == alone
+    for s in sessions[::-1]:
+        s.destroy()

@@ -1,0 +1,56 @@
+"""Host code of the decode session without a device: libnerva_hip.so on a stand-in for the HIP runtime (tests/host/hip_double.cpp), in a process of
+its own."""
+import os
+import shutil
+import subprocess
+import sys
+
+import pytest
+
+ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
+SOURCE = os.path.join(ROOT, "tests", "host", "hip_double.cpp")
+
+PRELUDE = """
+import ctypes, sys
+double = ctypes.CDLL(sys.argv[1], mode=ctypes.RTLD_GLOBAL)
+double.double_launches.restype = double.double_copies.restype = ctypes.c_long
+double.double_fail_copy.argtypes = [ctypes.c_long]
+sys.path[:0] = [%r, %r]
+import numpy as np
+import nerva_amd as N
+from test_gpu_session import BF16, F16, random_model
+NARROW = (BF16, 256, 4, 2, 64, 512, 64, 4, 5)   # (dtype, hidden, heads, kv, hd, inter, vocab, layers, seed)
+
+def model(shape=NARROW):
+    return random_model(*shape)[0]
+
+def step(session):
+    assert session.start(np.arange(5, dtype=np.uint32))[0] == 0
+    return session.advance(2)[1]
+""" % (ROOT, os.path.join(ROOT, "tests"))
+
+
+@pytest.fixture(scope="module")
+def double(tmp_path_factory):
+    if shutil.which("g++") is None:
+        pytest.skip("no g++")
+    out = str(tmp_path_factory.mktemp("double") / "libhip_double.so")
+    res = subprocess.run(["g++", "-std=c++17", "-O1", "-Wall", "-shared", "-fPIC", "-I/opt/rocm/include", SOURCE, "-o", out], capture_output=True, text=True)
+    assert res.returncode == 0, res.stderr
+    return out
+
+
+def run(double, body):
+    res = subprocess.run([sys.executable, "-c", PRELUDE + body, double], capture_output=True, text=True, timeout=300)
+    assert res.returncode == 0, res.stdout + res.stderr
+
+
+def test_chains_only_where_the_device_holds_all_their_workgroups(double):
+    """A chain's workgroups wait for each other: a device (or a partition of one) with places for fewer of them takes the step's launches."""
+    run(double, """
+for cus, each, chained in ((256, 2, True), (16, 2, True), (16, 1, False), (8, 3, False), (32, 0, False)):   # 32 workgroups at this width
+    double.double_device(cus, each)
+    s = N.DecodeSession.create(model(), 64)
+    assert step(s).graph_nodes == (3 if chained else 3 + 5 * 4), (cus, each)
+    s.destroy()
+""")
