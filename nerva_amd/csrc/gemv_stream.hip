@@ -66,7 +66,8 @@ hipError_t launch_one(const GemvParams &p, const GemvPlan &plan, size_t lds, hip
     constexpr uint32_t kBatchCols = kWave * 8u * (4 / NR);
     const uint32_t units_per_wave = (p.rows + blocks * kWavesPerBlock - 1) / (blocks * kWavesPerBlock);
     const int forced = tuning(kTuneGemvExactStart);
-    const bool can = kShortShapes && p.cols >= 2u * kBatchCols;
+    // (behind the norm only where its row fits the registers: the exact variant has no loops there)
+    const bool can = kShortShapes && p.cols >= 2u * kBatchCols && (PRO != kProRmsNorm || p.cols <= static_cast<uint32_t>(wg) * kWave * 16u);
     const bool want = forced == 1 || (forced == 0 && units_per_wave <= 2 && p.cols == 2u * kBatchCols);
     // Waves per workgroup: the same waves in fewer workgroups (see the kernel).
     const uint32_t waves = blocks * kWavesPerBlock;

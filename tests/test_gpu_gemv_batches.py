@@ -39,3 +39,27 @@ def test_gemv_of_every_number_of_batches(rows, cols):
     N.gemv(dtype, dw, rows, cols, input_f32=dxf, gamma=dg, eps=1e-6, out16=y16, epilogue=2)
     # one 16-bit rounding of the result, as in the plain 16-bit output
     assert rel_l2(O.decode16(dtype, y16.numpy(np.uint16, rows)), g / (1 + np.exp(-g)) * u) <= 4e-3
+
+
+@pytest.mark.parametrize("rows,cols", [(1030, 4096), (1030, 6144), (514, 8192), (130, 12288)])
+def test_forced_start_up_behind_a_norm_of_any_width(rows, cols):
+    """With the exact start-up asked for everywhere, rows behind the norm that do not fit the registers (more than 4096 columns with four waves) are
+    normalised whole all the same: bit for bit the launch's without."""
+    rng = np.random.default_rng(rows + cols)
+    w = O.synth_16(BF16, 5, 17, rows * cols, 0.0, 0.02).reshape(rows, cols)
+    xf = rng.normal(0, 1, cols).astype(np.float32)
+    gamma = O.encode16(BF16, rng.normal(1, 0.1, cols).astype(np.float32))
+    dw, dxf, dg, y = dev(w), dev(xf), dev(gamma), N.DeviceBuffer(rows * 4)
+    outs = {}
+    try:
+        for waves in (4, 16):
+            for mode in (2, 1):
+                N.Device.set_tuning("gemv_workgroup_waves", waves)
+                N.Device.set_tuning("gemv_exact_start", mode)
+                N.gemv(BF16, dw, rows, cols, input_f32=dxf, gamma=dg, eps=1e-6, out_f32=y)
+                outs[waves, mode] = y.numpy(np.float32).copy()
+    finally:
+        N.Device.reset_tuning()
+    ref = O.gemv_x16(BF16, w, O.encode16(BF16, O.rms_norm(BF16, xf, gamma, 1e-6)))
+    for waves in (4, 16):
+        assert np.array_equal(outs[waves, 1], outs[waves, 2]) and rel_l2(outs[waves, 1], ref) <= REL_L2
