@@ -1526,7 +1526,6 @@ int create_impl(const NervaHipHfDecodeSequenceSessionCreateRequest *rq, bool syn
                            w16(lo[l].k_bias),   w16(lo[l].v_bias),  w16(lo[l].wo),
                            w16(lo[l].o_bias),   w16(lo[l].wgu),     w16(lo[l].wdown)};
   }
-  err = upload_chain(s);
 
   // ---- weights -------------------------------------------------------------
   out->failure_stage = 4;
@@ -1616,6 +1615,7 @@ int create_impl(const NervaHipHfDecodeSequenceSessionCreateRequest *rq, bool syn
       upload(lo[l].wdown, src.w_down, H * I);
     }
   }
+  if (err == hipSuccess) err = upload_chain(s);
   if (err != hipSuccess) {
     out->hip_error = static_cast<int32_t>(err);
     destroy_session(s);

@@ -54,3 +54,36 @@ for cus, each, chained in ((256, 2, True), (16, 2, True), (16, 1, False), (8, 3,
     assert step(s).graph_nodes == (3 if chained else 3 + 5 * 4), (cus, each)
     s.destroy()
 """)
+
+
+@pytest.mark.parametrize("source", ["tensors", "plan", "synthetic", "fork"])
+def test_a_copy_that_fails_fails_the_creation(double, source):
+    """Whichever of the copies of a session's creation or of a fork fails - tables, weights, what a chain's launch reads -, the call does."""
+    run(double, """
+weights = model()
+plan = N.WeightPlan.from_weights(weights) if %(source)r == "plan" else None
+cfg = dict(dtype=BF16, hidden=256, heads=4, kv_heads=2, head_dim=64, intermediate=512, vocab=64, layers=4, rms_eps=1e-6, rope_theta=1e6)
+parent = N.DecodeSession.create(weights, 64)
+
+def make():
+    if %(source)r == "fork":
+        return parent.fork_shared_weights()
+    if %(source)r == "synthetic":
+        return N.DecodeSession.create_synthetic(cfg, 64)
+    return N.DecodeSession.create(weights, 64, plan=plan, tensor_pointers=plan is None)
+
+double.double_fail_copy(-1)
+s = make()
+copies = double.double_copies()
+assert copies >= 3 and step(s).graph_nodes == 3
+s.destroy()
+for i in range(copies):
+    double.double_fail_copy(i)
+    try:
+        make().destroy()
+    except RuntimeError as e:
+        assert "hip_error=999" in str(e) and ("stage=0" not in str(e)), e
+    else:
+        raise SystemExit("copy %%d of %%d failed and nobody said so" %% (i, copies))
+double.double_fail_copy(-1)
+""" % dict(source=source))
