@@ -731,7 +731,7 @@ bool latent_attention_wide(uint32_t heads, uint32_t key_dim, uint32_t rot_dim, u
 
 bool latent_riders_fit(uint32_t kv_rank, uint32_t hidden, uint32_t top, uint32_t ff, uint32_t shared_ff) {
   const uint32_t rows = 2u * kUnitKeys * (kv_rank + 64u) * 2u, columns = layer::back_columns(0, top, ff, shared_ff);
-  return 2u * layer::padded(hidden) <= std::min<uint32_t>(rows, 32u * 1024u) && 2u * columns <= 36u * 1024u;   // (beside the launches' own LDS, four workgroups a CU)
+  return 2u * layer::padded(hidden) <= std::min<uint32_t>(rows, 32u * 1024u) && 2u * columns <= 36u * 1024u;   // (beside the launches' own LDS: four workgroups a CU, of the value launch from 28 KiB on three)
 }
 
 uint64_t latent_workspace_bytes(uint32_t heads, uint32_t rot_dim, uint32_t kv_rank, uint32_t max_tokens) {
@@ -766,7 +766,8 @@ hipError_t launch_latent_attention_wide(uint32_t dtype, const LatentAttnParams &
     return hipErrorInvalidValue;
   const bool rides = riders.absorb.begin != riders.absorb.end || riders.rows.begin != riders.rows.end || riders.back.y != nullptr;
   if (rides && (p.cursor == nullptr || !latent_riders_fit(p.kv_rank, riders.back.hidden, riders.back.top, riders.back.ff, riders.back.shared_ff) ||
-                riders.absorb.begin > riders.absorb.end || riders.rows.begin > riders.rows.end || riders.back.mix_cols != 0))
+                riders.absorb.begin > riders.absorb.end || riders.rows.begin > riders.rows.end || riders.back.mix_cols != 0 ||
+                riders.absorb.experts == 0 || riders.rows.experts == 0 || riders.back.experts == 0))
     return hipErrorInvalidValue;
   if (p.cursor != nullptr ? p.tokens != 1 : (p.position + p.tokens - 1) / kKvBlockTokens > p.last_block) return hipErrorInvalidValue;
   if (p.kv_rank == 512) return launch_shape<512, 64>(p, riders, stream, launches);

@@ -64,7 +64,7 @@ struct LayerBack {
   const uint16_t *e_out, *act;             // [experts][hidden][ff], [top][ff]
   const uint32_t *ids;
   const float *weights;
-  uint32_t ff, top;                        // top 0: no feed-forward
+  uint32_t ff, top, experts;               // top 0: no feed-forward
   const uint16_t *shared_out, *shared_act;
   uint32_t shared_ff;                      // 0: no shared expert
   float *y;                                // riders: the sums go here instead ...
@@ -84,6 +84,7 @@ struct RiderPairs {
   const uint16_t *h16;                     // [hidden]
   const uint16_t *w;                       // [matrices][2 * ff][hidden]
   const uint32_t *ids;                     // the matrix of pairs k * ff .., or null: there is one
+  uint32_t experts;                        // matrices there are
   uint32_t hidden, ff, begin, end;         // pairs begin .. end-1; none: begin == end
   float limit;
   uint16_t *act;                           // [pairs]

@@ -186,7 +186,7 @@ hipError_t launch_layer_middle(uint32_t dtype, const LayerMiddle &p, hipStream_t
 hipError_t launch_layer_back(uint32_t dtype, const LayerBack &p, hipStream_t stream) {
   if (dtype != kBF16 || p.x == nullptr || p.w_o == nullptr || p.mixed == nullptr || p.hidden == 0 || p.mix_cols == 0 || p.y != nullptr || p.cursor == nullptr ||
       !layer_gemv_takes(8, 8, p.mix_cols, 0, p.top, p.top != 0 ? p.ff : 0, p.shared_ff) ||
-      (p.top != 0 && (p.e_out == nullptr || p.act == nullptr || p.ids == nullptr || p.weights == nullptr || p.ff == 0)) ||
+      (p.top != 0 && (p.e_out == nullptr || p.act == nullptr || p.ids == nullptr || p.weights == nullptr || p.ff == 0 || p.experts == 0)) ||
       (p.shared_ff != 0 && (p.shared_out == nullptr || p.shared_act == nullptr)) || !whole(p.w_o) || !whole(p.mixed) || !whole(p.e_out) ||
       !whole(p.act) || !whole(p.shared_out) || !whole(p.shared_act))
     return hipErrorInvalidValue;

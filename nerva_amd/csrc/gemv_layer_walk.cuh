@@ -121,6 +121,12 @@ __device__ __forceinline__ Unit gate_and_up(const uint16_t *w, uint32_t cols, ui
   return Unit{w + static_cast<uint64_t>(i) * cols, w + static_cast<uint64_t>(ff + i) * cols, at, cols, nullptr, nullptr, act + i, limit};
 }
 
+// The expert chosen in a place. A step past the end of the context leaves none there: what earlier launches had in this memory, and weights are asked for
+// before the step's guard is known, so the number is kept among those there are.
+__device__ __forceinline__ uint32_t expert_of(const uint32_t *ids, uint32_t k, uint32_t experts) {
+  return __builtin_amdgcn_readfirstlane(min(ids[k], experts - 1u));
+}
+
 // Gate/up pairs begin .. end-1 of the chosen experts (or of one matrix) beside another launch's workgroups: workgroup `block` of `blocks`,
 // `xs` LDS for the row.
 template <uint32_t DT, int WAVES>
@@ -128,12 +134,12 @@ __device__ __forceinline__ void ride_pairs(const RiderPairs &p, const uint32_t *
   const uint32_t wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
   const auto unit_at = [&](uint32_t i) {
     i += p.begin;
-    const uint32_t k = i / p.ff, e = p.ids != nullptr ? __builtin_amdgcn_readfirstlane(p.ids[k]) : 0u;
+    const uint32_t k = i / p.ff, e = p.ids != nullptr ? expert_of(p.ids, k, p.experts) : 0u;
     return gate_and_up(p.w + static_cast<uint64_t>(e) * 2u * p.ff * p.hidden, p.hidden, p.ff, i - k * p.ff, 0u, p.act + k * p.ff, p.limit);
   };
   PairWalk<DT, decltype(unit_at)> walk(unit_at, p.end - p.begin, wave * blocks + block, blocks * WAVES);
   walk.start();
-  if (*cursor < max_steps) {   // (after the requests, which do not depend on it)
+  if (*cursor < max_steps) {   // (after the requests, which read matrices that exist whatever it says)
     stage_vector<WAVES * kWave>(xs, p.h16, p.hidden);
     __syncthreads();
     walk.run(xs);
@@ -169,7 +175,7 @@ __device__ __forceinline__ void walk_back(const LayerBack &p, uint16_t *xs, Chun
       c = at - shared_at;
     } else if (at >= expert_at) {
       const uint32_t k = (at - expert_at) / padded(p.ff);
-      base = p.e_out + static_cast<uint64_t>(p.ids[k]) * p.hidden * p.ff;
+      base = p.e_out + static_cast<uint64_t>(min(p.ids[k], p.experts - 1u)) * p.hidden * p.ff;
       cols = p.ff;
       c = at - expert_at - k * padded(p.ff);
       factor = p.weights[k];
@@ -213,7 +219,7 @@ __device__ __forceinline__ void walk_back(const LayerBack &p, uint16_t *xs, Chun
   };
   issue(b0);
   issue(b1);
-  if (*p.cursor >= p.max_steps) return;   // (after the requests: an expert's number that no step has left is one that exists, too)
+  if (*p.cursor >= p.max_steps) return;   // (after the requests, which read matrices that exist whatever it says)
   // the inputs, under the first requests
   if (p.mix_cols != 0) stage_vector<kThreads>(xs, p.mixed, p.mix_cols);
   for (uint32_t k = 0; k < p.top; ++k) stage_vector<kThreads>(xs + expert_at + k * padded(p.ff), p.act + k * p.ff, p.ff);

@@ -373,6 +373,7 @@ hipError_t parallel_step_16(Session *s) {
     b.weights = plan.weights;
     b.ff = d.expert_ff;
     b.top = d.experts != 0 ? d.experts_per_token : 0u;
+    b.experts = d.experts;
     b.shared_out = w.shared_out;
     b.shared_act = s->ff16;
     b.shared_ff = d.shared_ff;
@@ -381,7 +382,7 @@ hipError_t parallel_step_16(Session *s) {
     LayerRiders riders{};
     if (rides) {
       const uint32_t pairs = d.experts_per_token * d.expert_ff;
-      riders.absorb = RiderPairs{f.h16, w.e_in, plan.ids, s->hidden, d.expert_ff, 0u, pairs / 2, d.expert_limit, g.act};
+      riders.absorb = RiderPairs{f.h16, w.e_in, plan.ids, d.experts, s->hidden, d.expert_ff, 0u, pairs / 2, d.expert_limit, g.act};
       riders.rows = riders.absorb;
       riders.rows.begin = riders.absorb.end;
       riders.rows.end = pairs;
