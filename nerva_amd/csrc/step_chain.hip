@@ -28,6 +28,8 @@
 // No word is written before all its readers have read what it held. Every workgroup has rows of o, of gate and up and of down, and writes
 // them behind its own reads of what came before; so when x is whole, everyone has read the activation and the r of that layer, and the
 // attention's output and the x before it.
+#include <float.h>
+
 #include <algorithm>
 #include <type_traits>
 
@@ -587,9 +589,12 @@ __global__ __launch_bounds__(kThreads, 2) void step_chain_kernel(ChainLaunch p) 
     ss = wave_sum(ss);
     if (thread % kWave == 0) sh.red[turn][wave] = ss;
     __syncthreads();
-    // 1 / sqrt by the hardware's (an ulp) and a step of Newton's: what a square root and a division leave of it, in a tenth of the time
+    // 1 / sqrt by the hardware's (an ulp) and a step of Newton's: what a square root and a division leave of it, in a tenth of the time. Neither where
+    // the hardware takes the mean for zero (a denormal), nor where the step multiplies zero and infinity (a sum that overflowed, whose row is zero).
     const float mean = fmaf((sh.red[turn][0] + sh.red[turn][1]) + (sh.red[turn][2] + sh.red[turn][3]), m->inv_hidden, m->eps);
-    const float rough = __builtin_amdgcn_rsqf(mean), scale = fmaf(rough * 0.5f, fmaf(-mean * rough, rough, 1.0f), rough);
+    const float rough = __builtin_amdgcn_rsqf(mean);
+    float scale = fmaf(rough * 0.5f, fmaf(-mean * rough, rough, 1.0f), rough);
+    if (__builtin_expect(!(scale <= FLT_MAX), 0)) scale = 1.0f / sqrtf(mean);
     turn ^= 1u;
 #pragma unroll
     for (int i = 0; i < kX; ++i) {

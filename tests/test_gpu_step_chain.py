@@ -247,3 +247,33 @@ def test_many_chains_and_a_wide_attention_at_once():
     assert together == alone
     for s in sessions[::-1]:
         s.destroy()
+
+
+@pytest.mark.parametrize("scale,eps", [(1e20, 1e-6), (1e-20, 0.0), (2e-19, 0.0), (1e15, 1e-6)])
+def test_norms_of_rows_at_the_ends_of_f32(scale, eps):
+    """Rows whose sum of squares overflows (their norm is zero), whose mean square is a denormal or just not: what the launches give."""
+    dtype, hidden, heads, kv, hd, inter, vocab, layers = BF16, 256, 4, 2, 64, 512, 64, 4
+    rng = np.random.default_rng(4)
+
+    def matrix(shape, mean=0.0, std=0.05):
+        return O.encode16(dtype, rng.normal(mean, std, shape).astype(np.float32))
+    A, KV = heads * hd, kv * hd
+    blocks = [dict(rms_attn=matrix(hidden, 1.0), rms_mlp=matrix(hidden, 1.0), w_q=matrix((A, hidden)), w_k=matrix((KV, hidden)), w_v=matrix((KV, hidden)),
+                   w_o=O.encode16(dtype, rng.normal(0, 0.05 * min(scale, 1.0), (hidden, A)).astype(np.float32)), w_gate=matrix((inter, hidden)),
+                   w_up=matrix((inter, hidden)), w_down=O.encode16(dtype, rng.normal(0, 0.05 * min(scale, 1.0), (hidden, inter)).astype(np.float32)))
+              for _ in range(layers)]
+    weights = N.ModelWeights(dtype, hidden, heads, kv, hd, inter, vocab, eps, 1e4, matrix((vocab, hidden), 0.0, scale), blocks, matrix(hidden, 1.0), matrix((vocab, hidden)))
+    out = []
+    try:
+        for mode in (2, 0):
+            N.Device.set_tuning("step_chain", mode)
+            s = N.DecodeSession.create(weights, 32)
+            for t in (3, 9, 27):
+                rc, res, rows, _ = s.extend([t], [0])
+                assert rc == 0 and res.graph_nodes == (3 if mode == 0 else 3 + 5 * layers)
+            out.append(rows[0])
+            s.destroy()
+    finally:
+        N.Device.reset_tuning()
+    assert np.all(np.isfinite(out[0])) and np.all(np.isfinite(out[1]))
+    assert np.linalg.norm(out[1] - out[0]) <= chain_budget(layers) * np.linalg.norm(out[0])
