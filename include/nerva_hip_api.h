@@ -275,7 +275,8 @@ typedef struct NervaHipHfDecodeSequenceBatchAdvanceRequest {
 /* mirrors NervaCudaHfDecodeSequenceBatchAdvanceResult (nerva_cuda_api.h:945-976). The launch
  * counters count this library's launches: pack = embedding and RMSNorm rows, projection = the
  * multi-row GEMMs (or GEMVs), scatter = K/V rows into the caches, dependency = attention,
- * sampling = sampler launches. *_elapsed_ns stay 0 except projection_elapsed_ns, which is the
+ * sampling = sampler launches; where a sequence's layers are one launch ("step_chain" below), that launch
+ * counts as a projection and is the pack and dependency launches too. *_elapsed_ns stay 0 except projection_elapsed_ns, which is the
  * device time of the whole batch step (the projections are not timed apart from the rest). */
 typedef struct NervaHipHfDecodeSequenceBatchAdvanceResult {
   int32_t status, hip_error, device_count;

@@ -2063,6 +2063,13 @@ int nerva_hip_hf_decode_sequence_batch_advance_one(const NervaHipHfDecodeSequenc
     // workgroups that poll for each other, and two such launches side by side could hold each other's CUs
     NervaHipHfDecodeSequenceResult scratch{};
     Session *before = nullptr;
+    const auto count_step = [out](const Session *q) {   // (a narrow model's layers are one launch, embedding and attention included)
+      const bool chained = decode_graph(q, q->cursor) >= 3;
+      out->pack_kernel_launches += chained ? 0 : 1;
+      out->projection_kernel_launches += chained ? 2ull : 4ull * q->layers + 1;
+      out->dependency_kernel_launches += chained ? 0 : q->layers;
+      out->sampling_kernel_launches += q->sampler.mode == kSamplerGreedy ? 1 : 2;
+    };
     for (uint32_t t = 0; err == hipSuccess && t < T; ++t) {
       Session *q = seqs[t];
       err = ensure_graph(q, decode_graph(q, q->cursor), &scratch);
@@ -2074,10 +2081,7 @@ int nerva_hip_hf_decode_sequence_batch_advance_one(const NervaHipHfDecodeSequenc
         err = hipMemcpyAsync(&q->host_slots[q->cursor], &q->slots[q->cursor], sizeof(Slot), hipMemcpyDeviceToHost,
                              q->stream);
       out->d2h_bytes += sizeof(Slot);
-      out->pack_kernel_launches += 1;
-      out->projection_kernel_launches += 4ull * q->layers + 1;
-      out->dependency_kernel_launches += q->layers;
-      out->sampling_kernel_launches += q->sampler.mode == kSamplerGreedy ? 1 : 2;
+      count_step(q);
     }
     for (uint32_t t = 0; err == hipSuccess && t < T; ++t) {
       Session *q = seqs[t];
@@ -2088,6 +2092,7 @@ int nerva_hip_hf_decode_sequence_batch_advance_one(const NervaHipHfDecodeSequenc
         if (err == hipSuccess)
           err = hipMemcpyAsync(&q->host_slots[q->cursor], &q->slots[q->cursor], sizeof(Slot), hipMemcpyDeviceToHost, q->stream);
         if (err == hipSuccess) err = hipStreamSynchronize(q->stream);
+        count_step(q);
         out->d2h_bytes += sizeof(Slot);
         out->sync_calls += 1;
       }

@@ -122,6 +122,26 @@ def test_a_wait_that_runs_out_ends_the_sequence():
     s.destroy()
 
 
+@pytest.mark.parametrize("mode", [0, 2])
+def test_a_batch_counts_the_launches_of_its_sequences_own_steps(mode):
+    """Sequences of a narrow model step one by one: two projections each where the layers are one launch (that one and the head), else all there are."""
+    dtype, hidden, heads, kv, hd, inter, vocab, layers, theta, qk_norm, bias = SHAPES[1]
+    cfg = dict(dtype=dtype, hidden=hidden, heads=heads, kv_heads=kv, head_dim=hd, intermediate=inter, vocab=vocab, layers=layers, rms_eps=1e-6, rope_theta=theta)
+    try:
+        N.Device.set_tuning("step_chain", mode)
+        s = N.DecodeSession.create_synthetic(cfg, 64, weight_hash=7, weight_std=0.05)
+        sessions = [s] + [s.fork_shared_weights() for _ in range(2)]
+    finally:
+        N.Device.reset_tuning()
+    for i, q in enumerate(sessions):
+        assert q.start(np.arange(5 + i, dtype=np.uint32))[0] == 0 and q.advance(1)[0] == 0
+    rc, res, tokens = N.DecodeSession.batch_advance_one(sessions, 3, 3)
+    got = (res.pack_kernel_launches, res.projection_kernel_launches, res.dependency_kernel_launches, res.sampling_kernel_launches)
+    assert rc == 0 and got == tuple(3 * n for n in ((0, 2, 0, 1) if mode == 0 else (1, 4 * layers + 1, layers, 1)))
+    for q in sessions[::-1]:
+        q.destroy()
+
+
 # Polls that a wait is given where a test has many run out: an eighth of what it has, and far more than a healthy one takes
 SHORT_WAIT = 2000
 
