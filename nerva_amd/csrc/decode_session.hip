@@ -1260,7 +1260,7 @@ hipError_t setup_state(Session *s, int32_t *failure_stage, bool with_weights) {
     s->attn_plan = reinterpret_cast<uint32_t *>(s->arena + off_attn_plan);
   s->sample_ws = s->arena + off_sample_ws;
   if (chain) {
-    s->chain_context = kChainContext;
+    s->chain_context = chain_context(s->hidden, s->heads, s->kv_heads, s->head_dim, s->intermediate);
     s->given_up = s->host_state;
     *s->given_up = 0;
     s->chain_model.words = reinterpret_cast<uint64_t *>(s->arena + off_chain_words);

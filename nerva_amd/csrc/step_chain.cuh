@@ -43,13 +43,15 @@ struct ChainModel {
 // Cache blocks up to which a key head's attention stays with one workgroup: 61 / 101 / 151 keys in one 65.5 / 66 / 68 us a step, in several
 // 67.9 / 68.3 / 68.6; 201 keys 73 and 68.6.
 constexpr uint32_t kChainSingleBlocks = 8;
-constexpr uint32_t kChainMaxHidden = 1024, kChainMaxIn = 4096, kChainMaxSplits = 16;
-// Tokens of context up to which steps run as a chain: with 4000 keys, sixteen splits of sixteen blocks, it is 0.87 to 0.99 of the launches' time.
+constexpr uint32_t kChainMaxHidden = 1024, kChainMaxIn = 4096, kChainMaxQkv = 8192, kChainMaxSplits = 16;
+// Tokens of context up to which any model's steps run as a chain (chain_context: less for some)
 constexpr uint32_t kChainContext = 4096;
 // Polls after which a wait gives up: 3.1 ms (a step whose workgroup 0 stays away), where the longest wait of a healthy launch is some 20 us.
 constexpr uint32_t kChainSpinLimit = 1u << 14;
 // Whether a model's steps can run as a chain.
 bool chain_takes(uint32_t layers, uint32_t hidden, uint32_t heads, uint32_t kv_heads, uint32_t head_dim, uint32_t ff);
+// Tokens of context up to which they do.
+uint32_t chain_context(uint32_t hidden, uint32_t heads, uint32_t kv_heads, uint32_t head_dim, uint32_t ff);
 uint32_t chain_workgroups(uint32_t hidden, uint32_t heads, uint32_t kv_heads, uint32_t head_dim, uint32_t ff);
 // ... and whether the device holds all of them at once.
 bool chain_resident(uint32_t dtype, uint32_t hidden, uint32_t heads, uint32_t kv_heads, uint32_t head_dim, uint32_t ff);

@@ -699,10 +699,15 @@ __global__ __launch_bounds__(kThreads, 2) void step_chain_kernel(ChainLaunch p) 
 
 bool chain_takes(uint32_t layers, uint32_t hidden, uint32_t heads, uint32_t kv_heads, uint32_t head_dim, uint32_t ff) {
   if (!attn_matrix_cores(heads, kv_heads, head_dim) || heads > 512 || hidden > kChainMaxHidden || ff > kChainMaxIn || heads * head_dim > kChainMaxIn) return false;
-  // At least as many units of every projection as workgroups, whole 16-byte pieces, and a table of layers that the tags can tell
-  // apart. Stacks of one to three layers keep their launches: callers look at those piece by piece.
+  // At least as many units of o, of gate and up and of down as workgroups, whole 16-byte pieces, and a table of layers that the tags can tell
+  // apart. Stacks of one to three layers would gain what taller ones do (512 x 1376, 700 keys: 38.2 us in launches and 30.0, 56.4 and 42.4, 75.1 and 54.8);
+  // they keep their launches: the smallest models are what a step is inspected on, launch by launch.
   if (layers < 4 || layers >= 255 || hidden < kMaxWorkgroups || hidden % 8 != 0 || ff < 2 * kMaxWorkgroups || ff % 8 != 0 || kv_heads > 32) return false;
-  // Up to 10 MB of weights a layer (see above: 9.4 MB 1.14 to 1.10 times as fast, 13.8 MB 0.93)
+  // More rows of qkv than that are most of a layer, and their words most of its hand-overs (256 x 768, 32 heads of 128 on 32, 12 / 150 / 400 / 1000
+  // keys: 20.4 / 22.0 / 23.3 / 24.0 us a layer in launches, 21.3 / 22.0 / 23.2 / 26.1; 128 x 1024: 20.4 / 22.2 / 23.7 / 24.4, 19.6 / 20.4 / 21.6 / 24.4).
+  if ((heads + 2 * kv_heads) * head_dim > kChainMaxQkv) return false;
+  // Up to 10 MB of weights a layer. That is no line between faster and slower, but as far as all that was measured is faster: 1.00 to 1.32 times
+  // as fast at 40 keys and 1.04 to 1.42 at 700 below it (5 to 10 MB); above it eleven stacks of 10.1 to 14.2 MB 1.04 to 1.17 and 1.07 to 1.25.
   return hidden * (2 * heads + 2 * kv_heads) * head_dim + 3 * hidden * ff <= 5000000u;
 }
 
@@ -713,6 +718,24 @@ uint32_t chain_workgroups(uint32_t hidden, uint32_t heads, uint32_t kv_heads, ui
   uint32_t grid = 32;
   while (grid < want && grid < kMaxWorkgroups) grid *= 2;
   return grid;
+}
+
+// A wave's cache blocks follow one another, so that a chain's attention grows with the blocks that a wave has where the launches' attention, on more
+// workgroups, hardly does: by 1.0 to 1.2 us a layer for each, of a gain of 0.4 to 6. With up to two - 2048 keys in sixteen splits - no stack is
+// slower by more than 2.4 % (1024 x 768, 8 heads of 128 on one, 1600 keys: 21.0 us a layer in launches, 21.5 here), most are 5 to 40 % faster. With three and four
+// those stay faster whose projections are at most seven request groups a wave, one after the other (512 x 1376, 8 heads of 64 on 4, 3950 keys: 21.5 and 18.0; of
+// seventeen one is slower, by 2.4 %), but for eight heads of 128 on one; of twenty with more groups nine are slower at 3000 keys (1024 x 768, 8 of 128 on 2: 20.5 and
+// 22.2; 432 x 872, 6 on 3, would not be: 21.9 and 20.5). Where there are fewer than sixteen splits there are more key heads, whose blocks the launches'
+// attention feels too: up to four all are faster (768 x 768, 16 of 64 on 16, 1600 keys: 22.6 and 22.2), with eight not (3950 keys: 23.8 and 25.8). 48 stacks
+// of eight layers, eight contexts each.
+uint32_t chain_context(uint32_t hidden, uint32_t heads, uint32_t kv_heads, uint32_t head_dim, uint32_t ff) {
+  const uint32_t grid = chain_workgroups(hidden, heads, kv_heads, head_dim, ff), waves = grid * kWaves, splits = std::min(kChainMaxSplits, grid / kv_heads);
+  const auto up = [](uint32_t n, uint32_t d) { return (n + d - 1) / d; };
+  const uint32_t wide = up(hidden, 128 * kGroup);   // request groups of a row of qkv or of gate and up; of o and of down below
+  const uint32_t walks = up((heads + 2 * kv_heads) * head_dim / 4, waves) * wide + up(ff / 2, waves) * wide +
+                         up(hidden, waves) * (up(heads * head_dim, 512 * kGroup) + up(ff, 512 * kGroup));
+  const bool long_contexts = splits < kChainMaxSplits || (walks <= 7 && !(head_dim == 128 && heads / kv_heads == 8));
+  return std::min(kChainContext, (long_contexts ? 4 : 2) * kWaves * splits * kKvBlockTokens);
 }
 
 uint64_t chain_place(ChainModel &m, uint32_t head_dim) {

@@ -23,6 +23,7 @@ SHAPES = [
     (F16, 1016, 7, 1, 128, 776, 301, 4, 1e6, False, False),
     (BF16, 256, 32, 4, 128, 3000, 301, 4, 1e6, True, True),
     (F16, 264, 20, 20, 64, 4096, 301, 4, 1e4, True, False),
+    (BF16, 1024, 1, 1, 64, 776, 301, 4, 1e4, False, True),      # (fewer heads' rows than workgroups)
 ]
 
 
@@ -93,10 +94,75 @@ def test_sampled_and_stopped_chains_and_forks():
     assert fork.advance(8)[2].tolist() == rest
     assert s.start(prompt, sampler=sampler)[0] == 0
     assert s.advance(16)[2].tolist() == drawn.tolist()
-    rc, res, walked = s.run(prompt, 14)
-    assert rc == 0 and len(walked) == 14
+    stop = greedy.tolist() + rest
+    last = next(i for i in range(2, 14) if stop[i] not in stop[:i])
+    assert s.start(prompt, eos=stop[last])[0] == 0
+    rc, res, stopped = s.advance(14)
+    assert rc == 0 and stopped.tolist() == stop[:last + 1]
     fork.destroy()
     s.destroy()
+
+
+def test_a_prompt_walked_by_chains_is_the_one_that_launches_walk():
+    """run() takes a prompt's tokens step by step: the logits behind it, the tokens from them, the rows in the cache."""
+    dtype, hidden, heads, kv, hd, inter, vocab, layers, theta, qk_norm, bias = SHAPES[0]
+    weights, _ = random_model(dtype, hidden, heads, kv, hd, inter, vocab, layers, 5, theta, qk_norm, bias)
+    prompt = np.random.default_rng(2).integers(0, vocab, 37).astype(np.uint32)
+    results = []
+    try:
+        for mode in (2, 0):
+            N.Device.set_tuning("step_chain", mode)
+            s = N.DecodeSession.create(weights, 64)
+            rc, res, tokens = s.run(prompt, 1)
+            logits = s.logits()
+            assert rc == 0 and res.graph_replays == 37 and tokens.tolist() == [O.greedy_argmax(logits, skip_nonfinite=True)]
+            results.append((logits, s.kv_range(layers - 1, 0, 37)))
+            rc, res, more = s.run(prompt, 14)
+            assert rc == 0 and len(more) == 14 and more[0] == tokens[0]
+            s.destroy()
+    finally:
+        N.Device.reset_tuning()
+    (want, want_rows), (got, got_rows) = results
+    assert np.all(np.isfinite(got)) and rel_l2(got, want) <= chain_budget(layers)
+    for a, b in zip(want_rows, got_rows):
+        assert rel_l2(O.decode16(dtype, b), O.decode16(dtype, a)) <= chain_budget(layers)
+
+
+@pytest.mark.parametrize("shape,line", [(SHAPES[0], 4096), (SHAPES[4], 2048)])
+def test_a_sequence_that_leaves_the_chain_goes_on_with_launches(shape, line):
+    """From some number of keys on a step is its launches again: one call across that line, the steps on either side of it against a session
+    that has the launches throughout - the logits, the launches counted, the rows that the chain left in the cache - and a fork behind it."""
+    dtype, hidden, heads, kv, hd, inter, vocab, layers, theta, qk_norm, bias = shape
+    weights, _ = random_model(dtype, hidden, heads, kv, hd, inter, vocab, layers, 7, theta, qk_norm, bias)
+    prompt = np.random.default_rng(3).integers(0, vocab, line - 5).astype(np.uint32)
+    results = []
+    try:
+        for mode in (2, 0):
+            N.Device.set_tuning("step_chain", mode)
+            s = N.DecodeSession.create(weights, line + 32)
+            assert s.start(prompt)[0] == 0
+            rc, res, tokens = s.advance(12)     # the prompt's token and eleven steps, five of them in one launch
+            assert rc == 0 and res.graph_replays == 11 and res.kernel_launches == (11 * (3 + 5 * layers) if mode == 2 else 5 * 3 + 6 * (3 + 5 * layers))
+            fork = s.fork_shared_weights()
+            assert fork.advance(4)[2].tolist() == s.advance(4)[2].tolist()
+            fork.destroy()
+            s.release_sequence()
+            assert s.extend(prompt)[0] == 0
+            rows = []
+            for i, t in enumerate(prompt[:10]):               # the same tokens whatever the logits say
+                rc, res, logits, _ = s.extend([t], [0])
+                assert rc == 0 and res.kernel_launches == (3 if mode == 0 and i < 5 else 3 + 5 * layers)
+                rows.append(logits[0])
+            results.append((np.array(rows), s.kv_range(layers - 1, len(prompt), 10)))
+            s.destroy()
+    finally:
+        N.Device.reset_tuning()
+    (want, want_rows), (got, got_rows) = results
+    assert np.all(np.isfinite(got))
+    for i in range(10):
+        assert rel_l2(got[i], want[i]) <= chain_budget(layers), i
+    for a, b in zip(want_rows, got_rows):
+        assert rel_l2(O.decode16(dtype, b), O.decode16(dtype, a)) <= chain_budget(layers)
 
 
 def test_a_wait_that_runs_out_ends_the_sequence():

@@ -56,6 +56,41 @@ for cus, each, chained in ((256, 2, True), (16, 2, True), (16, 1, False), (8, 3,
 """)
 
 
+def test_the_models_that_a_chain_takes(double):
+    """Either side of every line: layers, width, feed-forward, key heads, weights a layer."""
+    run(double, """
+double.double_device(256, 2)
+base = dict(dtype=BF16, hidden=256, heads=4, kv_heads=2, head_dim=64, intermediate=512, vocab=64, layers=4, rms_eps=1e-6, rope_theta=1e4)
+for change, chained in (({}, True), (dict(layers=3), False), (dict(layers=254, hidden=128, intermediate=256), True), (dict(layers=255, hidden=128, intermediate=256), False),
+                        (dict(hidden=128), True), (dict(hidden=120), False), (dict(hidden=1024), True), (dict(hidden=1032), False), (dict(hidden=260), False),
+                        (dict(intermediate=256), True), (dict(intermediate=248), False), (dict(intermediate=4096), True), (dict(intermediate=4104), False), (dict(intermediate=516), False),
+                        (dict(heads=32, kv_heads=32), True), (dict(heads=33, kv_heads=33), False), (dict(heads=64, kv_heads=8), True), (dict(heads=65, kv_heads=13), False),
+                        (dict(heads=9, kv_heads=1), False), (dict(heads=32, kv_heads=16, head_dim=128), True), (dict(heads=17, kv_heads=17, head_dim=128), True),
+                        (dict(heads=22, kv_heads=22, head_dim=128), False), (dict(head_dim=96), False),
+                        (dict(hidden=1024, heads=1, kv_heads=1, intermediate=1536), True), (dict(hidden=1024, heads=1, kv_heads=1, intermediate=1544), False)):
+    s = N.DecodeSession.create_synthetic(dict(base, **change), 64)
+    nodes = step(s).graph_nodes
+    assert (nodes == 3) == chained, (change, nodes)
+    s.destroy()
+""")
+
+
+def test_the_contexts_that_a_chain_takes(double):
+    """A step at the last position of a chain's and at the first behind it: blocks a wave by the splits there are, the length of its walks, the heads."""
+    run(double, """
+double.double_device(256, 2)
+base = dict(dtype=BF16, vocab=64, layers=4, rms_eps=1e-6, rope_theta=1e4)
+for hidden, heads, kv, hd, ff, context in ((512, 8, 4, 64, 1376, 4096), (512, 16, 2, 128, 1280, 2048), (1024, 8, 2, 128, 768, 2048), (624, 3, 1, 128, 1808, 2048),
+                                           (176, 8, 1, 128, 864, 2048), (128, 64, 8, 64, 1024, 4096), (768, 16, 16, 64, 768, 2048), (512, 32, 32, 64, 512, 1024),
+                                           (312, 5, 5, 128, 504, 3072), (264, 20, 20, 64, 4096, 1536)):
+    s = N.DecodeSession.create_synthetic(dict(base, hidden=hidden, heads=heads, kv_heads=kv, head_dim=hd, intermediate=ff), 4200)
+    for tokens, nodes in ((context - 1, 3), (context, 3 + 5 * 4)):
+        assert s.start(np.zeros(tokens, np.uint32))[0] == 0
+        assert s.advance(2)[1].graph_nodes == nodes, (hidden, heads, kv, hd, ff, tokens)
+    s.destroy()
+""")
+
+
 @pytest.mark.parametrize("source", ["tensors", "plan", "synthetic", "fork"])
 def test_a_copy_that_fails_fails_the_creation(double, source):
     """Whichever of the copies of a session's creation or of a fork fails - tables, weights, what a chain's launch reads -, the call does."""
