@@ -77,15 +77,18 @@ hipError_t launch_one(const GemvParams &p, const GemvPlan &plan, size_t lds, hip
     const bool xreg = PRO == kProX16 && p.cols == 4096u && tuning(kTuneGemvXRegisters) != 2;
 #define NV_GEMV_WALK(BB, EX, W, XR, RT, RG, WALK) \
   hipLaunchKernelGGL((gemv_fast_kernel<DT, PRO, EPI, NR, BB, EX, W, XR, RT, RG, WALK>), dim3((waves + W - 1) / W), dim3(W * kWave), lds, stream, p)
+// (rows of one batch, and those that do not fit the registers: not the rotated qkv projection, whose rows have 4096 columns, and not behind the norm in
+// sixteen waves, which hold 16384)
 #define NV_GEMV_LAUNCH_AS(BB, EX, W, XR, RT, RG)                                                             \
   do {                                                                                                       \
-    if constexpr (PRO != kProJoin && EPI != kEpiArgmax && !EX && !XR) {                                       \
+    constexpr bool kOtherRows = !EX && !XR && !(PRO == kProRmsNorm && EPI == kEpiF32 && RT && !RG);            \
+    if constexpr (PRO != kProJoin && EPI != kEpiArgmax && kOtherRows) {                                       \
       if (p.cols <= BB * kWave * 8u && p.rows <= (waves + W - 1) / W * W) {                                   \
         NV_GEMV_WALK(BB, EX, W, XR, RT, RG, kWalkOne);                                                       \
         break;                                                                                               \
       }                                                                                                      \
     }                                                                                                        \
-    if constexpr (PRO == kProRmsNorm && !EX && !XR) {                                                        \
+    if constexpr (PRO == kProRmsNorm && kOtherRows && W * kWave * 16u < kFastMaxCols) {                       \
       if (p.cols > W * kWave * 16u) {                                                                        \
         NV_GEMV_WALK(BB, EX, W, XR, RT, RG, kWalkLoops);                                                     \
         break;                                                                                               \
