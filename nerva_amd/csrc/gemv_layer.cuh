@@ -73,7 +73,7 @@ struct LayerBack {
   uint32_t max_steps;
 };
 
-// What rides with the attention's launches (attn_latent.cuh): the chosen experts' gate/up pairs with the first two, the way back of them and of the
+// What rides with the attention's launches (attn_latent.cuh) where a layer's feed-forward is not too large for it (layer_stack.hip): the chosen experts' gate/up pairs with the first two, the way back of them and of the
 // shared expert with the third, in workgroups behind those of the attention. Its launches are latency - 2 MB of W_uk, a window's keys, 2 MB of
 // W_uv -, and leave most of the chip idle; what bounds a layer is some 4 us a launch and its bytes at 5.5 TB/s, so the bytes go where a launch
 // waits anyway. 16 heads in a window of 1024, 2048 wide, 6 of 64 experts of 768 and a shared one of 1536, us: front 7.8 -> 5.9, middle 13.2 -> 6.6,

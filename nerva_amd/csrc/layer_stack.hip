@@ -294,6 +294,16 @@ hipError_t decode_step_16(Session *s) {
   return err == hipSuccess ? decode_head(s, row) : err;
 }
 
+// Bytes of a token's feed-forward up to which it rides with the attention. Riders are few workgroups of four waves beside the attention's own, at a lower rate
+// than the launches of the chip's whole width they are taken from, so that what they save, a launch's wait, is lost on many bytes. us a layer and step at
+// 600 to 1000 keys, on their own and riding: 4 MB (1024 wide) 34.8, 31.8; 31 MB (2048) 52.6, 49.2; 63 MB (4096) 66.2, 63.9; 75 MB (2048, 6 experts of 768, a
+// shared one of 1536) 55.6, 51.2; (2560) 63.3, 62.2; between 86 and 111 MB three stacks are 1.0 to 2.4 % faster, two the same, three 1.4 to 4.0 % slower; 112 MB (4096)
+// 72.6, 75.9; 151 MB (4096) 82.9, 85.6; (3072) 71.9, 74.8; 302 MB (4096, 6 of 1536, shared 3072) 102.2, 110.1. Below the line the slowest of twenty loses 0.9 %.
+constexpr uint64_t kMostRidingBytes = 80u << 20;
+uint64_t feed_forward_bytes(uint32_t hidden, const NervaHipStackLayer &d) {
+  return 3ull * 2ull * hidden * (static_cast<uint64_t>(d.experts_per_token) * d.expert_ff + d.shared_ff);
+}
+
 // Parallel layers of attention over latents and routed experts.
 hipError_t parallel_step_16(Session *s) {
   const StackModel &m = *s->stack;
@@ -307,7 +317,8 @@ hipError_t parallel_step_16(Session *s) {
     const bool fast = takes_latent_wide(s, d);
     // Most of the feed-forward rides with the attention's three launches, which are latency and leave most of the chip idle: the experts'
     // gate and up rows with the first two, the way back with the third.
-    const bool rides = fast && d.experts != 0 && latent_riders_fit(d.kv_rank, s->hidden, d.experts_per_token, d.expert_ff, d.shared_ff);
+    const bool rides = fast && d.experts != 0 && feed_forward_bytes(s->hidden, d) <= kMostRidingBytes &&
+                       latent_riders_fit(d.kv_rank, s->hidden, d.experts_per_token, d.expert_ff, d.shared_ff);
     LayerFront f{};
     f.x = s->x;
     f.mixer_norm = w.norm[0];

@@ -91,6 +91,22 @@ for hidden, heads, kv, hd, ff, context in ((512, 8, 4, 64, 1376, 4096), (512, 16
 """)
 
 
+def test_the_feed_forwards_that_ride_with_the_attention(double):
+    """Up to 80 MiB of a token's experts and shared expert: on either side of the line, by the middle launch's two forms."""
+    run(double, """
+from nerva_amd import stackbench, stacks
+stackbench.VOCAB = 64
+for hidden, experts, top, ff, shared, rides in ((2048, 8, 6, 768, 1536, True), (4096, 4, 4, 512, 512, True), (4096, 8, 6, 768, 1536, False), (3584, 8, 6, 768, 1536, False),
+                                                (2048, 2, 2, 2048, 2728, True), (2048, 2, 2, 2048, 2736, False), (1024, 20, 20, 1024, 64, False)):
+    s = N.DecodeSession.create_stack_synthetic(stackbench.expert_stack_config(hidden, 8, experts, top, ff, shared, 256, 128, 1, 64), 64)
+    before = [double.double_launches(b"layer_middle_kernelILj1ELb%d" % i) for i in (0, 1)]
+    step(s)
+    after = [double.double_launches(b"layer_middle_kernelILj1ELb%d" % i) for i in (0, 1)]
+    assert [b - a for a, b in zip(before, after)] == ([0, 1] if rides else [1, 0]), (hidden, top, ff, shared, before, after)
+    s.destroy()
+""")
+
+
 @pytest.mark.parametrize("source", ["tensors", "plan", "synthetic", "fork"])
 def test_a_copy_that_fails_fails_the_creation(double, source):
     """Whichever of the copies of a session's creation or of a fork fails - tables, weights, what a chain's launch reads -, the call does."""
