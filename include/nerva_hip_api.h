@@ -147,7 +147,8 @@ typedef struct NervaHipHfDecodeSequenceRequest {
   NervaHipHfDecodeSamplerConfig sampler;
 } NervaHipHfDecodeSequenceRequest;
 
-/* mirrors NervaCudaHfDecodeSequenceResult (nerva_cuda_api.h:436-513) */
+/* mirrors NervaCudaHfDecodeSequenceResult (nerva_cuda_api.h:436-513). graph_nodes: of the captured step that the call
+ * ended with (a narrow model has two, one for contexts of up to 4096 keys or fewer: "step_chain" below). */
 typedef struct NervaHipHfDecodeSequenceResult {
   int32_t status, hip_error, device_count;
   uint32_t dtype, hidden, heads, kv_heads, head_dim, intermediate, vocab_size, layer_count,
@@ -848,7 +849,9 @@ typedef struct NervaHipStepProfile {
 /* Runs `repeats` decode steps eagerly at the session's current cursor WITHOUT
  * advancing it or publishing tokens, bracketing each launch with hipEvents on
  * the session stream (the reference's detailed_profile pass:
- * session_profile.inc.cu:35-56, session_decode_prefill.inc.cu:374-809). */
+ * session_profile.inc.cu:35-56, session_decode_prefill.inc.cu:374-809). Always the step launch by launch: of a
+ * narrow model, whose steps run their layers in one launch ("step_chain" below), these are the launches which that one stands
+ * in for, and neither their number nor their times are an advance's. */
 int nerva_hip_session_profile_step(NervaHipHfDecodeSequenceSession *session, uint32_t repeats,
                                    NervaHipStepProfile *out);
 

@@ -155,7 +155,8 @@ __global__ __launch_bounds__(kBlock, RIDES ? 4 : 1) void latent_absorb_kernel(La
   f32x4_t acc[RT];
 #pragma unroll
   for (int i = 0; i < RT; ++i) acc[i] = f32x4_t{0.0f, 0.0f, 0.0f, 0.0f};
-  // The weights and queries of four steps are asked for together: four round trips one behind the other were most of a decode step's launch.
+  // The weights and queries of four steps are asked for together: four round trips one behind the other were most of a decode step's launch
+  // (a block of 2048 tokens: 66 -> 61 us at 32 heads, 36 and 36 at 16).
   for (uint32_t d = 0; d < p.key_dim; d += 128) {
     AbsorbStep<RT> s0, s1, s2, s3;
     const uint32_t last = p.key_dim - 32u;

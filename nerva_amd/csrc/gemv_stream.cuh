@@ -462,10 +462,12 @@ constexpr int kFastMaxColsLoop = 30720;  // ... or, with a 16-bit input, copied 
 // activations - a wave without a row asks for the last one's data, one without a second batch (kWalkOne aside) for its row's again - and in
 // the loop the batch after next is, so that the compiler can count what is on its way behind what it needs: with the requests under
 // `if (total > n)`, or through pointers that it takes for flat ones (global_u16), it waits for everything - the prologue for the first weights, every batch
-// for the next one's. us before -> after: gate/up pairs 8192 x 2048 13.5 -> 12.1, 2560 wide qkv 8.4 -> 7.3, o 6.4 -> 5.5, down 10.5 -> 9.9, 3584 wide o 7.5 -> 6.4,
-// down 25.4 -> 24.1, behind a join at 4096 columns 19.5 -> 19.0, 19.8 -> 18.9 (minGRU), 15.9 -> 14.8 (qkv); decode steps 2048 wide 2.6 % less in all, 2560 wide
-// 1.6 %. Launches with many batches a wave and enough waves on their way gain nothing (pairs of 12288 x 4096 31.0, down 16.8), and two lose, which keep the waits (kLoose): the head
-// (256 workgroups of 16 waves 82.6 -> 84.3) and the rotated qkv projection (9.67 -> 9.89).
+// for the next one's. us a launch of traced steps, before -> after: gate/up pairs 8192 x 2048 13.6 -> 13.0, 2560 wide qkv 8.3 -> 7.3, down 10.2 -> 9.9, 3584 wide pairs
+// 42.4 -> 41.6, o and down together 31.8 -> 30.9, behind a join at 4096 columns 19.6 -> 19.3, 19.7 -> 19.1 (minGRU), 15.6 -> 14.7 (qkv). Launches of steps drawn over
+// widths of 512 to 8192, captured, with other weights each time: of 105, 63 are faster by 1 to 24 %, 34 the same, 8 slower by 1.2 to 4.8 % (ragged pairs
+// 6784 x 2304, 6924 x 3072 behind the norm, down 7168 x 20416), in no whole step of 34 models. Launches with many batches a wave and enough waves on their way gain
+// nothing, and two lose, which keep the waits (kLoose), each measured at the one size: the head (65536 x 4096, 256 workgroups of 16 waves, 82.6 -> 84.3) and the rotated qkv
+// projection (6144 x 4096, 9.67 -> 9.89).
 // WALK: kWalkOne where a wave's share is one batch - the second request, which is not used, made those launches 10 % longer -; kWalkLoops where the norm's
 // row does not fit the registers (its loops would be on the way to every wait, too).
 // EXACT: the shape in which everything about that is a constant (two batches a row, the input in registers): o at 4096 columns 7.5 -> 7.2 us.

@@ -84,7 +84,8 @@ struct NervaHipHfDecodeSequenceSession : nv::RowScratch {
   uint16_t *kc = nullptr, *vc = nullptr;
   uint32_t block_count = 0;
   uint32_t *table = nullptr, *prompt = nullptr;
-  uint32_t *state = nullptr;  // state[0] cursor, state[1] prompt count, state[2] steps executed so far,
+  uint32_t *state = nullptr;  // state[0] cursor, state[1] prompt count, state[2] step number: another one for every step's tags (embed counts it up, a
+                              // narrow model's sampler too, so that its longer contexts count by two),
                               // state[3] fault word (set by a kernel whose bounded wait gave up; cleared by start),
                               // state[4] the step's chain gave up, state[5] how many in a row have (step_given_up)
   nv::Slot *slots = nullptr;

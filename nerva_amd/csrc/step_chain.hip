@@ -3,13 +3,13 @@
 // What bounds a step of a narrow model is neither its bytes (5.8 MB a layer at 512 x 1376: a microsecond) nor its arithmetic but the
 // five launches a layer, 3.4 to 4.2 us each, of which a boundary and the first accesses behind it are most. Here the workgroups stay for the
 // whole step and hand vectors to each other as words of (value, tag), which a reader polls until the tag is its own, and the
-// weights of the next projection are requested before the wait for its input begins: 12 us a layer instead of 19. us a step, 12 / 100 / 260 / 1000
-// / 4000 keys, launches and chain, head and sampler (10 us) included:
-//   4 layers  512 x 1376,  8 heads of  64 on 4:   81 /  84 /  88 /  91 /  92     59 /  64 /  64 /  67 /  76
-//   8 layers  512 x 1792,  4 heads of 128 on 2:  151 / 158 / 173 / 168 / 171    112 / 124 / 127 / 131 / 154
-//   6 layers  640 x 1600,  5 heads of 128 on 5:  125 / 130 / 142 / 137 / 143    107 / 116 / 118 / 121 / 140
-//   8 layers  768 x 2304, 12 heads of  64 on 4:  175 / 178 / 188 / 191 / -      188 / 197 / 207 / 208 / -      (not taken)
-// (in a stack of 13.8 MB a layer the requests, which a launch of 128 workgroups has too few of in flight, cost what the boundaries did).
+// weights of the next projection are requested before the wait for its input begins: 12 us a layer instead of 19. us a step of a call of 24, 12 / 100 /
+// 260 / 1000 / 3950 keys, launches and chain, head and sampler (10 us) and the call's own share included:
+//   4 layers  512 x 1376,  8 heads of  64 on 4:   86 /  87 /  93 /  93 /  94     65 /  68 /  68 /  72 /  80
+//   8 layers  512 x 1792,  4 heads of 128 on 2:  161 / 168 / 176 / 174 / 176    127 / 132 / 133 / 141 / 160
+//   6 layers  640 x 1600,  5 heads of 128 on 5:  133 / 139 / 142 / 143 / 148    120 / 124 / 125 / 131 / 144
+//   8 layers  768 x 2304, 12 heads of  64 on 4:  171 / 174 / 184 / 185 / 188    165 / 167 / 168 / 175 / 191     (not taken: chain_takes)
+// (in a stack of 13.8 MB a layer the requests, which a launch of 128 workgroups has too few of in flight, cost most of what the boundaries did).
 //
 // A layer is five hand-overs: x -> qkv -> attention -> r = x + o -> activation -> x = r + down. Every workgroup reads the whole of x, of
 // the attention's output, of r and of the activation (the residual rows and the norms come with them); a key head's q, k
@@ -727,7 +727,7 @@ uint32_t chain_workgroups(uint32_t hidden, uint32_t heads, uint32_t kv_heads, ui
 // seventeen one is slower, by 2.4 %), but for eight heads of 128 on one; of twenty with more groups nine are slower at 3000 keys (1024 x 768, 8 of 128 on 2: 20.5 and
 // 22.2; 432 x 872, 6 on 3, would not be: 21.9 and 20.5). Where there are fewer than sixteen splits there are more key heads, whose blocks the launches'
 // attention feels too: up to four all are faster (768 x 768, 16 of 64 on 16, 1600 keys: 22.6 and 22.2), with eight not (3950 keys: 23.8 and 25.8). 48 stacks
-// of eight layers, eight contexts each.
+// of eight layers, eight contexts each; of forty others, drawn, the slowest step is so by 3.6 %.
 uint32_t chain_context(uint32_t hidden, uint32_t heads, uint32_t kv_heads, uint32_t head_dim, uint32_t ff) {
   const uint32_t grid = chain_workgroups(hidden, heads, kv_heads, head_dim, ff), waves = grid * kWaves, splits = std::min(kChainMaxSplits, grid / kv_heads);
   const auto up = [](uint32_t n, uint32_t d) { return (n + d - 1) / d; };
