@@ -303,7 +303,7 @@ def test_a_chain_that_never_runs_is_a_step_fault():
 def test_many_chains_and_a_wide_attention_at_once():
     """Six sessions of the largest chains, and one whose attention wants every CU, from threads of their own: whatever of it is resident at a
     time, each gives what it gives alone."""
-    narrow = (BF16, 1024, 8, 4, 128, 1024, 301, 6, 1e6, True, False)
+    narrow = (BF16, 1024, 4, 2, 128, 1024, 301, 6, 1e6, True, False)
     wide = (BF16, 2048, 16, 8, 128, 2048, 301, 2, 1e6, True, False)
     rng = np.random.default_rng(8)
     prompts = [rng.integers(0, 301, n).astype(np.uint32) for n in (1800, 20, 150, 300, 40, 700, 9)]
@@ -317,7 +317,7 @@ def test_many_chains_and_a_wide_attention_at_once():
         for _ in range(20):
             if rc == 0:
                 rc, res, tokens = s.advance(10)
-                out.append((rc, tokens.tolist()))
+                out.append((rc, res.graph_nodes, tokens.tolist()))
         out.append(rc)
 
     alone = [[] for _ in sessions]
@@ -331,6 +331,7 @@ def test_many_chains_and_a_wide_attention_at_once():
         t.join()
     assert all(out[-1] == 0 for out in alone + together)
     assert together == alone
+    assert all(nodes == (3 if i else 3 + 5 * 2) for i, out in enumerate(alone) for rc, nodes, tokens in out[:-1])
     for s in sessions[::-1]:
         s.destroy()
 
