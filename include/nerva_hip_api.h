@@ -34,7 +34,8 @@ extern "C" {
 #define NERVA_HIP_SLOT_SEQUENCE_ID 1u /* types.cuh:35 */
 #define NERVA_HIP_SLOT_DEVICE_COMPLETE 1u /* types.cuh:36 */
 /* No counterpart in the reference: the slot of a token whose step a device-side bounded wait gave up on (the
- * attention's split merge). The token is not valid; the call that reads the slot returns -1 with
+ * attention's split merge; the layers of a narrow model in one launch, where the step was taken again and given up 256 times in a
+ * row). The token is not valid; the call that reads the slot, or the extend of one token that the step was, returns -1 with
  * hip_error = NERVA_HIP_ERROR_STEP_FAULT, and the sequence has to be started again. */
 #define NERVA_HIP_SLOT_DEVICE_FAULT 2u
 #define NERVA_HIP_ERROR_STEP_FAULT 719 /* hipErrorLaunchFailure */
