@@ -11,14 +11,14 @@ use std::process::Command;
 /// must compile without scratch memory, which this script checks like the library's own build (build.py). What
 /// the check cannot see - a register copy the compiler places between such a load and its wait - is covered by
 /// the library's parity tests only, which is why the kernels are built for the one target they were checked on.
-const HAND_ISSUED_LOADS: &[&str] = &["attn_step_kernel", "attn_prompt_kernel", "moe_gate_up_lean_kernel", "moe_down_lean_kernel", "fp8_gemv_lean_kernel", "gemm_deep_kernel", "gemm_flow_kernel", "latent_rows_kernel", "latent_absorb_kernel", "expert_deep_kernel"];
+const HAND_ISSUED_LOADS: &[&str] = &["attn_step_kernel", "attn_prompt_kernel", "moe_gate_up_lean_kernel", "moe_down_lean_kernel", "fp8_gemv_lean_kernel", "gemm_deep_kernel", "gemm_flow_kernel", "latent_rows_kernel", "latent_absorb_kernel", "expert_deep_kernel", "step_wide_kernel"];
 /// Kernels whose tiles take nearly all registers there are: a spill is a trip to memory in every step of their loops.
 const REGISTER_TILES: &[&str] = &["gemm_wide_kernel", "gemm_block_kernel"];
 const SUPPORTED_ARCH: &str = "gfx950";
 
 const SOURCES: &[&str] = &[
     "gemv_stream", "fp8_gemv", "attn_decode", "attn_prompt", "argmax", "synth_fill",
-    "sampler", "gemm_rows", "gemm_block", "gemm_flow", "gemm_few", "gemm_any", "norm_join", "mingru", "attn_mixed", "attn_mixed_wide", "norm_rms", "attn_latent", "attn_latent_wide", "moe_rows", "gemv_layer", "step_chain", "op_entry", "decode_session", "layer_stack",
+    "sampler", "gemm_rows", "gemm_block", "gemm_flow", "gemm_few", "gemm_any", "norm_join", "mingru", "attn_mixed", "attn_mixed_wide", "norm_rms", "attn_latent", "attn_latent_wide", "moe_rows", "gemv_layer", "step_chain", "step_wide", "op_entry", "decode_session", "layer_stack",
 ];
 
 fn main() {

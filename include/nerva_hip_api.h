@@ -34,7 +34,7 @@ extern "C" {
 #define NERVA_HIP_SLOT_SEQUENCE_ID 1u /* types.cuh:35 */
 #define NERVA_HIP_SLOT_DEVICE_COMPLETE 1u /* types.cuh:36 */
 /* No counterpart in the reference: the slot of a token whose step a device-side bounded wait gave up on (the
- * attention's split merge; the layers of a narrow model in one launch, where the step was taken again and given up 256 times in a
+ * attention's split merge; a step's layers in one launch, where the step was taken again and given up 256 times in a
  * row). The token is not valid; the call that reads the slot, or the extend of one token that the step was, returns -1 with
  * hip_error = NERVA_HIP_ERROR_STEP_FAULT, and the sequence has to be started again. */
 #define NERVA_HIP_SLOT_DEVICE_FAULT 2u
@@ -149,7 +149,8 @@ typedef struct NervaHipHfDecodeSequenceRequest {
 } NervaHipHfDecodeSequenceRequest;
 
 /* mirrors NervaCudaHfDecodeSequenceResult (nerva_cuda_api.h:436-513). graph_nodes: of the captured step that the call
- * ended with (a narrow model has two, one for contexts of up to 4096 keys or fewer: "step_chain" below). */
+ * ended with (a model whose steps run their layers in one launch has two, that one for contexts up to some length - and, where the device has other such
+ * sessions, with a launch on either side that waits for its turn and ends it: "step_chain" below). */
 typedef struct NervaHipHfDecodeSequenceResult {
   int32_t status, hip_error, device_count;
   uint32_t dtype, hidden, heads, kv_heads, head_dim, intermediate, vocab_size, layer_count,
@@ -851,7 +852,7 @@ typedef struct NervaHipStepProfile {
  * advancing it or publishing tokens, bracketing each launch with hipEvents on
  * the session stream (the reference's detailed_profile pass:
  * session_profile.inc.cu:35-56, session_decode_prefill.inc.cu:374-809). Always the step launch by launch: of a
- * narrow model, whose steps run their layers in one launch ("step_chain" below), these are the launches which that one stands
+ * model whose steps run their layers in one launch ("step_chain" below), these are the launches which that one stands
  * in for, and neither their number nor their times are an advance's. */
 int nerva_hip_session_profile_step(NervaHipHfDecodeSequenceSession *session, uint32_t repeats,
                                    NervaHipStepProfile *out);
@@ -876,8 +877,9 @@ int nerva_hip_session_profile_step(NervaHipHfDecodeSequenceSession *session, uin
  * never in three-wave workgroups), "gemm_block_rotate" (1 + the K-blocks between the places where consecutive row
  * groups of that kernel start their walk; 1: a common start), "mixed_attention_wide" (2: a mixed stack's attention layers
  * through the general kernel, whatever their shape; read at every launch, so a captured step keeps what it was
- * captured with), "latent_attention_wide" (2: the same for layers of attention over latents), "step_chain" (2: sessions of narrow models
- * created afterwards never run a step's layers in one launch), "step_chain_withhold" (a workgroup of that launch stays away so often in a row: the
+ * captured with), "latent_attention_wide" (2: the same for layers of attention over latents), "step_chain" (2: sessions
+ * created afterwards never run a step's layers in one launch; 0: those of dense models of four layers and more do, up to 1024 wide and 10 MB of weights
+ * a layer or from 12 MB on, heads of 64 or 128, one to eight query heads a key head), "step_chain_withhold" (a workgroup of that launch stays away so often in a row: the
  * step gives up and is taken again). Values a kernel
  * cannot take are ignored where they are read. -1 for an unknown name. A null name restores every built-in
  * choice. */

@@ -24,6 +24,9 @@
 #include <algorithm>
 #include <string>
 #include <atomic>
+#include <map>
+#include <memory>
+#include <mutex>
 #include <utility>
 #include <vector>
 
@@ -201,6 +204,49 @@ bool layer_supported(const NervaHipHfDecodeChainLayer &l) {
   return true;
 }
 
+// The sessions of a device whose steps are launches of workgroups that wait for each other. Launches of the wide kind need every CU, and any two of them, or one and
+// a narrow one, that start at the same time may each get part of the chip: while there are such, every step asks for the device's turn first and gives it back.
+struct ChainTurns {
+  std::mutex mutex;
+  std::map<int, std::unique_ptr<nv::ChainTurn>> of;   // by device, for good
+};
+ChainTurns &chain_turns() {
+  static ChainTurns *turns = new ChainTurns;   // (sessions may outlive the library's statics)
+  return *turns;
+}
+// Counts a session; its first of the wide kind on a device allocates the word.
+hipError_t join_chains(Session *s) {
+  int device = 0;
+  hipError_t err = hipGetDevice(&device);
+  if (err != hipSuccess) return err;
+  ChainTurns &turns = chain_turns();
+  const std::lock_guard<std::mutex> lock(turns.mutex);
+  std::unique_ptr<nv::ChainTurn> &turn = turns.of[device];
+  if (turn == nullptr) turn = std::make_unique<nv::ChainTurn>();
+  if (turn->word == nullptr) {
+    void *word = nullptr;
+    err = hipMalloc(&word, 256);
+    if (err == hipSuccess) err = hipMemset(word, 0, 256);
+    if (err != hipSuccess) {
+      if (word != nullptr) (void)hipFree(word);
+      return err;
+    }
+    turn->word = static_cast<uint32_t *>(word);
+  }
+  if (++turn->numbers == 0) turn->numbers = 1;
+  s->chain_number = turn->numbers;
+  s->chain_turn = turn.get();
+  turn->sessions += 1;
+  if (s->chain_wide) turn->wide += 1;
+  return hipSuccess;
+}
+void leave_chains(Session *s) {
+  if (s->chain_turn == nullptr) return;
+  s->chain_turn->sessions -= 1;
+  if (s->chain_wide) s->chain_turn->wide -= 1;
+  s->chain_turn = nullptr;
+}
+
 bool layer_has_weights(const NervaHipHfDecodeChainLayer &l) {
   return l.rms_attn_weight && l.rms_mlp_weight && l.w_q && l.w_k && l.w_v && l.w_o && l.w_gate &&
          l.w_up && l.w_down;
@@ -211,7 +257,8 @@ bool layer_has_weights(const NervaHipHfDecodeChainLayer &l) {
 void nv::destroy_session(Session *s) {
   if (s == nullptr) return;
   if (s->stream) (void)hipStreamSynchronize(s->stream);
-  for (int i = 0; i < 5; ++i) {
+  leave_chains(s);
+  for (int i = 0; i < Session::kGraphs; ++i) {
     if (s->exec[i]) (void)hipGraphExecDestroy(s->exec[i]);
     if (s->graph[i]) (void)hipGraphDestroy(s->graph[i]);
   }
@@ -441,15 +488,17 @@ hipError_t enqueue_step(Session *s, StepMode mode, StepProfiler *prof, int only 
   return hipSuccess;
 }
 
-// The same for a narrow model: its layers in one launch.
-hipError_t enqueue_chain_step(Session *s) {
+// The same with its layers in one launch; `turn`: when it is the session's turn.
+hipError_t enqueue_chain_step(Session *s, bool turn) {
   const int spins = tuning(kTuneAttnMergeSpinLimit);
   ChainLaunch c{};
   c.model = s->chain_model_dev;
   c.trace = s->trace_buf;
   c.spin_limit = spins > 0 ? static_cast<uint32_t>(spins) : kChainSpinLimit;
   c.withhold = static_cast<uint32_t>(std::max(tuning(kTuneStepChainWithhold), 0));
-  hipError_t err = launch_step_chain(s->dtype, s->head_dim, s->chain_model, c, s->stream);
+  hipError_t err = turn ? launch_chain_turn(s->chain_turn->word, s->chain_number, false, s->stream) : hipSuccess;
+  if (err == hipSuccess) err = (s->chain_wide ? launch_step_wide : launch_step_chain)(s->dtype, s->head_dim, s->chain_model, c, s->stream);
+  if (err == hipSuccess && turn) err = launch_chain_turn(s->chain_turn->word, s->chain_number, true, s->stream);
   GemvParams p = head_launch(s, s->x);
   const auto slot = [](uint64_t bytes) { return (bytes + 255u) & ~uint64_t{255}; };
   char *trace = s->trace_buf;
@@ -465,7 +514,7 @@ hipError_t enqueue_chain_step(Session *s) {
   return err == hipSuccess ? head_sample(s, p.sample, head_blocks) : err;
 }
 hipError_t enqueue_graph_step(Session *s, int which) {
-  return which >= 3 ? enqueue_chain_step(s) : enqueue_step(s, which == 1 ? kPromptStep : kDecodeStep, nullptr);
+  return which >= 3 ? enqueue_chain_step(s, which >= 5) : enqueue_step(s, which == 1 ? kPromptStep : kDecodeStep, nullptr);
 }
 
 // Steps are launched kernel by kernel instead of as graph replays when NERVA_HIP_EAGER_STEPS=1 is
@@ -494,10 +543,10 @@ bool eager_steps() {
   return eager;
 }
 
-// Kernel launches of one step (which = 0: decode step, 1: prompt step, 3 and 4: a decode step as a chain).
+// Kernel launches of one step (which = 0: decode step, 1: prompt step, 3 to 6: a decode step as a chain).
 uint64_t step_launches(const Session *s, int which) {
   if (s->stack != nullptr) return stack_step_launches(s);
-  if (which >= 3) return s->sampler.mode == kSamplerGreedy ? 3 : 4;
+  if (which >= 3) return (s->sampler.mode == kSamplerGreedy ? 3 : 4) + (which >= 5 ? 2 : 0);
   // embed + (lm head + greedy finish | lm head + two sampler launches | cursor advance)
   const uint64_t fixed = which == 1 ? 2 : (s->sampler.mode == kSamplerGreedy ? 3 : 4);
   return fixed + 5ull * s->layers;
@@ -509,11 +558,15 @@ hipError_t launch_step(Session *s, int which, NervaHipHfDecodeSequenceResult *ou
 // Index of the captured decode step for the active sampler, at a position.
 int decode_graph(const Session *s, uint32_t position) {
   const bool greedy = s->sampler.mode == kSamplerGreedy;
-  if (position < s->chain_context) return greedy ? 3 : 4;
+  if (position < s->chain_context) {
+    const nv::ChainTurn *t = s->chain_turn;
+    const bool turn = t != nullptr && t->wide != 0 && t->sessions > 1;
+    return (greedy ? 3 : 4) + (turn ? 2 : 0);
+  }
   return greedy ? 0 : 2;
 }
 
-// graph index 0 / 2: decode step (greedy finish / sampler), 1: prompt step, 3 / 4: decode step as a chain
+// graph index 0 / 2: decode step (greedy finish / sampler), 1: prompt step, 3 / 4: decode step as a chain, 5 / 6: behind its turn
 hipError_t ensure_graph(Session *s, int which, NervaHipHfDecodeSequenceResult *out) {
   if (eager_steps()) return hipSuccess;
   if (s->exec[which] != nullptr) {
@@ -595,7 +648,9 @@ hipError_t launch_step(Session *s, int which, NervaHipHfDecodeSequenceResult *ou
       out->kernel_launches += step_launches(s, which);
     return err;
   }
-  hipError_t err = hipGraphLaunch(s->exec[which], s->stream);
+  // (another session may have come or gone since the call made its graphs)
+  hipError_t err = s->exec[which] == nullptr ? ensure_graph(s, which, out) : hipSuccess;
+  if (err == hipSuccess) err = hipGraphLaunch(s->exec[which], s->stream);
   if (err == hipSuccess) {
     out->graph_replays += 1;
     out->graph_launches += 1;
@@ -1101,10 +1156,16 @@ hipError_t upload_chain(Session *s) {
   m.pair_gap = s->pair_gap;
   m.eps = s->eps;
   m.inv_hidden = 1.0f / static_cast<float>(s->hidden);
-  std::vector<ChainStage> stages(4 * s->layer.size());
-  for (size_t l = 0; l < s->layer.size(); ++l) chain_stages(m, s->head_dim, s->layer[l], reinterpret_cast<ChainStage(&)[4]>(stages[4 * l]));
   hipError_t err = hipMemcpy(const_cast<LayerDev *>(m.layer), s->layer.data(), s->layer.size() * sizeof(LayerDev), hipMemcpyHostToDevice);
-  if (err == hipSuccess) err = hipMemcpy(const_cast<ChainStage *>(m.stage), stages.data(), stages.size() * sizeof(ChainStage), hipMemcpyHostToDevice);
+  if (s->chain_wide) {
+    std::vector<WideStage> stages(4 * s->layer.size());
+    for (size_t l = 0; l < s->layer.size(); ++l) wide_stages(m, s->head_dim, s->layer[l], reinterpret_cast<WideStage(&)[4]>(stages[4 * l]));
+    if (err == hipSuccess) err = hipMemcpy(const_cast<WideStage *>(m.wide), stages.data(), stages.size() * sizeof(WideStage), hipMemcpyHostToDevice);
+  } else {
+    std::vector<ChainStage> stages(4 * s->layer.size());
+    for (size_t l = 0; l < s->layer.size(); ++l) chain_stages(m, s->head_dim, s->layer[l], reinterpret_cast<ChainStage(&)[4]>(stages[4 * l]));
+    if (err == hipSuccess) err = hipMemcpy(const_cast<ChainStage *>(m.stage), stages.data(), stages.size() * sizeof(ChainStage), hipMemcpyHostToDevice);
+  }
   return err == hipSuccess ? hipMemcpy(s->chain_model_dev, &m, sizeof(m), hipMemcpyHostToDevice) : err;
 }
 
@@ -1145,9 +1206,11 @@ hipError_t setup_state(Session *s, int32_t *failure_stage, bool with_weights) {
   const uint64_t off_attn_plan = c.take(attn_plan_bytes(kAttnMaxSplits));
   const uint64_t off_attn_tagged = c.take(attn_step_workspace_bytes(s->heads));
   const uint64_t off_sample_ws = c.take(sample_workspace_bytes());
-  const bool chain = tuning(kTuneStepChain) != 2 && tuning(kTuneAttnSplits) == 0 &&
-                     chain_takes(s->layers, s->hidden, s->heads, s->kv_heads, s->head_dim, s->intermediate) &&
-                     chain_resident(s->dtype, s->hidden, s->heads, s->kv_heads, s->head_dim, s->intermediate);
+  const bool chains = tuning(kTuneStepChain) != 2 && tuning(kTuneAttnSplits) == 0;
+  s->chain_wide = chains && wide_takes(s->dtype, s->layers, s->hidden, s->heads, s->kv_heads, s->head_dim, s->intermediate) &&
+                  wide_resident(s->dtype, s->heads, s->kv_heads, s->head_dim);
+  const bool chain = s->chain_wide || (chains && chain_takes(s->layers, s->hidden, s->heads, s->kv_heads, s->head_dim, s->intermediate) &&
+                                       chain_resident(s->dtype, s->hidden, s->heads, s->kv_heads, s->head_dim, s->intermediate));
   if (chain) {
     ChainModel &m = s->chain_model;
     m.layers = s->layers;
@@ -1159,7 +1222,7 @@ hipError_t setup_state(Session *s, int32_t *failure_stage, bool with_weights) {
   }
   const uint64_t off_chain_words = c.take(s->chain_word_bytes);
   const uint64_t off_chain_layers = c.take(chain ? L * sizeof(LayerDev) : 0), off_chain_model = c.take(chain ? sizeof(ChainModel) : 0),
-                 off_chain_stages = c.take(chain ? 4 * L * sizeof(ChainStage) : 0);
+                 off_chain_stages = c.take(chain ? 4 * L * std::max(sizeof(ChainStage), sizeof(WideStage)) : 0);
   // Rows of a prompt block (or a batch step)
   const uint64_t pB = kGemmDeepMaxTokens, widest = std::max<uint64_t>(H, A + 2 * KV);
   struct RowOffsets {
@@ -1260,12 +1323,13 @@ hipError_t setup_state(Session *s, int32_t *failure_stage, bool with_weights) {
     s->attn_plan = reinterpret_cast<uint32_t *>(s->arena + off_attn_plan);
   s->sample_ws = s->arena + off_sample_ws;
   if (chain) {
-    s->chain_context = chain_context(s->hidden, s->heads, s->kv_heads, s->head_dim, s->intermediate);
+    s->chain_context = s->chain_wide ? wide_context(s->kv_heads) : chain_context(s->hidden, s->heads, s->kv_heads, s->head_dim, s->intermediate);
     s->given_up = s->host_state;
     *s->given_up = 0;
     s->chain_model.words = reinterpret_cast<uint64_t *>(s->arena + off_chain_words);
     s->chain_model.layer = reinterpret_cast<LayerDev *>(s->arena + off_chain_layers);
     s->chain_model.stage = reinterpret_cast<ChainStage *>(s->arena + off_chain_stages);
+    s->chain_model.wide = reinterpret_cast<WideStage *>(s->arena + off_chain_stages);
     s->chain_model_dev = reinterpret_cast<ChainModel *>(s->arena + off_chain_model);
   }
   const auto bind_rows = [&](RowScratch &rows, const RowOffsets &o, uint64_t gemm_bytes) {
@@ -1319,6 +1383,7 @@ hipError_t setup_state(Session *s, int32_t *failure_stage, bool with_weights) {
   if (err == hipSuccess) err = hipMemsetAsync(s->arena + off_attn_tagged, 0, attn_step_workspace_bytes(s->heads), s->stream);
   if (err == hipSuccess) err = hipMemsetAsync(s->arena + off_sample_ws, 0, sample_workspace_bytes(), s->stream);
   if (err == hipSuccess && chain) err = hipMemsetAsync(s->chain_model.words, 0, s->chain_word_bytes, s->stream);
+  if (err == hipSuccess && chain) err = join_chains(s);
   if (err == hipSuccess) err = hipMemsetAsync(s->arena + off_pattn_ws, 0, pB * pattn_ws_stride, s->stream);
   if (err == hipSuccess && L > 0) err = hipMemsetAsync(s->arena + off_attn_trace, 0, L * 32 * 8, s->stream);
   if (err == hipSuccess) err = hipMemsetAsync(s->arena + off_kc, 0, 2 * ((kv_half + 255) & ~uint64_t{255}), s->stream);

@@ -62,6 +62,13 @@ struct BatchTable {
   SamplerParams sample[kGemmMaxTokens];
 };
 
+// Of a device: the word that says whose turn it is, and who is there (join_chains).
+struct ChainTurn {
+  uint32_t *word = nullptr;          // device memory
+  uint32_t numbers = 0;
+  std::atomic<uint32_t> sessions{0}, wide{0};   // whose steps run as one launch; of those, with the whole device to themselves
+};
+
 struct StackModel;   // layer_stack.hpp
 
 }  // namespace nv
@@ -102,15 +109,20 @@ struct NervaHipHfDecodeSequenceSession : nv::RowScratch {
   uint32_t *host_state = nullptr;    // 64 words
   // captured steps: 0 decode step with the greedy finish, 1 prompt step, 2 decode step with the
   // temperature / top-k / top-p sampler (its parameters live in device memory, so one capture
-  // serves every such configuration), 3 and 4 the two decode steps with their layers in one launch
-  hipGraph_t graph[5] = {};
-  hipGraphExec_t exec[5] = {};
-  uint64_t graph_nodes[5] = {};
-  // narrow models: positions below chain_context step with their layers in one launch (step_chain.cuh); 0: never
+  // serves every such configuration), 3 and 4 the two decode steps with their layers in one launch, 5 and 6 the
+  // same where the device has other sessions whose launches they must not meet (ChainTurn)
+  static constexpr int kGraphs = 7;
+  hipGraph_t graph[kGraphs] = {};
+  hipGraphExec_t exec[kGraphs] = {};
+  uint64_t graph_nodes[kGraphs] = {};
+  // positions below chain_context step with their layers in one launch (step_chain.cuh); 0: never
   uint32_t chain_context = 0;
   nv::ChainModel chain_model{};      // ... what that launch works on, and its copy on the device
   nv::ChainModel *chain_model_dev = nullptr;
   uint64_t chain_word_bytes = 0;
+  bool chain_wide = false;           // ... of the kind that has the whole device to itself (step_wide.hip)
+  nv::ChainTurn *chain_turn = nullptr;   // the device's, where this session is counted
+  uint32_t chain_number = 0;         // ... under this number
   uint32_t *given_up = nullptr;      // host_state[0]: steps that gave up since the host looked (step_given_up writes it)
   // prompt blocks: up to prefill_pass_tokens prompt tokens per pass through the layers (weights streamed
   // once per pass on the matrix cores), in a long prompt prefill_long_tokens; false = one prompt step per token

@@ -1,4 +1,4 @@
-// A decode step's layers in one launch, for narrow models (step_chain.hip).
+// A decode step's layers in one launch: of narrow models (step_chain.hip) and of wider ones (step_wide.hip).
 #pragma once
 
 #include "nv_common.cuh"
@@ -21,10 +21,19 @@ struct alignas(64) ChainStage {
   uint32_t in_at, in_words, out_at;           // 8-byte words of ChainModel::words
   uint32_t whole, spare;                      // every request of a row is a whole one, and every group has four
 };
+// The same as a wide model's workgroups walk it (pairs of rows of gate and up).
+struct alignas(64) WideStage {
+  const uint16_t *w;
+  const uint16_t *vec;
+  uint32_t cols, row_bytes, rows, up_bytes;   // up_bytes: from a gate row to its up row
+  uint32_t log_parts, per_part;               // parts a row is cut into, requests a part
+  uint32_t in_at, in_words, out_at, spare;
+};
 // What a model's chain works on, in device memory (a session's, written once).
 struct ChainModel {
   const LayerDev *layer;       // device memory, [layers]
-  const ChainStage *stage;     // ..., [layers][4]
+  const ChainStage *stage;     // ..., [layers][4]; a wide model's are `wide`
+  const WideStage *wide;
   const uint16_t *emb;
   const uint32_t *prompt;
   const NervaHipSyntheticTokenSlot *slots;
@@ -46,6 +55,9 @@ constexpr uint32_t kChainSingleBlocks = 8;
 constexpr uint32_t kChainMaxHidden = 1024, kChainMaxIn = 4096, kChainMaxQkv = 8192, kChainMaxSplits = 16;
 // Tokens of context up to which any model's steps run as a chain (chain_context: less for some)
 constexpr uint32_t kChainContext = 4096;
+// ... and those of a wide model: as far as that is the faster step at every shape measured, by the workgroups that read its keys (3584 x 18944, 28 heads on 4, 8000 /
+// 16000 / 32000 keys: 94.4 / 96.9 / 103.3 us a layer in launches, 92.8 / 97.1 / 106.5; 2048 x 8192, 32 heads of 64 on 8: 38.3 / 41.7 / 45.7 and 33.7 / 37.3 / 45.0)
+constexpr uint32_t wide_context(uint32_t kv_heads) { return kv_heads >= 8 ? 32768u : 8192u; }
 // Polls after which a wait gives up: 3.1 ms (a step whose workgroup 0 stays away), where the longest wait of a healthy launch is some 20 us.
 constexpr uint32_t kChainSpinLimit = 1u << 14;
 // Whether a model's steps can run as a chain.
@@ -64,8 +76,19 @@ struct ChainLaunch {
   char *trace;                 // test hook: every link's vector, 256 bytes apart (step_trace_bytes), or null
   uint32_t spin_limit;         // polls after which a wait gives up
   uint32_t withhold;           // test hook: so often in a row a workgroup is missing
+  uint32_t row_at, ring_at, rounds;   // wide models: places in LDS (launch_step_wide)
 };
 // `model`: the same on the host.
 hipError_t launch_step_chain(uint32_t dtype, uint32_t head_dim, const ChainModel &model, const ChainLaunch &p, hipStream_t stream);
+
+// Whether a wider model's steps run as one launch, and whether the device holds all of it.
+bool wide_takes(uint32_t dtype, uint32_t layers, uint32_t hidden, uint32_t heads, uint32_t kv_heads, uint32_t head_dim, uint32_t ff);
+bool wide_resident(uint32_t dtype, uint32_t heads, uint32_t kv_heads, uint32_t head_dim);
+void wide_stages(const ChainModel &model, uint32_t head_dim, const LayerDev &layer, WideStage (&stage)[4]);
+hipError_t launch_step_wide(uint32_t dtype, uint32_t head_dim, const ChainModel &model, const ChainLaunch &p, hipStream_t stream);
+// Where a device has several sessions with such launches: waits for session `of`'s turn, or ends it. `turn`: the device's word.
+// Tries, 64 x 16 cycles and a look each: some 100 ms, many times what a launch lasts that nobody disturbs.
+constexpr uint32_t kChainTurnLimit = 1u << 17;
+hipError_t launch_chain_turn(uint32_t *turn, uint32_t of, bool over, hipStream_t stream);
 
 }  // namespace nv

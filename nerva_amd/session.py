@@ -338,7 +338,7 @@ class DecodeSession:
         return rc, res, out[:res.observed_tokens]
 
     def profile_step(self, repeats=3):
-        """Launch times of a step at the cursor, launch by launch, also where a narrow model's steps run their layers in one."""
+        """Launch times of a step at the cursor, launch by launch, also where steps run their layers in one."""
         res = abi.NervaHipStepProfile()
         rc = self.lib.nerva_hip_session_profile_step(self.handle, repeats, C.byref(res))
         return rc, res

@@ -1,0 +1,148 @@
+"""Decode steps of wider models whose layers run in one launch of a workgroup a CU, against the oracle and against the launches they stand in for."""
+import threading
+
+import numpy as np
+import pytest
+
+import nerva_amd as N
+import oracle as O
+from nerva_amd import abi
+from oracle.links import chain_budget, run_traced_stream
+from test_gpu_session import BF16, F16, random_model, rel_l2
+
+pytestmark = pytest.mark.gpu
+
+# dtype, hidden, heads, kv, hd, inter, vocab, layers, theta, qk_norm, bias: rows of whole and of part requests, rows in one, two, four and eight parts, shares
+# that do not go round, one to eight query heads a key head of both sizes, rows of one to eight pairs a thread, inputs smaller and larger than the attention's place
+SHAPES = [
+    (BF16, 1024, 16, 8, 128, 2816, 301, 4, 1e6, True, False),
+    (F16, 1000, 9, 3, 128, 3608, 301, 4, 1e4, False, True),
+    (BF16, 264, 4, 4, 64, 7704, 301, 4, 1e6, True, True),
+    (F16, 2568, 7, 1, 64, 1032, 301, 4, 0, True, False),
+    (BF16, 512, 64, 8, 128, 520, 301, 4, 1e6, False, False),
+    (BF16, 2048, 16, 2, 64, 1800, 301, 5, 5e5, True, False),
+    (F16, 5128, 2, 2, 128, 520, 301, 4, 1e6, False, True),       # (in bf16 its launches are 2.7e-2 from the oracle after ten steps, too)
+    (F16, 256, 10, 2, 64, 12288, 301, 4, 1e4, True, False),
+]
+
+
+@pytest.mark.parametrize("shape", SHAPES)
+def test_every_link_of_a_step_in_one_launch_matches_the_oracle(shape):
+    """Each vector that a layer hands on, at 1e-3 of the oracle's operator on the device's own input, and the stream's logits within the
+    budget of the chain; the same stream from one call. Positions cross a cache block."""
+    dtype, hidden, heads, kv, hd, inter, vocab, layers, theta, qk_norm, bias = shape
+    weights, model = random_model(dtype, hidden, heads, kv, hd, inter, vocab, layers, hidden, theta, qk_norm, bias)
+    prompt = np.random.default_rng(1).integers(0, vocab, 11).astype(np.uint32)
+    s = N.DecodeSession.create(weights, 64)
+    tokens, worst, e2e = run_traced_stream(s, model, prompt, 10, 64)
+    assert s.start(prompt)[0] == 0
+    rc, res, again = s.advance(10)
+    assert rc == 0 and res.graph_nodes == 3 and res.graph_replays == 9 and again.tolist() == tokens
+    s.destroy()
+    print(sorted(worst.items()), e2e, flush=True)
+
+
+@pytest.mark.parametrize("shape", SHAPES[:6])
+def test_longer_contexts_in_one_launch_give_what_launches_give(shape):
+    """Contexts of one split, of the first several, of as many as there are and of several blocks a wave, behind prompts that both kinds of session
+    have read alike: logits and cache rows of the steps. Only roundings of 16-bit values that lie on a boundary may fall differently."""
+    dtype, hidden, heads, kv, hd, inter, vocab, layers, theta, qk_norm, bias = shape
+    weights, _ = random_model(dtype, hidden, heads, kv, hd, inter, vocab, layers, 7, theta, qk_norm, bias)
+    rng = np.random.default_rng(3)
+    results = []
+    lengths = (30, 125, 130, 255, 1100, 4500)
+    prompts = [rng.integers(0, vocab, n).astype(np.uint32) for n in lengths]
+    try:
+        for mode in (2, 0):
+            N.Device.set_tuning("step_chain", mode)
+            s = N.DecodeSession.create(weights, 4600)
+            out = []
+            for prompt in prompts:
+                assert s.start(prompt)[0] == 0
+                assert s.advance(1)[0] == 0
+                for step in range(3):
+                    rc, res = s.extend(prompt[step:step + 1])[:2]     # the same tokens whatever the logits say
+                    assert rc == 0 and res.kernel_launches == (3 if mode == 0 else 3 + 5 * layers)
+                out.append((s.logits(), s.kv_range(layers - 1, len(prompt), 3)))
+            results.append(out)
+            s.destroy()
+    finally:
+        N.Device.reset_tuning()
+    for n, (want, want_rows), (got, got_rows) in zip(lengths, *results):
+        assert np.all(np.isfinite(got)) and rel_l2(got, want) <= chain_budget(layers), (n, rel_l2(got, want))
+        for a, b in zip(want_rows, got_rows):
+            assert rel_l2(O.decode16(dtype, b), O.decode16(dtype, a)) <= chain_budget(layers), n
+
+
+def test_wide_steps_that_give_up_are_taken_again():
+    """A workgroup that stays away twice at every position: the other waits end, the step is void and taken again, and the tokens are those of a session
+    where nobody does; one that stays away for good is a step fault."""
+    dtype, hidden, heads, kv, hd, inter, vocab, layers, theta, qk_norm, bias = SHAPES[0]
+    cfg = dict(dtype=dtype, hidden=hidden, heads=heads, kv_heads=kv, head_dim=hd, intermediate=inter, vocab=vocab, layers=layers, rms_eps=1e-6, rope_theta=theta)
+    prompt = np.random.default_rng(2).integers(0, vocab, 9).astype(np.uint32)
+    s = N.DecodeSession.create_synthetic(cfg, 64, weight_hash=7, weight_std=0.05)
+    assert s.start(prompt)[0] == 0
+    rc, res, want = s.advance(8)
+    assert rc == 0 and res.graph_replays == 7
+    s.destroy()
+    try:
+        N.Device.set_tuning("attn_merge_spin_limit", 1000)
+        N.Device.set_tuning("step_chain_withhold", 2)
+        s = N.DecodeSession.create_synthetic(cfg, 64, weight_hash=7, weight_std=0.05)
+        assert s.start(prompt)[0] == 0
+        rc, res, got = s.advance(8)
+        assert rc == 0 and res.graph_replays == 3 * 7 and got.tolist() == want.tolist()
+        s.destroy()
+        N.Device.set_tuning("attn_merge_spin_limit", 20)
+        N.Device.set_tuning("step_chain_withhold", 100000)
+        s = N.DecodeSession.create_synthetic(cfg, 64, weight_hash=7, weight_std=0.05)
+        assert s.start(prompt)[0] == 0
+        rc, res, got = s.advance(3)
+        assert rc == -1 and res.hip_error == abi.NERVA_HIP_ERROR_STEP_FAULT
+        s.destroy()
+    finally:
+        N.Device.reset_tuning()
+
+
+def test_sessions_of_wide_and_narrow_models_take_turns():
+    """Three sessions of a wide model and one of a narrow one, from threads of their own: each gives what it gives alone, in steps that ask for their turn
+    (two launches more), and a session that is left alone no longer does."""
+    wide = (BF16, 1024, 16, 8, 128, 2816, 301, 4, 1e6, True, False)
+    narrow = (BF16, 512, 4, 2, 128, 1024, 301, 6, 1e6, True, False)
+    rng = np.random.default_rng(8)
+    prompts = [rng.integers(0, 301, n).astype(np.uint32) for n in (20, 300, 900, 150)]
+    weights = [random_model(*g[:8], 3, *g[8:])[0] for g in (wide, narrow)]
+    first = N.DecodeSession.create(weights[0], 1300)
+
+    def all_steps(s, prompt, out):
+        rc = s.start(prompt)[0]
+        for _ in range(15):
+            if rc == 0:
+                rc, res, tokens = s.advance(10)
+                out.append((rc, tokens.tolist()))
+                out.append(res.graph_nodes)
+        out.append(rc)
+
+    lone = []
+    all_steps(first, prompts[0], lone)
+    assert lone[-1] == 0 and lone[1] == 3
+    sessions = [first] + [first.fork_shared_weights() for _ in range(2)] + [N.DecodeSession.create(weights[1], 1300)]
+    alone = [[] for _ in sessions]
+    for s, prompt, out in zip(sessions, prompts, alone):
+        all_steps(s, prompt, out)
+    together = [[] for _ in sessions]
+    threads = [threading.Thread(target=all_steps, args=a) for a in zip(sessions, prompts, together)]
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join()
+    assert all(out[-1] == 0 for out in alone + together)
+    assert together == alone
+    assert all(nodes == 5 for out in alone for nodes in out[1:-1:2])
+    assert alone[0][::2] == lone[::2]
+    for s in sessions[:0:-1]:
+        s.destroy()
+    again = []
+    all_steps(first, prompts[0], again)
+    assert again == lone
+    first.destroy()

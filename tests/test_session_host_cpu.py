@@ -91,6 +91,66 @@ for hidden, heads, kv, hd, ff, context in ((512, 8, 4, 64, 1376, 4096), (512, 16
 """)
 
 
+def test_the_models_that_a_launch_of_the_whole_device_takes(double):
+    """Either side of every line of the wider models: layers, weights a layer, widths, heads, what fits the LDS; a device that does not hold 256 workgroups; contexts."""
+    run(double, """
+double.double_device(256, 1)
+base = dict(dtype=BF16, hidden=1024, heads=8, kv_heads=2, head_dim=128, intermediate=4096, vocab=64, layers=4, rms_eps=1e-6, rope_theta=1e4)
+for change, wide in (({}, True), (dict(layers=3), False), (dict(layers=254, intermediate=2048), True), (dict(layers=255, intermediate=2048), False),
+                     (dict(intermediate=1096), False), (dict(intermediate=1104), True), (dict(intermediate=4100), False), (dict(hidden=1036), False), (dict(hidden=1032), True),
+                     (dict(hidden=256, intermediate=16384), True), (dict(hidden=248, intermediate=16384), False), (dict(hidden=8192, intermediate=512), True),
+                     (dict(hidden=8200, intermediate=512), False), (dict(hidden=8192, intermediate=504), False), (dict(hidden=512, intermediate=30720), True),
+                     (dict(heads=9, kv_heads=1), False), (dict(heads=32, kv_heads=32), True), (dict(heads=33, kv_heads=33), False),
+                     (dict(heads=64, kv_heads=8, head_dim=64), True), (dict(head_dim=96), False)):
+    s = N.DecodeSession.create_synthetic(dict(base, **change), 64)
+    nodes = step(s).graph_nodes
+    assert (nodes == 3) == wide, (change, nodes)
+    s.destroy()
+for cus, each, wide in ((256, 1, True), (255, 1, False), (128, 2, True), (304, 0, False)):
+    double.double_device(cus, each)
+    s = N.DecodeSession.create_synthetic(base, 64)
+    assert step(s).graph_nodes == (3 if wide else 3 + 5 * 4), (cus, each)
+    s.destroy()
+double.double_device(256, 1)
+for kv, context in ((2, 8192), (8, 32768)):
+    s = N.DecodeSession.create_synthetic(dict(base, kv_heads=kv), context + 8)
+    for tokens, nodes in ((context - 1, 3), (context, 3 + 5 * 4)):
+        assert s.start(np.zeros(tokens, np.uint32))[0] == 0
+        assert s.advance(2)[1].graph_nodes == nodes, (kv, tokens)
+    s.destroy()
+""")
+
+
+def test_steps_take_turns_where_a_device_has_several_such_sessions(double):
+    """With a session whose launches need the whole device there, every session with such a launch, of a narrow model too, steps between two launches more; no longer when it
+    is alone, and never where all are narrow."""
+    run(double, """
+double.double_device(256, 2)
+wide = dict(dtype=BF16, hidden=1024, heads=8, kv_heads=2, head_dim=128, intermediate=4096, vocab=64, layers=4, rms_eps=1e-6, rope_theta=1e4)
+a = N.DecodeSession.create(model(), 64)
+b = a.fork_shared_weights()
+assert step(a).graph_nodes == step(b).graph_nodes == 3
+c = N.DecodeSession.create_synthetic(wide, 64)
+before = double.double_launches(b"chain_turn_kernel")
+assert [step(s).graph_nodes for s in (a, b, c)] == [5, 5, 5]
+assert double.double_launches(b"chain_turn_kernel") - before == 6      # (each was captured once)
+d = N.DecodeSession.create_synthetic(dict(wide, layers=2), 64)         # (steps in launches: no matter)
+a.destroy()
+assert step(c).graph_nodes == 5 and step(d).graph_nodes == 3 + 5 * 2
+b.destroy()
+assert step(c).graph_nodes == 3
+e = N.DecodeSession.create_synthetic(wide, 64)
+assert step(c).graph_nodes == step(e).graph_nodes == 5
+c.destroy()
+a = N.DecodeSession.create(model(), 64)
+assert step(e).graph_nodes == step(a).graph_nodes == 5
+e.destroy()
+assert step(a).graph_nodes == 3
+for s in (a, d):
+    s.destroy()
+""")
+
+
 def test_the_feed_forwards_that_ride_with_the_attention(double):
     """Up to 80 MiB of a token's experts and shared expert: on either side of the line, by the middle launch's two forms."""
     run(double, """
