@@ -262,6 +262,10 @@ void nv::destroy_session(Session *s) {
     if (s->exec[i]) (void)hipGraphExecDestroy(s->exec[i]);
     if (s->graph[i]) (void)hipGraphDestroy(s->graph[i]);
   }
+  for (int i = 0; i < 4; ++i) {
+    if (s->together[i]) (void)hipGraphExecDestroy(s->together[i]);
+    if (s->together_graph[i]) (void)hipGraphDestroy(s->together_graph[i]);
+  }
   if (s->ev0) (void)hipEventDestroy(s->ev0);
   if (s->ev1) (void)hipEventDestroy(s->ev1);
   for (hipEvent_t e : s->staged)
@@ -566,6 +570,24 @@ int decode_graph(const Session *s, uint32_t position) {
   return greedy ? 0 : 2;
 }
 
+// `steps` steps of kind `which`, captured.
+hipError_t capture_steps(Session *s, int which, uint32_t steps, hipGraph_t *graph, hipGraphExec_t *exec) {
+  hipError_t err = hipStreamBeginCapture(s->stream, hipStreamCaptureModeThreadLocal);
+  if (err != hipSuccess) return err;
+  // (a trace that is armed is the next step's: its copies would stay in the graph, and write to the caller's buffer ever after)
+  char *const trace = std::exchange(s->trace_buf, nullptr);
+  hipError_t step_err = hipSuccess;
+  for (uint32_t i = 0; step_err == hipSuccess && i < steps; ++i) step_err = enqueue_graph_step(s, which);
+  s->trace_buf = trace;
+  err = hipStreamEndCapture(s->stream, graph);
+  if (step_err != hipSuccess) err = step_err;
+  if (err == hipSuccess) err = hipGraphInstantiate(exec, *graph, nullptr, nullptr, 0);
+  if (err != hipSuccess) {
+    if (*graph) (void)hipGraphDestroy(*graph);
+    *graph = nullptr;
+  }
+  return err;
+}
 // graph index 0 / 2: decode step (greedy finish / sampler), 1: prompt step, 3 / 4: decode step as a chain, 5 / 6: behind its turn
 hipError_t ensure_graph(Session *s, int which, NervaHipHfDecodeSequenceResult *out) {
   if (eager_steps()) return hipSuccess;
@@ -577,22 +599,14 @@ hipError_t ensure_graph(Session *s, int which, NervaHipHfDecodeSequenceResult *o
     return hipSuccess;
   }
   hipGraph_t graph = nullptr;
-  hipError_t err = hipStreamBeginCapture(s->stream, hipStreamCaptureModeThreadLocal);
-  if (err != hipSuccess) return err;
-  // (a trace that is armed is the next step's: its copies would stay in the graph, and write to the caller's buffer ever after)
-  char *const trace = std::exchange(s->trace_buf, nullptr);
-  hipError_t step_err = enqueue_graph_step(s, which);
-  s->trace_buf = trace;
-  err = hipStreamEndCapture(s->stream, &graph);
-  if (step_err != hipSuccess) err = step_err;
-  size_t nodes = 0;
-  if (err == hipSuccess) err = hipGraphGetNodes(graph, nullptr, &nodes);
   hipGraphExec_t exec = nullptr;
-  if (err == hipSuccess) err = hipGraphInstantiate(&exec, graph, nullptr, nullptr, 0);
-  if (err != hipSuccess) {
-    if (graph) (void)hipGraphDestroy(graph);
-    return err;
+  size_t nodes = 0;
+  hipError_t err = capture_steps(s, which, 1, &graph, &exec);
+  if (err == hipSuccess && (err = hipGraphGetNodes(graph, nullptr, &nodes)) != hipSuccess) {
+    (void)hipGraphExecDestroy(exec);
+    (void)hipGraphDestroy(graph);
   }
+  if (err != hipSuccess) return err;
   s->graph[which] = graph;
   s->exec[which] = exec;
   s->graph_nodes[which] = nodes;
@@ -603,11 +617,27 @@ hipError_t ensure_graph(Session *s, int which, NervaHipHfDecodeSequenceResult *o
   return hipSuccess;
 }
 
+// A graph's launch leaves the device idle for 4 us, which the launches within it do not (replays of three launches of 17.4 us each: 56.4 us, of 24
+// 415; the launches alone 52.4 and 419), so steps of few launches go out kStepsTogether at a time once a session has taken enough of them to pay for that graph
+// (some 0.15 ms). Of steps of five launches a layer that is nothing, and their graphs take longer to make.
+constexpr uint64_t kTogetherFrom = 64;
+void ensure_together(Session *s, uint32_t position, uint32_t steps, NervaHipHfDecodeSequenceResult *out) {
+  const int which = decode_graph(s, position);
+  if (eager_steps() || which < 3 || steps < Session::kStepsTogether || s->together[which - 3] != nullptr || s->chain_steps + steps < kTogetherFrom) return;
+  if (capture_steps(s, which, Session::kStepsTogether, &s->together_graph[which - 3], &s->together[which - 3]) == hipSuccess) {
+    out->graph_captures += 1;
+  } else {   // (the single ones do)
+    (void)hipGetLastError();
+    s->chain_steps = 0;
+  }
+}
+
 // Those of `steps` decode steps from a position on.
 hipError_t ensure_graphs(Session *s, uint32_t position, uint32_t steps, NervaHipHfDecodeSequenceResult *out) {
   const int first = decode_graph(s, position), last = decode_graph(s, position + steps - 1);
   hipError_t err = ensure_graph(s, first, out);
   if (err == hipSuccess && last != first) err = ensure_graph(s, last, out);
+  if (err == hipSuccess) ensure_together(s, position, steps, out);
   return err;
 }
 
@@ -655,6 +685,24 @@ hipError_t launch_step(Session *s, int which, NervaHipHfDecodeSequenceResult *ou
     out->graph_replays += 1;
     out->graph_launches += 1;
     out->kernel_launches += s->graph_nodes[which];
+    if (which >= 3) s->chain_steps += 1;
+  }
+  return err;
+}
+// As many of `steps` steps from a position on as go out together: *taken.
+hipError_t launch_steps(Session *s, uint32_t position, uint32_t steps, uint32_t *taken, NervaHipHfDecodeSequenceResult *out) {
+  constexpr uint32_t kMost = Session::kStepsTogether;
+  const int which = decode_graph(s, position);
+  *taken = 1;
+  if (which < 3 || steps < kMost || s->trace_buf != nullptr || s->together[which - 3] == nullptr || position + kMost > s->chain_context)
+    return launch_step(s, which, out);
+  *taken = kMost;
+  hipError_t err = hipGraphLaunch(s->together[which - 3], s->stream);
+  if (err == hipSuccess) {
+    out->graph_replays += kMost;
+    out->graph_launches += 1;
+    out->kernel_launches += kMost * s->graph_nodes[which];
+    s->chain_steps += kMost;
   }
   return err;
 }
@@ -2392,8 +2440,8 @@ int nerva_hip_hf_decode_sequence_session_advance(const NervaHipHfDecodeSequenceS
   if (run_count != 0) err = ensure_graphs(s, s->cursor, run_count, out);
   const uint64_t allocs_before = allocation_count();
   if (err == hipSuccess && run_count != 0) err = hipEventRecord(s->ev0, s->stream);
-  for (uint32_t step = 0; err == hipSuccess && step < run_count; ++step) {
-    err = launch_step(s, decode_graph(s, s->cursor + step), out);
+  for (uint32_t step = 0, taken = 1; err == hipSuccess && step < run_count; step += taken) {
+    err = launch_steps(s, s->cursor + step, s->has_eos != 0 ? 1 : run_count - step, &taken, out);
     // With a stop token the host looks at each token so that it can stop launching
     // (session_api_lifecycle.inc.cu:1206-1234); without one the loop never syncs.
     if (err == hipSuccess && s->has_eos != 0) {
@@ -2489,9 +2537,7 @@ int nerva_hip_hf_decode_sequence_session_run(const NervaHipHfDecodeSequenceSessi
   if (err == hipSuccess) err = ensure_graphs(s, 0, context_steps, out);
   const uint64_t allocs_before = allocation_count();
   if (err == hipSuccess) err = hipEventRecord(s->ev0, s->stream);
-  for (uint32_t step = 0; err == hipSuccess && step < context_steps; ++step) {
-    err = launch_step(s, decode_graph(s, step), out);
-  }
+  for (uint32_t step = 0, taken = 1; err == hipSuccess && step < context_steps; step += taken) err = launch_steps(s, step, context_steps - step, &taken, out);
   const uint64_t slots_bytes = static_cast<uint64_t>(context_steps) * sizeof(Slot);
   for (uint32_t again = 0; err == hipSuccess;) {
     err = launch_steps_again(s, context_steps, again, out);

@@ -115,6 +115,11 @@ struct NervaHipHfDecodeSequenceSession : nv::RowScratch {
   hipGraph_t graph[kGraphs] = {};
   hipGraphExec_t exec[kGraphs] = {};
   uint64_t graph_nodes[kGraphs] = {};
+  // Of graphs 3 to 6, kStepsTogether steps of them in one graph (ensure_together)
+  static constexpr uint32_t kStepsTogether = 6;   // (calls of 8 to 32 steps: the fewest launches with what is left over, which goes out singly)
+  hipGraph_t together_graph[4] = {};
+  hipGraphExec_t together[4] = {};
+  uint64_t chain_steps = 0;          // steps that went out as chains
   // positions below chain_context step with their layers in one launch (step_chain.cuh); 0: never
   uint32_t chain_context = 0;
   nv::ChainModel chain_model{};      // ... what that launch works on, and its copy on the device

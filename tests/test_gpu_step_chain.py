@@ -364,3 +364,29 @@ def test_norms_of_rows_at_the_ends_of_f32(scale, eps):
         N.Device.reset_tuning()
     assert np.all(np.isfinite(out[0])) and np.all(np.isfinite(out[1]))
     assert np.linalg.norm(out[1] - out[0]) <= chain_budget(layers) * np.linalg.norm(out[0])
+
+
+@pytest.mark.parametrize("wide", [False, True])
+def test_steps_that_go_out_together_give_what_single_ones_give(wide):
+    """Greedy and sampled, one session and a second beside it that makes steps take turns, past the context where steps become launches: a call of 100 steps against
+    calls of one."""
+    shape = (BF16, 1024, 16, 8, 128, 2816, 301, 4, 1e6, True, False) if wide else SHAPES[0]
+    dtype, hidden, heads, kv, hd, inter, vocab, layers, theta, qk_norm, bias = shape
+    weights, _ = random_model(dtype, hidden, heads, kv, hd, inter, vocab, layers, 5, theta, qk_norm, bias)
+    prompt = np.random.default_rng(2).integers(0, vocab, 9).astype(np.uint32)
+    sampler = abi.NervaHipHfDecodeSamplerConfig()
+    sampler.temperature, sampler.top_p, sampler.top_k, sampler.seed = 0.9, 0.95, 0, 11
+    s = N.DecodeSession.create(weights, 160)
+    for beside in (False, True):
+        other = s.fork_shared_weights() if beside else None
+        for config in (None, sampler):
+            assert s.start(prompt, sampler=config)[0] == 0
+            single = np.concatenate([s.advance(1)[2] for _ in range(101)])
+            logits = s.logits()
+            assert s.start(prompt, sampler=config)[0] == 0
+            rc, res, tokens = s.advance(101)
+            assert rc == 0 and res.graph_replays == 100 and res.graph_launches == 16 + 4
+            assert tokens.tolist() == single.tolist() and np.array_equal(s.logits(), logits)
+        if other is not None:
+            other.destroy()
+    s.destroy()

@@ -198,3 +198,34 @@ for i in range(copies):
         raise SystemExit("copy %%d of %%d failed and nobody said so" %% (i, copies))
 double.double_fail_copy(-1)
 """ % dict(source=source))
+
+
+def test_steps_that_go_out_together(double):
+    """Steps of few launches share graphs once a session has taken 64, in calls of six and more without a stop token and short of the context where other steps begin:
+    as many replays as steps, as many launches as sixes and single ones. (The stand-in publishes no tokens, so every call starts anew.)"""
+    run(double, """
+def go(s, n, prompt=5, eos=None):
+    assert s.start(np.zeros(prompt, np.uint32), eos=eos)[0] == 0
+    res = s.advance(n + 1)[1]                             # (the first token is the prompt's)
+    return res.graph_replays, res.graph_launches, res.kernel_launches, res.graph_captures
+
+s = N.DecodeSession.create(model(), 4200)
+assert go(s, 40) == (40, 40, 120, 1)
+assert go(s, 23) == (23, 23, 69, 0)
+assert go(s, 5) == (5, 5, 15, 0)
+assert go(s, 24) == (24, 4, 72, 1)
+assert go(s, 5) == (5, 5, 15, 0)
+assert go(s, 23) == (23, 3 + 5, 69, 0)
+assert go(s, 23, eos=63)[1:] == (23, 69, 0)
+context = next(p for p in range(1024, 4200, 1024) if go(s, 1, p)[2] != 3)
+assert go(s, 24, context - 15) == (24, 2 + 12, 15 * 3 + 9 * (3 + 5 * 4), 0)
+wide = dict(dtype=BF16, hidden=1024, heads=8, kv_heads=2, head_dim=128, intermediate=4096, vocab=64, layers=4, rms_eps=1e-6, rope_theta=1e4)
+c = N.DecodeSession.create_synthetic(wide, 64)            # its turn now: graphs of their own for that
+assert go(s, 12) == (12, 2, 60, 2)
+c.destroy()
+assert go(s, 12) == (12, 2, 36, 0)
+s.destroy()
+launches = N.DecodeSession.create_synthetic(dict(wide, layers=2), 512)
+assert go(launches, 100)[:2] == (100, 100)
+launches.destroy()
+""")
