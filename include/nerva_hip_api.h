@@ -151,7 +151,8 @@ typedef struct NervaHipHfDecodeSequenceRequest {
 /* mirrors NervaCudaHfDecodeSequenceResult (nerva_cuda_api.h:436-513). graph_nodes: of the captured step that the call
  * ended with (a model whose steps run their layers in one launch has two, that one for contexts up to some length - and, where the device has other such
  * sessions, with a launch on either side that waits for its turn and ends it: "step_chain" below). graph_replays: steps that
- * were replayed, several of which may share one of graph_launches. */
+ * were replayed, several of which may share one of graph_launches: graphs made of a captured step several times over, which graph_captures and
+ * graph_cache_hits do not count. */
 typedef struct NervaHipHfDecodeSequenceResult {
   int32_t status, hip_error, device_count;
   uint32_t dtype, hidden, heads, kv_heads, head_dim, intermediate, vocab_size, layer_count,

@@ -621,12 +621,10 @@ hipError_t ensure_graph(Session *s, int which, NervaHipHfDecodeSequenceResult *o
 // 415; the launches alone 52.4 and 419), so steps of few launches go out kStepsTogether at a time once a session has taken enough of them to pay for that graph
 // (some 0.15 ms). Of steps of five launches a layer that is nothing, and their graphs take longer to make.
 constexpr uint64_t kTogetherFrom = 64;
-void ensure_together(Session *s, uint32_t position, uint32_t steps, NervaHipHfDecodeSequenceResult *out) {
+void ensure_together(Session *s, uint32_t position, uint32_t steps) {
   const int which = decode_graph(s, position);
   if (eager_steps() || which < 3 || steps < Session::kStepsTogether || s->together[which - 3] != nullptr || s->chain_steps + steps < kTogetherFrom) return;
-  if (capture_steps(s, which, Session::kStepsTogether, &s->together_graph[which - 3], &s->together[which - 3]) == hipSuccess) {
-    out->graph_captures += 1;
-  } else {   // (the single ones do)
+  if (capture_steps(s, which, Session::kStepsTogether, &s->together_graph[which - 3], &s->together[which - 3]) != hipSuccess) {   // (the single ones do)
     (void)hipGetLastError();
     s->chain_steps = 0;
   }
@@ -637,7 +635,7 @@ hipError_t ensure_graphs(Session *s, uint32_t position, uint32_t steps, NervaHip
   const int first = decode_graph(s, position), last = decode_graph(s, position + steps - 1);
   hipError_t err = ensure_graph(s, first, out);
   if (err == hipSuccess && last != first) err = ensure_graph(s, last, out);
-  if (err == hipSuccess) ensure_together(s, position, steps, out);
+  if (err == hipSuccess) ensure_together(s, position, steps);
   return err;
 }
 
