@@ -146,3 +146,27 @@ def test_sessions_of_wide_and_narrow_models_take_turns():
     all_steps(first, prompts[0], again)
     assert again == lone
     first.destroy()
+
+
+@pytest.mark.parametrize("layers,hidden,heads,kv,hd,inter", [(1, 4096, 32, 8, 128, 10008), (2, 2048, 16, 8, 128, 4360), (3, 2056, 6, 2, 64, 5608)])
+def test_models_of_few_layers(layers, hidden, heads, kv, hd, inter):
+    """One to three layers, the first and the last of a launch among them: the logits of a step behind a prompt that both kinds of session have read alike, at contexts of one split and
+    of several, within the budget of the chain."""
+    cfg = dict(dtype=BF16, hidden=hidden, heads=heads, kv_heads=kv, head_dim=hd, intermediate=inter, vocab=301, layers=layers, rms_eps=1e-6, rope_theta=1e6)
+    results = []
+    try:
+        for mode in (2, 0):
+            N.Device.set_tuning("step_chain", mode)
+            s = N.DecodeSession.create_synthetic(cfg, 400)
+            out = []
+            for n in (9, 300):
+                assert s.start(np.arange(n, dtype=np.uint32) % 301)[0] == 0
+                rc, res, _ = s.advance(2)
+                assert rc == 0 and res.graph_nodes == (3 if mode == 0 else 3 + 5 * layers)
+                out.append(s.logits())
+            results.append(out)
+            s.destroy()
+    finally:
+        N.Device.reset_tuning()
+    for launches, one in zip(*results):
+        assert rel_l2(one, launches) <= chain_budget(layers)

@@ -101,7 +101,10 @@ for change, wide in (({}, True), (dict(layers=3), False), (dict(layers=254, inte
                      (dict(hidden=256, intermediate=16384), True), (dict(hidden=248, intermediate=16384), False), (dict(hidden=8192, intermediate=512), True),
                      (dict(hidden=8200, intermediate=512), False), (dict(hidden=8192, intermediate=504), False), (dict(hidden=512, intermediate=30720), True),
                      (dict(heads=9, kv_heads=1), False), (dict(heads=32, kv_heads=32), True), (dict(heads=33, kv_heads=33), False),
-                     (dict(heads=64, kv_heads=8, head_dim=64), True), (dict(head_dim=96), False)):
+                     (dict(heads=64, kv_heads=8, head_dim=64), True), (dict(head_dim=96), False),
+                     (dict(layers=3, hidden=2048, intermediate=4352), False), (dict(layers=3, hidden=2048, intermediate=4360), True),    # (32 M weights)
+                     (dict(layers=2, hidden=2048, intermediate=4360), True), (dict(layers=1, hidden=2048, intermediate=4360), False),
+                     (dict(layers=1, hidden=4096, intermediate=9560), False), (dict(layers=1, hidden=4096, intermediate=9568), True)):   # (128 M)
     s = N.DecodeSession.create_synthetic(dict(base, **change), 64)
     nodes = step(s).graph_nodes
     assert (nodes == 3) == wide, (change, nodes)
