@@ -127,12 +127,33 @@ __global__ __launch_bounds__(kBlock) void embed_rows_kernel(const uint16_t *emb,
 }
 
 // Batch step: row t is the embedding of the token sequence t produced last (slot[position - 1]), and
-// the rotation table of its position.
+// the rotation table of its position. What the step's other launches read of the sequence comes with it: `from` is the host's table in pinned memory, of which a
+// workgroup brings its sequence's entries to `table`. (A copy by the runtime
+// ahead of the launch: 9 to 12 us more a step, 820 -> 808 us on the device with 32 sequences 4096 wide, 446 -> 437 with 6 of 1024; the slots' way out likewise.)
 template <uint32_t DT>
-__global__ __launch_bounds__(kBlock) void embed_batch_kernel(const uint16_t *emb, const BatchTable *table, uint32_t hidden,
+__global__ __launch_bounds__(kBlock) void embed_batch_kernel(const uint16_t *emb, const BatchTable *from, BatchTable *table, uint32_t hidden,
                                                              uint32_t vocab, float *x, const float *rope_freq,
                                                              float *rope_cs, uint32_t half_dim) {
-  const uint32_t t = blockIdx.x, pos = table->seq[t].position;
+  constexpr uint32_t kSeq = sizeof(AttnSeq) / 4, kSlots = sizeof(const Slot *) / 4, kSample = sizeof(SamplerParams) / 4;
+  static_assert(sizeof(AttnSeq) % 4 == 0 && sizeof(SamplerParams) % 4 == 0 && kSeq + kSlots + kSample <= kBlock, "a word a thread");
+  const uint32_t t = blockIdx.x;
+  const AttnSeq seq = from->seq[t];
+  const Slot *const slots = from->slots[t];
+  const uint32_t *src = nullptr;
+  uint32_t *dst = nullptr;
+  if (const uint32_t w = threadIdx.x; w < kSeq) {
+    src = reinterpret_cast<const uint32_t *>(&from->seq[t]) + w;
+    dst = reinterpret_cast<uint32_t *>(&table->seq[t]) + w;
+  } else if (w < kSeq + kSlots) {
+    src = reinterpret_cast<const uint32_t *>(&from->slots[t]) + (w - kSeq);
+    dst = reinterpret_cast<uint32_t *>(&table->slots[t]) + (w - kSeq);
+  } else if (w < kSeq + kSlots + kSample) {
+    src = reinterpret_cast<const uint32_t *>(&from->sample[t]) + (w - kSeq - kSlots);
+    dst = reinterpret_cast<uint32_t *>(&table->sample[t]) + (w - kSeq - kSlots);
+  }
+  if (src != nullptr) *dst = *src;
+  const uint32_t pos = seq.position;
+  uint32_t token = pos == 0 ? 0u : slots[pos - 1].token;
   if (rope_freq != nullptr) {
     for (uint32_t i = threadIdx.x; i < half_dim; i += kBlock) {
       float sn, cs;
@@ -141,14 +162,13 @@ __global__ __launch_bounds__(kBlock) void embed_batch_kernel(const uint16_t *emb
       rope_cs[static_cast<uint64_t>(t) * 2 * half_dim + half_dim + i] = sn;
     }
   }
-  uint32_t token = pos == 0 ? 0u : table->slots[t][pos - 1].token;
   if (token >= vocab) token = 0;  // sampled ids are < vocab
   const uint16_t *row = emb + static_cast<uint64_t>(token) * hidden;
   for (uint32_t i = threadIdx.x; i < hidden; i += kBlock) x[static_cast<uint64_t>(t) * hidden + i] = dec16<DT>(row[i]);
 }
 
-// Batch step: the slot every sequence has just published, side by side, for one copy to the host instead of one
-// per sequence (a slot is 10 words; thread = (sequence, word)).
+// Batch step: the slot every sequence has just published, side by side into the host's memory
+// (a slot is 10 words; thread = (sequence, word)).
 __global__ void gather_slots_kernel(const BatchTable *table, uint32_t count, Slot *out) {
   constexpr uint32_t kWords = sizeof(Slot) / sizeof(uint32_t);
   const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x, t = i / kWords, w = i % kWords;
@@ -1313,7 +1333,6 @@ hipError_t setup_state(Session *s, int32_t *failure_stage, bool with_weights) {
   s->batch_ready = head_block && (A + KV) * H * 2 + 3 * H * I >= (9u << 18);
   const uint64_t off_blogits = head_block ? c.take(static_cast<uint64_t>(NERVA_HIP_BATCH_MAX_BLOCK_TOKENS) * V * 4) : 0;
   const uint64_t off_btable = c.take(sizeof(BatchTable));
-  const uint64_t off_bslots = c.take(static_cast<uint64_t>(NERVA_HIP_BATCH_MAX_BLOCK_TOKENS) * sizeof(Slot));
   // ("prefill_walk" override = 1, read here: one prompt step per token where prompt blocks would be possible)
   s->block_prefill = s->rows_ready && tuning(kTunePrefillWalk) != 1;
   // Prompt blocks of 512 tokens where all four projections of a layer have the kernel for them (256 weight rows x
@@ -1401,7 +1420,6 @@ hipError_t setup_state(Session *s, int32_t *failure_stage, bool with_weights) {
   s->pattn_ws_stride = pattn_ws_stride;
   s->blogits = head_block ? reinterpret_cast<float *>(s->arena + off_blogits) : nullptr;
   s->btable = reinterpret_cast<BatchTable *>(s->arena + off_btable);
-  s->bslots = reinterpret_cast<Slot *>(s->arena + off_bslots);
   s->sampler_dev = reinterpret_cast<SamplerDev *>(s->arena + off_sampler_dev);
   s->sampler_keys = reinterpret_cast<uint64_t *>(s->arena + off_sampler_keys);
   {
@@ -1787,13 +1805,11 @@ hipError_t enqueue_batch_step(Session *lead, Session *const *seqs, uint32_t T,
   if (used_blocks <= attn_batch_single_split(lead->heads, lead->kv_heads, lead->head_dim, T)) batch_splits = 1;
   if (const int want = tuning(kTuneBatchSplits); want >= 1 && want <= static_cast<int>(kAttnMaxSplits))
     batch_splits = std::min<uint32_t>(static_cast<uint32_t>(want), min_blocks);
-  hipError_t err = hipMemcpyAsync(lead->btable, host, sizeof(BatchTable), hipMemcpyHostToDevice, st);
-  if (err != hipSuccess) return err;
   if (lead->dtype == kBF16)
-    hipLaunchKernelGGL(embed_batch_kernel<kBF16>, dim3(T), dim3(kBlock), 0, st, lead->emb, lead->btable, H, lead->vocab,
+    hipLaunchKernelGGL(embed_batch_kernel<kBF16>, dim3(T), dim3(kBlock), 0, st, lead->emb, host, lead->btable, H, lead->vocab,
                        lead->px, rope_freq, lead->prope, lead->head_dim / 2);
   else
-    hipLaunchKernelGGL(embed_batch_kernel<kF16>, dim3(T), dim3(kBlock), 0, st, lead->emb, lead->btable, H, lead->vocab,
+    hipLaunchKernelGGL(embed_batch_kernel<kF16>, dim3(T), dim3(kBlock), 0, st, lead->emb, host, lead->btable, H, lead->vocab,
                        lead->px, rope_freq, lead->prope, lead->head_dim / 2);
   err = hipGetLastError();
   out->pack_kernel_launches += 1;
@@ -2150,16 +2166,13 @@ int nerva_hip_hf_decode_sequence_batch_advance_one(const NervaHipHfDecodeSequenc
     err = hipEventRecord(lead->ev0, lead->stream);
     if (err == hipSuccess) err = enqueue_batch_step(lead, seqs, T, out);
     if (err == hipSuccess) err = hipEventRecord(lead->ev1, lead->stream);
-    if (err == hipSuccess) {   // the published slots: gathered on the device, one copy, dealt out on the host
+    if (err == hipSuccess) {   // the published slots: left in pinned memory by the device, dealt out on the host
       constexpr uint32_t kWords = sizeof(Slot) / sizeof(uint32_t);
       hipLaunchKernelGGL(gather_slots_kernel, dim3((T * kWords + 255u) / 256u), dim3(256), 0, lead->stream, lead->btable, T,
-                         lead->bslots);
+                         lead->host_bslots);
       err = hipGetLastError();
       out->pack_kernel_launches += 1;
     }
-    if (err == hipSuccess)
-      err = hipMemcpyAsync(lead->host_bslots, lead->bslots, static_cast<size_t>(T) * sizeof(Slot), hipMemcpyDeviceToHost,
-                           lead->stream);
     out->d2h_bytes += static_cast<uint64_t>(T) * sizeof(Slot);
     if (err == hipSuccess) err = hipStreamSynchronize(lead->stream);
     out->sync_calls += 1;

@@ -139,7 +139,7 @@ struct NervaHipHfDecodeSequenceSession : nv::RowScratch {
   float *blogits = nullptr;          // [NERVA_HIP_BATCH_MAX_BLOCK_TOKENS][vocab] logits of a batch step, or of rows of a prompt block
   uint32_t head_run = 0;             // rows of the last of the latter
   nv::BatchTable *btable = nullptr, *host_btable = nullptr;
-  nv::Slot *bslots = nullptr, *host_bslots = nullptr;   // a batch step's published slots, gathered for one copy
+  nv::Slot *host_bslots = nullptr;   // a batch step's published slots, side by side in pinned memory
   char *pattn_ws = nullptr;
   uint64_t pattn_ws_stride = 0;
   uint32_t prefill_long_tokens = 0;   // tokens a pass of a prompt of more than prefill_pass_tokens takes, with the rows of all sessions on these weights (0: no such passes)
