@@ -1811,7 +1811,7 @@ hipError_t enqueue_batch_step(Session *lead, Session *const *seqs, uint32_t T,
   else
     hipLaunchKernelGGL(embed_batch_kernel<kF16>, dim3(T), dim3(kBlock), 0, st, lead->emb, host, lead->btable, H, lead->vocab,
                        lead->px, rope_freq, lead->prope, lead->head_dim / 2);
-  err = hipGetLastError();
+  hipError_t err = hipGetLastError();
   out->pack_kernel_launches += 1;
   // where the down projection's K slices are added by a launch of their own, that launch writes the RMSNorm that
   // follows as well (the next layer's attention norm, or the final norm): one launch less per layer
