@@ -177,6 +177,36 @@ __global__ void gather_slots_kernel(const BatchTable *table, uint32_t count, Slo
   reinterpret_cast<uint32_t *>(out + t)[w] = reinterpret_cast<const uint32_t *>(slot)[w];
 }
 
+// What a call brings of a sequence before its prompt is read: tokens, from the host's pinned memory to their places, and the position words; of a new sequence
+// its sampler, and what an earlier one has left is cleared. One launch: two copies by the runtime, which the host waited for, and up to five launches more took 30 to 40 us a call, and
+// ones the host waits for keep the sequences of one caller from following each other without a gap.
+struct SequenceParams {
+  const uint32_t *from;        // pinned
+  uint32_t *prompt, *state;
+  uint32_t first, count;       // tokens
+  uint32_t fresh;              // a new sequence
+  SamplerDev sampler;
+  SamplerDev *sampler_dev;
+  uint4 *clear[4];             // on 16-byte boundaries, whole 16-byte pieces of allocations of their own
+  uint64_t pieces[4];
+};
+__global__ __launch_bounds__(kBlock) void sequence_kernel(SequenceParams p) {
+  const uint64_t thread = static_cast<uint64_t>(blockIdx.x) * kBlock + threadIdx.x, threads = static_cast<uint64_t>(gridDim.x) * kBlock;
+  for (uint64_t i = thread; i < p.count; i += threads) p.prompt[p.first + i] = p.from[p.first + i];
+  if (thread == 0) {
+    p.state[0] = p.first;
+    p.state[1] = p.first + p.count;
+    if (p.fresh != 0) {
+      p.state[3] = p.state[4] = p.state[5] = 0u;
+      *p.sampler_dev = p.sampler;
+    }
+  }
+  if (p.fresh == 0) return;
+#pragma unroll
+  for (int r = 0; r < 4; ++r)
+    for (uint64_t i = thread; i < p.pieces[r]; i += threads) p.clear[r][i] = make_uint4(0u, 0u, 0u, 0u);
+}
+
 __global__ void set_state_kernel(uint32_t *state, uint32_t cursor, uint32_t prompt_count, uint32_t clear_fault) {
   if (threadIdx.x == 0 && blockIdx.x == 0) {
     state[0] = cursor;
@@ -293,6 +323,8 @@ void nv::destroy_session(Session *s) {
   if (s->arena && !s->arena_in_weights) (void)hipFree(s->arena);
   if (s->weights != nullptr && s->weights->refs.fetch_sub(1) == 1) {
     if (s->weights->pass_done) (void)hipEventDestroy(s->weights->pass_done);
+    for (hipEvent_t e : s->weights->prompt_done)
+      if (e) (void)hipEventDestroy(e);
     if (s->weights->origin) (void)hipFree(s->weights->origin);
     delete s->weights;
   }
@@ -751,14 +783,6 @@ void fill_header(const Session *s, NervaHipHfDecodeSequenceResult *out, uint32_t
   out->planned_weight_descriptor_hash = s->planned_weight_descriptor_hash;
 }
 
-// The sampler of the sequence that is about to start: normalised the way the reference's ABI does
-// (sampler.cu:422-433; its callers validate before the call, the ABI itself never refuses a
-// configuration) and copied to the device words the sampler kernels read. Not on the per-token path.
-hipError_t set_sampler(Session *s, const NervaHipHfDecodeSamplerConfig &config) {
-  s->sampler = sampler_device_config(config);
-  return hipMemcpy(s->sampler_dev, &s->sampler, sizeof(SamplerDev), hipMemcpyHostToDevice);
-}
-
 uint32_t observed_count(uint32_t steps, uint32_t has_eos, uint32_t eos, const Slot *slots) {
   uint32_t count = steps;
   for (uint32_t i = 0; i < steps; ++i) {
@@ -791,30 +815,46 @@ bool slots_faulted(const Slot *slots, uint32_t count) {
   return false;
 }
 
-hipError_t reset_sequence(Session *s, const uint32_t *prompt_tokens, uint32_t prompt_count,
+// Tokens `first` .. of the sequence, as many as `count`, and its position there, behind what the session's stream holds, for which this waits: the way
+// leads through the session's pinned copy. The caller's memory may be used again as soon as this returns.
+hipError_t bring_tokens(Session *s, SequenceParams p, const uint32_t *tokens, uint32_t first, uint32_t count, NervaHipHfDecodeSequenceResult *out) {
+  const hipError_t err = hipStreamSynchronize(s->stream);
+  if (err != hipSuccess) return err;
+  if (p.fresh != 0 && s->given_up != nullptr) *s->given_up = 0;
+  memcpy(s->host_prompt + first, tokens, static_cast<uint64_t>(count) * sizeof(uint32_t));
+  p.from = s->host_prompt;
+  p.prompt = s->prompt;
+  p.state = s->state;
+  p.first = first;
+  p.count = count;
+  uint64_t most = count;
+  for (const uint64_t pieces : p.pieces) most = std::max(most, pieces);
+  hipLaunchKernelGGL(sequence_kernel, dim3(static_cast<uint32_t>(std::min<uint64_t>((most + kBlock - 1) / kBlock, 256u))), dim3(kBlock), 0, s->stream, p);
+  out->h2d_bytes = static_cast<uint64_t>(count) * sizeof(uint32_t);
+  return hipGetLastError();
+}
+// A new sequence, with its sampler: normalised the way the reference's ABI does
+// (sampler.cu:422-433; its callers validate before the call, the ABI itself never refuses a configuration).
+hipError_t reset_sequence(Session *s, const NervaHipHfDecodeSamplerConfig &config, const uint32_t *prompt_tokens, uint32_t prompt_count,
                           NervaHipHfDecodeSequenceResult *out) {
-  // Not on the per-token path: the prompt is copied synchronously (the caller's buffer may be
-  // reused as soon as this returns) and the cursor is set by a one-thread kernel in stream order.
-  hipError_t err = hipStreamSynchronize(s->stream);
-  if (err == hipSuccess)
-    err = hipMemcpy(s->prompt, prompt_tokens, static_cast<uint64_t>(prompt_count) * sizeof(uint32_t),
-                    hipMemcpyHostToDevice);
-  if (err == hipSuccess)
-    err = hipMemsetAsync(s->slots, 0, static_cast<uint64_t>(s->max_ctx) * sizeof(Slot), s->stream);
+  s->sampler = sampler_device_config(config);
+  SequenceParams p{};
+  p.fresh = 1;
+  p.sampler = s->sampler;
+  p.sampler_dev = s->sampler_dev;
+  int regions = 0;
+  const auto clear = [&](void *at, uint64_t bytes) {
+    if (at == nullptr || bytes == 0) return;
+    p.clear[regions] = static_cast<uint4 *>(at);
+    p.pieces[regions++] = (bytes + 15u) / 16u;
+  };
+  clear(s->slots, static_cast<uint64_t>(s->max_ctx) * sizeof(Slot));
   // the attention's tagged split partials: a tag is unique for 2^23 steps, which no sequence reaches, so with
   // the words cleared here none of an earlier sequence's can ever match
-  if (err == hipSuccess && s->attn_tagged != nullptr)
-    err = hipMemsetAsync(s->attn_tagged, 0, attn_step_workspace_bytes(s->heads), s->stream);
-  if (s->given_up != nullptr) *s->given_up = 0;
-  if (err == hipSuccess && s->chain_word_bytes != 0) err = hipMemsetAsync(s->chain_model.words, 0, s->chain_word_bytes, s->stream);
-  if (err == hipSuccess && s->stack_state_bytes != 0)   // a new sequence's recurrent state
-    err = hipMemsetAsync(s->stack_state, 0, s->stack_state_bytes, s->stream);
-  if (err == hipSuccess) {
-    hipLaunchKernelGGL(set_state_kernel, dim3(1), dim3(64), 0, s->stream, s->state, 0u, prompt_count, 1u);
-    err = hipGetLastError();
-  }
-  out->h2d_bytes = static_cast<uint64_t>(prompt_count) * sizeof(uint32_t);
-  return err;
+  clear(s->attn_tagged, s->attn_tagged != nullptr ? attn_step_workspace_bytes(s->heads) : 0);
+  clear(s->chain_model.words, s->chain_word_bytes);
+  clear(s->stack_state, s->stack_state_bytes);   // a new sequence's recurrent state
+  return bring_tokens(s, p, prompt_tokens, 0, prompt_count, out);
 }
 
 // Token blocks (prompt blocks, batch steps) of more than one row keep their 16-bit activations -
@@ -1083,6 +1123,9 @@ hipError_t allocate_session(Session *s, int32_t *failure_stage, bool with_weight
   if (err == hipSuccess) err = hipEventCreate(&s->ev1);
   for (hipEvent_t &e : s->staged)
     if (err == hipSuccess) err = hipEventCreateWithFlags(&e, hipEventDisableTiming);
+  if (with_weights)
+    for (hipEvent_t &e : s->weights->prompt_done)
+      if (err == hipSuccess) err = hipEventCreateWithFlags(&e, hipEventDisableTiming);
   if (err != hipSuccess) return err;
   s->stage = s->pinned + pinned_seq + pinned_table + pinned_slots;
   s->host_slots = reinterpret_cast<Slot *>(s->pinned);
@@ -2307,8 +2350,9 @@ int nerva_hip_hf_decode_sequence_session_start(const NervaHipHfDecodeSequenceSes
   const uint32_t P = request->prompt_token_count;
   fill_header(s, out, 0, request->prompt_tokens[P - 1]);
   s->started = false;
-  hipError_t err = set_sampler(s, request->sampler);   // session_api_lifecycle.inc.cu:1026
-  if (err == hipSuccess) err = reset_sequence(s, request->prompt_tokens, P, out);
+  const nv::PromptTurn prompt(s);
+  hipError_t err = prompt.error;
+  if (err == hipSuccess) err = reset_sequence(s, request->sampler, request->prompt_tokens, P, out);   // session_api_lifecycle.inc.cu:1026
   // prefill: the first P-1 prompt tokens (in blocks on the matrix cores where the shapes allow,
   // else one captured prompt step per token), then one prompt step with the LM head and sampler
   if (err == hipSuccess && P > 1 && s->stack == nullptr && !s->block_prefill) err = ensure_graph(s, 1, out);
@@ -2359,15 +2403,10 @@ int nerva_hip_session_extend(const NervaHipSessionExtendRequest *request, NervaH
   if (!going_on) {
     s->started = false;
     NervaHipHfDecodeSamplerConfig greedy{};
-    err = set_sampler(s, greedy);
-    if (err == hipSuccess) err = reset_sequence(s, request->tokens, n, out);
+    err = reset_sequence(s, greedy, request->tokens, n, out);
     s->has_eos = 0;
   } else {
-    err = hipStreamSynchronize(s->stream);
-    if (err == hipSuccess)
-      err = hipMemcpy(s->prompt + begin, request->tokens, static_cast<uint64_t>(n) * sizeof(uint32_t), hipMemcpyHostToDevice);
-    if (err == hipSuccess) err = set_device_position(s, begin, end, 0);
-    out->h2d_bytes = static_cast<uint64_t>(n) * sizeof(uint32_t);
+    err = bring_tokens(s, SequenceParams{}, request->tokens, begin, n, out);
   }
   bool idle = false;
   const auto logits_out = [&](uint32_t i) {   // the last step's logits are wanted row i
@@ -2542,8 +2581,7 @@ int nerva_hip_hf_decode_sequence_session_run(const NervaHipHfDecodeSequenceSessi
     if (request->prompt_tokens[i] >= s->vocab) return -1;
   fill_header(s, out, request->steps, request->seed_token);
   s->started = false;
-  hipError_t err = set_sampler(s, request->sampler);   // session_api_lifecycle.inc.cu:770
-  if (err == hipSuccess) err = reset_sequence(s, request->prompt_tokens, P, out);
+  hipError_t err = reset_sequence(s, request->sampler, request->prompt_tokens, P, out);   // session_api_lifecycle.inc.cu:770
   // the decode-step graph walks every position, prompt included (session_api_lifecycle.inc.cu:748-990)
   if (err == hipSuccess) err = ensure_graphs(s, 0, context_steps, out);
   const uint64_t allocs_before = allocation_count();

@@ -6,6 +6,7 @@ import pytest
 
 import nerva_amd as N
 import stack_models as M
+from nerva_amd import abi
 from test_gpu_any_width import walked
 from test_gpu_session import BF16, E2E_REL_L2, F16, random_model, rel_l2
 
@@ -120,3 +121,51 @@ def test_a_fork_made_under_other_overrides():
             s.destroy()
     for got in logits[1:]:
         assert rel_l2(got, logits[0]) <= E2E_REL_L2
+
+
+@pytest.mark.parametrize("geom", [(BF16, 512, 8, 2, 64, 1024, 301, 3), (BF16, 1024, 16, 8, 128, 2816, 301, 4)])   # (steps of launches, of one for the whole device)
+def test_sequences_begun_one_behind_the_other(geom):
+    """Starts and extensions whose callers wait for nothing in between, on sessions of one set of weights and on one session that begins again, the callers' memory written over as soon as
+    a call returns: tokens, logits and cache rows of each as when it is alone."""
+    dtype, hidden, heads, kv, hd, inter, vocab, layers = geom
+    weights, _ = random_model(dtype, hidden, heads, kv, hd, inter, vocab, layers, 4, 1e6, True, False)
+    rng = np.random.default_rng(6)
+    prompts = [rng.integers(0, 301, n).astype(np.uint32) for n in (5, 300, 1, 17, 130, 64)]
+    sampler = abi.NervaHipHfDecodeSamplerConfig()
+    sampler.temperature, sampler.top_p, sampler.top_k, sampler.seed = 0.8, 0.9, 0, 3
+    first = N.DecodeSession.create(weights, 400)
+    sessions = [first] + [first.fork_shared_weights() for _ in prompts[1:]]
+
+    def result(s, n):
+        rc, res, tokens = s.advance(6)
+        assert rc == 0
+        return tokens.tolist(), s.logits().tolist(), [rows.tolist() for rows in s.kv_range(2, 0, n + 5)]
+    alone = []
+    for i, prompt in enumerate(prompts):
+        assert first.start(prompt, sampler=sampler if i % 2 else None)[0] == 0
+        alone.append(result(first, len(prompt)))
+    for round_ in range(3):
+        for i, (s, prompt) in enumerate(zip(sessions, prompts)):
+            buffer = prompts[(i + 1) % len(prompts)].copy()
+            assert s.start(buffer, sampler=None if i % 2 else sampler)[0] == 0      # (begun again at once, with another prompt and sampler)
+            buffer = prompt.copy()
+            assert s.start(buffer, sampler=sampler if i % 2 else None)[0] == 0
+            buffer[:] = 7
+        for i in (range(len(prompts)) if round_ % 2 == 0 else reversed(range(len(prompts)))):
+            assert result(sessions[i], len(prompts[i])) == alone[i], (round_, i)
+    parts = [rng.integers(0, 301, n).astype(np.uint32) for n in (40, 3, 1, 20)]
+
+    def extended(s):
+        s.release_sequence()
+        out = []
+        for part in parts:
+            buffer = part.copy()
+            rc, _, rows, _ = s.extend(buffer, [len(part) - 1])
+            buffer[:] = 7
+            assert rc == 0
+            out.append(rows.tolist())
+        return out
+    want = extended(first)
+    assert all(extended(s) == want for s in sessions[1:])
+    for s in sessions[::-1]:
+        s.destroy()
