@@ -1240,6 +1240,45 @@ hipError_t prompt_tokens(Session *s, uint32_t begin, uint32_t end, const uint32_
   return err;
 }
 
+// Whether a prompt's launches include a decode step's attention, whose workgroups wait for each other: prompts that are walked, and a last token that is alone in its pass.
+bool prompt_steps(const Session *s, uint32_t tokens) {
+  if (s->stack != nullptr) return false;
+  return !s->block_prefill || tuning(kTuneAttnWithholdSplit) != 0 || tokens % s->prefill_pass_tokens == 1 ||
+         (s->prefill_long_tokens != 0 && tokens % s->prefill_long_tokens == 1);
+}
+// Two such launches at once could hold each other's places (a step's attention takes every CU), and a start returns while its own are under way. So a start that has any
+// waits until those of the device's last such start have ended; prompts in blocks may run beside them.
+struct StepPrompts {
+  std::mutex mutex;
+  std::map<int, hipEvent_t> done;   // by device, for good
+};
+class StepPromptTurn {
+ public:
+  StepPromptTurn(Session *session, bool steps) : s(session) {
+    if (!steps) return;
+    static StepPrompts *prompts = new StepPrompts;   // (sessions may outlive the library's statics)
+    turn = std::unique_lock<std::mutex>(prompts->mutex);
+    int device = 0;
+    error = hipGetDevice(&device);
+    if (error != hipSuccess) return;
+    hipEvent_t &event = prompts->done[device];
+    if (event == nullptr) error = hipEventCreateWithFlags(&event, hipEventDisableTiming);
+    if (error == hipSuccess) error = hipEventSynchronize(event);   // (nothing to wait for before its first record)
+    done = event;
+  }
+  ~StepPromptTurn() {
+    if (done != nullptr && hipEventRecord(done, s->stream) != hipSuccess) (void)hipStreamSynchronize(s->stream);
+  }
+  StepPromptTurn(const StepPromptTurn &) = delete;
+  StepPromptTurn &operator=(const StepPromptTurn &) = delete;
+  hipError_t error = hipSuccess;
+
+ private:
+  Session *s;
+  hipEvent_t done = nullptr;
+  std::unique_lock<std::mutex> turn;
+};
+
 // Everything of a session that is not weights, from the dimensions already in `s`: stream, events,
 // the state arena (KV cache, block table, prompt, token slots, cursor words, activations and
 // workspaces), the pinned host mirrors, the step modes. Shared by create and fork.
@@ -2351,7 +2390,8 @@ int nerva_hip_hf_decode_sequence_session_start(const NervaHipHfDecodeSequenceSes
   fill_header(s, out, 0, request->prompt_tokens[P - 1]);
   s->started = false;
   const nv::PromptTurn prompt(s);
-  hipError_t err = prompt.error;
+  const StepPromptTurn steps(s, prompt_steps(s, P));
+  hipError_t err = prompt.error != hipSuccess ? prompt.error : steps.error;
   if (err == hipSuccess) err = reset_sequence(s, request->sampler, request->prompt_tokens, P, out);   // session_api_lifecycle.inc.cu:1026
   // prefill: the first P-1 prompt tokens (in blocks on the matrix cores where the shapes allow,
   // else one captured prompt step per token), then one prompt step with the LM head and sampler

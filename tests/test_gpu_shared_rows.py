@@ -169,3 +169,32 @@ def test_sequences_begun_one_behind_the_other(geom):
     assert all(extended(s) == want for s in sessions[1:])
     for s in sessions[::-1]:
         s.destroy()
+
+
+def test_walked_prompts_begun_one_behind_the_other():
+    """Prompts walked step by step, whose attention launches wait within themselves: begun on five sessions of two models without a wait in between."""
+    geoms = [(BF16, 2048, 16, 8, 128, 2048, 301, 2), (BF16, 512, 8, 2, 64, 1024, 301, 2)]
+    rng = np.random.default_rng(8)
+    prompts = [rng.integers(0, 301, n).astype(np.uint32) for n in (300, 260, 310, 290, 280)]
+    try:
+        N.Device.set_tuning("prefill_walk", 1)
+        models = [N.DecodeSession.create(random_model(*g, 4, 1e6, True, False)[0], 400) for g in geoms]
+        sessions = [models[0], models[1], models[0].fork_shared_weights(), models[1].fork_shared_weights(), models[0].fork_shared_weights()]
+
+        def result(s):
+            rc, _, tokens = s.advance(4)
+            assert rc == 0
+            return tokens.tolist(), s.logits().tolist()
+        alone = []
+        for s, prompt in zip(sessions, prompts):
+            assert s.start(prompt)[0] == 0
+            alone.append(result(s))
+        for s, prompt in zip(sessions, prompts):
+            assert s.start(prompt)[0] == 0
+        for s in sessions:
+            assert s.logits().shape == (301,)      # (waits for the session's own work, so that no step meets another's prompt)
+        assert [result(s) for s in sessions] == alone
+        for s in sessions[::-1]:
+            s.destroy()
+    finally:
+        N.Device.reset_tuning()
