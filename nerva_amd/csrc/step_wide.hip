@@ -608,7 +608,7 @@ bool wide_takes(uint32_t dtype, uint32_t layers, uint32_t hidden, uint32_t heads
   // From 12 MB of weights a layer on (chain_takes ends at 10). 27 stacks drawn between 14 and 501 MB, widths of 768 to 3520, 40 / 700 / 3000 keys: 0.85 of the launches' time
   // on average, 0.71 the least; one is no faster (3520 x 8096, 27 heads of 128 on 27, whose q, k and v are as long as its attention: 59.5 / 61.3 / 66.3 us a layer in launches, 59.7 /
   // 62.1 / 66.1).
-  // Two and three layers: from 64 MB each on, where 14 models take 0.77 to 0.97 of the launches' time a step, at 40 to 3000 keys (2 layers of 2048 x 6144 82.6 -> 67.0 us at 700
+  // Two and three layers: from 64 MB each on, where 21 models, those of one layer among them, take 0.77 to 0.97 of the launches' time a step, at 40 to 3000 keys (2 layers of 2048 x 6144 82.6 -> 67.0 us at 700
   // keys, 3 of 4096 x 12288 238 -> 223); smaller ones would gain as well, and keep the launches. One layer: from 256 MB on, what the memory-side cache holds (4096 x 12288 96.6 -> 87.6,
   // 5120 x 13824 136 -> 116); of a smaller one the launches read the weights there, and past 2000 keys some are the faster steps (1536 x 7000 51.6, 61.3 in one launch; 2560 x 7000 65.0, 66.2).
   const uint64_t weights = static_cast<uint64_t>(hidden) * (2 * heads + 2 * kv_heads) * head_dim + 3ull * hidden * ff;
