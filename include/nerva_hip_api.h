@@ -881,7 +881,7 @@ int nerva_hip_session_profile_step(NervaHipHfDecodeSequenceSession *session, uin
  * through the general kernel, whatever their shape; read at every launch, so a captured step keeps what it was
  * captured with), "latent_attention_wide" (2: the same for layers of attention over latents), "step_chain" (2: sessions
  * created afterwards never run a step's layers in one launch; 0: those of dense models of four layers and more do, up to 1024 wide and 10 MB of weights
- * a layer or from 12 MB on, heads of 64 or 128, one to eight query heads a key head), "step_chain_withhold" (a workgroup of that launch stays away so often in a row: the
+ * a layer or from 12 MB on, of two and three layers from 64 MB on, of one from 256 MB on, heads of 64 or 128, one to eight query heads a key head), "step_chain_withhold" (a workgroup of that launch stays away so often in a row: the
  * step gives up and is taken again). Values a kernel
  * cannot take are ignored where they are read. -1 for an unknown name. A null name restores every built-in
  * choice. */

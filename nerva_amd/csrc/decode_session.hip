@@ -1263,7 +1263,8 @@ class StepPromptTurn {
     if (error != hipSuccess) return;
     hipEvent_t &event = prompts->done[device];
     if (event == nullptr) error = hipEventCreateWithFlags(&event, hipEventDisableTiming);
-    if (error == hipSuccess) error = hipEventSynchronize(event);   // (nothing to wait for before its first record)
+    if (error != hipSuccess) return;
+    nv::wait_if_there(event);
     done = event;
   }
   ~StepPromptTurn() {
@@ -2391,7 +2392,7 @@ int nerva_hip_hf_decode_sequence_session_start(const NervaHipHfDecodeSequenceSes
   s->started = false;
   const nv::PromptTurn prompt(s);
   const StepPromptTurn steps(s, prompt_steps(s, P));
-  hipError_t err = prompt.error != hipSuccess ? prompt.error : steps.error;
+  hipError_t err = steps.error;
   if (err == hipSuccess) err = reset_sequence(s, request->sampler, request->prompt_tokens, P, out);   // session_api_lifecycle.inc.cu:1026
   // prefill: the first P-1 prompt tokens (in blocks on the matrix cores where the shapes allow,
   // else one captured prompt step per token), then one prompt step with the LM head and sampler

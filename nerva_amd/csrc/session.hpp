@@ -235,16 +235,20 @@ class PassTurn {
   std::unique_lock<std::mutex> turn;
 };
 
+// Waits for what an event was recorded behind. One whose stream is gone has nothing left to wait for (a session ends its stream's work before its stream), which the runtime reports as
+// an error; so it does for one that was never recorded. Whatever else goes wrong on the device the session's own stream reports.
+inline void wait_if_there(hipEvent_t event) {
+  if (hipEventSynchronize(event) != hipSuccess) (void)hipGetLastError();
+}
 // A prompt's place among those under way: as long as its launches are enqueued this lives.
 class PromptTurn {
  public:
   explicit PromptTurn(Session *session) : s(session), done(s->weights->prompt_done[s->weights->prompts.fetch_add(1) % SharedWeights::kPromptsAhead]) {
-    error = hipEventSynchronize(done);   // (nothing to wait for before its first record)
+    wait_if_there(done);
   }
   ~PromptTurn() { (void)hipEventRecord(done, s->stream); }
   PromptTurn(const PromptTurn &) = delete;
   PromptTurn &operator=(const PromptTurn &) = delete;
-  hipError_t error = hipSuccess;
 
  private:
   Session *s;

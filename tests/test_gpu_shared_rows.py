@@ -198,3 +198,26 @@ def test_walked_prompts_begun_one_behind_the_other():
             s.destroy()
     finally:
         N.Device.reset_tuning()
+
+
+def test_starts_behind_sessions_that_are_gone():
+    """What the last starts have left to wait for may have been on sessions that have ended since: walked prompts, single tokens, prompts in blocks, on the same weights and on others."""
+    prompts = [np.arange(n, dtype=np.uint32) for n in (1, 40, 300)]
+    tokens = []
+    for walk in (0, 1, 0):
+        N.Device.set_tuning("prefill_walk", walk)
+        try:
+            s = decoder_session(400)
+        finally:
+            N.Device.reset_tuning()
+        for _ in range(4):
+            for prompt in prompts:
+                fork = s.fork_shared_weights()
+                assert fork.start(prompt)[0] == 0
+                fork.destroy()
+                assert s.start(prompt)[0] == 0
+                rc, _, out = s.advance(3)
+                assert rc == 0
+                tokens.append((walk, len(prompt), out.tolist()))
+        s.destroy()
+    assert all(a[2] == b[2] for a in tokens for b in tokens if a[:2] == b[:2])
