@@ -149,8 +149,7 @@ typedef struct NervaHipHfDecodeSequenceRequest {
 } NervaHipHfDecodeSequenceRequest;
 
 /* mirrors NervaCudaHfDecodeSequenceResult (nerva_cuda_api.h:436-513). graph_nodes: of the captured step that the call
- * ended with (a model whose steps run their layers in one launch has two, that one for contexts up to some length - and, where the device has other such
- * sessions, with a launch on either side that waits for its turn and ends it: "step_chain" below). graph_replays: steps that
+ * ended with (a model whose steps run their layers in one launch has two, that one for contexts up to some length: "step_chain" below). graph_replays: steps that
  * were replayed, several of which may share one of graph_launches: graphs made of a captured step several times over, which graph_captures and
  * graph_cache_hits do not count. */
 typedef struct NervaHipHfDecodeSequenceResult {

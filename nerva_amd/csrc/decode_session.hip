@@ -254,47 +254,34 @@ bool layer_supported(const NervaHipHfDecodeChainLayer &l) {
   return true;
 }
 
-// The sessions of a device whose steps are launches of workgroups that wait for each other. Launches of the wide kind need every CU, and any two of them, or one and
-// a narrow one, that start at the same time may each get part of the chip: while there are such, every step asks for the device's turn first and gives it back.
-struct ChainTurns {
-  std::mutex mutex;
-  std::map<int, std::unique_ptr<nv::ChainTurn>> of;   // by device, for good
-};
-ChainTurns &chain_turns() {
-  static ChainTurns *turns = new ChainTurns;   // (sessions may outlive the library's statics)
-  return *turns;
-}
-// Counts a session; its first of the wide kind on a device allocates the word.
-hipError_t join_chains(Session *s) {
+// Counts a session among those of its device that come in order (InOrder).
+hipError_t join_order(Session *s) {
+  struct Orders {
+    std::mutex mutex;
+    std::map<int, std::unique_ptr<nv::LaunchOrder>> of;   // by device, for good
+  };
+  static Orders *orders = new Orders;   // (sessions may outlive the library's statics)
   int device = 0;
   hipError_t err = hipGetDevice(&device);
+  if (err == hipSuccess) err = hipEventCreateWithFlags(&s->launched, hipEventDisableTiming);
+  if (err == hipSuccess) err = hipEventCreateWithFlags(&s->mark, hipEventDisableTiming);
   if (err != hipSuccess) return err;
-  ChainTurns &turns = chain_turns();
-  const std::lock_guard<std::mutex> lock(turns.mutex);
-  std::unique_ptr<nv::ChainTurn> &turn = turns.of[device];
-  if (turn == nullptr) turn = std::make_unique<nv::ChainTurn>();
-  if (turn->word == nullptr) {
-    void *word = nullptr;
-    err = hipMalloc(&word, 256);
-    if (err == hipSuccess) err = hipMemset(word, 0, 256);
-    if (err != hipSuccess) {
-      if (word != nullptr) (void)hipFree(word);
-      return err;
-    }
-    turn->word = static_cast<uint32_t *>(word);
-  }
-  if (++turn->numbers == 0) turn->numbers = 1;
-  s->chain_number = turn->numbers;
-  s->chain_turn = turn.get();
-  turn->sessions += 1;
-  if (s->chain_wide) turn->wide += 1;
+  // 2 ms at 5 TB/s, a step of 40 us at the least
+  const double step = std::max(static_cast<double>(s->resident_weight_bytes) / 5e12, 40e-6);
+  s->steps_ahead = std::max(1u, static_cast<uint32_t>(2e-3 / step));
+  const std::lock_guard<std::mutex> lock(orders->mutex);
+  std::unique_ptr<nv::LaunchOrder> &order = orders->of[device];
+  if (order == nullptr) order = std::make_unique<nv::LaunchOrder>();
+  s->order = order.get();
+  s->order->sessions += 1;
   return hipSuccess;
 }
-void leave_chains(Session *s) {
-  if (s->chain_turn == nullptr) return;
-  s->chain_turn->sessions -= 1;
-  if (s->chain_wide) s->chain_turn->wide -= 1;
-  s->chain_turn = nullptr;
+void leave_order(Session *s) {
+  nv::out_of_order(s);
+  if (s->order != nullptr) s->order->sessions -= 1;
+  s->order = nullptr;
+  if (s->launched) (void)hipEventDestroy(s->launched);
+  if (s->mark) (void)hipEventDestroy(s->mark);
 }
 
 bool layer_has_weights(const NervaHipHfDecodeChainLayer &l) {
@@ -307,12 +294,12 @@ bool layer_has_weights(const NervaHipHfDecodeChainLayer &l) {
 void nv::destroy_session(Session *s) {
   if (s == nullptr) return;
   if (s->stream) (void)hipStreamSynchronize(s->stream);
-  leave_chains(s);
+  leave_order(s);
   for (int i = 0; i < Session::kGraphs; ++i) {
     if (s->exec[i]) (void)hipGraphExecDestroy(s->exec[i]);
     if (s->graph[i]) (void)hipGraphDestroy(s->graph[i]);
   }
-  for (int i = 0; i < 4; ++i) {
+  for (int i = 0; i < 2; ++i) {
     if (s->together[i]) (void)hipGraphExecDestroy(s->together[i]);
     if (s->together_graph[i]) (void)hipGraphDestroy(s->together_graph[i]);
   }
@@ -544,17 +531,15 @@ hipError_t enqueue_step(Session *s, StepMode mode, StepProfiler *prof, int only 
   return hipSuccess;
 }
 
-// The same with its layers in one launch; `turn`: when it is the session's turn.
-hipError_t enqueue_chain_step(Session *s, bool turn) {
+// The same with its layers in one launch.
+hipError_t enqueue_chain_step(Session *s) {
   const int spins = tuning(kTuneAttnMergeSpinLimit);
   ChainLaunch c{};
   c.model = s->chain_model_dev;
   c.trace = s->trace_buf;
   c.spin_limit = spins > 0 ? static_cast<uint32_t>(spins) : kChainSpinLimit;
   c.withhold = static_cast<uint32_t>(std::max(tuning(kTuneStepChainWithhold), 0));
-  hipError_t err = turn ? launch_chain_turn(s->chain_turn->word, s->chain_number, false, s->stream) : hipSuccess;
-  if (err == hipSuccess) err = (s->chain_wide ? launch_step_wide : launch_step_chain)(s->dtype, s->head_dim, s->chain_model, c, s->stream);
-  if (err == hipSuccess && turn) err = launch_chain_turn(s->chain_turn->word, s->chain_number, true, s->stream);
+  hipError_t err = (s->chain_wide ? launch_step_wide : launch_step_chain)(s->dtype, s->head_dim, s->chain_model, c, s->stream);
   GemvParams p = head_launch(s, s->x);
   const auto slot = [](uint64_t bytes) { return (bytes + 255u) & ~uint64_t{255}; };
   char *trace = s->trace_buf;
@@ -570,7 +555,7 @@ hipError_t enqueue_chain_step(Session *s, bool turn) {
   return err == hipSuccess ? head_sample(s, p.sample, head_blocks) : err;
 }
 hipError_t enqueue_graph_step(Session *s, int which) {
-  return which >= 3 ? enqueue_chain_step(s, which >= 5) : enqueue_step(s, which == 1 ? kPromptStep : kDecodeStep, nullptr);
+  return which >= 3 ? enqueue_chain_step(s) : enqueue_step(s, which == 1 ? kPromptStep : kDecodeStep, nullptr);
 }
 
 // Steps are launched kernel by kernel instead of as graph replays when NERVA_HIP_EAGER_STEPS=1 is
@@ -599,10 +584,10 @@ bool eager_steps() {
   return eager;
 }
 
-// Kernel launches of one step (which = 0: decode step, 1: prompt step, 3 to 6: a decode step as a chain).
+// Kernel launches of one step (which = 0: decode step, 1: prompt step, 3 and 4: a decode step as a chain).
 uint64_t step_launches(const Session *s, int which) {
   if (s->stack != nullptr) return stack_step_launches(s);
-  if (which >= 3) return (s->sampler.mode == kSamplerGreedy ? 3 : 4) + (which >= 5 ? 2 : 0);
+  if (which >= 3) return s->sampler.mode == kSamplerGreedy ? 3 : 4;
   // embed + (lm head + greedy finish | lm head + two sampler launches | cursor advance)
   const uint64_t fixed = which == 1 ? 2 : (s->sampler.mode == kSamplerGreedy ? 3 : 4);
   return fixed + 5ull * s->layers;
@@ -614,16 +599,19 @@ hipError_t launch_step(Session *s, int which, NervaHipHfDecodeSequenceResult *ou
 // Index of the captured decode step for the active sampler, at a position.
 int decode_graph(const Session *s, uint32_t position) {
   const bool greedy = s->sampler.mode == kSamplerGreedy;
-  if (position < s->chain_context) {
-    const nv::ChainTurn *t = s->chain_turn;
-    const bool turn = t != nullptr && t->wide != 0 && t->sessions > 1;
-    return (greedy ? 3 : 4) + (turn ? 2 : 0);
-  }
+  if (position < s->chain_context) return greedy ? 3 : 4;
   return greedy ? 0 : 2;
+}
+// Whom a step's launches must not meet.
+nv::Place step_place(const Session *s, int which) {
+  if (which < 3) return nv::Place::kAny;
+  return s->chain_wide ? nv::Place::kAlone : nv::Place::kBeside;
 }
 
 // `steps` steps of kind `which`, captured.
 hipError_t capture_steps(Session *s, int which, uint32_t steps, hipGraph_t *graph, hipGraphExec_t *exec) {
+  // (what another session records on this one's stream to come behind it would be captured too)
+  const std::unique_lock<std::mutex> quiet = s->order != nullptr ? std::unique_lock<std::mutex>(s->order->mutex) : std::unique_lock<std::mutex>();
   hipError_t err = hipStreamBeginCapture(s->stream, hipStreamCaptureModeThreadLocal);
   if (err != hipSuccess) return err;
   // (a trace that is armed is the next step's: its copies would stay in the graph, and write to the caller's buffer ever after)
@@ -640,7 +628,7 @@ hipError_t capture_steps(Session *s, int which, uint32_t steps, hipGraph_t *grap
   }
   return err;
 }
-// graph index 0 / 2: decode step (greedy finish / sampler), 1: prompt step, 3 / 4: decode step as a chain, 5 / 6: behind its turn
+// graph index 0 / 2: decode step (greedy finish / sampler), 1: prompt step, 3 / 4: decode step as a chain
 hipError_t ensure_graph(Session *s, int which, NervaHipHfDecodeSequenceResult *out) {
   if (eager_steps()) return hipSuccess;
   if (s->exec[which] != nullptr) {
@@ -706,30 +694,34 @@ hipError_t launch_steps_again(Session *s, uint32_t end, uint32_t count, NervaHip
   return err;
 }
 
+hipError_t enqueue_in_order(Session *s, int which) {
+  const nv::InOrder turn(s, step_place(s, which));
+  return turn.error == hipSuccess ? enqueue_graph_step(s, which) : turn.error;
+}
 hipError_t launch_step(Session *s, int which, NervaHipHfDecodeSequenceResult *out) {
   if (s->trace_buf != nullptr && which != 1) {
     // armed by nerva_hip_session_trace_next_step: this one step runs kernel by kernel with copies
     s->trace_used = 0;
-    hipError_t err = enqueue_graph_step(s, which);
+    hipError_t err = enqueue_in_order(s, which);
     if (err == hipSuccess) out->kernel_launches += step_launches(s, which);
     // (one that gave up is traced once more, now: its replays would be the caller's steps without a trace)
     while (err == hipSuccess && which >= 3) {
       err = hipStreamSynchronize(s->stream);
       if (err != hipSuccess || take_given_up(s) == 0) break;
-      err = enqueue_graph_step(s, which);
+      err = enqueue_in_order(s, which);
       if (err == hipSuccess) out->kernel_launches += step_launches(s, which);
     }
     s->trace_buf = nullptr;
     return err;
   }
   if (eager_steps()) {
-    hipError_t err = enqueue_graph_step(s, which);
+    hipError_t err = enqueue_in_order(s, which);
     if (err == hipSuccess)
       out->kernel_launches += step_launches(s, which);
     return err;
   }
-  // (another session may have come or gone since the call made its graphs)
-  hipError_t err = s->exec[which] == nullptr ? ensure_graph(s, which, out) : hipSuccess;
+  const nv::InOrder turn(s, step_place(s, which));
+  hipError_t err = turn.error;
   if (err == hipSuccess) err = hipGraphLaunch(s->exec[which], s->stream);
   if (err == hipSuccess) {
     out->graph_replays += 1;
@@ -747,7 +739,9 @@ hipError_t launch_steps(Session *s, uint32_t position, uint32_t steps, uint32_t 
   if (which < 3 || steps < kMost || s->trace_buf != nullptr || s->together[which - 3] == nullptr || position + kMost > s->chain_context)
     return launch_step(s, which, out);
   *taken = kMost;
-  hipError_t err = hipGraphLaunch(s->together[which - 3], s->stream);
+  const nv::InOrder turn(s, step_place(s, which));
+  hipError_t err = turn.error;
+  if (err == hipSuccess) err = hipGraphLaunch(s->together[which - 3], s->stream);
   if (err == hipSuccess) {
     out->graph_replays += kMost;
     out->graph_launches += 1;
@@ -820,6 +814,7 @@ bool slots_faulted(const Slot *slots, uint32_t count) {
 hipError_t bring_tokens(Session *s, SequenceParams p, const uint32_t *tokens, uint32_t first, uint32_t count, NervaHipHfDecodeSequenceResult *out) {
   const hipError_t err = hipStreamSynchronize(s->stream);
   if (err != hipSuccess) return err;
+  nv::out_of_order(s);
   if (p.fresh != 0 && s->given_up != nullptr) *s->given_up = 0;
   memcpy(s->host_prompt + first, tokens, static_cast<uint64_t>(count) * sizeof(uint32_t));
   p.from = s->host_prompt;
@@ -1530,7 +1525,7 @@ hipError_t setup_state(Session *s, int32_t *failure_stage, bool with_weights) {
   if (err == hipSuccess) err = hipMemsetAsync(s->arena + off_attn_tagged, 0, attn_step_workspace_bytes(s->heads), s->stream);
   if (err == hipSuccess) err = hipMemsetAsync(s->arena + off_sample_ws, 0, sample_workspace_bytes(), s->stream);
   if (err == hipSuccess && chain) err = hipMemsetAsync(s->chain_model.words, 0, s->chain_word_bytes, s->stream);
-  if (err == hipSuccess && chain) err = join_chains(s);
+  if (err == hipSuccess && chain) err = join_order(s);
   if (err == hipSuccess) err = hipMemsetAsync(s->arena + off_pattn_ws, 0, pB * pattn_ws_stride, s->stream);
   if (err == hipSuccess && L > 0) err = hipMemsetAsync(s->arena + off_attn_trace, 0, L * 32 * 8, s->stream);
   if (err == hipSuccess) err = hipMemsetAsync(s->arena + off_kc, 0, 2 * ((kv_half + 255) & ~uint64_t{255}), s->stream);
@@ -2304,6 +2299,7 @@ int nerva_hip_hf_decode_sequence_batch_advance_one(const NervaHipHfDecodeSequenc
         out->d2h_bytes += sizeof(Slot);
         out->sync_calls += 1;
       }
+      if (err == hipSuccess) nv::out_of_order(q);
     }
   }
   out->hot_path_allocations = allocation_count() - allocs_before;
@@ -2481,6 +2477,7 @@ int nerva_hip_session_extend(const NervaHipSessionExtendRequest *request, NervaH
     }
   }
   if (err == hipSuccess && !idle) err = hipStreamSynchronize(s->stream);
+  if (err == hipSuccess) nv::out_of_order(s);
   out->sync_calls += 1;
   const bool fault = s->given_up != nullptr && (*s->given_up & kHostFault) != 0;
   if (err != hipSuccess || fault) {
@@ -2531,8 +2528,10 @@ int nerva_hip_hf_decode_sequence_session_advance(const NervaHipHfDecodeSequenceS
   if (run_count != 0) err = ensure_graphs(s, s->cursor, run_count, out);
   const uint64_t allocs_before = allocation_count();
   if (err == hipSuccess && run_count != 0) err = hipEventRecord(s->ev0, s->stream);
-  for (uint32_t step = 0, taken = 1; err == hipSuccess && step < run_count; step += taken) {
-    err = launch_steps(s, s->cursor + step, s->has_eos != 0 ? 1 : run_count - step, &taken, out);
+  nv::RunAhead ahead(s);
+  for (uint32_t step = 0, taken = 0; err == hipSuccess && step < run_count; step += taken) {
+    if (s->has_eos == 0) err = ahead.room(taken);
+    if (err == hipSuccess) err = launch_steps(s, s->cursor + step, s->has_eos != 0 ? 1 : run_count - step, &taken, out);
     // With a stop token the host looks at each token so that it can stop launching
     // (session_api_lifecycle.inc.cu:1206-1234); without one the loop never syncs.
     if (err == hipSuccess && s->has_eos != 0) {
@@ -2566,6 +2565,7 @@ int nerva_hip_hf_decode_sequence_session_advance(const NervaHipHfDecodeSequenceS
     again = take_given_up(s);
     if (again == 0) break;
   }
+  if (err == hipSuccess) nv::out_of_order(s);
   out->hot_path_allocations = allocation_count() - allocs_before;
   if (err == hipSuccess && run_count != 0) {
     float ms = 0.0f;
@@ -2627,7 +2627,11 @@ int nerva_hip_hf_decode_sequence_session_run(const NervaHipHfDecodeSequenceSessi
   if (err == hipSuccess) err = ensure_graphs(s, 0, context_steps, out);
   const uint64_t allocs_before = allocation_count();
   if (err == hipSuccess) err = hipEventRecord(s->ev0, s->stream);
-  for (uint32_t step = 0, taken = 1; err == hipSuccess && step < context_steps; step += taken) err = launch_steps(s, step, context_steps - step, &taken, out);
+  nv::RunAhead ahead(s);
+  for (uint32_t step = 0, taken = 0; err == hipSuccess && step < context_steps; step += taken) {
+    err = ahead.room(taken);
+    if (err == hipSuccess) err = launch_steps(s, step, context_steps - step, &taken, out);
+  }
   const uint64_t slots_bytes = static_cast<uint64_t>(context_steps) * sizeof(Slot);
   for (uint32_t again = 0; err == hipSuccess;) {
     err = launch_steps_again(s, context_steps, again, out);
@@ -2643,6 +2647,7 @@ int nerva_hip_hf_decode_sequence_session_run(const NervaHipHfDecodeSequenceSessi
     again = take_given_up(s);
     if (again == 0) break;
   }
+  if (err == hipSuccess) nv::out_of_order(s);
   out->hot_path_allocations = allocation_count() - allocs_before;
   if (err == hipSuccess) {
     float ms = 0.0f;

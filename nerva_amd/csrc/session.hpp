@@ -1,6 +1,7 @@
 // A decode session's object and what the translation units that implement its steps share of it.
 #pragma once
 
+#include <algorithm>
 #include <atomic>
 #include <memory>
 #include <mutex>
@@ -68,11 +69,13 @@ struct BatchTable {
   SamplerParams sample[kGemmMaxTokens];
 };
 
-// Of a device: the word that says whose turn it is, and who is there (join_chains).
-struct ChainTurn {
-  uint32_t *word = nullptr;          // device memory
-  uint32_t numbers = 0;
-  std::atomic<uint32_t> sessions{0}, wide{0};   // whose steps run as one launch; of those, with the whole device to themselves
+// Launches whose workgroups wait for each other find a place for all of them or wait in vain, and two at once may each hold what the other one needs.
+// Of a device's sessions: who has such launches that may still be under way (InOrder).
+struct LaunchOrder {
+  std::mutex mutex;
+  NervaHipHfDecodeSequenceSession *alone = nullptr;             // the last one that needs the device to itself,
+  std::vector<NervaHipHfDecodeSequenceSession *> beside;        // and those behind it that fit beside each other
+  std::atomic<uint32_t> sessions{0};
 };
 
 struct StackModel;   // layer_stack.hpp
@@ -115,16 +118,15 @@ struct NervaHipHfDecodeSequenceSession : nv::RowScratch {
   uint32_t *host_state = nullptr;    // 64 words
   // captured steps: 0 decode step with the greedy finish, 1 prompt step, 2 decode step with the
   // temperature / top-k / top-p sampler (its parameters live in device memory, so one capture
-  // serves every such configuration), 3 and 4 the two decode steps with their layers in one launch, 5 and 6 the
-  // same where the device has other sessions whose launches they must not meet (ChainTurn)
-  static constexpr int kGraphs = 7;
+  // serves every such configuration), 3 and 4 the two decode steps with their layers in one launch
+  static constexpr int kGraphs = 5;
   hipGraph_t graph[kGraphs] = {};
   hipGraphExec_t exec[kGraphs] = {};
   uint64_t graph_nodes[kGraphs] = {};
-  // Of graphs 3 to 6, kStepsTogether steps of them in one graph (ensure_together)
+  // Of graphs 3 and 4, kStepsTogether steps of them in one graph (ensure_together)
   static constexpr uint32_t kStepsTogether = 6;   // (calls of 8 to 32 steps: the fewest launches with what is left over, which goes out singly)
-  hipGraph_t together_graph[4] = {};
-  hipGraphExec_t together[4] = {};
+  hipGraph_t together_graph[2] = {};
+  hipGraphExec_t together[2] = {};
   uint64_t chain_steps = 0;          // steps that went out as chains
   // positions below chain_context step with their layers in one launch (step_chain.cuh); 0: never
   uint32_t chain_context = 0;
@@ -132,8 +134,10 @@ struct NervaHipHfDecodeSequenceSession : nv::RowScratch {
   nv::ChainModel *chain_model_dev = nullptr;
   uint64_t chain_word_bytes = 0;
   bool chain_wide = false;           // ... of the kind that has the whole device to itself (step_wide.hip)
-  nv::ChainTurn *chain_turn = nullptr;   // the device's, where this session is counted
-  uint32_t chain_number = 0;         // ... under this number
+  nv::LaunchOrder *order = nullptr;  // the device's, where this session is counted
+  hipEvent_t launched = nullptr;     // recorded by whoever has to come behind this session's launches
+  uint32_t steps_ahead = 0;          // steps that a call sends ahead of those it has seen the end of, where others may be waiting (RunAhead)
+  hipEvent_t mark = nullptr;         // ... and the event that it looks at
   uint32_t *given_up = nullptr;      // host_state[0]: steps that gave up since the host looked (step_given_up writes it)
   // prompt blocks: up to prefill_pass_tokens prompt tokens per pass through the layers (weights streamed
   // once per pass on the matrix cores), in a long prompt prefill_long_tokens; false = one prompt step per token
@@ -233,6 +237,76 @@ class PassTurn {
   Session *s;
   RowScratch own;
   std::unique_lock<std::mutex> turn;
+};
+
+// While this lives the session enqueues a launch whose workgroups wait for each other, behind those of other sessions that it must not meet. The streams keep that
+// order: nobody waits on the host or on the device in front of what is to be waited for, and a session that has no other's launches under way beside it enqueues no more than
+// the launch. (Turns that a launch of one wave took by polling a word stood in front of what would have given the word back where two sessions share a hardware
+// queue; and they took two launches more a step beside any other session, idle or not: 69.4 -> 72.3 us at 512 wide,
+// 845 -> 848 at 4096.)
+enum class Place { kAny, kBeside, kAlone };   // meets anybody; nobody but its like (narrow models' steps); nobody
+class InOrder {
+ public:
+  InOrder(Session *session, Place place) {
+    LaunchOrder *const order = session->order;
+    if (order == nullptr || place == Place::kAny) return;
+    turn = std::unique_lock<std::mutex>(order->mutex);
+    std::vector<Session *> &beside = order->beside;
+    const auto at = std::find(beside.begin(), beside.end(), session);
+    if (place == Place::kBeside && at != beside.end()) return;   // (behind `alone` already)
+    if (order->alone != nullptr && order->alone != session) error = follow(session, order->alone);
+    if (place == Place::kBeside) {
+      if (error == hipSuccess) beside.push_back(session);
+      return;
+    }
+    for (Session *other : beside)
+      if (error == hipSuccess && other != session) error = follow(session, other);
+    if (error != hipSuccess) return;
+    beside.clear();
+    order->alone = session;
+  }
+  InOrder(const InOrder &) = delete;
+  InOrder &operator=(const InOrder &) = delete;
+  hipError_t error = hipSuccess;
+
+ private:
+  static hipError_t follow(Session *session, Session *other) {
+    hipError_t err = hipEventRecord(other->launched, other->stream);
+    if (err == hipSuccess) err = hipStreamWaitEvent(session->stream, other->launched, 0);
+    if (err == hipSuccess) return err;
+    (void)hipGetLastError();
+    return hipStreamSynchronize(other->stream);
+  }
+  std::unique_lock<std::mutex> turn;
+};
+// A session's stream is idle: there is nothing left to come behind.
+inline void out_of_order(Session *session) {
+  LaunchOrder *const order = session->order;
+  if (order == nullptr) return;
+  const std::lock_guard<std::mutex> lock(order->mutex);
+  if (order->alone == session) order->alone = nullptr;
+  order->beside.erase(std::remove(order->beside.begin(), order->beside.end(), session), order->beside.end());
+}
+// The steps that a call enqueues without looking at them: where a device has other sessions, no more than twice steps_ahead (some 2 ms each) before the call waits for
+// the older ones, so that whoever else steps comes in between.
+class RunAhead {
+ public:
+  explicit RunAhead(Session *session) : s(session) {}
+  // Ahead of the next steps; `sent`: with those that went out since it was last asked.
+  hipError_t room(uint32_t sent) {
+    unseen += sent;
+    if (unseen < s->steps_ahead || s->order == nullptr || s->order->sessions.load(std::memory_order_relaxed) < 2) return hipSuccess;
+    hipError_t err = marked ? hipEventSynchronize(s->mark) : hipSuccess;
+    if (err == hipSuccess) err = hipEventRecord(s->mark, s->stream);
+    marked = true;
+    unseen = 0;
+    return err;
+  }
+
+ private:
+  Session *s;
+  uint32_t unseen = 0;
+  bool marked = false;
 };
 
 // Waits for what an event was recorded behind. One whose stream is gone has nothing left to wait for (a session ends its stream's work before its stream), which the runtime reports as

@@ -86,9 +86,5 @@ bool wide_takes(uint32_t dtype, uint32_t layers, uint32_t hidden, uint32_t heads
 bool wide_resident(uint32_t dtype, uint32_t heads, uint32_t kv_heads, uint32_t head_dim);
 void wide_stages(const ChainModel &model, uint32_t head_dim, const LayerDev &layer, WideStage (&stage)[4]);
 hipError_t launch_step_wide(uint32_t dtype, uint32_t head_dim, const ChainModel &model, const ChainLaunch &p, hipStream_t stream);
-// Where a device has several sessions with such launches: waits for session `of`'s turn, or ends it. `turn`: the device's word.
-// Tries, 64 x 16 cycles and a look each: some 100 ms, many times what a launch lasts that nobody disturbs.
-constexpr uint32_t kChainTurnLimit = 1u << 17;
-hipError_t launch_chain_turn(uint32_t *turn, uint32_t of, bool over, hipStream_t stream);
 
 }  // namespace nv

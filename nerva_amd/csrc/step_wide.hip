@@ -28,7 +28,7 @@
 //
 // The loaders take part in no barrier, so the others' is a counter in LDS (Meet). Everything else - the places of words, who overwrites what when, waits
 // that run out, steps that are void and taken again - is as in step_chain.hip. A workgroup has a CU to itself here, all 256 wait for each other: two such launches that started
-// at once could each hold half of the chip until both give up. So where a device has other sessions with launches of this kind, a step takes its turn (launch_chain_turn).
+// at once could each hold half of the chip until both give up. So a step comes behind what other sessions of the device have under way of that sort (InOrder in session.hpp).
 #include <float.h>
 
 #include "step_parts.cuh"
@@ -548,17 +548,6 @@ __global__ __launch_bounds__(kThreads + kLoaders *kWave, 1) void step_wide_kerne
   }
 }
 
-// A session's turn on its device, ahead of its launch and, `over`, behind it: `turn` is 0 or names whose it is. Whoever does not get it in time goes on without: the launch
-// behind it gives up by itself where it is in somebody's way.
-__global__ __launch_bounds__(kWave) void chain_turn_kernel(uint32_t *turn, uint32_t of, bool over) {
-  if (threadIdx.x != 0) return;
-  for (uint32_t i = 0; i < (over ? 1u : kChainTurnLimit); ++i) {
-    uint32_t held = over ? of : 0u;
-    if (__hip_atomic_compare_exchange_strong(turn, &held, over ? 0u : of, __ATOMIC_RELAXED, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)) return;
-    __builtin_amdgcn_s_sleep(16);
-  }
-}
-
 using Kernel = void (*)(ChainLaunch);
 struct Variant {
   Kernel kernel;
@@ -661,12 +650,6 @@ void wide_stages(const ChainModel &m, uint32_t head_dim, const LayerDev &w, Wide
       }
     }
   }
-}
-
-hipError_t launch_chain_turn(uint32_t *turn, uint32_t of, bool over, hipStream_t stream) {
-  if (turn == nullptr || of == 0) return hipErrorInvalidValue;
-  hipLaunchKernelGGL(chain_turn_kernel, dim3(1), dim3(kWave), 0, stream, turn, of, over);
-  return hipGetLastError();
 }
 
 hipError_t launch_step_wide(uint32_t dtype, uint32_t head_dim, const ChainModel &m, const ChainLaunch &p, hipStream_t stream) {

@@ -1,9 +1,11 @@
 // A stand-in for the HIP runtime on machines without a device, for tests of the host code: memory is the host's, copies are copies, launches only
 // count (by the kernel's name), graphs hold the number of launches that were captured. Loaded with its symbols visible to all (RTLD_GLOBAL) ahead of
-// libnerva_hip.so, whose calls then end here. The double_* functions set what it answers and read what it saw.
+// libnerva_hip.so, whose calls then end here. The double_* functions set what it answers and read what it saw; double_log is what streams were given, one
+// line each: "kernel 1 name", "graph 1 nodes", "record 1 event", "wait 1 event", "sync 1", "sync event", streams and events numbered as they were created.
 #define __HIP_PLATFORM_AMD__ 1
 #include <hip/hip_runtime_api.h>
 
+#include <atomic>
 #include <cstdlib>
 #include <cstring>
 #include <map>
@@ -15,6 +17,15 @@ long g_copies = 0, g_fail_copy = -1;
 long g_captured = -1;   // launches since the capture began, or -1
 std::map<const void *, std::string> g_names;
 std::map<std::string, long> g_launches;
+std::string g_log;
+std::map<const void *, long> g_numbers;   // of streams and events
+long g_streams = 0, g_events = 0;
+std::atomic<long> g_held{0}, g_waits{0};
+
+void log(const char *what, const void *first, const std::string &rest = "") {
+  if (g_captured < 0) g_log += std::string(what) + " " + std::to_string(g_numbers[first]) + (rest.empty() ? "" : " " + rest) + "\n";
+}
+std::string number(const void *of) { return std::to_string(g_numbers[of]); }
 
 struct Graph {
   long nodes;
@@ -37,6 +48,11 @@ void double_fail_copy(long number) {
   g_fail_copy = number;
 }
 long double_copies() { return g_copies; }
+// Whoever waits for that stream waits until another one is named (0: none); whether somebody does.
+void double_hold(long stream) { g_held = stream; }
+long double_waits() { return g_waits; }
+void double_clear_log() { g_log.clear(); }
+const char *double_log() { return g_log.c_str(); }
 // Launches of kernels whose names hold `part`.
 long double_launches(const char *part) {
   long n = 0;
@@ -54,8 +70,9 @@ void __hipRegisterFunction(void **, const void *host, char *, const char *name, 
 void __hipRegisterVar(void **, void *, char *, char *, int, size_t, int, int) {}
 hipError_t __hipPushCallConfiguration(dim3, dim3, size_t, hipStream_t) { return hipSuccess; }
 hipError_t __hipPopCallConfiguration(dim3 *, dim3 *, size_t *, hipStream_t *) { return hipSuccess; }
-hipError_t hipLaunchKernel(const void *kernel, dim3, dim3, void **, size_t, hipStream_t) {
+hipError_t hipLaunchKernel(const void *kernel, dim3, dim3, void **, size_t, hipStream_t stream) {
   g_launches[g_names[kernel]] += 1;
+  log("kernel", stream, g_names[kernel]);
   if (g_captured >= 0) g_captured += 1;
   return hipSuccess;
 }
@@ -128,16 +145,26 @@ hipError_t hipGetSymbolAddress(void **ptr, const void *) {
 
 hipError_t hipStreamCreateWithFlags(hipStream_t *stream, unsigned) {
   *stream = reinterpret_cast<hipStream_t>(malloc(1));
+  g_numbers[*stream] = ++g_streams;
   return hipSuccess;
 }
 hipError_t hipStreamDestroy(hipStream_t stream) {
   free(stream);
   return hipSuccess;
 }
-hipError_t hipStreamSynchronize(hipStream_t) { return hipSuccess; }
-hipError_t hipStreamWaitEvent(hipStream_t, hipEvent_t, unsigned) { return hipSuccess; }
+hipError_t hipStreamSynchronize(hipStream_t stream) {
+  log("sync", stream);
+  while (g_held == g_numbers[stream]) g_waits = 1;
+  g_waits = 0;
+  return hipSuccess;
+}
+hipError_t hipStreamWaitEvent(hipStream_t stream, hipEvent_t event, unsigned) {
+  log("wait", stream, number(event));
+  return hipSuccess;
+}
 hipError_t hipEventCreateWithFlags(hipEvent_t *event, unsigned) {
   *event = reinterpret_cast<hipEvent_t>(malloc(1));
+  g_numbers[*event] = ++g_events;
   return hipSuccess;
 }
 hipError_t hipEventCreate(hipEvent_t *event) { return hipEventCreateWithFlags(event, 0); }
@@ -145,8 +172,14 @@ hipError_t hipEventDestroy(hipEvent_t event) {
   free(event);
   return hipSuccess;
 }
-hipError_t hipEventRecord(hipEvent_t, hipStream_t) { return hipSuccess; }
-hipError_t hipEventSynchronize(hipEvent_t) { return hipSuccess; }
+hipError_t hipEventRecord(hipEvent_t event, hipStream_t stream) {
+  log("record", stream, number(event));
+  return hipSuccess;
+}
+hipError_t hipEventSynchronize(hipEvent_t event) {
+  log("sync event", event);
+  return hipSuccess;
+}
 hipError_t hipEventElapsedTime(float *ms, hipEvent_t, hipEvent_t) {
   *ms = 1.0f;
   return hipSuccess;
@@ -169,7 +202,10 @@ hipError_t hipGraphInstantiate(hipGraphExec_t *exec, hipGraph_t graph, hipGraphN
   *exec = reinterpret_cast<hipGraphExec_t>(new Graph(*reinterpret_cast<Graph *>(graph)));
   return hipSuccess;
 }
-hipError_t hipGraphLaunch(hipGraphExec_t, hipStream_t) { return hipSuccess; }
+hipError_t hipGraphLaunch(hipGraphExec_t exec, hipStream_t stream) {
+  log("graph", stream, std::to_string(reinterpret_cast<Graph *>(exec)->nodes));
+  return hipSuccess;
+}
 hipError_t hipGraphDestroy(hipGraph_t graph) {
   delete reinterpret_cast<Graph *>(graph);
   return hipSuccess;

@@ -368,7 +368,7 @@ def test_norms_of_rows_at_the_ends_of_f32(scale, eps):
 
 @pytest.mark.parametrize("wide", [False, True])
 def test_steps_that_go_out_together_give_what_single_ones_give(wide):
-    """Greedy and sampled, one session and a second beside it that makes steps take turns, past the context where steps become launches: a call of 100 steps against
+    """Greedy and sampled, one session and a second beside it, past the context where steps become launches: a call of 100 steps against
     calls of one."""
     shape = (BF16, 1024, 16, 8, 128, 2816, 301, 4, 1e6, True, False) if wide else SHAPES[0]
     dtype, hidden, heads, kv, hd, inter, vocab, layers, theta, qk_norm, bias = shape

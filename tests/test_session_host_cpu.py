@@ -11,9 +11,12 @@ ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
 SOURCE = os.path.join(ROOT, "tests", "host", "hip_double.cpp")
 
 PRELUDE = """
-import ctypes, sys
+import ctypes, sys, threading, time
 double = ctypes.CDLL(sys.argv[1], mode=ctypes.RTLD_GLOBAL)
 double.double_launches.restype = double.double_copies.restype = ctypes.c_long
+double.double_waits.restype = ctypes.c_long
+double.double_hold.argtypes = [ctypes.c_long]
+double.double_log.restype = ctypes.c_char_p
 double.double_fail_copy.argtypes = [ctypes.c_long]
 sys.path[:0] = [%r, %r]
 import numpy as np
@@ -27,6 +30,21 @@ def model(shape=NARROW):
 def step(session):
     assert session.start(np.arange(5, dtype=np.uint32))[0] == 0
     return session.advance(2)[1]
+
+def log():
+    return double.double_log().decode().splitlines()
+
+# Makes the call in a thread, up to where it waits for that stream; what is returned lets it end.
+def while_held(stream, call):
+    double.double_hold(stream)
+    thread = threading.Thread(target=call)
+    thread.start()
+    while not double.double_waits():
+        time.sleep(0.001)
+    def over():
+        double.double_hold(0)
+        thread.join()
+    return over
 """ % (ROOT, os.path.join(ROOT, "tests"))
 
 
@@ -124,33 +142,72 @@ for kv, context in ((2, 8192), (8, 32768)):
 """)
 
 
-def test_steps_take_turns_where_a_device_has_several_such_sessions(double):
-    """With a session whose launches need the whole device there, every session with such a launch, of a narrow model too, steps between two launches more; no longer when it
-    is alone, and never where all are narrow."""
+def test_steps_come_behind_those_that_they_must_not_meet(double):
+    """A launch that needs the whole device comes behind those of other sessions that are under way, and they behind it: an event of that stream, waited for ahead of the launch. Narrow models' steps
+    meet each other, sessions that have nothing under way nobody; and captured steps are the same whoever else is there."""
     run(double, """
 double.double_device(256, 2)
 wide = dict(dtype=BF16, hidden=1024, heads=8, kv_heads=2, head_dim=128, intermediate=4096, vocab=64, layers=4, rms_eps=1e-6, rope_theta=1e4)
 a = N.DecodeSession.create(model(), 64)
 b = a.fork_shared_weights()
-assert step(a).graph_nodes == step(b).graph_nodes == 3
 c = N.DecodeSession.create_synthetic(wide, 64)
-before = double.double_launches(b"chain_turn_kernel")
-assert [step(s).graph_nodes for s in (a, b, c)] == [5, 5, 5]
-assert double.double_launches(b"chain_turn_kernel") - before == 6      # (each was captured once)
-d = N.DecodeSession.create_synthetic(dict(wide, layers=2), 64)         # (steps in launches: no matter)
-a.destroy()
-assert step(c).graph_nodes == 5 and step(d).graph_nodes == 3 + 5 * 2
-b.destroy()
-assert step(c).graph_nodes == 3
-e = N.DecodeSession.create_synthetic(wide, 64)
-assert step(c).graph_nodes == step(e).graph_nodes == 5
-c.destroy()
-a = N.DecodeSession.create(model(), 64)
-assert step(e).graph_nodes == step(a).graph_nodes == 5
-e.destroy()
-assert step(a).graph_nodes == 3
-for s in (a, d):
+d = c.fork_shared_weights()
+sessions = (a, b, c, d)
+stream = {}
+for s in sessions:
+    double.double_clear_log()
+    assert step(s).graph_nodes == 3
+    assert not any(line.startswith("wait") for line in log()), log()
+    stream[s], = (int(line.split()[1]) for line in log() if line.startswith("graph"))
+for held, meets in ((a, (b,)), (c, ())):
+    for other in sessions:
+        if other is held:
+            continue
+        assert held.start(np.arange(5, dtype=np.uint32))[0] == other.start(np.arange(5, dtype=np.uint32))[0] == 0
+        under_way = while_held(stream[held], lambda: held.advance(2))
+        double.double_clear_log()
+        assert other.advance(2)[1].graph_nodes == 3
+        lines = log()
+        launch = lines.index("graph %d 3" % stream[other])
+        waits = [line.split()[2] for line in lines[:launch] if line.startswith("wait %d " % stream[other])]
+        records = [line.split()[2] for line in lines[:launch] if line.startswith("record %d " % stream[held])]
+        assert waits == records and len(waits) == (0 if other in meets else 1), (lines, stream)
+        under_way()
+        double.double_clear_log()
+        other.start(np.arange(5, dtype=np.uint32))
+        other.advance(2)
+        assert not any(line.startswith("wait") for line in log())
+for s in (b, a, d, c):
     s.destroy()
+""")
+
+
+def test_long_calls_beside_other_sessions_do_not_run_far_ahead(double):
+    """Steps that nobody looks at: some 4 ms of them are under way at the most where a device has other sessions, so that these come in between, and any number where it has not."""
+    run(double, """
+def looks(s):
+    assert s.start(np.arange(5, dtype=np.uint32))[0] == 0
+    double.double_clear_log()
+    assert s.advance(201)[0] == -1                          # (the stand-in publishes no tokens)
+    sent = done = most = 0
+    at = {}
+    for words in (line.split() for line in log()):
+        if words[0] == "graph":
+            sent += int(words[2]) // 3
+            most = max(most, sent - done)
+        elif words[0] == "record":
+            at[words[2]] = sent
+        elif words[:2] == ["sync", "event"]:
+            done = at[words[2]]
+    return most, sum(line.startswith("sync event") for line in log())
+s = N.DecodeSession.create(model(), 300)
+assert looks(s) == (200, 0)
+other = s.fork_shared_weights()
+most, times = looks(s)
+assert times >= 2 and 50 <= most <= 2 * 56, (most, times)
+other.destroy()
+assert looks(s) == (200, 0)
+s.destroy()
 """)
 
 
@@ -223,8 +280,8 @@ assert go(s, 23, eos=63)[1:] == (23, 69, 0)
 context = next(p for p in range(1024, 4200, 1024) if go(s, 1, p)[2] != 3)
 assert go(s, 24, context - 15) == (24, 2 + 12, 15 * 3 + 9 * (3 + 5 * 4), 0)
 wide = dict(dtype=BF16, hidden=1024, heads=8, kv_heads=2, head_dim=128, intermediate=4096, vocab=64, layers=4, rms_eps=1e-6, rope_theta=1e4)
-c = N.DecodeSession.create_synthetic(wide, 64)            # its turn now: graphs of their own for that
-assert go(s, 12) == (12, 2, 60, 1)
+c = N.DecodeSession.create_synthetic(wide, 64)            # (nothing of it under way)
+assert go(s, 12) == (12, 2, 36, 0)
 c.destroy()
 assert go(s, 12) == (12, 2, 36, 0)
 s.destroy()
