@@ -254,7 +254,7 @@ bool layer_supported(const NervaHipHfDecodeChainLayer &l) {
   return true;
 }
 
-// Counts a session among those of its device that come in order (InOrder).
+// Counts a session of decoder layers among those of its device that come in order (InOrder).
 hipError_t join_order(Session *s) {
   struct Orders {
     std::mutex mutex;
@@ -602,10 +602,9 @@ int decode_graph(const Session *s, uint32_t position) {
   if (position < s->chain_context) return greedy ? 3 : 4;
   return greedy ? 0 : 2;
 }
-// Whom a step's launches must not meet.
+// Whom a step's launches must not meet (a step's attention takes every CU).
 nv::Place step_place(const Session *s, int which) {
-  if (which < 3) return nv::Place::kAny;
-  return s->chain_wide ? nv::Place::kAlone : nv::Place::kBeside;
+  return which < 3 || s->chain_wide ? nv::Place::kAlone : nv::Place::kBeside;
 }
 
 // `steps` steps of kind `which`, captured.
@@ -1226,7 +1225,10 @@ hipError_t prompt_tokens(Session *s, uint32_t begin, uint32_t end, const uint32_
     logits += static_cast<uint64_t>(ahead) * s->vocab;
     wanted_count -= ahead;
   }
-  if (err == hipSuccess) err = enqueue_step(s, kPromptHeadStep, nullptr);
+  if (err == hipSuccess) {
+    const nv::InOrder turn(s, nv::Place::kAlone);
+    err = turn.error == hipSuccess ? enqueue_step(s, kPromptHeadStep, nullptr) : turn.error;
+  }
   if (err == hipSuccess) out->kernel_launches += step_launches(s, 0);
   if (err == hipSuccess && wanted_count != 0) {
     err = copy_out(s, logits, s->logits, s->vocab * sizeof(float), &out->sync_calls, false);
@@ -1234,46 +1236,6 @@ hipError_t prompt_tokens(Session *s, uint32_t begin, uint32_t end, const uint32_
   }
   return err;
 }
-
-// Whether a prompt's launches include a decode step's attention, whose workgroups wait for each other: prompts that are walked, and a last token that is alone in its pass.
-bool prompt_steps(const Session *s, uint32_t tokens) {
-  if (s->stack != nullptr) return false;
-  return !s->block_prefill || tuning(kTuneAttnWithholdSplit) != 0 || tokens % s->prefill_pass_tokens == 1 ||
-         (s->prefill_long_tokens != 0 && tokens % s->prefill_long_tokens == 1);
-}
-// Two such launches at once could hold each other's places (a step's attention takes every CU), and a start returns while its own are under way. So a start that has any
-// waits until those of the device's last such start have ended; prompts in blocks may run beside them.
-struct StepPrompts {
-  std::mutex mutex;
-  std::map<int, hipEvent_t> done;   // by device, for good
-};
-class StepPromptTurn {
- public:
-  StepPromptTurn(Session *session, bool steps) : s(session) {
-    if (!steps) return;
-    static StepPrompts *prompts = new StepPrompts;   // (sessions may outlive the library's statics)
-    turn = std::unique_lock<std::mutex>(prompts->mutex);
-    int device = 0;
-    error = hipGetDevice(&device);
-    if (error != hipSuccess) return;
-    hipEvent_t &event = prompts->done[device];
-    if (event == nullptr) error = hipEventCreateWithFlags(&event, hipEventDisableTiming);
-    if (error != hipSuccess) return;
-    nv::wait_if_there(event);
-    done = event;
-  }
-  ~StepPromptTurn() {
-    if (done != nullptr && hipEventRecord(done, s->stream) != hipSuccess) (void)hipStreamSynchronize(s->stream);
-  }
-  StepPromptTurn(const StepPromptTurn &) = delete;
-  StepPromptTurn &operator=(const StepPromptTurn &) = delete;
-  hipError_t error = hipSuccess;
-
- private:
-  Session *s;
-  hipEvent_t done = nullptr;
-  std::unique_lock<std::mutex> turn;
-};
 
 // Everything of a session that is not weights, from the dimensions already in `s`: stream, events,
 // the state arena (KV cache, block table, prompt, token slots, cursor words, activations and
@@ -1525,7 +1487,7 @@ hipError_t setup_state(Session *s, int32_t *failure_stage, bool with_weights) {
   if (err == hipSuccess) err = hipMemsetAsync(s->arena + off_attn_tagged, 0, attn_step_workspace_bytes(s->heads), s->stream);
   if (err == hipSuccess) err = hipMemsetAsync(s->arena + off_sample_ws, 0, sample_workspace_bytes(), s->stream);
   if (err == hipSuccess && chain) err = hipMemsetAsync(s->chain_model.words, 0, s->chain_word_bytes, s->stream);
-  if (err == hipSuccess && chain) err = join_order(s);
+  if (err == hipSuccess) err = join_order(s);
   if (err == hipSuccess) err = hipMemsetAsync(s->arena + off_pattn_ws, 0, pB * pattn_ws_stride, s->stream);
   if (err == hipSuccess && L > 0) err = hipMemsetAsync(s->arena + off_attn_trace, 0, L * 32 * 8, s->stream);
   if (err == hipSuccess) err = hipMemsetAsync(s->arena + off_kc, 0, 2 * ((kv_half + 255) & ~uint64_t{255}), s->stream);
@@ -2263,7 +2225,8 @@ int nerva_hip_hf_decode_sequence_batch_advance_one(const NervaHipHfDecodeSequenc
   } else if (err == hipSuccess) {
     // shapes outside the multi-row kernels: every sequence runs its own captured step on its own stream - one
     // after the other (each stream waits for the step before it): a step's attention launch wants every CU for
-    // workgroups that poll for each other, and two such launches side by side could hold each other's CUs
+    // workgroups that poll for each other, and two such launches side by side could hold each other's CUs; narrow models' steps fit beside each other, but not all
+    // of them. The tokens leave behind the last step: a step that waits for the one before would wait for its token's copy too
     NervaHipHfDecodeSequenceResult scratch{};
     Session *before = nullptr;
     const auto count_step = [out](const Session *q) {   // (a narrow model's layers are one launch, embedding and attention included)
@@ -2276,15 +2239,17 @@ int nerva_hip_hf_decode_sequence_batch_advance_one(const NervaHipHfDecodeSequenc
     for (uint32_t t = 0; err == hipSuccess && t < T; ++t) {
       Session *q = seqs[t];
       err = ensure_graph(q, decode_graph(q, q->cursor), &scratch);
-      if (err == hipSuccess && before != nullptr) err = hipStreamWaitEvent(q->stream, before->ev1, 0);
+      const bool beside = q->stack != nullptr || step_place(q, decode_graph(q, q->cursor)) == nv::Place::kBeside;   // (else launch_step sees to it)
+      if (err == hipSuccess && beside && before != nullptr) err = hipStreamWaitEvent(q->stream, before->ev1, 0);
       if (err == hipSuccess) err = launch_step(q, decode_graph(q, q->cursor), &scratch);
-      if (err == hipSuccess) err = hipEventRecord(q->ev1, q->stream);
-      before = q;
-      if (err == hipSuccess)
-        err = hipMemcpyAsync(&q->host_slots[q->cursor], &q->slots[q->cursor], sizeof(Slot), hipMemcpyDeviceToHost,
-                             q->stream);
-      out->d2h_bytes += sizeof(Slot);
+      if (err == hipSuccess && beside) err = hipEventRecord(q->ev1, q->stream);
+      before = beside ? q : nullptr;
       count_step(q);
+    }
+    for (uint32_t t = 0; err == hipSuccess && t < T; ++t) {
+      Session *q = seqs[t];
+      err = hipMemcpyAsync(&q->host_slots[q->cursor], &q->slots[q->cursor], sizeof(Slot), hipMemcpyDeviceToHost, q->stream);
+      out->d2h_bytes += sizeof(Slot);
     }
     for (uint32_t t = 0; err == hipSuccess && t < T; ++t) {
       Session *q = seqs[t];
@@ -2387,9 +2352,7 @@ int nerva_hip_hf_decode_sequence_session_start(const NervaHipHfDecodeSequenceSes
   fill_header(s, out, 0, request->prompt_tokens[P - 1]);
   s->started = false;
   const nv::PromptTurn prompt(s);
-  const StepPromptTurn steps(s, prompt_steps(s, P));
-  hipError_t err = steps.error;
-  if (err == hipSuccess) err = reset_sequence(s, request->sampler, request->prompt_tokens, P, out);   // session_api_lifecycle.inc.cu:1026
+  hipError_t err = reset_sequence(s, request->sampler, request->prompt_tokens, P, out);   // session_api_lifecycle.inc.cu:1026
   // prefill: the first P-1 prompt tokens (in blocks on the matrix cores where the shapes allow,
   // else one captured prompt step per token), then one prompt step with the LM head and sampler
   if (err == hipSuccess && P > 1 && s->stack == nullptr && !s->block_prefill) err = ensure_graph(s, 1, out);
@@ -2501,6 +2464,7 @@ int nerva_hip_session_extend(const NervaHipSessionExtendRequest *request, NervaH
 int nerva_hip_session_release_sequence(NervaHipHfDecodeSequenceSession *session) {
   if (session == nullptr) return -1;
   const bool idle = hipStreamSynchronize(session->stream) == hipSuccess;
+  if (idle) nv::out_of_order(session);
   session->started = false;
   session->finished = false;
   session->prompt_count = session->observed = session->cursor = 0;
@@ -2753,7 +2717,10 @@ int nerva_hip_session_profile_step(NervaHipHfDecodeSequenceSession *s, uint32_t 
   for (uint32_t rep = 0; err == hipSuccess && rep < repeats + 1; ++rep) {  // first pass is a warm-up
     prof.used = 0;
     prof.kinds.clear();
-    err = enqueue_step(s, kDecodeStep, &prof);
+    {
+      const nv::InOrder turn(s, nv::Place::kAlone);
+      err = turn.error == hipSuccess ? enqueue_step(s, kDecodeStep, &prof) : turn.error;
+    }
     if (err == hipSuccess) err = hipStreamSynchronize(s->stream);
     // undo the step: cursor and the published slot
     if (err == hipSuccess) err = hipMemcpy(s->state, &pos, 4, hipMemcpyHostToDevice);
@@ -2786,7 +2753,10 @@ int nerva_hip_session_profile_step(NervaHipHfDecodeSequenceSession *s, uint32_t 
       hipLaunchKernelGGL(bump_step_counter_kernel, dim3(1), dim3(64), 0, s->stream, s->state, s->attn_plan);
       err = hipGetLastError();
       if (err == hipSuccess) err = hipEventRecord(s->ev0, s->stream);
-      if (err == hipSuccess) err = enqueue_step(s, kDecodeStep, nullptr, kind);
+      if (err == hipSuccess) {
+        const nv::InOrder turn(s, nv::Place::kAlone);
+        err = turn.error == hipSuccess ? enqueue_step(s, kDecodeStep, nullptr, kind) : turn.error;
+      }
       if (err == hipSuccess) err = hipEventRecord(s->ev1, s->stream);
       if (err == hipSuccess) err = hipStreamSynchronize(s->stream);
       float ms = 0.0f;

@@ -239,17 +239,18 @@ class PassTurn {
   std::unique_lock<std::mutex> turn;
 };
 
-// While this lives the session enqueues a launch whose workgroups wait for each other, behind those of other sessions that it must not meet. The streams keep that
+// While this lives the session enqueues a launch whose workgroups wait for each other, behind those of other sessions that it must not meet - of calls in other threads, and of
+// starts that have returned while a prompt that is walked, or whose last token takes a step, is under way. The streams keep that
 // order: nobody waits on the host or on the device in front of what is to be waited for, and a session that has no other's launches under way beside it enqueues no more than
 // the launch. (Turns that a launch of one wave took by polling a word stood in front of what would have given the word back where two sessions share a hardware
 // queue; and they took two launches more a step beside any other session, idle or not: 69.4 -> 72.3 us at 512 wide,
 // 845 -> 848 at 4096.)
-enum class Place { kAny, kBeside, kAlone };   // meets anybody; nobody but its like (narrow models' steps); nobody
+enum class Place { kBeside, kAlone };   // meets its like (narrow models' steps); nobody
 class InOrder {
  public:
   InOrder(Session *session, Place place) {
     LaunchOrder *const order = session->order;
-    if (order == nullptr || place == Place::kAny) return;
+    if (order == nullptr) return;
     turn = std::unique_lock<std::mutex>(order->mutex);
     std::vector<Session *> &beside = order->beside;
     const auto at = std::find(beside.begin(), beside.end(), session);
@@ -279,13 +280,15 @@ class InOrder {
   }
   std::unique_lock<std::mutex> turn;
 };
-// A session's stream is idle: there is nothing left to come behind.
+// A session's stream is idle: there is nothing left of it to come behind, nor of what it came behind.
 inline void out_of_order(Session *session) {
   LaunchOrder *const order = session->order;
   if (order == nullptr) return;
   const std::lock_guard<std::mutex> lock(order->mutex);
-  if (order->alone == session) order->alone = nullptr;
-  order->beside.erase(std::remove(order->beside.begin(), order->beside.end(), session), order->beside.end());
+  std::vector<Session *> &beside = order->beside;
+  const auto at = std::find(beside.begin(), beside.end(), session);
+  if (order->alone == session || at != beside.end()) order->alone = nullptr;
+  if (at != beside.end()) beside.erase(at);
 }
 // The steps that a call enqueues without looking at them: where a device has other sessions, no more than twice steps_ahead (some 2 ms each) before the call waits for
 // the older ones, so that whoever else steps comes in between.

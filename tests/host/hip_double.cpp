@@ -21,6 +21,7 @@ std::string g_log;
 std::map<const void *, long> g_numbers;   // of streams and events
 long g_streams = 0, g_events = 0;
 std::atomic<long> g_held{0}, g_waits{0};
+thread_local hipStream_t t_stream;
 
 void log(const char *what, const void *first, const std::string &rest = "") {
   if (g_captured < 0) g_log += std::string(what) + " " + std::to_string(g_numbers[first]) + (rest.empty() ? "" : " " + rest) + "\n";
@@ -68,8 +69,14 @@ void **__hipRegisterFatBinary(const void *) {
 void __hipUnregisterFatBinary(void **) {}
 void __hipRegisterFunction(void **, const void *host, char *, const char *name, unsigned, void *, void *, void *, void *, int *) { g_names[host] = name; }
 void __hipRegisterVar(void **, void *, char *, char *, int, size_t, int, int) {}
-hipError_t __hipPushCallConfiguration(dim3, dim3, size_t, hipStream_t) { return hipSuccess; }
-hipError_t __hipPopCallConfiguration(dim3 *, dim3 *, size_t *, hipStream_t *) { return hipSuccess; }
+hipError_t __hipPushCallConfiguration(dim3, dim3, size_t, hipStream_t stream) {
+  t_stream = stream;
+  return hipSuccess;
+}
+hipError_t __hipPopCallConfiguration(dim3 *, dim3 *, size_t *, hipStream_t *stream) {
+  *stream = t_stream;
+  return hipSuccess;
+}
 hipError_t hipLaunchKernel(const void *kernel, dim3, dim3, void **, size_t, hipStream_t stream) {
   g_launches[g_names[kernel]] += 1;
   log("kernel", stream, g_names[kernel]);

@@ -200,6 +200,51 @@ def test_walked_prompts_begun_one_behind_the_other():
         N.Device.reset_tuning()
 
 
+def test_calls_behind_walked_prompts_under_way():
+    """A start of a walked prompt, and of one whose last token takes a step, returns while its attention launches are under way. What the next call brings on another session - tokens walked or alone,
+    steps in launches, in one launch of the whole device, of a narrow model - comes behind them: every result as when nothing is under way."""
+    geoms = [(BF16, 2048, 16, 8, 128, 2048, 301, 2), (BF16, 1024, 16, 8, 128, 2816, 301, 4), (BF16, 512, 4, 2, 128, 1024, 301, 4)]
+    rng = np.random.default_rng(9)
+    prompt = rng.integers(0, 301, 700).astype(np.uint32)
+    sessions = []
+    try:
+        for walk in (1, 0):
+            N.Device.set_tuning("prefill_walk", walk)
+            sessions += [N.DecodeSession.create(random_model(*g, 4, 1e6, True, False)[0], 1100) for g in geoms]
+    finally:
+        N.Device.reset_tuning()
+    walked, blocks = sessions[:3], sessions[3:]
+
+    def begun(s):
+        assert s.start(prompt[:90])[0] == 0 and s.advance(2)[0] == 0
+
+    def stepped(s):
+        rc, _, tokens = s.advance(5)
+        return rc, tokens.tolist()
+
+    def extended(s):
+        return [(rc, rows.tolist()) for rc, _, rows, _ in (s.extend(prompt[:n], [n - 1]) for n in (30, 1))]
+
+    def ran(s):
+        rc, _, tokens = s.run(prompt[:40], 4)
+        return rc, tokens.tolist()
+    want = {}
+    for s in sessions:
+        for call in (stepped, extended, ran):
+            begun(s)
+            want[s, call] = call(s)
+    for first, start in [(s, prompt) for s in walked] + [(s, prompt[:1]) for s in blocks] + [(blocks[0], prompt[:513])]:
+        for s in sessions:
+            if s is first:
+                continue
+            for call in (stepped, extended, ran):
+                begun(s)
+                assert first.start(start)[0] == 0
+                assert call(s) == want[s, call]
+    for s in sessions[::-1]:
+        s.destroy()
+
+
 def test_starts_behind_sessions_that_are_gone():
     """What the last starts have left to wait for may have been on sessions that have ended since: walked prompts, single tokens, prompts in blocks, on the same weights and on others."""
     prompts = [np.arange(n, dtype=np.uint32) for n in (1, 40, 300)]

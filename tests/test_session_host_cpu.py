@@ -182,6 +182,67 @@ for s in (b, a, d, c):
 """)
 
 
+def test_whatever_follows_a_start_comes_behind_the_steps_of_its_prompt(double):
+    """A start returns while its prompt is under way: one that is walked, or whose last token takes a step, has attention launches there that must not meet a step of any other session. Every call
+    that brings one comes behind it - walked and lone tokens of starts and extensions, advance and run in launches and in one, a batch, a profile -; prompts in blocks neither wait nor are waited for."""
+    run(double, """
+double.double_device(256, 2)
+tokens = np.arange(9, dtype=np.uint32)
+few = dict(dtype=BF16, hidden=512, heads=8, kv_heads=2, head_dim=64, intermediate=1024, vocab=64, layers=2, rms_eps=1e-6, rope_theta=1e4)
+wide = dict(dtype=BF16, hidden=1024, heads=8, kv_heads=2, head_dim=128, intermediate=4096, vocab=64, layers=4, rms_eps=1e-6, rope_theta=1e4)
+narrow = dict(few, layers=4, hidden=256, intermediate=512)
+N.Device.set_tuning("prefill_walk", 1)
+walked = [N.DecodeSession.create_synthetic(cfg, 64, weight_hash=7) for cfg in (few, wide, narrow)]
+N.Device.reset_tuning()
+blocks = [N.DecodeSession.create_synthetic(cfg, 64, weight_hash=7) for cfg in (few, wide, narrow)]
+stream = {}
+for s in walked + blocks:
+    double.double_clear_log()
+    step(s)
+    stream[s], = {int(line.split()[1]) for line in log() if line.startswith("graph")}
+    s.profile_step(1)                                      # (every graph is there)
+
+def waits_behind(first, start, other, call):
+    assert other.start(tokens)[0] == 0 and first.start(tokens)[0] == 0
+    other.release_sequence(), first.release_sequence()
+    if call not in (extended, extended_one, ran, started, started_one):
+        assert other.start(tokens)[0] == 0
+    double.double_clear_log()
+    assert first.start(start)[0] == 0
+    begun = len(log())
+    call(other)
+    lines = log()
+    steps = [i for i, line in enumerate(lines) if line.split()[:2] in (["graph", "%d" % stream[other]], ["kernel", "%d" % stream[other]]) and "sequence_kernel" not in line and i >= begun]
+    events = [line.split()[2] for line in lines[begun:] if line.startswith("record %d " % stream[first])]
+    assert steps, (call, lines)
+    for i, line in enumerate(lines[begun:steps[-1]]):
+        if line.split()[0] == "wait" and line.split()[1] == "%d" % stream[other] and line.split()[2] in events:
+            return begun + i < steps[0]
+    return False
+
+def started(s): s.start(tokens)
+def started_one(s): s.start(tokens[:1])
+def extended(s): s.extend(tokens)
+def extended_one(s): s.extend(tokens[:1])
+def advanced(s): s.advance(3)
+def ran(s): s.run(tokens, 2)
+def profiled(s): s.profile_step(1)
+def batched(s): N.DecodeSession.batch_advance_one([s], 1, 1)
+for first in walked + blocks:
+    for other in walked + blocks:
+        if other is first:
+            continue
+        for start in (tokens, tokens[:1]):
+            steps = first in walked or len(start) == 1
+            for call in (advanced, ran, extended_one, started_one, profiled):
+                assert waits_behind(first, start, other, call) == steps, (first in walked, other in walked, len(start), call, log())
+            for call in (started, extended):
+                assert waits_behind(first, start, other, call) == (steps and other in walked), (first in walked, other in walked, len(start), call, log())
+for s in walked + blocks:
+    s.destroy()
+""")
+
+
 def test_long_calls_beside_other_sessions_do_not_run_far_ahead(double):
     """Steps that nobody looks at: some 4 ms of them are under way at the most where a device has other sessions, so that these come in between, and any number where it has not."""
     run(double, """
