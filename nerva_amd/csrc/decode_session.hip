@@ -2351,8 +2351,8 @@ int nerva_hip_hf_decode_sequence_session_start(const NervaHipHfDecodeSequenceSes
   const uint32_t P = request->prompt_token_count;
   fill_header(s, out, 0, request->prompt_tokens[P - 1]);
   s->started = false;
-  const nv::PromptTurn prompt(s);
   hipError_t err = reset_sequence(s, request->sampler, request->prompt_tokens, P, out);   // session_api_lifecycle.inc.cu:1026
+  const nv::PromptTurn prompt(s);
   // prefill: the first P-1 prompt tokens (in blocks on the matrix cores where the shapes allow,
   // else one captured prompt step per token), then one prompt step with the LM head and sampler
   if (err == hipSuccess && P > 1 && s->stack == nullptr && !s->block_prefill) err = ensure_graph(s, 1, out);

@@ -155,8 +155,9 @@ d = c.fork_shared_weights()
 sessions = (a, b, c, d)
 stream = {}
 for s in sessions:
+    assert s.start(np.arange(5, dtype=np.uint32))[0] == 0
     double.double_clear_log()
-    assert step(s).graph_nodes == 3
+    assert s.advance(2)[1].graph_nodes == 3
     assert not any(line.startswith("wait") for line in log()), log()
     stream[s], = (int(line.split()[1]) for line in log() if line.startswith("graph"))
 for held, meets in ((a, (b,)), (c, ())):
@@ -173,8 +174,8 @@ for held, meets in ((a, (b,)), (c, ())):
         records = [line.split()[2] for line in lines[:launch] if line.startswith("record %d " % stream[held])]
         assert waits == records and len(waits) == (0 if other in meets else 1), (lines, stream)
         under_way()
-        double.double_clear_log()
         other.start(np.arange(5, dtype=np.uint32))
+        double.double_clear_log()
         other.advance(2)
         assert not any(line.startswith("wait") for line in log())
 for s in (b, a, d, c):
@@ -241,6 +242,37 @@ for first in walked + blocks:
 for s in walked + blocks:
     s.destroy()
 """)
+
+
+@pytest.mark.parametrize("stack", [False, True])
+def test_starts_that_follow_each_other_wait_on_the_device(double, stack):
+    """No more than four prompts of a set of weights are under way: the fifth's stream comes behind the first's event, ahead of everything but what brings its tokens. The host waits for the
+    session's own stream and for nothing else."""
+    run(double, """
+if %r:
+    from nerva_amd import stackbench
+    stackbench.VOCAB = 64
+    first = N.DecodeSession.create_stack_synthetic(stackbench.expert_stack_config(1024, 8, 4, 2, 256, 256, 256, 128, 1, 64), 64)
+else:
+    first = N.DecodeSession.create(model(), 64)
+sessions = [first] + [first.fork_shared_weights() for _ in range(6)]
+streams, events = [], []
+for i, s in enumerate(sessions + sessions[:2]):
+    double.double_clear_log()
+    assert s.start(np.arange(20, dtype=np.uint32))[0] == 0
+    lines = log()
+    assert [line.split()[0] for line in lines[:2]] == ["sync", "kernel"] and "sequence_kernel" in lines[1], lines
+    streams.append(lines[0].split()[1])
+    waits = [line.split() for line in lines if line.startswith("wait")]
+    assert len(waits) == 1 and lines[2] == " ".join(waits[0]) and waits[0][1] == streams[-1], lines
+    assert sum(line.startswith("sync") for line in lines) == 1
+    assert lines[-1].startswith("record %%s " %% streams[-1])
+    events.append(lines[-1].split()[2])
+    assert i < 4 or waits[0][2] == events[i - 4]
+assert len(set(events)) == 4
+for s in sessions[::-1]:
+    s.destroy()
+""" % stack)
 
 
 def test_long_calls_beside_other_sessions_do_not_run_far_ahead(double):
