@@ -35,7 +35,7 @@ extern "C" {
 #define NERVA_HIP_SLOT_DEVICE_COMPLETE 1u /* types.cuh:36 */
 /* No counterpart in the reference: the slot of a token whose step a device-side bounded wait gave up on (the
  * attention's split merge; a step's layers in one launch, where the step was taken again and given up 256 times in a
- * row). The token is not valid; the call that reads the slot, or the extend of one token that the step was, returns -1 with
+ * row, which a call does not come to by itself: it goes on launch by launch before). The token is not valid; the call that reads the slot, or the extend of one token that the step was, returns -1 with
  * hip_error = NERVA_HIP_ERROR_STEP_FAULT, and the sequence has to be started again. */
 #define NERVA_HIP_SLOT_DEVICE_FAULT 2u
 #define NERVA_HIP_ERROR_STEP_FAULT 719 /* hipErrorLaunchFailure */
@@ -880,8 +880,9 @@ int nerva_hip_session_profile_step(NervaHipHfDecodeSequenceSession *session, uin
  * through the general kernel, whatever their shape; read at every launch, so a captured step keeps what it was
  * captured with), "latent_attention_wide" (2: the same for layers of attention over latents), "step_chain" (2: sessions
  * created afterwards never run a step's layers in one launch; 0: those of dense models of four layers and more do, up to 1024 wide and 10 MB of weights
- * a layer or from 12 MB on, of two and three layers from 64 MB on, of one from 256 MB on, heads of 64 or 128, one to eight query heads a key head), "step_chain_withhold" (a workgroup of that launch stays away so often in a row: the
- * step gives up and is taken again). Values a kernel
+ * a layer or from 12 MB on, of two and three layers from 64 MB on, of one from 256 MB on, heads of 64 or 128, one to eight query heads a key head; 1: as 0, and steps that
+ * give up again and again go launch by launch also where the next hook or "attn_merge_spin_limit" makes them), "step_chain_withhold" (a workgroup of that launch stays away so often in a row:
+ * the step gives up and is taken again). Values a kernel
  * cannot take are ignored where they are read. -1 for an unknown name. A null name restores every built-in
  * choice. */
 int nerva_hip_test_set_tuning(const char *name, int32_t value);

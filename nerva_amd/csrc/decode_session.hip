@@ -599,7 +599,7 @@ hipError_t launch_step(Session *s, int which, NervaHipHfDecodeSequenceResult *ou
 // Index of the captured decode step for the active sampler, at a position.
 int decode_graph(const Session *s, uint32_t position) {
   const bool greedy = s->sampler.mode == kSamplerGreedy;
-  if (position < s->chain_context) return greedy ? 3 : 4;
+  if (position < s->chain_context && s->chain_avoid == 0) return greedy ? 3 : 4;
   return greedy ? 0 : 2;
 }
 // Whom a step's launches must not meet (a step's attention takes every CU).
@@ -680,11 +680,28 @@ hipError_t ensure_graphs(Session *s, uint32_t position, uint32_t steps, NervaHip
 
 // Steps that have given up since the last look, of work that is done: the next step was the same one again, and as many are still to come. (One that
 // ends the sequence with a fault counts as done; the bit stays until another begins.)
+// Where nothing but such steps has been seen for kMissesMost of them (0.1 s), whoever holds the places will not let go soon: the next kAvoidSteps go launch by launch, which need
+// theirs for one layer's attention at a time. (Not where a test hook makes the waits run out, so that the end of it all is reached; "step_chain" = 1: there too.)
+constexpr uint32_t kMissesMost = 32, kAvoidSteps = 256;
 uint32_t take_given_up(Session *s) {
   if (s->given_up == nullptr) return 0;
   const uint32_t told = *static_cast<volatile uint32_t *>(s->given_up), count = told & ~kHostFault;
   if (count != 0) *static_cast<volatile uint32_t *>(s->given_up) = told & kHostFault;
+  s->chain_missed = count < std::exchange(s->chain_sent, 0u) ? 0u : s->chain_missed + count;
+  const bool made = tuning(kTuneStepChainWithhold) > 0 || tuning(kTuneAttnMergeSpinLimit) > 0;
+  if (s->chain_missed >= kMissesMost && (!made || tuning(kTuneStepChain) == 1)) {
+    s->chain_missed = 0;
+    s->chain_avoid = kAvoidSteps;
+  }
   return count;
+}
+// In the middle of a call, as soon as the host's word says that some have: how many of those sent so far are to be sent again.
+hipError_t look_back(Session *s, uint32_t *again) {
+  *again = 0;
+  if (s->given_up == nullptr || (*static_cast<volatile uint32_t *>(s->given_up) & ~kHostFault) == 0) return hipSuccess;
+  const hipError_t err = hipStreamSynchronize(s->stream);
+  if (err == hipSuccess) *again = take_given_up(s);
+  return err;
 }
 // `count` steps more, up to a position.
 hipError_t launch_steps_again(Session *s, uint32_t end, uint32_t count, NervaHipHfDecodeSequenceResult *out) {
@@ -693,9 +710,16 @@ hipError_t launch_steps_again(Session *s, uint32_t end, uint32_t count, NervaHip
   return err;
 }
 
+// Steps of a kind have gone out.
+void count_sent(Session *s, int which, uint32_t steps) {
+  if (which >= 3) s->chain_sent += steps;
+  else if (which != 1 && s->chain_avoid != 0) s->chain_avoid -= 1;
+}
 hipError_t enqueue_in_order(Session *s, int which) {
   const nv::InOrder turn(s, step_place(s, which));
-  return turn.error == hipSuccess ? enqueue_graph_step(s, which) : turn.error;
+  const hipError_t err = turn.error == hipSuccess ? enqueue_graph_step(s, which) : turn.error;
+  if (err == hipSuccess) count_sent(s, which, 1);
+  return err;
 }
 hipError_t launch_step(Session *s, int which, NervaHipHfDecodeSequenceResult *out) {
   if (s->trace_buf != nullptr && which != 1) {
@@ -707,6 +731,8 @@ hipError_t launch_step(Session *s, int which, NervaHipHfDecodeSequenceResult *ou
     while (err == hipSuccess && which >= 3) {
       err = hipStreamSynchronize(s->stream);
       if (err != hipSuccess || take_given_up(s) == 0) break;
+      if (s->chain_avoid != 0) which = which == 3 ? 0 : 2;
+      s->trace_used = 0;
       err = enqueue_in_order(s, which);
       if (err == hipSuccess) out->kernel_launches += step_launches(s, which);
     }
@@ -719,14 +745,18 @@ hipError_t launch_step(Session *s, int which, NervaHipHfDecodeSequenceResult *ou
       out->kernel_launches += step_launches(s, which);
     return err;
   }
+  hipError_t err = s->exec[which] == nullptr ? ensure_graph(s, which, out) : hipSuccess;   // (a call that goes on launch by launch)
+  if (err != hipSuccess) return err;
   const nv::InOrder turn(s, step_place(s, which));
-  hipError_t err = turn.error;
+  err = turn.error;
   if (err == hipSuccess) err = hipGraphLaunch(s->exec[which], s->stream);
   if (err == hipSuccess) {
     out->graph_replays += 1;
     out->graph_launches += 1;
+    out->graph_nodes = s->graph_nodes[which];
     out->kernel_launches += s->graph_nodes[which];
     if (which >= 3) s->chain_steps += 1;
+    count_sent(s, which, 1);
   }
   return err;
 }
@@ -746,6 +776,7 @@ hipError_t launch_steps(Session *s, uint32_t position, uint32_t steps, uint32_t 
     out->graph_launches += 1;
     out->kernel_launches += kMost * s->graph_nodes[which];
     s->chain_steps += kMost;
+    count_sent(s, which, kMost);
   }
   return err;
 }
@@ -2229,8 +2260,8 @@ int nerva_hip_hf_decode_sequence_batch_advance_one(const NervaHipHfDecodeSequenc
     // of them. The tokens leave behind the last step: a step that waits for the one before would wait for its token's copy too
     NervaHipHfDecodeSequenceResult scratch{};
     Session *before = nullptr;
-    const auto count_step = [out](const Session *q) {   // (a narrow model's layers are one launch, embedding and attention included)
-      const bool chained = decode_graph(q, q->cursor) >= 3;
+    const auto count_step = [out](const Session *q, int which) {   // (layers in one launch: the embedding and attention included)
+      const bool chained = which >= 3;
       out->pack_kernel_launches += chained ? 0 : 1;
       out->projection_kernel_launches += chained ? 2ull : 4ull * q->layers + 1;
       out->dependency_kernel_launches += chained ? 0 : q->layers;
@@ -2238,13 +2269,14 @@ int nerva_hip_hf_decode_sequence_batch_advance_one(const NervaHipHfDecodeSequenc
     };
     for (uint32_t t = 0; err == hipSuccess && t < T; ++t) {
       Session *q = seqs[t];
-      err = ensure_graph(q, decode_graph(q, q->cursor), &scratch);
-      const bool beside = q->stack != nullptr || step_place(q, decode_graph(q, q->cursor)) == nv::Place::kBeside;   // (else launch_step sees to it)
+      const int which = decode_graph(q, q->cursor);
+      err = ensure_graph(q, which, &scratch);
+      const bool beside = q->stack != nullptr || step_place(q, which) == nv::Place::kBeside;   // (else launch_step sees to it)
       if (err == hipSuccess && beside && before != nullptr) err = hipStreamWaitEvent(q->stream, before->ev1, 0);
-      if (err == hipSuccess) err = launch_step(q, decode_graph(q, q->cursor), &scratch);
+      if (err == hipSuccess) err = launch_step(q, which, &scratch);
       if (err == hipSuccess && beside) err = hipEventRecord(q->ev1, q->stream);
       before = beside ? q : nullptr;
-      count_step(q);
+      count_step(q, which);
     }
     for (uint32_t t = 0; err == hipSuccess && t < T; ++t) {
       Session *q = seqs[t];
@@ -2256,11 +2288,12 @@ int nerva_hip_hf_decode_sequence_batch_advance_one(const NervaHipHfDecodeSequenc
       err = hipStreamSynchronize(q->stream);
       out->sync_calls += 1;
       while (err == hipSuccess && take_given_up(q) != 0) {
-        err = launch_step(q, decode_graph(q, q->cursor), &scratch);
+        const int which = decode_graph(q, q->cursor);
+        err = launch_step(q, which, &scratch);
         if (err == hipSuccess)
           err = hipMemcpyAsync(&q->host_slots[q->cursor], &q->slots[q->cursor], sizeof(Slot), hipMemcpyDeviceToHost, q->stream);
         if (err == hipSuccess) err = hipStreamSynchronize(q->stream);
-        count_step(q);
+        count_step(q, which);
         out->d2h_bytes += sizeof(Slot);
         out->sync_calls += 1;
       }
@@ -2494,7 +2527,10 @@ int nerva_hip_hf_decode_sequence_session_advance(const NervaHipHfDecodeSequenceS
   if (err == hipSuccess && run_count != 0) err = hipEventRecord(s->ev0, s->stream);
   nv::RunAhead ahead(s);
   for (uint32_t step = 0, taken = 0; err == hipSuccess && step < run_count; step += taken) {
+    uint32_t again = 0;
     if (s->has_eos == 0) err = ahead.room(taken);
+    if (err == hipSuccess && s->has_eos == 0) err = look_back(s, &again);
+    step -= again;
     if (err == hipSuccess) err = launch_steps(s, s->cursor + step, s->has_eos != 0 ? 1 : run_count - step, &taken, out);
     // With a stop token the host looks at each token so that it can stop launching
     // (session_api_lifecycle.inc.cu:1206-1234); without one the loop never syncs.
@@ -2593,7 +2629,10 @@ int nerva_hip_hf_decode_sequence_session_run(const NervaHipHfDecodeSequenceSessi
   if (err == hipSuccess) err = hipEventRecord(s->ev0, s->stream);
   nv::RunAhead ahead(s);
   for (uint32_t step = 0, taken = 0; err == hipSuccess && step < context_steps; step += taken) {
+    uint32_t again = 0;
     err = ahead.room(taken);
+    if (err == hipSuccess) err = look_back(s, &again);
+    step -= again;
     if (err == hipSuccess) err = launch_steps(s, step, context_steps - step, &taken, out);
   }
   const uint64_t slots_bytes = static_cast<uint64_t>(context_steps) * sizeof(Slot);

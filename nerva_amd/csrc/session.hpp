@@ -140,6 +140,8 @@ struct NervaHipHfDecodeSequenceSession : nv::RowScratch {
   uint32_t steps_ahead = 0;          // steps that a call sends ahead of those it has seen the end of, where others may be waiting (RunAhead)
   hipEvent_t mark = nullptr;         // ... and the event that it looks at
   uint32_t *given_up = nullptr;      // host_state[0]: steps that gave up since the host looked (step_given_up writes it)
+  uint32_t chain_sent = 0, chain_missed = 0;   // such steps sent since then; those that gave up with none between them that did not, as far as looks tell
+  uint32_t chain_avoid = 0;          // steps that are still taken launch by launch instead (take_given_up)
   // prompt blocks: up to prefill_pass_tokens prompt tokens per pass through the layers (weights streamed
   // once per pass on the matrix cores), in a long prompt prefill_long_tokens; false = one prompt step per token
   bool block_prefill = false;
@@ -292,14 +294,19 @@ inline void out_of_order(Session *session) {
   if (at != beside.end()) beside.erase(at);
 }
 // The steps that a call enqueues without looking at them: where a device has other sessions, no more than twice steps_ahead (some 2 ms each) before the call waits for
-// the older ones, so that whoever else steps comes in between.
+// the older ones, so that whoever else steps comes in between; of steps in one launch never more than twice kUnseen, so that the host hears of those that give up before so many
+// have in a row that the device ends the sequence.
 class RunAhead {
+  static constexpr uint32_t kUnseen = 96;
+  static_assert(2 * kUnseen + Session::kStepsTogether < kMostGivenUp, "");
+
  public:
   explicit RunAhead(Session *session) : s(session) {}
   // Ahead of the next steps; `sent`: with those that went out since it was last asked.
   hipError_t room(uint32_t sent) {
     unseen += sent;
-    if (unseen < s->steps_ahead || s->order == nullptr || s->order->sessions.load(std::memory_order_relaxed) < 2) return hipSuccess;
+    const bool others = s->order != nullptr && s->order->sessions.load(std::memory_order_relaxed) > 1;
+    if (unseen < (others ? s->steps_ahead : kUnseen) || (!others && s->given_up == nullptr)) return hipSuccess;
     hipError_t err = marked ? hipEventSynchronize(s->mark) : hipSuccess;
     if (err == hipSuccess) err = hipEventRecord(s->mark, s->stream);
     marked = true;

@@ -105,6 +105,61 @@ def test_wide_steps_that_give_up_are_taken_again():
         N.Device.reset_tuning()
 
 
+@pytest.mark.parametrize("shape", [SHAPES[0], (BF16, 256, 2, 2, 128, 512, 301, 4, 1e6, True, True)], ids=["wide", "narrow"])
+def test_steps_that_never_find_their_places_go_launch_by_launch(shape):
+    """Waits that run out at once, as where somebody else keeps the places for good: after some of them a call goes on in launches, whichever call it is, and gives what launches give."""
+    dtype, hidden, heads, kv, hd, inter, vocab, layers, theta, qk_norm, bias = shape
+    weights, _ = random_model(dtype, hidden, heads, kv, hd, inter, vocab, layers, 5, theta, qk_norm, bias)
+    prompt = np.random.default_rng(2).integers(0, vocab, 9).astype(np.uint32)
+    sampler = abi.NervaHipHfDecodeSamplerConfig()
+    sampler.temperature, sampler.top_p, sampler.top_k, sampler.seed = 0.9, 0.95, 0, 11
+
+    def calls(s, mode):
+        out = []
+        assert s.start(prompt)[0] == 0
+        for n in (1, 2, 40):
+            rc, res, tokens = s.advance(n)
+            assert rc == 0 and (n == 1 or res.graph_nodes == 3 + 5 * layers)
+            out.append(tokens)
+        out.append(s.logits())
+        s.destroy()
+        s = fresh(mode)
+        assert s.start(prompt, eos=vocab - 1, sampler=sampler)[0] == 0
+        rc, res, tokens = s.advance(20)
+        assert rc == 0
+        out.append(tokens)
+        s.destroy()
+        s = fresh(mode)
+        rc, res, tokens = s.run(prompt, 30)
+        assert rc == 0
+        out.append(tokens)
+        s.destroy()
+        s = fresh(mode)
+        assert s.extend(prompt)[0] == 0
+        rc, res, rows, _ = s.extend([3], [0])
+        assert rc == 0
+        out.append(rows)
+        s.destroy()
+        s = fresh(mode)
+        assert s.start(prompt)[0] == 0 and s.advance(1)[0] == 0
+        rc, res, token, trace = s.traced_advance()
+        assert rc == 0
+        out += [token, trace["logits"]]
+        s.destroy()
+        return out
+
+    def fresh(mode):
+        N.Device.set_tuning("step_chain", mode)
+        N.Device.set_tuning("attn_merge_spin_limit", 1)       # (contexts of one split: the attention launches wait for nothing)
+        return N.DecodeSession.create(weights, 64)
+    try:
+        got, want = (calls(fresh(mode), mode) for mode in (1, 2))
+    finally:
+        N.Device.reset_tuning()
+    for i, (a, b) in enumerate(zip(got, want)):
+        assert np.array_equal(a, b), i
+
+
 def test_sessions_of_wide_and_narrow_models_take_turns():
     """Six sessions of a wide model and two of a narrow one, more than there are hardware queues, from threads of their own: each gives what it gives alone, in the same
     launches, and all of them together take no longer than one after the other (a step in front of the one that it waits for would stand still for as long as the waits' limits)."""

@@ -276,12 +276,13 @@ for s in sessions[::-1]:
 
 
 def test_long_calls_beside_other_sessions_do_not_run_far_ahead(double):
-    """Steps that nobody looks at: some 4 ms of them are under way at the most where a device has other sessions, so that these come in between, and any number where it has not."""
+    """Steps that nobody looks at: some 4 ms of them are under way at the most where a device has other sessions, so that these come in between, and fewer than give up in a row before the
+    device ends a sequence where it has not; of steps in launches any number."""
     run(double, """
 def looks(s):
     assert s.start(np.arange(5, dtype=np.uint32))[0] == 0
     double.double_clear_log()
-    assert s.advance(201)[0] == -1                          # (the stand-in publishes no tokens)
+    assert s.advance(301)[0] == -1                          # (the stand-in publishes no tokens)
     sent = done = most = 0
     at = {}
     for words in (line.split() for line in log()):
@@ -293,13 +294,20 @@ def looks(s):
         elif words[:2] == ["sync", "event"]:
             done = at[words[2]]
     return most, sum(line.startswith("sync event") for line in log())
-s = N.DecodeSession.create(model(), 300)
-assert looks(s) == (200, 0)
+def lone(s):
+    most, times = looks(s)
+    return times >= 1 and 150 <= most < 256
+s = N.DecodeSession.create(model(), 400)
+assert lone(s)
 other = s.fork_shared_weights()
 most, times = looks(s)
 assert times >= 2 and 50 <= most <= 2 * 56, (most, times)
 other.destroy()
-assert looks(s) == (200, 0)
+assert lone(s)
+s.destroy()
+N.Device.set_tuning("step_chain", 2)
+s = N.DecodeSession.create(model(), 400)
+assert looks(s)[1] == 0
 s.destroy()
 """)
 
