@@ -368,8 +368,7 @@ def test_norms_of_rows_at_the_ends_of_f32(scale, eps):
 
 @pytest.mark.parametrize("wide", [False, True])
 def test_steps_that_go_out_together_give_what_single_ones_give(wide):
-    """Greedy and sampled, one session and a second beside it, past the context where steps become launches: a call of 100 steps against
-    calls of one."""
+    """Greedy and sampled, one session and a second beside it: a call of 100 steps against calls of one."""
     shape = (BF16, 1024, 16, 8, 128, 2816, 301, 4, 1e6, True, False) if wide else SHAPES[0]
     dtype, hidden, heads, kv, hd, inter, vocab, layers, theta, qk_norm, bias = shape
     weights, _ = random_model(dtype, hidden, heads, kv, hd, inter, vocab, layers, 5, theta, qk_norm, bias)
@@ -389,4 +388,22 @@ def test_steps_that_go_out_together_give_what_single_ones_give(wide):
             assert tokens.tolist() == single.tolist() and np.array_equal(s.logits(), logits)
         if other is not None:
             other.destroy()
+    s.destroy()
+
+
+@pytest.mark.parametrize("shape,context", [(SHAPES[0], 4096), (SHAPES[7], 1536)])
+def test_one_call_across_the_context_where_steps_become_launches(shape, context):
+    """From sixes to single steps to launches: one call against calls of one step."""
+    dtype, hidden, heads, kv, hd, inter, vocab, layers, theta, qk_norm, bias = shape
+    weights, _ = random_model(dtype, hidden, heads, kv, hd, inter, vocab, layers, 5, theta, qk_norm, bias)
+    prompt = np.random.default_rng(2).integers(0, vocab, context - 70).astype(np.uint32)
+    s = N.DecodeSession.create(weights, context + 64)
+    assert s.start(prompt)[0] == 0
+    single = [s.advance(1) for _ in range(91)]
+    assert [res.graph_nodes for _, res, _ in single[1:]] == [3] * 70 + [3 + 5 * layers] * 20
+    want, logits = [int(tokens[0]) for _, _, tokens in single], s.logits()
+    assert s.start(prompt)[0] == 0
+    rc, res, tokens = s.advance(91)
+    assert rc == 0 and res.graph_replays == 90 and res.graph_launches == 11 + 4 + 20 and res.graph_nodes == 3 + 5 * layers
+    assert tokens.tolist() == want and np.array_equal(s.logits(), logits)
     s.destroy()

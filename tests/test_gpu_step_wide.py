@@ -24,6 +24,8 @@ SHAPES = [
     (BF16, 2048, 16, 2, 64, 1800, 301, 5, 5e5, True, False),
     (F16, 5128, 2, 2, 128, 520, 301, 4, 1e6, False, True),       # (in bf16 its launches are 2.7e-2 from the oracle after ten steps, too)
     (F16, 256, 10, 2, 64, 12288, 301, 4, 1e4, True, False),
+    (F16, 5120, 5, 1, 128, 520, 301, 4, 1e6, True, False),       # (five pairs a thread; five and seven query heads a key head of 128)
+    (F16, 3584, 7, 1, 128, 1032, 301, 4, 1e6, False, True),
 ]
 
 
@@ -43,7 +45,7 @@ def test_every_link_of_a_step_in_one_launch_matches_the_oracle(shape):
     print(sorted(worst.items()), e2e, flush=True)
 
 
-@pytest.mark.parametrize("shape", SHAPES[:6])
+@pytest.mark.parametrize("shape", SHAPES[:6] + [(dtype,) + shape[1:] for shape in SHAPES[8:] for dtype in (BF16, F16)])
 def test_longer_contexts_in_one_launch_give_what_launches_give(shape):
     """Contexts of one split, of the first several, of as many as there are and of several blocks a wave, behind prompts that both kinds of session
     have read alike: logits and cache rows of the steps. Only roundings of 16-bit values that lie on a boundary may fall differently."""
@@ -73,6 +75,40 @@ def test_longer_contexts_in_one_launch_give_what_launches_give(shape):
         assert np.all(np.isfinite(got)) and rel_l2(got, want) <= chain_budget(layers), (n, rel_l2(got, want))
         for a, b in zip(want_rows, got_rows):
             assert rel_l2(O.decode16(dtype, b), O.decode16(dtype, a)) <= chain_budget(layers), n
+
+
+@pytest.mark.parametrize("dtype,hidden,heads,kv,hd,inter,context", [(BF16, 1024, 16, 8, 128, 4096, 32768), (F16, 1024, 16, 8, 64, 4096, 32768), (BF16, 1024, 8, 1, 128, 4096, 8192),
+                                                                    (F16, 1280, 20, 4, 64, 5120, 8192)])
+def test_the_longest_contexts_in_one_launch_and_the_first_behind_them(dtype, hidden, heads, kv, hd, inter, context):
+    """As many blocks a wave as there can be: the logits of the steps of the last positions that one launch takes, against launches; and one call across the line, in sixes, singly and launch by
+    launch, against calls of one step."""
+    layers, vocab = 4, 301
+    cfg = dict(dtype=dtype, hidden=hidden, heads=heads, kv_heads=kv, head_dim=hd, intermediate=inter, vocab=vocab, layers=layers, rms_eps=1e-6, rope_theta=1e6)
+    prompt = np.random.default_rng(3).integers(0, vocab, context - 40).astype(np.uint32)
+    rows = []
+    try:
+        for mode in (2, 0):
+            N.Device.set_tuning("step_chain", mode)
+            s = N.DecodeSession.create_synthetic(cfg, context + 64)
+            assert s.start(prompt[:-2])[0] == 0
+            for token in prompt[-2:]:
+                rc, res, logits, _ = s.extend([token], [0])
+                assert rc == 0 and res.graph_nodes == (3 if mode == 0 else 3 + 5 * layers)
+            rows.append(logits[0])
+            if mode == 2:
+                s.destroy()
+    finally:
+        N.Device.reset_tuning()
+    assert np.all(np.isfinite(rows[1])) and rel_l2(rows[1], rows[0]) <= chain_budget(layers)
+    assert s.start(prompt)[0] == 0
+    single = [s.advance(1) for _ in range(61)]
+    assert [res.graph_nodes for _, res, _ in single[1:]] == [3] * 40 + [3 + 5 * layers] * 20
+    want, logits = [int(tokens[0]) for _, _, tokens in single], s.logits()
+    assert s.start(prompt)[0] == 0
+    rc, res, tokens = s.advance(61)
+    assert rc == 0 and res.graph_replays == 60 and res.graph_launches == 6 + 4 + 20
+    assert tokens.tolist() == want and np.array_equal(s.logits(), logits)
+    s.destroy()
 
 
 def test_wide_steps_that_give_up_are_taken_again():
