@@ -270,7 +270,8 @@ def main():
     # Per-kernel durations, timed live with hipEvents on the session stream. "stream" figures
     # bracket all 36 launches of one kind (one per layer, distinct weights) with ONE event pair and
     # divide by the count: the kernel's own duration, which is what a kernel trace reports. The
-    # per-launch event pairs of the eager pass add the event/dispatch gap of every launch.
+    # per-launch event pairs of the eager pass add the event/dispatch gap of every launch. Where a step's
+    # layers run in one launch these are the launches that it stands in for.
     rc, prof = session.profile_step(3)
     assert rc == 0
     per_kind = {}
@@ -281,14 +282,21 @@ def main():
         per_kind[k] = (ns, getattr(prof, k + "_bytes"))
         log("[profile] %-9s %8.2f us (event pair per launch %8.2f us)  %7.1f GB/s  (%.1f%% of HBM peak)" % (
             k, ns / 1e3, paired / 1e3, per_kind[k][1] / max(ns, 1), 100 * per_kind[k][1] / max(ns, 1) / HBM_PEAK_GBS))
-    dom_ns, dom_bytes = per_kind["gate_up"]
-    dom_name = "gemv_fast_kernel<bf16, rmsnorm prologue, swiglu epilogue> (gate_up 24576x4096)"
-    traffic = GATE_UP_TRAFFIC_BYTES.get((cfg["hidden"], cfg["intermediate"]) + N.gemv_launch_plan(
-        1, 2, cfg["intermediate"], cfg["hidden"]))
+    if res.kernel_launches <= 4 * args.steps:
+        # the timed steps are the layers in one launch, the head and the sampler: the first's share is the step's device time
+        # without the head's (with what little the sampler and the gaps between them take, so the rate is no less than this)
+        dom_ns, dom_bytes = res.device_elapsed_ns / args.steps - prof.lm_head_ns, bytes_step - prof.lm_head_bytes
+        dom_name, traffic = "step_wide_kernel (all layers of a step)", None
+    else:
+        dom_ns, dom_bytes = per_kind["gate_up"]
+        dom_name = "gemv_fast_kernel<bf16, rmsnorm prologue, swiglu epilogue> (gate_up 24576x4096)"
+        traffic = GATE_UP_TRAFFIC_BYTES.get((cfg["hidden"], cfg["intermediate"]) + N.gemv_launch_plan(
+            1, 2, cfg["intermediate"], cfg["hidden"]))
+    log("[bench] dominant launch: %s, %.1f us, %.1f GB/s" % (dom_name, dom_ns / 1e3, dom_bytes / dom_ns))
     roofline = dict(bound="hbm", kernel=dom_name,
                     achieved=round(dom_bytes / dom_ns, 1), peak=HBM_PEAK_GBS, unit="GB/s",
                     frac=round(dom_bytes / dom_ns / HBM_PEAK_GBS, 4), traffic=traffic,
-                    bytes_per_launch=dom_bytes, avg_launch_us=round(dom_ns / 1e3, 2),
+                    bytes_per_launch=int(dom_bytes), avg_launch_us=round(dom_ns / 1e3, 2),
                     whole_step_bytes=bytes_step, whole_step_frac=round(bytes_step * tok_s / 1e9 / HBM_PEAK_GBS, 4),
                     per_kernel_frac={k: round(b / max(ns, 1) / HBM_PEAK_GBS, 4) for k, (ns, b) in per_kind.items()})
 
