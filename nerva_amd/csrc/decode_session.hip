@@ -2531,7 +2531,7 @@ int nerva_hip_hf_decode_sequence_session_advance(const NervaHipHfDecodeSequenceS
     if (s->has_eos == 0) err = ahead.room(taken);
     if (err == hipSuccess && s->has_eos == 0) err = look_back(s, &again);
     step -= again;
-    if (err == hipSuccess) err = launch_steps(s, s->cursor + step, s->has_eos != 0 ? 1 : run_count - step, &taken, out);
+    if (err == hipSuccess) err = launch_steps(s, s->cursor + step, s->has_eos != 0 || ahead.singly() ? 1 : run_count - step, &taken, out);
     // With a stop token the host looks at each token so that it can stop launching
     // (session_api_lifecycle.inc.cu:1206-1234); without one the loop never syncs.
     if (err == hipSuccess && s->has_eos != 0) {
@@ -2633,7 +2633,7 @@ int nerva_hip_hf_decode_sequence_session_run(const NervaHipHfDecodeSequenceSessi
     err = ahead.room(taken);
     if (err == hipSuccess) err = look_back(s, &again);
     step -= again;
-    if (err == hipSuccess) err = launch_steps(s, step, context_steps - step, &taken, out);
+    if (err == hipSuccess) err = launch_steps(s, step, ahead.singly() ? 1 : context_steps - step, &taken, out);
   }
   const uint64_t slots_bytes = static_cast<uint64_t>(context_steps) * sizeof(Slot);
   for (uint32_t again = 0; err == hipSuccess;) {

@@ -76,7 +76,7 @@ struct LaunchOrder {
   std::mutex mutex;
   NervaHipHfDecodeSequenceSession *alone = nullptr;             // the last one that needs the device to itself,
   std::vector<NervaHipHfDecodeSequenceSession *> beside;        // and those behind it that fit beside each other
-  std::atomic<uint32_t> sessions{0};
+  std::atomic<uint32_t> sessions{0}, calls{0};   // calls of theirs that are taking steps
 };
 
 struct StackModel;   // layer_stack.hpp
@@ -293,15 +293,24 @@ inline void out_of_order(Session *session) {
   if (order->alone == session || at != beside.end()) order->alone = nullptr;
   if (at != beside.end()) beside.erase(at);
 }
-// The steps that a call enqueues without looking at them: where a device has other sessions, no more than twice steps_ahead (some 2 ms each) before the call waits for
-// the older ones, so that whoever else steps comes in between; of steps in one launch never more than twice kUnseen, so that the host hears of those that give up before so many
+// The steps that a call enqueues without looking at them: where a device has other sessions, no more than twice steps_ahead (some 2 ms each, or a graph of several) before the call
+// waits for the older ones, so that whoever else steps comes in between; of steps in one launch never more than twice kUnseen, so that the host hears of those that give up before so many
 // have in a row that the device ends the sequence.
 class RunAhead {
   static constexpr uint32_t kUnseen = 96;
   static_assert(2 * kUnseen + Session::kStepsTogether < kMostGivenUp, "");
 
  public:
-  explicit RunAhead(Session *session) : s(session) {}
+  explicit RunAhead(Session *session) : s(session) {
+    if (s->order != nullptr) s->order->calls += 1;
+  }
+  ~RunAhead() {
+    if (s->order != nullptr) s->order->calls -= 1;
+  }
+  RunAhead(const RunAhead &) = delete;
+  RunAhead &operator=(const RunAhead &) = delete;
+  // Whether it is one step at a time: long ones, while others are calling.
+  bool singly() const { return s->order != nullptr && s->steps_ahead < Session::kStepsTogether && s->order->calls.load(std::memory_order_relaxed) > 1; }
   // Ahead of the next steps; `sent`: with those that went out since it was last asked.
   hipError_t room(uint32_t sent) {
     unseen += sent;

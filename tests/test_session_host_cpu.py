@@ -309,6 +309,22 @@ N.Device.set_tuning("step_chain", 2)
 s = N.DecodeSession.create(model(), 400)
 assert looks(s)[1] == 0
 s.destroy()
+N.Device.reset_tuning()
+large = dict(dtype=BF16, hidden=4096, heads=32, kv_heads=8, head_dim=128, intermediate=12288, vocab=64, layers=8, rms_eps=1e-6, rope_theta=1e4)   # (steps of .6 ms)
+s = N.DecodeSession.create_synthetic(large, 400)
+other = s.fork_shared_weights()
+double.double_clear_log()
+step(other)
+stream, = {line.split()[1] for line in log() if line.startswith("graph")}
+for held in (False, True, False):
+    assert other.start(np.arange(5, dtype=np.uint32))[0] == 0
+    looks(s)                                                # (the graph of six is there)
+    over = while_held(int(stream), lambda: other.advance(2)) if held else lambda: None
+    most, _ = looks(s)
+    assert most <= (6 if held else 18) and {line.split()[2] for line in log() if line.startswith("graph")} == {"3" if held else "18"}, (held, most)
+    over()
+other.destroy()
+s.destroy()
 """)
 
 
