@@ -126,10 +126,10 @@ __global__ __launch_bounds__(kBlock) void embed_rows_kernel(const uint16_t *emb,
   for (uint32_t i = threadIdx.x; i < hidden; i += kBlock) x[static_cast<uint64_t>(t) * hidden + i] = dec16<DT>(row[i]);
 }
 
-// Batch step: row t is the embedding of the token sequence t produced last (slot[position - 1]), and
-// the rotation table of its position. What the step's other launches read of the sequence comes with it: `from` is the host's table in pinned memory, of which a
-// workgroup brings its sequence's entries to `table`. (A copy by the runtime
-// ahead of the launch: 9 to 12 us more a step, 820 -> 808 us on the device with 32 sequences 4096 wide, 446 -> 437 with 6 of 1024; the slots' way out likewise.)
+// Batch step: row t is the embedding of the token sequence t produced last (slot[position - 1]), and the rotation table of its
+// position. What the step's other launches read of the sequence comes with it: `from` is the host's table in pinned memory, of
+// which a workgroup brings its sequence's entries to `table`. (A copy by the runtime ahead of the launch: 9 to 12 us more a step,
+// 820 -> 808 us on the device with 32 sequences 4096 wide, 446 -> 437 with 6 of 1024; the slots' way out likewise.)
 template <uint32_t DT>
 __global__ __launch_bounds__(kBlock) void embed_batch_kernel(const uint16_t *emb, const BatchTable *from, BatchTable *table, uint32_t hidden,
                                                              uint32_t vocab, float *x, const float *rope_freq,
@@ -177,9 +177,10 @@ __global__ void gather_slots_kernel(const BatchTable *table, uint32_t count, Slo
   reinterpret_cast<uint32_t *>(out + t)[w] = reinterpret_cast<const uint32_t *>(slot)[w];
 }
 
-// What a call brings of a sequence before its prompt is read: tokens, from the host's pinned memory to their places, and the position words; of a new sequence
-// its sampler, and what an earlier one has left is cleared. One launch: two copies by the runtime, which the host waited for, and up to five launches more took 30 to 40 us a call, and
-// ones the host waits for keep the sequences of one caller from following each other without a gap.
+// What a call brings of a sequence before its prompt is read: tokens, from the host's pinned memory to their places, and the
+// position words; of a new sequence its sampler, and what an earlier one has left is cleared. One launch: two copies by the
+// runtime, which the host waited for, and up to five launches more took 30 to 40 us a call, and ones the host waits for keep the
+// sequences of one caller from following each other without a gap.
 struct SequenceParams {
   const uint32_t *from;        // pinned
   uint32_t *prompt, *state;
@@ -656,9 +657,10 @@ hipError_t ensure_graph(Session *s, int which, NervaHipHfDecodeSequenceResult *o
   return hipSuccess;
 }
 
-// A graph's launch leaves the device idle for 4 us, which the launches within it do not (replays of three launches of 17.4 us each: 56.4 us, of 24
-// 415; the launches alone 52.4 and 419), so steps of few launches go out kStepsTogether at a time once a session has taken enough of them to pay for that graph
-// (some 0.15 ms). Of steps of five launches a layer that is nothing, and their graphs take longer to make.
+// A graph's launch leaves the device idle for 4 us, which the launches within it do not (replays of three launches of 17.4 us
+// each: 56.4 us, of 24 415; the launches alone 52.4 and 419), so steps of few launches go out kStepsTogether at a time once a
+// session has taken enough of them to pay for that graph (some 0.15 ms). Of steps of five launches a layer that is nothing, and
+// their graphs take longer to make.
 constexpr uint64_t kTogetherFrom = 64;
 void ensure_together(Session *s, uint32_t position, uint32_t steps) {
   const int which = decode_graph(s, position);
@@ -678,10 +680,11 @@ hipError_t ensure_graphs(Session *s, uint32_t position, uint32_t steps, NervaHip
   return err;
 }
 
-// Steps that have given up since the last look, of work that is done: the next step was the same one again, and as many are still to come. (One that
-// ends the sequence with a fault counts as done; the bit stays until another begins.)
-// Where nothing but such steps has been seen for kMissesMost of them (0.1 s), whoever holds the places will not let go soon: the next kAvoidSteps go launch by launch, which need
-// theirs for one layer's attention at a time. (Not where a test hook makes the waits run out, so that the end of it all is reached; "step_chain" = 1: there too.)
+// Steps that have given up since the last look, of work that is done: the next step was the same one again, and as many are still
+// to come. (One that ends the sequence with a fault counts as done; the bit stays until another begins.) Where nothing but such
+// steps has been seen for kMissesMost of them (0.1 s), whoever holds the places will not let go soon: the next kAvoidSteps go
+// launch by launch, which need theirs for one layer's attention at a time. (Not where a test hook makes the waits run out, so
+// that the end of it all is reached; "step_chain" = 1: there too.)
 constexpr uint32_t kMissesMost = 32, kAvoidSteps = 256;
 uint32_t take_given_up(Session *s) {
   if (s->given_up == nullptr) return 0;
@@ -839,8 +842,9 @@ bool slots_faulted(const Slot *slots, uint32_t count) {
   return false;
 }
 
-// Tokens `first` .. of the sequence, as many as `count`, and its position there, behind what the session's stream holds, for which this waits: the way
-// leads through the session's pinned copy. The caller's memory may be used again as soon as this returns.
+// Tokens `first` .. of the sequence, as many as `count`, and its position there, behind what the session's stream holds, for
+// which this waits: the way leads through the session's pinned copy. The caller's memory may be used again as soon as this
+// returns.
 hipError_t bring_tokens(Session *s, SequenceParams p, const uint32_t *tokens, uint32_t first, uint32_t count, NervaHipHfDecodeSequenceResult *out) {
   const hipError_t err = hipStreamSynchronize(s->stream);
   if (err != hipSuccess) return err;
@@ -1161,12 +1165,13 @@ hipError_t allocate_session(Session *s, int32_t *failure_stage, bool with_weight
   return hipSuccess;
 }
 
-// The runtime's own copy into memory that is not pinned is the faster one between 16 KiB and 1 MiB: a call of 64 tokens with 8 rows of logits
-// apart, 32 KB / 128 KB / 608 KB a row, 371 / 453 / 920 us, through pinned memory 421 / 591 / 983. Smaller pieces arrive in pinned memory
-// by a kernel: 8 rows of 16 KB 298 us, with the runtime's copies 341. For larger ones the runtime pins the caller's pages (us behind a kernel into memory written
-// before / fresh: 1.2 MB 91 / 289, 3 MB 174 / 628, 4.9 MB 277 / 1064): those leave in pieces of 512 KiB through two pinned halves, the session's own,
-// one on its way while the other is copied on (78 / 219, 157 / 479, 244 / 770) - where a few rows are as much. Where the caller's memory is
-// pinned (or managed) itself the copy goes straight there, and the host goes on with the next launches.
+// The runtime's own copy into memory that is not pinned is the faster one between 16 KiB and 1 MiB: a call of 64 tokens with 8
+// rows of logits apart, 32 KB / 128 KB / 608 KB a row, 371 / 453 / 920 us, through pinned memory 421 / 591 / 983. Smaller pieces
+// arrive in pinned memory by a kernel: 8 rows of 16 KB 298 us, with the runtime's copies 341. For larger ones the runtime pins
+// the caller's pages (us behind a kernel into memory written before / fresh: 1.2 MB 91 / 289, 3 MB 174 / 628, 4.9 MB 277 / 1064):
+// those leave in pieces of 512 KiB through two pinned halves, the session's own, one on its way while the other is copied on (78
+// / 219, 157 / 479, 244 / 770) - where a few rows are as much. Where the caller's memory is pinned (or managed) itself the copy
+// goes straight there, and the host goes on with the next launches.
 hipError_t copy_out(Session *s, void *dst, const void *src, uint64_t bytes, uint64_t *waits, bool now) {
   bool staged = bytes <= kStageLeast || (bytes >= kStageFrom && s->stage_half == kStageMost);
   if (staged) {
@@ -2254,10 +2259,11 @@ int nerva_hip_hf_decode_sequence_batch_advance_one(const NervaHipHfDecodeSequenc
         out->projection_elapsed_ns = std::max<uint64_t>(1, static_cast<uint64_t>(static_cast<double>(ms) * 1e6));
     }
   } else if (err == hipSuccess) {
-    // shapes outside the multi-row kernels: every sequence runs its own captured step on its own stream - one
-    // after the other (each stream waits for the step before it): a step's attention launch wants every CU for
-    // workgroups that poll for each other, and two such launches side by side could hold each other's CUs; narrow models' steps fit beside each other, but not all
-    // of them. The tokens leave behind the last step: a step that waits for the one before would wait for its token's copy too
+    // shapes outside the multi-row kernels: every sequence runs its own captured step on its own stream - one after the other
+    // (each stream waits for the step before it): a step's attention launch wants every CU for workgroups that poll for each
+    // other, and two such launches side by side could hold each other's CUs; narrow models' steps fit beside each other, but not
+    // all of them. The tokens leave behind the last step: a step that waits for the one before would wait for its token's copy
+    // too
     NervaHipHfDecodeSequenceResult scratch{};
     Session *before = nullptr;
     const auto count_step = [out](const Session *q, int which) {   // (layers in one launch: the embedding and attention included)

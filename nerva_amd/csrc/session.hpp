@@ -49,9 +49,10 @@ struct SharedWeights {
   RowScratch pass;
   std::mutex pass_turn;
   hipEvent_t pass_done = nullptr;
-  // Prompts under way of the creating session and all its forks, each behind an event: one that begins comes behind the last but kPromptsAhead
-  // (PromptTurn), so that no more than those (and one for each thread that is enqueuing its own) are on the device at once, however many a caller begins. As many as there are
-  // hardware queues: 32 prompts of 65 to 195 tokens 4096 wide take 27.8 ms with four or with eight, 29.5 with two; six of 37 to 112 tokens 1024 wide 2.6 and 3.7.
+  // Prompts under way of the creating session and all its forks, each behind an event: one that begins comes behind the last but
+  // kPromptsAhead (PromptTurn), so that no more than those (and one for each thread that is enqueuing its own) are on the device
+  // at once, however many a caller begins. As many as there are hardware queues: 32 prompts of 65 to 195 tokens 4096 wide take
+  // 27.8 ms with four or with eight, 29.5 with two; six of 37 to 112 tokens 1024 wide 2.6 and 3.7.
   static constexpr uint32_t kPromptsAhead = 4;
   hipEvent_t prompt_done[kPromptsAhead] = {};
   uint64_t prompts = 0;              // recorded so far
@@ -70,8 +71,8 @@ struct BatchTable {
   SamplerParams sample[kGemmMaxTokens];
 };
 
-// Launches whose workgroups wait for each other find a place for all of them or wait in vain, and two at once may each hold what the other one needs.
-// Of a device's sessions: who has such launches that may still be under way (InOrder).
+// Launches whose workgroups wait for each other find a place for all of them or wait in vain, and two at once may each hold what
+// the other one needs. Of a device's sessions: who has such launches that may still be under way (InOrder).
 struct LaunchOrder {
   std::mutex mutex;
   NervaHipHfDecodeSequenceSession *alone = nullptr;             // the last one that needs the device to itself,
@@ -124,8 +125,9 @@ struct NervaHipHfDecodeSequenceSession : nv::RowScratch {
   hipGraph_t graph[kGraphs] = {};
   hipGraphExec_t exec[kGraphs] = {};
   uint64_t graph_nodes[kGraphs] = {};
-  // Of graphs 3 and 4, kStepsTogether steps of them in one graph (ensure_together)
-  static constexpr uint32_t kStepsTogether = 6;   // (calls of 8 to 32 steps: the fewest launches with what is left over, which goes out singly)
+  // Of graphs 3 and 4, kStepsTogether steps of them in one graph (ensure_together) (each graph saves all but one of its steps' 4
+  // us; what a call has left over goes out singly: six save 3.3 us a step and leave five at the most, twelve 3.7 and eleven)
+  static constexpr uint32_t kStepsTogether = 6;
   hipGraph_t together_graph[2] = {};
   hipGraphExec_t together[2] = {};
   uint64_t chain_steps = 0;          // steps that went out as chains
@@ -242,12 +244,13 @@ class PassTurn {
   std::unique_lock<std::mutex> turn;
 };
 
-// While this lives the session enqueues a launch whose workgroups wait for each other, behind those of other sessions that it must not meet - of calls in other threads, and of
-// starts that have returned while a prompt that is walked, or whose last token takes a step, is under way. The streams keep that
-// order: nobody waits on the host or on the device in front of what is to be waited for, and a session that has no other's launches under way beside it enqueues no more than
-// the launch. (Turns that a launch of one wave took by polling a word stood in front of what would have given the word back where two sessions share a hardware
-// queue; and they took two launches more a step beside any other session, idle or not: 69.4 -> 72.3 us at 512 wide,
-// 845 -> 848 at 4096.)
+// While this lives the session enqueues a launch whose workgroups wait for each other, behind those of other sessions that it
+// must not meet - of calls in other threads, and of starts that have returned while a prompt that is walked, or whose last token
+// takes a step, is under way. The streams keep that order: nobody waits on the host or on the device in front of what is to be
+// waited for, and a session that has no other's launches under way beside it enqueues no more than the launch. (Turns that a
+// launch of one wave took by polling a word stood in front of what would have given the word back where two sessions share a
+// hardware queue; and they took two launches more a step beside any other session, idle or not: 69.4 -> 72.3 us at 512 wide, 845
+// -> 848 at 4096.)
 enum class Place { kBeside, kAlone };   // meets its like (narrow models' steps); nobody
 class InOrder {
  public:
@@ -293,9 +296,10 @@ inline void out_of_order(Session *session) {
   if (order->alone == session || at != beside.end()) order->alone = nullptr;
   if (at != beside.end()) beside.erase(at);
 }
-// The steps that a call enqueues without looking at them: where a device has other sessions, no more than twice steps_ahead (some 2 ms each, or a graph of several) before the call
-// waits for the older ones, so that whoever else steps comes in between; of steps in one launch never more than twice kUnseen, so that the host hears of those that give up before so many
-// have in a row that the device ends the sequence.
+// The steps that a call enqueues without looking at them: where a device has other sessions, no more than twice steps_ahead (some
+// 2 ms each, or a graph of several) before the call waits for the older ones, so that whoever else steps comes in between; of
+// steps in one launch never more than twice kUnseen, so that the host hears of those that give up before so many have in a row
+// that the device ends the sequence.
 class RunAhead {
   static constexpr uint32_t kUnseen = 96;
   static_assert(2 * kUnseen + Session::kStepsTogether < kMostGivenUp, "");
@@ -329,8 +333,9 @@ class RunAhead {
   bool marked = false;
 };
 
-// A prompt's place among those under way: as long as its launches are enqueued this lives. The stream waits, not the host (five starts of 8000 tokens, 12 layers 4096 wide:
-// 47.9 -> 3.3 ms of the caller, done after 262 either way; 20 steps of another session behind them 22.8 ms and 25.4), so it is made behind whatever the host itself waits for.
+// A prompt's place among those under way: as long as its launches are enqueued this lives. The stream waits, not the host (five
+// starts of 8000 tokens, 12 layers 4096 wide: 47.9 -> 3.3 ms of the caller, done after 262 either way; 20 steps of another
+// session behind them 22.8 ms and 25.4), so it is made behind whatever the host itself waits for.
 class PromptTurn {
  public:
   explicit PromptTurn(Session *session) : s(session) {

@@ -55,10 +55,15 @@ constexpr uint32_t kChainSingleBlocks = 8;
 constexpr uint32_t kChainMaxHidden = 1024, kChainMaxIn = 4096, kChainMaxQkv = 8192, kChainMaxSplits = 16;
 // Tokens of context up to which any model's steps run as a chain (chain_context: less for some)
 constexpr uint32_t kChainContext = 4096;
-// ... and those of a wide model: as far as that is the faster step at every shape measured, by the workgroups that read its keys (3584 x 18944, 28 heads on 4, 8000 /
-// 16000 / 32000 keys: 94.4 / 96.9 / 103.3 us a layer in launches, 92.8 / 97.1 / 106.5; 2048 x 8192, 32 heads of 64 on 8: 38.3 / 41.7 / 45.7 and 33.7 / 37.3 / 45.0)
+// ... and those of a wide model, by its key heads: the fewer, the fewer workgroups have a part of the context (sixteen splits of
+// each at the most, where a step's attention launch makes as many as there are CUs), and the sooner its attention outlasts what
+// the ring holds. 43 shapes of 1 to 32 key heads, one to four layers, 768 to 8192 wide, 22 to 1380 MB a layer, at 700 to 32000
+// keys, time over that of the step in launches. Less than eight key heads, 8000 keys: .87 to .996 and one 1.003 (4096 x 12288,
+// one key head of eight query heads, two layers); at 12000 .89 to 1.03, at 32000 .99 to 1.24. Eight and more, 32000 keys: .88 to
+// .987 and one 1.005 (768 x 4096, nine heads of 64).
 constexpr uint32_t wide_context(uint32_t kv_heads) { return kv_heads >= 8 ? 32768u : 8192u; }
-// Polls after which a wait gives up: 3.1 ms (a step whose workgroup 0 stays away), where the longest wait of a healthy launch is some 20 us.
+// Polls after which a wait gives up: 3.1 ms (a step whose workgroup 0 stays away), where the longest wait of a healthy launch is
+// some 20 us.
 constexpr uint32_t kChainSpinLimit = 1u << 14;
 // Whether a model's steps can run as a chain.
 bool chain_takes(uint32_t layers, uint32_t hidden, uint32_t heads, uint32_t kv_heads, uint32_t head_dim, uint32_t ff);

@@ -1,5 +1,6 @@
-// What the launches that hold a whole step's layers share (step_chain.hip, step_wide.hip): the model through the scalar path, bounded waits for
-// tagged words, and the attention of one layer as its q, k and v arrive. W: waves of a workgroup that take part; Meet: their barrier.
+// What the launches that hold a whole step's layers share (step_chain.hip, step_wide.hip): the model through the scalar path,
+// bounded waits for tagged words, and the attention of one layer as its q, k and v arrive. W: waves of a workgroup that take
+// part; Meet: their barrier.
 #pragma once
 
 #include <algorithm>
@@ -15,8 +16,8 @@ namespace chain {
 
 using namespace attn;
 
-// The model through the scalar path. `fresh` forgets what has been read of it, so that a stage holds what it uses and no more: held over the
-// whole loop, the model's and the layer's words and the addresses made of them take more registers than there are.
+// The model through the scalar path. `fresh` forgets what has been read of it, so that a stage holds what it uses and no more:
+// held over the whole loop, the model's and the layer's words and the addresses made of them take more registers than there are.
 typedef const __attribute__((address_space(4))) ChainModel *Model;
 __device__ __forceinline__ void fresh(Model &m) { asm volatile("" : "+s"(m)); }
 __device__ __forceinline__ uint32_t fresh_thread() {
@@ -81,8 +82,8 @@ __device__ __forceinline__ void chain_splits(uint32_t kv_heads, uint32_t pos, ui
   active = (nblk + bps - 1) / bps;
 }
 
-// The attention of one (key head, split): its q, k and v as they arrive, the cache's tiles through the matrix cores (attn_tile), and the 16-bit
-// output or, of several splits, the partial sums.
+// The attention of one (key head, split): its q, k and v as they arrive, the cache's tiles through the matrix cores (attn_tile),
+// and the 16-bit output or, of several splits, the partial sums.
 template <uint32_t DT, int HD, int G, bool PARTS, int W, typename Meet>
 __device__ __forceinline__ void chain_attention(Model m_, uint32_t layer, uint32_t pos, uint32_t kvh, uint32_t split, uint32_t nblk, uint32_t bps,
                                                 uint32_t active, uint32_t tag, Waiter &wait, const float *rotation, ChainAttnShared<HD, G, PARTS, W> &sh, Meet &meet) {

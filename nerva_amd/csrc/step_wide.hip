@@ -1,34 +1,40 @@
 // A decode step's layers in one launch, for models whose layers are too large for step_chain.hip.
 //
-// What a step of these models costs beyond its bytes is the five launches a layer: behind each boundary memory stands idle until the next launch's
-// first requests are served (2.5 to 3 us, a layer of 101 MB 30 us for 15 us of reads). Here a workgroup a CU stays for the whole step and
-// hands vectors on as words of (value, tag), as in step_chain.hip, and the weights run ahead of that: two waves of a workgroup do nothing but ask for
-// them, in the order in which they will be used, whole layers long, straight into a ring in LDS (80 to 140 KiB) that the other eight read. So while those wait for a
-// vector, memory goes on until the ring is full - 20 to 35 MB over the chip, 3 to 5 us of it. us a layer, launches and here, 40 / 700 / 8000 keys of context:
+// What a step of these models costs beyond its bytes is the five launches a layer: behind each boundary memory stands idle until
+// the next launch's first requests are served (2.5 to 3 us, a layer of 101 MB 30 us for 15 us of reads). Here a workgroup a CU
+// stays for the whole step and hands vectors on as words of (value, tag), as in step_chain.hip, and the weights run ahead of
+// that: two waves of a workgroup do nothing but ask for them, in the order in which they will be used, whole layers long,
+// straight into a ring in LDS (what the vectors leave of it, 64 to 140 KiB) that the other eight read. So while those wait for a
+// vector, memory goes on until the ring is full - 16 to 35 MB over the chip, 2.5 to 5 us of it. us a layer, launches and here, 40
+// / 700 / 8000 keys of context:
 //    1024 x  3072, 16 heads of 128 on 8:  20.9 / 23.4 / 26.9    18.1 / 20.3 / 25.0     (31 MB)
 //    2048 x  6144, 16 heads of 128 on 8:  30.2 / 32.7 / 36.2    25.0 / 27.4 / 32.1     (101 MB)
 //    2048 x  8192, 32 heads of  64 on 8:  33.6 / 36.3 / 38.3    29.2 / 30.3 / 33.7     (122 MB)
 //    2560 x  9728, 32 heads of 128 on 8:  47.2 / 49.7 / 53.7    41.3 / 44.1 / 48.6     (202 MB)
 //    4096 x 12288, 32 heads of 128 on 8:  70.6 / 73.1 / 77.0    68.0 / 69.8 / 74.7     (386 MB)
 //    5120 x 13824, 40 heads of 128 on 8: 106.0 / 109 / 114      97.0 / 98.8 / 103      (551 MB)
-// What bounds it now: the hand-overs (1.2 us each and more under load, for the words travel through the memory that the weights come from), and the
-// slowest of 256 shares of a projection.
+// What bounds it now: the hand-overs (1.2 us each and more under load, for the words travel through the memory that the weights
+// come from), and the slowest of 256 shares of a projection.
 //
 // Three things that cost more than they look:
-//   * how much is on its way. The more weights a CU has asked for, the longer a word waits behind them: with 16 KiB a loader 2048 x 6144 took 25.2 us a layer, with
-//     40 KiB 28, with 52 KiB 32; with 4 KiB, too few, 27.
-//   * polling too early. A workgroup that looks for words while their writers still write them takes those lines from them: words of 256 writers, eight to a line, are
-//     there after 0.9 us if everyone waits half of that before the first look, after 2 us otherwise. So a wait begins with a pause (kPause:
-//     none / 14 / 22 / 30: 28.3 / 27.2 / 25.0 / 24.9 us a layer at 2048 x 6144, 16.9 / 15.3 / 14.3 / 15.0 at 512 x 1376).
-//   * where the rows begin. Consecutive rows start their walk a request further on, and wrap: rows are a multiple of the memory channels' interleave apart.
+//   * how much is on its way. The more weights a CU has asked for, the longer a word waits behind them: with 16 KiB a loader 2048
+//     x 6144 took 25.2 us a layer, with 40 KiB 28, with 52 KiB 32; with 4 KiB, too few, 27.
+//   * polling too early. A workgroup that looks for words while their writers still write them takes those lines from them: words
+//     of 256 writers, eight to a line, are there after 0.9 us if everyone waits half of that before the first look, after 2 us
+//     otherwise. So a wait begins with a pause (kPause: none / 14 / 22 / 30: 28.3 / 27.2 / 25.0 / 24.9 us a layer at 2048 x 6144,
+//     16.9 / 15.3 / 14.3 / 15.0 at 512 x 1376).
+//   * where the rows begin. Consecutive rows start their walk a request further on, and wrap: rows are a multiple of the memory
+//     channels' interleave apart.
 //
-// The ring: a round is a request of 1 KiB (512 columns of a row) for each of the eight waves; a loader asks for four waves' and says how many rounds have arrived, a wave
-// says how many it has used. A projection's rows lie together in a workgroup. Where they do not go round the waves evenly a row is cut into two to eight parts (ten rows of
-// nineteen requests: five rounds of five in four parts, not two of nineteen); parts meet in LDS.
+// The ring: a round is a request of 1 KiB (512 columns of a row) for each of the eight waves; a loader asks for four waves' and
+// says how many rounds have arrived, a wave says how many it has used. A projection's rows lie together in a workgroup. Where
+// they do not go round the waves evenly a row is cut into two to eight parts (ten rows of nineteen requests: five rounds of five
+// in four parts, not two of nineteen); parts meet in LDS.
 //
-// The loaders take part in no barrier, so the others' is a counter in LDS (Meet). Everything else - the places of words, who overwrites what when, waits
-// that run out, steps that are void and taken again - is as in step_chain.hip. A workgroup has a CU to itself here, all 256 wait for each other: two such launches that started
-// at once could each hold half of the chip until both give up. So a step comes behind what other sessions of the device have under way of that sort (InOrder in session.hpp).
+// The loaders take part in no barrier, so the others' is a counter in LDS (Meet). Everything else - the places of words, who
+// overwrites what when, waits that run out, steps that are void and taken again - is as in step_chain.hip. A workgroup has a CU
+// to itself here, all 256 wait for each other: two such launches that started at once could each hold half of the chip until both
+// give up. So a step comes behind what other sessions of the device have under way of that sort (InOrder in session.hpp).
 #include <float.h>
 
 #include "step_parts.cuh"
@@ -409,7 +415,8 @@ __global__ __launch_bounds__(kThreads + kLoaders *kWave, 1) void step_wide_kerne
     return p.trace + at;
   };
 
-  // A row of x or r as it comes (`first`: the token's embedding), pairs of elements thread + i * 512: normalised into x16, the workgroup's own elements kept.
+  // A row of x or r as it comes (`first`: the token's embedding), pairs of elements thread + i * 512: normalised into x16, the
+  // workgroup's own elements kept.
   uint32_t turn = 0;
   const auto take_row = [&](auto n_, const uint64_t *src, const uint16_t *gamma, uint32_t tag, float *own, bool first, char *raw) {
     constexpr int N = decltype(n_)::value, kAtOnce = N <= 5 ? N : N / 2;
@@ -446,7 +453,8 @@ __global__ __launch_bounds__(kThreads + kLoaders *kWave, 1) void step_wide_kerne
     ss = wave_sum(ss);
     if (thread % kWave == 0) sh.red[turn][wave] = ss;
     meet();
-    // (as in step_chain.hip: 1 / sqrt by the hardware's and a step of Newton's, but for means that it takes for zero and sums that overflowed)
+    // (as in step_chain.hip: 1 / sqrt by the hardware's and a step of Newton's, but for means that it takes for zero and sums
+    // that overflowed)
     const float4 r0 = *reinterpret_cast<const float4 *>(&sh.red[turn][0]), r1 = *reinterpret_cast<const float4 *>(&sh.red[turn][4]);
     const float mean = fmaf(((r0.x + r0.y) + (r0.z + r0.w)) + ((r1.x + r1.y) + (r1.z + r1.w)), m->inv_hidden, m->eps);
     const float rough = __builtin_amdgcn_rsqf(mean);
@@ -594,12 +602,14 @@ bool wide_takes(uint32_t dtype, uint32_t layers, uint32_t hidden, uint32_t heads
   if (!attn_matrix_cores(heads, kv_heads, head_dim) || heads > 512 || kv_heads > 32) return false;
   // Every workgroup has rows of o and down and pairs of gate and up, whole 16-byte pieces of them, no more of x than it keeps.
   if (layers == 0 || layers >= 255 || hidden < kWorkgroups || hidden > kWorkgroups * kMostOwn || hidden % 8 != 0 || ff < 2 * kWorkgroups || ff % 8 != 0) return false;
-  // From 12 MB of weights a layer on (chain_takes ends at 10). 27 stacks drawn between 14 and 501 MB, widths of 768 to 3520, 40 / 700 / 3000 keys: 0.85 of the launches' time
-  // on average, 0.71 the least; one is no faster (3520 x 8096, 27 heads of 128 on 27, whose q, k and v are as long as its attention: 59.5 / 61.3 / 66.3 us a layer in launches, 59.7 /
-  // 62.1 / 66.1).
-  // Two and three layers: from 64 MB each on, where 21 models, those of one layer among them, take 0.77 to 0.97 of the launches' time a step, at 40 to 3000 keys (2 layers of 2048 x 6144 82.6 -> 67.0 us at 700
-  // keys, 3 of 4096 x 12288 238 -> 223); smaller ones would gain as well, and keep the launches. One layer: from 256 MB on, what the memory-side cache holds (4096 x 12288 96.6 -> 87.6,
-  // 5120 x 13824 136 -> 116); of a smaller one the launches read the weights there, and past 2000 keys some are the faster steps (1536 x 7000 51.6, 61.3 in one launch; 2560 x 7000 65.0, 66.2).
+  // From 12 MB of weights a layer on (chain_takes ends at 10). 27 stacks drawn between 14 and 501 MB, widths of 768 to 3520, 40 /
+  // 700 / 3000 keys: 0.85 of the launches' time on average, 0.71 the least; one is no faster (3520 x 8096, 27 heads of 128 on 27,
+  // whose q, k and v are as long as its attention: 59.5 / 61.3 / 66.3 us a layer in launches, 59.7 / 62.1 / 66.1). Two and three
+  // layers: from 64 MB each on, where 21 models, those of one layer among them, take 0.77 to 0.97 of the launches' time a step,
+  // at 40 to 3000 keys (2 layers of 2048 x 6144 82.6 -> 67.0 us at 700 keys, 3 of 4096 x 12288 238 -> 223); smaller ones would
+  // gain as well, and keep the launches. One layer: from 256 MB on, what the memory-side cache holds (4096 x 12288 96.6 -> 87.6,
+  // 5120 x 13824 136 -> 116); of a smaller one the launches read the weights there, and past 2000 keys some are the faster steps
+  // (1536 x 7000 51.6, 61.3 in one launch; 2560 x 7000 65.0, 66.2).
   const uint64_t weights = static_cast<uint64_t>(hidden) * (2 * heads + 2 * kv_heads) * head_dim + 3ull * hidden * ff;
   if (weights <= (layers >= 4 ? 6000000u : layers >= 2 ? 32000000u : 128000000u)) return false;
   const uint32_t rows = std::max((heads + 2 * kv_heads) * head_dim, 2 * ff + 2 * kWorkgroups);
